@@ -25,8 +25,6 @@
 #include "common.h"
 #include "quant_math.h"
 
-#include <stdlib.h>
-
 #include <type_traits>
 
 namespace mi {
@@ -49,7 +47,6 @@ struct GemmArgs {
   int tiles_m, tiles_n;
   void *c;
   int64_t ldc;
-  int diag_same_panel;  // timing what-if (wrong results): every tile fetches the operands of tile (0, 0), see diag_same_panel()
 };
 
 // Asynchronous 16-byte-per-lane copy global -> LDS: lane L's 16 bytes land at lds_wave_base + 16 * L;
@@ -801,9 +798,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 // above.  T = 2 (128 x 128, slots of 16 KiB, 80 KiB of LDS, a quarter of the registers) lets two workgroups share a
 // CU: for shapes with fewer than one 256 x 256 tile per CU, or short K, where one tile's prologue and epilogue have
 // to overlap another tile's main loop.  Per quarter a wave then has 4 MFMAs, 4 fragment reads and 2 loads.
-// DIAG: timing what-ifs of the main loop (wrong results, see diag_kblock128()): bit 0 = no operand loads after the
-// first two K blocks, bit 1 = no wait and no barrier between K blocks.
-template <int T, int EPI, bool HAS_ZW, bool FAST, int DIAG = 0>
+template <int T, int EPI, bool HAS_ZW, bool FAST>
 __device__ __forceinline__ void gemm_kblock_body(const GemmArgs &g, const RequantParams &rq, const DequantParams &dq) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the buffer-resource type exists in the device pass only; the host pass needs just the stub
   constexpr int TILE = 64 * T, KB = 128;  // wave tile 32 T x 32 T = T x T MFMA tiles
@@ -834,11 +829,10 @@ __device__ __forceinline__ void gemm_kblock_body(const GemmArgs &g, const Requan
   // issuing one costs scalar instructions only.
   const int drow = lane >> 3;
   const int dchunk = (lane & 7) ^ (drow >> 1);  // for even i; odd i: ^ 4
-  const int ld_n0 = g.diag_same_panel ? 0 : n0, ld_m0 = g.diag_same_panel ? 0 : m0;
   const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<int8_t *>(g.w) + (int64_t)(ld_n0 + wave * WROWS) * g.ldw, (short)0, -1, 0x00020000);
+      const_cast<int8_t *>(g.w) + (int64_t)(n0 + wave * WROWS) * g.ldw, (short)0, -1, 0x00020000);
   const __amdgpu_buffer_rsrc_t a_rsrc =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(g.a) + (int64_t)ld_m0 * g.lda, (short)0, -1, 0x00020000);
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(g.a) + (int64_t)m0 * g.lda, (short)0, -1, 0x00020000);
   const int w_voff = drow * g.ldw + dchunk * 16;  // ldw is a multiple of 256: odd i is w_voff ^ 64
   int a_voff[LPW];
 #pragma unroll
@@ -861,7 +855,6 @@ __device__ __forceinline__ void gemm_kblock_body(const GemmArgs &g, const Requan
   auto lds_ptr = [](char *p) { return (__attribute__((address_space(3))) void *)p; };
   // half: 0 = the first half of the wave's loader instructions (the upper half of its rows), 1 = the other half
   auto dma_w = [&](int slot, int kb, int half) {
-    if ((DIAG & 1) && kb > 1) return;
     char *dst = lds + slot * SLOT + wave * WROWS * KB;
 #pragma unroll
     for (int ii = 0; ii < LPW / 2; ++ii) {
@@ -871,7 +864,6 @@ __device__ __forceinline__ void gemm_kblock_body(const GemmArgs &g, const Requan
     }
   };
   auto dma_a = [&](int slot, int kb, int half) {
-    if ((DIAG & 1) && kb > 1) return;
     char *dst = lds + (3 + slot) * SLOT + wave * WROWS * KB;
 #pragma unroll
     for (int ii = 0; ii < LPW / 2; ++ii) {
@@ -1016,9 +1008,7 @@ __device__ __forceinline__ void gemm_kblock_body(const GemmArgs &g, const Requan
     if (NEXT2) dma_w(ws2, b + 2, 1);
     mma(f0, b * 8 + 4 + h);
     hints();
-    if (DIAG & 2) {
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    } else if (NEXT2) {
+    if (NEXT2) {
       // everything but the loads of W block b+2 has landed: that includes all of block b+1
       asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LPW) : "memory");
     } else if (NEXT1) {
@@ -1069,36 +1059,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   gemm_kblock_body<2, EPI, HAS_ZW, FAST>(g, rq, dq);
 }
 
-template <int EPI, int DIAG>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_kblock128_diag_kernel(
-    GemmArgs g, RequantParams rq, DequantParams dq) {
-  gemm_kblock_body<2, EPI, false, true, DIAG>(g, rq, dq);
-}
-
 // ---- host side -----------------------------------------------------------------------------------------------
-// Measurement aid, off unless the environment says MI355X_DIAG_SAME_PANEL=1 when the library is first used: the
-// K-block kernels then fetch tile (0, 0)'s operands for every tile, so that every operand line is an L2 hit.  The
-// results are wrong; the launch time shows what the L2 misses of the real access pattern cost.
-static int diag_same_panel() {
-  static const int on = [] {
-    const char *e = getenv("MI355X_DIAG_SAME_PANEL");
-    return (e != nullptr && e[0] == '1') ? 1 : 0;
-  }();
-  return on;
-}
-
-// A second one, MI355X_DIAG_KBLOCK128=<1|2|3>: builds of the 128 x 128 K-block kernel (no weight zero point, the
-// one-multiply epilogue) without the operand loads after the first two K blocks (1), without the wait and the barrier
-// between K blocks (2), or without both (3).  The results are wrong; the launch times say what the main loop spends
-// on the matrix cores and what on feeding them.
-static int diag_kblock128() {
-  static const int v = [] {
-    const char *e = getenv("MI355X_DIAG_KBLOCK128");
-    return (e != nullptr && e[0] >= '1' && e[0] <= '3') ? e[0] - '0' : 0;
-  }();
-  return v;
-}
-
 template <int TILE_N, int TILE_M, int EPI, bool HAS_ZW, bool FAST, int NST = 4, int OCC = 1>
 static int launch_cfg(GemmArgs g, const RequantParams &rq, const DequantParams &dq, hipStream_t stream) {
   g.tiles_m = (g.m + TILE_M - 1) / TILE_M;
@@ -1114,7 +1075,6 @@ template <int EPI, bool HAS_ZW, bool FAST>
 static int launch_kblock(GemmArgs g, const RequantParams &rq, const DequantParams &dq, hipStream_t stream) {
   g.tiles_m = (g.m + 255) / 256;
   g.tiles_n = (g.n + 255) / 256;
-  if ((g.m & 255) != 0 || (g.n & 255) != 0) g.diag_same_panel = 0;  // (the row clamps of ragged tiles assume the tile's own base)
   hipLaunchKernelGGL((gemm_kblock_kernel<EPI, HAS_ZW, FAST>), dim3(g.tiles_m * g.tiles_n), dim3(256), 0, stream, g, rq,
                      dq);
   MI_HIP_CHECK(hipGetLastError());
@@ -1125,17 +1085,6 @@ template <int EPI, bool HAS_ZW, bool FAST>
 static int launch_kblock128(GemmArgs g, const RequantParams &rq, const DequantParams &dq, hipStream_t stream) {
   g.tiles_m = (g.m + 127) / 128;
   g.tiles_n = (g.n + 127) / 128;
-  if ((g.m & 127) != 0 || (g.n & 127) != 0) g.diag_same_panel = 0;
-  if constexpr (!HAS_ZW && FAST) {
-    if (const int d = diag_kblock128(); d != 0) {
-      auto kern = d == 1   ? gemm_kblock128_diag_kernel<EPI, 1>
-                  : d == 2 ? gemm_kblock128_diag_kernel<EPI, 2>
-                           : gemm_kblock128_diag_kernel<EPI, 3>;
-      hipLaunchKernelGGL(kern, dim3(g.tiles_m * g.tiles_n), dim3(256), 0, stream, g, rq, dq);
-      MI_HIP_CHECK(hipGetLastError());
-      return MI_OK;
-    }
-  }
   hipLaunchKernelGGL((gemm_kblock128_kernel<EPI, HAS_ZW, FAST>), dim3(g.tiles_m * g.tiles_n), dim3(256), 0, stream, g,
                      rq, dq);
   MI_HIP_CHECK(hipGetLastError());
@@ -1234,7 +1183,7 @@ int launch_gemm_requant(const int8_t *a, int64_t lda, int m, int k, const Weight
                         const RequantParams &rq, int8_t *c, int64_t ldc, hipStream_t stream) {
   int rc = check_args(a, lda, m, k, w, n, c, ldc, 4);
   if (rc != MI_OK) return rc;
-  GemmArgs g{a, lda, m, k, w.w, w.ldw, w.k_pad, n, 0, 0, c, ldc, diag_same_panel()};
+  GemmArgs g{a, lda, m, k, w.w, w.ldw, w.k_pad, n, 0, 0, c, ldc};
   DequantParams dq{};
   if (rq.has_zw) {
     return rq.fast2 ? launch_pick_tile<EPI_REQUANT, true, true>(g, rq, dq, stream)
@@ -1291,7 +1240,7 @@ int launch_gemm_conv_requant(const int8_t *in, const ConvGeom &cg, const int8_t 
   ConvGather cv{cg.in_h,     cg.in_w,       cg.in_c,       cg.out_w,  cg.out_h * cg.out_w, cg.kernel_w, cg.stride_h,
                 cg.stride_w, cg.dilation_h, cg.dilation_w, cg.pad_u,  cg.pad_l,            magic(cg.in_c),
                 magic(cg.kernel_w), fill16};
-  GemmArgs g{in, 0, (int)m64, (int)k64, w.w, w.ldw, w.k_pad, cg.out_c, 0, 0, out, cg.out_c, 0};
+  GemmArgs g{in, 0, (int)m64, (int)k64, w.w, w.ldw, w.k_pad, cg.out_c, 0, 0, out, cg.out_c};
   if (rq.has_zw) {
     return rq.fast2 ? launch_conv_pick_tile<true, true>(g, cv, rq, stream)
                     : launch_conv_pick_tile<true, false>(g, cv, rq, stream);
@@ -1304,7 +1253,7 @@ int launch_gemm_dequant(const int8_t *a, int64_t lda, int m, int k, const Weight
                         const DequantParams &dq, float *c, int64_t ldc, hipStream_t stream) {
   int rc = check_args(a, lda, m, k, w, n, c, ldc, 16);
   if (rc != MI_OK) return rc;
-  GemmArgs g{a, lda, m, k, w.w, w.ldw, w.k_pad, n, 0, 0, c, ldc, diag_same_panel()};
+  GemmArgs g{a, lda, m, k, w.w, w.ldw, w.k_pad, n, 0, 0, c, ldc};
   RequantParams rq{};
   // the third parameter (the fast-rounding switch of the int8 epilogue) selects non-temporal stores here
   const bool nt = stream_out_hint((int64_t)m * n * 4);

@@ -14,7 +14,6 @@
 #include "quant_math.h"
 
 #include <algorithm>
-#include <cstdlib>
 #include <type_traits>
 
 
@@ -471,13 +470,11 @@ static int launch_m(const GemvArgs &g, const RequantParams &rq, hipStream_t stre
 // Measured over a decoder layer against fragments fetched from global memory, eight partial reads per output and two
 // channel groups: 8 rows 4.57 -> 4.95 TB/s, 16 rows 3.95 -> 4.58, 32 rows 2.67 -> 3.66.
 // =====================================================================================================================
-// DIAG: timing what-ifs (wrong results, see gemv_diag()): bit 0 = no activation fetches, bit 1 = no barrier before the
-// final sum.
 // DEQ: the fp32 epilogue of the dynamic-quant MatMul (DynamicMatmul4x16x4AIWI,
 // mindspore/ccsrc/plugin/device/cpu/kernel/nnacl/int8/dynamic_matmul_int8.c:99-143) instead of the requantising one:
 // value = sum - zx * sum_k w - zw * sum_k a + K * zx * zw, out = (sx[row] * sw[c]) * (float)value (+ bias) (activation);
 // g.c then points at floats.
-template <int WAVES, int RG, int D, int MR, int DIAG = 0, bool DEQ = false>
+template <int WAVES, int RG, int D, int MR, bool DEQ = false>
 __device__ __forceinline__ void gemv_mfma_lds_body(const GemvArgs &g, int m_rows, const RequantParams &rq,
                                                    const DequantParams &dq, int block) {
   const bool has_zw = DEQ ? dq.zw0 != 0 : rq.has_zw != 0;
@@ -540,10 +537,9 @@ __device__ __forceinline__ void gemv_mfma_lds_body(const GemvArgs &g, int m_rows
   };
 
   // activations first: they return first, and the rows can be in LDS while the weights are still on their way
-  constexpr bool kFetchA = (DIAG & 1) == 0, kMeet = (DIAG & 2) == 0;
   v4i abuf[NLD];
 #pragma unroll
-  for (int i = 0; i < NLD; ++i) abuf[i] = kFetchA ? load_a(0, i) : v4i{lane, 1, 2, 3};
+  for (int i = 0; i < NLD; ++i) abuf[i] = load_a(0, i);
   v4i wbuf[D][RG];
 #pragma unroll
   for (int j = 0; j < D; ++j)
@@ -596,7 +592,7 @@ __device__ __forceinline__ void gemv_mfma_lds_body(const GemvArgs &g, int m_rows
   auto pass = [&](int base, auto refill) {
 #pragma unroll
     for (int i = 0; i < NLD; ++i) store_a(base, i, abuf[i]);
-    if (decltype(refill)::value && kFetchA) {
+    if (decltype(refill)::value) {
 #pragma unroll
       for (int i = 0; i < NLD; ++i) abuf[i] = load_a(base + D, i);
     }
@@ -642,7 +638,7 @@ __device__ __forceinline__ void gemv_mfma_lds_body(const GemvArgs &g, int m_rows
     if (has_zw)
       __hip_atomic_fetch_add(dst + 4 * RG * 64, asum[mg][0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   }
-  if (kMeet) __syncthreads();
+  __syncthreads();
 #pragma unroll
   for (int t = 0; t < NQ; ++t) {
     const int qq = wave + WAVES * t;
@@ -683,14 +679,14 @@ __device__ __forceinline__ void gemv_mfma_lds_body(const GemvArgs &g, int m_rows
   }
 }
 
-template <int WAVES, int RG, int D, int MR, int DIAG = 0>
+template <int WAVES, int RG, int D, int MR>
 __global__ __launch_bounds__(WAVES * 64) void gemv_mfma_lds_kernel(GemvArgs g, int m_rows, RequantParams rq) {
-  gemv_mfma_lds_body<WAVES, RG, D, MR, DIAG, false>(g, m_rows, rq, DequantParams{}, (int)blockIdx.x);
+  gemv_mfma_lds_body<WAVES, RG, D, MR, false>(g, m_rows, rq, DequantParams{}, (int)blockIdx.x);
 }
 
 template <int WAVES, int RG, int D, int MR>
 __global__ __launch_bounds__(WAVES * 64) void gemv_mfma_lds_deq_kernel(GemvArgs g, int m_rows, DequantParams dq) {
-  gemv_mfma_lds_body<WAVES, RG, D, MR, 0, true>(g, m_rows, RequantParams{}, dq, (int)blockIdx.x);
+  gemv_mfma_lds_body<WAVES, RG, D, MR, true>(g, m_rows, RequantParams{}, dq, (int)blockIdx.x);
 }
 
 template <int WAVES, int RG, int D, int MR>
@@ -699,7 +695,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_mfma_lds_group_kernel(GemvGro
   RequantParams rq;
   int block;
   pick_member(grp, (int)blockIdx.x, &g, &rq, &block);
-  gemv_mfma_lds_body<WAVES, RG, D, MR, 0, false>(g, m_rows, rq, DequantParams{}, block);
+  gemv_mfma_lds_body<WAVES, RG, D, MR, false>(g, m_rows, rq, DequantParams{}, block);
 }
 
 template <int WAVES, int RG, int D, int MR>
@@ -708,7 +704,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_mfma_lds_group_deq_kernel(Gem
   DequantParams dq;
   int block;
   pick_member(grp, (int)blockIdx.x, &g, &dq, &block);
-  gemv_mfma_lds_body<WAVES, RG, D, MR, 0, true>(g, m_rows, RequantParams{}, dq, block);
+  gemv_mfma_lds_body<WAVES, RG, D, MR, true>(g, m_rows, RequantParams{}, dq, block);
 }
 
 template <int WAVES, int D, typename F>
@@ -825,30 +821,6 @@ static int launch_mfma_lds_deq(const GemvArgs &g, int m, const DequantParams &dq
   });
 }
 
-// Measurement aid, off unless the environment says MI355X_DIAG_GEMV=1, 2 or 3 when the library is first used: a
-// single-matrix launch with 5..8 activation rows then runs a build of the matrix-core kernel without its activation
-// fetches (1), without the barrier before the final sum (2) or without both (3).  The results are wrong; the launch
-// times show what each of the two costs.
-static int gemv_diag() {
-  static const int v = [] {
-    const char *e = getenv("MI355X_DIAG_GEMV");
-    return e != nullptr ? atoi(e) & 3 : 0;
-  }();
-  return v;
-}
-
-template <int RG, int D>
-static int launch_mfma_lds_diag(const GemvArgs &g, int m, const RequantParams &rq, hipStream_t stream) {
-  const int blocks = (g.n + RG * 16 - 1) / (RG * 16);
-  switch (gemv_diag()) {
-    case 1: hipLaunchKernelGGL((gemv_mfma_lds_kernel<8, RG, D, 8, 1>), dim3(blocks), dim3(512), 0, stream, g, m, rq); break;
-    case 2: hipLaunchKernelGGL((gemv_mfma_lds_kernel<8, RG, D, 8, 2>), dim3(blocks), dim3(512), 0, stream, g, m, rq); break;
-    default: hipLaunchKernelGGL((gemv_mfma_lds_kernel<8, RG, D, 8, 3>), dim3(blocks), dim3(512), 0, stream, g, m, rq); break;
-  }
-  MI_HIP_CHECK(hipGetLastError());
-  return MI_OK;
-}
-
 // Two activation rows run faster on the matrix-core kernel than on the v_dot4 kernel (measured over a decoder layer:
 // 4.78 against 4.67 TB/s) when the handle has the blocked weight copy; without it the v_dot4 kernel takes them.
 static bool prefers_mfma(int m, const WeightView &wv) {
@@ -922,10 +894,6 @@ int launch_gemv_requant(const int8_t *a, int64_t lda, int m, int k, const Weight
     if (m > 64) return launch_mfma_lds_128(g, m, rq, stream);
     if (m > 32) {
       return n >= 8192 && k_pad <= 4096 ? launch_mfma_lds_64<3>(g, m, rq, stream) : launch_mfma_lds_64<1>(g, m, rq, stream);
-    }
-    if (gemv_diag() != 0 && m > 4 && m <= 8) {
-      return n >= 8192 && k_pad <= 4096 ? launch_mfma_lds_diag<3, 4>(g, m, rq, stream)
-                                        : launch_mfma_lds_diag<1, 8>(g, m, rq, stream);
     }
     if (m > 16 && !(n >= 8192 && k_pad <= 4096)) return launch_mfma_lds<8, 1, 4>(g, m, rq, stream);
     if (n >= 8192 && k_pad <= 4096) return launch_mfma_lds<8, 3, 4>(g, m, rq, stream);
