@@ -48,7 +48,9 @@ static int ensure_device() {
     set_error("mi_init has not been called (or found no gfx950 device)");
     return MI_ERROR;
   }
-  MI_HIP_CHECK(hipSetDevice(g_device));
+  // (asking for the thread's device is cheaper than setting it, and it hardly ever is another one)
+  int current = -1;
+  if (hipGetDevice(&current) != hipSuccess || current != g_device) MI_HIP_CHECK(hipSetDevice(g_device));
   return MI_OK;
 }
 

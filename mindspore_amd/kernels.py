@@ -10,7 +10,8 @@ behaviour: construction = Prepare(), ``run`` = Run()):
 
 ``run`` accepts either NumPy arrays (host tensors: copied to the GPU, computed, copied back) or torch CUDA tensors
 (device tensors: computed in place on torch's current stream, no copies).  torch is only used as a device-memory
-and stream provider.
+and stream provider.  A call on device tensors is one call of the native module csrc/device_calls.cc, which checks the
+operand, allocates the output and calls the C ABI; it returns NotImplemented for anything that is not a torch tensor.
 """
 import ctypes as C
 from collections import namedtuple
@@ -21,10 +22,6 @@ from . import lib as _lib
 
 QuantParam = namedtuple("QuantParam", ["scale", "zero_point"])
 ACT_NONE, ACT_RELU, ACT_RELU6 = _lib.ACT_NONE, _lib.ACT_RELU, _lib.ACT_RELU6
-
-
-def _is_torch(x):
-    return type(x).__module__.startswith("torch")
 
 
 def _stream():
@@ -53,9 +50,15 @@ class _Handle:
 
     def __init__(self):
         self._h = C.c_void_p(None)
+        self._raw = 0  # the handle's address, as the native calls take it
+
+    def _created(self):
+        self._raw = self._h.value or 0
+        self._device = _lib.device_calls()
 
     def close(self):
         if getattr(self, "_h", None) is not None and self._h.value:
+            self._raw = 0
             getattr(_lib.load(), self._destroy)(self._h)
             self._h = C.c_void_p(None)
 
@@ -96,23 +99,16 @@ class MatmulInt8Kernel(_Handle):
                             zps, 0 if decode_pack else _lib.MATMUL_NO_DECODE_PACK, self.b_batch)
         _lib.check(L.mi_matmul_create(C.byref(d), weight.ctypes.data, None if bias is None else bias.ctypes.data,
                                       C.byref(self._h)), "mi_matmul_create")
+        self._created()
 
     def run(self, a, out=None):
         """a: int8 [..., K] as a numpy array (host path) or a contiguous CUDA tensor (device path, current stream).
         `out` (device path only) is a preallocated contiguous CUDA int8 tensor [..., N] to write into."""
+        if self._device is not None:
+            y = self._device.matmul_run(self._raw, a, self.n, self.k, out)
+            if y is not NotImplemented:
+                return y
         L = _lib.load()
-        if _is_torch(a):
-            import torch
-            if a.dtype != torch.int8 or not a.is_cuda or not a.is_contiguous() or a.shape[-1] != self.k:
-                raise ValueError("expected a contiguous CUDA int8 tensor [..., %d]" % self.k)
-            rows = a.numel() // self.k
-            if out is None:
-                out = torch.empty(a.shape[:-1] + (self.n,), dtype=torch.int8, device=a.device)
-            elif (out.dtype != torch.int8 or not out.is_cuda or not out.is_contiguous()
-                  or out.numel() != rows * self.n):
-                raise ValueError("out must be a contiguous CUDA int8 tensor with %d elements" % (rows * self.n))
-            _lib.check(L.mi_matmul_run(self._h, a.data_ptr(), rows, out.data_ptr(), _stream()), "mi_matmul_run")
-            return out
         a = _host_i8(a)
         if a.shape[-1] != self.k:
             raise ValueError("expected [..., %d], got %s" % (self.k, a.shape))
@@ -170,18 +166,10 @@ class FullconnectionInt8Kernel(MatmulInt8Kernel):
 def matmul_run_group(kernels, a, outs=None):
     """Runs several MatmulInt8Kernel objects that share the input `a` (a contiguous CUDA int8 tensor [..., K]) as
     mi_matmul_run_group does: decode-sized inputs go out as one launch.  Returns the list of outputs."""
-    import torch
-    L = _lib.load()
-    k = kernels[0].k
-    if a.dtype != torch.int8 or not a.is_cuda or not a.is_contiguous() or a.shape[-1] != k:
-        raise ValueError("expected a contiguous CUDA int8 tensor [..., %d]" % k)
-    rows = a.numel() // k
-    if outs is None:
-        outs = [torch.empty(a.shape[:-1] + (kn.n,), dtype=torch.int8, device=a.device) for kn in kernels]
-    hs = (C.c_void_p * len(kernels))(*[kn._h.value for kn in kernels])
-    cs = (C.c_void_p * len(kernels))(*[o.data_ptr() for o in outs])
-    _lib.check(L.mi_matmul_run_group(hs, len(kernels), a.data_ptr(), rows, cs, _stream()), "mi_matmul_run_group")
-    return outs
+    y = kernels[0]._device.matmul_run_group(kernels, a, kernels[0].k, outs)
+    if y is NotImplemented:
+        raise ValueError("expected a contiguous CUDA int8 tensor [..., %d]" % kernels[0].k)
+    return y
 
 
 def dynmm_run_group(kernels, a, in_quant=None, params_dev=None, row_params=None, outs=None):
@@ -189,26 +177,10 @@ def dynmm_run_group(kernels, a, in_quant=None, params_dev=None, row_params=None,
     as mi_dynmm_run_group does: decode-sized inputs go out as one launch.  The input's quantisation comes as one
     QuantParam (in_quant), as the address of the block a DynamicQuantKernel.run left on the device (params_dev) or as
     the tensor DynamicQuantKernel.run_rows returned (row_params).  Returns the list of fp32 outputs."""
-    import torch
-    L = _lib.load()
-    k = kernels[0].k
-    if a.dtype != torch.int8 or not a.is_cuda or not a.is_contiguous() or a.shape[-1] != k:
-        raise ValueError("expected a contiguous CUDA int8 tensor [..., %d]" % k)
-    rows = a.numel() // k
-    if outs is None:
-        outs = [torch.empty(a.shape[:-1] + (kn.n,), dtype=torch.float32, device=a.device) for kn in kernels]
-    hs = (C.c_void_p * len(kernels))(*[kn._h.value for kn in kernels])
-    cs = (C.c_void_p * len(kernels))(*[o.data_ptr() for o in outs])
-    scale, zp, dev, per_row = 0.0, 0, None, 0
-    if row_params is not None:
-        dev, per_row = row_params.data_ptr(), 1
-    elif params_dev is not None:
-        dev = params_dev
-    else:
-        scale, zp = float(in_quant.scale), int(in_quant.zero_point)
-    _lib.check(L.mi_dynmm_run_group(hs, len(kernels), a.data_ptr(), rows, scale, zp, dev, per_row, cs, _stream()),
-               "mi_dynmm_run_group")
-    return outs
+    y = kernels[0]._device.dynmm_run_group(kernels, a, kernels[0].k, outs, in_quant, params_dev, row_params)
+    if y is NotImplemented:
+        raise ValueError("expected a contiguous CUDA int8 tensor [..., %d]" % kernels[0].k)
+    return y
 
 
 class ConvolutionInt8Kernel(_Handle):
@@ -246,6 +218,7 @@ class ConvolutionInt8Kernel(_Handle):
                           _lib.CONV_3X3_EXACT if exact_3x3 else 0)
         _lib.check(L.mi_conv_create(C.byref(d), weight.ctypes.data, None if bias is None else bias.ctypes.data,
                                     C.byref(self._h)), "mi_conv_create")
+        self._created()
 
     def out_shape(self, in_h, in_w):
         oh, ow = C.c_int32(0), C.c_int32(0)
@@ -255,22 +228,15 @@ class ConvolutionInt8Kernel(_Handle):
     def run(self, x, out=None):
         """x: int8 NHWC as a numpy array (host path) or a contiguous CUDA tensor (device path, current stream);
         `out` (device path only) is a preallocated contiguous CUDA int8 tensor of the output shape."""
+        if self._device is not None:
+            y = self._device.conv_run(self._raw, x, self.ic, self.oc, out)
+            if y is not NotImplemented:
+                return y
         L = _lib.load()
         if x.ndim != 4 or x.shape[3] != self.ic:
             raise ValueError("expected NHWC with %d channels, got %s" % (self.ic, tuple(x.shape)))
         b, ih, iw, _ = x.shape
         oh, ow = self.out_shape(ih, iw)
-        if _is_torch(x):
-            import torch
-            if x.dtype != torch.int8 or not x.is_cuda or not x.is_contiguous():
-                raise ValueError("expected a contiguous CUDA int8 tensor")
-            if out is None:
-                out = torch.empty((b, oh, ow, self.oc), dtype=torch.int8, device=x.device)
-            elif (out.dtype != torch.int8 or not out.is_cuda or not out.is_contiguous()
-                  or out.numel() != b * oh * ow * self.oc):
-                raise ValueError("out must be a contiguous CUDA int8 tensor with %d elements" % (b * oh * ow * self.oc))
-            _lib.check(L.mi_conv_run(self._h, x.data_ptr(), b, ih, iw, out.data_ptr(), _stream()), "mi_conv_run")
-            return out
         x = _host_i8(x)
         out = np.empty((b, oh, ow, self.oc), np.int8)
         _lib.check(L.mi_conv_run_host(self._h, x.ctypes.data, b, ih, iw, out.ctypes.data), "mi_conv_run_host")
@@ -286,28 +252,23 @@ class DynamicQuantKernel(_Handle):
         super().__init__()
         L = _lib.init(device)
         _lib.check(L.mi_dynquant_create(1 if symmetric else 0, C.byref(self._h)), "mi_dynquant_create")
+        self._created()
         self.last = None
 
     def run(self, x, fetch_params=True):
-        L = _lib.load()
         p = _lib.DqParams()
-        if _is_torch(x):
-            import torch
-            if x.dtype != torch.float32 or not x.is_cuda or not x.is_contiguous():
-                raise ValueError("expected a contiguous CUDA float32 tensor")
-            q = torch.empty(x.shape, dtype=torch.int8, device=x.device)
-            s = _stream()
-            _lib.check(L.mi_dynquant_run(self._h, x.data_ptr(), x.numel(), q.data_ptr(), s), "mi_dynquant_run")
-            if not fetch_params:
-                return q, None
-            _lib.check(L.mi_dynquant_get_params(self._h, s, C.byref(p)), "mi_dynquant_get_params")
-        else:
+        q = NotImplemented
+        if self._device is not None:
+            q = self._device.dynquant_run(self._raw, x, C.addressof(p) if fetch_params else 0)
+        if q is NotImplemented:
             x = np.ascontiguousarray(x)
             if x.dtype != np.float32:
                 raise TypeError("DynamicQuant needs a float32 input")  # dynamic_quant.cc:389-395
             q = np.empty(x.shape, np.int8)
-            _lib.check(L.mi_dynquant_run_host(self._h, x.ctypes.data, x.size, q.ctypes.data, C.byref(p)),
+            _lib.check(_lib.load().mi_dynquant_run_host(self._h, x.ctypes.data, x.size, q.ctypes.data, C.byref(p)),
                        "mi_dynquant_run_host")
+        elif not fetch_params:
+            return q, None
         self.last = p
         return q, QuantParam(p.scale, p.zero_point)
 
@@ -319,18 +280,12 @@ class DynamicQuantKernel(_Handle):
         but the last): x [..., K] -> (q, [QuantParam per row]).  numpy in: host path, list of QuantParam out.
         CUDA tensor in: device path, returns (q, params) with params a CUDA uint8 tensor of `rows` parameter
         blocks to hand to MatmulDynamicInt8Kernel.run(..., row_params=params)."""
+        if self._device is not None:
+            both = self._device.dynquant_run_rows(self._raw, x)
+            if both is not NotImplemented:
+                return both
         L = _lib.load()
         unit = x.shape[-1]
-        if _is_torch(x):
-            import torch
-            if x.dtype != torch.float32 or not x.is_cuda or not x.is_contiguous():
-                raise ValueError("expected a contiguous CUDA float32 tensor")
-            rows = x.numel() // unit
-            q = torch.empty(x.shape, dtype=torch.int8, device=x.device)
-            params = torch.empty(rows * C.sizeof(_lib.DqParams), dtype=torch.uint8, device=x.device)
-            _lib.check(L.mi_dynquant_run_segments(self._h, x.data_ptr(), rows, unit, q.data_ptr(), params.data_ptr(),
-                                                  _stream()), "mi_dynquant_run_segments")
-            return q, params
         x = np.ascontiguousarray(x)
         if x.dtype != np.float32:
             raise TypeError("DynamicQuant needs a float32 input")
@@ -380,30 +335,17 @@ class MatmulDynamicInt8Kernel(_Handle):
                            | (0 if decode_pack else _lib.DYNMM_NO_DECODE_PACK), sums)
         _lib.check(L.mi_dynmm_create(C.byref(d), weight.ctypes.data, None if bias is None else bias.ctypes.data,
                                      C.byref(self._h)), "mi_dynmm_create")
+        self._created()
 
     def run(self, a, in_quant=None, params_dev=None, row_params=None):
         """in_quant: one QuantParam (per-tensor input) or a list with one per row (per-channel input; the zero point
         used is the first one, as in the reference).  Device path alternatives: params_dev (address of the block a
         DynamicQuantKernel.run left on the device) or row_params (the tensor DynamicQuantKernel.run_rows returned)."""
+        if self._device is not None:
+            y = self._device.dynmm_run(self._raw, a, self.n, self.k, in_quant, params_dev, row_params)
+            if y is not NotImplemented:
+                return y
         L = _lib.load()
-        if _is_torch(a):
-            import torch
-            if a.dtype != torch.int8 or not a.is_cuda or not a.is_contiguous() or a.shape[-1] != self.k:
-                raise ValueError("expected a contiguous CUDA int8 tensor [..., %d]" % self.k)
-            rows = a.numel() // self.k
-            out = torch.empty(a.shape[:-1] + (self.n,), dtype=torch.float32, device=a.device)
-            if row_params is not None:
-                if row_params.numel() != rows * C.sizeof(_lib.DqParams):
-                    raise ValueError("row_params does not hold %d parameter blocks" % rows)
-                _lib.check(L.mi_dynmm_run_rows(self._h, a.data_ptr(), rows, row_params.data_ptr(), out.data_ptr(),
-                                               _stream()), "mi_dynmm_run_rows")
-            elif params_dev is not None:
-                _lib.check(L.mi_dynmm_run_chained(self._h, a.data_ptr(), rows, params_dev, out.data_ptr(), _stream()),
-                           "mi_dynmm_run_chained")
-            else:
-                _lib.check(L.mi_dynmm_run(self._h, a.data_ptr(), rows, float(in_quant.scale),
-                                          int(in_quant.zero_point), out.data_ptr(), _stream()), "mi_dynmm_run")
-            return out
         a = _host_i8(a)
         rows = a.size // self.k
         out = np.empty(a.shape[:-1] + (self.n,), np.float32)

@@ -26,6 +26,11 @@ EXPORTS = [
 ]
 # libmi355x_diag.so (include/mi355x_diag.h): the benchmark's measurement aids, not part of the product library
 DIAG_LIB_PATH = os.path.join(HERE, "libmi355x_diag.so")
+# the native module behind kernels.py's calls on device tensors (csrc/device_calls.cc)
+DEVICE_CALLS_PATH = os.path.join(HERE, "_device_calls.so")
+DEVICE_CALLS_USES = ["mi_matmul_run", "mi_matmul_run_group", "mi_conv_out_shape", "mi_conv_run", "mi_dynquant_run",
+                     "mi_dynquant_get_params", "mi_dynquant_run_segments", "mi_dynmm_run", "mi_dynmm_run_chained",
+                     "mi_dynmm_run_rows", "mi_dynmm_run_group"]
 DIAG_EXPORTS = ["mi_diag_stream_read", "mi_diag_copy", "mi_diag_mfma_rate"]
 
 
@@ -165,6 +170,27 @@ def load():
     L.mi_stream_destroy.argtypes = [vp]
     _lib = L
     return L
+
+
+_device_calls = None
+
+
+def device_calls():
+    """The native module of the device-tensor calls, or None in a process without torch (no device tensors there)."""
+    global _device_calls
+    if _device_calls is None:
+        try:
+            import torch
+        except ImportError:
+            return None
+        if not os.path.exists(DEVICE_CALLS_PATH):
+            raise RuntimeError("%s is not built: run `python -m mindspore_amd.build`" % DEVICE_CALLS_PATH)
+        from . import _device_calls as module
+        L = load()
+        module.bind({f: C.cast(getattr(L, f), C.c_void_p).value for f in DEVICE_CALLS_USES}, check,
+                    torch.OutOfMemoryError)
+        _device_calls = module
+    return _device_calls
 
 
 _diag = None
