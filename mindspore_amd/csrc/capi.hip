@@ -464,7 +464,7 @@ struct mi_conv {
 
 struct mi_dynquant {
   int symmetric = 0;
-  DevBuf partials, params, h_in, h_out, h_params;
+  DevBuf partials, slots, params, h_in, h_out, h_params;
 };
 
 struct mi_dynmm {
@@ -1141,9 +1141,11 @@ int mi_dynquant_create(int32_t symmetric, mi_dynquant **out) {
   if (h == nullptr) return MI_MEMORY_FAILED;
   h->symmetric = symmetric ? 1 : 0;
   if ((rc = h->partials.ensure(sizeof(float2) * kDqMaxBlocks)) != MI_OK ||
-      (rc = h->params.ensure(sizeof(mi_dq_params))) != MI_OK) {
+      (rc = h->slots.ensure(kDqSlotBytes)) != MI_OK || (rc = h->params.ensure(sizeof(mi_dq_params))) != MI_OK) {
     return rc;
   }
+  MI_HIP_CHECK(hipMemset(h->slots.p, 0xff, kDqSlotBytes));
+  MI_HIP_CHECK(hipStreamSynchronize(nullptr));  // runs may come in on any stream
   *out = owner.release();
   return MI_OK;
 }
@@ -1156,7 +1158,7 @@ int mi_dynquant_run(mi_dynquant *h, const float *x_dev, int64_t n, int8_t *q_dev
   if (n < 0) return MI_PARAM_INVALID;
   int rc = ensure_device();
   if (rc != MI_OK) return rc;
-  return launch_dynquant(x_dev, n, h->symmetric, static_cast<float2 *>(h->partials.p),
+  return launch_dynquant(x_dev, n, h->symmetric, static_cast<float2 *>(h->partials.p), h->slots.p,
                          static_cast<mi_dq_params *>(h->params.p), q_dev, static_cast<hipStream_t>(stream));
 }
 

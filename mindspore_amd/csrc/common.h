@@ -159,8 +159,11 @@ int launch_gemm_conv_requant(const int8_t *in, const ConvGeom &g, const int8_t *
 
 // DynamicQuant: per-block min/max partials, then quantise (every block re-reduces the partials).
 constexpr int kDqMaxBlocks = 1024;
-int launch_dynquant(const float *x, int64_t n, int symmetric, float2 *partials, mi_dq_params *params, int8_t *q,
-                    hipStream_t stream);
+// slots: kDqSlotBytes of device memory, all ones when made, through which the workgroups of the one-launch form meet.
+constexpr int kDqFusedMost = 256;  // workgroups of the one-launch form: one per CU
+constexpr size_t kDqSlotBytes = (2 * sizeof(uint64_t) + sizeof(uint32_t)) * kDqFusedMost;
+int launch_dynquant(const float *x, int64_t n, int symmetric, float2 *partials, void *slots, mi_dq_params *params,
+                    int8_t *q, hipStream_t stream);
 // One {scale, zero point} per contiguous run of `unit` elements; params has `segments` entries.
 int launch_dynquant_segments(const float *x, int64_t segments, int64_t unit, int symmetric, mi_dq_params *params,
                              int8_t *q, hipStream_t stream);

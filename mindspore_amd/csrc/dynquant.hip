@@ -1,16 +1,15 @@
-// DynamicQuant, per tensor: fp32 -> int8 with scale / zero point taken from the tensor's min and max.
-//   pass 1  dq_minmax   : one streaming read; per-lane running min/max with the strict </> updates of
-//                         CalculateMinMaxFp32 (reference mindspore/ccsrc/plugin/device/cpu/kernel/nnacl/int8/
-//                         dynamic_quant_int8.c:19-27; a NaN is never selected), wavefront shuffle reduction, one
-//                         (min, max) partial per workgroup
-//   pass 2  dq_quantize : every workgroup re-reduces the <= 256 partials (2 KiB, L2 resident), derives
-//                         scale / zero point exactly as DynamicQuantCPUKernel::CalculatePerlayerScaleZp does
-//                         (mindspore/lite/src/litert/kernel/cpu/int8/dynamic_quant.cc:156-186: float range, float
-//                         division, zero point in double) and quantises its slice with the arithmetic of
-//                         DoQuantizeFp32ToInt8 (.../nnacl/int8/quant_dtype_cast_int8.c:180-203: float reciprocal,
-//                         float multiply, float add, round half away, clamp).  Workgroup 0 publishes the parameters.
-// The second read of x (12.6 MB for the BERT activation) is served by L2 / Infinity Cache; no atomics, no third
-// launch, results independent of scheduling.
+// DynamicQuant: fp32 -> int8 with scale / zero point taken from the min and max of the tensor, or of each of its rows.
+// Bound by HBM for large tensors (5 bytes per value) and by the latency of one chain -- fetch, reduce, derive the
+// parameters, quantise, store -- for small ones, so a thread requests all its values before it uses the first and
+// keeps them in registers until the parameters are known:
+//   dq_fused    : a tensor in one launch; the workgroups exchange their min and max through memory
+//   dq_rows     : one scale per row, a wave or a workgroup per row (dq_long_rows: rows too long for registers)
+//   dq_minmax + dq_quantize : tensors larger than the registers of the device, two launches and two reads
+// Arithmetic: running min/max with the strict </> updates of CalculateMinMaxFp32 (reference mindspore/ccsrc/plugin/
+// device/cpu/kernel/nnacl/int8/dynamic_quant_int8.c:19-27; a NaN is never selected); scale / zero point exactly as
+// DynamicQuantCPUKernel::CalculatePerlayerScaleZp (mindspore/lite/src/litert/kernel/cpu/int8/dynamic_quant.cc:156-186:
+// float range, float division, zero point in double); DoQuantizeFp32ToInt8 (.../nnacl/int8/
+// quant_dtype_cast_int8.c:180-203: float reciprocal, float multiply, float add, round half away, clamp).
 #include <float.h>
 
 #include "common.h"
@@ -27,14 +26,34 @@ __device__ __forceinline__ void upd(float v, float &lo, float &hi) {
   hi = v > hi ? v : hi;
 }
 
+// Minimum and maximum over the 64 lanes of a wave, in every lane: DPP steps inside each row of 16 lanes (quad_perm
+// [1,0,3,2], quad_perm [2,3,0,1], row_ror:4, row_ror:8), then one lane per row is read back.
+__device__ __forceinline__ void wave_minmax(float &lo, float &hi) {
+#define MI_DPP_STEP(ctrl)                                                                                     \
+  {                                                                                                           \
+    const int l2 = __builtin_amdgcn_update_dpp(__float_as_int(lo), __float_as_int(lo), ctrl, 0xF, 0xF, false); \
+    const int h2 = __builtin_amdgcn_update_dpp(__float_as_int(hi), __float_as_int(hi), ctrl, 0xF, 0xF, false); \
+    lo = __int_as_float(l2) < lo ? __int_as_float(l2) : lo;                                                   \
+    hi = __int_as_float(h2) > hi ? __int_as_float(h2) : hi;                                                   \
+  }
+  MI_DPP_STEP(0xB1)
+  MI_DPP_STEP(0x4E)
+  MI_DPP_STEP(0x124)
+  MI_DPP_STEP(0x128)
+#undef MI_DPP_STEP
+  const float l = lo, h = hi;
+#pragma unroll
+  for (int row = 0; row < 4; ++row) {
+    const float l2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(l), row * 16));
+    const float h2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(h), row * 16));
+    lo = row == 0 || l2 < lo ? l2 : lo;
+    hi = row == 0 || h2 > hi ? h2 : hi;
+  }
+}
+
 template <int THREADS = 256>
 __device__ __forceinline__ void block_minmax(float &lo, float &hi, float *slo, float *shi) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    const float l2 = __shfl_xor(lo, off), h2 = __shfl_xor(hi, off);
-    lo = l2 < lo ? l2 : lo;
-    hi = h2 > hi ? h2 : hi;
-  }
+  wave_minmax(lo, hi);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   if (lane == 0) {
     slo[wave] = lo;
@@ -104,6 +123,30 @@ __device__ __forceinline__ int8_t quant_one(float v, float inv, float zpf) {
   return (int8_t)q;
 }
 
+// Four values -> four bytes.  quant_one in about half the instructions where |t| < 2^20 for all four: adding the
+// largest float below one half, with t's sign, and truncating rounds half away from zero exactly (a sum that should
+// stay below the next integer stays there, t = k + 0.5 ties up to it), and the clamp is one v_med3.  Infinities, NaN
+// and values a broken scale throws out of range have |t| >= 2^20 or t != t and take quant_one.
+__device__ __forceinline__ int quant_four(v4f v, float inv, float zpf) {
+  int q[4];
+  bool rare = false;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float t = __fadd_rn(__fmul_rn(v[e], inv), zpf);
+    rare |= !(__builtin_fabsf(t) < 1048576.0f);
+    const int r = (int)__fadd_rn(t, __builtin_copysignf(0x1.fffffep-2f, t));
+    const int lo = r > -128 ? r : -128;
+    q[e] = lo < 127 ? lo : 127;
+  }
+  if (rare) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) q[e] = quant_one(v[e], inv, zpf);
+  }
+  const uint32_t p01 = __builtin_amdgcn_perm((uint32_t)q[1], (uint32_t)q[0], 0x0c0c0400u);
+  const uint32_t p23 = __builtin_amdgcn_perm((uint32_t)q[3], (uint32_t)q[2], 0x0c0c0400u);
+  return (int)__builtin_amdgcn_perm(p23, p01, 0x05040100u);
+}
+
 // scale and zero point from the tensor's min and max (CalculatePerlayerScaleZp, dynamic_quant.cc:156-186)
 __device__ __forceinline__ void scale_and_zp(float lo, float hi, int symmetric, float *scale_f, int *zp) {
   *zp = 0;
@@ -119,67 +162,154 @@ __device__ __forceinline__ void scale_and_zp(float lo, float hi, int symmetric, 
   }
 }
 
-// Small tensors (a few activation rows: the decode step) in ONE launch of ONE workgroup: every thread keeps its up to
-// 6 groups of four values in registers, the workgroup reduces min and max, derives the parameters and quantises from
-// the registers.  The two-launch form costs such a tensor two launch latencies for a few microseconds of work
-// (1 x 4096 values: 6.3 -> 4.2 us, 2 x 4096: 6.8 -> 4.9, 1 x 11008: 7.4 -> 5.1, 2 x 11008: 7.6 -> 7.0); from about
-// 25 000 values on the arithmetic of a single CU takes longer than the second launch (8 x 4096: 9.0 against 7.5 us).
-constexpr int kDqSingleThreads = 1024;
-constexpr int kDqSingleGroups = 6;  // float4 groups per thread: up to 24576 values
-__global__ __launch_bounds__(kDqSingleThreads) void dq_single_kernel(const float *__restrict__ x, int n, int symmetric,
-                                                                     mi_dq_params *__restrict__ params,
-                                                                     int8_t *__restrict__ q) {
-  __shared__ float slo[kDqSingleThreads / 64], shi[kDqSingleThreads / 64];
-  const int tid = threadIdx.x, n4 = n >> 2;
-  const v4f *x4 = reinterpret_cast<const v4f *>(x);  // (the host checked the alignment)
-  v4f v[kDqSingleGroups];
+// float4 at any float's address (the hardware loads 16 bytes from any 4-byte boundary in one instruction), and the
+// four bytes it becomes, at any byte's address
+typedef v4f v4f_any __attribute__((aligned(4)));
+typedef int int_any __attribute__((aligned(1)));
+
+__device__ __forceinline__ void upd4(v4f v, float &lo, float &hi) {
+  upd(v.x, lo, hi);
+  upd(v.y, lo, hi);
+  upd(v.z, lo, hi);
+  upd(v.w, lo, hi);
+}
+
+__device__ __forceinline__ void publish_params(mi_dq_params *p, float scale_f, int zp, float lo, float hi) {
+  p->scale = (double)scale_f;
+  p->scale_f = scale_f;
+  p->zero_point = zp;
+  p->real_min = lo;
+  p->real_max = hi;
+}
+
+// The whole of DynamicQuant in one launch: a workgroup keeps its share of the tensor (G float4 per thread, all of them
+// requested before the first is used) in registers, publishes its min and max, waits for those of the other
+// workgroups and quantises from the registers.  The tensor crosses HBM once, and a second launch and its re-read are
+// saved for one exchange through memory.
+//
+// The exchange: slot s of the current half holds workgroup s's {min, max}, one 64-bit store that either arrives whole
+// or not at all, so no fence and no atomic read-modify-write (those serialise across the XCDs' separate L2s).  An empty
+// slot is all ones (a minimum is never NaN).  The halves take turns from launch to launch: while one is filled and
+// read, the other, which nobody reads any more, is emptied for the next launch.  Whose turn it is stands in memory as
+// well (a captured launch has no other way to know), one copy per slot; every launch writes all kDqSlots slots --
+// workgroup b takes b, b + W, .. for W workgroups, of which the first W are waited for -- so the copies agree.  Launches
+// on one handle are ordered by their stream.
+//
+// The wait is bounded: workgroups that are not resident together (the device is shared) are not waited for for ever; a
+// workgroup that has waited `patience` ticks of the 100 MHz counter reads the whole tensor itself.
+constexpr int kDqSlots = kDqFusedMost;
+constexpr uint64_t kDqEmpty = ~(uint64_t)0;
+constexpr uint32_t kDqPatience = 20000;  // 200 us
+struct DqSlots {
+  uint64_t range[2][kDqSlots];
+  uint32_t turn[kDqSlots];
+};
+static_assert(sizeof(DqSlots) == kDqSlotBytes, "what the handle allocates and fills with ones");
+
+template <int T, int G>
+__global__ __launch_bounds__(T) void dq_fused_kernel(const float *__restrict__ x, int64_t n, int symmetric,
+                                                     DqSlots *slots, uint32_t patience,
+                                                     mi_dq_params *__restrict__ params, int8_t *__restrict__ q) {
+  __shared__ float slo[T / 64], shi[T / 64], all[2];
+  __shared__ int late_wg;
+  const int tid = threadIdx.x, w = blockIdx.x, wgs = gridDim.x;
+  const int64_t n4 = n >> 2, first = (int64_t)w * (T * G) + tid;
+  const v4f_any *x4 = reinterpret_cast<const v4f_any *>(x);
+  uint32_t turn = 0;
+  if (wgs > 1 && tid < 64) turn = __hip_atomic_load(&slots->turn[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 1;
+  v4f v[G];
   float lo = FLT_MAX, hi = -FLT_MAX;
+  if (n4 > 0) {
 #pragma unroll
-  for (int j = 0; j < kDqSingleGroups; ++j) {
-    const int i = tid + j * kDqSingleThreads;
-    if (i < n4) {
-      v[j] = x4[i];
-      upd(v[j].x, lo, hi);
-      upd(v[j].y, lo, hi);
-      upd(v[j].z, lo, hi);
-      upd(v[j].w, lo, hi);
+    for (int j = 0; j < G; ++j) {  // past the end: the last group again, which changes neither minimum nor maximum
+      const int64_t i = first + j * T;
+      v[j] = __builtin_nontemporal_load(x4 + (i < n4 ? i : n4 - 1));
     }
+#pragma unroll
+    for (int j = 0; j < G; ++j) upd4(v[j], lo, hi);
   }
   float tail = 0.0f;  // the up to three values past the last whole group
-  const int ti = (n4 << 2) + tid;
-  if (ti < n) {
+  const int64_t ti = (n4 << 2) + tid;
+  const bool has_tail = w == 0 && ti < n;
+  if (has_tail) {
     tail = x[ti];
     upd(tail, lo, hi);
   }
-  block_minmax<kDqSingleThreads>(lo, hi, slo, shi);
+  if (wgs == 1) {
+    block_minmax<T>(lo, hi, slo, shi);
+  } else {
+    wave_minmax(lo, hi);
+    if ((tid & 63) == 0) {
+      slo[tid >> 6] = lo;
+      shi[tid >> 6] = hi;
+    }
+    __syncthreads();
+    if (tid < 64) {  // one wave speaks for the workgroup
+#pragma unroll
+      for (int i = 0; i < T / 64; ++i) {
+        lo = slo[i] < lo ? slo[i] : lo;
+        hi = shi[i] > hi ? shi[i] : hi;
+      }
+      const uint64_t mine = (uint64_t)__float_as_uint(hi) << 32 | __float_as_uint(lo);
+      for (int s = w + tid * wgs; s < kDqSlots; s += 64 * wgs) {
+        __hip_atomic_store(&slots->range[turn][s], mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&slots->range[turn ^ 1][s], kDqEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&slots->turn[s], turn ^ 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      const uint64_t began = __builtin_amdgcn_s_memrealtime();
+      bool late = false;
+      uint64_t got[kDqSlots / 64];
+      while (true) {
+        bool missing = false;
+#pragma unroll
+        for (int i = 0; i < kDqSlots / 64; ++i) {
+          const int s = tid + i * 64;
+          got[i] = s < wgs ? __hip_atomic_load(&slots->range[turn][s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : mine;
+        }
+#pragma unroll
+        for (int i = 0; i < kDqSlots / 64; ++i) missing |= got[i] == kDqEmpty;
+        if (!__any(missing)) break;
+        if (__builtin_amdgcn_s_memrealtime() - began > patience) {
+          late = true;
+          break;
+        }
+      }
+      if (!late) {
+#pragma unroll
+        for (int i = 0; i < kDqSlots / 64; ++i) {
+          const float l2 = __uint_as_float((uint32_t)got[i]), h2 = __uint_as_float((uint32_t)(got[i] >> 32));
+          lo = l2 < lo ? l2 : lo;
+          hi = h2 > hi ? h2 : hi;
+        }
+        wave_minmax(lo, hi);
+      }
+      if (tid == 0) {
+        all[0] = lo;
+        all[1] = hi;
+        late_wg = late;
+      }
+    }
+    __syncthreads();
+    lo = all[0];
+    hi = all[1];
+    if (late_wg) {
+      for (int64_t i = tid; i < n4; i += T) upd4(x4[i], lo, hi);
+      if (ti < n) upd(x[ti], lo, hi);
+      block_minmax<T>(lo, hi, slo, shi);
+    }
+  }
   float scale_f;
   int zp;
   scale_and_zp(lo, hi, symmetric, &scale_f, &zp);
-  if (tid == 0) {
-    params->scale = (double)scale_f;
-    params->scale_f = scale_f;
-    params->zero_point = zp;
-    params->real_min = lo;
-    params->real_max = hi;
-  }
+  if (w == 0 && tid == 0) publish_params(params, scale_f, zp, lo, hi);
   const float inv = __fdiv_rn(1.0f, scale_f);
   const float zpf = (float)zp;
 #pragma unroll
-  for (int j = 0; j < kDqSingleGroups; ++j) {
-    const int i = tid + j * kDqSingleThreads;
-    if (i < n4) {
-      union {
-        int w;
-        int8_t b[4];
-      } u;
-      u.b[0] = quant_one(v[j].x, inv, zpf);
-      u.b[1] = quant_one(v[j].y, inv, zpf);
-      u.b[2] = quant_one(v[j].z, inv, zpf);
-      u.b[3] = quant_one(v[j].w, inv, zpf);
-      reinterpret_cast<int *>(q)[i] = u.w;
-    }
+  for (int j = 0; j < G; ++j) {
+    const int64_t i = first + j * T;
+    if (i < n4) *reinterpret_cast<int_any *>(q + 4 * i) = quant_four(v[j], inv, zpf);
   }
-  if (ti < n) q[ti] = quant_one(tail, inv, zpf);
+  if (has_tail) q[ti] = quant_one(tail, inv, zpf);
 }
 
 __global__ __launch_bounds__(kDqThreads) void dq_quantize_kernel(const float *__restrict__ x, int64_t n,
@@ -214,31 +344,17 @@ __global__ __launch_bounds__(kDqThreads) void dq_quantize_kernel(const float *__
   float scale_f;
   int zp;
   scale_and_zp(lo, hi, symmetric, &scale_f, &zp);
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    params->scale = (double)scale_f;
-    params->scale_f = scale_f;
-    params->zero_point = zp;
-    params->real_min = lo;
-    params->real_max = hi;
-  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) publish_params(params, scale_f, zp, lo, hi);
   const float inv = __fdiv_rn(1.0f, scale_f);
   const float zpf = (float)zp;
 
   if (base >= n) return;
   if (fast) {
-    union {
-      int4 v;
-      int8_t b[16];
-    } u;
+    typedef int v4i __attribute__((ext_vector_type(4)));
+    v4i o;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const v4f v = xv[j];
-      u.b[4 * j + 0] = quant_one(v.x, inv, zpf);
-      u.b[4 * j + 1] = quant_one(v.y, inv, zpf);
-      u.b[4 * j + 2] = quant_one(v.z, inv, zpf);
-      u.b[4 * j + 3] = quant_one(v.w, inv, zpf);
-    }
-    *reinterpret_cast<int4 *>(q + base) = u.v;
+    for (int j = 0; j < 4; ++j) o[j] = quant_four(xv[j], inv, zpf);
+    *reinterpret_cast<v4i *>(q + base) = o;
   } else {
     const int64_t end = base + kDqElemsPerThread < n ? base + kDqElemsPerThread : n;
     for (int64_t i = base; i < end; ++i) q[i] = quant_one(x[i], inv, zpf);
@@ -248,96 +364,176 @@ __global__ __launch_bounds__(kDqThreads) void dq_quantize_kernel(const float *__
 // DynamicQuant with preferred axes (one scale / zero point per segment): after the preferred axes lead, the tensor is
 // `segments` contiguous runs of `unit` elements (DynamicQuantCPUKernel::ReSize / CalculateMinMax / QuantData,
 // mindspore/lite/src/litert/kernel/cpu/int8/dynamic_quant.cc:59-94,118-143,236-246; scale and zero point per segment
-// as CalculatePerChannelScaleZp :188-218, the same formulas as the per-tensor case).  One wave per segment: first
-// sweep min/max, second sweep (the run is L1/L2 resident by then) quantises.
-__global__ __launch_bounds__(kDqThreads) void dq_segments_kernel(const float *__restrict__ x, int64_t segments,
-                                                                 int64_t unit, int symmetric,
-                                                                 mi_dq_params *__restrict__ params,
-                                                                 int8_t *__restrict__ q) {
-  const int lane = threadIdx.x & 63;
-  const int64_t seg = (int64_t)blockIdx.x * (kDqThreads / 64) + (threadIdx.x >> 6);
-  if (seg >= segments) return;
+// as CalculatePerChannelScaleZp :188-218, the same formulas as the per-tensor case).  T threads per run keep it in
+// registers, G float4 each, all requested before the first is used: one read of the tensor, and enough of it in
+// flight.  T = 64: a wave per run, four runs per workgroup, no barrier; otherwise a workgroup per run.
+template <int T, int G>
+__global__ __launch_bounds__(T == 64 ? 256 : T) void dq_rows_kernel(const float *__restrict__ x, int64_t segments,
+                                                                    int unit, int symmetric,
+                                                                    mi_dq_params *__restrict__ params,
+                                                                    int8_t *__restrict__ q) {
+  const int tid = T == 64 ? threadIdx.x & 63 : threadIdx.x;
+  const int64_t seg = T == 64 ? (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6) : (int64_t)blockIdx.x;
+  if (seg >= segments) return;  // a whole wave, and a whole workgroup where T > 64
   const float *xs = x + seg * unit;
   int8_t *qs = q + seg * unit;
-  const bool vec = ((reinterpret_cast<uintptr_t>(xs) & 15) == 0) && ((reinterpret_cast<uintptr_t>(qs) & 3) == 0);
-  const int64_t n4 = vec ? unit >> 2 : 0;
+  const int n4 = unit >> 2;
+  const v4f_any *x4 = reinterpret_cast<const v4f_any *>(xs);
+  v4f v[G];
   float lo = FLT_MAX, hi = -FLT_MAX;
-  const v4f *x4 = reinterpret_cast<const v4f *>(xs);
-  for (int64_t i = lane; i < n4; i += 64) {
-    const v4f v = x4[i];
-    upd(v.x, lo, hi);
-    upd(v.y, lo, hi);
-    upd(v.z, lo, hi);
-    upd(v.w, lo, hi);
-  }
-  for (int64_t i = (n4 << 2) + lane; i < unit; i += 64) upd(xs[i], lo, hi);
+  if (n4 > 0) {
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    const float l2 = __shfl_xor(lo, off), h2 = __shfl_xor(hi, off);
-    lo = l2 < lo ? l2 : lo;
-    hi = h2 > hi ? h2 : hi;
+    for (int j = 0; j < G; ++j) {  // past the end: the last group again
+      const int i = tid + j * T;
+      v[j] = __builtin_nontemporal_load(x4 + (i < n4 ? i : n4 - 1));
+    }
+#pragma unroll
+    for (int j = 0; j < G; ++j) upd4(v[j], lo, hi);
+  }
+  float tail = 0.0f;  // the up to three values past the last whole group
+  const int ti = (n4 << 2) + tid;
+  if (ti < unit) {
+    tail = xs[ti];
+    upd(tail, lo, hi);
+  }
+  if constexpr (T == 64) {
+    wave_minmax(lo, hi);
+  } else {
+    __shared__ float slo[T / 64], shi[T / 64];
+    block_minmax<T>(lo, hi, slo, shi);
   }
   float scale_f;
-  double scale_d;
-  int zp = 0;
-  if (!symmetric) {
-    float range = __fsub_rn(hi, lo);
-    if (range <= 0) range = 0.01f;
-    scale_f = __fdiv_rn(range, 255.0f);
-    scale_d = (double)scale_f;
-    zp = double_to_int_x86(round(-128.0 - (double)lo / scale_d));
-  } else {
-    const float a = fabsf(hi), b = fabsf(lo);
-    const float big = (a < b) ? b : a;
-    scale_f = __fdiv_rn(__fmul_rn(2.0f, big), 254.0f);
-    scale_d = (double)scale_f;
-  }
-  if (lane == 0) {
-    mi_dq_params *p = params + seg;
-    p->scale = scale_d;
-    p->scale_f = scale_f;
-    p->zero_point = zp;
-    p->real_min = lo;
-    p->real_max = hi;
-  }
+  int zp;
+  scale_and_zp(lo, hi, symmetric, &scale_f, &zp);
+  if (tid == 0) publish_params(params + seg, scale_f, zp, lo, hi);
   const float inv = __fdiv_rn(1.0f, scale_f);
   const float zpf = (float)zp;
-  for (int64_t i = lane; i < n4; i += 64) {
-    const v4f v = x4[i];
-    union {
-      int w;
-      int8_t b[4];
-    } u;
-    u.b[0] = quant_one(v.x, inv, zpf);
-    u.b[1] = quant_one(v.y, inv, zpf);
-    u.b[2] = quant_one(v.z, inv, zpf);
-    u.b[3] = quant_one(v.w, inv, zpf);
-    *reinterpret_cast<int *>(qs + 4 * i) = u.w;
+#pragma unroll
+  for (int j = 0; j < G; ++j) {
+    const int i = tid + j * T;
+    if (i < n4) *reinterpret_cast<int_any *>(qs + 4 * i) = quant_four(v[j], inv, zpf);
   }
-  for (int64_t i = (n4 << 2) + lane; i < unit; i += 64) qs[i] = quant_one(xs[i], inv, zpf);
+  if (ti < unit) qs[ti] = quant_one(tail, inv, zpf);
+}
+
+// Runs too long for registers: a workgroup per run, two sweeps.
+__global__ __launch_bounds__(1024) void dq_long_rows_kernel(const float *__restrict__ x, int64_t segments, int64_t unit,
+                                                            int symmetric, mi_dq_params *__restrict__ params,
+                                                            int8_t *__restrict__ q) {
+  __shared__ float slo[16], shi[16];
+  const int tid = threadIdx.x;
+  const float *xs = x + (int64_t)blockIdx.x * unit;
+  int8_t *qs = q + (int64_t)blockIdx.x * unit;
+  const int64_t n4 = unit >> 2;
+  const v4f_any *x4 = reinterpret_cast<const v4f_any *>(xs);
+  float lo = FLT_MAX, hi = -FLT_MAX;
+  int64_t i = tid;
+  for (; i + 3 * 1024 < n4; i += 4 * 1024) {
+    v4f v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = x4[i + j * 1024];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) upd4(v[j], lo, hi);
+  }
+  for (; i < n4; i += 1024) upd4(x4[i], lo, hi);
+  const int64_t ti = (n4 << 2) + tid;
+  if (ti < unit) upd(xs[ti], lo, hi);
+  block_minmax<1024>(lo, hi, slo, shi);
+  float scale_f;
+  int zp;
+  scale_and_zp(lo, hi, symmetric, &scale_f, &zp);
+  if (tid == 0) publish_params(params + blockIdx.x, scale_f, zp, lo, hi);
+  const float inv = __fdiv_rn(1.0f, scale_f);
+  const float zpf = (float)zp;
+  for (int64_t k = tid; k < n4; k += 1024) *reinterpret_cast<int_any *>(qs + 4 * k) = quant_four(x4[k], inv, zpf);
+  if (ti < unit) qs[ti] = quant_one(xs[ti], inv, zpf);
+}
+
+template <int T, int G>
+static void launch_rows(const float *x, int64_t segments, int unit, int symmetric, mi_dq_params *params, int8_t *q,
+                        hipStream_t stream) {
+  const int64_t blocks = T == 64 ? (segments + 3) / 4 : segments;
+  hipLaunchKernelGGL((dq_rows_kernel<T, G>), dim3((unsigned)blocks), dim3(T == 64 ? 256 : T), 0, stream, x, segments,
+                     unit, symmetric, params, q);
 }
 
 int launch_dynquant_segments(const float *x, int64_t segments, int64_t unit, int symmetric, mi_dq_params *params,
                              int8_t *q, hipStream_t stream) {
-  const int64_t blocks = (segments + kDqThreads / 64 - 1) / (kDqThreads / 64);
-  if (blocks > 0x7fffffff) {
+  if (segments > 0x7fffffff) {
     set_error("dynquant: too many segments");
     return MI_PARAM_INVALID;
   }
-  hipLaunchKernelGGL(dq_segments_kernel, dim3((unsigned)blocks), dim3(kDqThreads), 0, stream, x, segments, unit,
-                     symmetric, params, q);
+  // A wave per run where there are enough short runs to fill the device with waves; otherwise more threads per run, for
+  // few runs to shorten each thread's chain and for long ones to have 2 to 6 loads of 16 bytes per thread.  us per
+  // launch, before (one wave per run, two sweeps) -> now: 8 x 4096 11.6 -> 2.9, 8 x 11008 28.0 -> 3.6,
+  // 512 x 4096 14.8 -> 4.7, 4096 x 768 6.7 -> 5.2, 2048 x 4096 21.8 -> 9.1 (4.6 TB/s), 2048 x 11008 60.4 -> 20.4
+  // (5.5 TB/s; a copy reaches 5.0).  2048 x 4096 takes 10.8 with a wave and 10.1 with 512 threads per run, 197 x 768
+  // 3.0 with a wave and 2.7 with 256 threads, 4096 x 768 6.6 with 256 threads.
+  const int64_t n4 = unit >> 2;
+#define MI_DQ_ROWS(T, G) launch_rows<T, G>(x, segments, (int)unit, symmetric, params, q, stream)
+  if (n4 <= 64) MI_DQ_ROWS(64, 1);
+  else if (n4 <= 256 && segments >= 512) {
+    if (n4 <= 128) MI_DQ_ROWS(64, 2);
+    else if (n4 <= 192) MI_DQ_ROWS(64, 3);
+    else MI_DQ_ROWS(64, 4);
+  }
+  else if (n4 <= 256) MI_DQ_ROWS(256, 1);
+  else if (n4 <= 1024 && segments >= 256) {
+    if (n4 <= 512) MI_DQ_ROWS(256, 2);
+    else if (n4 <= 768) MI_DQ_ROWS(256, 3);
+    else MI_DQ_ROWS(256, 4);
+  }
+  else if (n4 <= 1024) MI_DQ_ROWS(512, 2);
+  else if (n4 <= 2048) MI_DQ_ROWS(512, 4);
+  else if (n4 <= 3072) MI_DQ_ROWS(512, 6);
+  else if (n4 <= 4096) MI_DQ_ROWS(512, 8);
+  else if (n4 <= 16384) MI_DQ_ROWS(1024, 16);
+  else
+    hipLaunchKernelGGL(dq_long_rows_kernel, dim3((unsigned)segments), dim3(1024), 0, stream, x, segments, unit, symmetric,
+                       params, q);
+#undef MI_DQ_ROWS
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }
 
-int launch_dynquant(const float *x, int64_t n, int symmetric, float2 *partials, mi_dq_params *params, int8_t *q,
-                    hipStream_t stream) {
-  if (n <= (int64_t)kDqSingleThreads * kDqSingleGroups * 4 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
-      (reinterpret_cast<uintptr_t>(q) & 3) == 0) {
-    hipLaunchKernelGGL(dq_single_kernel, dim3(1), dim3(kDqSingleThreads), 0, stream, x, (int)n, symmetric, params, q);
-    MI_HIP_CHECK(hipGetLastError());
-    return MI_OK;
-  }
+template <int T, int G>
+static void launch_fused(const float *x, int64_t n, int symmetric, void *slots, mi_dq_params *params, int8_t *q,
+                         hipStream_t stream) {
+  const int64_t wgs = ((n >> 2) + T * G - 1) / (T * G);
+  hipLaunchKernelGGL((dq_fused_kernel<T, G>), dim3(wgs < 1 ? 1 : (unsigned)wgs), dim3(T), 0, stream, x, n, symmetric,
+                     static_cast<DqSlots *>(slots), kDqPatience, params, q);
+}
+
+int launch_dynquant(const float *x, int64_t n, int symmetric, float2 *partials, void *slots, mi_dq_params *params,
+                    int8_t *q, hipStream_t stream) {
+  // One launch as long as the tensor fits the registers of one workgroup per CU.  Up to 8192 values one workgroup is
+  // faster than any exchange (about 1.2 us); from there on as many workgroups as there are slots, with the fewest
+  // values per thread that allows: what counts at these sizes is the latency of each thread's chain.  us per tensor,
+  // before (up to 24576 values one workgroup, else two launches) -> now: 4096 3.9 -> 2.9, 16384 5.9 -> 3.7,
+  // 32768 7.2 -> 4.2, 88064 7.4 -> 4.4, 300000 7.7 -> 5.0, 1 M 8.0 -> 5.6, 4096 x 768 11.3 -> 8.9,
+  // 2048 x 4096 20.0 -> 13.5, 4096 x 3072 26.9 -> 17.5, 2048 x 11008 40.8 -> 26.7.
+  const int64_t n4 = n >> 2;
+#define MI_DQ_FUSED(T, G)                                                   \
+  do {                                                                      \
+    launch_fused<T, G>(x, n, symmetric, slots, params, q, stream);          \
+    MI_HIP_CHECK(hipGetLastError());                                        \
+    return MI_OK;                                                           \
+  } while (0)
+  constexpr int64_t kMost = kDqFusedMost;
+  if (n4 <= 256) MI_DQ_FUSED(256, 1);
+  if (n4 <= 512 * 2) MI_DQ_FUSED(512, 2);
+  if (n4 <= 512 * 4) MI_DQ_FUSED(512, 4);
+  if (n4 <= kMost * 256) MI_DQ_FUSED(256, 1);
+  if (n4 <= kMost * 512) MI_DQ_FUSED(512, 1);
+  if (n4 <= kMost * 256 * 4) MI_DQ_FUSED(256, 4);
+  if (n4 <= kMost * 512 * 4) MI_DQ_FUSED(512, 4);
+  if (n4 <= kMost * 1024 * 3) MI_DQ_FUSED(1024, 3);
+  if (n4 <= kMost * 1024 * 6) MI_DQ_FUSED(1024, 6);
+  if (n4 <= kMost * 1024 * 8) MI_DQ_FUSED(1024, 8);
+  if (n4 <= kMost * 1024 * 12) MI_DQ_FUSED(1024, 12);
+  if (n4 <= kMost * 1024 * 16) MI_DQ_FUSED(1024, 16);
+  if (n4 <= kMost * 1024 * 24) MI_DQ_FUSED(1024, 24);
+#undef MI_DQ_FUSED
   const int64_t per_block = (int64_t)kDqThreads * kDqElemsPerThread;
   int64_t want = (n + per_block - 1) / per_block;
   // pass 1: at most one workgroup per partial a thread of pass 2 reads in a single step

@@ -1,0 +1,60 @@
+"""Sizes at the edges of the rules by which the library picks a kernel: the last size of one variant and the first of
+the next, remainders, misaligned operands.  Full-tensor, bit-exact comparisons with the oracle."""
+import numpy as np
+import pytest
+
+from mindspore_amd import kernels as K
+
+pytestmark = pytest.mark.gpu
+
+
+def _values(rng, n):
+    x = rng.standard_normal(n, dtype=np.float32)
+    x[rng.integers(0, n, max(1, n // 100))] *= 50
+    return x
+
+
+@pytest.mark.parametrize("symmetric", [False, True])
+@pytest.mark.parametrize("n", [1, 3, 4, 1023, 1024, 1027, 1028, 4096, 4100, 8195, 8196, 262144, 262147, 262148, 524288,
+                               524292, 1048579, 1048580, 2097155, 2097156, 3145731, 3145732, 6291460, 8388612,
+                               12582916, 16777220, 25165827, 25165828])
+def test_dynamic_quant_one_launch_sizes(orc, n, symmetric):
+    import torch
+    rng = np.random.default_rng(n)
+    x = _values(rng, n + 1)
+    dev = torch.from_numpy(x).cuda()
+    dq = K.DynamicQuantKernel(symmetric)
+    for lead in (0, 1):  # 1: the tensor starts 4 bytes past a 16-byte boundary
+        for repeat in range(2):  # the exchange between workgroups alternates between two halves of its slots
+            q, p = dq.run(dev[lead:lead + n])
+            want, scale, zp = orc.dynamic_quant(x[lead:lead + n], symmetric)
+            assert np.array_equal(q.cpu().numpy(), want) and (p.scale, p.zero_point) == (scale, zp), (n, lead, repeat)
+
+
+@pytest.mark.parametrize("special", [np.nan, np.inf, -np.inf, 0.0])
+@pytest.mark.parametrize("n", [5, 40000, 3000001])
+def test_dynamic_quant_one_launch_special_values(orc, n, special):
+    import torch
+    x = _values(np.random.default_rng(n), n)
+    for where in ([0], [n - 1], list(range(n))):
+        y = x.copy()
+        y[where] = special
+        dq = K.DynamicQuantKernel(False)
+        q, p = dq.run(torch.from_numpy(y).cuda())
+        want, scale, zp = orc.dynamic_quant(y)
+        assert np.array_equal(q.cpu().numpy(), want), (n, special, where[:2])
+        assert np.array_equal([p.scale], [scale], equal_nan=True) and p.zero_point == zp
+
+
+@pytest.mark.parametrize("rows,unit", [(1, 1), (3, 255), (511, 259), (512, 259), (512, 260), (600, 515), (513, 771), (700, 1027),
+                                       (255, 1028), (256, 1028), (300, 2051), (257, 3075), (256, 4099), (20, 4100), (7, 8195),
+                                       (5, 8196), (3, 12292), (2, 16387), (2, 16388), (2, 65539), (2, 65540)])
+def test_dynamic_quant_row_sizes(orc, rows, unit):
+    import torch
+    x = _values(np.random.default_rng(rows * unit), rows * unit).reshape(rows, unit)
+    dq = K.DynamicQuantKernel(True)
+    q, params = dq.run_rows(torch.from_numpy(x).cuda())
+    want, scales, zps = orc.dynamic_quant_segments(x, True)
+    got = params.cpu().numpy().view([("scale", "f8"), ("scale_f", "f4"), ("zp", "i4"), ("lo", "f4"), ("hi", "f4")])
+    assert np.array_equal(q.cpu().numpy(), want)
+    assert np.array_equal(got["scale"], scales) and np.array_equal(got["zp"], zps)
