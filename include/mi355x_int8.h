@@ -240,6 +240,9 @@ int mi_dynquant_create(int32_t symmetric, mi_dynquant **out);
 int mi_dynquant_run(mi_dynquant *h, const float *x_dev, int64_t n, int8_t *q_dev, void *stream);
 /* Waits for the last run on `stream` and returns its parameters (what the provider writes with SetQuantParams). */
 int mi_dynquant_get_params(mi_dynquant *h, void *stream, mi_dq_params *params_host);
+/* The same for callers that go on working on `stream`: returns as soon as the parameters are known, when the last
+ * values of q_dev may still be on their way (they are complete for everything that is ordered behind the run). */
+int mi_dynquant_await_params(mi_dynquant *h, void *stream, mi_dq_params *params_host);
 /* Device address of the mi_dq_params block of the last run. */
 const mi_dq_params *mi_dynquant_device_params(const mi_dynquant *h);
 int mi_dynquant_run_host(mi_dynquant *h, const float *x_host, int64_t n, int8_t *q_host, mi_dq_params *params_host);

@@ -162,8 +162,15 @@ constexpr int kDqMaxBlocks = 1024;
 // slots: kDqSlotBytes of device memory, all ones when made, through which the workgroups of the one-launch form meet.
 constexpr int kDqFusedMost = 256;  // workgroups of the one-launch form: one per CU
 constexpr size_t kDqSlotBytes = (2 * sizeof(uint64_t) + sizeof(uint32_t)) * kDqFusedMost;
-int launch_dynquant(const float *x, int64_t n, int symmetric, float2 *partials, void *slots, mi_dq_params *params,
-                    int8_t *q, hipStream_t stream);
+// Page-locked host memory into which a run whose ticket is not 0 also writes {scale, zero point, min, max} as float /
+// int32 bits in the low halves of kDqHostWords words, with the ticket in the high halves.
+constexpr int kDqHostWords = 4;
+struct DqHostNote {
+  uint64_t *words;
+  uint32_t ticket;
+};
+int launch_dynquant(const float *x, int64_t n, int symmetric, float2 *partials, void *slots, const DqHostNote &note,
+                    mi_dq_params *params, int8_t *q, hipStream_t stream);
 // One {scale, zero point} per contiguous run of `unit` elements; params has `segments` entries.
 int launch_dynquant_segments(const float *x, int64_t segments, int64_t unit, int symmetric, mi_dq_params *params,
                              int8_t *q, hipStream_t stream);

@@ -22,7 +22,7 @@ struct Api {
   decltype(&mi_conv_out_shape) conv_out_shape;
   decltype(&mi_conv_run) conv_run;
   decltype(&mi_dynquant_run) dynquant_run;
-  decltype(&mi_dynquant_get_params) dynquant_get_params;
+  decltype(&mi_dynquant_await_params) dynquant_await_params;
   decltype(&mi_dynquant_run_segments) dynquant_run_segments;
   decltype(&mi_dynmm_run) dynmm_run;
   decltype(&mi_dynmm_run_chained) dynmm_run_chained;
@@ -123,7 +123,7 @@ PyObject *bind(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   PyObject *d = args[0];
   if (!take(d, "mi_matmul_run", &api.matmul_run) || !take(d, "mi_matmul_run_group", &api.matmul_run_group) ||
       !take(d, "mi_conv_out_shape", &api.conv_out_shape) || !take(d, "mi_conv_run", &api.conv_run) ||
-      !take(d, "mi_dynquant_run", &api.dynquant_run) || !take(d, "mi_dynquant_get_params", &api.dynquant_get_params) ||
+      !take(d, "mi_dynquant_run", &api.dynquant_run) || !take(d, "mi_dynquant_await_params", &api.dynquant_await_params) ||
       !take(d, "mi_dynquant_run_segments", &api.dynquant_run_segments) || !take(d, "mi_dynmm_run", &api.dynmm_run) ||
       !take(d, "mi_dynmm_run_chained", &api.dynmm_run_chained) || !take(d, "mi_dynmm_run_rows", &api.dynmm_run_rows) ||
       !take(d, "mi_dynmm_run_group", &api.dynmm_run_group))
@@ -375,8 +375,8 @@ PyObject *conv_run(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   });
 }
 
-// dynquant_run(handle, x, address of a host parameter block or 0) -> int8 tensor; with an address the call waits for
-// the run and fills the block
+// dynquant_run(handle, x, address of a host parameter block or 0) -> int8 tensor; with an address the call waits
+// until the parameters of the run are known and fills the block
 PyObject *dynquant_run(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   if (!count_args(nargs, 3)) return nullptr;
   if (!THPVariable_Check(args[1])) Py_RETURN_NOTIMPLEMENTED;
@@ -392,8 +392,8 @@ PyObject *dynquant_run(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     mi_dynquant *dq = static_cast<mi_dynquant *>(h);
     void *s = stream();
     if (!call_library("mi_dynquant_run", [&] { return api.dynquant_run(dq, xp, n, qp, s); })) return nullptr;
-    if (host != nullptr && !call_library("mi_dynquant_get_params", [&] {
-          return api.dynquant_get_params(dq, s, static_cast<mi_dq_params *>(host));
+    if (host != nullptr && !call_library("mi_dynquant_await_params", [&] {
+          return api.dynquant_await_params(dq, s, static_cast<mi_dq_params *>(host));
         }))
       return nullptr;
     return THPVariable_Wrap(std::move(q));

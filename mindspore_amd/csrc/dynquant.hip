@@ -182,6 +182,16 @@ __device__ __forceinline__ void publish_params(mi_dq_params *p, float scale_f, i
   p->real_max = hi;
 }
 
+// The same to the host that is waiting for them, if one is: each word carries the run's ticket beside its value, so the
+// stores need no order among themselves, and they leave before the quantising starts.
+__device__ __forceinline__ void publish_to_host(const DqHostNote &note, float scale_f, int zp, float lo, float hi) {
+  if (note.ticket == 0) return;
+  const uint32_t v[kDqHostWords] = {__float_as_uint(scale_f), (uint32_t)zp, __float_as_uint(lo), __float_as_uint(hi)};
+#pragma unroll
+  for (int i = 0; i < kDqHostWords; ++i)
+    __hip_atomic_store(note.words + i, (uint64_t)note.ticket << 32 | v[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // The whole of DynamicQuant in one launch: a workgroup keeps its share of the tensor (G float4 per thread, all of them
 // requested before the first is used) in registers, publishes its min and max, waits for those of the other
 // workgroups and quantises from the registers.  The tensor crosses HBM once, and a second launch and its re-read are
@@ -208,7 +218,7 @@ static_assert(sizeof(DqSlots) == kDqSlotBytes, "what the handle allocates and fi
 
 template <int T, int G>
 __global__ __launch_bounds__(T) void dq_fused_kernel(const float *__restrict__ x, int64_t n, int symmetric,
-                                                     DqSlots *slots, uint32_t patience,
+                                                     DqSlots *slots, uint32_t patience, DqHostNote note,
                                                      mi_dq_params *__restrict__ params, int8_t *__restrict__ q) {
   __shared__ float slo[T / 64], shi[T / 64], all[2];
   __shared__ int late_wg;
@@ -301,7 +311,10 @@ __global__ __launch_bounds__(T) void dq_fused_kernel(const float *__restrict__ x
   float scale_f;
   int zp;
   scale_and_zp(lo, hi, symmetric, &scale_f, &zp);
-  if (w == 0 && tid == 0) publish_params(params, scale_f, zp, lo, hi);
+  if (w == 0 && tid == 0) {
+    publish_to_host(note, scale_f, zp, lo, hi);
+    publish_params(params, scale_f, zp, lo, hi);
+  }
   const float inv = __fdiv_rn(1.0f, scale_f);
   const float zpf = (float)zp;
 #pragma unroll
@@ -314,7 +327,7 @@ __global__ __launch_bounds__(T) void dq_fused_kernel(const float *__restrict__ x
 
 __global__ __launch_bounds__(kDqThreads) void dq_quantize_kernel(const float *__restrict__ x, int64_t n,
                                                                  int symmetric,
-                                                                 const float2 *__restrict__ partials, int nparts,
+                                                                 const float2 *__restrict__ partials, int nparts, DqHostNote note,
                                                                  mi_dq_params *__restrict__ params,
                                                                  int8_t *__restrict__ q) {
   __shared__ float slo[kDqThreads / 64], shi[kDqThreads / 64];
@@ -344,7 +357,10 @@ __global__ __launch_bounds__(kDqThreads) void dq_quantize_kernel(const float *__
   float scale_f;
   int zp;
   scale_and_zp(lo, hi, symmetric, &scale_f, &zp);
-  if (blockIdx.x == 0 && threadIdx.x == 0) publish_params(params, scale_f, zp, lo, hi);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    publish_to_host(note, scale_f, zp, lo, hi);
+    publish_params(params, scale_f, zp, lo, hi);
+  }
   const float inv = __fdiv_rn(1.0f, scale_f);
   const float zpf = (float)zp;
 
@@ -497,15 +513,15 @@ int launch_dynquant_segments(const float *x, int64_t segments, int64_t unit, int
 }
 
 template <int T, int G>
-static void launch_fused(const float *x, int64_t n, int symmetric, void *slots, mi_dq_params *params, int8_t *q,
-                         hipStream_t stream) {
+static void launch_fused(const float *x, int64_t n, int symmetric, void *slots, const DqHostNote &note,
+                         mi_dq_params *params, int8_t *q, hipStream_t stream) {
   const int64_t wgs = ((n >> 2) + T * G - 1) / (T * G);
   hipLaunchKernelGGL((dq_fused_kernel<T, G>), dim3(wgs < 1 ? 1 : (unsigned)wgs), dim3(T), 0, stream, x, n, symmetric,
-                     static_cast<DqSlots *>(slots), kDqPatience, params, q);
+                     static_cast<DqSlots *>(slots), kDqPatience, note, params, q);
 }
 
-int launch_dynquant(const float *x, int64_t n, int symmetric, float2 *partials, void *slots, mi_dq_params *params,
-                    int8_t *q, hipStream_t stream) {
+int launch_dynquant(const float *x, int64_t n, int symmetric, float2 *partials, void *slots, const DqHostNote &note,
+                    mi_dq_params *params, int8_t *q, hipStream_t stream) {
   // One launch as long as the tensor fits the registers of one workgroup per CU.  Up to 8192 values one workgroup is
   // faster than any exchange (about 1.2 us); from there on as many workgroups as there are slots, with the fewest
   // values per thread that allows: what counts at these sizes is the latency of each thread's chain.  us per tensor,
@@ -515,7 +531,7 @@ int launch_dynquant(const float *x, int64_t n, int symmetric, float2 *partials, 
   const int64_t n4 = n >> 2;
 #define MI_DQ_FUSED(T, G)                                                   \
   do {                                                                      \
-    launch_fused<T, G>(x, n, symmetric, slots, params, q, stream);          \
+    launch_fused<T, G>(x, n, symmetric, slots, note, params, q, stream);    \
     MI_HIP_CHECK(hipGetLastError());                                        \
     return MI_OK;                                                           \
   } while (0)
@@ -547,7 +563,7 @@ int launch_dynquant(const float *x, int64_t n, int symmetric, float2 *partials, 
     return MI_PARAM_INVALID;
   }
   hipLaunchKernelGGL(dq_quantize_kernel, dim3((unsigned)qblocks), dim3(kDqThreads), 0, stream, x, n, symmetric,
-                     partials, nparts, params, q);
+                     partials, nparts, note, params, q);
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }

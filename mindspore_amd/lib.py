@@ -16,7 +16,7 @@ EXPORTS = [
     "mi_multiply_by_quantized_multiplier",
     "mi_matmul_create", "mi_matmul_reserve", "mi_matmul_run", "mi_matmul_run_noalloc", "mi_matmul_run_host", "mi_matmul_run_group", "mi_matmul_run_batched", "mi_matmul_broadcast_offsets", "mi_matmul_get_params", "mi_matmul_destroy",
     "mi_conv_create", "mi_conv_out_shape", "mi_conv_same_pad", "mi_conv_run", "mi_conv_run_host", "mi_conv_reserve", "mi_conv_destroy",
-    "mi_dynquant_create", "mi_dynquant_run", "mi_dynquant_get_params", "mi_dynquant_device_params",
+    "mi_dynquant_create", "mi_dynquant_run", "mi_dynquant_get_params", "mi_dynquant_await_params", "mi_dynquant_device_params",
     "mi_dynquant_run_host", "mi_dynquant_run_segments", "mi_dynquant_run_segments_host", "mi_dynquant_destroy",
     "mi_unpack_weight_4x16", "mi_dynmm_create", "mi_dynmm_run", "mi_dynmm_run_chained", "mi_dynmm_run_host", "mi_dynmm_run_rows", "mi_dynmm_run_group", "mi_dynmm_run_rows_host", "mi_dynmm_reserve",
     "mi_dynmm_destroy",
@@ -29,7 +29,7 @@ DIAG_LIB_PATH = os.path.join(HERE, "libmi355x_diag.so")
 # the native module behind kernels.py's calls on device tensors (csrc/device_calls.cc)
 DEVICE_CALLS_PATH = os.path.join(HERE, "_device_calls.so")
 DEVICE_CALLS_USES = ["mi_matmul_run", "mi_matmul_run_group", "mi_conv_out_shape", "mi_conv_run", "mi_dynquant_run",
-                     "mi_dynquant_get_params", "mi_dynquant_run_segments", "mi_dynmm_run", "mi_dynmm_run_chained",
+                     "mi_dynquant_await_params", "mi_dynquant_run_segments", "mi_dynmm_run", "mi_dynmm_run_chained",
                      "mi_dynmm_run_rows", "mi_dynmm_run_group"]
 DIAG_EXPORTS = ["mi_diag_stream_read", "mi_diag_copy", "mi_diag_mfma_rate"]
 
@@ -136,6 +136,7 @@ def load():
     L.mi_dynquant_create.argtypes = [i32, C.POINTER(vp)]
     L.mi_dynquant_run.argtypes = [vp, vp, i64, vp, vp]
     L.mi_dynquant_get_params.argtypes = [vp, vp, C.POINTER(DqParams)]
+    L.mi_dynquant_await_params.argtypes = [vp, vp, C.POINTER(DqParams)]
     L.mi_dynquant_device_params.argtypes = [vp]
     L.mi_dynquant_device_params.restype = vp
     L.mi_dynquant_run_host.argtypes = [vp, vp, i64, vp, C.POINTER(DqParams)]

@@ -58,3 +58,35 @@ def test_dynamic_quant_row_sizes(orc, rows, unit):
     got = params.cpu().numpy().view([("scale", "f8"), ("scale_f", "f4"), ("zp", "i4"), ("lo", "f4"), ("hi", "f4")])
     assert np.array_equal(q.cpu().numpy(), want)
     assert np.array_equal(got["scale"], scales) and np.array_equal(got["zp"], zps)
+
+
+def test_dynamic_quant_parameters_follow_their_run(orc):
+    """Parameters fetched run after run, after runs whose parameters nobody asked for, and from a stream that is being
+    replayed as a graph: always those of the last run."""
+    import torch
+    rng = np.random.default_rng(3)
+    xs = [_values(rng, n) * s for n, s in ((5000, 1.0), (40000, 3.0), (200000, 0.2), (26000000, 2.0), (700, 9.0))]
+    devs = [torch.from_numpy(x).cuda() for x in xs]
+    want = [orc.dynamic_quant(x)[1:] for x in xs]
+    dq = K.DynamicQuantKernel(False)
+    for fetch in (1, 1, 0, 1, 0, 0, 1, 1):
+        for x, w in zip(devs, want):
+            q, p = dq.run(x, fetch_params=bool(fetch))
+            assert not fetch or (p.scale, p.zero_point) == w
+    lib, p = K._lib, K._lib.DqParams()
+    L = lib.load()
+    side = torch.cuda.Stream()
+    x = torch.empty_like(devs[1])
+    with torch.cuda.stream(side):
+        x.copy_(devs[1])
+        dq.run(x)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            dq.run(x, fetch_params=False)
+        for scale in (1.0, 2.0, 0.5, 4.0):
+            x.copy_(devs[1] * scale)
+            graph.replay()
+            for fetch in (L.mi_dynquant_get_params, L.mi_dynquant_await_params):
+                assert fetch(dq._h, side.cuda_stream, p) == lib.MI_OK
+                assert (p.scale, p.zero_point) == orc.dynamic_quant(xs[1] * np.float32(scale))[1:]
+        dq.run(devs[0])
