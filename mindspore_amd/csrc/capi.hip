@@ -460,6 +460,7 @@ struct mi_conv {
   int fill = 0;
   RequantState st;
   DevBuf w16, dw_bias, dw_bias_folded, col_ws, c_ws, h_in, h_out;
+  DevBuf w_rows;  // the weights of a convolution on few channels as launch_conv_rows takes them, or empty
   DevBuf fill16;  // 16 bytes of `fill`: where the gathering GEMM loader reads taps outside the image
 };
 
@@ -1028,6 +1029,9 @@ static int mi_conv_create_impl(const mi_conv_desc *d, const int8_t *weight_host,
     h->fill = is_1x1 ? 0 : d->in_zp;
     rc = h->st.build(weight_host, oc, kdim, bias_host, d->in_scale, d->in_zp, d->out_scale, d->out_zp,
                      d->filter_quant_num, d->filter_scales, d->filter_zps, d->act_type, true);
+    if (rc == MI_OK && conv_rows_supported(ConvGeom{1, 16, 16, d->in_channel, 1, 1, oc, d->kernel_h, d->kernel_w, d->stride_h,
+                                                    d->stride_w, d->dilation_h, d->dilation_w, d->pad_u, d->pad_l}))
+      rc = upload(&h->w_rows, conv_rows_weights(weight_host, oc, d->kernel_h, d->kernel_w, d->in_channel));
     if (rc == MI_OK) rc = upload(&h->fill16, std::vector<int8_t>(16, (int8_t)h->fill));
   }
   if (rc != MI_OK) {
@@ -1102,15 +1106,18 @@ int mi_conv_run(mi_conv *h, const int8_t *in_dev, int32_t batch, int32_t in_h, i
   int k16 = 0;
   if (h->direct_1x1) {
     if ((rc = prepare_rows(in_dev, (int)pixels, k, Workspace::growable(&h->col_ws), s, &a, &lda, &k16)) != MI_OK) return rc;
-  } else if (k <= 64 && d.out_channel <= 128 && (d.out_channel & 3) == 0 &&
-             (reinterpret_cast<uintptr_t>(out_dev) & 3) == 0) {
-    // a first-layer convolution: gathered straight from the image, no im2col buffer
-    return launch_conv_smallk(in_dev, g, h->fill, k, static_cast<const int8_t *>(h->st.w.p), h->st.ldw, h->st.params(),
-                              out_dev, s);
-  } else if (pixels > 128 && gemm_conv_supported(g, in_dev, out_dev)) {
-    // 16-channel-aligned images: the GEMM gathers its activation operand from the image, no im2col buffer
+  } else if (h->w_rows.p != nullptr && conv_rows_supported(g)) {
+    // a first-layer convolution: window rows straight from the image
+    return launch_conv_rows(in_dev, g, h->fill, static_cast<const int8_t *>(h->w_rows.p), h->st.params(), out_dev, s);
+  } else if ((pixels > 128 || k <= 64) && gemm_conv_supported(g, in_dev, out_dev)) {
+    // 16-channel-aligned images: the GEMM gathers its activation operand from the image, no im2col buffer (with few
+    // pixels the buffer is small and the decode kernel streams the weights faster, unless there are next to none)
     WeightView w{static_cast<const int8_t *>(h->st.w.p), h->st.k_pad, h->st.ldw, nullptr};
     return launch_gemm_conv_requant(in_dev, g, static_cast<const int8_t *>(h->fill16.p), w, h->st.params(), out_dev, s);
+  } else if (k <= 64 && d.out_channel <= 128 && (d.out_channel & 3) == 0 &&
+             (reinterpret_cast<uintptr_t>(out_dev) & 3) == 0) {
+    return launch_conv_smallk(in_dev, g, h->fill, k, static_cast<const int8_t *>(h->st.w.p), h->st.ldw, h->st.params(),
+                              out_dev, s);
   } else {
     k16 = round_up(k, 16);
     if ((rc = h->col_ws.ensure((size_t)pixels * k16)) != MI_OK) return rc;

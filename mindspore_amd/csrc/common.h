@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <vector>
+
 #include "../../include/mi355x_int8.h"
 
 namespace mi {
@@ -145,6 +147,13 @@ int launch_im2col(const int8_t *in, const ConvGeom &g, int fill, int8_t *dst, in
 // (no im2col buffer); w: packed row-major weights with row stride ldw, K order (kh, kw, ic).
 int launch_conv_smallk(const int8_t *in, const ConvGeom &g, int fill, int k_true, const int8_t *w, int ldw,
                        const RequantParams &rq, int8_t *out, hipStream_t stream);
+// Dense convolution on few input channels (in_c % 16 != 0, kernel_w * in_c <= 32, dilation_w 1), straight from the image
+// with 16-byte loads; w: the weights as conv_rows_weights lays them out, in device memory.
+constexpr int kConvRowsSteps = 8;  // at most this many 32-byte contraction steps
+bool conv_rows_supported(const ConvGeom &g);
+std::vector<int8_t> conv_rows_weights(const int8_t *w, int oc, int kernel_h, int kernel_w, int in_c);
+int launch_conv_rows(const int8_t *in, const ConvGeom &g, int fill, const int8_t *w, const RequantParams &rq, int8_t *out,
+                     hipStream_t stream);
 // Depthwise conv + requantisation, weights pre-offset to int16 [KH*KW][C].  bias_folded = bias - zx8 * sum_t w16[t][c]
 // (used by the channel-vectorised kernel, which reads out-of-image taps as zx8); rq.fast: the host proved the cheap
 // rounding form exact for every channel.

@@ -8,9 +8,12 @@
 //              convolution_1x1_int8.cc:396)
 //   conv_dw  : depthwise conv + requantisation (ConvDwInt8 / ConvDwInt8Post,
 //              .../nnacl/int8/conv_depthwise_int8.c:24-140)
-//   conv_smallk : dense convolution with kernel_h * kernel_w * in_c <= 64 in one launch, gathered from the image
+//   conv_rows : first-layer convolutions (few input channels) in one launch, window rows straight from the image
+//   conv_smallk : what is left with kernel_h * kernel_w * in_c <= 64 in one launch, gathered byte by byte
 // The first three are HBM/latency bound byte movers: one thread produces 16 contiguous output bytes (or one output
 // element for the depthwise kernel, consecutive threads on consecutive channels) so stores coalesce.
+#include <string.h>
+
 #include "common.h"
 #include "quant_math.h"
 
@@ -123,8 +126,8 @@ int launch_im2col(const int8_t *in, const ConvGeom &g, int fill, int8_t *dst, in
   return MI_OK;
 }
 
-// Dense convolution with a short contraction (kernel_h * kernel_w * in_c <= 64, the first layer of an image network:
-// 3x3 on 3 channels is K = 27) without an im2col buffer and its extra launch.  One wave produces 32 output pixels x
+// Dense convolution with a short contraction (kernel_h * kernel_w * in_c <= 64) that neither conv_rows_kernel nor the
+// gathering GEMM takes, without an im2col buffer and its extra launch.  One wave produces 32 output pixels x
 // all output channels with v_mfma_i32_32x32x32_i8: lane (r, h) gathers bytes [16h, 16h + 16) of every 32-byte K step
 // of pixel r straight from the image, in the K order (kh, kw, ic) of Im2ColPackUnitInt8Opt (conv_int8.c:758-807),
 // taps outside the image read as `fill` (conv_int8.c:877), bytes past K as 0; the weights come from the packed
@@ -281,6 +284,298 @@ int launch_conv_smallk(const int8_t *in, const ConvGeom &g, int fill, int k_true
     else MI_SMALLK(2, 4);
   }
 #undef MI_SMALLK
+  MI_HIP_CHECK(hipGetLastError());
+  return MI_OK;
+}
+
+// First-layer convolutions: few input channels, so that one row of the window -- kernel_w * in_c consecutive bytes of an
+// image row (dilation_w = 1) -- is at most 32 bytes.  The contraction is laid out row by row of the window, each padded
+// to 16 or 32 bytes (PARTS chunks of 16), with zero weights in the padding: a lane's 16 bytes of operand are then one
+// 16-byte load from any byte address of the image instead of 16 gathered bytes, and nothing is written in between (the
+// im2col buffer of 32 x 224 x 224 x 3, 7x7, is 64 MB).  Out-of-image bytes of a row are a byte range, the same for all
+// window rows, merged in with two masks made once per pixel.
+// The pixels are the MFMA's row operand: a lane ends up with ONE output channel of 16 pixels per accumulator block, its
+// requantisation parameters are loaded once and live in registers, and a 4 x 4 byte transposition across neighbouring
+// lanes makes dwords of four channels for the stores.  A wave keeps the weights of its up to 64 channels in registers
+// and walks tiles of 32 pixels, fetching the next tile's operand before it requantises the current one.
+// Bound at large sizes by the vector ALU (about 6 instructions per output byte, half of them the requantisation) and the
+// unaligned fetches, at small ones by the latency of one tile.  us per launch, before -> now: 32 x 224 x 224 x 3 -> 64,
+// 7x7, stride 2 134 (im2col and GEMM) -> 23; one such image 8.7 -> 4.8; 1 x 224 x 224 x 3 -> 32, 3x3, stride 2
+// 4.6 (sixteen byte loads per K step) -> 2.8.
+struct ConvRows {
+  const int8_t *in;
+  int in_bytes;
+  int in_h, in_w, in_c, out_w, out_hw, out_c;
+  int kernel_h, stride_h, stride_w, dil_h, pad_u, pad_l;
+  int parts;      // 16-byte chunks per window row: 1 or 2
+  int row_bytes;  // kernel_w * in_c
+  int fill;
+  int pixels;
+  const int8_t *w;  // [out_c padded to 64][32 * KS]
+};
+
+__device__ __forceinline__ uint32_t quad_transpose(uint32_t d, uint32_t sel1, uint32_t sel2) {
+  const uint32_t p = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)d, 0xB1, 0xF, 0xF, false);  // lane ^ 1
+  const uint32_t r = __builtin_amdgcn_perm(p, d, sel1);
+  const uint32_t q = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)r, 0x4E, 0xF, 0xF, false);  // lane ^ 2
+  return __builtin_amdgcn_perm(q, r, sel2);
+}
+
+// FAST: the one-multiply rounding form without weight zero points (RequantParams::fast2, !has_zw).
+template <int KS, int OCB, bool FAST>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void conv_rows_kernel(
+    ConvRows g, RequantParams rq, int8_t *__restrict__ out) {
+  typedef v4i v4i_any __attribute__((aligned(1)));
+  typedef uint32_t u32_any __attribute__((aligned(1)));
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+  const int n0 = blockIdx.y * (32 * OCB);
+  const int tiles = (g.pixels + 31) >> 5, step = gridDim.x * 4;
+  int tile = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (tile >= tiles) return;
+
+  v4i wf[OCB][KS];
+#pragma unroll
+  for (int ob = 0; ob < OCB; ++ob)
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+      wf[ob][s] = *reinterpret_cast<const v4i *>(g.w + (n0 + ob * 32 + r) * (32 * KS) + 32 * s + 16 * h);
+  // this lane's channel of each block (the arrays are padded to a multiple of 256 channels)
+  int32_t mult[OCB], bias[OCB], shift[OCB], lsh[OCB], zw[OCB];
+  uint64_t c2[OCB];
+#pragma unroll
+  for (int ob = 0; ob < OCB; ++ob) {
+    const int n = n0 + ob * 32 + r;
+    shift[ob] = rq.rshift[n];
+    if (FAST) {
+      mult[ob] = (int32_t)rq.mult2[n];
+      c2[ob] = (uint64_t)rq.c2hi[n] << 32 | rq.c2lo[n];
+      bias[ob] = rq.pre[n];
+    } else {
+      mult[ob] = rq.mult[n];
+      bias[ob] = (int32_t)((uint32_t)rq.bias2[n] - kAccBias);
+      lsh[ob] = rq.lshift[n];
+      zw[ob] = rq.zw[n];
+    }
+  }
+  int amin_v = rq.amin, amax_v = rq.amax;
+  asm volatile("" : "+v"(amin_v), "+v"(amax_v));  // kept in vector registers, as v_med3 wants them
+  const uint32_t sel1 = (lane & 1) ? 0x03070105u : 0x06020400u, sel2 = (lane & 2) ? 0x03020706u : 0x05040100u;
+  const uint32_t fill4 = (uint32_t)(g.fill & 0xff) * 0x01010101u;
+  const int part = g.parts == 2 ? h : 0;  // which chunk of a window row this lane holds
+  const int line = g.in_w * g.in_c, last16 = g.in_bytes - 16;
+  auto window_row = [&](int s) { return g.parts == 2 ? s : 2 * s + h; };
+
+  // where a tile's operand is: the image, the window's first row, the chunk's first byte in an image row
+  int img, ih0, t0;
+  auto locate = [&](int tl) {
+    const int want = tl * 32 + r, p = want < g.pixels ? want : g.pixels - 1;
+    const int b = (uint32_t)p / (uint32_t)g.out_hw, rem = p - b * g.out_hw;
+    const int oh = (uint32_t)rem / (uint32_t)g.out_w, ow = rem - oh * g.out_w;
+    img = b * (g.in_h * line);
+    ih0 = oh * g.stride_h - g.pad_u;
+    t0 = (ow * g.stride_w - g.pad_l) * g.in_c + 16 * part;
+  };
+  // Every load is a whole 16 bytes inside the tensor: rows above or below the image are clamped (their bytes are
+  // replaced), and an address before its first or behind its last 16 bytes is moved in.
+  auto address = [&](int s) {
+    int kh = window_row(s);
+    kh = kh < g.kernel_h ? kh : g.kernel_h - 1;
+    const int ih = min(max(ih0 + kh * g.dil_h, 0), g.in_h - 1);
+    return img + ih * line + t0;
+  };
+  auto fetch = [&](v4i (&x)[KS]) {
+#pragma unroll
+    for (int s = 0; s < KS; ++s) x[s] = *reinterpret_cast<const v4i_any *>(g.in + min(max(address(s), 0), last16));
+  };
+
+  locate(tile);
+  v4i x[KS];
+  fetch(x);
+  for (; tile < tiles; tile += step) {
+    if (__any(address(0) < 0 || address(KS - 1) > last16)) {  // a load that was moved in: move its bytes back
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        const int off = address(s), by = off - min(max(off, 0), last16);
+        if (by != 0) {
+          unsigned __int128 v = __builtin_bit_cast(unsigned __int128, x[s]);
+          v = by <= -16 || by >= 16 ? 0 : (by >= 0 ? v >> (8 * by) : v << (-8 * by));
+          x[s] = __builtin_bit_cast(v4i, v);
+        }
+      }
+    }
+    // bytes [-t0, line - t0) of this lane's chunk lie inside the image row, the others are fill
+    uint32_t in_row[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      const int a = min(max(-t0 - 4 * d, 0), 4), b = min(max(line - t0 - 4 * d, 0), 4);
+      in_row[d] = (uint32_t)((((uint64_t)1 << (8 * b)) - 1) & ~(((uint64_t)1 << (8 * a)) - 1));
+    }
+    const bool rows_inside = ih0 >= 0 && ih0 + (g.kernel_h - 1) * g.dil_h < g.in_h;
+    if (__all(rows_inside)) {
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+#pragma unroll
+        for (int d = 0; d < 4; ++d) x[s][d] = (int)(((uint32_t)x[s][d] & in_row[d]) | (fill4 & ~in_row[d]));
+    } else {
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        const bool row_ok = (unsigned)(ih0 + window_row(s) * g.dil_h) < (unsigned)g.in_h;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+          const uint32_t m = row_ok ? in_row[d] : 0u;
+          x[s][d] = (int)(((uint32_t)x[s][d] & m) | (fill4 & ~m));
+        }
+      }
+    }
+    v16i acc[OCB], sums;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+#pragma unroll
+      for (int ob = 0; ob < OCB; ++ob) acc[ob][e] = (int)kAccBias;
+      sums[e] = 0;
+    }
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int ob = 0; ob < OCB; ++ob) acc[ob] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x[s], wf[ob][s], acc[ob], 0, 0, 0);
+    if (!FAST && rq.has_zw) {  // the pixels' input sums, in the accumulators' layout: against ones where a window byte is
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        v4i one;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+          const int b = window_row(s) < g.kernel_h ? min(max(g.row_bytes - 16 * part - 4 * d, 0), 4) : 0;
+          one[d] = (int)(0x01010101u & (uint32_t)(((uint64_t)1 << (8 * b)) - 1));
+        }
+        sums = __builtin_amdgcn_mfma_i32_32x32x32_i8(x[s], one, sums, 0, 0, 0);
+      }
+    }
+    const int first = tile * 32;
+    if (tile + step < tiles) {  // (wave-uniform)
+      locate(tile + step);
+      fetch(x);
+    }
+    // acc[ob][4 * q + e] is pixel 8 * q + 4 * h + e of the tile, channel n0 + 32 * ob + r; after the transposition this
+    // lane holds channels r & ~3 .. + 3 of pixel 8 * q + 4 * h + (lane & 3)
+    const bool whole = first + 32 <= g.pixels && (g.out_c & 3) == 0;
+    const int my_n = n0 + (r & ~3), my_p = first + 4 * h + (lane & 3);
+    int8_t *dst = out + (int64_t)my_p * g.out_c + my_n;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+#pragma unroll
+      for (int ob = 0; ob < OCB; ++ob) {
+        int y[4];
+        if (FAST) {
+          // one 64-bit multiply-add per output; its carry is the rounding's "+1 unless negative"
+          uint64_t p2[4], carry[4], unused;
+          int32_t t[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            asm("v_mad_u64_u32 %0, %1, %2, %3, %4"
+                : "=&v"(p2[e]), "=s"(carry[e])
+                : "v"(acc[ob][4 * q + e]), "v"(mult[ob]), "v"(c2[ob]));
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            asm("v_addc_co_u32_e64 %0, %1, %2, %3, %4"
+                : "=v"(t[e]), "=s"(unused)
+                : "v"((int32_t)(p2[e] >> 32)), "v"(bias[ob]), "s"(carry[e]));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            t[e] >>= shift[ob];
+            asm("v_med3_i32 %0, %1, %2, %3" : "=v"(y[e]) : "v"(t[e]), "v"(amin_v), "v"(amax_v));
+          }
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            uint32_t v = (uint32_t)acc[ob][4 * q + e] - (uint32_t)sums[4 * q + e] * (uint32_t)zw[ob] + (uint32_t)bias[ob];
+            int32_t t = rdiv_pot(srdhm((int32_t)(v << lsh[ob]), mult[ob]), shift[ob]);
+            t = (int32_t)((uint32_t)t + (uint32_t)rq.zo);
+            t = t < rq.amax ? t : rq.amax;
+            y[e] = t > rq.amin ? t : rq.amin;
+          }
+        }
+        const uint32_t p01 = __builtin_amdgcn_perm((uint32_t)y[1], (uint32_t)y[0], 0x0c0c0400u);
+        const uint32_t p23 = __builtin_amdgcn_perm((uint32_t)y[3], (uint32_t)y[2], 0x0c0c0400u);
+        const uint32_t four = quad_transpose(__builtin_amdgcn_perm(p23, p01, 0x05040100u), sel1, sel2);
+        int8_t *to = dst + 8 * q * g.out_c + 32 * ob;
+        if (whole) {
+          if (my_n + 32 * ob < g.out_c) *reinterpret_cast<u32_any *>(to) = four;
+        } else if (my_p + 8 * q < g.pixels) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (my_n + 32 * ob + e < g.out_c) to[e] = (int8_t)(four >> (8 * e));
+        }
+      }
+    }
+  }
+}
+
+bool conv_rows_supported(const ConvGeom &g) {
+  const int row = g.kernel_w * g.in_c, parts = row <= 16 ? 1 : 2;
+  const int64_t bytes = (int64_t)g.batch * g.in_h * g.in_w * g.in_c;
+  return (g.in_c & 15) != 0 && g.dilation_w == 1 && row <= 32 && (g.kernel_h * parts + 1) / 2 <= kConvRowsSteps &&
+         bytes >= 16 && bytes < (int64_t)1 << 31;
+}
+
+// Weights [oc][kh][kw][ic] -> [oc padded to 64][steps of 32 bytes], see ConvRows.
+std::vector<int8_t> conv_rows_weights(const int8_t *w, int oc, int kernel_h, int kernel_w, int in_c) {
+  const int row = kernel_w * in_c, parts = row <= 16 ? 1 : 2, bytes = 32 * ((kernel_h * parts + 1) / 2);
+  std::vector<int8_t> out((size_t)round_up(oc, 64) * bytes, 0);
+  for (int c = 0; c < oc; ++c)
+    for (int kh = 0; kh < kernel_h; ++kh)
+      memcpy(&out[(size_t)c * bytes + (size_t)kh * parts * 16], w + ((size_t)c * kernel_h + kh) * row, (size_t)row);
+  return out;
+}
+
+int launch_conv_rows(const int8_t *in, const ConvGeom &g, int fill, const int8_t *w, const RequantParams &rq, int8_t *out,
+                     hipStream_t stream) {
+  ConvRows c{};
+  c.in = in;
+  c.in_bytes = g.batch * g.in_h * g.in_w * g.in_c;
+  c.in_h = g.in_h, c.in_w = g.in_w, c.in_c = g.in_c;
+  c.out_w = g.out_w, c.out_hw = g.out_h * g.out_w, c.out_c = g.out_c;
+  c.kernel_h = g.kernel_h, c.stride_h = g.stride_h, c.stride_w = g.stride_w, c.dil_h = g.dilation_h;
+  c.pad_u = g.pad_u, c.pad_l = g.pad_l;
+  c.row_bytes = g.kernel_w * g.in_c;
+  c.parts = c.row_bytes <= 16 ? 1 : 2;
+  c.fill = fill;
+  const int64_t pixels = (int64_t)g.batch * g.out_h * g.out_w;
+  c.pixels = (int)pixels;
+  c.w = w;
+  const int ks = (c.kernel_h * c.parts + 1) / 2;
+  if (!conv_rows_supported(g) || pixels < 1 || pixels > 0x7fffffff - 4096) {
+    set_error("conv_rows: unsupported geometry ic=%d kernel %dx%d", g.in_c, g.kernel_h, g.kernel_w);
+    return MI_PARAM_INVALID;
+  }
+  const int64_t wgs = (pixels + 127) / 128;
+  const bool two = g.out_c > 32, fast = rq.fast2 != 0 && rq.has_zw == 0;
+  const int gy = (g.out_c + (two ? 63 : 31)) / (two ? 64 : 32);
+  // three workgroups per CU: a wave then walks several tiles on one set of weight registers, and three waves per SIMD
+  // hide the fetches.  us at 32 x 224 x 224 x 3 -> 64, 7x7: 256 workgroups 25.7, 512 23.0, 768 23.9, 2048 27.1;
+  // 16 x 192 x 192 x 3 -> 32, 3x3: 6.8, 4.9, 4.7, 5.1
+  constexpr int64_t most = 768;
+  const dim3 grid((unsigned)(wgs < most ? wgs : most), (unsigned)gy);
+#define MI_ROWS(KS)                                                                                          \
+  case KS:                                                                                                   \
+    if (fast) {                                                                                              \
+      if (two) hipLaunchKernelGGL((conv_rows_kernel<KS, 2, true>), grid, dim3(256), 0, stream, c, rq, out);  \
+      else hipLaunchKernelGGL((conv_rows_kernel<KS, 1, true>), grid, dim3(256), 0, stream, c, rq, out);      \
+    } else {                                                                                                 \
+      if (two) hipLaunchKernelGGL((conv_rows_kernel<KS, 2, false>), grid, dim3(256), 0, stream, c, rq, out); \
+      else hipLaunchKernelGGL((conv_rows_kernel<KS, 1, false>), grid, dim3(256), 0, stream, c, rq, out);     \
+    }                                                                                                        \
+    break
+  switch (ks) {
+    MI_ROWS(1);
+    MI_ROWS(2);
+    MI_ROWS(3);
+    MI_ROWS(4);
+    MI_ROWS(5);
+    MI_ROWS(6);
+    MI_ROWS(7);
+    MI_ROWS(8);
+  }
+#undef MI_ROWS
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }

@@ -90,3 +90,30 @@ def test_dynamic_quant_parameters_follow_their_run(orc):
                 assert fetch(dq._h, side.cuda_stream, p) == lib.MI_OK
                 assert (p.scale, p.zero_point) == orc.dynamic_quant(xs[1] * np.float32(scale))[1:]
         dq.run(devs[0])
+
+
+@pytest.mark.parametrize("kernel,ic,oc", [((7, 7), 3, 64), ((5, 5), 3, 33), ((3, 3), 3, 32), ((3, 3), 5, 65), ((1, 1), 24, 130),
+                                          ((5, 3), 10, 6), ((3, 8), 4, 31), ((16, 1), 16 + 1, 40), ((8, 4), 8, 64),
+                                          ((9, 2), 16 - 1, 68), ((17, 3), 3, 36), ((4, 4), 8, 96), ((3, 11), 3, 32)])
+@pytest.mark.parametrize("asymmetric", [False, True])
+def test_first_layer_convolution_windows(orc, kernel, ic, oc, asymmetric):
+    """One and two 16-byte chunks per window row, every remainder of the contraction steps, the first window rows the
+    kernel does not take; images whose first and last bytes are inside padded windows."""
+    import torch
+    from oracle import pyoracle
+    rng = np.random.default_rng(kernel[0] * 1000 + kernel[1] * 100 + ic)
+    zp = rng.integers(-9, 10, oc).astype(np.int32) if asymmetric else np.zeros(oc, np.int32)
+    w = rng.integers(-128, 128, (oc, *kernel, ic), dtype=np.int8)
+    sw = rng.uniform(0.001, 0.01, oc).astype(np.float32).astype(np.float64)
+    bias = rng.integers(-2000, 2001, oc).astype(np.int32)
+    for (ih, iw), stride, pad in (((kernel[0], kernel[1]), (1, 1), (0, 0, 0, 0)), ((21, 19), (1, 2), (3, 2, 4, 1)),
+                                  ((40, 35), (2, 1), (kernel[0] // 2, kernel[0] // 2, kernel[1] // 2, kernel[1] // 2))):
+        x = rng.integers(-128, 128, (2, ih, iw, ic), dtype=np.int8)
+        shape = pyoracle.conv_shape(2, ih, iw, ic, oc, kernel, stride, (1, 1), pad)
+        conv = K.ConvolutionInt8Kernel(w, bias, K.QuantParam(0.02, 4), [K.QuantParam(float(s), int(z)) for s, z in zip(sw, zp)],
+                                       K.QuantParam(0.2, -6), stride, (1, 1), pad, 1, K.ACT_RELU, exact_3x3=True)
+        want = orc.conv_int8(x, w, bias, shape, 0.02, 4, sw, zp, 0.2, -6, K.ACT_RELU)
+        assert np.array_equal(conv.run(torch.from_numpy(x).cuda()).cpu().numpy(), want), (kernel, ic, oc, ih, iw)
+        flat = torch.zeros(x.size + 3, dtype=torch.int8, device="cuda")  # an image at an odd address
+        flat[3:] = torch.from_numpy(x.reshape(-1)).cuda()
+        assert np.array_equal(conv.run(flat[3:].view(x.shape)).cpu().numpy(), want), (kernel, ic, oc, ih, iw)
