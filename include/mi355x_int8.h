@@ -109,23 +109,23 @@ typedef struct mi_matmul_desc {
 } mi_matmul_desc;
 
 /* All weight packing happens in mi_matmul_create (the role of TransferB, LK/int8/matmul_base_int8.cc:360-384: pack
- * once at Prepare).  Two packed forms are kept: K-contiguous rows (GEMM tiles; one activation row) and 1 KiB
- * blocks of 16 channels x 64 K-bytes in matrix-core operand order (2..64 activation rows, 2..128 against at most
- * 4096 channels with deep >= 1024: the batched decode kernel).  MI_MATMUL_NO_DECODE_PACK skips the second form (deep x col bytes of device memory less) for callers
- * that know they never run with 2..64 rows; such a handle still accepts those row counts and runs two rows on the
- * one-row kernel's two-row form and the others on the GEMM tiles.  mi_matmul_run never packs, allocates for packing or waits. */
+ * once at Prepare).  Two packed forms are kept: K-contiguous rows (one activation row) and 1 KiB blocks of 16 channels x
+ * 64 K-bytes in matrix-core operand order (the decode kernel for a few rows and the GEMM tiles for more).
+ * MI_MATMUL_NO_DECODE_PACK skips the second form (deep x col bytes of device memory less); such a handle accepts the same
+ * row counts and runs two rows on the one-row kernel's two-row form and more on GEMM tiles over the first form, slower.
+ * mi_matmul_run never packs, allocates for packing or waits. */
 #define MI_MATMUL_NO_DECODE_PACK 1
 
 /* weight_host: int8 const weight; bias_host: int32 [col] or NULL.  Both are consumed during the call. */
 int mi_matmul_create(const mi_matmul_desc *desc, const int8_t *weight_host, const int32_t *bias_host,
                      mi_matmul **out);
 /* Sizes the handle's workspaces for runs of up to `max_rows` rows, so that later runs allocate nothing: the role of
- * the buffers MatmulBaseInt8CPUKernel::ReSize allocates (LK/int8/matmul_base_int8.cc:296-325).  Workspaces exist only
- * for operand shapes the kernels cannot take in place (deep % 16 != 0 or a misaligned activation base: a padded copy
- * of the activations; col % 4 != 0 or a misaligned output base: a padded output).  Without this call the first run
- * that needs a larger workspace allocates it with hipMalloc, at least twice the previous size; the outgrown buffer
- * may still be in use by kernels in flight, so it is kept until the handle is destroyed (a handle therefore holds at
- * most about twice its largest workspace; the same holds for the im2col and output workspaces of mi_conv). */
+ * the buffers MatmulBaseInt8CPUKernel::ReSize allocates (LK/int8/matmul_base_int8.cc:296-325).  A workspace exists only
+ * for operands the kernels cannot take in place (deep % 16 != 0 or a misaligned activation base: a padded copy of the
+ * activations).  Without this call the first run that needs a larger workspace allocates it with hipMalloc, at least
+ * twice the previous size; the outgrown buffer may still be in use by kernels in flight, so it is kept until the handle is
+ * destroyed (a handle therefore holds at most about twice its largest workspace; the same holds for the im2col workspace
+ * of mi_conv). */
 int mi_matmul_reserve(mi_matmul *h, int32_t max_rows);
 /* a_dev: int8 [rows, deep]; c_dev: int8 [rows, col].  Asynchronous on `stream`. */
 int mi_matmul_run(mi_matmul *h, const int8_t *a_dev, int32_t rows, int8_t *c_dev, void *stream);
@@ -215,7 +215,7 @@ int mi_conv_same_pad(int32_t in, int32_t kernel, int32_t stride, int32_t dilatio
 int mi_conv_run(mi_conv *h, const int8_t *in_dev, int32_t batch, int32_t in_h, int32_t in_w, int8_t *out_dev,
                 void *stream);
 int mi_conv_run_host(mi_conv *h, const int8_t *in_host, int32_t batch, int32_t in_h, int32_t in_w, int8_t *out_host);
-/* Sizes the handle's workspaces (im2col buffer, padded rows / output, where the shape needs them) for this input
+/* Sizes the handle's workspace (im2col buffer or padded rows, where the shape needs them) for this input
  * geometry, so that later runs of it allocate nothing: the role of ConvolutionInt8CPUKernel::InitTmpBuffer
  * (LK/int8/convolution_int8.cc:159-197). */
 int mi_conv_reserve(mi_conv *h, int32_t batch, int32_t in_h, int32_t in_w);
@@ -288,8 +288,8 @@ typedef struct mi_dynmm_desc {
  * sums.  b_transpose is ignored with this flag. */
 #define MI_DYNMM_WEIGHT_PACKED_SDOT 1
 /* Like mi_matmul, a dynamic MatMul handle holds a second, blocked form of its weights (deep x col bytes more) that
- * serves 1..64 activation rows (decode) with the matrix-core weight-streaming kernel; MI_DYNMM_NO_DECODE_PACK skips it
- * for handles that will only see larger row counts (few rows then run on the GEMM tiles, same results). */
+ * serves two activation rows and more; MI_DYNMM_NO_DECODE_PACK skips it (same results on GEMM tiles over the first form,
+ * slower). */
 #define MI_DYNMM_NO_DECODE_PACK 2
 /* The unpacking by itself (host arithmetic, no GPU needed): packed -> weight_nk [col][deep] row-major. */
 int mi_unpack_weight_4x16(const int8_t *packed, int32_t col, int32_t deep, int8_t *weight_nk);

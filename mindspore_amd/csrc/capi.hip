@@ -212,7 +212,7 @@ struct RequantState {
   int n = 0, k = 0, n_pad = 0, k_pad = 0, ldw = 0;
   DevBuf w, mult, bias2, rshift, lshift, zw;
   DevBuf mult2, c2lo, c2hi, pre;  // the GEMM epilogue's per-channel constants (RequantParams::fast2)
-  DevBuf w_blocked;  // the same weights in 1 KiB matrix-core blocks (2..64 activation rows, some shapes ..128); built in create or absent
+  DevBuf w_blocked;  // the same weights in 1 KiB matrix-core blocks (two activation rows and more); built in create or absent
   std::vector<int32_t> h_mult, h_ls, h_rs, h_bias2;
   int32_t amin = -128, amax = 127, zo = 0;
   bool has_zw = false, fast = false, fast2 = false;
@@ -319,8 +319,8 @@ struct RequantState {
       for (int c = 0; c < n; ++c) memcpy(packed.data() + (size_t)c * ldw, w_nk + (size_t)c * k, (size_t)k);
       if ((rc = upload(&w, packed)) != MI_OK) return rc;
       if (pack_decode) {
-        // The blocked copy is an optimisation for 2..64 activation rows (some shapes: ..128), not a requirement: without it those row
-        // counts run on the v_dot4 kernel (two rows) or the GEMM tiles.  A device that has no room for it still gets
+        // The blocked copy is an optimisation, not a requirement: without it two rows run on the v_dot4 kernel and more on
+        // the GEMM tiles over the row-major weights.  A device that has no room for it still gets
         // a working handle.
         rc = w_blocked.ensure((size_t)n_pad * k_pad);
         if (rc == MI_OK)
@@ -416,29 +416,17 @@ static int prepare_rows(const int8_t *a, int rows, int k, const Workspace &ws, h
   return MI_OK;
 }
 
-// The GEMM kernels write rows with vector stores; when the caller's row length or base address does not allow that,
-// they write to a padded scratch output which is then compacted into the caller's tensor.
 static int run_requant_gemm(RequantState &st, const int8_t *a, int64_t lda, int rows, int k16, int8_t *c,
-                            const Workspace &c_ws, hipStream_t stream) {
+                            hipStream_t stream) {
   const RequantParams rq = st.params();
-  WeightView w{static_cast<const int8_t *>(st.w.p), st.k_pad, st.ldw, nullptr};
-  // one row: the dot kernel on the row-major weights; 2..64 rows (..128 against at most 4096 channels and K >= 1024): the matrix-core decode kernel on the blocked copy
-  // made at create time -- a handle without it runs two rows on the dot kernel and 3..64 on the GEMM tiles
+  // (the blocked copy may be absent: two rows then take the v_dot4 kernel)
+  const WeightView w{static_cast<const int8_t *>(st.w.p), st.k_pad, st.ldw, static_cast<const int8_t *>(st.w_blocked.p)};
+  // one row: the dot kernel on the row-major weights; few rows: the matrix-core decode kernel on the blocked copy made at
+  // create time (a handle without it runs two rows on the dot kernel and the others on the GEMM tiles)
   const bool skinny = rows <= kGemvDotRows ? (int64_t)rows * k16 <= 150 * 1024
-                                           : gemv_takes_rows(rows, st.n, st.k_pad) && st.w_blocked.p != nullptr && st.k_pad <= 1 << 20;
-  if (skinny) {
-    if (rows >= 2) w.blocked = static_cast<const int8_t *>(st.w_blocked.p);  // (may be absent: two rows then take the v_dot4 kernel)
-    return launch_gemv_requant(a, lda, rows, k16, w, st.n, rq, c, st.n, stream);
-  }
-  if ((st.n & 3) == 0 && (reinterpret_cast<uintptr_t>(c) & 3) == 0)
-    return launch_gemm_requant(a, lda, rows, k16, w, st.n, rq, c, st.n, stream);
-  const int n4 = round_up(st.n, 4);
-  void *buf = nullptr;
-  int rc = c_ws.get((size_t)rows * n4, &buf);
-  if (rc != MI_OK) return rc;
-  rc = launch_gemm_requant(a, lda, rows, k16, w, n4, rq, static_cast<int8_t *>(buf), n4, stream);
-  if (rc != MI_OK) return rc;
-  return launch_copy_rows(buf, n4, rows, st.n, c, st.n, stream);
+                                           : gemv_takes_rows(rows, st.n) && st.w_blocked.p != nullptr && st.k_pad <= 1 << 20;
+  if (skinny) return launch_gemv_requant(a, lda, rows, k16, w, st.n, rq, c, st.n, stream);
+  return launch_gemm_requant(a, lda, rows, k16, w, st.n, rq, c, st.n, stream);
 }
 
 }  // namespace mi
@@ -449,7 +437,7 @@ using namespace mi;
 struct mi_matmul {
   RequantState st;  // weight matrix 0
   std::vector<std::unique_ptr<RequantState>> more;  // weight matrices 1 .. b_batch - 1 of a batched constant weight
-  DevBuf a_ws, c_ws, h_in, h_out;
+  DevBuf a_ws, h_in, h_out;
   int b_batch() const { return 1 + (int)more.size(); }
   RequantState &state(int b) { return b == 0 ? st : *more[(size_t)b - 1]; }
 };
@@ -459,7 +447,7 @@ struct mi_conv {
   bool depthwise = false, direct_1x1 = false, dw_fast = false;
   int fill = 0;
   RequantState st;
-  DevBuf w16, dw_bias, dw_bias_folded, col_ws, c_ws, h_in, h_out;
+  DevBuf w16, dw_bias, dw_bias_folded, col_ws, h_in, h_out;
   DevBuf w_rows;  // the weights of a convolution on few channels as launch_conv_rows takes them, or empty
   DevBuf fill16;  // 16 bytes of `fill`: where the gathering GEMM loader reads taps outside the image
 };
@@ -487,8 +475,8 @@ struct mi_dynmm {
   int n = 0, k = 0, n_pad = 0, k_pad = 0, ldw = 0, act = 0;
   int32_t zw0 = 0;
   bool has_bias = false;
-  DevBuf w, wscale, wsum, bias, a_ws, c_ws, h_in, h_out, h_params;
-  DevBuf w_blocked;  // the weights in 1 KiB matrix-core blocks for 2..64 activation rows (some shapes ..128); built in create or absent
+  DevBuf w, wscale, wsum, bias, a_ws, h_in, h_out, h_params;
+  DevBuf w_blocked;  // the weights in 1 KiB matrix-core blocks for two activation rows and more; built in create or absent
 };
 
 // No C++ exception may cross the C ABI: host allocations in the create calls can throw.
@@ -739,9 +727,8 @@ int mi_matmul_reserve(mi_matmul *h, int32_t max_rows) {
   if (max_rows < 0) return MI_PARAM_INVALID;
   int rc = ensure_device();
   if (rc != MI_OK) return rc;
-  // sized for the worst case of either workspace: whether a run needs them also depends on its pointers
-  if ((rc = h->a_ws.ensure((size_t)max_rows * round_up(h->st.k, 16))) != MI_OK) return rc;
-  return h->c_ws.ensure((size_t)max_rows * round_up(h->st.n, 4));
+  // sized for the worst case: whether a run needs the workspace also depends on its pointers
+  return h->a_ws.ensure((size_t)max_rows * round_up(h->st.k, 16));
 }
 
 int mi_matmul_run(mi_matmul *h, const int8_t *a_dev, int32_t rows, int8_t *c_dev, void *stream) {
@@ -757,11 +744,15 @@ int mi_matmul_run(mi_matmul *h, const int8_t *a_dev, int32_t rows, int8_t *c_dev
   int rc = ensure_device();
   if (rc != MI_OK) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  // Whether a run copies its activations depends on its pointer as well.  A MatMul with odd-sized rows sits among tensors
+  // whose parts start anywhere, so its first run of a row count makes the room at once: no later run of that row count
+  // allocates, and one with a misaligned pointer can be the one under graph capture.
+  if ((h->st.n & 3) != 0 && (rc = h->a_ws.ensure((size_t)rows * round_up(h->st.k, 16))) != MI_OK) return rc;
   const int8_t *a = nullptr;
   int64_t lda = 0;
   int k16 = 0;
   if ((rc = prepare_rows(a_dev, rows, h->st.k, Workspace::growable(&h->a_ws), s, &a, &lda, &k16)) != MI_OK) return rc;
-  return run_requant_gemm(h->st, a, lda, rows, k16, c_dev, Workspace::growable(&h->c_ws), s);
+  return run_requant_gemm(h->st, a, lda, rows, k16, c_dev, s);
 }
 
 int mi_matmul_run_batched(mi_matmul *h, const int8_t *a_dev, int32_t rows, int32_t batch, const int32_t *a_offsets,
@@ -795,8 +786,7 @@ int mi_matmul_run_batched(mi_matmul *h, const int8_t *a_dev, int32_t rows, int32
     if ((rc = prepare_rows(a_dev + (size_t)a_offsets[i] * a_mat, rows, h->st.k, Workspace::growable(&h->a_ws), s, &a, &lda,
                            &k16)) != MI_OK)
       return rc;
-    if ((rc = run_requant_gemm(h->state(b_offsets[i]), a, lda, rows, k16, c_dev + (size_t)i * c_mat,
-                               Workspace::growable(&h->c_ws), s)) != MI_OK)
+    if ((rc = run_requant_gemm(h->state(b_offsets[i]), a, lda, rows, k16, c_dev + (size_t)i * c_mat, s)) != MI_OK)
       return rc;
   }
   return MI_OK;
@@ -850,7 +840,7 @@ int mi_matmul_run_group(mi_matmul *const *handles, int32_t count, const int8_t *
     return launch_gemv_group(a, lda, rows, k16, count, wv, n, rq, c_dev, s);
   }
   for (int i = 0; i < count; ++i)
-    if ((rc = run_requant_gemm(handles[i]->st, a, lda, rows, k16, c_dev[i], Workspace::growable(&handles[i]->c_ws), s)) != MI_OK)
+    if ((rc = run_requant_gemm(handles[i]->st, a, lda, rows, k16, c_dev[i], s)) != MI_OK)
       return rc;
   return MI_OK;
 }
@@ -872,9 +862,8 @@ int mi_matmul_run_noalloc(mi_matmul *h, const int8_t *a_dev, int32_t rows, int8_
     set_error("mi_matmul_run_noalloc: no scratch memory on device %d", g_device);
     return MI_ERROR;
   }
-  // the padded activation rows first, the padded output behind them; a part is only needed when the operand's shape
-  // or this call's pointer alignment asks for it, and only the needed parts count against the maximum (so a shape
-  // that passes with aligned pointers can be refused with misaligned ones)
+  // The scratch area holds the padded activation rows.  The documented maximum also counts a padded output where
+  // col % 4 != 0 or c_dev is not 4-byte aligned: no kernel needs one, the limit callers know stays.
   const size_t a_bytes = round_up64((int64_t)rows * round_up(h->st.k, 16), 256);
   const size_t c_bytes = (size_t)rows * round_up(h->st.n, 4);
   const bool a_padded = (h->st.k & 15) != 0, c_padded = (h->st.n & 3) != 0;
@@ -886,15 +875,13 @@ int mi_matmul_run_noalloc(mi_matmul *h, const int8_t *a_dev, int32_t rows, int8_
               "maximum is %zu; use mi_matmul_run", rows, h->st.k, h->st.n, need, kScratchBytes);
     return MI_PARAM_INVALID;
   }
-  unsigned char *p = static_cast<unsigned char *>(base);
-  const Workspace a_ws = Workspace::region(p, a_bytes);
-  const Workspace c_ws = Workspace::region(p + ((a_padded || a_unaligned) ? a_bytes : 0), c_bytes);
+  const Workspace a_ws = Workspace::region(base, a_bytes);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int8_t *a = nullptr;
   int64_t lda = 0;
   int k16 = 0;
   if ((rc = prepare_rows(a_dev, rows, h->st.k, a_ws, s, &a, &lda, &k16)) != MI_OK) return rc;
-  return run_requant_gemm(h->st, a, lda, rows, k16, c_dev, c_ws, s);
+  return run_requant_gemm(h->st, a, lda, rows, k16, c_dev, s);
 }
 
 int mi_matmul_run_host(mi_matmul *h, const int8_t *a_host, int32_t rows, int8_t *c_host) {
@@ -1067,10 +1054,9 @@ int mi_conv_reserve(mi_conv *h, int32_t batch, int32_t in_h, int32_t in_w) {
   if (h->depthwise || batch == 0) return MI_OK;
   if ((rc = ensure_device()) != MI_OK) return rc;
   const size_t pixels = (size_t)batch * oh * ow;
-  // the im2col buffer (or, for a 1x1, the padded copy of the image rows) and the padded output, whether or not this
-  // geometry and the run's pointers end up needing them
-  if ((rc = h->col_ws.ensure(pixels * round_up(h->st.k, 16))) != MI_OK) return rc;
-  return h->c_ws.ensure(pixels * round_up(h->st.n, 4));
+  // the im2col buffer (or, for a 1x1, the padded copy of the image rows), whether or not this geometry and the run's
+  // pointers end up needing it
+  return h->col_ws.ensure(pixels * round_up(h->st.k, 16));
 }
 
 int mi_conv_run(mi_conv *h, const int8_t *in_dev, int32_t batch, int32_t in_h, int32_t in_w, int8_t *out_dev,
@@ -1109,7 +1095,7 @@ int mi_conv_run(mi_conv *h, const int8_t *in_dev, int32_t batch, int32_t in_h, i
   } else if (h->w_rows.p != nullptr && conv_rows_supported(g)) {
     // a first-layer convolution: window rows straight from the image
     return launch_conv_rows(in_dev, g, h->fill, static_cast<const int8_t *>(h->w_rows.p), h->st.params(), out_dev, s);
-  } else if ((pixels > 128 || k <= 64) && gemm_conv_supported(g, in_dev, out_dev)) {
+  } else if ((pixels > 128 || k <= 64) && gemm_conv_supported(g, in_dev)) {
     // 16-channel-aligned images: the GEMM gathers its activation operand from the image, no im2col buffer (with few
     // pixels the buffer is small and the decode kernel streams the weights faster, unless there are next to none)
     WeightView w{static_cast<const int8_t *>(h->st.w.p), h->st.k_pad, h->st.ldw, nullptr};
@@ -1125,7 +1111,7 @@ int mi_conv_run(mi_conv *h, const int8_t *in_dev, int32_t batch, int32_t in_h, i
     a = static_cast<const int8_t *>(h->col_ws.p);
     lda = k16;
   }
-  return run_requant_gemm(h->st, a, lda, (int)pixels, k16, out_dev, Workspace::growable(&h->c_ws), s);
+  return run_requant_gemm(h->st, a, lda, (int)pixels, k16, out_dev, s);
 }
 
 int mi_conv_run_host(mi_conv *h, const int8_t *in_host, int32_t batch, int32_t in_h, int32_t in_w, int8_t *out_host) {
@@ -1434,16 +1420,10 @@ static int dynmm_run_impl(mi_dynmm *h, const int8_t *a_dev, int32_t rows, float 
                      static_cast<const int8_t *>(h->w_blocked.p)};
   // decode-sized runs: the matrix-core decode kernel streams the blocked weights once (any N, any output alignment)
   // (one row runs on the row-major weights and needs no blocked copy, as long as the row fits the kernel's LDS form)
-  if (gemv_takes_rows(rows, h->n, h->k_pad) && (rows > kGemvDotRows || (int64_t)rows * k16 <= 150 * 1024) &&
+  if (gemv_takes_rows(rows, h->n) && (rows > kGemvDotRows || (int64_t)rows * k16 <= 150 * 1024) &&
       (rows == 1 || (w.blocked != nullptr && h->k_pad <= 1 << 20)))
     return launch_gemv_dequant(a, lda, rows, k16, w, h->n, dq, c_dev, h->n, s);
-  if ((h->n & 3) == 0 && (reinterpret_cast<uintptr_t>(c_dev) & 15) == 0)
-    return launch_gemm_dequant(a, lda, rows, k16, w, h->n, dq, c_dev, h->n, s);
-  const int n4 = round_up(h->n, 4);
-  if ((rc = h->c_ws.ensure((size_t)rows * n4 * sizeof(float))) != MI_OK) return rc;
-  if ((rc = launch_gemm_dequant(a, lda, rows, k16, w, n4, dq, static_cast<float *>(h->c_ws.p), n4, s)) != MI_OK)
-    return rc;
-  return launch_copy_rows(h->c_ws.p, (int64_t)n4 * 4, rows, h->n * 4, c_dev, (int64_t)h->n * 4, s);
+  return launch_gemm_dequant(a, lda, rows, k16, w, h->n, dq, c_dev, h->n, s);
 }
 
 int mi_dynmm_reserve(mi_dynmm *h, int32_t max_rows) {
@@ -1451,8 +1431,7 @@ int mi_dynmm_reserve(mi_dynmm *h, int32_t max_rows) {
   if (max_rows < 0) return MI_PARAM_INVALID;
   int rc = ensure_device();
   if (rc != MI_OK) return rc;
-  if ((rc = h->a_ws.ensure((size_t)max_rows * round_up(h->k, 16))) != MI_OK) return rc;
-  return h->c_ws.ensure((size_t)max_rows * round_up(h->n, 4) * sizeof(float));
+  return h->a_ws.ensure((size_t)max_rows * round_up(h->k, 16));
 }
 
 int mi_dynmm_run(mi_dynmm *h, const int8_t *a_dev, int32_t rows, double in_scale, int32_t in_zp, float *c_dev,

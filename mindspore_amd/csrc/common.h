@@ -76,7 +76,7 @@ struct WeightView {
   const int8_t *w;
   int k_pad;
   int ldw;
-  // Second copy for the matrix-core decode kernel (2..64 activation rows), or nullptr: the same bytes regrouped into
+  // Second copy for the matrix-core decode kernel and the GEMM's K-block loops, or nullptr: the same bytes regrouped into
   // 1 KiB blocks [row / 16][k / 64], the 64 16-byte chunks of a block in the order the lanes of the MFMA operand take
   // them ([(k % 64) / 16][row % 16]), so that a wave instruction fetches 1 KiB front to back.  Built on the device
   // when the handle is created (launch_block_weights).
@@ -85,8 +85,7 @@ struct WeightView {
 inline int weight_row_stride(int k_pad) { return (k_pad / 256) % 2 == 0 ? k_pad + 256 : k_pad; }
 
 // A: int8 activations [M][lda] (lda in bytes, multiple of 16, base 16-byte aligned, K % 16 == 0);
-// W: packed weights (above); C: [M][ldc] elements with n % 4 == 0, ldc % 4 == 0 and a 4-byte (int8) /
-// 16-byte (fp32) aligned base -- other output shapes go through a padded scratch buffer and launch_copy_rows.
+// W: packed weights (above); C: [M][ldc] elements, any n and ldc >= n, any address of the element type.
 int launch_gemm_requant(const int8_t *a, int64_t lda, int m, int k, const WeightView &w, int n,
                         const RequantParams &rq, int8_t *c, int64_t ldc, hipStream_t stream);
 int launch_gemm_dequant(const int8_t *a, int64_t lda, int m, int k, const WeightView &w, int n,
@@ -95,16 +94,14 @@ int launch_gemm_dequant(const int8_t *a, int64_t lda, int m, int k, const Weight
 // Skinny-M path (m <= kGemvMaxRows): streams the weights once with 16-byte coalesced loads.
 constexpr int kGemvMaxRows = 64;
 constexpr int kGemvGroupMaxRows = 32;  // the group launches (several matrices, one launch) stop here
-// 65..128 rows keep the matrix-core decode kernel only where it has at most one workgroup per CU (16 channels each,
-// so at most 4096 channels) and a reduction long enough to pay for its set-up.  Measured against the GEMM's
-// weight-stream tiles at 128 rows, weights not cache-resident (us per launch): 4096 x 4096 14.5 against 22.6,
-// 4096 x 11008 31.5 against 52.7, 1024 x 4096 12.7 against 22.5, 4096 x 1024 6.8 against 8.8, 2048 x 768 7.1 against
-// 6.7; 6144 x 4096 25.0 against 22.9, 8192 x 4096 26.6 against 23.1.
-constexpr int kGemvNarrowMaxRows = 128;
-constexpr int kGemvNarrowChannels = 4096;  // at most this many
-constexpr int kGemvNarrowMinK = 1024;      // padded reduction length from which those rows come here
-inline bool gemv_takes_rows(int rows, int n, int k_pad) {
-  return rows <= kGemvMaxRows || (rows <= kGemvNarrowMaxRows && n <= kGemvNarrowChannels && k_pad >= kGemvNarrowMinK);
+// 33..64 rows come here against at most 4096 channels, of which the kernel's workgroups hold 16 each and the GEMM's smallest
+// tile 64; against more channels the GEMM tiles have CUs enough and re-read the activations less.  us per launch at 64
+// rows, this path / the tiles: 4096 x 4096 8.8 / 11.0, 4096 x 11008 18.7 / 27.5, 768 x 3072 6.8 / 7.5, 6144 x 2048
+// 9.2 / 7.6, 12288 x 4096 14.5 / 13.8; at 80 rows, where a form of the kernel with eight row groups existed: 4096 x 4096
+// 11.9 / 9.8, 4096 x 11008 25.6 / 21.0, 768 x 3072 9.6 / 7.5.
+constexpr int kGemvNarrowChannels = 4096;
+inline bool gemv_takes_rows(int rows, int n) {
+  return rows <= kGemvGroupMaxRows || (rows <= kGemvMaxRows && n <= kGemvNarrowChannels);
 }
 constexpr int kGemvDotRows = 2;  // up to here the v_dot4 kernel can run (it does for one row, and for two when the handle has no blocked copy), above it the MFMA kernel
 int launch_gemv_requant(const int8_t *a, int64_t lda, int m, int k, const WeightView &w, int n,
@@ -133,10 +130,6 @@ int launch_block_weights(const int8_t *w, int n_pad, int k_pad, int ldw, int8_t 
 // Copies [rows][k] (row stride src_ld bytes) into a zero-padded [rows][k16] buffer, k16 = round_up(k, 16).
 int launch_pad_rows(const int8_t *src, int64_t src_ld, int rows, int k, int8_t *dst, int k16, hipStream_t stream);
 
-// dst[row][0..row_bytes) = src[row][0..row_bytes); strides in bytes.
-int launch_copy_rows(const void *src, int64_t src_ld, int rows, int row_bytes, void *dst, int64_t dst_ld,
-                     hipStream_t stream);
-
 struct ConvGeom {
   int batch, in_h, in_w, in_c, out_h, out_w, out_c;
   int kernel_h, kernel_w, stride_h, stride_w, dilation_h, dilation_w, pad_u, pad_l;
@@ -162,7 +155,7 @@ int launch_conv_dw(const int8_t *in, const ConvGeom &g, const int16_t *w16, cons
 
 // The requantising GEMM with its activation operand gathered from an NHWC image (in_c % 16 == 0): the im2col
 // convolution without the buffer.  fill16: 16 bytes of the value out-of-image taps take, in device memory.
-bool gemm_conv_supported(const ConvGeom &g, const void *in, const void *out);
+bool gemm_conv_supported(const ConvGeom &g, const void *in);
 int launch_gemm_conv_requant(const int8_t *in, const ConvGeom &g, const int8_t *fill16, const WeightView &w,
                              const RequantParams &rq, int8_t *out, hipStream_t stream);
 

@@ -717,42 +717,17 @@ static int with_row_class(int m, F &&f) {  // rows rounded up to 2, 4, 8, 16 or 
   return f(integral_constant<int, 32>());
 }
 
-// 33..64 rows: four groups of 16 activation rows against every weight fragment, two steps per pass (the staging
-// area of 64 rows and the accumulators leave room for no more).  Measured against the 64 x 64 GEMM tiles these row
-// counts ran on before (us per launch at 64 rows): 12288 x 4096 17.9 -> 14.9, 4096 x 4096 15.8 -> 8.9,
-// 4096 x 11008 34.9 -> 18.7.
-// 65..128 rows against at most 4096 channels with K >= 1024: eight fragments per weight fragment, one channel group
-// per workgroup (the staging area of 128 rows takes the LDS of a CU, so more than 4096 channels would need a second
-// round of workgroups, and shorter reductions do not pay for the set-up).  Every workgroup re-reads M / 16 = 8
-// activation bytes per weight byte from the L2s, which is what bounds it; the GEMM's weight-stream tiles of 64
-// channels, the alternative, occupy at most N / 64 CUs (us per launch at 128 rows, weights not cache-resident:
-// 4096 x 4096 22.6 -> 14.5, 4096 x 11008 52.7 -> 31.5; with the weights in the caches the two are level at
-// 4096 x 4096, 13.3 against 13.5).  Two channel groups per workgroup with one step per pass (what the LDS then has
-// room for) were 10-15 % ahead of the tiles between 4096 and 8192 channels and behind them above, and were not kept.
-static int launch_mfma_lds_128(const GemvArgs &g, int m, const RequantParams &rq, hipStream_t stream) {
-  hipLaunchKernelGGL((gemv_mfma_lds_kernel<8, 1, 2, 128>), dim3((g.n + 15) / 16), dim3(512), 0, stream, g, m, rq);
-  MI_HIP_CHECK(hipGetLastError());
-  return MI_OK;
-}
-
-static int launch_mfma_lds_deq_128(const GemvArgs &g, int m, const DequantParams &dq, hipStream_t stream) {
-  hipLaunchKernelGGL((gemv_mfma_lds_deq_kernel<8, 1, 2, 128>), dim3((g.n + 15) / 16), dim3(512), 0, stream, g, m, dq);
-  MI_HIP_CHECK(hipGetLastError());
-  return MI_OK;
-}
-
-template <int RG>
+// 33..64 rows (against at most 4096 channels, see gemv_takes_rows): four groups of 16 activation rows against every weight
+// fragment, two steps per pass (the staging area of 64 rows and the accumulators leave room for no more).  Measured
+// against 64 x 64 GEMM tiles in us per launch at 64 rows: 4096 x 4096 11.0 -> 8.8, 4096 x 11008 27.5 -> 18.7.
 static int launch_mfma_lds_64(const GemvArgs &g, int m, const RequantParams &rq, hipStream_t stream) {
-  const int blocks = (g.n + RG * 16 - 1) / (RG * 16);
-  hipLaunchKernelGGL((gemv_mfma_lds_kernel<8, RG, 2, 64>), dim3(blocks), dim3(512), 0, stream, g, m, rq);
+  hipLaunchKernelGGL((gemv_mfma_lds_kernel<8, 1, 2, 64>), dim3((g.n + 15) / 16), dim3(512), 0, stream, g, m, rq);
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }
 
-template <int RG>
 static int launch_mfma_lds_deq_64(const GemvArgs &g, int m, const DequantParams &dq, hipStream_t stream) {
-  const int blocks = (g.n + RG * 16 - 1) / (RG * 16);
-  hipLaunchKernelGGL((gemv_mfma_lds_deq_kernel<8, RG, 2, 64>), dim3(blocks), dim3(512), 0, stream, g, m, dq);
+  hipLaunchKernelGGL((gemv_mfma_lds_deq_kernel<8, 1, 2, 64>), dim3((g.n + 15) / 16), dim3(512), 0, stream, g, m, dq);
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }
@@ -832,7 +807,7 @@ static int check_gemv_operands(const int8_t *a, int64_t lda, int m, int k, const
     set_error("gemv: null pointer");
     return MI_NULL_PTR;
   }
-  if (m < 1 || !gemv_takes_rows(m, n, wv.k_pad) || n <= 0 || k <= 0 || (k & 15) != 0 || (lda & 15) != 0 || lda < k ||
+  if (m < 1 || !gemv_takes_rows(m, n) || n <= 0 || k <= 0 || (k & 15) != 0 || (lda & 15) != 0 || lda < k ||
       wv.k_pad % kKPad != 0 || wv.k_pad < k || wv.ldw < wv.k_pad || (wv.ldw & 15) != 0 ||
       (reinterpret_cast<uintptr_t>(a) & 15) != 0 ||
       (int64_t)(m - 1) * lda + k >= (int64_t)1 << 30 || wv.k_pad > 1 << 20 ||  // (32-bit buffer offsets)
@@ -891,10 +866,7 @@ int launch_gemv_requant(const int8_t *a, int64_t lda, int m, int k, const Weight
     g.w = wv.blocked;
     // three 16-channel groups per workgroup (a third of the activation traffic) once there are enough channels to
     // fill the device with 8-wave workgroups and the rows are short enough for a wave's share to be in flight at once
-    if (m > 64) return launch_mfma_lds_128(g, m, rq, stream);
-    if (m > 32) {
-      return n >= 8192 && k_pad <= 4096 ? launch_mfma_lds_64<3>(g, m, rq, stream) : launch_mfma_lds_64<1>(g, m, rq, stream);
-    }
+    if (m > 32) return launch_mfma_lds_64(g, m, rq, stream);
     if (m > 16 && !(n >= 8192 && k_pad <= 4096)) return launch_mfma_lds<8, 1, 4>(g, m, rq, stream);
     if (n >= 8192 && k_pad <= 4096) return launch_mfma_lds<8, 3, 4>(g, m, rq, stream);
     return launch_mfma_lds<8, 1, 8>(g, m, rq, stream);
@@ -921,8 +893,7 @@ int launch_gemv_dequant(const int8_t *a, int64_t lda, int m, int k, const Weight
   }
   GemvArgs g{a, lda, k / 16, wv.blocked, wv.ldw, wv.k_pad, n, reinterpret_cast<int8_t *>(c), ldc};
   const bool wide = n >= 8192 && wv.k_pad <= 4096;
-  if (m > 64) return launch_mfma_lds_deq_128(g, m, dq, stream);
-  if (m > 32) return wide ? launch_mfma_lds_deq_64<3>(g, m, dq, stream) : launch_mfma_lds_deq_64<1>(g, m, dq, stream);
+  if (m > 32) return launch_mfma_lds_deq_64(g, m, dq, stream);
   if (wide) return launch_mfma_lds_deq<8, 3, 4>(g, m, dq, stream);
   return m > 16 ? launch_mfma_lds_deq<8, 1, 4>(g, m, dq, stream) : launch_mfma_lds_deq<8, 1, 8>(g, m, dq, stream);
 }

@@ -117,3 +117,46 @@ def test_first_layer_convolution_windows(orc, kernel, ic, oc, asymmetric):
         flat = torch.zeros(x.size + 3, dtype=torch.int8, device="cuda")  # an image at an odd address
         flat[3:] = torch.from_numpy(x.reshape(-1)).cuda()
         assert np.array_equal(conv.run(flat[3:].view(x.shape)).cpu().numpy(), want), (kernel, ic, oc, ih, iw)
+
+
+def _matmul_pair(rng, n, k, asymmetric, dynamic, **kw):
+    w = rng.integers(-128, 128, (n, k), dtype=np.int8)
+    sw = rng.uniform(0.001, 0.01, n).astype(np.float32).astype(np.float64)
+    zw = rng.integers(-9, 10, n) if asymmetric else np.zeros(n, np.int64)
+    if dynamic:
+        zw[:] = zw[0]
+    qp = [K.QuantParam(float(s), int(z)) for s, z in zip(sw, zw)]
+    if dynamic:
+        bias = rng.standard_normal(n).astype(np.float32)
+        make = lambda pack: K.MatmulDynamicInt8Kernel(w, bias, qp, decode_pack=pack)
+    else:
+        bias = rng.integers(-5000, 5001, n).astype(np.int32)
+        make = lambda pack: K.MatmulInt8Kernel(w, bias, K.QuantParam(0.02, 7), qp,
+                                               K.QuantParam(float(np.float32(0.02 * 0.0055 * k ** 0.5 * 140)), 3), decode_pack=pack)
+    return w, bias, sw, zw.astype(np.int32), make
+
+
+# the rule picks, in this order: 64 x 64 (one K block, two, more than the ring is deep), 64 x 128, 128 x 128, 192 x 128 (the
+# last tile reaches past the packed weights), 128 x 256, 256 x 128, 192 x 256, 256 x 256 tiles
+@pytest.mark.parametrize("m,n,k", [(65, 250, 128), (65, 250, 144), (130, 200, 1040), (129, 257, 1000), (700, 2100, 160),
+                                   (700, 2101, 1025), (1000, 2500, 176), (1000, 2503, 1040), (513, 9003, 1040),
+                                   (1100, 6001, 1040), (300, 21000, 1040), (1201, 8302, 1100), (1500, 9000, 1030)])
+@pytest.mark.parametrize("dynamic,asymmetric", [(False, False), (False, True), (True, False), (True, True)])
+def test_matmul_tile_shapes(orc, m, n, k, dynamic, asymmetric):
+    """Against the oracle where that takes seconds at most, against the row-major kernels (which have tests of their own)
+    everywhere."""
+    import torch
+    rng = np.random.default_rng(m + n + k)
+    w, bias, sw, zw, make = _matmul_pair(rng, n, k, asymmetric, dynamic)
+    a = rng.integers(-128, 128, (m, k), dtype=np.int8)
+    dev = torch.from_numpy(a).cuda()
+    args = dict(in_quant=K.QuantParam(0.03, -5)) if dynamic else {}
+    got = make(True).run(dev, **args).cpu().numpy()
+    assert np.array_equal(got, make(False).run(dev, **args).cpu().numpy())
+    if m * n * k < 2e9:
+        orc.set_threads(16)
+        if dynamic:
+            want = orc.dynamic_matmul(a, w, bias, 0.03, -5, sw, zw)
+        else:
+            want = orc.matmul_int8(a, w, bias, 0.02, 7, sw, zw, float(np.float32(0.02 * 0.0055 * k ** 0.5 * 140)), 3)
+        assert np.array_equal(got, want)
