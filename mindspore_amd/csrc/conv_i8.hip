@@ -439,6 +439,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
       locate(tile + step);
       fetch(x);
     }
+    // The compiler keeps the distance that a matrix product's result needs before the next instruction reads it, but not
+    // where that instruction is inline assembly, as below: 19 wait states after a 16-pass product.
+    if constexpr (OCB == 1) asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc[0]));
+    if constexpr (OCB == 2) asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc[0]), "+v"(acc[1]));
     // acc[ob][4 * q + e] is pixel 8 * q + 4 * h + e of the tile, channel n0 + 32 * ob + r; after the transposition this
     // lane holds channels r & ~3 .. + 3 of pixel 8 * q + 4 * h + (lane & 3)
     const bool whole = first + 32 <= g.pixels && (g.out_c & 3) == 0;
