@@ -448,6 +448,7 @@ struct mi_conv {
   int fill = 0;
   RequantState st;
   DevBuf w16, dw_bias, dw_bias_folded, col_ws, h_in, h_out;
+  DevBuf dw_rows, dw_rows_par;  // the operands of launch_conv_dw_rows, or empty
   DevBuf w_rows;  // the weights of a convolution on few channels as launch_conv_rows takes them, or empty
   DevBuf fill16;  // 16 bytes of `fill`: where the gathering GEMM loader reads taps outside the image
 };
@@ -1004,6 +1005,39 @@ static int mi_conv_create_impl(const mi_conv_desc *d, const int8_t *weight_host,
           xmax + ((int64_t)1 << (e - 1)) + llabs((long long)d->out_zp) + 1 > INT32_MAX)
         h->dw_fast = false;
     }
+    // The four-taps-per-instruction kernel: int8 weights, and constants of the one-multiply rounding form that leave no
+    // type (the conditions of RequantParams::fast2, with the sum of the window in place of K products).
+    const ConvGeom shape{1, 16, 16, oc, 16, 16, oc, d->kernel_h, d->kernel_w, d->stride_h, d->stride_w, d->dilation_h, d->dilation_w,
+                         d->pad_u, d->pad_l};
+    bool rows = h->dw_fast && conv_dw_rows_supported(shape);
+    std::vector<int8_t> w8(rows ? (size_t)plane * oc : 0);
+    std::vector<int32_t> par(rows ? (size_t)5 * oc : 0);
+    for (int c = 0; c < oc && rows; ++c) {
+      int64_t wsum = 0;
+      for (int t = 0; t < plane; ++t) {
+        const int16_t v = w16[(size_t)t * oc + c];
+        if (v < -128 || v > 127) rows = false;
+        w8[(size_t)c * plane + t] = (int8_t)v;
+        wsum += v;
+      }
+      const int32_t mult = h->st.h_mult[c], e = std::min(31, -h->st.h_rs[c]);
+      const int64_t folded = (int64_t)b[c] - (int64_t)zx8 * wsum, vmax = (int64_t)plane * 255 * 255 + llabs((long long)b[c]);
+      const int64_t xmax = ((vmax * llabs((long long)mult)) >> 31) + 1;
+      if (!rows || mult < 0 || llabs((long long)folded) >= ((int64_t)1 << 31) - 1 ||
+          xmax + ((int64_t)1 << (e - 1)) + (llabs((long long)d->out_zp) << e) > INT32_MAX) {
+        rows = false;
+        break;
+      }
+      const uint64_t c2 = (uint64_t)(2 * (folded - (int64_t)kAccBias)) * (uint64_t)(int64_t)mult + ((uint64_t)1 << 31);
+      if ((int64_t)c2 >= 0) rows = false;
+      par[c] = (int32_t)((uint32_t)mult << 1);
+      par[(size_t)oc + c] = (int32_t)(uint32_t)c2;
+      par[(size_t)2 * oc + c] = (int32_t)(c2 >> 32);
+      par[(size_t)3 * oc + c] = (int32_t)(((uint32_t)1 << (e - 1)) + ((uint32_t)d->out_zp << e) - 1u);
+      par[(size_t)4 * oc + c] = e;
+    }
+    if (rows && rc == MI_OK) rc = upload(&h->dw_rows, conv_dw_rows_weights(w8.data(), oc, d->kernel_h));
+    if (rows && rc == MI_OK) rc = upload(&h->dw_rows_par, par);
     if (rc == MI_OK) rc = upload(&h->w16, w16);
     if (rc == MI_OK) rc = upload(&h->dw_bias, b);
     if (rc == MI_OK) rc = upload(&h->dw_bias_folded, bf);
@@ -1081,6 +1115,11 @@ int mi_conv_run(mi_conv *h, const int8_t *in_dev, int32_t batch, int32_t in_h, i
     return MI_PARAM_INVALID;
   }
   if (h->depthwise) {
+    if (h->dw_rows_par.p != nullptr && conv_dw_rows_supported(g) &&
+        ((reinterpret_cast<uintptr_t>(in_dev) | reinterpret_cast<uintptr_t>(out_dev)) & 3) == 0)
+      return launch_conv_dw_rows(in_dev, g, static_cast<const int32_t *>(h->dw_rows.p),
+                                 static_cast<const int32_t *>(h->dw_rows_par.p), (int)(int8_t)d.in_zp, h->st.amin, h->st.amax,
+                                 out_dev, s);
     RequantParams rq = h->st.params();
     rq.fast = h->dw_fast ? 1 : 0;
     return launch_conv_dw(in_dev, g, static_cast<const int16_t *>(h->w16.p), static_cast<const int32_t *>(h->dw_bias.p),

@@ -152,6 +152,13 @@ int launch_conv_rows(const int8_t *in, const ConvGeom &g, int fill, const int8_t
 // rounding form exact for every channel.
 int launch_conv_dw(const int8_t *in, const ConvGeom &g, const int16_t *w16, const int32_t *bias,
                    const int32_t *bias_folded, int zx8, const RequantParams &rq, int8_t *out, hipStream_t stream);
+// The same with stride 1, a 3x3 or 5x5 window, int8 weights and out_c % 4 == 0 (in and out 4-byte aligned); w: the weights as
+// conv_dw_rows_weights lays them out, par: {mult2, c2lo, c2hi, pre, shift}[out_c] of the one-multiply rounding form
+// (RequantParams::fast2) with the bias of bias_folded.
+bool conv_dw_rows_supported(const ConvGeom &g);
+std::vector<int32_t> conv_dw_rows_weights(const int8_t *w, int ch, int ks);
+int launch_conv_dw_rows(const int8_t *in, const ConvGeom &g, const int32_t *w, const int32_t *par, int zx8, int amin, int amax,
+                        int8_t *out, hipStream_t stream);
 
 // The requantising GEMM with its activation operand gathered from an NHWC image (in_c % 16 == 0): the im2col
 // convolution without the buffer.  fill16: 16 bytes of the value out-of-image taps take, in device memory.

@@ -568,6 +568,214 @@ int launch_conv_rows(const int8_t *in, const ConvGeom &g, int fill, const int8_t
   return MI_OK;
 }
 
+// Stride-1 depthwise convolutions with a 3x3 or 5x5 window, int8 weights (no weight zero point) and C % 4 == 0.
+// A thread computes four channels of a tile of 4 x OT output pixels.  The byte products are taken four at a time along
+// the window row with v_dot4: the dwords of neighbouring pixels (four channels each) are transposed so that a dword holds
+// four neighbouring pixels of ONE channel, and an output at an odd position takes the window that starts one pixel before
+// it, against weights moved up by one byte.  An image row is fetched and transposed once for the up to KS output rows it
+// belongs to.  Accumulators start from kAccBias and are requantised with one 64-bit multiply-add (RequantParams::fast2).
+// Bound by the vector ALU at large sizes (3x3: about 10 instructions per output, half of them the requantisation; one
+// multiply per product and an unpacking instruction for each operand took about 30), by latency at one image.  us per launch,
+// before (conv_dw16_kernel below) -> now: 3x3, 16 x 112 x 112 x 192 70.1 -> 22.1 (3.5 TB/s), one such image 8.6 -> 4.8; 5x5,
+// 4 x 80 x 80 x 72 16.4 -> 6.0, 1 x 64 x 64 x 64 7.1 -> 4.1.
+struct ConvDwRows {
+  const int8_t *in;
+  const int32_t *w;    // [KS * (KS == 3 ? 1 : 3)][C]: bytes w0..w2 0 of a window row; 5x5: w0..w3, w4 0 0 0, w3 w4 0 0
+  const int32_t *par;  // [5][C]: mult2, c2lo, c2hi, pre, shift
+  int8_t *out;
+  int in_h, in_w, ch, out_h, out_w, pad_u, pad_l;
+  int groups, strips, bands;  // channels / 4, output columns / 4, output rows / OT, rounded up
+  int total;                  // batch * bands * strips * groups
+  int zsplat, amin, amax;
+};
+
+template <int KS, int OT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void conv_dw_rows_kernel(ConvDwRows g) {
+  constexpr int PX = KS + 3;       // input pixels per row of four outputs
+  constexpr int WR = KS == 3 ? 1 : 3;  // weight dwords per channel and window row
+  // as below: workgroups that share an XCD get one contiguous band of the output
+  int bid = blockIdx.x;
+  const int per = gridDim.x >> 3;
+  if (bid < per * 8) bid = (bid & 7) * per + (bid >> 3);
+  const int idx = bid * 256 + threadIdx.x;
+  if (idx >= g.total) return;
+  uint32_t rest = (uint32_t)idx / (uint32_t)g.groups;
+  const int c0 = (idx - (int)rest * g.groups) * 4;
+  uint32_t up = rest / (uint32_t)g.strips;
+  const int ow0 = (int)(rest - up * g.strips) * 4;
+  const int b = (int)(up / (uint32_t)g.bands), oh0 = (int)(up - b * g.bands) * OT;
+  const int ih0 = oh0 - g.pad_u, iw0 = ow0 - g.pad_l;
+  const int line = g.in_w * g.ch;
+
+  uint32_t px[OT + KS - 1][PX];
+  const int8_t *img = g.in + (int64_t)b * g.in_h * line + c0;
+  const bool inside = ih0 >= 0 && iw0 >= 0 && ih0 + OT + KS - 2 < g.in_h && iw0 + PX <= g.in_w;
+  if (__all(inside)) {
+    const int8_t *row = img + (int64_t)ih0 * line + iw0 * g.ch;
+#pragma unroll
+    for (int i = 0; i < OT + KS - 1; ++i)
+#pragma unroll
+      for (int j = 0; j < PX; ++j) px[i][j] = *reinterpret_cast<const uint32_t *>(row + i * line + j * g.ch);
+  } else {  // (every load is inside the tensor; what lies outside the image is replaced by the input zero point)
+#pragma unroll
+    for (int i = 0; i < OT + KS - 1; ++i) {
+      const int ih = ih0 + i, ihc = min(max(ih, 0), g.in_h - 1);
+#pragma unroll
+      for (int j = 0; j < PX; ++j) {
+        const int iw = iw0 + j, iwc = min(max(iw, 0), g.in_w - 1);
+        px[i][j] = *reinterpret_cast<const uint32_t *>(img + ihc * line + iwc * g.ch);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < OT + KS - 1; ++i)
+#pragma unroll
+      for (int j = 0; j < PX; ++j)
+        if (ih0 + i != min(max(ih0 + i, 0), g.in_h - 1) || iw0 + j != min(max(iw0 + j, 0), g.in_w - 1))
+          px[i][j] = (uint32_t)g.zsplat;
+  }
+
+  v4i acc[OT][4];  // [row][column], four channels
+#pragma unroll
+  for (int o = 0; o < OT; ++o)
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[o][x][c] = (int)kAccBias;
+  v4i w[KS][WR];
+#pragma unroll
+  for (int k = 0; k < KS; ++k)
+#pragma unroll
+    for (int p = 0; p < WR; ++p) w[k][p] = *reinterpret_cast<const v4i *>(g.w + (int64_t)(k * WR + p) * g.ch + c0);
+  v4i par[5];
+#pragma unroll
+  for (int a = 0; a < 5; ++a) par[a] = *reinterpret_cast<const v4i *>(g.par + (int64_t)a * g.ch + c0);
+
+#pragma unroll
+  for (int i = 0; i < OT + KS - 1; ++i) {
+    uint32_t lo[PX / 2], hi[PX / 2];  // pixel pairs: bytes a0 b0 a1 b1 / a2 b2 a3 b3
+#pragma unroll
+    for (int t = 0; t < PX / 2; ++t) {
+      lo[t] = __builtin_amdgcn_perm(px[i][2 * t + 1], px[i][2 * t], 0x05010400u);
+      hi[t] = __builtin_amdgcn_perm(px[i][2 * t + 1], px[i][2 * t], 0x07030602u);
+    }
+    int win[PX / 2 - 1][4];  // [first pixel / 2][channel]: four pixels of a channel
+#pragma unroll
+    for (int t = 0; t < PX / 2 - 1; ++t) {
+      win[t][0] = (int)__builtin_amdgcn_perm(lo[t + 1], lo[t], 0x05040100u);
+      win[t][1] = (int)__builtin_amdgcn_perm(lo[t + 1], lo[t], 0x07060302u);
+      win[t][2] = (int)__builtin_amdgcn_perm(hi[t + 1], hi[t], 0x05040100u);
+      win[t][3] = (int)__builtin_amdgcn_perm(hi[t + 1], hi[t], 0x07060302u);
+    }
+#pragma unroll
+    for (int o = 0; o < OT; ++o) {
+      const int k = i - o;
+      if (k < 0 || k >= KS) continue;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int w0 = w[k][0][c], w1 = (int)((uint32_t)w0 << 8);
+        acc[o][0][c] = __builtin_amdgcn_sdot4(win[0][c], w0, acc[o][0][c], false);
+        acc[o][1][c] = __builtin_amdgcn_sdot4(win[0][c], w1, acc[o][1][c], false);
+        acc[o][2][c] = __builtin_amdgcn_sdot4(win[1][c], w0, acc[o][2][c], false);
+        acc[o][3][c] = __builtin_amdgcn_sdot4(win[1][c], w1, acc[o][3][c], false);
+        if constexpr (KS == 5) {  // the window's last pixels: columns 4..7 hold what the first windows left out
+          const int e = w[k][1][c], d = w[k][2][c];
+          acc[o][0][c] = __builtin_amdgcn_sdot4(win[2][c], e, acc[o][0][c], false);
+          acc[o][1][c] = __builtin_amdgcn_sdot4(win[2][c], d, acc[o][1][c], false);
+          acc[o][2][c] = __builtin_amdgcn_sdot4(win[2][c], (int)((uint32_t)e << 16), acc[o][2][c], false);
+          acc[o][3][c] = __builtin_amdgcn_sdot4(win[2][c], (int)((uint32_t)d << 16), acc[o][3][c], false);
+        }
+      }
+    }
+  }
+
+  int amin_v = g.amin, amax_v = g.amax;
+  asm volatile("" : "+v"(amin_v), "+v"(amax_v));  // kept in vector registers, as v_med3 wants them
+  // (a dot product's result needs three wait states before another instruction reads it; the compiler keeps them, but not
+  //  where that instruction is inline assembly)
+#pragma unroll
+  for (int o = 0; o < OT; ++o) asm volatile("s_nop 3" : "+v"(acc[o][0]), "+v"(acc[o][1]), "+v"(acc[o][2]), "+v"(acc[o][3]));
+  int8_t *dst = g.out + (((int64_t)b * g.out_h + oh0) * g.out_w + ow0) * g.ch + c0;
+#pragma unroll
+  for (int o = 0; o < OT; ++o)
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      int y[4];
+      uint64_t p2[4], carry[4], unused;
+      int32_t t[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const uint64_t c2 = (uint64_t)(uint32_t)par[2][c] << 32 | (uint32_t)par[1][c];
+        asm("v_mad_u64_u32 %0, %1, %2, %3, %4" : "=&v"(p2[c]), "=s"(carry[c]) : "v"(acc[o][x][c]), "v"(par[0][c]), "v"(c2));
+      }
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        asm("v_addc_co_u32_e64 %0, %1, %2, %3, %4"
+            : "=v"(t[c]), "=s"(unused)
+            : "v"((int32_t)(p2[c] >> 32)), "v"(par[3][c]), "s"(carry[c]));
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        t[c] >>= par[4][c];
+        asm("v_med3_i32 %0, %1, %2, %3" : "=v"(y[c]) : "v"(t[c]), "v"(amin_v), "v"(amax_v));
+      }
+      const uint32_t p01 = __builtin_amdgcn_perm((uint32_t)y[1], (uint32_t)y[0], 0x0c0c0400u);
+      const uint32_t p23 = __builtin_amdgcn_perm((uint32_t)y[3], (uint32_t)y[2], 0x0c0c0400u);
+      if (oh0 + o < g.out_h && ow0 + x < g.out_w)
+        *reinterpret_cast<uint32_t *>(dst + ((int64_t)o * g.out_w + x) * g.ch) = __builtin_amdgcn_perm(p23, p01, 0x05040100u);
+    }
+}
+
+bool conv_dw_rows_supported(const ConvGeom &g) {
+  return (g.kernel_h == 3 || g.kernel_h == 5) && g.kernel_w == g.kernel_h && g.stride_h == 1 && g.stride_w == 1 &&
+         g.dilation_h == 1 && g.dilation_w == 1 && (g.out_c & 3) == 0 &&
+         (int64_t)g.in_h * g.in_w * g.out_c < (int64_t)1 << 31 &&
+         (int64_t)g.batch * g.out_h * ((g.out_w + 3) / 4) * (g.out_c / 4) < ((int64_t)1 << 31) - 256;
+}
+
+// Weights [C][KS][KS] -> the dwords of ConvDwRows::w.
+std::vector<int32_t> conv_dw_rows_weights(const int8_t *w, int ch, int ks) {
+  const int wr = ks == 3 ? 1 : 3;
+  std::vector<int32_t> out((size_t)ks * wr * ch);
+  for (int c = 0; c < ch; ++c)
+    for (int k = 0; k < ks; ++k) {
+      const int8_t *row = w + ((size_t)c * ks + k) * ks;
+      uint8_t d[3][4] = {};
+      for (int i = 0; i < (ks < 4 ? ks : 4); ++i) d[0][i] = (uint8_t)row[i];
+      if (ks == 5) d[1][0] = (uint8_t)row[4], d[2][0] = (uint8_t)row[3], d[2][1] = (uint8_t)row[4];
+      for (int p = 0; p < wr; ++p) memcpy(&out[(size_t)(k * wr + p) * ch + c], d[p], 4);
+    }
+  return out;
+}
+
+template <int KS, int OT>
+static int launch_dw_rows(ConvDwRows c, int batch, hipStream_t stream) {
+  c.bands = (c.out_h + OT - 1) / OT;
+  c.total = batch * c.bands * c.strips * c.groups;
+  hipLaunchKernelGGL((conv_dw_rows_kernel<KS, OT>), dim3((c.total + 255) / 256), dim3(256), 0, stream, c);
+  MI_HIP_CHECK(hipGetLastError());
+  return MI_OK;
+}
+
+int launch_conv_dw_rows(const int8_t *in, const ConvGeom &g, const int32_t *w, const int32_t *par, int zx8, int amin, int amax,
+                        int8_t *out, hipStream_t stream) {
+  if (!conv_dw_rows_supported(g) || ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 3) != 0) {
+    set_error("conv_dw_rows: unsupported geometry");
+    return MI_PARAM_INVALID;
+  }
+  ConvDwRows c{in,      w,       par,     out,     g.in_h,      g.in_w, g.out_c, g.out_h, g.out_w,
+               g.pad_u, g.pad_l, g.out_c / 4, (g.out_w + 3) / 4, 0,      0,       (zx8 & 0xff) * 0x01010101, amin, amax};
+  // Tall tiles fetch and transpose fewer rows twice, flat ones make more threads.  us at one / two / four / eight rows: 3x3,
+  // 1 x 112 x 112 x 192 4.8, 5.3, 5.5, 7.6; 8 x 115 x 115 x 240 20.3, 17.8, 17.1, 19.6; 16 x 112 x 112 x 192 28.2, 23.5, 22.1,
+  // 23.8; 5x5, 1 x 64 x 64 x 64 4.1, 4.9, 6.4; 4 x 80 x 80 x 72 6.4, 6.0, 7.6.
+  const int64_t flat = (int64_t)g.batch * g.out_h * c.strips * c.groups;  // threads at one row each
+  if (g.kernel_h == 3) {
+    if (flat >= 1 << 20) return launch_dw_rows<3, 4>(c, g.batch, stream);
+    if (flat >= 1 << 18) return launch_dw_rows<3, 2>(c, g.batch, stream);
+    return launch_dw_rows<3, 1>(c, g.batch, stream);
+  }
+  if (flat >= 1 << 16) return launch_dw_rows<5, 2>(c, g.batch, stream);
+  return launch_dw_rows<5, 1>(c, g.batch, stream);
+}
+
 __global__ __launch_bounds__(256) void conv_dw_kernel(const int8_t *__restrict__ in, ConvGeom g,
                                                       const int16_t *__restrict__ w16,
                                                       const int32_t *__restrict__ bias, int zx8, RequantParams rq,

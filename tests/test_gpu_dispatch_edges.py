@@ -160,3 +160,20 @@ def test_matmul_tile_shapes(orc, m, n, k, dynamic, asymmetric):
         else:
             want = orc.matmul_int8(a, w, bias, 0.02, 7, sw, zw, float(np.float32(0.02 * 0.0055 * k ** 0.5 * 140)), 3)
         assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("taps", [3, 5])
+@pytest.mark.parametrize("b,ih,iw,ch,pad", [(1, 5, 5, 4, (0, 0, 0, 0)), (1, 5, 6, 8, (1, 1, 1, 1)), (2, 7, 9, 12, (2, 0, 0, 2)),
+                                            (1, 9, 11, 20, (4, 4, 4, 4)), (3, 6, 8, 192, (1, 2, 3, 0)), (1, 33, 31, 36, (1, 1, 1, 1)),
+                                            (4, 61, 53, 192, (1, 1, 1, 1)), (9, 70, 127, 96, (2, 2, 2, 2)),
+                                            (16, 75, 77, 192, (1, 1, 1, 1))])
+def test_depthwise_stride_one_tiles(orc, b, ih, iw, ch, pad, taps):
+    """Partial tiles on either side, windows that reach over every border, one, two and four output rows per thread."""
+    from tests.test_gpu_parity import _conv_case, _gpu_conv
+    rng = np.random.default_rng(ih * iw + taps)
+    orc.set_threads(16)
+    for act in (0, 3):
+        case = _conv_case(rng, b, ih, iw, ch, ch, (taps, taps), (1, 1), (1, 1), pad, True, False, True, act, dw=True)
+        case["w"].reshape(ch, -1)[:2] = -128  # the largest products
+        got = _gpu_conv(case, (1, 1), (1, 1), pad, ch, device_tensors=True)
+        assert np.array_equal(got, orc.conv_dw_int8(**case)), act
