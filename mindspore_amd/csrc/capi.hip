@@ -450,6 +450,7 @@ struct mi_conv {
   DevBuf w16, dw_bias, dw_bias_folded, col_ws, h_in, h_out;
   DevBuf dw_rows, dw_rows_par;  // the operands of launch_conv_dw_rows, or empty
   DevBuf w_rows;  // the weights of a convolution on few channels as launch_conv_rows takes them, or empty
+  DevBuf w_thin;  // the weights of a 1x1 on few channels as launch_conv_thin takes them, or empty
   DevBuf fill16;  // 16 bytes of `fill`: where the gathering GEMM loader reads taps outside the image
 };
 
@@ -1050,9 +1051,13 @@ static int mi_conv_create_impl(const mi_conv_desc *d, const int8_t *weight_host,
     h->fill = is_1x1 ? 0 : d->in_zp;
     rc = h->st.build(weight_host, oc, kdim, bias_host, d->in_scale, d->in_zp, d->out_scale, d->out_zp,
                      d->filter_quant_num, d->filter_scales, d->filter_zps, d->act_type, true);
-    if (rc == MI_OK && conv_rows_supported(ConvGeom{1, 16, 16, d->in_channel, 1, 1, oc, d->kernel_h, d->kernel_w, d->stride_h,
-                                                    d->stride_w, d->dilation_h, d->dilation_w, d->pad_u, d->pad_l}))
+    const ConvGeom shape{1, 16, 16, d->in_channel, 1, 1, oc, d->kernel_h, d->kernel_w, d->stride_h, d->stride_w, d->dilation_h,
+                         d->dilation_w, d->pad_u, d->pad_l};
+    if (rc == MI_OK && !h->direct_1x1 && conv_rows_supported(shape)) {
       rc = upload(&h->w_rows, conv_rows_weights(weight_host, oc, d->kernel_h, d->kernel_w, d->in_channel));
+    } else if (rc == MI_OK && h->direct_1x1 && conv_thin_supported(kdim, oc)) {
+      rc = upload(&h->w_thin, conv_thin_weights(weight_host, oc, kdim));
+    }
     if (rc == MI_OK) rc = upload(&h->fill16, std::vector<int8_t>(16, (int8_t)h->fill));
   }
   if (rc != MI_OK) {
@@ -1129,7 +1134,9 @@ int mi_conv_run(mi_conv *h, const int8_t *in_dev, int32_t batch, int32_t in_h, i
   const int8_t *a = nullptr;
   int64_t lda = 0;
   int k16 = 0;
-  if (h->direct_1x1) {
+  if (h->w_thin.p != nullptr && pixels > 128 && pixels <= kConvThinMostPixels) {
+    return launch_conv_thin(in_dev, pixels, k, d.out_channel, static_cast<const int8_t *>(h->w_thin.p), h->st.params(), out_dev, s);
+  } else if (h->direct_1x1) {
     if ((rc = prepare_rows(in_dev, (int)pixels, k, Workspace::growable(&h->col_ws), s, &a, &lda, &k16)) != MI_OK) return rc;
   } else if (h->w_rows.p != nullptr && conv_rows_supported(g)) {
     // a first-layer convolution: window rows straight from the image

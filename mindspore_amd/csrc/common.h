@@ -147,6 +147,13 @@ bool conv_rows_supported(const ConvGeom &g);
 std::vector<int8_t> conv_rows_weights(const int8_t *w, int oc, int kernel_h, int kernel_w, int in_c);
 int launch_conv_rows(const int8_t *in, const ConvGeom &g, int fill, const int8_t *w, const RequantParams &rq, int8_t *out,
                      hipStream_t stream);
+// 1x1 convolution (stride 1, no padding) of a short contraction against few output channels, any alignment, pixels * k >= 16;
+// w: the weights as conv_thin_weights lays them out, in device memory.
+constexpr int64_t kConvThinMostPixels = 0x7fffffff - 65536;
+bool conv_thin_supported(int k, int oc);
+std::vector<int8_t> conv_thin_weights(const int8_t *w, int oc, int k);
+int launch_conv_thin(const int8_t *in, int64_t pixels, int k, int oc, const int8_t *w, const RequantParams &rq, int8_t *out,
+                     hipStream_t stream);
 // Depthwise conv + requantisation, weights pre-offset to int16 [KH*KW][C].  bias_folded = bias - zx8 * sum_t w16[t][c]
 // (used by the channel-vectorised kernel, which reads out-of-image taps as zx8); rq.fast: the host proved the cheap
 // rounding form exact for every channel.

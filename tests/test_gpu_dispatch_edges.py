@@ -177,3 +177,20 @@ def test_depthwise_stride_one_tiles(orc, b, ih, iw, ch, pad, taps):
         case["w"].reshape(ch, -1)[:2] = -128  # the largest products
         got = _gpu_conv(case, (1, 1), (1, 1), pad, ch, device_tensors=True)
         assert np.array_equal(got, orc.conv_dw_int8(**case)), act
+
+
+@pytest.mark.parametrize("b,ih,iw,ic,oc", [(1, 12, 11, 1, 5),  # one byte of K, the tensor's end inside many loads
+                                           (1, 13, 10, 15, 33), (2, 9, 9, 24, 144), (1, 40, 33, 32, 192), (3, 21, 19, 100, 31),
+                                           (1, 30, 30, 240, 40), (1, 17, 17, 480, 256), (1, 13, 10, 1024, 64),
+                                           (9, 130, 131, 16, 96)])  # several tiles per wave
+def test_conv_1x1_few_channels(orc, b, ih, iw, ic, oc):
+    """Contractions and channel counts around the batches of steps and the blocks of channels, with and without weight zero
+    points, per-tensor and per-channel scales."""
+    from tests.test_gpu_parity import _conv_case, _gpu_conv
+    rng = np.random.default_rng(ih * iw + oc)
+    orc.set_threads(16)
+    pad = (0, 0, 0, 0)
+    for it in range(3):
+        case = _conv_case(rng, b, ih, iw, ic, oc, (1, 1), (1, 1), (1, 1), pad, it != 1, it == 1, it != 2, [0, 1, 3][it])
+        got = _gpu_conv(case, (1, 1), (1, 1), pad, 1, device_tensors=True)
+        assert np.array_equal(got, orc.conv_int8(**case)), it
