@@ -33,7 +33,7 @@ struct ConvThin {
   int k;       // contraction bytes
   int chunks;  // of CH steps; weights are zero from k on
   int out_c, pixels;
-  const int8_t *w;  // [channel block of OCB x 32][step][OCB][lane][16]
+  const int8_t *w;  // [32 channels][step][lane][16]
 };
 
 __device__ __forceinline__ uint32_t thin_quad_transpose(uint32_t d, uint32_t sel1, uint32_t sel2) {
@@ -93,10 +93,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
   };
 
   {
-    const v4i *src = reinterpret_cast<const v4i *>(g.w + (int64_t)blockIdx.y * steps * OCB * 1024);
+    const v4i *src = reinterpret_cast<const v4i *>(g.w + (int64_t)(n0 / 32) * steps * 1024);
+    const int have = min(OCB, (g.out_c - n0 + 31) / 32) * steps * 64;  // (the last group of blocks may reach past the weights)
     v4i *dst = reinterpret_cast<v4i *>(lds);
 #pragma unroll 4
-    for (int i = tid; i < steps * OCB * 64; i += 256) dst[i] = src[i];
+    for (int i = tid; i < have; i += 256) dst[i] = src[i];
     __syncthreads();
   }
   if (tile >= tiles) return;
@@ -132,12 +133,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
         locate(tile + step);
         fetch(x, 0);
       }
-      const char *wl = lds + c * CH * OCB * 1024 + lane * 16;
+      const char *wl = lds + c * CH * 1024 + lane * 16;
 #pragma unroll
       for (int s = 0; s < CH; ++s)
 #pragma unroll
         for (int ob = 0; ob < OCB; ++ob)
-          acc[ob] = __builtin_amdgcn_mfma_i32_32x32x32_i8(y[s], *reinterpret_cast<const v4i *>(wl + (s * OCB + ob) * 1024),
+          acc[ob] = __builtin_amdgcn_mfma_i32_32x32x32_i8(y[s], *reinterpret_cast<const v4i *>(wl + (ob * steps + s) * 1024),
                                                           acc[ob], 0, 0, 0);
       if (!FAST && rq.has_zw) {  // the pixels' input sums, in the accumulators' layout: against ones up to K
 #pragma unroll
@@ -211,38 +212,45 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
   }
 }
 
-// How a contraction of k bytes and oc channels is cut: the number of steps per batch of loads that pads least (and of those
-// the largest), two or three blocks of 32 channels per workgroup, whichever pads less.
+// How a contraction of k bytes is cut: the number of steps per batch of loads that pads least (of those the largest).
 struct ThinCut {
-  int ch, chunks, ocb, nblocks;
+  int ch, chunks;
+  int steps() const { return ch * chunks; }
 };
-static ThinCut thin_cut(int k, int oc) {
-  const int steps = (k + 31) / 32, blocks = (oc + 31) / 32;
-  ThinCut t{0, 0, 0, 0};
+static ThinCut thin_cut(int k) {
+  const int steps = (k + 31) / 32;
+  ThinCut t{0, 0};
   for (int ch = 4; ch > 0; --ch) {
     const int chunks = (steps + ch - 1) / ch;
-    if (t.ch == 0 || chunks * ch < t.chunks * t.ch) t.ch = ch, t.chunks = chunks;
+    if (t.ch == 0 || chunks * ch < t.steps()) t.ch = ch, t.chunks = chunks;
   }
-  t.ocb = blocks == 1 ? 1 : (blocks + 2) / 3 * 3 <= (blocks + 1) / 2 * 2 ? 3 : 2;
-  t.nblocks = (blocks + t.ocb - 1) / t.ocb;
   return t;
 }
-
-static size_t thin_lds_bytes(const ThinCut &t) { return (size_t)t.chunks * t.ch * t.ocb * 1024; }
+// Blocks of 32 channels per workgroup: two or three, whichever pads less, so that a pixel's bytes serve 64 or 96 channels;
+// one as long as a CU then gets no more than four workgroups, all of them at once: what such a launch lasts is one wave's chain of
+// requantisations.  us at three blocks / one: 1 x 112 x 112, 32 -> 192 channels (588 workgroups of one block) 4.8 / 4.2;
+// 4 x 80 x 80, 24 -> 72 (600) 4.6 / 3.8; at two / one: 1 x 64 x 64, 16 -> 64 (64) 3.8 / 3.1, and 8 x 115 x 115, 240 -> 40 (1654)
+// 9.4 / 11.2.
+static int thin_blocks(int64_t wgs, int oc) {
+  const int blocks = (oc + 31) / 32;
+  if (blocks == 1 || wgs * blocks <= 1024) return 1;
+  return (blocks + 2) / 3 * 3 <= (blocks + 1) / 2 * 2 ? 3 : 2;
+}
 
 // Weights that leave a CU's LDS room for two workgroups or more, and few enough channels that re-reading the image for every
 // 64 or 96 of them stays in the caches.
-bool conv_thin_supported(int k, int oc) { return k <= 1024 && oc <= 256 && thin_lds_bytes(thin_cut(k, oc)) <= 64 * 1024; }
+bool conv_thin_supported(int k, int oc) {
+  return k <= 1024 && oc <= 256 && thin_cut(k).steps() * 1024 * thin_blocks((int64_t)1 << 30, oc) <= 64 * 1024;
+}
 
 // Weights [oc][k] -> ConvThin::w.
 std::vector<int8_t> conv_thin_weights(const int8_t *w, int oc, int k) {
-  const ThinCut t = thin_cut(k, oc);
-  const int steps = t.ch * t.chunks;
-  std::vector<int8_t> out((size_t)t.nblocks * steps * t.ocb * 1024, 0);
+  const int steps = thin_cut(k).steps();
+  std::vector<int8_t> out((size_t)((oc + 31) / 32) * steps * 1024, 0);
   for (int n = 0; n < oc; ++n)
     for (int k0 = 0; k0 < k; k0 += 16) {
-      const int blk = n / (32 * t.ocb), ob = n / 32 % t.ocb, lane = n % 32 + 32 * (k0 / 16 % 2);
-      memcpy(&out[((((size_t)blk * steps + k0 / 32) * t.ocb + ob) * 64 + lane) * 16], w + (size_t)n * k + k0,
+      const int lane = n % 32 + 32 * (k0 / 16 % 2);
+      memcpy(&out[(((size_t)(n / 32) * steps + k0 / 32) * 64 + lane) * 16], w + (size_t)n * k + k0,
              (size_t)(k - k0 < 16 ? k - k0 : 16));
     }
   return out;
@@ -265,17 +273,18 @@ int launch_conv_thin(const int8_t *in, int64_t pixels, int k, int oc, const int8
     set_error("conv_thin: unsupported geometry k=%d oc=%d pixels=%lld", k, oc, (long long)pixels);
     return MI_PARAM_INVALID;
   }
-  const ThinCut t = thin_cut(k, oc);
+  const ThinCut t = thin_cut(k);
   const ConvThin c{in, pixels * k, k, t.chunks, oc, (int)pixels, w};
-  // four workgroups per CU, which the LDS allows up to 40 KiB of weights; more would only load the weights more often
   const int64_t wgs = (pixels + 127) / 128;
-  const int most = (1024 + t.nblocks - 1) / t.nblocks;
-  const dim3 grid((unsigned)(wgs < most ? wgs : most), (unsigned)t.nblocks);
-  const size_t lds = thin_lds_bytes(t);
-#define MI_THIN(CH)                                                                 \
-  return t.ocb == 1   ? launch_thin<CH, 1>(c, rq, out, grid, lds, stream)           \
-         : t.ocb == 2 ? launch_thin<CH, 2>(c, rq, out, grid, lds, stream)           \
-                      : launch_thin<CH, 3>(c, rq, out, grid, lds, stream)
+  const int ocb = thin_blocks(wgs, oc), groups = (oc + 32 * ocb - 1) / (32 * ocb);
+  // four workgroups per CU, which the LDS allows up to 40 KiB of weights; more would only load the weights more often
+  const int most = (1024 + groups - 1) / groups;
+  const dim3 grid((unsigned)(wgs < most ? wgs : most), (unsigned)groups);
+  const size_t lds = (size_t)t.steps() * ocb * 1024;
+#define MI_THIN(CH)                                                              \
+  return ocb == 1   ? launch_thin<CH, 1>(c, rq, out, grid, lds, stream)          \
+         : ocb == 2 ? launch_thin<CH, 2>(c, rq, out, grid, lds, stream)          \
+                    : launch_thin<CH, 3>(c, rq, out, grid, lds, stream)
   switch (t.ch) {
     case 1: MI_THIN(1);
     case 2: MI_THIN(2);
