@@ -13,8 +13,12 @@ namespace mi {
 // need holds further stages instead.  Everything else is as above: four quarters per block, double-buffered fragments,
 // one barrier per block between quarter three and four; the loads of block b + S - 1 are spread over quarters 1 to 3 of
 // block b and quarter 4 of the block before, which is the first moment its stage is free.
+// Bound by the loads, where weights come from HBM: without its MFMAs the loop takes as long (512 x 12288 x 4096 29.8 of 30.1 us), with
+// the weights in the caches 17; a CU gets 50 to 60 GB/s, whatever the number of CUs and of bytes in flight beyond 100 KiB, since
+// its loads return in order, the activations' L2 hits behind the weights' misses.
+// STREAM: weight loads carry the non-temporal hint (see launch_ring).
 // =====================================================================================================================
-template <int TN, int TM, int S, int EPI, bool HAS_ZW, bool FAST>
+template <int TN, int TM, int S, int EPI, bool HAS_ZW, bool FAST, bool STREAM>
 __device__ __forceinline__ void gemm_ring_body(const GemmArgs &g, const RequantParams &rq, const DequantParams &dq) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the buffer-resource type exists in the device pass only; the host pass needs just the stub
   constexpr int TILE_N = 64 * TN, TILE_M = 64 * TM, KB = 128;
@@ -76,7 +80,7 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs &g, const RequantP
     for (int l = from; l < to; ++l) {
       if (l < 2 * TN) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, lds_ptr(sw + l * 1024), 16, lane * 16,
-                                                 ((l >> 1) * k64 + 2 * kb + (l & 1)) * 1024, 0, 0);
+                                                 ((l >> 1) * k64 + 2 * kb + (l & 1)) * 1024, 0, STREAM ? 2 : 0);
       } else {
         const int i = l - 2 * TN;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, lds_ptr(sa + i * 1024), 16, a_voff[i], kb * KB, 0, 0);
@@ -227,19 +231,30 @@ constexpr int ring_occupancy() {
   return 8 * (TN + TM) * S * 2 <= 160 ? 2 : 1;
 }
 
-template <int TN, int TM, int S, int EPI, bool HAS_ZW, bool FAST>
+template <int TN, int TM, int S, int EPI, bool HAS_ZW, bool FAST, bool STREAM>
 __global__ __launch_bounds__(256)
     __attribute__((amdgpu_waves_per_eu(ring_occupancy<TN, TM, S>(), ring_occupancy<TN, TM, S>()))) void gemm_ring_kernel(
         GemmArgs g, RequantParams rq, DequantParams dq) {
-  gemm_ring_body<TN, TM, S, EPI, HAS_ZW, FAST>(g, rq, dq);
+  gemm_ring_body<TN, TM, S, EPI, HAS_ZW, FAST, STREAM>(g, rq, dq);
 }
+
+// Up to two row tiles the weights stream past the L2s, which then keep the activations that every channel tile re-reads.  With
+// more row tiles too many workgroups rely on finding them there.  us per launch, weights from HBM, plain -> streamed: one row
+// tile, 128 x 12288 x 4096 18.4 -> 16.3, 128 x 11008 x 4096 17.6 -> 16.0; two, 256 x 12288 x 4096 26.3 -> 23.4,
+// 128 x 4096 x 4096 11.8 -> 11.0; three, 300 x 5504 x 2048 (fp32) 13.9 -> 14.8; four, 197 x 768 x 3072 (fp32) 8.2 -> 9.4;
+// thirty-two, 4096 x 768 x 3072 (fp32) 16.3 -> 22.0.
+constexpr int kStreamRowTiles = 2;
 
 template <int TN, int TM, int S, int EPI, bool HAS_ZW, bool FAST>
 static int launch_ring(GemmArgs g, const RequantParams &rq, const DequantParams &dq, hipStream_t stream) {
   g.tiles_m = (g.m + 64 * TM - 1) / (64 * TM);
   g.tiles_n = (g.n + 64 * TN - 1) / (64 * TN);
-  hipLaunchKernelGGL((gemm_ring_kernel<TN, TM, S, EPI, HAS_ZW, FAST>), dim3(g.tiles_m * g.tiles_n), dim3(256), 0, stream, g,
-                     rq, dq);
+  const dim3 grid(g.tiles_m * g.tiles_n);
+  if (g.tiles_m <= kStreamRowTiles) {
+    hipLaunchKernelGGL((gemm_ring_kernel<TN, TM, S, EPI, HAS_ZW, FAST, true>), grid, dim3(256), 0, stream, g, rq, dq);
+  } else {
+    hipLaunchKernelGGL((gemm_ring_kernel<TN, TM, S, EPI, HAS_ZW, FAST, false>), grid, dim3(256), 0, stream, g, rq, dq);
+  }
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }
