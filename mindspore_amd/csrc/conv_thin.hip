@@ -2,6 +2,8 @@
 // memory into the matrix cores' operand registers.
 #include <string.h>
 
+#include <type_traits>
+
 #include "common.h"
 #include "quant_math.h"
 
@@ -23,7 +25,7 @@ typedef uint32_t u32_any __attribute__((aligned(1)));
 // channels for the stores (as in conv_rows_kernel).
 // Bound by the vector ALU (the requantisation, 7 instructions per output byte) where there are more channels than bytes of
 // K, by memory where there are fewer.  us per launch, before -> now: 16 x 112 x 112, 192 -> 32 channels 45.2 -> 10.6,
-// 32 -> 192 21.0 -> 15.8; 8 x 115 x 115, 240 -> 40 26.5 -> 9.6; 4 x 80 x 80, 72 -> 24 9.0 (in two launches) -> 3.5; one
+// 32 -> 192 21.0 -> 14.7; 8 x 115 x 115, 240 -> 40 26.5 -> 9.6; 4 x 80 x 80, 72 -> 24 9.0 (in two launches) -> 3.5; one
 // image of 112 x 112, where any launch takes most of it, 192 -> 32 3.7 -> 3.8.
 // Windows of several taps stay with the gathering GEMM: 32 x 56 x 56 x 64, 3x3, took 13.6 us in this form against 14.0, one
 // such image 6.2 against 5.1, stride 2 10.6 against 7.1.
@@ -101,18 +103,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
     __syncthreads();
   }
   if (tile >= tiles) return;
+  v16i start;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) start[e] = (int)kAccBias;
   locate(tile);
   v4i x[CH];
   fetch(x, 0);
   for (; tile < tiles; tile += step) {
     v16i acc[OCB], sums;
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-#pragma unroll
-      for (int ob = 0; ob < OCB; ++ob) acc[ob][e] = (int)kAccBias;
-      sums[e] = 0;
-    }
-    for (int c = 0; c < g.chunks; ++c) {
+    for (int e = 0; e < 16; ++e) sums[e] = 0;
+    auto chunk = [&](int c, auto first_c) {  // the first one starts the accumulators, from one register block for all
       v4i y[CH];
 #pragma unroll
       for (int s = 0; s < CH; ++s) y[s] = x[s];
@@ -139,7 +140,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
 #pragma unroll
         for (int ob = 0; ob < OCB; ++ob)
           acc[ob] = __builtin_amdgcn_mfma_i32_32x32x32_i8(y[s], *reinterpret_cast<const v4i *>(wl + (ob * steps + s) * 1024),
-                                                          acc[ob], 0, 0, 0);
+                                                          decltype(first_c)::value && s == 0 ? start : acc[ob], 0, 0, 0);
       if (!FAST && rq.has_zw) {  // the pixels' input sums, in the accumulators' layout: against ones up to K
 #pragma unroll
         for (int s = 0; s < CH; ++s) {
@@ -152,6 +153,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
           sums = __builtin_amdgcn_mfma_i32_32x32x32_i8(y[s], one, sums, 0, 0, 0);
         }
       }
+    };
+    // (One block of channels: few instructions to save, and a launch of so few that fetching the longer code shows:
+    //  4 x 80 x 80, 72 -> 24 3.3 us, with the split forms 3.6.  Three blocks: 16 x 112 x 112, 32 -> 192 16.2 us, with them 14.7.)
+    if constexpr (OCB > 1) {
+      chunk(0, std::true_type());
+      for (int c = 1; c < g.chunks; ++c) chunk(c, std::false_type());
+    } else {
+      acc[0] = start;
+      for (int c = 0; c < g.chunks; ++c) chunk(c, std::false_type());
     }
     // (the wait states that a matrix product's result needs before inline assembly reads it, as in conv_rows_kernel)
     if constexpr (OCB == 1) asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc[0]));
@@ -160,9 +170,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
     // acc[ob][4 * q + e] is pixel 8 * q + 4 * h + e of the tile, channel n0 + 32 * ob + r; after the transposition this
     // lane holds channels r & ~3 .. + 3 of pixel 8 * q + 4 * h + (lane & 3)
     const int first = tile * 32;
-    const bool whole = first + 32 <= g.pixels && (g.out_c & 3) == 0;
+    const bool whole = first + 32 <= g.pixels && n0 + 32 * OCB <= g.out_c;
     const int my_n = n0 + (r & ~3), my_p = first + 4 * h + (lane & 3);
     int8_t *dst = out + (int64_t)my_p * g.out_c + my_n;
+    auto store = [&](auto whole_c) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
 #pragma unroll
@@ -200,14 +211,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
         const uint32_t p23 = __builtin_amdgcn_perm((uint32_t)y[3], (uint32_t)y[2], 0x0c0c0400u);
         const uint32_t four = thin_quad_transpose(__builtin_amdgcn_perm(p23, p01, 0x05040100u), sel1, sel2);
         int8_t *to = dst + 8 * q * g.out_c + 32 * ob;
-        if (whole) {
-          if (my_n + 32 * ob < g.out_c) *reinterpret_cast<u32_any *>(to) = four;
+        if (decltype(whole_c)::value || (my_p + 8 * q < g.pixels && my_n + 32 * ob + 4 <= g.out_c)) {
+          *reinterpret_cast<u32_any *>(to) = four;
         } else if (my_p + 8 * q < g.pixels) {
 #pragma unroll
           for (int e = 0; e < 4; ++e)
             if (my_n + 32 * ob + e < g.out_c) to[e] = (int8_t)(four >> (8 * e));
         }
       }
+    }
+    };
+    if (OCB > 1 && whole) {
+      store(std::true_type());
+    } else {
+      store(std::false_type());
     }
   }
 }
