@@ -7,7 +7,8 @@
 //              .../nnacl/base/conv1x1_base.c:19-40, mindspore/lite/src/litert/kernel/cpu/int8/
 //              convolution_1x1_int8.cc:396)
 //   conv_dw  : depthwise conv + requantisation (ConvDwInt8 / ConvDwInt8Post,
-//              .../nnacl/int8/conv_depthwise_int8.c:24-140)
+//              .../nnacl/int8/conv_depthwise_int8.c:24-140); conv_dw_rows: the same with stride 1 and int8 weights, four
+//              taps per instruction
 //   conv_rows : first-layer convolutions (few input channels) in one launch, window rows straight from the image
 //   conv_smallk : what is left with kernel_h * kernel_w * in_c <= 64 in one launch, gathered byte by byte
 // The first three are HBM/latency bound byte movers: one thread produces 16 contiguous output bytes (or one output
