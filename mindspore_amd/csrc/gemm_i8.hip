@@ -470,12 +470,17 @@ template <bool HAS_ZW, bool FAST>
 static int launch_conv_pick_tile(const GemmArgs &g, const ConvGather &cv, const RequantParams &rq,
                                  hipStream_t stream) {
   const int64_t tiles_m = (int64_t)((g.m + 127) / 128) * ((g.n + 127) / 128);
-  // up to 64 output channels: half-width tiles (three workgroups per CU) instead of half-empty square ones
-  // (more such tiles than three per CU: a fourth workgroup per CU on three stages saves the second round)
-  if (g.n <= 64 && (g.m + 127) / 128 > 768) return launch_conv_cfg<64, 128, HAS_ZW, FAST, 3, 4>(g, cv, rq, stream);
-  if (g.n <= 64 && g.m >= 128 * 128) return launch_conv_cfg<64, 128, HAS_ZW, FAST, 4, 3>(g, cv, rq, stream);
-  if (tiles_m >= 128) return launch_conv_cfg<128, 128, HAS_ZW, FAST, 4, 2>(g, cv, rq, stream);
-  return launch_conv_cfg<64, 64, HAS_ZW, FAST, 4, 1>(g, cv, rq, stream);
+  // 64 x 64 tiles, four workgroups per CU (an allocation of 132 registers let in three, of which the second round was often
+  // next to empty): a step's gathered loads take longer than its products, and what hides them is other workgroups.  us per
+  // launch, three per CU / four: 8 x 28 x 28, 3x3, 96 -> 192 channels 11.0 / 7.4, 1x1 there 5.6 / 4.3; with few enough tiles for one
+  // round of three no change (8 x 40 x 40, 48 -> 48 4.7; one 56 x 56 image, 64 -> 64 5.0).  64 x 128 tiles at 16 x 50 x 50,
+  // 32 -> 32 5.9, these 5.7.
+  // Where up to 64 channels give them more than one and a half rounds: the same number of pixels at once on 64 x 256 tiles,
+  // which read the weights a quarter as often (32 x 56 x 56, 64 -> 64 14.0 -> 12.5).
+  // 128 x 128 tiles against more channels as soon as there are enough of them (32 x 28 x 28, 64 -> 128 7.2, on 64 x 64 9.1).
+  if (g.n <= 64 && (g.m + 127) / 128 > 768) return launch_conv_cfg<64, 256, HAS_ZW, FAST, 4, 2>(g, cv, rq, stream);
+  if (g.n > 64 && tiles_m >= 128) return launch_conv_cfg<128, 128, HAS_ZW, FAST, 4, 2>(g, cv, rq, stream);
+  return launch_conv_cfg<64, 64, HAS_ZW, FAST, 4, 4>(g, cv, rq, stream);
 }
 
 bool gemm_conv_supported(const ConvGeom &cg, const void *in) {

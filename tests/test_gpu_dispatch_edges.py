@@ -194,3 +194,18 @@ def test_conv_1x1_few_channels(orc, b, ih, iw, ic, oc):
         case = _conv_case(rng, b, ih, iw, ic, oc, (1, 1), (1, 1), (1, 1), pad, it != 1, it == 1, it != 2, [0, 1, 3][it])
         got = _gpu_conv(case, (1, 1), (1, 1), pad, 1, device_tensors=True)
         assert np.array_equal(got, orc.conv_int8(**case)), it
+
+
+@pytest.mark.parametrize("b,ih,iw,ic,oc", [(1, 12, 11, 16, 7), (2, 31, 33, 48, 64), (1, 40, 41, 32, 65), (2, 91, 90, 16, 130),
+                                           (8, 111, 111, 16, 64),  # 771 rows of 128 pixels: 64 x 256 tiles
+                                           (8, 110, 111, 16, 33)])  # 764: 64 x 64
+def test_conv_gather_tiles(orc, b, ih, iw, ic, oc):
+    """Either side of the rules by which the gathering GEMM picks its tile, with and without weight zero points."""
+    from tests.test_gpu_parity import _conv_case, _gpu_conv
+    rng = np.random.default_rng(ih * iw + oc)
+    orc.set_threads(16)
+    pad = (1, 1, 1, 1)
+    for it in range(2):
+        case = _conv_case(rng, b, ih, iw, ic, oc, (3, 3), (1, 1), (1, 1), pad, True, it == 1, True, it)
+        got = _gpu_conv(case, (1, 1), (1, 1), pad, 1, device_tensors=True, exact_3x3=True)
+        assert np.array_equal(got, orc.conv_int8(**case)), it
