@@ -98,7 +98,9 @@ def test_no_alloc_entry_point_leaves_free_device_memory_unchanged(orc):
     import torch
     L = lib.load()
     rng = np.random.default_rng(9)
-    n, k = 1030, 4000  # deep % 16 != 0 and col % 4 != 0: both workspaces are needed
+    # deep % 16 == 4 and col % 4 == 2: padded rows are needed, and the limit counts a padded output as well
+    # (1600 x 4016 + 1600 x 1032 = 8.08e6 bytes of the 8.39e6)
+    n, k = 1030, 4004
     case = _case(rng, n, k, True)
 
     def make():
