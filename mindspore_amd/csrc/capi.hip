@@ -464,10 +464,10 @@ struct mi_dynquant {
   uint32_t ticket = 0;    // of the last run that writes the note
   bool asked = false;     // the parameters of the run before were fetched
   bool noted = false;     // the last run writes the note
-  // A captured run may be replayed at any time, unseen by the host: a handle that may have one makes no notes.  Asking
-  // whether a stream is captured costs 0.4 us, so runs of a handle without a note are not asked about; the fetch that
-  // follows such a run shows that it was not captured, and one that none follows counts as captured.
-  bool captured = false, unchecked = false;
+  // A run was captured: its graph may be replayed at any time, unseen by the host, also between an eager run and the
+  // fetch that follows it, so from then on the parameters are copied from the device.  Every run asks its stream (0.4 us; the
+  // null stream cannot be captured): that a fetch follows a run does not show it was eager, a replay is fetched from too.
+  bool captured = false;
   ~mi_dynquant() {
     if (note != nullptr) (void)hipHostFree(note);
   }
@@ -1213,10 +1213,7 @@ int mi_dynquant_run(mi_dynquant *h, const float *x_dev, int64_t n, int8_t *q_dev
   int rc = ensure_device();
   if (rc != MI_OK) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (h->note == nullptr) {
-    h->captured |= h->unchecked;
-    h->unchecked = true;
-  } else if (!h->captured && s != nullptr) {
+  if (!h->captured && s != nullptr) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     h->captured = hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
   }
@@ -1257,7 +1254,6 @@ static int dynquant_params(mi_dynquant *h, void *stream, bool whole_run, mi_dq_p
   if (rc != MI_OK) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   h->asked = true;
-  h->unchecked = false;
   if (h->note == nullptr && !h->captured) {
     void *p = nullptr;
     if (hipHostMalloc(&p, kDqHostWords * sizeof(uint64_t), hipHostMallocCoherent) == hipSuccess) {

@@ -209,3 +209,34 @@ def test_conv_gather_tiles(orc, b, ih, iw, ic, oc):
         case = _conv_case(rng, b, ih, iw, ic, oc, (3, 3), (1, 1), (1, 1), pad, True, it == 1, True, it)
         got = _gpu_conv(case, (1, 1), (1, 1), pad, 1, device_tensors=True, exact_3x3=True)
         assert np.array_equal(got, orc.conv_int8(**case)), it
+
+
+def test_dynamic_quant_parameters_of_a_handle_first_run_under_capture(orc):
+    """A handle whose very first run was captured: its graph may be replayed at any time, also between an eager run and
+    the fetch that follows, and the fetch returns the parameters of whatever ran last."""
+    import torch
+    rng = np.random.default_rng(5)
+    one, other = _values(rng, 40000), _values(rng, 5000) * 7
+    other_dev = torch.from_numpy(other).cuda()
+    lib, p = K._lib, K._lib.DqParams()
+    L = lib.load()
+    K.DynamicQuantKernel(False).run(torch.from_numpy(one).cuda())  # the kernels are loaded before the capture
+    side = torch.cuda.Stream()
+    x = torch.from_numpy(one).cuda()
+    torch.cuda.synchronize()
+    dq = K.DynamicQuantKernel(False)
+    with torch.cuda.stream(side):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            dq.run(x, fetch_params=False)
+        scale = np.float32(1.0)
+        for fetch in (L.mi_dynquant_get_params, L.mi_dynquant_await_params):
+            for eager_fetch in (None, False, True, False):
+                if eager_fetch is not None:
+                    _, q = dq.run(other_dev, fetch_params=eager_fetch)
+                    assert not eager_fetch or (q.scale, q.zero_point) == orc.dynamic_quant(other)[1:]
+                scale *= np.float32(1.5)
+                x.copy_(torch.from_numpy(one * scale))
+                graph.replay()
+                assert fetch(dq._h, side.cuda_stream, p) == lib.MI_OK
+                assert (p.scale, p.zero_point) == orc.dynamic_quant(one * scale)[1:], (fetch.__name__, eager_fetch)
