@@ -746,10 +746,6 @@ int mi_matmul_run(mi_matmul *h, const int8_t *a_dev, int32_t rows, int8_t *c_dev
   int rc = ensure_device();
   if (rc != MI_OK) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // Whether a run copies its activations depends on its pointer as well.  A MatMul with odd-sized rows sits among tensors
-  // whose parts start anywhere, so its first run of a row count makes the room at once: no later run of that row count
-  // allocates, and one with a misaligned pointer can be the one under graph capture.
-  if ((h->st.n & 3) != 0 && (rc = h->a_ws.ensure((size_t)rows * round_up(h->st.k, 16))) != MI_OK) return rc;
   const int8_t *a = nullptr;
   int64_t lda = 0;
   int k16 = 0;

@@ -240,3 +240,40 @@ def test_dynamic_quant_parameters_of_a_handle_first_run_under_capture(orc):
                 graph.replay()
                 assert fetch(dq._h, side.cuda_stream, p) == lib.MI_OK
                 assert (p.scale, p.zero_point) == orc.dynamic_quant(one * scale)[1:], (fetch.__name__, eager_fetch)
+
+
+@pytest.mark.parametrize("n,k,rows", [(201, 512, 8), (201, 512, 100), (1030, 4096, 300), (7, 48, 1)])
+def test_first_run_of_odd_output_rows_under_capture(orc, n, k, rows):
+    """Rows of a length the kernels store in place, from an aligned activation tensor: no run allocates, so the very first
+    may be captured, and none leaves the handle holding memory."""
+    import torch
+    rng = np.random.default_rng(n + rows)
+    orc.set_threads(16)
+    w, bias, sw, zw, make = _matmul_pair(rng, n, k, False, False)
+    make(True).run(torch.zeros((rows, k), dtype=torch.int8, device="cuda"))  # the kernels are loaded before the capture
+    kern = make(True)
+    a = torch.from_numpy(rng.integers(-128, 128, (rows, k), dtype=np.int8)).cuda()
+    out = torch.zeros((rows, n), dtype=torch.int8, device="cuda")
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            kern.run(a, out=out)
+    for _ in range(3):
+        a.copy_(torch.from_numpy(rng.integers(-128, 128, (rows, k), dtype=np.int8)))
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        want = orc.matmul_int8(a.cpu().numpy(), w, bias, 0.02, 7, sw, zw, float(np.float32(0.02 * 0.0055 * k ** 0.5 * 140)), 3)
+        assert np.array_equal(out.cpu().numpy(), want)
+        assert np.array_equal(kern.run(a).cpu().numpy(), want)
+    many = (64 << 20) // k  # 64 MiB of activation rows
+    a = torch.zeros((many, k), dtype=torch.int8, device="cuda")
+    out = torch.zeros((many, n), dtype=torch.int8, device="cuda")
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    kern.run(a, out=out)
+    torch.cuda.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] < 32 << 20
