@@ -3,6 +3,7 @@
 
 #include "common.h"
 #include "quant_math.h"
+#include "weight_loads.h"
 
 #include <type_traits>
 

@@ -71,12 +71,11 @@ __device__ __forceinline__ void gemm_kblock_body(const GemmArgs &g, const Requan
   const int drow = lane >> 3;
   const int dchunk = (lane & 7) ^ (drow >> 1);  // for even i; odd i: ^ 4
   const int k64 = g.k_pad >> 6;
-  // (the packed weights have n rounded up to 256 rows; a tile of 192 channels can reach past them, where loads return 0)
-  int w_groups = (((g.n + kNPad - 1) & -kNPad) - n0) / 16 - wave * TN;
-  w_groups = __builtin_amdgcn_readfirstlane(w_groups < 0 ? 0 : (w_groups < TN ? w_groups : TN));  // (stays scalar)
-  const int64_t w_first = WB ? (int64_t)(n0 / 16 + wave * TN) * k64 * 1024 : (int64_t)(n0 + wave * 16 * TN) * g.ldw;
+  const WaveWeightGroups<TN> wg(g.n, n0, wave, kNPad);
+  const int64_t group_bytes = WB ? k64 * 1024 : 16 * g.ldw;
   const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<int8_t *>(WB ? g.wb : g.w) + w_first, (short)0, w_groups * (WB ? k64 * 1024 : 16 * g.ldw), 0x00020000);
+      const_cast<int8_t *>(WB ? g.wb : g.w) + wg.first * group_bytes, (short)0,
+      wg.inside * (int)group_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t a_rsrc =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(g.a) + (int64_t)m0 * g.lda, (short)0, -1, 0x00020000);
   // row-major: ldw is a multiple of 256, so odd i is w_voff ^ 64
@@ -107,7 +106,8 @@ __device__ __forceinline__ void gemm_kblock_body(const GemmArgs &g, const Requan
     for (int ii = 0; ii < TN; ++ii) {
       const int i = half * TN + ii;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, lds_ptr(dst + i * 1024), 16, WB ? w_voff : w_voff ^ ((i & 1) << 6),
-                                               WB ? ((i >> 1) * k64 + 2 * kb + (i & 1)) * 1024 : 8 * i * g.ldw + kb * KB, 0, 0);
+                                               WB ? blocked_weight_offset(wg.group(i >> 1), i & 1, k64, kb)
+                                                  : row_major_weight_offset(wg.group(i >> 1), i & 1, g.ldw, kb), 0, 0);
     }
   };
   auto dma_a = [&](int slot, int kb, int half) {

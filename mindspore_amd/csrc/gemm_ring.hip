@@ -49,11 +49,9 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs &g, const RequantP
   const int drow = lane >> 3;
   const int dchunk = (lane & 7) ^ (drow >> 1);  // for even i; odd i: ^ 4
   const int k64 = g.k_pad >> 6;
-  // (the packed weights have n rounded up to 256 rows; a tile of 192 channels can reach past them, where loads return 0)
-  int w_groups = (((g.n + kNPad - 1) & -kNPad) - n0) / 16 - wave * TN;
-  w_groups = __builtin_amdgcn_readfirstlane(w_groups < 0 ? 0 : (w_groups < TN ? w_groups : TN));  // (stays scalar)
+  const WaveWeightGroups<TN> wg(g.n, n0, wave, kNPad);
   const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<int8_t *>(g.wb) + (int64_t)(n0 / 16 + wave * TN) * k64 * 1024, (short)0, w_groups * k64 * 1024, 0x00020000);
+      const_cast<int8_t *>(g.wb) + (int64_t)wg.first * k64 * 1024, (short)0, wg.inside * k64 * 1024, 0x00020000);
   const __amdgpu_buffer_rsrc_t a_rsrc =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(g.a) + (int64_t)m0 * g.lda, (short)0, -1, 0x00020000);
   int a_voff[2 * TM];
@@ -80,7 +78,7 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs &g, const RequantP
     for (int l = from; l < to; ++l) {
       if (l < 2 * TN) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, lds_ptr(sw + l * 1024), 16, lane * 16,
-                                                 ((l >> 1) * k64 + 2 * kb + (l & 1)) * 1024, 0, STREAM ? 2 : 0);
+                                                 blocked_weight_offset(wg.group(l >> 1), l & 1, k64, kb), 0, STREAM ? 2 : 0);
       } else {
         const int i = l - 2 * TN;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, lds_ptr(sa + i * 1024), 16, a_voff[i], kb * KB, 0, 0);
