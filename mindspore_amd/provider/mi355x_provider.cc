@@ -29,6 +29,9 @@
 //   device_only_outputs=<tensor name>,<tensor name>,...      (or * for every output)
 // (Model::LoadConfig / UpdateConfig, delivered through Kernel::GetConfig, include/api/kernel_api.h:112-126) names
 // outputs that only kernels of this provider consume: their host copy is skipped as well.
+//   weight_copies=1
+// in the same section makes MatMul / FullConnection kernels hold one packed form of their weights instead of two (half the
+// device memory, slower from two rows on: MI_MATMUL_NO_DECODE_PACK, MI_DYNMM_NO_DECODE_PACK).
 // Dense 3x3 stride-1 convolutions are declined by default: x86 builds of the reference run an integer Winograd there
 // (convolution_int8_creator.cc:81-94), whose results are not those of the exact convolution.  MI355X_CONV3X3=exact in
 // the environment makes the provider take them and compute the exact convolution, which is what the reference runs
@@ -404,21 +407,18 @@ class MatmulKernel : public kernel::Kernel {
     std::vector<int32_t> zps;
     FilterQuant(w, &scales, &zps);
     const void *bias = inputs_.size() > kBiasIndex ? inputs_[kBiasIndex].Data().get() : nullptr;
-    // The second packed form of the weights serves up to 64 activation rows; a node whose inferred output already has
-    // more rows than that does without it (half the device memory per weight).  Should the model later be resized
-    // to a few rows, they run on the GEMM tiles.
-    const auto oshape = outputs_[0].Shape();
-    bool rows_known = !oshape.empty();
-    for (int64_t e : oshape) rows_known = rows_known && e >= 0;
-    const int64_t rows_now = batched_ && oshape.size() >= 2 ? oshape[oshape.size() - 2] : RowsOfOutput(outputs_[0]);
-    const bool no_decode_pack = rows_known && rows_now > (n <= 4096 && k >= 1024 ? 2 * kDecodeMaxRows : kDecodeMaxRows);
+    // Two packed forms of the weights: the decode kernel and the fast GEMM tiles read the second one, at every row count from
+    // two on, so doing without it is the session's choice and not a matter of the rows.
+    const auto section = GetConfig("mi355x");
+    const auto copies = section.find("weight_copies");
+    const bool one_copy = copies != section.end() && copies->second == "1";
     if (outputs_[0].DataType() == DataType::kNumberTypeInt8) {
       const auto iq = inputs_[0].QuantParams().front();
       const auto oq = outputs_[0].QuantParams().front();
       mi_matmul_desc d{k, n, b_transpose_ ? 1 : 0, act_, iq.scale, iq.zero_point, oq.scale, oq.zero_point,
                        static_cast<int32_t>(scales.size()), scales.data(), zps.data()};
       d.b_batch = static_cast<int32_t>(b_batch);
-      if (no_decode_pack) d.flags |= MI_MATMUL_NO_DECODE_PACK;
+      if (one_copy) d.flags |= MI_MATMUL_NO_DECODE_PACK;
       const int rc = mi_matmul_create(&d, static_cast<const int8_t *>(w.Data().get()),
                                       static_cast<const int32_t *>(bias), &full_);
       // (a session that runs its nodes in parallel gives no order to lean on: no groups there)
@@ -430,7 +430,7 @@ class MatmulKernel : public kernel::Kernel {
     }
     if (batched_) return kLiteError;  // (the creator declines batched weights for the dynamic MatMul)
     mi_dynmm_desc d{k, n, b_transpose_ ? 1 : 0, act_, static_cast<int32_t>(scales.size()), scales.data(), zps.data()};
-    if (no_decode_pack) d.flags |= MI_DYNMM_NO_DECODE_PACK;
+    if (one_copy) d.flags |= MI_DYNMM_NO_DECODE_PACK;
     const int rc =
       mi_dynmm_create(&d, static_cast<const int8_t *>(w.Data().get()), static_cast<const float *>(bias), &dyn_);
     // dynamic MatMuls that read the same DynamicQuant output (q / k / v, gate / up) form groups like the full-quant ones
@@ -506,8 +506,6 @@ class MatmulKernel : public kernel::Kernel {
 
  private:
   static constexpr int32_t kSiblingMaxRows = 32;  // the row counts that mi_matmul_run_group runs as one launch
-  static constexpr int32_t kDecodeMaxRows = 64;   // the row counts that the blocked second copy of the weights serves
-                                                  // (twice as many against at most 4096 channels with K >= 1024)
   static constexpr int kNotGrouped = -1000;
 
   // Runs this kernel and every sibling that is ready for the same rows as one launch.  kNotGrouped: nothing was

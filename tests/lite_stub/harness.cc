@@ -209,7 +209,18 @@ int Infer(Session *s) {
 std::shared_ptr<mindspore::kernel::KernelInterface> TestInterfaceCreator() { return std::make_shared<BuiltinInference>(); }
 }  // namespace
 
+// What ph_set_config put into the [mi355x] section of the session config of nodes made from then on.
+std::map<std::string, std::string> g_config;
+
 extern "C" {
+void ph_set_config(const char *key, const char *value) {  // value NULL: the key goes
+  if (value != nullptr) {
+    g_config[key] = value;
+  } else {
+    g_config.erase(key);
+  }
+}
+
 // Builds the node: tensors, shape inference, creator lookup and call, Prepare().  *stage tells how far it got;
 // *code is the status of the failing call (0 otherwise).  Returns NULL unless the kernel is ready to execute.
 // `producer` (optional): a node made earlier whose output tensor becomes this node's input 0 -- the same tensor
@@ -224,6 +235,7 @@ void *ph_create_node(const ph_op *op, const char *arch, const char *provider, co
   *stage = kOk;
   *code = 0;
   Fill(*op, &s->prim);
+  if (!g_config.empty()) s->config["mi355x"] = g_config;
   if (device_only_outputs != nullptr) s->config["mi355x"]["device_only_outputs"] = device_only_outputs;
   for (int i = 0; i < n_in; ++i) {
     if (i == 0 && producer != nullptr) {

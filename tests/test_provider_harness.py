@@ -54,6 +54,8 @@ def _load_harness():
     h.ph_destroy.restype = None
     h.ph_create_node.restype = C.c_void_p
     h.ph_create_node.argtypes = h.ph_create.argtypes[:9] + [C.c_void_p, C.c_char_p, C.c_char_p] + h.ph_create.argtypes[9:]
+    h.ph_set_config.argtypes = [C.c_char_p, C.c_char_p]
+    h.ph_set_config.restype = None
     h.ph_execute_linked.argtypes = [C.c_void_p, C.POINTER(C.c_int32)]
     h.ph_resize_linked.argtypes = [C.c_void_p, C.POINTER(C.c_int32)]
     h.ph_set_enable_parallel.argtypes = [C.c_void_p, C.c_int32]
@@ -319,6 +321,41 @@ def test_fullconnection_and_matmul_through_the_provider(H, orc):
                            False)
     assert y.shape == (2, 7, n) and np.array_equal(y.reshape(14, n), want)
     node.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 300])
+@pytest.mark.parametrize("dynamic", [False, True])
+def test_matmul_kernels_hold_both_weight_forms_unless_the_session_says_one(H, orc, rows, dynamic):
+    """The kernels for two rows and more read the second form, whatever row count a node was built for; a session may give
+    it up for memory.  Same results either way."""
+    import torch
+    rng = np.random.default_rng(rows)
+    orc.set_threads(16)
+    n, k = 2048, 4096
+    a, w, sw, b, ins = _fc_inputs(rng, rows, n, k, bias=False)
+    if dynamic:
+        ins[0] = tensor(I8, (rows, k), None)
+        want = orc.dynamic_matmul(a, w, None, 0.02, -3, sw, np.zeros(n, np.int32))
+    else:
+        want = orc.matmul_int8(a, w, None, 0.02, -3, sw, np.zeros(n, np.int32), 0.5, 5, 0, True)
+    held = {}
+    for copies in (None, b"1"):
+        H.ph_set_config(b"weight_copies", copies)
+        try:
+            torch.cuda.synchronize()
+            free = torch.cuda.mem_get_info()[0]
+            nodes = [Node(H, op(MATMUL, transpose_b=1), ins, F32 if dynamic else I8, () if dynamic else [(0.5, 5)])
+                     for _ in range(4)]
+            assert all(node.stage == OK for node in nodes)
+            held[copies] = (free - torch.cuda.mem_get_info()[0]) / (4 * n * k)
+        finally:
+            H.ph_set_config(b"weight_copies", None)
+        y, _ = nodes[0].run(a, [(0.02, -3)])
+        assert np.array_equal(y.view(np.uint32) if dynamic else y, want.view(np.uint32) if dynamic else want)
+        for node in nodes:
+            node.close()
+    assert held[None] > 1.75 and held[b"1"] < 1.5, held
 
 
 @pytest.mark.gpu
