@@ -457,18 +457,21 @@ struct mi_conv {
 struct mi_dynquant {
   int symmetric = 0;
   DevBuf partials, slots, params, h_in, h_out, h_params;
-  // Where a run leaves its parameters for the host that asks for them.  Polled by the host (mi_dynquant_await_params)
-  // they are there a few microseconds after the launch; a copy and a stream synchronisation behind it took 22 us more
-  // (197 x 768: 34 us per run and fetch -> 10.5, and 16 for mi_dynquant_get_params, which waits for the stream).  Writing to host memory lengthens the kernel, so only the runs of a handle whose last parameters were asked for do.
+  // Where a run leaves its parameters for the host that asks for them: page-locked, made with the handle, or absent (every
+  // fetch is then a copy).  Polled by the host (mi_dynquant_await_params) they are there a few microseconds after the launch; a
+  // copy and a stream synchronisation behind it took 22 us more (197 x 768: 34 us per run and fetch -> 10.5, and 16 for
+  // mi_dynquant_get_params, which waits for the stream).  Writing to host memory lengthens the kernel, so only the first run
+  // and the runs of a handle whose last parameters were asked for do.
   uint64_t *note = nullptr;
   uint32_t ticket = 0;    // of the last run that writes the note
-  bool asked = false;     // the parameters of the run before were fetched
+  bool asked = true;      // the parameters of the run before were fetched (or there was none)
   bool noted = false;     // the last run writes the note
   // A run was captured: its graph may be replayed at any time, unseen by the host, also between an eager run and the
   // fetch that follows it, so from then on the parameters are copied from the device.  Every run asks its stream (0.4 us; the
   // null stream cannot be captured): that a fetch follows a run does not show it was eager, a replay is fetched from too.
   bool captured = false;
   ~mi_dynquant() {
+    params.release();  // (waits for the device: no run still writes the note)
     if (note != nullptr) (void)hipHostFree(note);
   }
 };
@@ -1196,6 +1199,13 @@ int mi_dynquant_create(int32_t symmetric, mi_dynquant **out) {
   }
   MI_HIP_CHECK(hipMemset(h->slots.p, 0xff, kDqSlotBytes));
   MI_HIP_CHECK(hipStreamSynchronize(nullptr));  // runs may come in on any stream
+  void *note = nullptr;
+  if (hipHostMalloc(&note, kDqHostWords * sizeof(uint64_t), hipHostMallocCoherent) == hipSuccess) {
+    memset(note, 0, kDqHostWords * sizeof(uint64_t));
+    h->note = static_cast<uint64_t *>(note);
+  } else {
+    (void)hipGetLastError();
+  }
   *out = owner.release();
   return MI_OK;
 }
@@ -1250,15 +1260,6 @@ static int dynquant_params(mi_dynquant *h, void *stream, bool whole_run, mi_dq_p
   if (rc != MI_OK) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   h->asked = true;
-  if (h->note == nullptr && !h->captured) {
-    void *p = nullptr;
-    if (hipHostMalloc(&p, kDqHostWords * sizeof(uint64_t), hipHostMallocCoherent) == hipSuccess) {
-      h->note = static_cast<uint64_t *>(p);
-      memset(p, 0, kDqHostWords * sizeof(uint64_t));
-    } else {
-      (void)hipGetLastError();  // (without it every fetch is a copy)
-    }
-  }
   if (!whole_run && take_noted_params(h, std::chrono::microseconds(1000), params_host)) {
     g_sync_count.fetch_add(1, std::memory_order_relaxed);
     return MI_OK;

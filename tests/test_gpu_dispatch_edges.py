@@ -277,3 +277,37 @@ def test_first_run_of_odd_output_rows_under_capture(orc, n, k, rows):
     kern.run(a, out=out)
     torch.cuda.synchronize()
     assert free - torch.cuda.mem_get_info()[0] < 32 << 20
+
+
+@pytest.mark.parametrize("unfetched", [0, 2])
+def test_dynamic_quant_parameters_do_not_wait_for_later_work(orc, unfetched):
+    """The parameters of a run are known before the work that was queued behind it: for a new handle's first run, and for one
+    whose first runs nobody asked about, from the run after its first fetch on."""
+    import time
+    import torch
+    lib, p = K._lib, K._lib.DqParams()
+    L = lib.load()
+    x = _values(np.random.default_rng(8), 197 * 768)
+    dev, big = torch.from_numpy(x).cuda(), torch.randn(4096, 4096, device="cuda")
+    side = torch.cuda.Stream()
+    K.DynamicQuantKernel(False).run(dev)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        big @ big
+        dq = K.DynamicQuantKernel(False)
+        for _ in range(unfetched):
+            dq.run(dev, fetch_params=False)
+        if unfetched:
+            dq.run(dev)
+        torch.cuda.synchronize()
+        began = time.perf_counter()
+        dq.run(dev, fetch_params=False)
+        for _ in range(64):  # tens of milliseconds
+            y = big @ big
+        queued = time.perf_counter()
+        assert L.mi_dynquant_await_params(dq._h, side.cuda_stream, p) == lib.MI_OK
+        known = time.perf_counter()
+        side.synchronize()
+        done = time.perf_counter()
+    assert (p.scale, p.zero_point) == orc.dynamic_quant(x)[1:]
+    assert known - queued < 0.25 * (done - began), (queued - began, known - queued, done - began)
