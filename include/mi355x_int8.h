@@ -236,7 +236,9 @@ typedef struct mi_dq_params {
 } mi_dq_params;
 
 int mi_dynquant_create(int32_t symmetric, mi_dynquant **out);
-/* x_dev: fp32 [n]; q_dev: int8 [n].  Asynchronous; the parameters stay on the device. */
+/* x_dev: fp32 [n]; q_dev: int8 [n].  Asynchronous; the parameters stay on the device.  The runs of one handle, replays of
+ * captured ones included, share its state: they are ordered by their stream, or by events where they go to several.  Runs that
+ * overlap all the same leave their own results and parameters unspecified, and no later run's. */
 int mi_dynquant_run(mi_dynquant *h, const float *x_dev, int64_t n, int8_t *q_dev, void *stream);
 /* Waits for the last run on `stream` and returns its parameters (what the provider writes with SetQuantParams). */
 int mi_dynquant_get_params(mi_dynquant *h, void *stream, mi_dq_params *params_host);

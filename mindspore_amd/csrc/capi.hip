@@ -470,6 +470,7 @@ struct mi_dynquant {
   // fetch that follows it, so from then on the parameters are copied from the device.  Every run asks its stream (0.4 us; the
   // null stream cannot be captured): that a fetch follows a run does not show it was eager, a replay is fetched from too.
   bool captured = false;
+  uint32_t launches = 0;  // number of the last launch (kDqReplayed - 1 is followed by 1)
   ~mi_dynquant() {
     params.release();  // (waits for the device: no run still writes the note)
     if (note != nullptr) (void)hipHostFree(note);
@@ -1197,7 +1198,7 @@ int mi_dynquant_create(int32_t symmetric, mi_dynquant **out) {
       (rc = h->slots.ensure(kDqSlotBytes)) != MI_OK || (rc = h->params.ensure(sizeof(mi_dq_params))) != MI_OK) {
     return rc;
   }
-  MI_HIP_CHECK(hipMemset(h->slots.p, 0xff, kDqSlotBytes));
+  MI_HIP_CHECK(hipMemset(h->slots.p, 0, kDqSlotBytes));
   MI_HIP_CHECK(hipStreamSynchronize(nullptr));  // runs may come in on any stream
   void *note = nullptr;
   if (hipHostMalloc(&note, kDqHostWords * sizeof(uint64_t), hipHostMallocCoherent) == hipSuccess) {
@@ -1226,7 +1227,8 @@ int mi_dynquant_run(mi_dynquant *h, const float *x_dev, int64_t n, int8_t *q_dev
   h->noted = h->asked && h->note != nullptr && !h->captured;
   h->asked = false;
   if (h->noted && ++h->ticket == 0) h->ticket = 1;
-  return launch_dynquant(x_dev, n, h->symmetric, static_cast<float2 *>(h->partials.p), h->slots.p,
+  if (++h->launches == kDqReplayed) h->launches = 1;
+  return launch_dynquant(x_dev, n, h->symmetric, static_cast<float2 *>(h->partials.p), h->slots.p, h->captured ? 0 : h->launches,
                          DqHostNote{h->note, h->noted ? h->ticket : 0}, static_cast<mi_dq_params *>(h->params.p), q_dev, s);
 }
 

@@ -175,9 +175,12 @@ int launch_gemm_conv_requant(const int8_t *in, const ConvGeom &g, const int8_t *
 
 // DynamicQuant: per-block min/max partials, then quantise (every block re-reduces the partials).
 constexpr int kDqMaxBlocks = 1024;
-// slots: kDqSlotBytes of device memory, all ones when made, through which the workgroups of the one-launch form meet.
+// slots: kDqSlotBytes of device memory, all zeros when made, through which the workgroups of the one-launch form meet.
 constexpr int kDqFusedMost = 256;  // workgroups of the one-launch form: one per CU
-constexpr size_t kDqSlotBytes = (2 * sizeof(uint64_t) + sizeof(uint32_t)) * kDqFusedMost;
+// launch: the number of a launch among those on these slots, 1 .. kDqReplayed - 1 and never that of the launch before, or 0
+// for a launch that may be replayed.
+constexpr uint32_t kDqReplayed = 0x80000000u;
+constexpr size_t kDqSlotBytes = sizeof(uint64_t) * (2 + 2 * kDqFusedMost);
 // Page-locked host memory into which a run whose ticket is not 0 also writes {scale, zero point, min, max} as float /
 // int32 bits in the low halves of kDqHostWords words, with the ticket in the high halves.
 constexpr int kDqHostWords = 4;
@@ -185,8 +188,8 @@ struct DqHostNote {
   uint64_t *words;
   uint32_t ticket;
 };
-int launch_dynquant(const float *x, int64_t n, int symmetric, float2 *partials, void *slots, const DqHostNote &note,
-                    mi_dq_params *params, int8_t *q, hipStream_t stream);
+int launch_dynquant(const float *x, int64_t n, int symmetric, float2 *partials, void *slots, uint32_t launch,
+                    const DqHostNote &note, mi_dq_params *params, int8_t *q, hipStream_t stream);
 // One {scale, zero point} per contiguous run of `unit` elements; params has `segments` entries.
 int launch_dynquant_segments(const float *x, int64_t segments, int64_t unit, int symmetric, mi_dq_params *params,
                              int8_t *q, hipStream_t stream);

@@ -197,36 +197,46 @@ __device__ __forceinline__ void publish_to_host(const DqHostNote &note, float sc
 // workgroups and quantises from the registers.  The tensor crosses HBM once, and a second launch and its re-read are
 // saved for one exchange through memory.
 //
-// The exchange: slot s of the current half holds workgroup s's {min, max}, one 64-bit store that either arrives whole
-// or not at all, so no fence and no atomic read-modify-write (those serialise across the XCDs' separate L2s).  An empty
-// slot is all ones (a minimum is never NaN).  The halves take turns from launch to launch: while one is filled and
-// read, the other, which nobody reads any more, is emptied for the next launch.  Whose turn it is stands in memory as
-// well (a captured launch has no other way to know), one copy per slot; every launch writes all kDqSlots slots --
-// workgroup b takes b, b + W, .. for W workgroups, of which the first W are waited for -- so the copies agree.  Launches
-// on one handle are ordered by their stream.
+// The exchange: workgroup s leaves its min and its max in slot s, each beside the launch's tag in one 64-bit word that either
+// arrives whole or not at all, so no fence is needed and a word of an earlier launch is never taken for one of this.  Every
+// launch fills all kDqSlots slots -- workgroup b takes b, b + W, .. for W workgroups, of which the first W are waited for --
+// so a tag that comes round again after 2^31 launches finds none of its kind.  The host numbers the launches, except those
+// that may be captured: a replay repeats its arguments, so there the number stands in memory (`replays`), and workgroup 0
+// raises it when it has found the tag in every slot in use, hence after the last workgroup has read it.
+//
+// Launches on one handle are ordered by their stream.  Should two overlap, they disturb each other and no later one.  For
+// numbers from memory: a workgroup that has given up waiting raises the number past its own tag too, and one that has not has
+// seen its tag in slot 0, whose writer raises it, so in the end it is past every tag that was left in a slot.
+//
+// us per launch, eager / replayed: 8 x 4096 4.1 / 4.1, 8 x 11008 4.4 / 4.3, 4096 x 768 8.1 / 8.2, 4096 x 3072 17.2 / 17.3 (slots
+// without tags that were emptied in turn, whose turn it was in a word per slot: 4.3 / 4.1, 4.6 / 4.4, 8.4 / 8.5, 17.5 / 17.6; two
+// 8-byte loads per slot instead of one of 16: 4.5 / 4.4, 4.6 / 4.6, 8.8 / 8.9, 17.6 / 17.6).
 //
 // The wait is bounded: workgroups that are not resident together (the device is shared) are not waited for for ever; a
 // workgroup that has waited `patience` ticks of the 100 MHz counter reads the whole tensor itself.
 constexpr int kDqSlots = kDqFusedMost;
-constexpr uint64_t kDqEmpty = ~(uint64_t)0;
 constexpr uint32_t kDqPatience = 20000;  // 200 us
+constexpr int kAgentScope = 16;  // cache policy of a load from the device's coherence point (sc1)
 struct DqSlots {
-  uint64_t range[2][kDqSlots];
-  uint32_t turn[kDqSlots];
+  unsigned long long replays;
+  uint64_t pad;
+  uint64_t range[kDqSlots][2];  // {min, max}, each below its tag
 };
-static_assert(sizeof(DqSlots) == kDqSlotBytes, "what the handle allocates and fills with ones");
+static_assert(sizeof(DqSlots) == kDqSlotBytes, "what the handle allocates and fills with zeros");
 
 template <int T, int G>
 __global__ __launch_bounds__(T) void dq_fused_kernel(const float *__restrict__ x, int64_t n, int symmetric,
-                                                     DqSlots *slots, uint32_t patience, DqHostNote note,
+                                                     DqSlots *slots, uint32_t launch, uint32_t patience, DqHostNote note,
                                                      mi_dq_params *__restrict__ params, int8_t *__restrict__ q) {
   __shared__ float slo[T / 64], shi[T / 64], all[2];
   __shared__ int late_wg;
   const int tid = threadIdx.x, w = blockIdx.x, wgs = gridDim.x;
   const int64_t n4 = n >> 2, first = (int64_t)w * (T * G) + tid;
   const v4f_any *x4 = reinterpret_cast<const v4f_any *>(x);
-  uint32_t turn = 0;
-  if (wgs > 1 && tid < 64) turn = __hip_atomic_load(&slots->turn[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 1;
+  const bool counted = launch == 0;  // the number of this launch stands in memory
+  unsigned long long replay = 0;
+  if (counted && wgs > 1 && tid < 64)
+    replay = __hip_atomic_load(&slots->replays, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
   v4f v[G];
   float lo = FLT_MAX, hi = -FLT_MAX;
   if (n4 > 0) {
@@ -260,34 +270,41 @@ __global__ __launch_bounds__(T) void dq_fused_kernel(const float *__restrict__ x
         lo = slo[i] < lo ? slo[i] : lo;
         hi = shi[i] > hi ? shi[i] : hi;
       }
-      const uint64_t mine = (uint64_t)__float_as_uint(hi) << 32 | __float_as_uint(lo);
+      const uint32_t tag = counted ? (uint32_t)replay | kDqReplayed : launch;
+      const uint64_t my_lo = (uint64_t)tag << 32 | __float_as_uint(lo), my_hi = (uint64_t)tag << 32 | __float_as_uint(hi);
       for (int s = w + tid * wgs; s < kDqSlots; s += 64 * wgs) {
-        __hip_atomic_store(&slots->range[turn][s], mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(&slots->range[turn ^ 1][s], kDqEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(&slots->turn[s], turn ^ 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&slots->range[s][0], my_lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&slots->range[s][1], my_hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
       const uint64_t began = __builtin_amdgcn_s_memrealtime();
       bool late = false;
-      uint64_t got[kDqSlots / 64];
+      // (16 bytes a load, past the caches of this XCD: two words that need not belong together, hence a tag in each)
+      const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(slots->range, (short)0, sizeof(slots->range), 0x00020000);
+      typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+      v4u got[kDqSlots / 64];
       while (true) {
-        bool missing = false;
 #pragma unroll
         for (int i = 0; i < kDqSlots / 64; ++i) {
           const int s = tid + i * 64;
-          got[i] = s < wgs ? __hip_atomic_load(&slots->range[turn][s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : mine;
+          got[i] = v4u{(uint32_t)my_lo, tag, (uint32_t)my_hi, tag};
+          if (i * 64 < wgs)
+            got[i] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(rsrc, 16 * (s < wgs ? s : w), 0, kAgentScope));
         }
+        asm volatile("" ::: "memory");  // (requested anew every time round)
+        bool missing = false;
 #pragma unroll
-        for (int i = 0; i < kDqSlots / 64; ++i) missing |= got[i] == kDqEmpty;
+        for (int i = 0; i < kDqSlots / 64; ++i) missing |= got[i][1] != tag || got[i][3] != tag;
         if (!__any(missing)) break;
         if (__builtin_amdgcn_s_memrealtime() - began > patience) {
           late = true;
           break;
         }
       }
+      if (counted && tid == 0 && (w == 0 || late)) atomicMax(&slots->replays, replay);
       if (!late) {
 #pragma unroll
         for (int i = 0; i < kDqSlots / 64; ++i) {
-          const float l2 = __uint_as_float((uint32_t)got[i]), h2 = __uint_as_float((uint32_t)(got[i] >> 32));
+          const float l2 = __uint_as_float(got[i][0]), h2 = __uint_as_float(got[i][2]);
           lo = l2 < lo ? l2 : lo;
           hi = h2 > hi ? h2 : hi;
         }
@@ -513,15 +530,15 @@ int launch_dynquant_segments(const float *x, int64_t segments, int64_t unit, int
 }
 
 template <int T, int G>
-static void launch_fused(const float *x, int64_t n, int symmetric, void *slots, const DqHostNote &note,
+static void launch_fused(const float *x, int64_t n, int symmetric, void *slots, uint32_t launch, const DqHostNote &note,
                          mi_dq_params *params, int8_t *q, hipStream_t stream) {
   const int64_t wgs = ((n >> 2) + T * G - 1) / (T * G);
   hipLaunchKernelGGL((dq_fused_kernel<T, G>), dim3(wgs < 1 ? 1 : (unsigned)wgs), dim3(T), 0, stream, x, n, symmetric,
-                     static_cast<DqSlots *>(slots), kDqPatience, note, params, q);
+                     static_cast<DqSlots *>(slots), launch, kDqPatience, note, params, q);
 }
 
-int launch_dynquant(const float *x, int64_t n, int symmetric, float2 *partials, void *slots, const DqHostNote &note,
-                    mi_dq_params *params, int8_t *q, hipStream_t stream) {
+int launch_dynquant(const float *x, int64_t n, int symmetric, float2 *partials, void *slots, uint32_t launch,
+                    const DqHostNote &note, mi_dq_params *params, int8_t *q, hipStream_t stream) {
   // One launch as long as the tensor fits the registers of one workgroup per CU.  Up to 8192 values one workgroup is
   // faster than any exchange (about 1.2 us); from there on as many workgroups as there are slots, with the fewest
   // values per thread that allows: what counts at these sizes is the latency of each thread's chain.  us per tensor,
@@ -529,11 +546,11 @@ int launch_dynquant(const float *x, int64_t n, int symmetric, float2 *partials, 
   // 32768 7.2 -> 4.2, 88064 7.4 -> 4.4, 300000 7.7 -> 5.0, 1 M 8.0 -> 5.6, 4096 x 768 11.3 -> 8.9,
   // 2048 x 4096 20.0 -> 13.5, 4096 x 3072 26.9 -> 17.5, 2048 x 11008 40.8 -> 26.7.
   const int64_t n4 = n >> 2;
-#define MI_DQ_FUSED(T, G)                                                   \
-  do {                                                                      \
-    launch_fused<T, G>(x, n, symmetric, slots, note, params, q, stream);    \
-    MI_HIP_CHECK(hipGetLastError());                                        \
-    return MI_OK;                                                           \
+#define MI_DQ_FUSED(T, G)                                                        \
+  do {                                                                           \
+    launch_fused<T, G>(x, n, symmetric, slots, launch, note, params, q, stream); \
+    MI_HIP_CHECK(hipGetLastError());                                             \
+    return MI_OK;                                                                \
   } while (0)
   constexpr int64_t kMost = kDqFusedMost;
   if (n4 <= 256) MI_DQ_FUSED(256, 1);

@@ -311,3 +311,44 @@ def test_dynamic_quant_parameters_do_not_wait_for_later_work(orc, unfetched):
         done = time.perf_counter()
     assert (p.scale, p.zero_point) == orc.dynamic_quant(x)[1:]
     assert known - queued < 0.25 * (done - began), (queued - began, known - queued, done - began)
+
+
+def test_dynamic_quant_runs_that_overlapped_spoil_no_later_run(orc):
+    """Runs of one handle that overlap on two streams have unspecified results (every wait in the kernel is bounded); those
+    that follow in order are right and wait for nobody."""
+    import torch
+    lib = K._lib
+    L = lib.load()
+    rng = np.random.default_rng(12)
+    xs = [_values(rng, n) for n in (40000, 260000, 1200000, 9000)]
+    devs = [torch.from_numpy(x).cuda() for x in xs]
+    qs = [torch.empty(x.size, dtype=torch.int8, device="cuda") for x in xs]
+    want = [orc.dynamic_quant(x) for x in xs]
+    dq = K.DynamicQuantKernel(False)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+
+    def run(i, stream):
+        assert L.mi_dynquant_run(dq._h, devs[i].data_ptr(), xs[i].size, qs[i].data_ptr(), stream.cuda_stream) == lib.MI_OK
+
+    for overlap in range(5):
+        for it in range(20):
+            run(it % 4, streams[0])
+            run((it + 1 + overlap) % 4, streams[1])
+        torch.cuda.synchronize()
+        for i in range(4):
+            qs[i].zero_()
+        torch.cuda.synchronize()
+        for i in range(4):
+            run(i, streams[0])
+        streams[0].synchronize()
+        for i in range(4):
+            assert np.array_equal(qs[i].cpu().numpy(), want[i][0]), (overlap, i)
+        first, last = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        with torch.cuda.stream(streams[0]):
+            first.record()
+            for it in range(40):
+                run(it % 4, streams[0])
+            last.record()
+        last.synchronize()
+        assert first.elapsed_time(last) / 40 < 0.15, "ms per run; a workgroup that waits in vain takes 0.2"
