@@ -11,6 +11,7 @@
 #include <atomic>
 #include <chrono>
 #include <memory>
+#include <mutex>
 #include <new>
 #include <vector>
 
@@ -165,6 +166,60 @@ struct DevBuf {
     p = nullptr;
     bytes = 0;
   }
+};
+
+// Page-locked notes of kDqHostWords words (mi_dynquant::note).  An allocation of its own takes 30 us and 200 to give
+// back, the rest of a handle 17 and 3, so handles share pages; a page goes back with the last note in it.
+class NotePages {
+ public:
+  static uint64_t *take() {  // zeroed; null if there is no page-locked memory
+    std::lock_guard<std::mutex> lock(mutex_);
+    Page *page = first_;
+    while (page != nullptr && page->used == ~(uint64_t)0) page = page->next;
+    if (page == nullptr) {
+      page = new (std::nothrow) Page();
+      if (page == nullptr) return nullptr;
+      if (hipHostMalloc(&page->p, 64 * kNoteBytes, hipHostMallocCoherent | hipHostMallocPortable) != hipSuccess) {
+        (void)hipGetLastError();
+        delete page;
+        return nullptr;
+      }
+      page->next = first_;
+      first_ = page;
+    }
+    const int i = __builtin_ctzll(~page->used);
+    page->used |= (uint64_t)1 << i;
+    char *note = static_cast<char *>(page->p) + i * kNoteBytes;
+    memset(note, 0, kNoteBytes);
+    return reinterpret_cast<uint64_t *>(note);
+  }
+  static void give(uint64_t *note) {  // nothing on the device writes it any more
+    if (note == nullptr) return;
+    std::lock_guard<std::mutex> lock(mutex_);
+    for (Page **link = &first_; *link != nullptr; link = &(*link)->next) {
+      Page *page = *link;
+      const ptrdiff_t at = reinterpret_cast<char *>(note) - static_cast<char *>(page->p);
+      if (at < 0 || at >= (ptrdiff_t)(64 * kNoteBytes)) continue;
+      page->used &= ~((uint64_t)1 << (at / kNoteBytes));
+      if (page->used == 0) {
+        *link = page->next;
+        (void)hipHostFree(page->p);
+        delete page;
+      }
+      return;
+    }
+  }
+
+ private:
+  static constexpr size_t kNoteBytes = 64;  // a cache line each
+  static_assert(kDqHostWords * sizeof(uint64_t) <= kNoteBytes, "a note fits its line");
+  struct Page {
+    void *p = nullptr;
+    uint64_t used = 0;
+    Page *next = nullptr;
+  };
+  static inline std::mutex mutex_;
+  static inline Page *first_ = nullptr;
 };
 
 // Where a run takes temporary device memory from: a buffer of the handle that grows on demand, or a fixed region
@@ -457,7 +512,7 @@ struct mi_conv {
 struct mi_dynquant {
   int symmetric = 0;
   DevBuf partials, slots, params, h_in, h_out, h_params;
-  // Where a run leaves its parameters for the host that asks for them: page-locked, made with the handle, or absent (every
+  // Where a run leaves its parameters for the host that asks for them: page-locked, taken with the handle, or absent (every
   // fetch is then a copy).  Polled by the host (mi_dynquant_await_params) they are there a few microseconds after the launch; a
   // copy and a stream synchronisation behind it took 22 us more (197 x 768: 34 us per run and fetch -> 10.5, and 16 for
   // mi_dynquant_get_params, which waits for the stream).  Writing to host memory lengthens the kernel, so only the first run
@@ -473,7 +528,7 @@ struct mi_dynquant {
   uint32_t launches = 0;  // number of the last launch (kDqReplayed - 1 is followed by 1)
   ~mi_dynquant() {
     params.release();  // (waits for the device: no run still writes the note)
-    if (note != nullptr) (void)hipHostFree(note);
+    NotePages::give(note);
   }
 };
 
@@ -1200,13 +1255,7 @@ int mi_dynquant_create(int32_t symmetric, mi_dynquant **out) {
   }
   MI_HIP_CHECK(hipMemset(h->slots.p, 0, kDqSlotBytes));
   MI_HIP_CHECK(hipStreamSynchronize(nullptr));  // runs may come in on any stream
-  void *note = nullptr;
-  if (hipHostMalloc(&note, kDqHostWords * sizeof(uint64_t), hipHostMallocCoherent) == hipSuccess) {
-    memset(note, 0, kDqHostWords * sizeof(uint64_t));
-    h->note = static_cast<uint64_t *>(note);
-  } else {
-    (void)hipGetLastError();
-  }
+  h->note = NotePages::take();
   *out = owner.release();
   return MI_OK;
 }

@@ -352,3 +352,27 @@ def test_dynamic_quant_runs_that_overlapped_spoil_no_later_run(orc):
             last.record()
         last.synchronize()
         assert first.elapsed_time(last) / 40 < 0.15, "ms per run; a workgroup that waits in vain takes 0.2"
+
+
+def test_dynamic_quant_handles_by_the_hundred(orc):
+    """More handles than one page of parameter notes holds, some destroyed and made again: each fetches its own parameters."""
+    import torch
+    x = _values(np.random.default_rng(2), 3000)
+    dev = torch.from_numpy(x).cuda()
+    want = {}
+    handles = {}
+    for turn in range(3):
+        for i in range(130):
+            if i % 3 == turn:
+                handles.pop(i, None)
+                handles[i] = K.DynamicQuantKernel(False)
+            elif i not in handles:
+                handles[i] = K.DynamicQuantKernel(True)
+        for repeat in range(2):
+            for i, dq in handles.items():
+                n = 1000 + 10 * i
+                key = (n, i % 3 <= turn)
+                if key not in want:
+                    want[key] = orc.dynamic_quant(x[:n], not key[1])[1:]
+                _, p = dq.run(dev[:n])
+                assert (p.scale, p.zero_point) == want[key], (turn, i)
