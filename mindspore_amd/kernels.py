@@ -12,6 +12,7 @@ behaviour: construction = Prepare(), ``run`` = Run()):
 (device tensors: computed in place on torch's current stream, no copies).  torch is only used as a device-memory
 and stream provider.  A call on device tensors is one call of the native module csrc/device_calls.cc, which checks the
 operand, allocates the output and calls the C ABI; it returns NotImplemented for anything that is not a torch tensor.
+Host tensors need neither torch nor that module.
 """
 import ctypes as C
 from collections import namedtuple
@@ -38,8 +39,14 @@ def _quant_arrays(params):
     return len(params), scales, zps
 
 
+def _host(a):
+    if type(a).__module__.startswith("torch"):
+        raise RuntimeError("torch tensors need the native module of the device calls: %s" % _lib.device_calls_missing())
+    return np.ascontiguousarray(a)
+
+
 def _host_i8(a):
-    a = np.ascontiguousarray(a)
+    a = _host(a)
     if a.dtype != np.int8:
         raise TypeError("expected an int8 tensor, got %s" % a.dtype)
     return a
@@ -166,8 +173,10 @@ class FullconnectionInt8Kernel(MatmulInt8Kernel):
 def matmul_run_group(kernels, a, outs=None):
     """Runs several MatmulInt8Kernel objects that share the input `a` (a contiguous CUDA int8 tensor [..., K]) as
     mi_matmul_run_group does: decode-sized inputs go out as one launch.  Returns the list of outputs."""
-    y = kernels[0]._device.matmul_run_group(kernels, a, kernels[0].k, outs)
+    device = kernels[0]._device
+    y = NotImplemented if device is None else device.matmul_run_group(kernels, a, kernels[0].k, outs)
     if y is NotImplemented:
+        _host(a)
         raise ValueError("expected a contiguous CUDA int8 tensor [..., %d]" % kernels[0].k)
     return y
 
@@ -177,8 +186,11 @@ def dynmm_run_group(kernels, a, in_quant=None, params_dev=None, row_params=None,
     as mi_dynmm_run_group does: decode-sized inputs go out as one launch.  The input's quantisation comes as one
     QuantParam (in_quant), as the address of the block a DynamicQuantKernel.run left on the device (params_dev) or as
     the tensor DynamicQuantKernel.run_rows returned (row_params).  Returns the list of fp32 outputs."""
-    y = kernels[0]._device.dynmm_run_group(kernels, a, kernels[0].k, outs, in_quant, params_dev, row_params)
+    device = kernels[0]._device
+    y = (NotImplemented if device is None
+         else device.dynmm_run_group(kernels, a, kernels[0].k, outs, in_quant, params_dev, row_params))
     if y is NotImplemented:
+        _host(a)
         raise ValueError("expected a contiguous CUDA int8 tensor [..., %d]" % kernels[0].k)
     return y
 
@@ -261,7 +273,7 @@ class DynamicQuantKernel(_Handle):
         if self._device is not None:
             q = self._device.dynquant_run(self._raw, x, C.addressof(p) if fetch_params else 0)
         if q is NotImplemented:
-            x = np.ascontiguousarray(x)
+            x = _host(x)
             if x.dtype != np.float32:
                 raise TypeError("DynamicQuant needs a float32 input")  # dynamic_quant.cc:389-395
             q = np.empty(x.shape, np.int8)
@@ -286,7 +298,7 @@ class DynamicQuantKernel(_Handle):
                 return both
         L = _lib.load()
         unit = x.shape[-1]
-        x = np.ascontiguousarray(x)
+        x = _host(x)
         if x.dtype != np.float32:
             raise TypeError("DynamicQuant needs a float32 input")
         rows = x.size // unit

@@ -174,24 +174,31 @@ def load():
 
 
 _device_calls = None
+_device_calls_missing = None  # why there is none, once that is known
 
 
 def device_calls():
-    """The native module of the device-tensor calls, or None in a process without torch (no device tensors there)."""
-    global _device_calls
-    if _device_calls is None:
+    """The native module of the device-tensor calls, or None where there is none: in a process without torch, with a torch that
+    has no HIP libraries, or if the module was not built.  Host tensors need neither; device_calls_missing() says why."""
+    global _device_calls, _device_calls_missing
+    if _device_calls is None and _device_calls_missing is None:
         try:
             import torch
-        except ImportError:
+            if not os.path.exists(DEVICE_CALLS_PATH):
+                raise ImportError("%s is not built: run `python -m mindspore_amd.build`" % DEVICE_CALLS_PATH)
+            from . import _device_calls as module
+        except ImportError as e:
+            _device_calls_missing = str(e)
             return None
-        if not os.path.exists(DEVICE_CALLS_PATH):
-            raise RuntimeError("%s is not built: run `python -m mindspore_amd.build`" % DEVICE_CALLS_PATH)
-        from . import _device_calls as module
         L = load()
         module.bind({f: C.cast(getattr(L, f), C.c_void_p).value for f in DEVICE_CALLS_USES}, check,
                     torch.OutOfMemoryError)
         _device_calls = module
     return _device_calls
+
+
+def device_calls_missing():
+    return _device_calls_missing
 
 
 _diag = None

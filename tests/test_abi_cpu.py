@@ -154,3 +154,44 @@ def test_public_header_is_plain_c(tmp_path):
                 ["g++", "-std=c++11", "-Wall", "-Werror", "-x", "c++"]):
         p = subprocess.run(cmd + ["-I", inc, "-fsyntax-only", str(src)], capture_output=True, text=True)
         assert p.returncode == 0, p.stderr
+
+
+WITHOUT_TORCH = """
+import sys
+{hide}
+sys.path.insert(0, {root!r})
+import numpy as np
+from mindspore_amd import kernels as K, lib
+handle = K._Handle()
+handle._created()  # what every kernel's constructor ends with
+assert handle._device is None and lib.device_calls_missing(), lib.device_calls_missing()
+class Tensor:
+    shape = (4, 8)
+Tensor.__module__ = "torch"
+for call in (lambda: K._host_i8(Tensor()), lambda: K.matmul_run_group([type("Kernel", (), dict(_device=None, k=8))], Tensor())):
+    try:
+        call()
+        raise AssertionError("a device tensor without the native module must raise")
+    except RuntimeError as e:
+        assert lib.device_calls_missing() in str(e)
+{more}
+print("ok")
+"""
+HIDE_TORCH = {"none": "sys.modules['torch'] = None",
+              "without HIP": "sys.path.insert(0, {fake!r})\nimport torch"}  # an importable torch that brings no libraries
+
+
+def run_without_torch(tmp_path, torch, more=""):
+    """Runs `more` in a process without torch (or with one that has no HIP libraries)."""
+    import subprocess
+    import sys
+    (tmp_path / "torch").mkdir()
+    (tmp_path / "torch" / "__init__.py").write_text("class OutOfMemoryError(RuntimeError):\n    pass\n")
+    code = WITHOUT_TORCH.format(hide=HIDE_TORCH[torch].format(fake=str(tmp_path)), root=ROOT, more=more)
+    p = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100, cwd=str(tmp_path))
+    assert p.returncode == 0 and p.stdout.endswith("ok\n"), p.stdout + p.stderr
+
+
+@pytest.mark.parametrize("torch", sorted(HIDE_TORCH))
+def test_kernels_are_made_without_torch(L, tmp_path, torch):
+    run_without_torch(tmp_path, torch)

@@ -376,3 +376,19 @@ def test_dynamic_quant_handles_by_the_hundred(orc):
                     want[key] = orc.dynamic_quant(x[:n], not key[1])[1:]
                 _, p = dq.run(dev[:n])
                 assert (p.scale, p.zero_point) == want[key], (turn, i)
+
+
+@pytest.mark.parametrize("torch_is", ["none", "without HIP"])
+def test_host_tensors_without_torch(orc, tmp_path, torch_is):
+    from tests.test_abi_cpu import run_without_torch
+    rng = np.random.default_rng(6)
+    w, bias, sw, _, _ = _matmul_pair(rng, 40, 64, False, False)
+    a, x = rng.integers(-128, 128, (9, 64), dtype=np.int8), _values(rng, 700)
+    np.savez(tmp_path / "case.npz", w=w, bias=bias, sw=sw, a=a, x=x, want=orc.matmul_int8(a, w, bias, 0.02, 7, sw, np.zeros(40, np.int32), 0.5, 3),
+             q=orc.dynamic_quant(x)[0])
+    run_without_torch(tmp_path, torch_is, """
+c = np.load("case.npz")
+kern = K.MatmulInt8Kernel(c["w"], c["bias"], K.QuantParam(0.02, 7), [K.QuantParam(float(s), 0) for s in c["sw"]], K.QuantParam(0.5, 3))
+assert np.array_equal(kern.run(c["a"]), c["want"])
+assert np.array_equal(K.DynamicQuantKernel(False).run(c["x"])[0], c["q"])
+""")
