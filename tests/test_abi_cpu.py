@@ -195,3 +195,29 @@ def run_without_torch(tmp_path, torch, more=""):
 @pytest.mark.parametrize("torch", sorted(HIDE_TORCH))
 def test_kernels_are_made_without_torch(L, tmp_path, torch):
     run_without_torch(tmp_path, torch)
+
+
+@pytest.mark.parametrize("torch", [None, "without HIP"])
+def test_the_library_builds_without_torch(monkeypatch, torch):
+    import sys
+    import types
+    from mindspore_amd import build
+    assert build.device_calls_command()[0] == "g++"
+    fake = torch and types.ModuleType("torch")
+    if fake:
+        fake.version = types.SimpleNamespace(hip=None)
+    monkeypatch.setitem(sys.modules, "torch", fake)
+    ran = []
+
+    class Popen:
+        returncode = 0
+
+        def __init__(self, cmd, **kwargs):
+            ran.append(cmd)
+
+        def communicate(self):
+            return "", None
+    monkeypatch.setattr(build.subprocess, "Popen", Popen)
+    monkeypatch.setattr(build.subprocess, "check_call", ran.append)
+    build.build_library()
+    assert len(ran) == len(build.SOURCES) + 3 and all(cmd[0] == "hipcc" for cmd in ran)
