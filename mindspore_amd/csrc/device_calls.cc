@@ -30,6 +30,7 @@ struct Api {
   decltype(&mi_dynmm_run_group) dynmm_run_group;
 } api;
 PyObject *check_fn = nullptr;  // lib.check(code, what): raises MiError
+PyObject *address_fn = nullptr;  // lib.address(pointer): the address a ctypes pointer holds
 PyObject *memory_error = nullptr;  // torch.OutOfMemoryError
 PyObject *name_raw = nullptr, *name_n = nullptr, *name_scale = nullptr, *name_zero_point = nullptr;
 constexpr int kGroupMost = 64;  // members of one group call
@@ -87,6 +88,35 @@ const at::Tensor *given_out(PyObject *o, int64_t elements) {
   return nullptr;
 }
 
+// A device address: a whole number, or whatever ctypes takes for a void pointer.
+bool as_address(PyObject *o, const void **p) {
+  if (PyLong_Check(o)) {
+    *p = PyLong_AsVoidPtr(o);
+    return !PyErr_Occurred();
+  }
+  PyObject *v = PyObject_CallOneArg(address_fn, o);
+  if (v == nullptr) return false;
+  *p = PyLong_AsVoidPtr(v);
+  Py_DECREF(v);
+  return !PyErr_Occurred();
+}
+
+// float(o) and int(o), the latter into 32 bits as ctypes narrows it
+bool as_float(PyObject *o, double *x) {
+  PyObject *f = PyNumber_Float(o);
+  if (f == nullptr) return false;
+  *x = PyFloat_AS_DOUBLE(f);
+  Py_DECREF(f);
+  return true;
+}
+bool as_int32(PyObject *o, int32_t *x) {
+  PyObject *i = PyNumber_Long(o);
+  if (i == nullptr) return false;
+  *x = (int32_t)PyLong_AsUnsignedLongLongMask(i);
+  Py_DECREF(i);
+  return !PyErr_Occurred();
+}
+
 bool count_args(Py_ssize_t nargs, Py_ssize_t want) {
   if (nargs == want) return true;
   PyErr_Format(PyExc_TypeError, "expected %zd arguments, got %zd", want, nargs);
@@ -117,9 +147,9 @@ bool take(PyObject *addresses, const char *name, T *fn) {
   return !PyErr_Occurred();
 }
 
-// bind({entry point: address}, check, torch.OutOfMemoryError)
+// bind({entry point: address}, check, torch.OutOfMemoryError, address)
 PyObject *bind(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
-  if (!count_args(nargs, 3)) return nullptr;
+  if (!count_args(nargs, 4)) return nullptr;
   PyObject *d = args[0];
   if (!take(d, "mi_matmul_run", &api.matmul_run) || !take(d, "mi_matmul_run_group", &api.matmul_run_group) ||
       !take(d, "mi_conv_out_shape", &api.conv_out_shape) || !take(d, "mi_conv_run", &api.conv_run) ||
@@ -132,6 +162,8 @@ PyObject *bind(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   Py_XSETREF(check_fn, args[1]);
   Py_INCREF(args[2]);
   Py_XSETREF(memory_error, args[2]);
+  Py_INCREF(args[3]);
+  Py_XSETREF(address_fn, args[3]);
   Py_RETURN_NONE;
 }
 
@@ -267,18 +299,18 @@ struct InQuant {
       row_bytes = t.numel();
       per_row = 1;
     } else if (args[1] != Py_None) {
-      dev = static_cast<const mi_dq_params *>(PyLong_AsVoidPtr(args[1]));
+      const void *p = nullptr;
+      if (!as_address(args[1], &p)) return false;
+      dev = static_cast<const mi_dq_params *>(p);
     } else {
       PyObject *so = PyObject_GetAttr(args[0], name_scale);
       PyObject *zo = so == nullptr ? nullptr : PyObject_GetAttr(args[0], name_zero_point);
-      if (zo != nullptr) {
-        scale = PyFloat_AsDouble(so);
-        zp = (int32_t)PyLong_AsLongLong(zo);
-      }
+      const bool ok = zo != nullptr && as_float(so, &scale) && as_int32(zo, &zp);
       Py_XDECREF(so);
       Py_XDECREF(zo);
+      return ok;
     }
-    return !PyErr_Occurred();
+    return true;
   }
 };
 

@@ -192,9 +192,14 @@ def device_calls():
             return None
         L = load()
         module.bind({f: C.cast(getattr(L, f), C.c_void_p).value for f in DEVICE_CALLS_USES}, check,
-                    torch.OutOfMemoryError)
+                    torch.OutOfMemoryError, address)
         _device_calls = module
     return _device_calls
+
+
+def address(pointer):
+    """The address that `pointer` holds, for anything ctypes takes for a void pointer."""
+    return C.cast(pointer, C.c_void_p).value or 0
 
 
 def device_calls_missing():

@@ -392,3 +392,30 @@ kern = K.MatmulInt8Kernel(c["w"], c["bias"], K.QuantParam(0.02, 7), [K.QuantPara
 assert np.array_equal(kern.run(c["a"]), c["want"])
 assert np.array_equal(K.DynamicQuantKernel(False).run(c["x"])[0], c["q"])
 """)
+
+
+def test_dynamic_matmul_argument_forms(orc):
+    """The input's quantisation as Python programs hold it: whole and floating zero points, device addresses as numbers and as
+    ctypes pointers, for one kernel and for a group."""
+    import ctypes as C
+    import torch
+    rng = np.random.default_rng(9)
+    w, bias, sw, zw, make = _matmul_pair(rng, 48, 96, True, True)
+    kern = make(True)
+    x = _values(rng, 5 * 96).reshape(5, 96)
+    dq = K.DynamicQuantKernel(False)
+    q, p = dq.run(torch.from_numpy(x).cuda())
+    want = orc.dynamic_matmul(q.cpu().numpy(), w, bias, p.scale, p.zero_point, sw, zw)
+
+    def check(**args):
+        for y in [kern.run(q, **args)] + K.dynmm_run_group([kern, kern], q, **args):
+            assert np.array_equal(y.cpu().numpy().view(np.uint32), want.view(np.uint32)), args
+
+    for scale in (p.scale, np.float64(p.scale), np.array(p.scale)):
+        for zero_point in (p.zero_point, float(p.zero_point), np.float32(p.zero_point), np.int64(p.zero_point)):
+            check(in_quant=K.QuantParam(scale, zero_point))
+    addr = dq.device_params()
+    for params in (addr, C.c_void_p(addr), C.cast(addr, C.POINTER(K._lib.DqParams))):
+        check(params_dev=params)
+    with pytest.raises((TypeError, C.ArgumentError)):
+        kern.run(q, params_dev=1.5)
