@@ -288,6 +288,7 @@ struct InQuant {
   int32_t zp = 0, per_row = 0;
   int64_t row_bytes = 0;
   const mi_dq_params *dev = nullptr;
+  bool chained = false;  // an address was given (a null one is the library's to refuse)
   bool fill(PyObject *const *args) {
     if (args[2] != Py_None) {  // the tensor of parameter blocks that dynquant_run_rows made
       if (!THPVariable_Check(args[2])) {
@@ -302,6 +303,7 @@ struct InQuant {
       const void *p = nullptr;
       if (!as_address(args[1], &p)) return false;
       dev = static_cast<const mi_dq_params *>(p);
+      chained = true;
     } else {
       PyObject *so = PyObject_GetAttr(args[0], name_scale);
       PyObject *zo = so == nullptr ? nullptr : PyObject_GetAttr(args[0], name_zero_point);
@@ -335,10 +337,10 @@ PyObject *dynmm_run(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     float *cp = static_cast<float *>(out.data_ptr());
     mi_dynmm *mm = static_cast<mi_dynmm *>(h);
     void *s = stream();
-    const char *what = q.per_row ? "mi_dynmm_run_rows" : q.dev != nullptr ? "mi_dynmm_run_chained" : "mi_dynmm_run";
+    const char *what = q.per_row ? "mi_dynmm_run_rows" : q.chained ? "mi_dynmm_run_chained" : "mi_dynmm_run";
     if (!call_library(what, [&] {
           if (q.per_row) return api.dynmm_run_rows(mm, ap, (int32_t)rows, q.dev, cp, s);
-          if (q.dev != nullptr) return api.dynmm_run_chained(mm, ap, (int32_t)rows, q.dev, cp, s);
+          if (q.chained) return api.dynmm_run_chained(mm, ap, (int32_t)rows, q.dev, cp, s);
           return api.dynmm_run(mm, ap, (int32_t)rows, q.scale, q.zp, cp, s);
         }))
       return nullptr;

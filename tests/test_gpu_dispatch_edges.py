@@ -419,3 +419,14 @@ def test_dynamic_matmul_argument_forms(orc):
         check(params_dev=params)
     with pytest.raises((TypeError, C.ArgumentError)):
         kern.run(q, params_dev=1.5)
+
+
+def test_dynamic_matmul_refuses_a_null_parameter_block():
+    import ctypes as C
+    import torch
+    kern = K.MatmulDynamicInt8Kernel(np.ones((8, 16), np.int8), None, [K.QuantParam(0.1, 0)])
+    q = torch.ones((2, 16), dtype=torch.int8, device="cuda")
+    for null in (0, C.c_void_p(None)):
+        with pytest.raises(K._lib.MiError) as e:
+            kern.run(q, params_dev=null)
+        assert e.value.code == K._lib.MI_NULL_PTR
