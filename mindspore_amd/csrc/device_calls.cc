@@ -33,7 +33,6 @@ PyObject *check_fn = nullptr;  // lib.check(code, what): raises MiError
 PyObject *address_fn = nullptr;  // lib.address(pointer): the address a ctypes pointer holds
 PyObject *memory_error = nullptr;  // torch.OutOfMemoryError
 PyObject *name_raw = nullptr, *name_n = nullptr, *name_scale = nullptr, *name_zero_point = nullptr;
-constexpr int kGroupMost = 64;  // members of one group call
 
 // Runs `call` without the interpreter lock; false with a Python error set when it failed.
 template <typename F>
@@ -198,7 +197,7 @@ PyObject *matmul_run(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
 // The members of a group call: handles, and the outputs given or made.
 struct Group {
   int count = 0;
-  void *handle[kGroupMost], *out[kGroupMost];
+  c10::SmallVector<void *, 8> handle, out;
   PyObject *outs = nullptr;  // what the call returns: the caller's sequence, or a new list
   ~Group() { Py_XDECREF(outs); }
   bool fill(PyObject *kernels, PyObject *given, const at::Tensor &a, at::ScalarType type) {
@@ -212,11 +211,13 @@ struct Group {
  private:
   bool fill_from(PyObject *seq, PyObject *given, const at::Tensor &a, at::ScalarType type) {
     const Py_ssize_t members = PySequence_Fast_GET_SIZE(seq);
-    if (members > kGroupMost) {
-      PyErr_Format(PyExc_ValueError, "at most %d kernels in a group", kGroupMost);
+    if (members > INT_MAX) {
+      PyErr_SetString(PyExc_ValueError, "too many kernels");
       return false;
     }
     count = (int)members;
+    handle.resize(members);
+    out.resize(members);
     if (given == Py_None) {
       outs = PyList_New(count);
       if (outs == nullptr) return false;
@@ -272,8 +273,8 @@ PyObject *matmul_run_group(PyObject *, PyObject *const *args, Py_ssize_t nargs) 
     const int32_t rows = (int32_t)(a->numel() / k);
     void *s = stream();
     if (!call_library("mi_matmul_run_group", [&] {
-          return api.matmul_run_group(reinterpret_cast<mi_matmul *const *>(g.handle), g.count, ap, rows,
-                                      reinterpret_cast<int8_t *const *>(g.out), s);
+          return api.matmul_run_group(reinterpret_cast<mi_matmul *const *>(g.handle.data()), g.count, ap, rows,
+                                      reinterpret_cast<int8_t *const *>(g.out.data()), s);
         }))
       return nullptr;
     Py_INCREF(g.outs);
@@ -363,8 +364,8 @@ PyObject *dynmm_run_group(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     const int32_t rows = (int32_t)(a->numel() / k);
     void *s = stream();
     if (!call_library("mi_dynmm_run_group", [&] {
-          return api.dynmm_run_group(reinterpret_cast<mi_dynmm *const *>(g.handle), g.count, ap, rows, q.scale, q.zp, q.dev,
-                                     q.per_row, reinterpret_cast<float *const *>(g.out), s);
+          return api.dynmm_run_group(reinterpret_cast<mi_dynmm *const *>(g.handle.data()), g.count, ap, rows, q.scale, q.zp, q.dev,
+                                     q.per_row, reinterpret_cast<float *const *>(g.out.data()), s);
         }))
       return nullptr;
     Py_INCREF(g.outs);

@@ -430,3 +430,16 @@ def test_dynamic_matmul_refuses_a_null_parameter_block():
         with pytest.raises(K._lib.MiError) as e:
             kern.run(q, params_dev=null)
         assert e.value.code == K._lib.MI_NULL_PTR
+
+
+@pytest.mark.parametrize("dynamic", [False, True])
+def test_group_of_many_kernels(dynamic):
+    import torch
+    rng = np.random.default_rng(10)
+    kernels = [_matmul_pair(rng, n, 32, False, dynamic)[4](True) for n in range(1, 101)]
+    a = torch.from_numpy(rng.integers(-128, 128, (3, 32), dtype=np.int8)).cuda()
+    args = dict(in_quant=K.QuantParam(0.03, -5)) if dynamic else {}
+    outs = K.dynmm_run_group(kernels, a, **args) if dynamic else K.matmul_run_group(kernels, a)
+    assert len(outs) == 100
+    for kern, y in zip(kernels, outs):
+        assert torch.equal(y, kern.run(a, **args))
