@@ -268,6 +268,11 @@ class DynamicQuantKernel(_Handle):
         self.last = None
 
     def run(self, x, fetch_params=True):
+        """x: fp32 as a numpy array (host path) or a contiguous CUDA tensor (device path, current stream).  On the device path
+        the call returns as soon as the parameters are known, when the last values of q may still be on their way: q is
+        complete for everything on the same stream, and another stream or a host copy of its own has to be ordered behind
+        this one, as for any torch operation.  fetch_params=False returns (q, None) without waiting; device_params() then
+        hands the parameters on in device memory.  The runs of one object are ordered by their stream, or by events."""
         p = _lib.DqParams()
         q = NotImplemented
         if self._device is not None:
