@@ -475,10 +475,21 @@ static int launch_conv_pick_tile(const GemmArgs &g, const ConvGather &cv, const 
   // launch, three per CU / four: 8 x 28 x 28, 3x3, 96 -> 192 channels 11.0 / 7.4, 1x1 there 5.6 / 4.3; with few enough tiles for one
   // round of three no change (8 x 40 x 40, 48 -> 48 4.7; one 56 x 56 image, 64 -> 64 5.0).  64 x 128 tiles at 16 x 50 x 50,
   // 32 -> 32 5.9, these 5.7.
-  // Where up to 64 channels give them more than one and a half rounds: the same number of pixels at once on 64 x 256 tiles,
-  // which read the weights a quarter as often (32 x 56 x 56, 64 -> 64 14.0 -> 12.5).
+  // Up to 64 channels, 64 x 256 tiles, two per CU: the same number of pixels at once, weights read a quarter as often, but a
+  // round of them (1024 rows of 128 pixels) is two of the small ones.  They win (a) where their last round is more than three
+  // quarters full, unless the contraction is so short that prologue and stores are most of a tile, and (b) over several rounds
+  // once the contraction pays for what the last one wastes.  us per launch, small /
+  // tall, 64 -> 64 channels 3x3 (K = 576): 640 rows 10.4 / 12.0, 768 11.8 / 12.1, 800 13.0 / 12.2, 1024 14.8 / 13.5,
+  // 1040 16.2 / 19.6, 1600 22.2 / 23.4, 2048 29.9 / 24.3, 3000 40.4 / 35.3; time of the tall ones relative to the small ones
+  // at 1100 / 1400 / 1664 / 2300 / 3200 / 4300 rows: K = 288 1.19 1.05 1.06 1.04 1.03 0.91, with stride 2 1.27 1.12 1.11
+  // 1.18 1.15 0.96, K = 576 1.13 1.00 1.01 1.00 0.88 0.86, stride 2 1.18 1.00 1.06 0.89 0.87 0.86, K = 864 1.08 0.93 0.91
+  // 0.89 0.83 0.79, K = 144 1.28 1.12 1.16 1.15 1.15 1.09; (a) at 900 / 1950 rows: K = 144 0.99 1.05 (32 channels 0.92
+  // 0.92), K = 288 0.98 0.93, stride 2 1.01 1.06, K = 576 0.89 0.88, stride 2 0.93 1.01; at 900 rows 1x1 with K = 64 1.08.
   // 128 x 128 tiles against more channels as soon as there are enough of them (32 x 28 x 28, 64 -> 128 7.2, on 64 x 64 9.1).
-  if (g.n <= 64 && (g.m + 127) / 128 > 768) return launch_conv_cfg<64, 256, HAS_ZW, FAST, 4, 2>(g, cv, rq, stream);
+  const int64_t rows = (g.m + 127) / 128;
+  const bool full_last_round = (rows - 1) % 1024 >= 768 && g.k >= (g.n <= 32 ? 144 : 288 * cv.stride_w);
+  const bool many_rounds = rows >= 1400 && rows * g.k >= 1300000;
+  if (g.n <= 64 && (full_last_round || many_rounds)) return launch_conv_cfg<64, 256, HAS_ZW, FAST, 4, 2>(g, cv, rq, stream);
   if (g.n > 64 && tiles_m >= 128) return launch_conv_cfg<128, 128, HAS_ZW, FAST, 4, 2>(g, cv, rq, stream);
   return launch_conv_cfg<64, 64, HAS_ZW, FAST, 4, 4>(g, cv, rq, stream);
 }

@@ -197,8 +197,12 @@ def test_conv_1x1_few_channels(orc, b, ih, iw, ic, oc):
 
 
 @pytest.mark.parametrize("b,ih,iw,ic,oc", [(1, 12, 11, 16, 7), (2, 31, 33, 48, 64), (1, 40, 41, 32, 65), (2, 91, 90, 16, 130),
-                                           (8, 111, 111, 16, 64),  # 771 rows of 128 pixels: 64 x 256 tiles
-                                           (8, 110, 111, 16, 33)])  # 764: 64 x 64
+                                           # rows of 128 pixels: 771, K = 144: 64 x 64 tiles, with up to 32 channels 64 x 256
+                                           (8, 111, 111, 16, 64), (8, 111, 111, 16, 32),
+                                           (8, 110, 111, 16, 33),  # 764: 64 x 64
+                                           (8, 111, 111, 32, 64),  # 771, K = 288: 64 x 256
+                                           (8, 128, 128, 32, 50), (8, 128, 129, 32, 50),  # 1024: 64 x 256; 1032: 64 x 64
+                                           (4, 219, 219, 96, 37), (4, 221, 219, 96, 37)])  # 1499, 1513, K = 864: either side
 def test_conv_gather_tiles(orc, b, ih, iw, ic, oc):
     """Either side of the rules by which the gathering GEMM picks its tile, with and without weight zero points."""
     from tests.test_gpu_parity import _conv_case, _gpu_conv
