@@ -22,7 +22,7 @@ sys.path.insert(0, ROOT)
 PEAK_INT8_TOPS = 5000.0  # MI355X dense int8 MFMA peak, TOP/s (5.0 POP/s)
 PEAK_HBM_GBPS = 8000.0   # MI355X HBM3E peak, GB/s
 
-HEADLINE_KERNEL = "mi::gemm_kblock_kernel<0, false, true>"
+HEADLINE_KERNEL = "mi::gemm_kblock_kernel<4, 4, 0, false, true, true>"
 # HBM-side bytes per launch of the dominant kernel come from `rocprofv3 --pmc FETCH_SIZE` / `--pmc WRITE_SIZE` runs of
 # this script, each scaled by what the same counter reads for the 256 MiB copy of --calibrate.  The figures are read
 # from the committed summary of those runs, which also names the kernel and the commit it was measured at, so that

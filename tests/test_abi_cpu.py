@@ -221,3 +221,13 @@ def test_the_library_builds_without_torch(monkeypatch, torch):
     monkeypatch.setattr(build.subprocess, "check_call", ran.append)
     build.build_library()
     assert len(ran) == len(build.SOURCES) + 3 and all(cmd[0] == "hipcc" for cmd in ran)
+
+
+def test_the_benchmark_names_kernels_that_exist(L):
+    """The kernel bench.py reports for the headline GEMM is in the library, and the committed traffic figure is that kernel's."""
+    import subprocess
+    import bench
+    symbols = subprocess.run(["nm", "-C", lib.LIB_PATH], capture_output=True, text=True, check=True).stdout
+    name = bench.HEADLINE_KERNEL.replace("mi::", "")
+    assert "mi::__device_stub__%s(" % name in symbols
+    assert bench.measured_traffic("gemm4096")["kernel"] == bench.HEADLINE_KERNEL
