@@ -11,14 +11,16 @@
 // one output row: the epilogue packs them into one 32-bit store, per-channel parameters are 16-byte loads, and
 // the input-row sum a lane needs is the one it accumulated itself (v_dot4 against 0x01010101).
 //
-// Two main loops, both moving tiles global -> LDS with asynchronous 16-byte-per-lane loads and reading operand
-// fragments for the next K sub-step from LDS while the MFMAs of the current one run:
-//   * K blocks of 128 bytes (gemm_kblock_body): whole cache lines per load, five LDS slots, one barrier per block;
-//     256 x 256 tiles with one workgroup per CU for the large compute-bound shapes, 128 x 128 tiles with two
-//     workgroups per CU for the mid-sized ones;
-//   * K steps of 64 bytes through NST LDS stages (gemm_direct_body): the smaller tiles, up to four workgroups per
-//     CU, the few-rows weight stream (NST = 8 / 16) and the convolution whose activation operand is gathered from
-//     the image.
+// Three main loops, all moving tiles global -> LDS with asynchronous 16-byte-per-lane loads and reading operand
+// fragments for the next K sub-step from LDS while the MFMAs of the current one run.  Handles hold their weights in
+// 1 KiB matrix-core blocks beside the row-major form, and with those nearly every shape runs on K blocks of 128 bytes, on
+// the tile that launch_pick_tile expects to be the quickest:
+//   * gemm_kblock.hip: five LDS slots, one barrier per block; 256 x 256 and 192 x 256 tiles, one workgroup per CU, for the
+//     large shapes, 128 x 128 tiles, two per CU, where fp32 stores have to overlap another tile's loop;
+//   * gemm_ring.hip: a ring of stages that hold both operands, as deep as the LDS allows: every smaller tile;
+//   * gemm_direct_body below, K steps of 64 bytes through NST LDS stages over row-major weights: short K, handles
+//     without the blocked copy (whose large shapes run on gemm_kblock.hip's row-major form) and the convolution whose
+//     activation operand is gathered from the image.
 // Any K that is a multiple of 16: the weights are zero padded, so an activation chunk past K only has to be a valid
 // read (it re-reads the row's last chunk).  LDS rows are XOR-swizzled in units of 16 bytes so that the 16-byte
 // fragment reads of a wave are bank-conflict free.
@@ -71,10 +73,9 @@ __device__ __forceinline__ void hint_interleave_reads() {
 
 // =====================================================================================================================
 // direct main loop: NST LDS stages x 64 bytes of K, asynchronous global -> LDS loads NST - 1 tiles ahead.
-// NST = 4 for the compute-bound shapes (3 for short K, where a third workgroup per CU is worth more than depth); NST = 16 with 64 x 64 tiles for a few (<= 64) activation rows, where the
-// kernel is a weight stream and what counts is the number of bytes in flight per CU.
-// OCC = workgroups the register allocation leaves room for on one CU (waves per SIMD): 1 for the 256 x 256 tile, which
-// needs the whole register file, 2 for the 128 x 128 tile.
+// NST = 4 in general (3 for short K, where a third workgroup per CU is worth more than depth); NST = 8 and 16 for handles
+// without the blocked copy where few tiles walk a long K, a weight stream in which the number of bytes in flight per CU counts.
+// OCC = workgroups the register allocation leaves room for on one CU (waves per SIMD).
 // =====================================================================================================================
 // CONV: the activation operand is not a matrix in memory but the im2col view of an NHWC image (in_c % 16 == 0): row m
 // is output pixel m, and the 16-byte chunk at K offset k is 16 channels of tap k / in_c, fetched straight from the
@@ -174,7 +175,7 @@ __device__ __forceinline__ void gemm_direct_body(const GemmArgs &g, const Requan
 #pragma unroll
     for (int j = 0; j < TM; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = (int)kAccBias;  // see gemm_kblock_kernel
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = (int)kAccBias;  // see kAccBias
   int rowsum[TM];
 #pragma unroll
   for (int j = 0; j < TM; ++j) rowsum[j] = 0;
@@ -359,6 +360,7 @@ static int launch_pick_tile(const GemmArgs &g, const RequantParams &rq, const De
     return t.ring ? launch_gemm_ring(10 * t.tn + t.tm, EPI == EPI_REQUANT, HAS_ZW, FAST, g, rq, dq, stream)
                   : launch_gemm_kblock(10 * t.tn + t.tm, EPI == EPI_REQUANT, HAS_ZW, FAST, g, rq, dq, stream);
   }
+  // From here on mostly handles without the blocked copy.
   // a few activation rows against a big weight matrix: one row of 64 x 64 tiles, deep prefetch (HBM-bound)
   if (g.m <= 64 && g.k_pad >= 1024) return launch_cfg<64, 64, EPI, HAS_ZW, FAST, 16>(g, rq, dq, stream);
   if (g.m <= 128 && g.k_pad >= 1024) return launch_cfg<64, 128, EPI, HAS_ZW, FAST, 8>(g, rq, dq, stream);

@@ -5,12 +5,12 @@
 namespace mi {
 
 // =====================================================================================================================
-// The same K blocks of 128 bytes through a ring of S LDS stages that hold both operands, S - 1 blocks ahead.
+// The K blocks of gemm_kblock.hip through a ring of S LDS stages that hold both operands, S - 1 blocks ahead.
 //
-// A block of a tile smaller than 256 x 256 lasts 0.25 to 0.5 us on the matrix cores, and the fetch window of the loop above
+// A block of a tile smaller than 256 x 256 lasts 0.25 to 0.5 us on the matrix cores, and the fetch window of that loop
 // (two blocks for W, one and a half for A) is then shorter than the way to memory and back: 192 x 128 tiles, one per CU,
 // took 0.74 us a block for 0.38 us of MFMAs.  Where a CU has only one workgroup to run, the LDS that a second one would
-// need holds further stages instead.  Everything else is as above: four quarters per block, double-buffered fragments,
+// need holds further stages instead.  Everything else is as there: four quarters per block, double-buffered fragments,
 // one barrier per block between quarter three and four; the loads of block b + S - 1 are spread over quarters 1 to 3 of
 // block b and quarter 4 of the block before, which is the first moment its stage is free.
 // Bound by the loads, where weights come from HBM: without its MFMAs the loop takes as long (512 x 12288 x 4096 29.8 of 30.1 us), with
