@@ -321,8 +321,11 @@ static int launch_kblock(GemmArgs g, const RequantParams &rq, const DequantParam
   const dim3 grid(g.tiles_m * g.tiles_n);
   if (g.wb != nullptr) {
     hipLaunchKernelGGL((gemm_kblock_kernel<TN, TM, EPI, HAS_ZW, FAST, true>), grid, dim3(256), 0, stream, g, rq, dq);
-  } else {
+  } else if constexpr (TN == TM) {
     hipLaunchKernelGGL((gemm_kblock_kernel<TN, TM, EPI, HAS_ZW, FAST, false>), grid, dim3(256), 0, stream, g, rq, dq);
+  } else {  // (rectangular tiles are chosen for the blocked copy only)
+    set_error("gemm: the blocked weight copy is missing");
+    return MI_NULL_PTR;
   }
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
