@@ -160,7 +160,9 @@ int mi_matmul_run_host(mi_matmul *h, const int8_t *a_host, int32_t rows, int8_t 
  * projections of a decoder layer or separate Q, K, V projections: equal to mi_matmul_run(handles[i], a_dev, rows,
  * c_dev[i], stream) for i = 0 .. count-1.  With at most 32 rows and two to four members the weight-streaming kernels
  * run them as ONE launch (one grid, the members' channel ranges side by side), which saves the start-up and drain of
- * the memory stream once per merged member; other cases run member by member.  The reference executes such sibling
+ * the memory stream once per merged member.  With more rows two to four members with a deep of at least 1024, symmetric
+ * weights and the packed copy of them share one launch of the GEMM where that takes fewer rounds of tiles; other cases run
+ * member by member.  The reference executes such sibling
  * kernels one after the other (mindspore/lite/src/executor/sub_graph_kernel.cc:456-466; each is a
  * MatmulBaseInt8CPUKernel::Run, LK/int8/matmul_base_int8.cc:530-570). */
 int mi_matmul_run_group(mi_matmul *const *handles, int32_t count, const int8_t *a_dev, int32_t rows,
@@ -313,8 +315,8 @@ int mi_dynmm_run_host(mi_dynmm *h, const int8_t *a_host, int32_t rows, double in
 int mi_dynmm_run_rows(mi_dynmm *h, const int8_t *a_dev, int32_t rows, const mi_dq_params *row_params_dev,
                       float *c_dev, void *stream);
 /* Dynamic MatMuls that read the same activation rows (q / k / v, gate / up of a dynamic-quant transformer), as
- * mi_matmul_run_group does for the full-quant MatMul: up to four handles with the same deep at up to 32 rows run as
- * one launch, anything else member by member.  The input's scale and zero point come by value (params_dev NULL), from
+ * mi_matmul_run_group does for the full-quant MatMul: up to four handles with the same deep run as
+ * one launch under the same conditions, anything else member by member.  The input's scale and zero point come by value (params_dev NULL), from
  * the block a DynamicQuant run left on the device (params_dev, per_row 0) or as one scale per row (per_row 1);
  * member i writes c_dev[i], fp32 [rows, col_i].  No counterpart in the reference, which runs one node at a time. */
 int mi_dynmm_run_group(mi_dynmm *const *handles, int32_t count, const int8_t *a_dev, int32_t rows, double in_scale,

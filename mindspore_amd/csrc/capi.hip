@@ -879,12 +879,16 @@ int mi_matmul_run_group(mi_matmul *const *handles, int32_t count, const int8_t *
   // the activation rows are brought into the kernels' form once, for all members
   if ((rc = prepare_rows(a_dev, rows, handles[0]->st.k, Workspace::growable(&handles[0]->a_ws), s, &a, &lda, &k16)) != MI_OK)
     return rc;
-  // decode-sized runs of up to four members go out as one launch; anything else runs member by member
-  bool one_launch = count >= 2 && count <= 4 && rows <= kGemvGroupMaxRows;
-  for (int i = 0; i < count && one_launch; ++i)
-    one_launch = rows <= kGemvDotRows ? (int64_t)rows * k16 <= 150 * 1024
-                                      : handles[i]->st.w_blocked.p != nullptr && handles[i]->st.k_pad <= 1 << 20;
-  if (one_launch) {
+  // up to four members go out as one launch if they are decode-sized, or if the GEMM expects to gain by it; anything else runs
+  // member by member
+  const bool few = count >= 2 && count <= 4;
+  bool decode = few && rows <= kGemvGroupMaxRows, tiles = few;
+  for (int i = 0; i < count && few; ++i) {
+    decode = decode && (rows <= kGemvDotRows ? (int64_t)rows * k16 <= 150 * 1024
+                                             : handles[i]->st.w_blocked.p != nullptr && handles[i]->st.k_pad <= 1 << 20);
+    tiles = tiles && !gemv_takes_rows(rows, handles[i]->st.n);
+  }
+  if (decode || tiles) {
     WeightView wv[4];
     RequantParams rq[4];
     int n[4];
@@ -894,7 +898,10 @@ int mi_matmul_run_group(mi_matmul *const *handles, int32_t count, const int8_t *
       rq[i] = st.params();
       n[i] = st.n;
     }
-    return launch_gemv_group(a, lda, rows, k16, count, wv, n, rq, c_dev, s);
+    if (decode) return launch_gemv_group(a, lda, rows, k16, count, wv, n, rq, c_dev, s);
+    bool taken = false;
+    rc = launch_gemm_group_requant(a, lda, rows, k16, count, wv, n, rq, c_dev, s, &taken);
+    if (rc != MI_OK || taken) return rc;
   }
   for (int i = 0; i < count; ++i)
     if ((rc = run_requant_gemm(handles[i]->st, a, lda, rows, k16, c_dev[i], s)) != MI_OK)
@@ -1578,12 +1585,14 @@ int mi_dynmm_run_group(mi_dynmm *const *handles, int32_t count, const int8_t *a_
   // the activation rows are brought into the kernels' form once, for all members
   if ((rc = prepare_rows(a_dev, rows, handles[0]->k, Workspace::growable(&handles[0]->a_ws), s, &a, &lda, &k16)) != MI_OK)
     return rc;
-  // decode-sized runs of up to four members go out as one launch; anything else runs member by member
-  bool one_launch = count >= 2 && count <= 4 && rows <= kGemvGroupMaxRows &&
-                    (rows > kGemvDotRows || (int64_t)rows * k16 <= 150 * 1024);
-  for (int i = 0; i < count && one_launch; ++i)
-    one_launch = rows == 1 || (handles[i]->w_blocked.p != nullptr && handles[i]->k_pad <= 1 << 20);
-  if (one_launch) {
+  // as in mi_matmul_run_group
+  const bool few = count >= 2 && count <= 4;
+  bool decode = few && rows <= kGemvGroupMaxRows && (rows > kGemvDotRows || (int64_t)rows * k16 <= 150 * 1024), tiles = few;
+  for (int i = 0; i < count && few; ++i) {
+    decode = decode && (rows == 1 || (handles[i]->w_blocked.p != nullptr && handles[i]->k_pad <= 1 << 20));
+    tiles = tiles && !gemv_takes_rows(rows, handles[i]->n);
+  }
+  if (decode || tiles) {
     WeightView wv[4];
     DequantParams dq[4];
     int n[4];
@@ -1593,7 +1602,10 @@ int mi_dynmm_run_group(mi_dynmm *const *handles, int32_t count, const int8_t *a_
       dq[i] = dequant_params(h, (float)in_scale, in_zp, params_dev, per_row != 0);
       n[i] = h->n;
     }
-    return launch_gemv_group_dequant(a, lda, rows, k16, count, wv, n, dq, c_dev, s);
+    if (decode) return launch_gemv_group_dequant(a, lda, rows, k16, count, wv, n, dq, c_dev, s);
+    bool taken = false;
+    rc = launch_gemm_group_dequant(a, lda, rows, k16, count, wv, n, dq, c_dev, s, &taken);
+    if (rc != MI_OK || taken) return rc;
   }
   for (int i = 0; i < count; ++i) {
     if ((rc = dynmm_run_impl(handles[i], a_dev, rows, (float)in_scale, in_zp, params_dev, c_dev[i], s, per_row != 0)) != MI_OK)

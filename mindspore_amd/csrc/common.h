@@ -91,6 +91,13 @@ int launch_gemm_requant(const int8_t *a, int64_t lda, int m, int k, const Weight
 int launch_gemm_dequant(const int8_t *a, int64_t lda, int m, int k, const WeightView &w, int n,
                         const DequantParams &dq, float *c, int64_t ldc, hipStream_t stream);
 
+// Up to four weight matrices with the same K against the same activation rows as one launch; member i writes c[i] with row
+// stride n[i].  *taken: it was launched; otherwise the members are to be run one by one.
+int launch_gemm_group_requant(const int8_t *a, int64_t lda, int m, int k, int count, const WeightView *w, const int *n,
+                              const RequantParams *rq, int8_t *const *c, hipStream_t stream, bool *taken);
+int launch_gemm_group_dequant(const int8_t *a, int64_t lda, int m, int k, int count, const WeightView *w, const int *n,
+                              const DequantParams *dq, float *const *c, hipStream_t stream, bool *taken);
+
 // Skinny-M path (m <= kGemvMaxRows): streams the weights once with 16-byte coalesced loads.
 constexpr int kGemvMaxRows = 64;
 constexpr int kGemvGroupMaxRows = 32;  // the group launches (several matrices, one launch) stop here

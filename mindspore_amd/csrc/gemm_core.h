@@ -56,6 +56,55 @@ __device__ __forceinline__ void tile_coords(const GemmArgs &g, int *tile_m, int 
   *tile_n = (id % width) / gsize;
 }
 
+// Several weight matrices with the same K against the same activation rows as one launch: their column tiles stand side by
+// side, and a workgroup first finds the member its tile belongs to.  Fields are picked with selects over constant indices (a
+// dynamically indexed kernel argument would be copied to scratch memory).
+constexpr int kGemmGroupMax = 4;
+template <typename P>  // P: the members' epilogue parameters (RequantParams or DequantParams)
+struct GemmGroup {
+  GemmArgs g;  // what they share; tiles_n counts the column tiles of all of them
+  int count;
+  int first_tile[kGemmGroupMax];  // a member's first column tile
+  int n[kGemmGroupMax];
+  const int8_t *wb[kGemmGroupMax];
+  void *c[kGemmGroupMax];  // rows of n values
+  P p[kGemmGroupMax];
+};
+
+template <typename P>
+__device__ __forceinline__ void pick_member(const GemmGroup<P> &grp, int *tile_n, GemmArgs *g, P *p) {
+  int first = 0;
+  *g = grp.g;
+  *p = grp.p[0];
+  g->wb = grp.wb[0];
+  g->n = grp.n[0];
+  g->c = grp.c[0];
+#pragma unroll
+  for (int i = 1; i < kGemmGroupMax; ++i) {
+    if (i < grp.count && *tile_n >= grp.first_tile[i]) {
+      *p = grp.p[i];
+      g->wb = grp.wb[i];
+      g->n = grp.n[i];
+      g->c = grp.c[i];
+      first = grp.first_tile[i];
+    }
+  }
+  g->ldc = g->n;
+  *tile_n -= first;
+}
+
+// Host side: the grid of a group on tiles of tile_n channels x tile_m rows.
+template <typename P>
+int group_tiles(GemmGroup<P> *grp, int tile_n, int tile_m) {
+  grp->g.tiles_m = (grp->g.m + tile_m - 1) / tile_m;
+  grp->g.tiles_n = 0;
+  for (int i = 0; i < grp->count; ++i) {
+    grp->first_tile[i] = grp->g.tiles_n;
+    grp->g.tiles_n += (grp->n[i] + tile_n - 1) / tile_n;
+  }
+  return grp->g.tiles_m * grp->g.tiles_n;
+}
+
 // clamp to [lo, hi] in one instruction (valid for lo <= hi)
 __device__ __forceinline__ int med3_i32(int x, int lo, int hi) {
   int y;
@@ -527,5 +576,10 @@ int launch_gemm_kblock(int tile, bool requant, bool has_zw, bool fast, GemmArgs 
                        const DequantParams &dq, hipStream_t stream);
 int launch_gemm_ring(int tile, bool requant, bool has_zw, bool fast, GemmArgs g, const RequantParams &rq,
                      const DequantParams &dq, hipStream_t stream);
+// The same for a group whose members have blocked weights without zero points (and, for int8 output, the fast2 form).
+int launch_gemm_kblock_group(int tile, GemmGroup<RequantParams> grp, hipStream_t stream);
+int launch_gemm_kblock_group(int tile, bool fast, GemmGroup<DequantParams> grp, hipStream_t stream);
+int launch_gemm_ring_group(int tile, GemmGroup<RequantParams> grp, hipStream_t stream);
+int launch_gemm_ring_group(int tile, bool fast, GemmGroup<DequantParams> grp, hipStream_t stream);
 
 }  // namespace mi

@@ -42,7 +42,8 @@ namespace mi {
 // arrive sooner that way than as 128-byte pieces of 8 rows (2048 x 4096 x 11008 93 -> 88 us; handles without the blocked
 // copy, and convolutions, read the row-major one).
 template <int TN, int TM, int EPI, bool HAS_ZW, bool FAST, bool WB>
-__device__ __forceinline__ void gemm_kblock_body(const GemmArgs &g, const RequantParams &rq, const DequantParams &dq) {
+__device__ __forceinline__ void gemm_kblock_body(const GemmArgs &g, const RequantParams &rq, const DequantParams &dq, int tile_m,
+                                                 int tile_n) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the buffer-resource type exists in the device pass only; the host pass needs just the stub
   constexpr int TILE_N = 64 * TN, TILE_M = 64 * TM, KB = 128;
   constexpr int SLOT_W = TILE_N * KB, SLOT_A = TILE_M * KB;
@@ -50,8 +51,6 @@ __device__ __forceinline__ void gemm_kblock_body(const GemmArgs &g, const Requan
   static_assert(LDS_BYTES >= kEpiArrays * TILE_N * 4 + epi_wg_bytes<EPI, TN, TM>(), "the epilogue staging must fit");
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
 
-  int tile_m, tile_n;
-  tile_coords(g, &tile_m, &tile_n);
   const int m0 = tile_m * TILE_M, n0 = tile_n * TILE_N;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -311,7 +310,33 @@ template <int TN, int TM, int EPI, bool HAS_ZW, bool FAST, bool WB>
 __global__ __launch_bounds__(256)
     __attribute__((amdgpu_waves_per_eu(kblock_occupancy<TN, TM>(), kblock_occupancy<TN, TM>()))) void gemm_kblock_kernel(
         GemmArgs g, RequantParams rq, DequantParams dq) {
-  gemm_kblock_body<TN, TM, EPI, HAS_ZW, FAST, WB>(g, rq, dq);
+  int tile_m, tile_n;
+  tile_coords(g, &tile_m, &tile_n);
+  gemm_kblock_body<TN, TM, EPI, HAS_ZW, FAST, WB>(g, rq, dq, tile_m, tile_n);
+}
+
+template <int TN, int TM>
+__global__ __launch_bounds__(256)
+    __attribute__((amdgpu_waves_per_eu(kblock_occupancy<TN, TM>(), kblock_occupancy<TN, TM>()))) void gemm_kblock_group_kernel(
+        GemmGroup<RequantParams> grp) {
+  int tile_m, tile_n;
+  tile_coords(grp.g, &tile_m, &tile_n);
+  GemmArgs g;
+  RequantParams rq;
+  pick_member(grp, &tile_n, &g, &rq);
+  gemm_kblock_body<TN, TM, EPI_REQUANT, false, true, true>(g, rq, DequantParams{}, tile_m, tile_n);
+}
+
+template <int TN, int TM, bool FAST>
+__global__ __launch_bounds__(256)
+    __attribute__((amdgpu_waves_per_eu(kblock_occupancy<TN, TM>(), kblock_occupancy<TN, TM>()))) void gemm_kblock_group_deq_kernel(
+        GemmGroup<DequantParams> grp) {
+  int tile_m, tile_n;
+  tile_coords(grp.g, &tile_m, &tile_n);
+  GemmArgs g;
+  DequantParams dq;
+  pick_member(grp, &tile_n, &g, &dq);
+  gemm_kblock_body<TN, TM, EPI_DEQUANT, false, FAST, true>(g, RequantParams{}, dq, tile_m, tile_n);
 }
 
 template <int TN, int TM, int EPI, bool HAS_ZW, bool FAST>
@@ -351,6 +376,42 @@ int launch_gemm_kblock(int tile, bool requant, bool has_zw, bool fast, GemmArgs 
     case 44: return with_form<4, 4>(requant, has_zw, fast, g, rq, dq, stream);
     case 34: return with_form<3, 4>(requant, has_zw, fast, g, rq, dq, stream);
     case 22: return with_form<2, 2>(requant, has_zw, fast, g, rq, dq, stream);
+  }
+  set_error("gemm: no such tile (%d)", tile);
+  return MI_ERROR;
+}
+
+template <int TN, int TM>
+static int launch_group(GemmGroup<RequantParams> grp, hipStream_t stream) {
+  const dim3 grid(group_tiles(&grp, 64 * TN, 64 * TM));
+  hipLaunchKernelGGL((gemm_kblock_group_kernel<TN, TM>), grid, dim3(256), 0, stream, grp);
+  MI_HIP_CHECK(hipGetLastError());
+  return MI_OK;
+}
+
+template <int TN, int TM, bool FAST>
+static int launch_group_deq(GemmGroup<DequantParams> grp, hipStream_t stream) {
+  const dim3 grid(group_tiles(&grp, 64 * TN, 64 * TM));
+  hipLaunchKernelGGL((gemm_kblock_group_deq_kernel<TN, TM, FAST>), grid, dim3(256), 0, stream, grp);
+  MI_HIP_CHECK(hipGetLastError());
+  return MI_OK;
+}
+
+int launch_gemm_kblock_group(int tile, GemmGroup<RequantParams> grp, hipStream_t stream) {
+  switch (tile) {
+    case 44: return launch_group<4, 4>(grp, stream);
+    case 34: return launch_group<3, 4>(grp, stream);
+    case 22: return launch_group<2, 2>(grp, stream);
+  }
+  set_error("gemm: no such tile (%d)", tile);
+  return MI_ERROR;
+}
+
+int launch_gemm_kblock_group(int tile, bool fast, GemmGroup<DequantParams> grp, hipStream_t stream) {
+  switch (tile) {
+    case 44: return fast ? launch_group_deq<4, 4, true>(grp, stream) : launch_group_deq<4, 4, false>(grp, stream);
+    case 34: return fast ? launch_group_deq<3, 4, true>(grp, stream) : launch_group_deq<3, 4, false>(grp, stream);
+    case 22: return fast ? launch_group_deq<2, 2, true>(grp, stream) : launch_group_deq<2, 2, false>(grp, stream);
   }
   set_error("gemm: no such tile (%d)", tile);
   return MI_ERROR;

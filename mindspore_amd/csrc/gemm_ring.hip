@@ -19,7 +19,8 @@ namespace mi {
 // STREAM: weight loads carry the non-temporal hint (see launch_ring).
 // =====================================================================================================================
 template <int TN, int TM, int S, int EPI, bool HAS_ZW, bool FAST, bool STREAM>
-__device__ __forceinline__ void gemm_ring_body(const GemmArgs &g, const RequantParams &rq, const DequantParams &dq) {
+__device__ __forceinline__ void gemm_ring_body(const GemmArgs &g, const RequantParams &rq, const DequantParams &dq, int tile_m,
+                                               int tile_n) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the buffer-resource type exists in the device pass only; the host pass needs just the stub
   constexpr int TILE_N = 64 * TN, TILE_M = 64 * TM, KB = 128;
   constexpr int STAGE = (TILE_N + TILE_M) * KB;
@@ -29,8 +30,6 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs &g, const RequantP
   static_assert(S * STAGE >= kEpiArrays * TILE_N * 4 + epi_wg_bytes<EPI, TN, TM>(), "the epilogue staging must fit");
   __shared__ __attribute__((aligned(1024))) char lds[S * STAGE];
 
-  int tile_m, tile_n;
-  tile_coords(g, &tile_m, &tile_n);
   const int m0 = tile_m * TILE_M, n0 = tile_n * TILE_N;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -233,7 +232,33 @@ template <int TN, int TM, int S, int EPI, bool HAS_ZW, bool FAST, bool STREAM>
 __global__ __launch_bounds__(256)
     __attribute__((amdgpu_waves_per_eu(ring_occupancy<TN, TM, S>(), ring_occupancy<TN, TM, S>()))) void gemm_ring_kernel(
         GemmArgs g, RequantParams rq, DequantParams dq) {
-  gemm_ring_body<TN, TM, S, EPI, HAS_ZW, FAST, STREAM>(g, rq, dq);
+  int tile_m, tile_n;
+  tile_coords(g, &tile_m, &tile_n);
+  gemm_ring_body<TN, TM, S, EPI, HAS_ZW, FAST, STREAM>(g, rq, dq, tile_m, tile_n);
+}
+
+template <int TN, int TM, int S, bool STREAM>
+__global__ __launch_bounds__(256)
+    __attribute__((amdgpu_waves_per_eu(ring_occupancy<TN, TM, S>(), ring_occupancy<TN, TM, S>()))) void gemm_ring_group_kernel(
+        GemmGroup<RequantParams> grp) {
+  int tile_m, tile_n;
+  tile_coords(grp.g, &tile_m, &tile_n);
+  GemmArgs g;
+  RequantParams rq;
+  pick_member(grp, &tile_n, &g, &rq);
+  gemm_ring_body<TN, TM, S, EPI_REQUANT, false, true, STREAM>(g, rq, DequantParams{}, tile_m, tile_n);
+}
+
+template <int TN, int TM, int S, bool FAST, bool STREAM>
+__global__ __launch_bounds__(256)
+    __attribute__((amdgpu_waves_per_eu(ring_occupancy<TN, TM, S>(), ring_occupancy<TN, TM, S>()))) void gemm_ring_group_deq_kernel(
+        GemmGroup<DequantParams> grp) {
+  int tile_m, tile_n;
+  tile_coords(grp.g, &tile_m, &tile_n);
+  GemmArgs g;
+  DequantParams dq;
+  pick_member(grp, &tile_n, &g, &dq);
+  gemm_ring_body<TN, TM, S, EPI_DEQUANT, false, FAST, STREAM>(g, RequantParams{}, dq, tile_m, tile_n);
 }
 
 // Up to two row tiles the weights stream past the L2s, which then keep the activations that every channel tile re-reads.  With
@@ -284,6 +309,56 @@ int launch_gemm_ring(int tile, bool requant, bool has_zw, bool fast, GemmArgs g,
     case 32: return with_form<3, 2, 4>(requant, has_zw, fast, g, rq, dq, stream);
     case 24: return with_form<2, 4, 3>(requant, has_zw, fast, g, rq, dq, stream);
     case 42: return with_form<4, 2, 3>(requant, has_zw, fast, g, rq, dq, stream);
+  }
+  set_error("gemm: no such tile (%d)", tile);
+  return MI_ERROR;
+}
+
+template <int TN, int TM, int S>
+static int launch_group(GemmGroup<RequantParams> grp, hipStream_t stream) {
+  const dim3 grid(group_tiles(&grp, 64 * TN, 64 * TM));
+  if (grp.g.tiles_m <= kStreamRowTiles) {
+    hipLaunchKernelGGL((gemm_ring_group_kernel<TN, TM, S, true>), grid, dim3(256), 0, stream, grp);
+  } else {
+    hipLaunchKernelGGL((gemm_ring_group_kernel<TN, TM, S, false>), grid, dim3(256), 0, stream, grp);
+  }
+  MI_HIP_CHECK(hipGetLastError());
+  return MI_OK;
+}
+
+template <int TN, int TM, int S, bool FAST>
+static int launch_group_deq(GemmGroup<DequantParams> grp, hipStream_t stream) {
+  const dim3 grid(group_tiles(&grp, 64 * TN, 64 * TM));
+  if (grp.g.tiles_m <= kStreamRowTiles) {
+    hipLaunchKernelGGL((gemm_ring_group_deq_kernel<TN, TM, S, FAST, true>), grid, dim3(256), 0, stream, grp);
+  } else {
+    hipLaunchKernelGGL((gemm_ring_group_deq_kernel<TN, TM, S, FAST, false>), grid, dim3(256), 0, stream, grp);
+  }
+  MI_HIP_CHECK(hipGetLastError());
+  return MI_OK;
+}
+
+int launch_gemm_ring_group(int tile, GemmGroup<RequantParams> grp, hipStream_t stream) {
+  switch (tile) {
+    case 11: return launch_group<1, 1, 5>(grp, stream);
+    case 12: return launch_group<1, 2, 6>(grp, stream);
+    case 22: return launch_group<2, 2, 5>(grp, stream);
+    case 32: return launch_group<3, 2, 4>(grp, stream);
+    case 24: return launch_group<2, 4, 3>(grp, stream);
+    case 42: return launch_group<4, 2, 3>(grp, stream);
+  }
+  set_error("gemm: no such tile (%d)", tile);
+  return MI_ERROR;
+}
+
+int launch_gemm_ring_group(int tile, bool fast, GemmGroup<DequantParams> grp, hipStream_t stream) {
+  switch (tile) {
+    case 11: return fast ? launch_group_deq<1, 1, 5, true>(grp, stream) : launch_group_deq<1, 1, 5, false>(grp, stream);
+    case 12: return fast ? launch_group_deq<1, 2, 6, true>(grp, stream) : launch_group_deq<1, 2, 6, false>(grp, stream);
+    case 22: return fast ? launch_group_deq<2, 2, 5, true>(grp, stream) : launch_group_deq<2, 2, 5, false>(grp, stream);
+    case 32: return fast ? launch_group_deq<3, 2, 4, true>(grp, stream) : launch_group_deq<3, 2, 4, false>(grp, stream);
+    case 24: return fast ? launch_group_deq<2, 4, 3, true>(grp, stream) : launch_group_deq<2, 4, 3, false>(grp, stream);
+    case 42: return fast ? launch_group_deq<4, 2, 3, true>(grp, stream) : launch_group_deq<4, 2, 3, false>(grp, stream);
   }
   set_error("gemm: no such tile (%d)", tile);
   return MI_ERROR;

@@ -162,6 +162,36 @@ def test_matmul_tile_shapes(orc, m, n, k, dynamic, asymmetric):
         assert np.array_equal(got, want)
 
 
+# groups on 64 x 64 (a member of one channel, rows to be padded), 64 x 128, 128 x 128, 192 x 128, 128 x 256, 256 x 128,
+# 256 x 256 and 192 x 256 tiles, a pair that gains nothing by one launch, pairs of 128 x 128 tiles
+@pytest.mark.parametrize("m,k,ns", [(65, 1024, (65, 1, 200)), (130, 1030, (500, 131)), (70, 1024, (9000, 4100)),
+                                    (300, 1024, (5000, 5000)), (257, 1030, (12000, 3001)), (500, 1024, (8192, 8000)),
+                                    (300, 1024, (6000, 6000, 6000)), (700, 1024, (11008, 11008)), (513, 1040, (8200, 8201)),
+                                    (1030, 2048, (9000, 9000)), (1878, 4320, (3929, 349))])
+@pytest.mark.parametrize("how", ["static", "value", "rows"])
+def test_matmul_group_on_tiles(orc, m, k, ns, how):
+    """A group's launch against a launch per member (whose tiles have tests of their own), and the smallest against the oracle."""
+    import torch
+    rng = np.random.default_rng(m + k + sum(ns))
+    members = [_matmul_pair(rng, n, k, False, how != "static") for n in ns]
+    kernels = [make(True) for *_, make in members]
+    a = rng.integers(-128, 128, (m, k), dtype=np.int8)
+    dev, args = torch.from_numpy(a).cuda(), {}
+    if how == "value":
+        args = dict(in_quant=K.QuantParam(0.03, -5))
+    if how == "rows":
+        dev, params = K.DynamicQuantKernel(True).run_rows(torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32)).cuda())
+        args = dict(row_params=params)
+    outs = K.matmul_run_group(kernels, dev) if how == "static" else K.dynmm_run_group(kernels, dev, **args)
+    for kern, y in zip(kernels, outs):
+        assert torch.equal(y, kern.run(dev, **args))
+    if m * k * sum(ns) < 2e8 and how != "rows":
+        for (w, bias, sw, zw, _), y in zip(members, outs):
+            want = (orc.dynamic_matmul(a, w, bias, 0.03, -5, sw, zw) if how == "value" else
+                    orc.matmul_int8(a, w, bias, 0.02, 7, sw, zw, float(np.float32(0.02 * 0.0055 * k ** 0.5 * 140)), 3))
+            assert np.array_equal(y.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("taps", [3, 5])
 @pytest.mark.parametrize("b,ih,iw,ch,pad", [(1, 5, 5, 4, (0, 0, 0, 0)), (1, 5, 6, 8, (1, 1, 1, 1)), (2, 7, 9, 12, (2, 0, 0, 2)),
                                             (1, 9, 11, 20, (4, 4, 4, 4)), (3, 6, 8, 192, (1, 2, 3, 0)), (1, 33, 31, 36, (1, 1, 1, 1)),
