@@ -284,10 +284,13 @@ int launch_conv_smallk(const int8_t *in, const ConvGeom &g, int fill, int k_true
 // requantisation parameters are loaded once and live in registers, and a 4 x 4 byte transposition across neighbouring
 // lanes makes dwords of four channels for the stores.  A wave keeps the weights of its up to 64 channels in registers
 // and walks tiles of 32 pixels, fetching the next tile's operand before it requantises the current one.
-// Bound at large sizes by the vector ALU (about 6 instructions per output byte, half of them the requantisation) and the
-// unaligned fetches, at small ones by the latency of one tile.  us per launch, before -> now: 32 x 224 x 224 x 3 -> 64,
-// 7x7, stride 2 134 (im2col and GEMM) -> 23; one such image 8.7 -> 4.8; 1 x 224 x 224 x 3 -> 32, 3x3, stride 2
-// 4.6 (sixteen byte loads per K step) -> 2.8.
+// Bound at large sizes by the vector ALU (about 230 instructions per tile of 32 pixels x 64 channels, 190 of them the
+// requantisation) and by the loads, whose 64 unaligned addresses take the address unit about 95 cycles; at small ones by the
+// latency of one tile.  32 x 224 x 224 x 3 -> 64, 7x7, stride 2: 22.6 us, without loads 18, without stores 18, without either
+// 14.4; the order of tiles over the XCDs and the number of waves change nothing, and the rows through LDS, once each, gain 2 us
+// there and lose 1 everywhere else.  With masks and branches in every tile, and divisions by the vector ALU, it took 461
+// instructions.  us per launch, before that / with it: that 25.4 / 22.6; one such image 5.2 / 4.65; 16 x 224 x 224 x 3 -> 32,
+// 3x3, stride 2 6.4 / 5.65; 16 x 160 x 160 x 3 -> 64, 3x3 14.4 / 12.4; 16 x 224 x 224 x 4 -> 32, 5x5 20.1 / 16.4.
 struct ConvRows {
   const int8_t *in;
   int in_bytes;
@@ -298,85 +301,77 @@ struct ConvRows {
   int fill;
   int pixels;
   const int8_t *w;  // [out_c padded to 64][32 * KS]
+  uint32_t magic_hw, magic_w;  // quotients by out_hw and out_w: umulhi(2 p, magic) >> shift (see magic31)
+  int shift_hw, shift_w;
 };
 
+// Quotients of p < 2^31 by d >= 1 as umulhi(2 p, magic) >> shift, with 2^(shift - 1) < d <= 2^shift and
+// magic = ceil(2^(31 + shift) / d): the product is p / d + p * e / (d * 2^(31 + shift)), e = magic * d - 2^(31 + shift) < 2^shift,
+// and the second term stays below 1 / d.
+static void magic31(int d, uint32_t *magic, int *shift) {
+  int s = 0;
+  while (((int64_t)1 << s) < d) ++s;
+  *shift = s;
+  *magic = (uint32_t)((((uint64_t)1 << (31 + s)) + (uint32_t)d - 1) / (uint32_t)d);
+}
+
+__device__ __forceinline__ int quotient31(int p, uint32_t magic, int shift) { return (int)(__umulhi(2 * (uint32_t)p, magic) >> shift); }
+
 __device__ __forceinline__ uint32_t quad_transpose(uint32_t d, uint32_t sel1, uint32_t sel2) {
-  const uint32_t p = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)d, 0xB1, 0xF, 0xF, false);  // lane ^ 1
+  const uint32_t p = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)d, 0xB1, 0xF, 0xF, true);  // lane ^ 1
   const uint32_t r = __builtin_amdgcn_perm(p, d, sel1);
-  const uint32_t q = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)r, 0x4E, 0xF, 0xF, false);  // lane ^ 2
+  const uint32_t q = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)r, 0x4E, 0xF, 0xF, true);  // lane ^ 2
   return __builtin_amdgcn_perm(q, r, sel2);
 }
 
-// FAST: the one-multiply rounding form without weight zero points (RequantParams::fast2, !has_zw).
-template <int KS, int OCB, bool FAST>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void conv_rows_kernel(
-    ConvRows g, RequantParams rq, int8_t *__restrict__ out) {
-  typedef uint32_t u32_any __attribute__((aligned(1)));
-  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
-  const int n0 = blockIdx.y * (32 * OCB);
-  const int tiles = (g.pixels + 31) >> 5, step = gridDim.x * 4;
-  int tile = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (tile >= tiles) return;
+// A tile's operand straight from the image: lane r (of each half) takes pixel 32 * tile + r.
+template <int KS>
+struct RowsGather {
+  const ConvRows &g;
+  int r, h, part, line, last16;  // part: which chunk of a window row this lane holds
+  int img, ih0, t0;  // the image, the window's first row, the chunk's first byte in an image row
+  // A plain tile, the usual one, has all its windows inside the image and all its loads inside the tensor: the loads then
+  // differ by a scalar, and no byte needs replacing (those past a window row meet zero weights).
+  bool plain;
 
-  v4i wf[OCB][KS];
-#pragma unroll
-  for (int ob = 0; ob < OCB; ++ob)
-#pragma unroll
-    for (int s = 0; s < KS; ++s)
-      wf[ob][s] = *reinterpret_cast<const v4i *>(g.w + (n0 + ob * 32 + r) * (32 * KS) + 32 * s + 16 * h);
-  // this lane's channel of each block (the arrays are padded to a multiple of 256 channels)
-  int32_t mult[OCB], bias[OCB], shift[OCB], lsh[OCB], zw[OCB];
-  uint64_t c2[OCB];
-#pragma unroll
-  for (int ob = 0; ob < OCB; ++ob) {
-    const int n = n0 + ob * 32 + r;
-    shift[ob] = rq.rshift[n];
-    if (FAST) {
-      mult[ob] = (int32_t)rq.mult2[n];
-      c2[ob] = (uint64_t)rq.c2hi[n] << 32 | rq.c2lo[n];
-      bias[ob] = rq.pre[n];
-    } else {
-      mult[ob] = rq.mult[n];
-      bias[ob] = (int32_t)((uint32_t)rq.bias2[n] - kAccBias);
-      lsh[ob] = rq.lshift[n];
-      zw[ob] = rq.zw[n];
-    }
-  }
-  int amin_v = rq.amin, amax_v = rq.amax;
-  asm volatile("" : "+v"(amin_v), "+v"(amax_v));  // kept in vector registers, as v_med3 wants them
-  const uint32_t sel1 = (lane & 1) ? 0x03070105u : 0x06020400u, sel2 = (lane & 2) ? 0x03020706u : 0x05040100u;
-  const uint32_t fill4 = (uint32_t)(g.fill & 0xff) * 0x01010101u;
-  const int part = g.parts == 2 ? h : 0;  // which chunk of a window row this lane holds
-  const int line = g.in_w * g.in_c, last16 = g.in_bytes - 16;
-  auto window_row = [&](int s) { return g.parts == 2 ? s : 2 * s + h; };
-
-  // where a tile's operand is: the image, the window's first row, the chunk's first byte in an image row
-  int img, ih0, t0;
-  auto locate = [&](int tl) {
-    const int want = tl * 32 + r, p = want < g.pixels ? want : g.pixels - 1;
-    const int b = (uint32_t)p / (uint32_t)g.out_hw, rem = p - b * g.out_hw;
-    const int oh = (uint32_t)rem / (uint32_t)g.out_w, ow = rem - oh * g.out_w;
+  __device__ __forceinline__ RowsGather(const ConvRows &g_, int lane)
+      : g(g_), r(lane & 31), h(lane >> 5), part(g_.parts == 2 ? h : 0), line(g_.in_w * g_.in_c), last16(g_.in_bytes - 16) {}
+  __device__ __forceinline__ int window_row(int s) const { return g.parts == 2 ? s : 2 * s + h; }
+  __device__ __forceinline__ void locate(int tile) {
+    const int want = tile * 32 + r, p = want < g.pixels ? want : g.pixels - 1;
+    const int b = quotient31(p, g.magic_hw, g.shift_hw), rem = p - b * g.out_hw;
+    const int oh = quotient31(rem, g.magic_w, g.shift_w), ow = rem - oh * g.out_w;
     img = b * (g.in_h * line);
     ih0 = oh * g.stride_h - g.pad_u;
     t0 = (ow * g.stride_w - g.pad_l) * g.in_c + 16 * part;
-  };
+    const int from = t0 - 16 * part, to_last = (g.parts == 2 ? KS - 1 : 2 * KS - 1) * g.dil_h;
+    plain = __all(ih0 >= 0 && ih0 + to_last < g.in_h && from >= 0 && from + g.row_bytes <= line &&
+                  (uint32_t)img + (uint32_t)(ih0 + to_last) * (uint32_t)line + (uint32_t)t0 <= (uint32_t)last16);
+  }
   // Every load is a whole 16 bytes inside the tensor: rows above or below the image are clamped (their bytes are
   // replaced), and an address before its first or behind its last 16 bytes is moved in.
-  auto address = [&](int s) {
+  __device__ __forceinline__ int address(int s) const {
     int kh = window_row(s);
     kh = kh < g.kernel_h ? kh : g.kernel_h - 1;
     const int ih = min(max(ih0 + kh * g.dil_h, 0), g.in_h - 1);
     return img + ih * line + t0;
-  };
-  auto fetch = [&](v4i (&x)[KS]) {
+  }
+  __device__ __forceinline__ void fetch(v4i (&x)[KS]) const {
+    if (plain) {
+      const int row_step = g.dil_h * line;
+      const uint32_t lane_off = (uint32_t)(img + ih0 * line + t0 + (g.parts == 2 ? 0 : h * row_step));
+      const int8_t *row = g.in;
+#pragma unroll
+      for (int s = 0; s < KS; ++s, row += g.parts == 2 ? row_step : 2 * row_step)
+        x[s] = *reinterpret_cast<const v4i_any *>(row + lane_off);
+      return;
+    }
 #pragma unroll
     for (int s = 0; s < KS; ++s) x[s] = *reinterpret_cast<const v4i_any *>(g.in + min(max(address(s), 0), last16));
-  };
-
-  locate(tile);
-  v4i x[KS];
-  fetch(x);
-  for (; tile < tiles; tile += step) {
+  }
+  // what was fetched, as the window sees it
+  __device__ __forceinline__ void mend(v4i (&x)[KS]) const {
+    if (plain) return;
     if (__any(address(0) < 0 || address(KS - 1) > last16)) {  // a load that was moved in: move its bytes back
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
@@ -388,13 +383,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
         }
       }
     }
-    // bytes [-t0, line - t0) of this lane's chunk lie inside the image row, the others are fill
+    const uint32_t fill4 = (uint32_t)(g.fill & 0xff) * 0x01010101u;
     uint32_t in_row[4];
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      const int a = min(max(-t0 - 4 * d, 0), 4), b = min(max(line - t0 - 4 * d, 0), 4);
-      in_row[d] = (uint32_t)((((uint64_t)1 << (8 * b)) - 1) & ~(((uint64_t)1 << (8 * a)) - 1));
-    }
+    row_mask(t0, line, in_row);
     const bool rows_inside = ih0 >= 0 && ih0 + (g.kernel_h - 1) * g.dil_h < g.in_h;
     if (__all(rows_inside)) {
 #pragma unroll
@@ -412,90 +403,182 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
         }
       }
     }
+  }
+  // of 16 bytes that start at byte t of an image row, those inside the row, [-t, line - t); the others are fill
+  static __device__ __forceinline__ void row_mask(int t, int line, uint32_t (&m)[4]) {
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      const int a = min(max(-t - 4 * d, 0), 4), b = min(max(line - t - 4 * d, 0), 4);
+      m[d] = (uint32_t)((((uint64_t)1 << (8 * b)) - 1) & ~(((uint64_t)1 << (8 * a)) - 1));
+    }
+  }
+};
+
+// A tile's accumulators -> bytes in memory.  acc[ob][4 * q + e] is pixel 8 * q + 4 * h + e of the tile, channel
+// n0 + 32 * ob + r; after the transposition a lane holds channels r & ~3 .. + 3 of pixel 8 * q + 4 * h + (lane & 3).
+// FAST: the one-multiply rounding form without weight zero points (RequantParams::fast2, !has_zw).
+template <int OCB, bool FAST>
+struct RowsStore {
+  int32_t mult[OCB], bias[OCB], shift[OCB], lsh[OCB], zw[OCB];  // of this lane's channel of each block
+  uint64_t c2[OCB];
+  int amin_v, amax_v, my_n, my_p;
+  uint32_t sel1, sel2, out_off;
+
+  __device__ __forceinline__ RowsStore(const ConvRows &g, const RequantParams &rq, int n0, int lane) {
+    const int r = lane & 31, h = lane >> 5;
+#pragma unroll
+    for (int ob = 0; ob < OCB; ++ob) {
+      const int n = n0 + ob * 32 + r;  // (the arrays are padded to a multiple of 256 channels)
+      shift[ob] = rq.rshift[n];
+      if (FAST) {
+        mult[ob] = (int32_t)rq.mult2[n];
+        c2[ob] = (uint64_t)rq.c2hi[n] << 32 | rq.c2lo[n];
+        bias[ob] = rq.pre[n];
+      } else {
+        mult[ob] = rq.mult[n];
+        bias[ob] = (int32_t)((uint32_t)rq.bias2[n] - kAccBias);
+        lsh[ob] = rq.lshift[n];
+        zw[ob] = rq.zw[n];
+      }
+    }
+    amin_v = rq.amin, amax_v = rq.amax;
+    asm volatile("" : "+v"(amin_v), "+v"(amax_v));  // kept in vector registers, as v_med3 wants them
+    sel1 = (lane & 1) ? 0x03070105u : 0x06020400u, sel2 = (lane & 2) ? 0x03020706u : 0x05040100u;
+    my_n = n0 + (r & ~3), my_p = 4 * h + (lane & 3);
+    out_off = (uint32_t)(my_p * g.out_c + my_n);
+  }
+  __device__ __forceinline__ uint32_t four_channels(const RequantParams &rq, const v16i (&acc)[OCB], const v16i &sums, int q,
+                                                    int ob) const {
+    int y[4];
+    if (FAST) {
+      // one 64-bit multiply-add per output; its carry is the rounding's "+1 unless negative"
+      uint64_t p2[4], carry[4], unused;
+      int32_t t[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        asm("v_mad_u64_u32 %0, %1, %2, %3, %4"
+            : "=&v"(p2[e]), "=s"(carry[e])
+            : "v"(acc[ob][4 * q + e]), "v"(mult[ob]), "v"(c2[ob]));
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        asm("v_addc_co_u32_e64 %0, %1, %2, %3, %4"
+            : "=v"(t[e]), "=s"(unused)
+            : "v"((int32_t)(p2[e] >> 32)), "v"(bias[ob]), "s"(carry[e]));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        t[e] >>= shift[ob];
+        asm("v_med3_i32 %0, %1, %2, %3" : "=v"(y[e]) : "v"(t[e]), "v"(amin_v), "v"(amax_v));
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        uint32_t v = (uint32_t)acc[ob][4 * q + e] - (uint32_t)sums[4 * q + e] * (uint32_t)zw[ob] + (uint32_t)bias[ob];
+        int32_t t = rdiv_pot(srdhm((int32_t)(v << lsh[ob]), mult[ob]), shift[ob]);
+        t = (int32_t)((uint32_t)t + (uint32_t)rq.zo);
+        t = t < rq.amax ? t : rq.amax;
+        y[e] = t > rq.amin ? t : rq.amin;
+      }
+    }
+    const uint32_t p01 = __builtin_amdgcn_perm((uint32_t)y[1], (uint32_t)y[0], 0x0c0c0400u);
+    const uint32_t p23 = __builtin_amdgcn_perm((uint32_t)y[3], (uint32_t)y[2], 0x0c0c0400u);
+    return quad_transpose(__builtin_amdgcn_perm(p23, p01, 0x05040100u), sel1, sel2);
+  }
+  __device__ __forceinline__ void store(const ConvRows &g, const RequantParams &rq, v16i (&acc)[OCB], const v16i &sums, int tile,
+                                        int n0, int8_t *out) const {
+    typedef uint32_t u32_any __attribute__((aligned(1)));
+    // The compiler keeps the distance that a matrix product's result needs before the next instruction reads it, but not
+    // where that instruction is inline assembly, as above: 19 wait states after a 16-pass product.
+    if constexpr (OCB == 1) asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc[0]));
+    if constexpr (OCB == 2) asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc[0]), "+v"(acc[1]));
+    int8_t *tile_out = out + (int64_t)tile * 32 * g.out_c;
+    // (no branch between the pieces of a whole tile: one's chain of dependent instructions fills the gaps of the next)
+    if (tile * 32 + 32 <= g.pixels && n0 + 32 * OCB <= g.out_c) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int ob = 0; ob < OCB; ++ob)
+          *reinterpret_cast<u32_any *>(tile_out + (8 * q * g.out_c + 32 * ob) + out_off) = four_channels(rq, acc, sums, q, ob);
+      return;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+#pragma unroll
+      for (int ob = 0; ob < OCB; ++ob) {
+        const uint32_t four = four_channels(rq, acc, sums, q, ob);
+        int8_t *to = tile_out + (8 * q * g.out_c + 32 * ob) + out_off;
+        if (tile * 32 + 8 * q + my_p >= g.pixels) continue;
+        if (my_n + 32 * ob + 4 <= g.out_c) {
+          *reinterpret_cast<u32_any *>(to) = four;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 3; ++e)
+            if (my_n + 32 * ob + e < g.out_c) to[e] = (int8_t)(four >> (8 * e));
+        }
+      }
+    }
+  }
+};
+
+// this lane's weights, as the matrix operand of channel block ob and step s
+template <int KS, int OCB>
+__device__ __forceinline__ void rows_weights(const ConvRows &g, int n0, int lane, v4i (&wf)[OCB][KS]) {
+#pragma unroll
+  for (int ob = 0; ob < OCB; ++ob)
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+      wf[ob][s] = *reinterpret_cast<const v4i *>(g.w + (n0 + ob * 32 + (lane & 31)) * (32 * KS) + 32 * s + 16 * (lane >> 5));
+}
+
+// waves per SIMD: three where the weights leave registers for it
+constexpr int rows_occupancy(int ks, int ocb, bool fast) { return fast && ks * ocb <= 8 ? 3 : 2; }
+
+template <int KS, int OCB, bool FAST>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(rows_occupancy(KS, OCB, FAST)))) void conv_rows_kernel(
+    ConvRows g, RequantParams rq, int8_t *__restrict__ out) {
+  const int lane = threadIdx.x & 63;
+  const int n0 = blockIdx.y * (32 * OCB);
+  const int tiles = (g.pixels + 31) >> 5, step = gridDim.x * 4;
+  int tile = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (tile >= tiles) return;
+
+  v4i wf[OCB][KS];
+  rows_weights(g, n0, lane, wf);
+  const RowsStore<OCB, FAST> store(g, rq, n0, lane);
+  RowsGather<KS> in(g, lane);
+  v16i start;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) start[e] = (int)kAccBias;
+  if (FAST) asm volatile("" : "+v"(start));  // one block of registers for every tile's first products
+  in.locate(tile);
+  v4i x[KS];
+  in.fetch(x);
+  for (; tile < tiles; tile += step) {
+    in.mend(x);
     v16i acc[OCB], sums;
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-#pragma unroll
-      for (int ob = 0; ob < OCB; ++ob) acc[ob][e] = (int)kAccBias;
-      sums[e] = 0;
-    }
+    for (int e = 0; e < 16; ++e) sums[e] = 0;
 #pragma unroll
     for (int s = 0; s < KS; ++s)
 #pragma unroll
-      for (int ob = 0; ob < OCB; ++ob) acc[ob] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x[s], wf[ob][s], acc[ob], 0, 0, 0);
+      for (int ob = 0; ob < OCB; ++ob)
+        acc[ob] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x[s], wf[ob][s], s == 0 ? start : acc[ob], 0, 0, 0);
     if (!FAST && rq.has_zw) {  // the pixels' input sums, in the accumulators' layout: against ones where a window byte is
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
         v4i one;
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
-          const int b = window_row(s) < g.kernel_h ? min(max(g.row_bytes - 16 * part - 4 * d, 0), 4) : 0;
+          const int b = in.window_row(s) < g.kernel_h ? min(max(g.row_bytes - 16 * in.part - 4 * d, 0), 4) : 0;
           one[d] = (int)(0x01010101u & (uint32_t)(((uint64_t)1 << (8 * b)) - 1));
         }
         sums = __builtin_amdgcn_mfma_i32_32x32x32_i8(x[s], one, sums, 0, 0, 0);
       }
     }
-    const int first = tile * 32;
     if (tile + step < tiles) {  // (wave-uniform)
-      locate(tile + step);
-      fetch(x);
+      in.locate(tile + step);
+      in.fetch(x);
     }
-    // The compiler keeps the distance that a matrix product's result needs before the next instruction reads it, but not
-    // where that instruction is inline assembly, as below: 19 wait states after a 16-pass product.
-    if constexpr (OCB == 1) asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc[0]));
-    if constexpr (OCB == 2) asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc[0]), "+v"(acc[1]));
-    // acc[ob][4 * q + e] is pixel 8 * q + 4 * h + e of the tile, channel n0 + 32 * ob + r; after the transposition this
-    // lane holds channels r & ~3 .. + 3 of pixel 8 * q + 4 * h + (lane & 3)
-    const bool whole = first + 32 <= g.pixels && (g.out_c & 3) == 0;
-    const int my_n = n0 + (r & ~3), my_p = first + 4 * h + (lane & 3);
-    int8_t *dst = out + (int64_t)my_p * g.out_c + my_n;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-#pragma unroll
-      for (int ob = 0; ob < OCB; ++ob) {
-        int y[4];
-        if (FAST) {
-          // one 64-bit multiply-add per output; its carry is the rounding's "+1 unless negative"
-          uint64_t p2[4], carry[4], unused;
-          int32_t t[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            asm("v_mad_u64_u32 %0, %1, %2, %3, %4"
-                : "=&v"(p2[e]), "=s"(carry[e])
-                : "v"(acc[ob][4 * q + e]), "v"(mult[ob]), "v"(c2[ob]));
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            asm("v_addc_co_u32_e64 %0, %1, %2, %3, %4"
-                : "=v"(t[e]), "=s"(unused)
-                : "v"((int32_t)(p2[e] >> 32)), "v"(bias[ob]), "s"(carry[e]));
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            t[e] >>= shift[ob];
-            asm("v_med3_i32 %0, %1, %2, %3" : "=v"(y[e]) : "v"(t[e]), "v"(amin_v), "v"(amax_v));
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            uint32_t v = (uint32_t)acc[ob][4 * q + e] - (uint32_t)sums[4 * q + e] * (uint32_t)zw[ob] + (uint32_t)bias[ob];
-            int32_t t = rdiv_pot(srdhm((int32_t)(v << lsh[ob]), mult[ob]), shift[ob]);
-            t = (int32_t)((uint32_t)t + (uint32_t)rq.zo);
-            t = t < rq.amax ? t : rq.amax;
-            y[e] = t > rq.amin ? t : rq.amin;
-          }
-        }
-        const uint32_t p01 = __builtin_amdgcn_perm((uint32_t)y[1], (uint32_t)y[0], 0x0c0c0400u);
-        const uint32_t p23 = __builtin_amdgcn_perm((uint32_t)y[3], (uint32_t)y[2], 0x0c0c0400u);
-        const uint32_t four = quad_transpose(__builtin_amdgcn_perm(p23, p01, 0x05040100u), sel1, sel2);
-        int8_t *to = dst + 8 * q * g.out_c + 32 * ob;
-        if (whole) {
-          if (my_n + 32 * ob < g.out_c) *reinterpret_cast<u32_any *>(to) = four;
-        } else if (my_p + 8 * q < g.pixels) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (my_n + 32 * ob + e < g.out_c) to[e] = (int8_t)(four >> (8 * e));
-        }
-      }
-    }
+    store.store(g, rq, acc, sums, tile, n0, out);
   }
 }
 
@@ -539,11 +622,13 @@ int launch_conv_rows(const int8_t *in, const ConvGeom &g, int fill, const int8_t
   const int64_t wgs = (pixels + 127) / 128;
   const bool two = g.out_c > 32, fast = rq.fast2 != 0 && rq.has_zw == 0;
   const int gy = (g.out_c + (two ? 63 : 31)) / (two ? 64 : 32);
-  // three workgroups per CU: a wave then walks several tiles on one set of weight registers, and three waves per SIMD
-  // hide the fetches.  us at 32 x 224 x 224 x 3 -> 64, 7x7: 256 workgroups 25.7, 512 23.0, 768 23.9, 2048 27.1;
-  // 16 x 192 x 192 x 3 -> 32, 3x3: 6.8, 4.9, 4.7, 5.1
-  constexpr int64_t most = 768;
+  // as many workgroups as the registers let the device hold, so that a wave walks several tiles on one set of weights.  us at
+  // 32 x 224 x 224 x 3 -> 64, 7x7 (two per SIMD): 512 workgroups 22.6, 768 25.4; 16 x 224 x 224 x 3 -> 32, 3x3 (three):
+  // 512 5.95, 768 5.65
+  const int most = 256 * rows_occupancy(ks, two ? 2 : 1, fast);
   const dim3 grid((unsigned)(wgs < most ? wgs : most), (unsigned)gy);
+  magic31(c.out_hw, &c.magic_hw, &c.shift_hw);
+  magic31(c.out_w, &c.magic_w, &c.shift_w);
 #define MI_ROWS(KS)                                                                                          \
   case KS:                                                                                                   \
     if (fast) {                                                                                              \

@@ -119,6 +119,25 @@ def test_first_layer_convolution_windows(orc, kernel, ic, oc, asymmetric):
         assert np.array_equal(conv.run(flat[3:].view(x.shape)).cpu().numpy(), want), (kernel, ic, oc, ih, iw)
 
 
+@pytest.mark.parametrize("kernel,ic,oc", [((7, 7), 3, 64), ((7, 7), 3, 33), ((3, 3), 3, 32), ((5, 5), 3, 40), ((4, 3), 10, 64)])
+@pytest.mark.parametrize("h,w,stride,pad,batch", [(7, 102, (1, 1), 0, 2), (9, 139, (1, 2), 0, 1), (13, 150, (2, 2), 2, 3),
+                                                  (11, 64 + 6, (3, 1), 1, 5), (70, 71, (1, 1), 3, 1)])
+def test_first_layer_convolution_long_rows(orc, kernel, ic, oc, h, w, stride, pad, batch):
+    """Output rows longer than a tile of 32 pixels: tiles wholly inside the image, up to the last bytes of the tensor."""
+    import torch
+    from oracle import pyoracle
+    rng = np.random.default_rng(h * w + kernel[1])
+    x = rng.integers(-128, 128, (batch, h, w, ic), dtype=np.int8)
+    wt = rng.integers(-128, 128, (oc, *kernel, ic), dtype=np.int8)
+    sw = rng.uniform(0.001, 0.01, oc).astype(np.float32).astype(np.float64)
+    bias, zp = rng.integers(-2000, 2001, oc).astype(np.int32), np.zeros(oc, np.int32)
+    shape = pyoracle.conv_shape(batch, h, w, ic, oc, kernel, stride, (1, 1), (pad,) * 4)
+    conv = K.ConvolutionInt8Kernel(wt, bias, K.QuantParam(0.02, 4), [K.QuantParam(float(s), 0) for s in sw], K.QuantParam(0.2, -6),
+                                   stride, (1, 1), (pad,) * 4, 1, K.ACT_NONE, exact_3x3=True)
+    want = orc.conv_int8(x, wt, bias, shape, 0.02, 4, sw, zp, 0.2, -6, K.ACT_NONE)
+    assert np.array_equal(conv.run(torch.from_numpy(x).cuda()).cpu().numpy(), want)
+
+
 def _matmul_pair(rng, n, k, asymmetric, dynamic, **kw):
     w = rng.integers(-128, 128, (n, k), dtype=np.int8)
     sw = rng.uniform(0.001, 0.01, n).astype(np.float32).astype(np.float64)
