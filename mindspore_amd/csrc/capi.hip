@@ -493,6 +493,7 @@ struct mi_matmul {
   RequantState st;  // weight matrix 0
   std::vector<std::unique_ptr<RequantState>> more;  // weight matrices 1 .. b_batch - 1 of a batched constant weight
   DevBuf a_ws, h_in, h_out;
+  HostCopyUser host_user;
   int b_batch() const { return 1 + (int)more.size(); }
   RequantState &state(int b) { return b == 0 ? st : *more[(size_t)b - 1]; }
 };
@@ -503,6 +504,7 @@ struct mi_conv {
   int fill = 0;
   RequantState st;
   DevBuf w16, dw_bias, dw_bias_folded, col_ws, h_in, h_out;
+  HostCopyUser host_user;
   DevBuf dw_rows, dw_rows_par;  // the operands of launch_conv_dw_rows, or empty
   DevBuf w_rows;  // the weights of a convolution on few channels as launch_conv_rows takes them, or empty
   DevBuf w_thin;  // the weights of a 1x1 on few channels as launch_conv_thin takes them, or empty
@@ -512,6 +514,7 @@ struct mi_conv {
 struct mi_dynquant {
   int symmetric = 0;
   DevBuf partials, slots, params, h_in, h_out, h_params;
+  HostCopyUser host_user;
   // Where a run leaves its parameters for the host that asks for them: page-locked, taken with the handle, or absent (every
   // fetch is then a copy).  Polled by the host (mi_dynquant_await_params) they are there a few microseconds after the launch; a
   // copy and a stream synchronisation behind it took 22 us more (197 x 768: 34 us per run and fetch -> 10.5, and 16 for
@@ -537,6 +540,7 @@ struct mi_dynmm {
   int32_t zw0 = 0;
   bool has_bias = false;
   DevBuf w, wscale, wsum, bias, a_ws, h_in, h_out, h_params;
+  HostCopyUser host_user;
   DevBuf w_blocked;  // the weights in 1 KiB matrix-core blocks for two activation rows and more; built in create or absent
 };
 
@@ -959,11 +963,11 @@ int mi_matmul_run_host(mi_matmul *h, const int8_t *a_host, int32_t rows, int8_t 
   if (rc != MI_OK) return rc;
   const size_t in_bytes = (size_t)rows * h->st.k, out_bytes = (size_t)rows * h->st.n;
   if ((rc = h->h_in.ensure(in_bytes)) != MI_OK || (rc = h->h_out.ensure(out_bytes)) != MI_OK) return rc;
-  MI_HIP_CHECK(hipMemcpy(h->h_in.p, a_host, in_bytes, hipMemcpyHostToDevice));
+  HostCopies copies(&h->host_user, std::max(in_bytes, out_bytes));
+  if ((rc = copies.in(h->h_in.p, a_host, in_bytes)) != MI_OK) return rc;
   rc = mi_matmul_run(h, static_cast<const int8_t *>(h->h_in.p), rows, static_cast<int8_t *>(h->h_out.p), nullptr);
   if (rc != MI_OK) return rc;
-  MI_HIP_CHECK(hipMemcpy(c_host, h->h_out.p, out_bytes, hipMemcpyDeviceToHost));
-  return MI_OK;
+  return copies.out(c_host, h->h_out.p, out_bytes);
 }
 
 int mi_matmul_get_params(const mi_matmul *h, int32_t *multiplier, int32_t *left_shift, int32_t *right_shift,
@@ -1236,12 +1240,12 @@ int mi_conv_run_host(mi_conv *h, const int8_t *in_host, int32_t batch, int32_t i
   const size_t in_bytes = (size_t)batch * in_h * in_w * h->d.in_channel;
   const size_t out_bytes = (size_t)batch * oh * ow * h->d.out_channel;
   if ((rc = h->h_in.ensure(in_bytes)) != MI_OK || (rc = h->h_out.ensure(out_bytes)) != MI_OK) return rc;
-  MI_HIP_CHECK(hipMemcpy(h->h_in.p, in_host, in_bytes, hipMemcpyHostToDevice));
+  HostCopies copies(&h->host_user, std::max(in_bytes, out_bytes));
+  if ((rc = copies.in(h->h_in.p, in_host, in_bytes)) != MI_OK) return rc;
   rc = mi_conv_run(h, static_cast<const int8_t *>(h->h_in.p), batch, in_h, in_w, static_cast<int8_t *>(h->h_out.p),
                    nullptr);
   if (rc != MI_OK) return rc;
-  MI_HIP_CHECK(hipMemcpy(out_host, h->h_out.p, out_bytes, hipMemcpyDeviceToHost));
-  return MI_OK;
+  return copies.out(out_host, h->h_out.p, out_bytes);
 }
 
 void mi_conv_destroy(mi_conv *h) { delete h; }  // every DevBuf member frees its device memory
@@ -1367,11 +1371,12 @@ int mi_dynquant_run_segments_host(mi_dynquant *h, const float *x_host, int64_t s
   if ((rc = h->h_in.ensure(n * 4 + 16)) != MI_OK || (rc = h->h_out.ensure(n + 16)) != MI_OK ||
       (rc = h->h_params.ensure(sizeof(mi_dq_params) * (size_t)segments)) != MI_OK)
     return rc;
-  MI_HIP_CHECK(hipMemcpy(h->h_in.p, x_host, n * 4, hipMemcpyHostToDevice));
+  HostCopies copies(&h->host_user, n * 4);
+  if ((rc = copies.in(h->h_in.p, x_host, n * 4)) != MI_OK) return rc;
   rc = mi_dynquant_run_segments(h, static_cast<const float *>(h->h_in.p), segments, unit,
                                 static_cast<int8_t *>(h->h_out.p), static_cast<mi_dq_params *>(h->h_params.p), nullptr);
   if (rc != MI_OK) return rc;
-  MI_HIP_CHECK(hipMemcpy(q_host, h->h_out.p, n, hipMemcpyDeviceToHost));
+  if ((rc = copies.out(q_host, h->h_out.p, n)) != MI_OK) return rc;
   MI_HIP_CHECK(hipMemcpy(params_host, h->h_params.p, sizeof(mi_dq_params) * (size_t)segments, hipMemcpyDeviceToHost));
   return MI_OK;
 }
@@ -1389,11 +1394,12 @@ int mi_dynquant_run_host(mi_dynquant *h, const float *x_host, int64_t n, int8_t 
   int rc = ensure_device();
   if (rc != MI_OK) return rc;
   if ((rc = h->h_in.ensure((size_t)n * 4 + 16)) != MI_OK || (rc = h->h_out.ensure((size_t)n + 16)) != MI_OK) return rc;
-  if (n > 0) MI_HIP_CHECK(hipMemcpy(h->h_in.p, x_host, (size_t)n * 4, hipMemcpyHostToDevice));
+  HostCopies copies(&h->host_user, (size_t)n * 4);
+  if (n > 0 && (rc = copies.in(h->h_in.p, x_host, (size_t)n * 4)) != MI_OK) return rc;
   rc = mi_dynquant_run(h, static_cast<const float *>(h->h_in.p), n, static_cast<int8_t *>(h->h_out.p), nullptr);
   if (rc != MI_OK) return rc;
   if ((rc = mi_dynquant_await_params(h, nullptr, params_host)) != MI_OK) return rc;
-  if (n > 0) MI_HIP_CHECK(hipMemcpy(q_host, h->h_out.p, (size_t)n, hipMemcpyDeviceToHost));
+  if (n > 0 && (rc = copies.out(q_host, h->h_out.p, (size_t)n)) != MI_OK) return rc;
   return MI_OK;
 }
 
@@ -1636,12 +1642,12 @@ static int mi_dynmm_run_rows_host_impl(mi_dynmm *h, const int8_t *a_host, int32_
     p[r].real_min = p[r].real_max = 0.0f;
   }
   MI_HIP_CHECK(hipMemcpy(h->h_params.p, p.data(), sizeof(mi_dq_params) * (size_t)rows, hipMemcpyHostToDevice));
-  MI_HIP_CHECK(hipMemcpy(h->h_in.p, a_host, in_bytes, hipMemcpyHostToDevice));
+  HostCopies copies(&h->host_user, std::max(in_bytes, out_bytes));
+  if ((rc = copies.in(h->h_in.p, a_host, in_bytes)) != MI_OK) return rc;
   rc = mi_dynmm_run_rows(h, static_cast<const int8_t *>(h->h_in.p), rows,
                          static_cast<const mi_dq_params *>(h->h_params.p), static_cast<float *>(h->h_out.p), nullptr);
   if (rc != MI_OK) return rc;
-  MI_HIP_CHECK(hipMemcpy(c_host, h->h_out.p, out_bytes, hipMemcpyDeviceToHost));
-  return MI_OK;
+  return copies.out(c_host, h->h_out.p, out_bytes);
 }
 
 int mi_dynmm_run_rows_host(mi_dynmm *h, const int8_t *a_host, int32_t rows, const double *in_scales, int32_t in_zp,
@@ -1660,12 +1666,12 @@ int mi_dynmm_run_host(mi_dynmm *h, const int8_t *a_host, int32_t rows, double in
   if (rc != MI_OK) return rc;
   const size_t in_bytes = (size_t)rows * h->k, out_bytes = (size_t)rows * h->n * sizeof(float);
   if ((rc = h->h_in.ensure(in_bytes)) != MI_OK || (rc = h->h_out.ensure(out_bytes)) != MI_OK) return rc;
-  MI_HIP_CHECK(hipMemcpy(h->h_in.p, a_host, in_bytes, hipMemcpyHostToDevice));
+  HostCopies copies(&h->host_user, std::max(in_bytes, out_bytes));
+  if ((rc = copies.in(h->h_in.p, a_host, in_bytes)) != MI_OK) return rc;
   rc = mi_dynmm_run(h, static_cast<const int8_t *>(h->h_in.p), rows, in_scale, in_zp, static_cast<float *>(h->h_out.p),
                     nullptr);
   if (rc != MI_OK) return rc;
-  MI_HIP_CHECK(hipMemcpy(c_host, h->h_out.p, out_bytes, hipMemcpyDeviceToHost));
-  return MI_OK;
+  return copies.out(c_host, h->h_out.p, out_bytes);
 }
 
 void mi_dynmm_destroy(mi_dynmm *h) { delete h; }  // every DevBuf member frees its device memory

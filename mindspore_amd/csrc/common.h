@@ -174,6 +174,35 @@ std::vector<int32_t> conv_dw_rows_weights(const int8_t *w, int ch, int ks);
 int launch_conv_dw_rows(const int8_t *in, const ConvGeom &g, const int32_t *w, const int32_t *par, int zx8, int amin, int amax,
                         int8_t *out, hipStream_t stream);
 
+// Host tensors of one call, in and out of device memory on the null stream (host_copy.hip).  `dev` holds a multiple of 16 bytes.
+// The page-locked slots that the copies go through stay for the next call while a handle that has used some lives.
+struct HostSlots;
+class HostCopyUser {  // a member of every handle with such calls
+ public:
+  HostCopyUser() = default;
+  HostCopyUser(const HostCopyUser &) = delete;
+  HostCopyUser &operator=(const HostCopyUser &) = delete;
+  ~HostCopyUser();
+
+ private:
+  friend class HostCopies;
+  bool used_ = false;
+};
+class HostCopies {
+ public:
+  HostCopies(HostCopyUser *user, size_t most_bytes);  // most_bytes: of the largest tensor
+  HostCopies(const HostCopies &) = delete;
+  HostCopies &operator=(const HostCopies &) = delete;
+  ~HostCopies();
+  int in(void *dev, const void *host, size_t bytes);   // may return before the bytes are there; `host` is the caller's again
+  int out(void *host, const void *dev, size_t bytes);  // returns when they are
+ private:
+  bool through_slots(const void *host, size_t bytes);
+  HostCopyUser *user_;
+  int size_;
+  HostSlots *slots_ = nullptr;
+};
+
 // The requantising GEMM with its activation operand gathered from an NHWC image (in_c % 16 == 0): the im2col
 // convolution without the buffer.  fill16: 16 bytes of the value out-of-image taps take, in device memory.
 bool gemm_conv_supported(const ConvGeom &g, const void *in);

@@ -496,3 +496,51 @@ def test_group_of_many_kernels(dynamic):
     assert len(outs) == 100
     for kern, y in zip(kernels, outs):
         assert torch.equal(y, kern.run(a, **args))
+
+
+# one chunk, a last chunk of one byte, as many chunks as slots, slots used several times, on the way in, out and both
+@pytest.mark.parametrize("rows,k,n", [(1, 1, 1), (3, 70001, 2), (65537, 1, 1), (517, 1000, 64), (2099, 1001, 5), (2100, 7, 1001),
+                                      (3001, 1500, 1401)])
+def test_host_tensors_in_and_out(rows, k, n):
+    """Against the same kernels on device tensors."""
+    import torch
+    rng = np.random.default_rng(rows + k)
+    a = rng.integers(-128, 128, (rows, k), dtype=np.int8)
+    dev = torch.from_numpy(a).cuda()
+    for dynamic in (False, True):
+        kern = _matmul_pair(rng, n, k, False, dynamic)[4](True)
+        args = dict(in_quant=K.QuantParam(0.03, -5)) if dynamic else {}
+        want = kern.run(dev, **args).cpu().numpy()
+        for _ in range(2):
+            assert np.array_equal(kern.run(a, **args), want)
+        locked = torch.from_numpy(a).pin_memory().numpy()  # goes past the slots
+        assert np.array_equal(kern.run(locked, **args), want)
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    for per_row in (False, True):
+        dq = K.DynamicQuantKernel(per_row)
+        there = dq.run_rows(torch.from_numpy(x).cuda())[0] if per_row else dq.run(torch.from_numpy(x).cuda())[0]
+        assert np.array_equal(dq.run_rows(x)[0] if per_row else dq.run(x)[0], there.cpu().numpy())
+
+
+def test_host_tensors_from_several_threads():
+    import threading
+    import torch
+    rng = np.random.default_rng(77)
+    work = []
+    for rows, k, n in ((700, 900, 1100), (64, 64, 64), (1500, 2000, 300), (2000, 300, 2000), (1, 5, 9)):
+        a = rng.integers(-128, 128, (rows, k), dtype=np.int8)
+        kern = _matmul_pair(rng, n, k, False, False)[4](True)
+        work.append((kern, a, kern.run(torch.from_numpy(a).cuda()).cpu().numpy()))
+    bad = []
+
+    def go(kern, a, want):
+        for _ in range(6):
+            if not np.array_equal(kern.run(a), want):
+                bad.append(a.shape)
+
+    threads = [threading.Thread(target=go, args=w) for w in work]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
