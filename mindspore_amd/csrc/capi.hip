@@ -449,12 +449,14 @@ static std::vector<int8_t> unpack_4x16(const int8_t *packed, int n, int k) {
   return out;
 }
 
+static bool whole_chunks(const int8_t *a, int k) { return (k & 15) == 0 && (reinterpret_cast<uintptr_t>(a) & 15) == 0; }
+
 // Activations must reach the GEMM/GEMV kernels as 16-byte aligned rows of k16 bytes; returns the pointer/stride to
 // use, copying through `ws` when the caller's layout does not qualify.
 static int prepare_rows(const int8_t *a, int rows, int k, const Workspace &ws, hipStream_t stream,
                         const int8_t **a_out, int64_t *lda_out, int *k16_out) {
   const int k16 = round_up(k, 16);
-  if (k16 == k && (reinterpret_cast<uintptr_t>(a) & 15) == 0) {
+  if (whole_chunks(a, k)) {
     *a_out = a;
     *lda_out = k;
     *k16_out = k;
@@ -471,17 +473,36 @@ static int prepare_rows(const int8_t *a, int rows, int k, const Workspace &ws, h
   return MI_OK;
 }
 
+// (the blocked copy may be absent: two rows then take the v_dot4 kernel)
+static WeightView weight_view(const RequantState &st) {
+  return WeightView{static_cast<const int8_t *>(st.w.p), st.k_pad, st.ldw, static_cast<const int8_t *>(st.w_blocked.p)};
+}
+
+// one row: the dot kernel on the row-major weights; few rows: the matrix-core decode kernel on the blocked copy made at
+// create time (a handle without it runs two rows on the dot kernel and the others on the GEMM tiles)
+static bool runs_on_gemv(const RequantState &st, int rows, int k16) {
+  return rows <= kGemvDotRows ? (int64_t)rows * k16 <= 150 * 1024
+                              : gemv_takes_rows(rows, st.n) && st.w_blocked.p != nullptr && st.k_pad <= 1 << 20;
+}
+
 static int run_requant_gemm(RequantState &st, const int8_t *a, int64_t lda, int rows, int k16, int8_t *c,
                             hipStream_t stream) {
   const RequantParams rq = st.params();
-  // (the blocked copy may be absent: two rows then take the v_dot4 kernel)
-  const WeightView w{static_cast<const int8_t *>(st.w.p), st.k_pad, st.ldw, static_cast<const int8_t *>(st.w_blocked.p)};
-  // one row: the dot kernel on the row-major weights; few rows: the matrix-core decode kernel on the blocked copy made at
-  // create time (a handle without it runs two rows on the dot kernel and the others on the GEMM tiles)
-  const bool skinny = rows <= kGemvDotRows ? (int64_t)rows * k16 <= 150 * 1024
-                                           : gemv_takes_rows(rows, st.n) && st.w_blocked.p != nullptr && st.k_pad <= 1 << 20;
-  if (skinny) return launch_gemv_requant(a, lda, rows, k16, w, st.n, rq, c, st.n, stream);
+  const WeightView w = weight_view(st);
+  if (runs_on_gemv(st, rows, k16)) return launch_gemv_requant(a, lda, rows, k16, w, st.n, rq, c, st.n, stream);
   return launch_gemm_requant(a, lda, rows, k16, w, st.n, rq, c, st.n, stream);
+}
+
+// The same for the caller's rows, whatever their length and address.
+static int run_requant_rows(RequantState &st, const int8_t *a_dev, int rows, const Workspace &ws, int8_t *c, hipStream_t stream) {
+  const WeightView w = weight_view(st);
+  if (!whole_chunks(a_dev, st.k) && !runs_on_gemv(st, rows, round_up(st.k, 16)) && gemm_anyrow_takes(rows, st.k, w, st.n))
+    return launch_gemm_anyrow_requant(a_dev, rows, st.k, w, st.n, st.params(), c, stream);
+  const int8_t *a = nullptr;
+  int64_t lda = 0;
+  int k16 = 0;
+  const int rc = prepare_rows(a_dev, rows, st.k, ws, stream, &a, &lda, &k16);
+  return rc != MI_OK ? rc : run_requant_gemm(st, a, lda, rows, k16, c, stream);
 }
 
 }  // namespace mi
@@ -808,12 +829,7 @@ int mi_matmul_run(mi_matmul *h, const int8_t *a_dev, int32_t rows, int8_t *c_dev
   if (rows == 0) return MI_OK;
   int rc = ensure_device();
   if (rc != MI_OK) return rc;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const int8_t *a = nullptr;
-  int64_t lda = 0;
-  int k16 = 0;
-  if ((rc = prepare_rows(a_dev, rows, h->st.k, Workspace::growable(&h->a_ws), s, &a, &lda, &k16)) != MI_OK) return rc;
-  return run_requant_gemm(h->st, a, lda, rows, k16, c_dev, s);
+  return run_requant_rows(h->st, a_dev, rows, Workspace::growable(&h->a_ws), c_dev, static_cast<hipStream_t>(stream));
 }
 
 int mi_matmul_run_batched(mi_matmul *h, const int8_t *a_dev, int32_t rows, int32_t batch, const int32_t *a_offsets,
@@ -841,13 +857,8 @@ int mi_matmul_run_batched(mi_matmul *h, const int8_t *a_dev, int32_t rows, int32
   // one launch per output matrix, in order on the stream (so the shared workspaces are reused safely), as the
   // reference runs one ParallelLaunch per batch (LK/int8/matmul_base_int8.cc:549-568)
   for (int i = 0; i < batch; ++i) {
-    const int8_t *a = nullptr;
-    int64_t lda = 0;
-    int k16 = 0;
-    if ((rc = prepare_rows(a_dev + (size_t)a_offsets[i] * a_mat, rows, h->st.k, Workspace::growable(&h->a_ws), s, &a, &lda,
-                           &k16)) != MI_OK)
-      return rc;
-    if ((rc = run_requant_gemm(h->state(b_offsets[i]), a, lda, rows, k16, c_dev + (size_t)i * c_mat, s)) != MI_OK)
+    if ((rc = run_requant_rows(h->state(b_offsets[i]), a_dev + (size_t)a_offsets[i] * a_mat, rows, Workspace::growable(&h->a_ws),
+                               c_dev + (size_t)i * c_mat, s)) != MI_OK)
       return rc;
   }
   return MI_OK;
@@ -943,13 +954,7 @@ int mi_matmul_run_noalloc(mi_matmul *h, const int8_t *a_dev, int32_t rows, int8_
               "maximum is %zu; use mi_matmul_run", rows, h->st.k, h->st.n, need, kScratchBytes);
     return MI_PARAM_INVALID;
   }
-  const Workspace a_ws = Workspace::region(base, a_bytes);
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const int8_t *a = nullptr;
-  int64_t lda = 0;
-  int k16 = 0;
-  if ((rc = prepare_rows(a_dev, rows, h->st.k, a_ws, s, &a, &lda, &k16)) != MI_OK) return rc;
-  return run_requant_gemm(h->st, a, lda, rows, k16, c_dev, s);
+  return run_requant_rows(h->st, a_dev, rows, Workspace::region(base, a_bytes), c_dev, static_cast<hipStream_t>(stream));
 }
 
 int mi_matmul_run_host(mi_matmul *h, const int8_t *a_host, int32_t rows, int8_t *c_host) {
@@ -1514,18 +1519,20 @@ static int dynmm_run_impl(mi_dynmm *h, const int8_t *a_dev, int32_t rows, float 
   if (rows == 0) return MI_OK;
   int rc = ensure_device();
   if (rc != MI_OK) return rc;
-  const int8_t *a = nullptr;
-  int64_t lda = 0;
-  int k16 = 0;
-  if ((rc = prepare_rows(a_dev, rows, h->k, Workspace::growable(&h->a_ws), s, &a, &lda, &k16)) != MI_OK) return rc;
   const DequantParams dq = dequant_params(h, sx, zx, qp_dev, per_row);
   const WeightView w{static_cast<const int8_t *>(h->w.p), h->k_pad, h->ldw,
                      static_cast<const int8_t *>(h->w_blocked.p)};
   // decode-sized runs: the matrix-core decode kernel streams the blocked weights once (any N, any output alignment)
   // (one row runs on the row-major weights and needs no blocked copy, as long as the row fits the kernel's LDS form)
-  if (gemv_takes_rows(rows, h->n) && (rows > kGemvDotRows || (int64_t)rows * k16 <= 150 * 1024) &&
-      (rows == 1 || (w.blocked != nullptr && h->k_pad <= 1 << 20)))
-    return launch_gemv_dequant(a, lda, rows, k16, w, h->n, dq, c_dev, h->n, s);
+  const bool on_gemv = gemv_takes_rows(rows, h->n) && (rows > kGemvDotRows || (int64_t)rows * round_up(h->k, 16) <= 150 * 1024) &&
+                       (rows == 1 || (w.blocked != nullptr && h->k_pad <= 1 << 20));
+  if (!on_gemv && !whole_chunks(a_dev, h->k) && gemm_anyrow_takes(rows, h->k, w, h->n))
+    return launch_gemm_anyrow_dequant(a_dev, rows, h->k, w, h->n, dq, c_dev, s);
+  const int8_t *a = nullptr;
+  int64_t lda = 0;
+  int k16 = 0;
+  if ((rc = prepare_rows(a_dev, rows, h->k, Workspace::growable(&h->a_ws), s, &a, &lda, &k16)) != MI_OK) return rc;
+  if (on_gemv) return launch_gemv_dequant(a, lda, rows, k16, w, h->n, dq, c_dev, h->n, s);
   return launch_gemm_dequant(a, lda, rows, k16, w, h->n, dq, c_dev, h->n, s);
 }
 

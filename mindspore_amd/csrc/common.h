@@ -91,6 +91,13 @@ int launch_gemm_requant(const int8_t *a, int64_t lda, int m, int k, const Weight
 int launch_gemm_dequant(const int8_t *a, int64_t lda, int m, int k, const WeightView &w, int n,
                         const DequantParams &dq, float *c, int64_t ldc, hipStream_t stream);
 
+// The same for activation rows of any length at any address, [m][k] without gaps, where that is quicker than a padded copy.
+bool gemm_anyrow_takes(int m, int k, const WeightView &w, int n);
+int launch_gemm_anyrow_requant(const int8_t *a, int m, int k, const WeightView &w, int n, const RequantParams &rq, int8_t *c,
+                               hipStream_t stream);
+int launch_gemm_anyrow_dequant(const int8_t *a, int m, int k, const WeightView &w, int n, const DequantParams &dq, float *c,
+                               hipStream_t stream);
+
 // Up to four weight matrices with the same K against the same activation rows as one launch; member i writes c[i] with row
 // stride n[i].  *taken: it was launched; otherwise the members are to be run one by one.
 int launch_gemm_group_requant(const int8_t *a, int64_t lda, int m, int k, int count, const WeightView *w, const int *n,

@@ -576,6 +576,9 @@ int launch_gemm_kblock(int tile, bool requant, bool has_zw, bool fast, GemmArgs 
                        const DequantParams &dq, hipStream_t stream);
 int launch_gemm_ring(int tile, bool requant, bool has_zw, bool fast, GemmArgs g, const RequantParams &rq,
                      const DequantParams &dq, hipStream_t stream);
+// 64 x 64 tiles over activation rows of any length, stride and address (gemm_anyrow.hip); g.k: bytes of K.
+int launch_gemm_anyrow(bool requant, bool has_zw, bool fast, const GemmArgs &g, const RequantParams &rq, const DequantParams &dq,
+                       hipStream_t stream);
 // The same for a group whose members have blocked weights without zero points (and, for int8 output, the fast2 form).
 int launch_gemm_kblock_group(int tile, GemmGroup<RequantParams> grp, hipStream_t stream);
 int launch_gemm_kblock_group(int tile, bool fast, GemmGroup<DequantParams> grp, hipStream_t stream);

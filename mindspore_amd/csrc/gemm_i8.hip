@@ -11,13 +11,15 @@
 // one output row: the epilogue packs them into one 32-bit store, per-channel parameters are 16-byte loads, and
 // the input-row sum a lane needs is the one it accumulated itself (v_dot4 against 0x01010101).
 //
-// Three main loops, all moving tiles global -> LDS with asynchronous 16-byte-per-lane loads and reading operand
+// Four main loops, most of them moving tiles global -> LDS with asynchronous 16-byte-per-lane loads and reading operand
 // fragments for the next K sub-step from LDS while the MFMAs of the current one run.  Handles hold their weights in
 // 1 KiB matrix-core blocks beside the row-major form, and with those nearly every shape runs on K blocks of 128 bytes, on
 // the tile that launch_pick_tile expects to be the quickest:
 //   * gemm_kblock.hip: five LDS slots, one barrier per block; 256 x 256 and 192 x 256 tiles, one workgroup per CU, for the
 //     large shapes, 128 x 128 tiles, two per CU, where fp32 stores have to overlap another tile's loop;
 //   * gemm_ring.hip: a ring of stages that hold both operands, as deep as the LDS allows: every smaller tile;
+//   * gemm_anyrow.hip: 64 x 64 tiles for activation rows that are no whole 16-byte chunks, where padding them first would cost
+//     more than the product;
 //   * gemm_direct_body below, K steps of 64 bytes through NST LDS stages over row-major weights: short K, handles
 //     without the blocked copy (whose large shapes run on gemm_kblock.hip's row-major form) and the convolution whose
 //     activation operand is gathered from the image.
@@ -547,6 +549,46 @@ int launch_gemm_dequant(const int8_t *a, int64_t lda, int m, int k, const Weight
   }
   return nt ? launch_pick_tile<EPI_DEQUANT, false, true>(g, rq, dq, stream)
             : launch_pick_tile<EPI_DEQUANT, false, false>(g, rq, dq, stream);
+}
+
+// Rows that are no whole 16-byte chunks, or not aligned to them: the padded copy is a launch of its own, so where 64 x 64 tiles
+// are the quickest they take the rows as they are, up to the K at which their unaligned loads, once per column tile, have
+// cost as much.  us, copy and tiles / this: 333 x 1001 x 1000 7.4 / 5.6, 100 x 500 x 500 7.2 / 4.4, 128 x 768 x 770 7.5 / 5.7,
+// 1000 x 1000 x 1001 8.0 / 6.8, 200 x 1000 x 1500 7.9 / 6.7, 200 x 1000 x 1793 8.5 / 9.2, x 2040 8.4 / 7.8, x 4003 12.5 / 16.5,
+// 500 x 2000 x 3001 12.3 / 14.2.
+constexpr int kAnyrowMostK = 1536;
+bool gemm_anyrow_takes(int m, int k, const WeightView &w, int n) {
+  if (w.blocked == nullptr || k < 128 || k > kAnyrowMostK || (int64_t)m * k < 16) return false;
+  float cost;
+  const TileCost &t = cheapest_tile(m, k, 1, &n, &cost);
+  return t.ring && t.tn == 1 && t.tm == 1;
+}
+
+static int anyrow_args(const int8_t *a, int m, int k, const WeightView &w, int n, void *c, GemmArgs *g) {
+  if (a == nullptr || c == nullptr) {
+    set_error("gemm: null pointer");
+    return MI_NULL_PTR;
+  }
+  if (m <= 0 || n <= 0 || !gemm_anyrow_takes(m, k, w, n) || w.k_pad % kKPad != 0 || w.k_pad < k) {
+    set_error("gemm: unsupported operand geometry m=%d n=%d k=%d k_pad=%d", m, n, k, w.k_pad);
+    return MI_PARAM_INVALID;
+  }
+  *g = GemmArgs{a, k, m, k, nullptr, 0, w.k_pad, w.blocked, n, 0, 0, c, n};
+  return MI_OK;
+}
+
+int launch_gemm_anyrow_requant(const int8_t *a, int m, int k, const WeightView &w, int n, const RequantParams &rq, int8_t *c,
+                               hipStream_t stream) {
+  GemmArgs g;
+  const int rc = anyrow_args(a, m, k, w, n, c, &g);
+  return rc != MI_OK ? rc : launch_gemm_anyrow(true, rq.has_zw != 0, rq.fast2 != 0, g, rq, DequantParams{}, stream);
+}
+
+int launch_gemm_anyrow_dequant(const int8_t *a, int m, int k, const WeightView &w, int n, const DequantParams &dq, float *c,
+                               hipStream_t stream) {
+  GemmArgs g;
+  const int rc = anyrow_args(a, m, k, w, n, c, &g);
+  return rc != MI_OK ? rc : launch_gemm_anyrow(false, dq.zw0 != 0, false, g, RequantParams{}, dq, stream);
 }
 
 // Several matrices against the same rows as one launch, where that is expected to take less than a launch each (*taken): a

@@ -544,3 +544,28 @@ def test_host_tensors_from_several_threads():
     for t in threads:
         t.join()
     assert not bad
+
+
+# rows of one block, of one set of four blocks, just into the next set, of three sets, the first that are padded; a chunk, a dword and a byte past a block;
+# one tile and several, with rows and channels past their last one
+@pytest.mark.parametrize("m,n,k", [(65, 20, 129), (64, 64, 511), (130, 257, 513), (333, 1001, 1000), (70, 260, 1535), (200, 31, 1291),
+                                   (129, 65, 1537)])
+@pytest.mark.parametrize("dynamic,asymmetric", [(False, False), (False, True), (True, False), (True, True)])
+def test_matmul_rows_of_any_length(orc, m, n, k, dynamic, asymmetric):
+    """Against the oracle, and at addresses that are no multiple of 16 against the aligned run; one of them with k % 16 == 0."""
+    import torch
+    rng = np.random.default_rng(m + n + k)
+    orc.set_threads(16)
+    for depth in (k, (k + 15) // 16 * 16):
+        w, bias, sw, zw, make = _matmul_pair(rng, n, depth, asymmetric, dynamic)
+        a = rng.integers(-128, 128, (m, depth), dtype=np.int8)
+        kern, args = make(True), dict(in_quant=K.QuantParam(0.03, -5)) if dynamic else {}
+        if dynamic:
+            want = orc.dynamic_matmul(a, w, bias, 0.03, -5, sw, zw)
+        else:
+            want = orc.matmul_int8(a, w, bias, 0.02, 7, sw, zw, float(np.float32(0.02 * 0.0055 * depth ** 0.5 * 140)), 3)
+        for shift in (0, 1, 4, 15):
+            flat = torch.zeros(a.size + shift, dtype=torch.int8, device="cuda")  # ends with the tensor's last byte
+            flat[shift:] = torch.from_numpy(a.reshape(-1)).cuda()
+            got = kern.run(flat[shift:].view(a.shape), **args).cpu().numpy()
+            assert np.array_equal(got, want), (depth, shift)
