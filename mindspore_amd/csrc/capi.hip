@@ -529,6 +529,7 @@ struct mi_conv {
   DevBuf dw_rows, dw_rows_par;  // the operands of launch_conv_dw_rows, or empty
   DevBuf w_rows;  // the weights of a convolution on few channels as launch_conv_rows takes them, or empty
   DevBuf w_thin;  // the weights of a 1x1 on few channels as launch_conv_thin takes them, or empty
+  DevBuf w_window;  // the weights of a window on aligned channels as launch_conv_window takes them, or empty
   DevBuf fill16;  // 16 bytes of `fill`: where the gathering GEMM loader reads taps outside the image
 };
 
@@ -599,6 +600,7 @@ int mi_init(int device) {
   }
   MI_HIP_CHECK(hipSetDevice(device));
   int rc = gemv_prepare_device();
+  if (rc == MI_OK) rc = conv_window_prepare_device();
   if (rc != MI_OK) return rc;
   if (device < kMaxDevices && g_scratch_ptr[device] == nullptr) {
     void *ptr = nullptr;
@@ -1128,6 +1130,8 @@ static int mi_conv_create_impl(const mi_conv_desc *d, const int8_t *weight_host,
       rc = upload(&h->w_rows, conv_rows_weights(weight_host, oc, d->kernel_h, d->kernel_w, d->in_channel));
     } else if (rc == MI_OK && h->direct_1x1 && conv_thin_supported(kdim, oc)) {
       rc = upload(&h->w_thin, conv_thin_weights(weight_host, oc, kdim));
+    } else if (rc == MI_OK && conv_window_weights_wanted(shape) && h->st.fast2 && !h->st.has_zw) {
+      rc = upload(&h->w_window, conv_window_weights(weight_host, oc, kdim));
     }
     if (rc == MI_OK) rc = upload(&h->fill16, std::vector<int8_t>(16, (int8_t)h->fill));
   }
@@ -1205,6 +1209,12 @@ int mi_conv_run(mi_conv *h, const int8_t *in_dev, int32_t batch, int32_t in_h, i
   const int8_t *a = nullptr;
   int64_t lda = 0;
   int k16 = 0;
+  if (h->w_window.p != nullptr) {
+    bool taken = false;
+    rc = launch_conv_window(in_dev, g, static_cast<const int8_t *>(h->fill16.p), static_cast<const int8_t *>(h->w_window.p),
+                            h->st.params(), out_dev, s, &taken);
+    if (taken || rc != MI_OK) return rc;
+  }
   if (h->w_thin.p != nullptr && pixels > 128 && pixels <= kConvThinMostPixels) {
     return launch_conv_thin(in_dev, pixels, k, d.out_channel, static_cast<const int8_t *>(h->w_thin.p), h->st.params(), out_dev, s);
   } else if (h->direct_1x1) {

@@ -168,6 +168,14 @@ bool conv_thin_supported(int k, int oc);
 std::vector<int8_t> conv_thin_weights(const int8_t *w, int oc, int k);
 int launch_conv_thin(const int8_t *in, int64_t pixels, int k, int oc, const int8_t *w, const RequantParams &rq, int8_t *out,
                      hipStream_t stream);
+// Convolution of several taps on 16-channel-aligned images (in 16-byte aligned), its window's pixels in LDS, in the fast2 form
+// without weight zero points; w: the weights as conv_window_weights lays them out, in device memory.  *taken false, and nothing
+// launched, where the gathering GEMM is faster or the window does not fit.
+bool conv_window_weights_wanted(const ConvGeom &g);
+std::vector<int8_t> conv_window_weights(const int8_t *w, int oc, int k);
+int conv_window_prepare_device();  // called by mi_init with the device current
+int launch_conv_window(const int8_t *in, const ConvGeom &g, const int8_t *fill16, const int8_t *w, const RequantParams &rq,
+                       int8_t *out, hipStream_t stream, bool *taken);
 // Depthwise conv + requantisation, weights pre-offset to int16 [KH*KW][C].  bias_folded = bias - zx8 * sum_t w16[t][c]
 // (used by the channel-vectorised kernel, which reads out-of-image taps as zx8); rq.fast: the host proved the cheap
 // rounding form exact for every channel.

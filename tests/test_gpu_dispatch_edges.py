@@ -569,3 +569,22 @@ def test_matmul_rows_of_any_length(orc, m, n, k, dynamic, asymmetric):
             flat[shift:] = torch.from_numpy(a.reshape(-1)).cuda()
             got = kern.run(flat[shift:].view(a.shape), **args).cpu().numpy()
             assert np.array_equal(got, want), (depth, shift)
+
+
+# one chunk per pixel and five, odd and even numbers of contraction steps and fewer than the late loads' ones; rectangles that the
+# image cuts off, channels that end inside a block; windows over every border, a stride and a dilation
+@pytest.mark.parametrize("ic,oc,kernel,stride,dilation,pad", [(64, 64, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)),
+                                                              (48, 37, (3, 3), (1, 1), (1, 1), (0, 2, 1, 0)),
+                                                              (16, 32, (3, 3), (1, 2), (1, 1), (1, 1, 1, 1)),
+                                                              (16, 7, (1, 3), (1, 1), (1, 1), (0, 0, 1, 1)),
+                                                              (32, 64, (5, 5), (1, 1), (1, 1), (2, 2, 2, 2)),
+                                                              (80, 33, (2, 3), (1, 1), (2, 1), (2, 0, 3, 1)),
+                                                              (32, 20, (3, 3), (2, 2), (1, 3), (3, 1, 2, 4))])
+@pytest.mark.parametrize("batch,h,w", [(16, 61, 53), (5, 131, 90), (208, 11, 19), (3, 300, 67)])
+def test_window_convolution_rectangles(orc, ic, oc, kernel, stride, dilation, pad, batch, h, w):
+    import torch
+    from tests.test_gpu_parity import _conv_case, _gpu_conv
+    rng = np.random.default_rng(ic * oc + h)
+    orc.set_threads(16)
+    case = _conv_case(rng, batch, h, w, ic, oc, kernel, stride, dilation, pad, True, False, True, 1)
+    assert np.array_equal(_gpu_conv(case, stride, dilation, pad, 1, device_tensors=True, exact_3x3=True), orc.conv_int8(**case))
