@@ -271,6 +271,7 @@ struct RequantState {
   std::vector<int32_t> h_mult, h_ls, h_rs, h_bias2;
   int32_t amin = -128, amax = 127, zo = 0;
   bool has_zw = false, fast = false, fast2 = false;
+  int most_shift = 0;
 
   RequantParams params() const {
     RequantParams rq{};
@@ -288,6 +289,7 @@ struct RequantState {
     rq.c2lo = static_cast<const uint32_t *>(c2lo.p);
     rq.c2hi = static_cast<const uint32_t *>(c2hi.p);
     rq.pre = static_cast<const int32_t *>(pre.p);
+    rq.most_shift = most_shift;
     rq.fast2 = fast2 ? 1 : 0;
     return rq;
   }
@@ -318,6 +320,7 @@ struct RequantState {
       h_ls[c] = l1[qi];
       h_rs[c] = r1[qi];
       e[c] = std::min(31, -r1[qi]);
+      most_shift = std::max(most_shift, e[c]);
       zwv[c] = zws[qi];
       if (zwv[c] != 0) has_zw = true;
       int32_t wsum = 0;
@@ -1130,9 +1133,9 @@ static int mi_conv_create_impl(const mi_conv_desc *d, const int8_t *weight_host,
       rc = upload(&h->w_rows, conv_rows_weights(weight_host, oc, d->kernel_h, d->kernel_w, d->in_channel));
     } else if (rc == MI_OK && h->direct_1x1 && conv_thin_supported(kdim, oc)) {
       rc = upload(&h->w_thin, conv_thin_weights(weight_host, oc, kdim));
-    } else if (rc == MI_OK && conv_window_weights_wanted(shape) && h->st.fast2 && !h->st.has_zw) {
-      rc = upload(&h->w_window, conv_window_weights(weight_host, oc, kdim));
     }
+    if (rc == MI_OK && conv_window_weights_wanted(shape) && h->st.fast2 && !h->st.has_zw)
+      rc = upload(&h->w_window, conv_window_weights(shape, weight_host));
     if (rc == MI_OK) rc = upload(&h->fill16, std::vector<int8_t>(16, (int8_t)h->fill));
   }
   if (rc != MI_OK) {

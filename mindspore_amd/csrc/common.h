@@ -52,6 +52,7 @@ struct RequantParams {
   const uint32_t *mult2;
   const uint32_t *c2lo, *c2hi;
   const int32_t *pre;
+  int most_shift;  // the largest e
   int fast2;   // fast, and every mult >= 0, every c2 < 0, and K * 16384 + K * 128 * |zw| <= kAccBias (a in [0, 2^31))
 };
 
@@ -172,7 +173,7 @@ int launch_conv_thin(const int8_t *in, int64_t pixels, int k, int oc, const int8
 // without weight zero points; w: the weights as conv_window_weights lays them out, in device memory.  *taken false, and nothing
 // launched, where the gathering GEMM is faster or the window does not fit.
 bool conv_window_weights_wanted(const ConvGeom &g);
-std::vector<int8_t> conv_window_weights(const int8_t *w, int oc, int k);
+std::vector<int8_t> conv_window_weights(const ConvGeom &g, const int8_t *w);
 int conv_window_prepare_device();  // called by mi_init with the device current
 int launch_conv_window(const int8_t *in, const ConvGeom &g, const int8_t *fill16, const int8_t *w, const RequantParams &rq,
                        int8_t *out, hipStream_t stream, bool *taken);

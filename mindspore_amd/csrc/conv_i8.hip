@@ -281,13 +281,13 @@ int launch_conv_smallk(const int8_t *in, const ConvGeom &g, int fill, int k_true
 // requantisation parameters are loaded once and live in registers, and a 4 x 4 byte transposition across neighbouring
 // lanes makes dwords of four channels for the stores.  A wave keeps the weights of its up to 64 channels in registers
 // and walks tiles of 32 pixels, fetching the next tile's operand before it requantises the current one.
-// Bound at large sizes by the vector ALU (about 230 instructions per tile of 32 pixels x 64 channels, 190 of them the
-// requantisation) and by the loads, whose 64 unaligned addresses take the address unit about 95 cycles; at small ones by the
-// latency of one tile.  32 x 224 x 224 x 3 -> 64, 7x7, stride 2: 22.6 us, without loads 18, without stores 18, without either
-// 14.4; the order of tiles over the XCDs and the number of waves change nothing, and the rows through LDS, once each, gain 2 us
-// there and lose 1 everywhere else.  With masks and branches in every tile, and divisions by the vector ALU, it took 461
-// instructions.  us per launch, before that / with it: that 25.4 / 22.6; one such image 5.2 / 4.65; 16 x 224 x 224 x 3 -> 32,
-// 3x3, stride 2 6.4 / 5.65; 16 x 160 x 160 x 3 -> 64, 3x3 14.4 / 12.4; 16 x 224 x 224 x 4 -> 32, 5x5 20.1 / 16.4.
+// Bound at large sizes by the vector ALU (about 160 instructions per tile of 32 pixels x 64 channels, 120 of them the
+// requantisation), by the loads, whose 64 unaligned addresses take the address unit about 95 cycles, and by the stores; at small
+// ones by the latency of one tile.  The order of tiles over the XCDs and the number of waves change nothing; windows of many
+// loads go through LDS (conv_window.hip).  us per launch with masks and branches in every tile and divisions by the vector
+// ALU (461 instructions) / plain tiles (230) / with the requantisation and stores of conv_store.h: 32 x 224 x 224 x 3 -> 64, 7x7,
+// stride 2 25.4 / 22.6 / 20.5; 32 x 224 x 224 x 3 -> 32, 3x3, stride 2 10.6 / - / 7.7; 16 of those 6.5 / 5.65 / 5.2;
+// 16 x 160 x 160 x 3 -> 64, 3x3 14.7 / 12.4 / 10.9; 16 x 224 x 224 x 4 -> 32, 5x5 20 / 16.4 / 14.8.
 struct ConvRows {
   const int8_t *in;
   int in_bytes;
@@ -393,40 +393,31 @@ struct RowsGather {
 };
 
 // A tile's accumulators -> bytes in memory (see conv_store.h).
-template <int OCB, bool FAST>
+template <int OCB, RequantForm FORM>
 struct RowsStore {
-  ChannelRequant<OCB, FAST> requant;
+  ChannelRequant<OCB, FORM> requant;
   int my_n, my_p;
   uint32_t out_off;
 
   __device__ __forceinline__ RowsStore(const ConvRows &g, const RequantParams &rq, int n0, int lane) : requant(rq, n0, lane) {
-    my_n = n0 + (lane & 31 & ~3), my_p = 4 * (lane >> 5) + (lane & 3);
+    my_n = n0 + column_channel(OCB, 0, lane & 31 & ~3), my_p = 4 * (lane >> 5) + (lane & 3);
     out_off = (uint32_t)(my_p * g.out_c + my_n);
   }
   __device__ __forceinline__ void store(const ConvRows &g, const RequantParams &rq, v16i (&acc)[OCB], const v16i &sums, int tile,
                                         int n0, int8_t *out) const {
-    typedef uint32_t u32_any __attribute__((aligned(1)));
     wait_for_products(acc);
     int8_t *tile_out = out + (int64_t)tile * 32 * g.out_c;
     // (no branch between the pieces of a whole tile: one's chain of dependent instructions fills the gaps of the next)
     if (tile * 32 + 32 <= g.pixels && n0 + 32 * OCB <= g.out_c) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int ob = 0; ob < OCB; ++ob)
-          *reinterpret_cast<u32_any *>(tile_out + (8 * q * g.out_c + 32 * ob) + out_off) =
-              requant.four_channels(rq, acc, sums, q, ob);
+      for (int q = 0; q < 4; ++q) requant.template store<true>(rq, acc, sums, q, tile_out + 8 * q * g.out_c + out_off, 0);
       return;
     }
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-#pragma unroll
-      for (int ob = 0; ob < OCB; ++ob) {
-        const uint32_t four = requant.four_channels(rq, acc, sums, q, ob);
-        if (tile * 32 + 8 * q + my_p < g.pixels)
-          store_channels(tile_out + (8 * q * g.out_c + 32 * ob) + out_off, four, g.out_c - my_n - 32 * ob);
-      }
-    }
+    for (int q = 0; q < 4; ++q)
+      // (the transposition needs every lane: those whose pixel is not there store none of their channels)
+      requant.template store<false>(rq, acc, sums, q, tile_out + 8 * q * g.out_c + out_off,
+                                    tile * 32 + 8 * q + my_p < g.pixels ? g.out_c - my_n : 0);
   }
 };
 
@@ -437,14 +428,14 @@ __device__ __forceinline__ void rows_weights(const ConvRows &g, int n0, int lane
   for (int ob = 0; ob < OCB; ++ob)
 #pragma unroll
     for (int s = 0; s < KS; ++s)
-      wf[ob][s] = *reinterpret_cast<const v4i *>(g.w + (n0 + ob * 32 + (lane & 31)) * (32 * KS) + 32 * s + 16 * (lane >> 5));
+      wf[ob][s] = *reinterpret_cast<const v4i *>(g.w + (n0 + column_channel(OCB, ob, lane & 31)) * (32 * KS) + 32 * s + 16 * (lane >> 5));
 }
 
 // waves per SIMD: three where the weights leave registers for it
-constexpr int rows_occupancy(int ks, int ocb, bool fast) { return fast && ks * ocb <= 8 ? 3 : 2; }
+constexpr int rows_occupancy(int ks, int ocb, RequantForm form) { return form != kGeneralForm && ks * ocb <= 8 ? 3 : 2; }
 
-template <int KS, int OCB, bool FAST>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(rows_occupancy(KS, OCB, FAST)))) void conv_rows_kernel(
+template <int KS, int OCB, RequantForm FORM>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(rows_occupancy(KS, OCB, FORM)))) void conv_rows_kernel(
     ConvRows g, RequantParams rq, int8_t *__restrict__ out) {
   const int lane = threadIdx.x & 63;
   const int n0 = blockIdx.y * (32 * OCB);
@@ -454,12 +445,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(rows_occupa
 
   v4i wf[OCB][KS];
   rows_weights(g, n0, lane, wf);
-  const RowsStore<OCB, FAST> store(g, rq, n0, lane);
+  const RowsStore<OCB, FORM> store(g, rq, n0, lane);
   RowsGather<KS> in(g, lane);
   v16i start;
 #pragma unroll
   for (int e = 0; e < 16; ++e) start[e] = (int)kAccBias;
-  if (FAST) asm volatile("" : "+v"(start));  // one block of registers for every tile's first products
+  if (FORM != kGeneralForm) asm volatile("" : "+v"(start));  // one block of registers for every tile's first products
   in.locate(tile);
   v4i x[KS];
   in.fetch(x);
@@ -473,7 +464,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(rows_occupa
 #pragma unroll
       for (int ob = 0; ob < OCB; ++ob)
         acc[ob] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x[s], wf[ob][s], s == 0 ? start : acc[ob], 0, 0, 0);
-    if (!FAST && rq.has_zw) {  // the pixels' input sums, in the accumulators' layout: against ones where a window byte is
+    if (FORM == kGeneralForm && rq.has_zw) {  // the pixels' input sums, in the accumulators' layout: against ones where a window byte is
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
         v4i one;
@@ -531,24 +522,28 @@ int launch_conv_rows(const int8_t *in, const ConvGeom &g, int fill, const int8_t
     return MI_PARAM_INVALID;
   }
   const int64_t wgs = (pixels + 127) / 128;
-  const bool two = g.out_c > 32, fast = rq.fast2 != 0 && rq.has_zw == 0;
+  const bool two = g.out_c > 32;
+  const RequantForm form = requant_form(rq);
   const int gy = (g.out_c + (two ? 63 : 31)) / (two ? 64 : 32);
   // as many workgroups as the registers let the device hold, so that a wave walks several tiles on one set of weights.  us at
   // 32 x 224 x 224 x 3 -> 64, 7x7 (two per SIMD): 512 workgroups 22.6, 768 25.4; 16 x 224 x 224 x 3 -> 32, 3x3 (three):
   // 512 5.95, 768 5.65
-  const int most = 256 * rows_occupancy(ks, two ? 2 : 1, fast);
+  const int most = 256 * rows_occupancy(ks, two ? 2 : 1, form);
   const dim3 grid((unsigned)(wgs < most ? wgs : most), (unsigned)gy);
   magic31(c.out_hw, &c.magic_hw, &c.shift_hw);
   magic31(c.out_w, &c.magic_w, &c.shift_w);
-#define MI_ROWS(KS)                                                                                          \
-  case KS:                                                                                                   \
-    if (fast) {                                                                                              \
-      if (two) hipLaunchKernelGGL((conv_rows_kernel<KS, 2, true>), grid, dim3(256), 0, stream, c, rq, out);  \
-      else hipLaunchKernelGGL((conv_rows_kernel<KS, 1, true>), grid, dim3(256), 0, stream, c, rq, out);      \
-    } else {                                                                                                 \
-      if (two) hipLaunchKernelGGL((conv_rows_kernel<KS, 2, false>), grid, dim3(256), 0, stream, c, rq, out); \
-      else hipLaunchKernelGGL((conv_rows_kernel<KS, 1, false>), grid, dim3(256), 0, stream, c, rq, out);     \
-    }                                                                                                        \
+#define MI_ROWS_FORM(KS, FORM)                                                                              \
+  if (two) hipLaunchKernelGGL((conv_rows_kernel<KS, 2, FORM>), grid, dim3(256), 0, stream, c, rq, out);      \
+  else hipLaunchKernelGGL((conv_rows_kernel<KS, 1, FORM>), grid, dim3(256), 0, stream, c, rq, out)
+#define MI_ROWS(KS)                     \
+  case KS:                              \
+    if (form == kReluForm) {            \
+      MI_ROWS_FORM(KS, kReluForm);      \
+    } else if (form == kCarryForm) {    \
+      MI_ROWS_FORM(KS, kCarryForm);     \
+    } else {                            \
+      MI_ROWS_FORM(KS, kGeneralForm);   \
+    }                                   \
     break
   switch (ks) {
     MI_ROWS(1);
@@ -561,6 +556,7 @@ int launch_conv_rows(const int8_t *in, const ConvGeom &g, int fill, const int8_t
     MI_ROWS(8);
   }
 #undef MI_ROWS
+#undef MI_ROWS_FORM
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }

@@ -30,44 +30,77 @@ __device__ __forceinline__ uint32_t quad_transpose(uint32_t d, uint32_t sel1, ui
   return __builtin_amdgcn_perm(q, r, sel2);
 }
 
-// acc[ob][4 * q + e] is pixel 8 * q + 4 * h + e of 32, channel n0 + 32 * ob + r; after the transposition a lane holds channels
-// r & ~3 .. + 3 of pixel 8 * q + 4 * h + (lane & 3).
-// FAST: the one-multiply rounding form without weight zero points (RequantParams::fast2, !has_zw).
-template <int OCB, bool FAST>
+// How the convolutions requantise, see requant_form.
+enum RequantForm { kGeneralForm, kCarryForm, kReluForm };
+
+// kCarryForm: the one-multiply rounding without weight zero points, shifts up to 23 (so that the output range, shifted, is an int32).
+// kReluForm: the same where no output is below the zero point (an activation): a negative x of RequantParams::fast2 ends below the
+// range with [x >= 0] = 1 as it does with 0, so that pre + 1 goes into c2's high dword, and the carry and its add are not needed.
+inline RequantForm requant_form(const RequantParams &rq) {
+  if (rq.fast2 == 0 || rq.has_zw != 0 || rq.most_shift > 23) return kGeneralForm;
+  return rq.amin >= rq.zo ? kReluForm : kCarryForm;
+}
+
+// The channel of a group of 32 * OCB that column r of channel block ob computes: with two blocks a lane's two quads of channels
+// (after the transposition) are neighbours in memory.
+__host__ __device__ __forceinline__ int column_channel(int ocb, int ob, int r) { return ocb == 2 ? 8 * (r >> 2) + 4 * ob + (r & 3) : r; }
+
+// acc[ob][4 * q + e] is pixel 8 * q + 4 * h + e of 32, channel n0 + column_channel(OCB, ob, r); after the transposition a lane holds
+// the quad of channels from n0 + column_channel(OCB, ob, r & ~3) of pixel 8 * q + 4 * h + (lane & 3).
+// Vector instructions per quad: 23 with a shift and a clamp of its own for each output and a carry, 19 in kCarryForm and 15 in
+// kReluForm, whose clamps come before the shift that saturates and packs.
+template <int OCB, RequantForm FORM>
 struct ChannelRequant {
   int32_t mult[OCB], bias[OCB], shift[OCB], lsh[OCB], zw[OCB];  // of this lane's channel of each block
+  int32_t least[OCB], most[OCB];  // the output range before the shift
   uint64_t c2[OCB];
-  int amin_v, amax_v;
   uint32_t sel1, sel2;
 
   __device__ __forceinline__ ChannelRequant(const RequantParams &rq, int n0, int lane) {
-    const int r = lane & 31;
 #pragma unroll
     for (int ob = 0; ob < OCB; ++ob) {
-      const int n = n0 + ob * 32 + r;  // (the arrays are padded to a multiple of 256 channels)
+      const int n = n0 + column_channel(OCB, ob, lane & 31);  // (the arrays are padded to a multiple of 256 channels)
       shift[ob] = rq.rshift[n];
-      if (FAST) {
-        mult[ob] = (int32_t)rq.mult2[n];
-        c2[ob] = (uint64_t)rq.c2hi[n] << 32 | rq.c2lo[n];
-        bias[ob] = rq.pre[n];
-      } else {
+      if (FORM == kGeneralForm) {
         mult[ob] = rq.mult[n];
         bias[ob] = (int32_t)((uint32_t)rq.bias2[n] - kAccBias);
         lsh[ob] = rq.lshift[n];
         zw[ob] = rq.zw[n];
+      } else {
+        mult[ob] = (int32_t)rq.mult2[n];
+        bias[ob] = rq.pre[n];
+        const uint32_t hi = rq.c2hi[n] + (FORM == kReluForm ? (uint32_t)bias[ob] + 1 : 0);
+        c2[ob] = (uint64_t)hi << 32 | rq.c2lo[n];
+        least[ob] = (int32_t)((uint32_t)rq.amin << shift[ob]);
+        most[ob] = (int32_t)((uint32_t)(rq.amax + 1) << shift[ob]) - 1;
       }
     }
-    amin_v = rq.amin, amax_v = rq.amax;
-    asm volatile("" : "+v"(amin_v), "+v"(amax_v));  // kept in vector registers, as v_med3 wants them
     sel1 = (lane & 1) ? 0x03070105u : 0x06020400u, sel2 = (lane & 2) ? 0x03020706u : 0x05040100u;
   }
   __device__ __forceinline__ uint32_t four_channels(const RequantParams &rq, const v16i (&acc)[OCB], const v16i &sums, int q,
                                                     int ob) const {
-    int y[4];
-    if (FAST) {
+    if (FORM == kGeneralForm) {
+      int y[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        uint32_t v = (uint32_t)acc[ob][4 * q + e] - (uint32_t)sums[4 * q + e] * (uint32_t)zw[ob] + (uint32_t)bias[ob];
+        int32_t t = rdiv_pot(srdhm((int32_t)(v << lsh[ob]), mult[ob]), shift[ob]);
+        t = (int32_t)((uint32_t)t + (uint32_t)rq.zo);
+        t = t < rq.amax ? t : rq.amax;
+        y[e] = t > rq.amin ? t : rq.amin;
+      }
+      const uint32_t p01 = __builtin_amdgcn_perm((uint32_t)y[1], (uint32_t)y[0], 0x0c0c0400u);
+      const uint32_t p23 = __builtin_amdgcn_perm((uint32_t)y[3], (uint32_t)y[2], 0x0c0c0400u);
+      return quad_transpose(__builtin_amdgcn_perm(p23, p01, 0x05040100u), sel1, sel2);
+    }
+    int32_t t[4];
+    if (FORM == kReluForm) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        t[e] = (int32_t)(((uint64_t)(uint32_t)acc[ob][4 * q + e] * (uint32_t)mult[ob] + c2[ob]) >> 32);
+    } else {
       // one 64-bit multiply-add per output; its carry is the rounding's "+1 unless negative"
       uint64_t p2[4], carry[4], unused;
-      int32_t t[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         asm("v_mad_u64_u32 %0, %1, %2, %3, %4"
@@ -78,24 +111,39 @@ struct ChannelRequant {
         asm("v_addc_co_u32_e64 %0, %1, %2, %3, %4"
             : "=v"(t[e]), "=s"(unused)
             : "v"((int32_t)(p2[e] >> 32)), "v"(bias[ob]), "s"(carry[e]));
+    }
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        t[e] >>= shift[ob];
-        asm("v_med3_i32 %0, %1, %2, %3" : "=v"(y[e]) : "v"(t[e]), "v"(amin_v), "v"(amax_v));
-      }
-    } else {
+    for (int e = 0; e < 4; ++e) asm("v_med3_i32 %0, %0, %1, %2" : "+v"(t[e]) : "v"(least[ob]), "v"(most[ob]));
+    const uint32_t p01 = (uint16_t)__builtin_amdgcn_ashr_pk_i8_i32((uint32_t)t[0], (uint32_t)t[1], (uint32_t)shift[ob]);
+    const uint32_t p23 = (uint16_t)__builtin_amdgcn_ashr_pk_i8_i32((uint32_t)t[2], (uint32_t)t[3], (uint32_t)shift[ob]);
+    return quad_transpose(__builtin_amdgcn_perm(p23, p01, 0x05040100u), sel1, sel2);
+  }
+  // Non-temporal: written out while the launch runs and not at its end.  us, temporal -> this: 32 x 224 x 224 x 3 -> 64, 7x7, stride 2
+  // 17.4 -> 16.5, eight of them 6.35 -> 5.8, 32 x 224 x 224 x 3 -> 32, 3x3, stride 2 9.55 -> 8.7.
+  // quad q of each block, which is 4 * OCB neighbouring channels, to `to`; WHOLE: all exist, otherwise `have` of them do
+  template <bool WHOLE>
+  __device__ __forceinline__ void store(const RequantParams &rq, const v16i (&acc)[OCB], const v16i &sums, int q, int8_t *to,
+                                        int have) const {
+    typedef uint32_t u32_any __attribute__((aligned(1)));
+    typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+    typedef v2u v2u_any __attribute__((aligned(1)));
+    uint32_t four[OCB];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        uint32_t v = (uint32_t)acc[ob][4 * q + e] - (uint32_t)sums[4 * q + e] * (uint32_t)zw[ob] + (uint32_t)bias[ob];
-        int32_t t = rdiv_pot(srdhm((int32_t)(v << lsh[ob]), mult[ob]), shift[ob]);
-        t = (int32_t)((uint32_t)t + (uint32_t)rq.zo);
-        t = t < rq.amax ? t : rq.amax;
-        y[e] = t > rq.amin ? t : rq.amin;
+    for (int ob = 0; ob < OCB; ++ob) four[ob] = four_channels(rq, acc, sums, q, ob);
+    if (WHOLE && OCB == 2) {
+      __builtin_nontemporal_store((v2u{four[0], four[OCB - 1]}), reinterpret_cast<v2u_any *>(to));
+      return;
+    }
+#pragma unroll
+    for (int ob = 0; ob < OCB; ++ob) {
+      if (WHOLE || have >= 4 * ob + 4) {
+        __builtin_nontemporal_store(four[ob], reinterpret_cast<u32_any *>(to + 4 * ob));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+          if (4 * ob + e < have) to[4 * ob + e] = (int8_t)(four[ob] >> (8 * e));
       }
     }
-    const uint32_t p01 = __builtin_amdgcn_perm((uint32_t)y[1], (uint32_t)y[0], 0x0c0c0400u);
-    const uint32_t p23 = __builtin_amdgcn_perm((uint32_t)y[3], (uint32_t)y[2], 0x0c0c0400u);
-    return quad_transpose(__builtin_amdgcn_perm(p23, p01, 0x05040100u), sel1, sel2);
   }
 };
 
@@ -105,18 +153,6 @@ template <int OCB>
 __device__ __forceinline__ void wait_for_products(v16i (&acc)[OCB]) {
   if constexpr (OCB == 1) asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc[0]));
   if constexpr (OCB == 2) asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc[0]), "+v"(acc[1]));
-}
-
-// four channels of a pixel, as far as they exist
-__device__ __forceinline__ void store_channels(int8_t *to, uint32_t four, int have) {
-  typedef uint32_t u32_any __attribute__((aligned(1)));
-  if (have >= 4) {
-    *reinterpret_cast<u32_any *>(to) = four;
-  } else {
-#pragma unroll
-    for (int e = 0; e < 3; ++e)
-      if (e < have) to[e] = (int8_t)(four >> (8 * e));
-  }
 }
 
 }  // namespace mi

@@ -15,14 +15,21 @@ namespace mi {
 // LDS: weights in operand order, 1 KiB per 32 channels and 32 bytes of K; the input pixels row by row, each an odd number of
 // 16-byte chunks apart, so that the 32 pixels of a fragment read (neighbours, or every second one) spread over the banks.
 // K runs over taps, then channels, in chunks of 16; a step is two chunks, one for each half of the wave, whose LDS offsets come
-// from a table.  The pixels are the MFMA's row operand and the stores those of conv_rows_kernel.
+// from a table.  The pixels are the MFMA's row operand, see conv_store.h.
 // A workgroup lasts about 4 us (fetch 1.5, products 1, requantisation and stores 1.5), which two per CU overlap: bound by that
 // chain up to 512 workgroups and by LDS reads and the vector ALU beyond.  us per launch, gathering GEMM -> this: 32 x 56 x 56,
-// 64 -> 64 channels 12.1 -> 9.2; 512 x 14 x 14 12.6 -> 9.7; 512 x 512, 16 -> 16 10.0 -> 7.4; 64 x 28 x 28, 32 -> 64, 5x5 9.3 -> 6.7;
-// 64 x 56 x 56, 32 -> 32, stride 2 5.8 -> 5.0.  With every load waited for at the first barrier 9.8 at the first of these, and
-// then as four waves of 64 pixels each 10.0, four of 32 in rectangles of 128 11.4, eight of 64 in 512 10.5.
+// 64 -> 64 channels 11.9 -> 7.8; 512 x 14 x 14 11.6 -> 7.9; 64 x 56 x 56, 32 -> 32, stride 2 5.6 -> 4.5.  With every load waited for
+// at the first barrier 0.9 more at the first of these, and then as four waves of 64 pixels each 2 % more, four of 32 in
+// rectangles of 128 16 %, eight of 64 in 512 7 %.
+//
+// PACKED: the first layer's three or four channels, four bytes a pixel in LDS.  A window row is one or two chunks of four pixels
+// (zero weights behind its last tap and in a fourth byte that is no channel), read at any pixel.  conv_rows_kernel takes such
+// rows straight from the image in unaligned 16-byte loads, about 95 cycles of the address unit each; here a pixel's bytes are
+// loaded once, four pixels a lane.  32 x 224 x 224 x 3 -> 64, 7x7, stride 2: 20.5 us -> 16.5, of which launch and prologue 5.9,
+// the pixels 2, products 3, stores about 5 (26 MB); vector instructions are 255 a wave.
 struct ConvWindow {
   const int8_t *in;
+  const int8_t *in_last4;  // the tensor's last four bytes
   int in_h, in_w, in_c, out_h, out_w, out_c;
   int kernel_h, kernel_w, stride_h, stride_w, dil_h, dil_w, pad_u, pad_l;
   int tile_h, tile_w, tiles_x, tiles_y;  // output pixels of a workgroup
@@ -30,7 +37,7 @@ struct ConvWindow {
   int cc, pitch;                         // chunks per pixel, and from one pixel to the next in LDS
   int steps;                             // of 32 bytes of K
   int weight_bytes, patch_bytes;         // in LDS, multiples of 1 KiB
-  uint32_t magic_pitch, magic_patch_w, magic_tile_w;  // ceil(2^32 / d): exact quotients for dividends < 2^16 (d >= 2; 0: d = 1)
+  uint32_t magic_pitch, magic_patch_w, magic_tile_w, magic_cc, magic_kernel_w, magic_quads;  // ceil(2^32 / d): exact quotients for dividends < 2^16 (d >= 2; 0: d = 1)
   uint32_t magic_tiles_x, magic_tiles_y;  // see magic31
   int shift_tiles_x, shift_tiles_y;
   const int8_t *w;       // [32 channels][step][lane][16]
@@ -40,8 +47,12 @@ struct ConvWindow {
 __device__ __forceinline__ int quotient16(int p, uint32_t magic) { return magic == 0 ? p : (int)__umulhi((uint32_t)p, magic); }
 
 constexpr int kWaves = 8;
+typedef uint32_t u32_any __attribute__((aligned(1)));
+typedef v4i v4i_4 __attribute__((aligned(4)));
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+typedef v4u v4u_any __attribute__((aligned(1)));
 
-template <int OCB>
+template <int OCB, bool PACKED, RequantForm FORM>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWaves / 2))) void conv_window_kernel(ConvWindow g, RequantParams rq,
                                                                                                 int8_t *__restrict__ out) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
@@ -49,7 +60,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWa
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int row_id = quotient31(blockIdx.x, g.magic_tiles_x, g.shift_tiles_x), b = quotient31(row_id, g.magic_tiles_y, g.shift_tiles_y);
   const int tx0 = (blockIdx.x - row_id * g.tiles_x) * g.tile_w, ty0 = (row_id - b * g.tiles_y) * g.tile_h;
-  const ChannelRequant<OCB, true> requant(rq, 0, lane);
+  const ChannelRequant<OCB, FORM> requant(rq, 0, lane);
 
   auto to_lds = [](const void *from, void *wave_base) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)from,
@@ -60,14 +71,40 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWa
   // The first weights, the pixels, the last two loads of weights of each wave: the products of the first weights begin while
   // those are on their way.
   constexpr int kLate = 2, kLateSteps = kWaves * kLate / OCB;
-  const int early = max(g.steps - kLateSteps, 0);  // steps whose weights come first
+  const int early = PACKED ? 0 : max(g.steps - kLateSteps, 0);  // steps whose weights come first
   auto load_weights = [&](int from, int to) {
     for (int i = from * OCB + wave; i < to * OCB; i += kWaves) {
       to_lds(g.w + (i % OCB * g.steps + i / OCB) * 1024 + lane * 16, lds + i * 1024);
     }
   };
+  // four pixels at a time; those of an image's edges, and the tensor's last ones, one by one
+  auto load_patch = [&] {
+    const int iy0 = ty0 * g.stride_h - g.pad_u, ix0 = tx0 * g.stride_w - g.pad_l, line = g.in_w * g.in_c;
+    const int8_t *image = g.in + (int64_t)b * g.in_h * line;
+    const int row_quads = g.patch_w >> 2, quads = g.patch_h * row_quads;
+    for (int i = tid; i < quads; i += 64 * kWaves) {
+      const int row = quotient16(i, g.magic_quads), iy = iy0 + row, ix = ix0 + 4 * (i - row * row_quads);
+      const int8_t *want = image + iy * line + ix * g.in_c;
+      v4u v;
+      if ((unsigned)iy < (unsigned)g.in_h && ix >= 0 && ix + 4 <= g.in_w && want <= g.in_last4 - 12) {
+        v = *reinterpret_cast<const v4u_any *>(want);
+        if (g.in_c == 3)
+          v = v4u{v[0], __builtin_amdgcn_alignbyte(v[1], v[0], 3), __builtin_amdgcn_alignbyte(v[2], v[1], 2), v[2] >> 8};
+      } else {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const bool inside = (unsigned)iy < (unsigned)g.in_h && (unsigned)(ix + u) < (unsigned)g.in_w;
+          const int8_t *px = want + u * g.in_c, *from = px < g.in_last4 ? px : g.in_last4;
+          v[u] = *reinterpret_cast<const u32_any *>(inside ? from : g.fill16) >> (inside ? (uint32_t)(px - from) * 8 : 0);
+        }
+      }
+      reinterpret_cast<v4u *>(patch)[i] = v;
+    }
+  };
   load_weights(0, early);
-  {
+  if constexpr (PACKED) {
+    load_patch();
+  } else {
     const int iy0 = ty0 * g.stride_h - g.pad_u, ix0 = tx0 * g.stride_w - g.pad_l;
     const int8_t *image = g.in + (int64_t)b * g.in_h * g.in_w * g.in_c;
     const int chunks = g.patch_h * g.patch_w * g.pitch;
@@ -79,22 +116,22 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWa
     }
   }
   load_weights(early, g.steps);
-  // the table: where chunk f of a window lies from its first byte (behind the last chunk: that one again, against zeros)
-  const int taps = g.kernel_h * g.kernel_w;
-  for (int f = tid; f < 2 * g.steps; f += 64 * kWaves) {
-    const int ff = min(f, taps * g.cc - 1), tap = ff / g.cc, kh = tap / g.kernel_w, kw = tap - kh * g.kernel_w;
-    table[f] = ((kh * g.dil_h * g.patch_w + kw * g.dil_w) * g.pitch + ff - tap * g.cc) * 16;
+  if constexpr (!PACKED) {
+    // the table: where chunk f of a window lies from its first byte (behind the last chunk: that one again, against zeros)
+    for (int f = tid; f < 2 * g.steps; f += 64 * kWaves) {
+      const int ff = min(f, g.kernel_h * g.kernel_w * g.cc - 1), tap = quotient16(ff, g.magic_cc);
+      const int kh = quotient16(tap, g.magic_kernel_w), kw = tap - kh * g.kernel_w;
+      table[f] = ((kh * g.dil_h * g.patch_w + kw * g.dil_w) * g.pitch + ff - tap * g.cc) * 16;
+    }
   }
   // Pixel t of the rectangle; where there is none, past the rectangle's last or outside the image, its first pixel again, which
   // is then computed and stored more than once.
-  auto locate = [&](int t, int *ty, int *tx) {
-    *ty = quotient16(t, g.magic_tile_w);
-    *tx = t - *ty * g.tile_w;
-    if (*ty >= g.tile_h || ty0 + *ty >= g.out_h || tx0 + *tx >= g.out_w) *ty = *tx = 0;
-  };
-  int my_ty, my_tx;
-  locate(wave * 32 + r, &my_ty, &my_tx);
-  const char *px = patch + (my_ty * g.stride_h * g.patch_w + my_tx * g.stride_w) * g.pitch * 16;
+  const int have_h = min(g.tile_h, g.out_h - ty0), have_w = min(g.tile_w, g.out_w - tx0);
+  const int my_ty = quotient16(wave * 32 + r, g.magic_tile_w), my_tx = wave * 32 + r - my_ty * g.tile_w;
+  const int my_px = my_ty < have_h && my_tx < have_w ? my_ty * g.stride_h * g.patch_w + my_tx * g.stride_w : 0;
+  // Packed, a step is one window row of two chunks or two of one chunk (behind the last row: one more, against zeros).
+  const int row_bytes = g.dil_h * g.patch_w * 4, step_bytes = g.cc == 2 ? row_bytes : 2 * row_bytes;
+  const char *px = patch + (PACKED ? my_px * 4 + h * (g.cc == 2 ? 16 : row_bytes) : my_px * g.pitch * 16);
   v16i start;
 #pragma unroll
   for (int e = 0; e < 16; ++e) start[e] = (int)kAccBias;
@@ -108,7 +145,11 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWa
   v16i acc[OCB];
   const char *wl = lds + lane * 16;
   auto read = [&](v4i &x, v4i (&w)[OCB], int s, int off) {
-    x = *reinterpret_cast<const v4i *>(px + off);
+    if constexpr (PACKED) {
+      x = *reinterpret_cast<const v4i_4 *>(px + off);
+    } else {
+      x = *reinterpret_cast<const v4i *>(px + off);
+    }
 #pragma unroll
     for (int ob = 0; ob < OCB; ++ob) w[ob] = *reinterpret_cast<const v4i *>(wl + (s * OCB + ob) * 1024);
   };
@@ -116,46 +157,54 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWa
 #pragma unroll
     for (int ob = 0; ob < OCB; ++ob) acc[ob] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x, w[ob], acc[ob], 0, 0, 0);
   };
-#pragma unroll
-  for (int ob = 0; ob < OCB; ++ob) acc[ob] = start;
-  // steps [from, to): operands one step ahead, offsets two
-  auto run = [&](int from, int to) {
+  auto offset = [&](int s) {
+    if constexpr (PACKED) return s * step_bytes;
+    return table[2 * s + h];
+  };
+  // steps [from, to), the first ones or not: operands one step ahead, offsets two
+  auto run = [&](int from, int to, auto first_c) {
     v4i x0, w0[OCB], x1, w1[OCB];
     const int last = to - 1;
-    read(x0, w0, from, table[2 * from + h]);
-    int off = table[2 * min(from + 1, last) + h];
-    int s = from;
-    for (; s < last; s += 2) {
-      read(x1, w1, s + 1, off);
-      off = table[2 * min(s + 2, last) + h];
+    read(x0, w0, from, offset(from));
+    read(x1, w1, min(from + 1, last), offset(min(from + 1, last)));
+    int off = offset(min(from + 2, last)), s = from + 1;
+    if constexpr (decltype(first_c)::value) {  // the accumulators from one block of registers
+#pragma unroll
+      for (int ob = 0; ob < OCB; ++ob) acc[ob] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x0, w0[ob], start, 0, 0, 0);
+    } else {
       mma(x0, w0);
-      read(x0, w0, min(s + 2, last), off);
-      off = table[2 * min(s + 3, last) + h];
-      mma(x1, w1);
     }
-    if (s == last) mma(x0, w0);
+    for (; s < last; s += 2) {
+      read(x0, w0, s + 1, off);
+      off = offset(min(s + 2, last));
+      mma(x1, w1);
+      read(x1, w1, min(s + 2, last), off);
+      off = offset(min(s + 3, last));
+      mma(x0, w0);
+    }
+    if (s == last) mma(x1, w1);
   };
   if (early > 0) {
-    run(0, early);
+    run(0, early, std::true_type());
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    run(early, g.steps, std::false_type());
+  } else {
+    run(0, g.steps, std::true_type());
   }
-  run(early, g.steps);
 
-  // acc[ob][4 * q + e]: pixel 32 * wave + 8 * q + 4 * h + e of the rectangle, channel 32 * ob + r
-  const int my_n = r & ~3;
-  int8_t *image_out = out + (int64_t)b * g.out_h * g.out_w * g.out_c;
+  // acc[ob][4 * q + e]: pixel 32 * wave + 8 * q + 4 * h + e of the rectangle
+  const int my_n = column_channel(OCB, 0, r & ~3), first = wave * 32 + 4 * h + (lane & 3);
+  int8_t *rectangle = out + ((int64_t)(b * g.out_h + ty0) * g.out_w + tx0) * g.out_c;
+  int ty = quotient16(first, g.magic_tile_w), tx = first - ty * g.tile_w;
+  uint32_t at = (uint32_t)(ty * g.out_w + tx) * g.out_c;
   wait_for_products(acc);
   auto store = [&](auto whole_c) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      int ty, tx;
-      locate(wave * 32 + 8 * q + 4 * h + (lane & 3), &ty, &tx);
-      int8_t *to = image_out + ((int64_t)(ty0 + ty) * g.out_w + tx0 + tx) * g.out_c + my_n;
-#pragma unroll
-      for (int ob = 0; ob < OCB; ++ob) {
-        const uint32_t four = requant.four_channels(rq, acc, start, q, ob);
-        store_channels(to + 32 * ob, four, decltype(whole_c)::value ? 4 : g.out_c - my_n - 32 * ob);
-      }
+      const uint32_t to = (ty < have_h && tx < have_w ? at : 0u) + my_n;
+      requant.template store<decltype(whole_c)::value>(rq, acc, start, q, rectangle + to, g.out_c - my_n);
+      tx += 8, at += 8 * g.out_c;  // (a rectangle is at least that wide)
+      if (tx >= g.tile_w) tx -= g.tile_w, ++ty, at += (g.out_w - g.tile_w) * g.out_c;
     }
   };
   if (32 * OCB <= g.out_c) {
@@ -168,13 +217,31 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWa
 // ---- host side -----------------------------------------------------------------------------------------------------
 static uint32_t magic16(int d) { return d <= 1 ? 0u : (uint32_t)((((uint64_t)1 << 32) + d - 1) / (uint64_t)d); }
 
-std::vector<int8_t> conv_window_weights(const int8_t *w, int oc, int k) {
-  const int steps = (k + 31) / 32;
+static std::vector<int8_t> operand_order(const int8_t *w, int oc, int k) {
+  const int steps = (k + 31) / 32, ocb = oc > 32 ? 2 : 1;
   std::vector<int8_t> out((size_t)((oc + 31) / 32) * steps * 1024, 0);
-  for (int n = 0; n < oc; ++n)
+  for (int column = 0; column < 32 * ocb; ++column) {
+    const int n = column_channel(ocb, column / 32, column % 32);
+    if (n >= oc) continue;
     for (int k0 = 0; k0 < k; k0 += 16)
-      memcpy(&out[(((size_t)(n / 32) * steps + k0 / 32) * 64 + n % 32 + 32 * (k0 / 16 % 2)) * 16], w + (size_t)n * k + k0, 16);
+      memcpy(&out[(((size_t)(column / 32) * steps + k0 / 32) * 64 + column % 32 + 32 * (k0 / 16 % 2)) * 16], w + (size_t)n * k + k0, 16);
+  }
   return out;
+}
+
+// few channels, four bytes a pixel in LDS
+static bool packed_window(const ConvGeom &g) { return g.in_c <= 4; }
+static int row_chunks(const ConvGeom &g) { return (g.kernel_w + 3) / 4; }
+
+std::vector<int8_t> conv_window_weights(const ConvGeom &g, const int8_t *w) {
+  if (!packed_window(g)) return operand_order(w, g.out_c, g.kernel_h * g.kernel_w * g.in_c);
+  const int k = g.kernel_h * row_chunks(g) * 16;
+  std::vector<int8_t> wide((size_t)g.out_c * k, 0);
+  for (int n = 0; n < g.out_c; ++n)
+    for (int kh = 0; kh < g.kernel_h; ++kh)
+      for (int kw = 0; kw < g.kernel_w; ++kw)
+        memcpy(&wide[(size_t)n * k + kh * row_chunks(g) * 16 + kw * 4], w + (((size_t)n * g.kernel_h + kh) * g.kernel_w + kw) * g.in_c, g.in_c);
+  return operand_order(wide.data(), g.out_c, k);
 }
 
 constexpr int kWindowLds = 80 << 10;  // two workgroups per CU
@@ -186,22 +253,25 @@ struct WindowCut {
 static bool cut_window(const ConvGeom &g, WindowCut *best) {
   const int cc = g.in_c / 16, most = 32 * kWaves;  // (tile_w <= most)
   WindowCut c{};
+  const bool packed = packed_window(g);
   c.pitch = cc | 1;
-  c.steps = (g.kernel_h * g.kernel_w * cc + 1) / 2;
+  c.steps = packed ? (g.kernel_h * row_chunks(g) + 1) / 2 : (g.kernel_h * g.kernel_w * cc + 1) / 2;
   c.weight_bytes = (g.out_c > 32 ? 2 : 1) * c.steps * 1024;
   best->tiles = 0;
   for (int nx = (g.out_w + 63) / 64, last = std::min(64, (g.out_w + 7) / 8); nx <= last; ++nx) {  // 8 to 64 pixels wide
     c.tile_w = (g.out_w + nx - 1) / nx;
+    if (c.tile_w < 8) continue;
     c.tiles_x = (g.out_w + c.tile_w - 1) / c.tile_w;
     c.tile_h = std::min(most / c.tile_w, g.out_h);
     c.tiles_y = (g.out_h + c.tile_h - 1) / c.tile_h;
     c.tile_h = (g.out_h + c.tiles_y - 1) / c.tiles_y;
     const int64_t ph = (int64_t)(c.tile_h - 1) * g.stride_h + (int64_t)(g.kernel_h - 1) * g.dilation_h + 1;
-    const int64_t pw = (int64_t)(c.tile_w - 1) * g.stride_w + (int64_t)(g.kernel_w - 1) * g.dilation_w + 1;
+    int64_t pw = (int64_t)(c.tile_w - 1) * g.stride_w + (packed ? 4 * row_chunks(g) : (int64_t)(g.kernel_w - 1) * g.dilation_w + 1);
+    if (packed) pw = (pw + 3) & ~3;
     if (ph > 4096 || pw > 4096) continue;
     c.patch_h = (int)ph;
     c.patch_w = (int)pw;
-    const int64_t bytes = (ph * pw * c.pitch * 16 + 1023) / 1024 * 1024;  // (hence fewer than 2^16 chunks)
+    const int64_t bytes = ((ph + (packed ? g.dilation_h : 0)) * pw * (packed ? 4 : c.pitch * 16) + 1023) / 1024 * 1024;  // (hence fewer than 2^16 chunks)
     if (c.weight_bytes + bytes + 8 * c.steps > kWindowLds) continue;
     c.patch_bytes = (int)bytes;
     c.tiles = (int64_t)c.tiles_x * c.tiles_y * g.batch;
@@ -213,40 +283,54 @@ static bool cut_window(const ConvGeom &g, WindowCut *best) {
 // Up to 64 channels, which one workgroup computes (more would fetch the pixels again), rectangles for two CUs in three, and at
 // least half of their pixels there.  Time of this relative to the gathering GEMM, 3x3: workgroups 112 1.01, 128 1.02, 140 1.02,
 // 160 1.02, 168 0.88 0.91, 192 0.87, 196 0.89, 224 0.87, 256 0.77, 448 0.75, 1024 0.70; stride 2 256 0.74; 5x5 128 0.84, 256 0.73.
-// Rectangles filled to 0.77 0.77, 0.56 0.87, 0.39 0.90 to 1.05, 0.25 1.43, 0.19 1.40 to 2.1.  Before its waits were cut, against
-// 65 to 128 channels 0.99 to 1.24.
+// Rectangles filled to 0.77 0.77, 0.56 0.87, 0.39 0.90 to 1.05, 0.25 1.43, 0.19 1.40 to 2.1.  Against 65 to 128 channels 0.99 to 1.24.
+// Three or four channels: windows for which conv_rows_kernel makes five or more loads.  Time relative to that one, us: 7x7 on 3
+// channels -> 64, 49 workgroups 4.42 / 4.42, 98 4.46 / 4.48, 196 6.2 / 4.65, 392 8.55 / 6.05, 784 12.2 / 9.55, 1568 20.5 / 16.5;
+// 5x5 on 4 (five loads) 4.85 / 4.4 and 14.8 / 14.7; 5x5 on 3 (three) 4.15 / 4.18; 3x3 on 3 (two) 5.17 / 5.55 and 7.7 / 8.8.
 constexpr int kWindowLeastTiles = 168;
 bool conv_window_weights_wanted(const ConvGeom &g) {
-  return (g.in_c & 15) == 0 && g.out_c <= 64 && g.kernel_h * g.kernel_w > 1 && (int64_t)g.kernel_h * g.kernel_w * g.in_c <= 2048;
+  const int taps = g.kernel_h * g.kernel_w;
+  if (g.in_c == 3 || g.in_c == 4)
+    return g.out_c <= 64 && g.kernel_w <= 8 && g.kernel_h <= 16 && g.dilation_w == 1 && g.kernel_h * (g.kernel_w * g.in_c > 16 ? 2 : 1) > 8;
+  return (g.in_c & 15) == 0 && g.out_c <= 64 && taps > 1 && (int64_t)taps * g.in_c <= 2048;
 }
 static bool choose_window(const ConvGeom &g, const void *in, WindowCut *c) {
-  return conv_window_weights_wanted(g) && (reinterpret_cast<uintptr_t>(in) & 15) == 0 && cut_window(g, c) && c->tiles >= kWindowLeastTiles &&
+  return conv_window_weights_wanted(g) && ((reinterpret_cast<uintptr_t>(in) & 15) == 0 || packed_window(g)) && (int64_t)g.batch * g.in_h * g.in_w * g.in_c >= 16 && (int64_t)g.in_h * g.in_w * g.in_c < (int64_t)1 << 31 && cut_window(g, c) && c->tiles >= kWindowLeastTiles &&
          c->tiles * (32 * kWaves / 2) <= (int64_t)g.batch * g.out_h * g.out_w && c->tiles < 1 << 23;  // (2^32 threads)
 }
 
+typedef void (*WindowKernel)(ConvWindow, RequantParams, int8_t *);
 int conv_window_prepare_device() {  // (more than 64 KiB of dynamic LDS)
-  for (const void *kernel : {reinterpret_cast<const void *>(conv_window_kernel<1>), reinterpret_cast<const void *>(conv_window_kernel<2>)})
-    MI_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kWindowLds));
+  for (const WindowKernel kernel : {conv_window_kernel<1, false, kCarryForm>, conv_window_kernel<2, false, kCarryForm>,
+                                    conv_window_kernel<1, false, kReluForm>, conv_window_kernel<2, false, kReluForm>})
+    MI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kWindowLds));
   return MI_OK;
 }
 
 int launch_conv_window(const int8_t *in, const ConvGeom &g, const int8_t *fill16, const int8_t *w, const RequantParams &rq,
                        int8_t *out, hipStream_t stream, bool *taken) {
   WindowCut t;
-  *taken = choose_window(g, in, &t);
+  *taken = requant_form(rq) != kGeneralForm && choose_window(g, in, &t);
   if (!*taken) return MI_OK;
-  ConvWindow c{in, g.in_h, g.in_w, g.in_c, g.out_h, g.out_w, g.out_c, g.kernel_h, g.kernel_w, g.stride_h, g.stride_w, g.dilation_h,
-               g.dilation_w, g.pad_u, g.pad_l, t.tile_h, t.tile_w, t.tiles_x, t.tiles_y, t.patch_h, t.patch_w, g.in_c / 16, t.pitch,
-               t.steps, t.weight_bytes, t.patch_bytes, magic16(t.pitch), magic16(t.patch_w), magic16(t.tile_w), 0, 0, 0, 0, w, fill16};
+  const bool packed = packed_window(g);
+  ConvWindow c{in, in + (int64_t)g.batch * g.in_h * g.in_w * g.in_c - 4, g.in_h, g.in_w, g.in_c, g.out_h, g.out_w, g.out_c, g.kernel_h, g.kernel_w, g.stride_h, g.stride_w, g.dilation_h,
+               g.dilation_w, g.pad_u, g.pad_l, t.tile_h, t.tile_w, t.tiles_x, t.tiles_y, t.patch_h, t.patch_w, packed ? row_chunks(g) : g.in_c / 16, t.pitch,
+               t.steps, t.weight_bytes, t.patch_bytes, magic16(t.pitch), magic16(t.patch_w), magic16(t.tile_w), magic16(packed ? row_chunks(g) : g.in_c / 16), magic16(g.kernel_w),
+               magic16(t.patch_w / 4), 0, 0, 0, 0, w, fill16};
   magic31(t.tiles_x, &c.magic_tiles_x, &c.shift_tiles_x);
   magic31(t.tiles_y, &c.magic_tiles_y, &c.shift_tiles_y);
   const size_t lds = (size_t)t.weight_bytes + t.patch_bytes + 8 * (size_t)t.steps;
   const dim3 grid((unsigned)t.tiles), threads(64 * kWaves);
-  if (g.out_c > 32) {
-    hipLaunchKernelGGL((conv_window_kernel<2>), grid, threads, lds, stream, c, rq, out);
-  } else {
-    hipLaunchKernelGGL((conv_window_kernel<1>), grid, threads, lds, stream, c, rq, out);
-  }
+  const bool relu = requant_form(rq) == kReluForm;
+  auto pick = [&](auto ocb, auto form) -> WindowKernel {
+    return packed ? conv_window_kernel<decltype(ocb)::value, true, decltype(form)::value>
+                  : conv_window_kernel<decltype(ocb)::value, false, decltype(form)::value>;
+  };
+  auto pick_form = [&](auto ocb) {
+    return relu ? pick(ocb, std::integral_constant<RequantForm, kReluForm>()) : pick(ocb, std::integral_constant<RequantForm, kCarryForm>());
+  };
+  const WindowKernel kernel = g.out_c > 32 ? pick_form(std::integral_constant<int, 2>()) : pick_form(std::integral_constant<int, 1>());
+  hipLaunchKernelGGL(kernel, grid, threads, lds, stream, c, rq, out);
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }

@@ -571,20 +571,25 @@ def test_matmul_rows_of_any_length(orc, m, n, k, dynamic, asymmetric):
             assert np.array_equal(got, want), (depth, shift)
 
 
-# one chunk per pixel and five, odd and even numbers of contraction steps and fewer than the late loads' ones; rectangles that the
-# image cuts off, channels that end inside a block; windows over every border, a stride and a dilation
+# one chunk per pixel and five, odd and even numbers of contraction steps and fewer than the late loads' ones; three and four
+# channels, one and two chunks per window row; rectangles that the image cuts off, channels that end inside a block and a quad;
+# windows over every border, a stride and a dilation; with and without an activation
 @pytest.mark.parametrize("ic,oc,kernel,stride,dilation,pad", [(64, 64, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)),
                                                               (48, 37, (3, 3), (1, 1), (1, 1), (0, 2, 1, 0)),
                                                               (16, 32, (3, 3), (1, 2), (1, 1), (1, 1, 1, 1)),
                                                               (16, 7, (1, 3), (1, 1), (1, 1), (0, 0, 1, 1)),
                                                               (32, 64, (5, 5), (1, 1), (1, 1), (2, 2, 2, 2)),
                                                               (80, 33, (2, 3), (1, 1), (2, 1), (2, 0, 3, 1)),
-                                                              (32, 20, (3, 3), (2, 2), (1, 3), (3, 1, 2, 4))])
-@pytest.mark.parametrize("batch,h,w", [(16, 61, 53), (5, 131, 90), (208, 11, 19), (3, 300, 67)])
-def test_window_convolution_rectangles(orc, ic, oc, kernel, stride, dilation, pad, batch, h, w):
+                                                              (32, 20, (3, 3), (2, 2), (1, 3), (3, 1, 2, 4)),
+                                                              (3, 64, (7, 7), (2, 2), (1, 1), (3, 3, 3, 3)),
+                                                              (3, 21, (9, 3), (1, 1), (1, 1), (4, 4, 1, 1)),
+                                                              (4, 42, (5, 8), (1, 2), (2, 1), (0, 4, 7, 2)),
+                                                              (4, 32, (10, 4), (2, 1), (1, 1), (0, 1, 5, 0))])
+@pytest.mark.parametrize("batch,h,w,act", [(16, 61, 53, 1), (5, 131, 90, 0), (208, 11, 19, 3), (3, 300, 67, 0), (171, 16, 16, 1)])
+def test_window_convolution_rectangles(orc, ic, oc, kernel, stride, dilation, pad, batch, h, w, act):
     import torch
     from tests.test_gpu_parity import _conv_case, _gpu_conv
     rng = np.random.default_rng(ic * oc + h)
     orc.set_threads(16)
-    case = _conv_case(rng, batch, h, w, ic, oc, kernel, stride, dilation, pad, True, False, True, 1)
+    case = _conv_case(rng, batch, h, w, ic, oc, kernel, stride, dilation, pad, True, False, True, act)
     assert np.array_equal(_gpu_conv(case, stride, dilation, pad, 1, device_tensors=True, exact_3x3=True), orc.conv_int8(**case))
