@@ -408,16 +408,13 @@ struct RowsStore {
     wait_for_products(acc);
     int8_t *tile_out = out + (int64_t)tile * 32 * g.out_c;
     // (no branch between the pieces of a whole tile: one's chain of dependent instructions fills the gaps of the next)
-    if (tile * 32 + 32 <= g.pixels && n0 + 32 * OCB <= g.out_c) {
+    requant.in_form(tile * 32 + 32 <= g.pixels, n0, g.out_c, [&](auto whole, auto streamed) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) requant.template store<true>(rq, acc, sums, q, tile_out + 8 * q * g.out_c + out_off, 0);
-      return;
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      // (the transposition needs every lane: those whose pixel is not there store none of their channels)
-      requant.template store<false>(rq, acc, sums, q, tile_out + 8 * q * g.out_c + out_off,
-                                    tile * 32 + 8 * q + my_p < g.pixels ? g.out_c - my_n : 0);
+      for (int q = 0; q < 4; ++q)
+        // (the transposition needs every lane: those whose pixel is not there store none of their channels)
+        requant.template store<decltype(whole)::value, decltype(streamed)::value>(
+            rq, acc, sums, q, tile_out + 8 * q * g.out_c + out_off, tile * 32 + 8 * q + my_p < g.pixels ? g.out_c - my_n : 0);
+    });
   }
 };
 

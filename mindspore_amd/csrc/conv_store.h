@@ -3,6 +3,8 @@
 // transposition across neighbouring lanes makes dwords of four channels for the stores.
 #pragma once
 
+#include <type_traits>
+
 #include "common.h"
 #include "quant_math.h"
 
@@ -41,9 +43,9 @@ inline RequantForm requant_form(const RequantParams &rq) {
   return rq.amin >= rq.zo ? kReluForm : kCarryForm;
 }
 
-// The channel of a group of 32 * OCB that column r of channel block ob computes: with two blocks a lane's two quads of channels
-// (after the transposition) are neighbours in memory.
-__host__ __device__ __forceinline__ int column_channel(int ocb, int ob, int r) { return ocb == 2 ? 8 * (r >> 2) + 4 * ob + (r & 3) : r; }
+// The channel of a group of 32 * OCB that column r of channel block ob computes: a lane's quads of channels (after the
+// transposition), one per block, are neighbours in memory.
+__host__ __device__ __forceinline__ int column_channel(int ocb, int ob, int r) { return 4 * ocb * (r >> 2) + 4 * ob + (r & 3); }
 
 // acc[ob][4 * q + e] is pixel 8 * q + 4 * h + e of 32, channel n0 + column_channel(OCB, ob, r); after the transposition a lane holds
 // the quad of channels from n0 + column_channel(OCB, ob, r & ~3) of pixel 8 * q + 4 * h + (lane & 3).
@@ -118,31 +120,71 @@ struct ChannelRequant {
     const uint32_t p23 = (uint16_t)__builtin_amdgcn_ashr_pk_i8_i32((uint32_t)t[2], (uint32_t)t[3], (uint32_t)shift[ob]);
     return quad_transpose(__builtin_amdgcn_perm(p23, p01, 0x05040100u), sel1, sel2);
   }
-  // Non-temporal: written out while the launch runs and not at its end.  us, temporal -> this: 32 x 224 x 224 x 3 -> 64, 7x7, stride 2
-  // 17.4 -> 16.5, eight of them 6.35 -> 5.8, 32 x 224 x 224 x 3 -> 32, 3x3, stride 2 9.55 -> 8.7.
   // quad q of each block, which is 4 * OCB neighbouring channels, to `to`; WHOLE: all exist, otherwise `have` of them do
-  template <bool WHOLE>
+  template <bool WHOLE, bool STREAMED>
   __device__ __forceinline__ void store(const RequantParams &rq, const v16i (&acc)[OCB], const v16i &sums, int q, int8_t *to,
                                         int have) const {
     typedef uint32_t u32_any __attribute__((aligned(1)));
     typedef uint32_t v2u __attribute__((ext_vector_type(2)));
     typedef v2u v2u_any __attribute__((aligned(1)));
+    typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+    typedef v4u v4u_any __attribute__((aligned(1)));
     uint32_t four[OCB];
 #pragma unroll
     for (int ob = 0; ob < OCB; ++ob) four[ob] = four_channels(rq, acc, sums, q, ob);
-    if (WHOLE && OCB == 2) {
-      __builtin_nontemporal_store((v2u{four[0], four[OCB - 1]}), reinterpret_cast<v2u_any *>(to));
-      return;
-    }
-#pragma unroll
-    for (int ob = 0; ob < OCB; ++ob) {
+    auto put = [&](auto *at, auto x) {
+      if (STREAMED) {
+        __builtin_nontemporal_store(x, at);
+      } else {
+        *at = x;
+      }
+    };
+    auto quad = [&](int ob) {
       if (WHOLE || have >= 4 * ob + 4) {
-        __builtin_nontemporal_store(four[ob], reinterpret_cast<u32_any *>(to + 4 * ob));
+        put(reinterpret_cast<u32_any *>(to + 4 * ob), four[ob]);
       } else {
 #pragma unroll
         for (int e = 0; e < 3; ++e)
           if (4 * ob + e < have) to[4 * ob + e] = (int8_t)(four[ob] >> (8 * e));
       }
+    };
+#pragma unroll
+    for (int ob = 0; ob < OCB;) {
+      if (ob + 4 <= OCB && WHOLE) {
+        put(reinterpret_cast<v4u_any *>(to + 4 * ob), v4u{four[ob], four[ob + 1], four[ob + 2], four[ob + 3]});
+        ob += 4;
+      } else if (ob + 2 <= OCB) {
+        if (WHOLE || have >= 4 * ob + 8) {
+          put(reinterpret_cast<v2u_any *>(to + 4 * ob), v2u{four[ob], four[ob + 1]});
+        } else {
+          quad(ob);
+          quad(ob + 1);
+        }
+        ob += 2;
+      } else {
+        quad(ob++);
+      }
+    }
+  }
+  // A store streams (non-temporal: written out while the launch runs and not at its end) if its launch's stores write whole lines
+  // together, that is if a workgroup has all channels of its pixels and, from three blocks, no piece of a lane is missing.  us,
+  // temporal -> streamed: 32 x 224 x 224 x 3 -> 64, 7x7, stride 2 17.4 -> 16.5, eight of them 6.35 -> 5.8; 32 x 224 x 224 x 3 -> 32, 3x3,
+  // stride 2 9.55 -> 8.7; 16 x 112 x 112, 32 -> 96 8.0 -> 6.2, -> 160 12.5 -> 10.8; but -> 192 in groups of 96 14.5 -> 24.4, and
+  // 32 x 56 x 56, 24 -> 144 in one of 160 14.0 -> 19.3.
+  // calls store(whole, streamed) with constants; whole: all pixels and channels of the tile exist
+  template <typename F>
+  static __device__ __forceinline__ void in_form(bool all_pixels, int n0, int out_c, F store) {
+    const bool whole = all_pixels && n0 + 32 * OCB <= out_c, streamed = n0 == 0 && (OCB <= 2 ? out_c <= 32 * OCB : out_c == 32 * OCB);
+    if (streamed) {
+      if (whole) {
+        store(std::true_type(), std::true_type());
+      } else {
+        store(std::false_type(), std::true_type());
+      }
+    } else if (whole) {
+      store(std::true_type(), std::false_type());
+    } else {
+      store(std::false_type(), std::false_type());
     }
   }
 };
@@ -151,8 +193,9 @@ struct ChannelRequant {
 // instruction is inline assembly, as above: 19 wait states after a 16-pass product.
 template <int OCB>
 __device__ __forceinline__ void wait_for_products(v16i (&acc)[OCB]) {
-  if constexpr (OCB == 1) asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc[0]));
-  if constexpr (OCB == 2) asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc[0]), "+v"(acc[1]));
+  asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc[0]));
+#pragma unroll
+  for (int ob = 1; ob < OCB; ++ob) asm volatile("" : "+v"(acc[ob]));
 }
 
 }  // namespace mi

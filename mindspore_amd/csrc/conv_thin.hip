@@ -4,15 +4,11 @@
 
 #include <type_traits>
 
-#include "common.h"
-#include "quant_math.h"
+#include "conv_store.h"
 
 namespace mi {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v16i __attribute__((ext_vector_type(16)));
 typedef v4i v4i_any __attribute__((aligned(1)));
-typedef uint32_t u32_any __attribute__((aligned(1)));
 
 // A workgroup holds the weights of OCB x 32 channels in LDS, in the order the MFMA operand takes them (1 KiB per 32 bytes
 // of K and 32 channels), and its four waves walk tiles of 32 pixels each by itself, without barriers: a lane's 16 bytes of
@@ -20,15 +16,12 @@ typedef uint32_t u32_any __attribute__((aligned(1)));
 // steps' loads in flight while this one's products run.  The GEMM's tiles stage both operands through LDS in barriered
 // steps, fetch nothing for the next tile before they have stored this one, and are 128 or 256 channels wide however few
 // there are; rows of any but a multiple of 16 bytes also had to be padded in a pass of their own.
-// The pixels are the MFMA's row operand: a lane ends up with one output channel of 16 pixels per block of 32 channels, with
-// its requantisation parameters in registers, and a 4 x 4 byte transposition across neighbouring lanes makes dwords of four
-// channels for the stores (as in conv_rows_kernel).
-// Bound by the vector ALU (the requantisation, 7 instructions per output byte) where there are more channels than bytes of
-// K, by memory where there are fewer.  us per launch, before -> now: 16 x 112 x 112, 192 -> 32 channels 45.2 -> 10.6,
-// 32 -> 192 21.0 -> 14.7; 8 x 115 x 115, 240 -> 40 26.5 -> 9.6; 4 x 80 x 80, 72 -> 24 9.0 (in two launches) -> 3.5; one
-// image of 112 x 112, where any launch takes most of it, 192 -> 32 3.7 -> 3.8.
-// Windows of several taps stay with the gathering GEMM: 32 x 56 x 56 x 64, 3x3, took 13.6 us in this form against 14.0, one
-// such image 6.2 against 5.1, stride 2 10.6 against 7.1.
+// The pixels are the MFMA's row operand, see conv_store.h.
+// Bound by the vector ALU (the requantisation, 4 instructions per output byte) and the stores where there are more channels than
+// bytes of K, by memory where there are fewer.  us per launch, GEMM -> with a clamp, shift and carry of its own for each output
+// and temporal stores of four bytes -> now: 16 x 112 x 112, 192 -> 32 channels 45.2 -> 10.7 -> 10.4, 32 -> 64 - -> 6.9 -> 5.2, 32 -> 128
+// - -> 11.2 -> 8.9, 32 -> 192 21.0 -> 16.2 -> 14.8; 32 x 112 x 112, 32 -> 16 - -> 7.2 -> 6.4; 8 x 115 x 115, 240 -> 40 26.5 -> 9.4 -> 9.5;
+// 4 x 80 x 80, 72 -> 24 9.0 (in two launches) -> 3.5; one image of 112 x 112, where any launch takes most of it, 192 -> 32 3.7 -> 3.8.
 struct ConvThin {
   const int8_t *in;
   int64_t in_bytes;
@@ -38,15 +31,7 @@ struct ConvThin {
   const int8_t *w;  // [32 channels][step][lane][16]
 };
 
-__device__ __forceinline__ uint32_t thin_quad_transpose(uint32_t d, uint32_t sel1, uint32_t sel2) {
-  const uint32_t p = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)d, 0xB1, 0xF, 0xF, false);  // lane ^ 1
-  const uint32_t r = __builtin_amdgcn_perm(p, d, sel1);
-  const uint32_t q = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)r, 0x4E, 0xF, 0xF, false);  // lane ^ 2
-  return __builtin_amdgcn_perm(q, r, sel2);
-}
-
-// FAST: the one-multiply rounding form without weight zero points (RequantParams::fast2, !has_zw).
-template <int CH, int OCB, bool FAST>
+template <int CH, int OCB, RequantForm FORM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void conv_thin_kernel(ConvThin g, RequantParams rq,
                                                                                               int8_t *__restrict__ out) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -56,27 +41,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
   int tile = blockIdx.x * 4 + (tid >> 6);
   const int steps = g.chunks * CH;
 
-  // this lane's channel of each block (the arrays are padded to a multiple of 256 channels)
-  int32_t mult[OCB], bias[OCB], shift[OCB], lsh[OCB], zw[OCB];
-  uint64_t c2[OCB];
-#pragma unroll
-  for (int ob = 0; ob < OCB; ++ob) {
-    const int n = n0 + ob * 32 + r;
-    shift[ob] = rq.rshift[n];
-    if (FAST) {
-      mult[ob] = (int32_t)rq.mult2[n];
-      c2[ob] = (uint64_t)rq.c2hi[n] << 32 | rq.c2lo[n];
-      bias[ob] = rq.pre[n];
-    } else {
-      mult[ob] = rq.mult[n];
-      bias[ob] = (int32_t)((uint32_t)rq.bias2[n] - kAccBias);
-      lsh[ob] = rq.lshift[n];
-      zw[ob] = rq.zw[n];
-    }
-  }
-  int amin_v = rq.amin, amax_v = rq.amax;
-  asm volatile("" : "+v"(amin_v), "+v"(amax_v));  // kept in vector registers, as v_med3 wants them
-  const uint32_t sel1 = (lane & 1) ? 0x03070105u : 0x06020400u, sel2 = (lane & 2) ? 0x03020706u : 0x05040100u;
+  const ChannelRequant<OCB, FORM> requant(rq, n0, lane);
 
   int64_t at = 0;  // this lane's first byte of a tile
   auto locate = [&](int tl) {
@@ -95,11 +60,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
   };
 
   {
-    const v4i *src = reinterpret_cast<const v4i *>(g.w + (int64_t)(n0 / 32) * steps * 1024);
-    const int have = min(OCB, (g.out_c - n0 + 31) / 32) * steps * 64;  // (the last group of blocks may reach past the weights)
+    // operand (block ob, step, lane) holds the weights of column_channel(OCB, ob, lane % 32), as far as there are channels
+    const v4i *src = reinterpret_cast<const v4i *>(g.w);
     v4i *dst = reinterpret_cast<v4i *>(lds);
+    const int blocks = (g.out_c + 31) / 32;
+#pragma unroll
+    for (int ob = 0; ob < OCB; ++ob) {
+      const int n = n0 + column_channel(OCB, ob, r), block = min(n >> 5, blocks - 1);
 #pragma unroll 4
-    for (int i = tid; i < have; i += 256) dst[i] = src[i];
+      for (int s = tid >> 6; s < steps; s += 4) dst[(ob * steps + s) * 64 + lane] = src[(block * steps + s) * 64 + (n & 31) + 32 * h];
+    }
     __syncthreads();
   }
   if (tile >= tiles) return;
@@ -141,7 +111,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
         for (int ob = 0; ob < OCB; ++ob)
           acc[ob] = __builtin_amdgcn_mfma_i32_32x32x32_i8(y[s], *reinterpret_cast<const v4i *>(wl + (ob * steps + s) * 1024),
                                                           decltype(first_c)::value && s == 0 ? start : acc[ob], 0, 0, 0);
-      if (!FAST && rq.has_zw) {  // the pixels' input sums, in the accumulators' layout: against ones up to K
+      if (FORM == kGeneralForm && rq.has_zw) {  // the pixels' input sums, in the accumulators' layout: against ones up to K
 #pragma unroll
         for (int s = 0; s < CH; ++s) {
           v4i one;
@@ -163,69 +133,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
       acc[0] = start;
       for (int c = 0; c < g.chunks; ++c) chunk(c, std::false_type());
     }
-    // (the wait states that a matrix product's result needs before inline assembly reads it, as in conv_rows_kernel)
-    if constexpr (OCB == 1) asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc[0]));
-    if constexpr (OCB == 2) asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc[0]), "+v"(acc[1]));
-    if constexpr (OCB == 3) asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]));
-    // acc[ob][4 * q + e] is pixel 8 * q + 4 * h + e of the tile, channel n0 + 32 * ob + r; after the transposition this
-    // lane holds channels r & ~3 .. + 3 of pixel 8 * q + 4 * h + (lane & 3)
-    const int first = tile * 32;
-    const bool whole = first + 32 <= g.pixels && n0 + 32 * OCB <= g.out_c;
-    const int my_n = n0 + (r & ~3), my_p = first + 4 * h + (lane & 3);
+    wait_for_products(acc);
+    const int first = tile * 32, my_n = n0 + column_channel(OCB, 0, r & ~3), my_p = first + 4 * h + (lane & 3);
     int8_t *dst = out + (int64_t)my_p * g.out_c + my_n;
-    auto store = [&](auto whole_c) {
+    requant.in_form(first + 32 <= g.pixels, n0, g.out_c, [&](auto whole, auto streamed) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-#pragma unroll
-      for (int ob = 0; ob < OCB; ++ob) {
-        int y[4];
-        if (FAST) {
-          uint64_t p2[4], carry[4], unused;
-          int32_t t[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            asm("v_mad_u64_u32 %0, %1, %2, %3, %4"
-                : "=&v"(p2[e]), "=s"(carry[e])
-                : "v"(acc[ob][4 * q + e]), "v"(mult[ob]), "v"(c2[ob]));
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            asm("v_addc_co_u32_e64 %0, %1, %2, %3, %4"
-                : "=v"(t[e]), "=s"(unused)
-                : "v"((int32_t)(p2[e] >> 32)), "v"(bias[ob]), "s"(carry[e]));
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            t[e] >>= shift[ob];
-            asm("v_med3_i32 %0, %1, %2, %3" : "=v"(y[e]) : "v"(t[e]), "v"(amin_v), "v"(amax_v));
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            uint32_t v = (uint32_t)acc[ob][4 * q + e] - (uint32_t)sums[4 * q + e] * (uint32_t)zw[ob] + (uint32_t)bias[ob];
-            int32_t t = rdiv_pot(srdhm((int32_t)(v << lsh[ob]), mult[ob]), shift[ob]);
-            t = (int32_t)((uint32_t)t + (uint32_t)rq.zo);
-            t = t < rq.amax ? t : rq.amax;
-            y[e] = t > rq.amin ? t : rq.amin;
-          }
-        }
-        const uint32_t p01 = __builtin_amdgcn_perm((uint32_t)y[1], (uint32_t)y[0], 0x0c0c0400u);
-        const uint32_t p23 = __builtin_amdgcn_perm((uint32_t)y[3], (uint32_t)y[2], 0x0c0c0400u);
-        const uint32_t four = thin_quad_transpose(__builtin_amdgcn_perm(p23, p01, 0x05040100u), sel1, sel2);
-        int8_t *to = dst + 8 * q * g.out_c + 32 * ob;
-        if (decltype(whole_c)::value || (my_p + 8 * q < g.pixels && my_n + 32 * ob + 4 <= g.out_c)) {
-          *reinterpret_cast<u32_any *>(to) = four;
-        } else if (my_p + 8 * q < g.pixels) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (my_n + 32 * ob + e < g.out_c) to[e] = (int8_t)(four >> (8 * e));
-        }
-      }
-    }
-    };
-    if (OCB > 1 && whole) {
-      store(std::true_type());
-    } else {
-      store(std::false_type());
-    }
+      for (int q = 0; q < 4; ++q)
+        requant.template store<decltype(whole)::value, decltype(streamed)::value>(rq, acc, sums, q, dst + 8 * q * g.out_c,
+                                                                                  my_p + 8 * q < g.pixels ? g.out_c - my_n : 0);
+    });
   }
 }
 
@@ -275,10 +191,13 @@ std::vector<int8_t> conv_thin_weights(const int8_t *w, int oc, int k) {
 
 template <int CH, int OCB>
 static int launch_thin(const ConvThin &c, const RequantParams &rq, int8_t *out, dim3 grid, size_t lds, hipStream_t stream) {
-  if (rq.fast2 != 0 && rq.has_zw == 0) {
-    hipLaunchKernelGGL((conv_thin_kernel<CH, OCB, true>), grid, dim3(256), lds, stream, c, rq, out);
-  } else {
-    hipLaunchKernelGGL((conv_thin_kernel<CH, OCB, false>), grid, dim3(256), lds, stream, c, rq, out);
+  const RequantForm form = requant_form(rq);
+  if (form == kReluForm) {
+    hipLaunchKernelGGL((conv_thin_kernel<CH, OCB, kReluForm>), grid, dim3(256), lds, stream, c, rq, out);
+  } else if (form == kCarryForm) {
+    hipLaunchKernelGGL((conv_thin_kernel<CH, OCB, kCarryForm>), grid, dim3(256), lds, stream, c, rq, out);
+  } else if constexpr (OCB <= 3) {
+    hipLaunchKernelGGL((conv_thin_kernel<CH, OCB, kGeneralForm>), grid, dim3(256), lds, stream, c, rq, out);
   }
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
@@ -293,7 +212,12 @@ int launch_conv_thin(const int8_t *in, int64_t pixels, int k, int oc, const int8
   const ThinCut t = thin_cut(k);
   const ConvThin c{in, pixels * k, k, t.chunks, oc, (int)pixels, w};
   const int64_t wgs = (pixels + 127) / 128;
-  const int ocb = thin_blocks(wgs, oc), groups = (oc + 32 * ocb - 1) / (32 * ocb);
+  const RequantForm form = requant_form(rq);
+  const int blocks = (oc + 31) / 32;
+  // Four or five whole blocks in one workgroup, whose stores then stream.  us, two groups -> this: 16 x 112 x 112, 32 -> 128 11.2 -> 8.9,
+  // -> 160 15.3 -> 10.9; 16 x 56 x 56, 128 -> 128 6.0 -> 5.6.  Six (too few waves) 14.7 -> 22, channels short of five 10.4 -> 14.
+  const bool rows = form != kGeneralForm && oc == 32 * blocks && blocks > 3 && blocks <= 5 && wgs * blocks > 1024 && t.steps() * blocks <= 64;
+  const int ocb = rows ? blocks : thin_blocks(wgs, oc), groups = (oc + 32 * ocb - 1) / (32 * ocb);
   // four workgroups per CU, which the LDS allows up to 40 KiB of weights; more would only load the weights more often
   const int most = (1024 + groups - 1) / groups;
   const dim3 grid((unsigned)(wgs < most ? wgs : most), (unsigned)groups);
@@ -301,7 +225,9 @@ int launch_conv_thin(const int8_t *in, int64_t pixels, int k, int oc, const int8
 #define MI_THIN(CH)                                                              \
   return ocb == 1   ? launch_thin<CH, 1>(c, rq, out, grid, lds, stream)          \
          : ocb == 2 ? launch_thin<CH, 2>(c, rq, out, grid, lds, stream)          \
-                    : launch_thin<CH, 3>(c, rq, out, grid, lds, stream)
+         : ocb == 3 ? launch_thin<CH, 3>(c, rq, out, grid, lds, stream)          \
+         : ocb == 4 ? launch_thin<CH, 4>(c, rq, out, grid, lds, stream)          \
+                    : launch_thin<CH, 5>(c, rq, out, grid, lds, stream)
   switch (t.ch) {
     case 1: MI_THIN(1);
     case 2: MI_THIN(2);

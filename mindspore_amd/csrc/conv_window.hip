@@ -198,20 +198,15 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWa
   int ty = quotient16(first, g.magic_tile_w), tx = first - ty * g.tile_w;
   uint32_t at = (uint32_t)(ty * g.out_w + tx) * g.out_c;
   wait_for_products(acc);
-  auto store = [&](auto whole_c) {
+  requant.in_form(true, 0, g.out_c, [&](auto whole, auto streamed) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const uint32_t to = (ty < have_h && tx < have_w ? at : 0u) + my_n;
-      requant.template store<decltype(whole_c)::value>(rq, acc, start, q, rectangle + to, g.out_c - my_n);
+      requant.template store<decltype(whole)::value, decltype(streamed)::value>(rq, acc, start, q, rectangle + to, g.out_c - my_n);
       tx += 8, at += 8 * g.out_c;  // (a rectangle is at least that wide)
       if (tx >= g.tile_w) tx -= g.tile_w, ++ty, at += (g.out_w - g.tile_w) * g.out_c;
     }
-  };
-  if (32 * OCB <= g.out_c) {
-    store(std::true_type());
-  } else {
-    store(std::false_type());
-  }
+  });
 }
 
 // ---- host side -----------------------------------------------------------------------------------------------------

@@ -593,3 +593,15 @@ def test_window_convolution_rectangles(orc, ic, oc, kernel, stride, dilation, pa
     orc.set_threads(16)
     case = _conv_case(rng, batch, h, w, ic, oc, kernel, stride, dilation, pad, True, False, True, act)
     assert np.array_equal(_gpu_conv(case, stride, dilation, pad, 1, device_tensors=True, exact_3x3=True), orc.conv_int8(**case))
+
+
+# two to five blocks of channels in a workgroup, whole and not, one group and two, K of one step to several and no multiple of them
+@pytest.mark.parametrize("ic,oc,act", [(16, 64, 0), (40, 40, 1), (24, 96, 0), (32, 112, 1), (32, 128, 0), (33, 128, 1), (200, 128, 3),
+                                       (24, 160, 1), (77, 160, 0), (16, 192, 1)])
+def test_thin_convolution_channel_blocks(orc, ic, oc, act):
+    import torch
+    from tests.test_gpu_parity import _conv_case, _gpu_conv
+    rng = np.random.default_rng(ic * oc)
+    orc.set_threads(16)
+    case = _conv_case(rng, 3, 113, 141, ic, oc, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, False, True, act)
+    assert np.array_equal(_gpu_conv(case, (1, 1), (1, 1), (0, 0, 0, 0), 1, device_tensors=True), orc.conv_int8(**case))
