@@ -1201,8 +1201,8 @@ int mi_conv_run(mi_conv *h, const int8_t *in_dev, int32_t batch, int32_t in_h, i
     if (h->dw_rows_par.p != nullptr && conv_dw_rows_supported(g) &&
         ((reinterpret_cast<uintptr_t>(in_dev) | reinterpret_cast<uintptr_t>(out_dev)) & 3) == 0)
       return launch_conv_dw_rows(in_dev, g, static_cast<const int32_t *>(h->dw_rows.p),
-                                 static_cast<const int32_t *>(h->dw_rows_par.p), (int)(int8_t)d.in_zp, h->st.amin, h->st.amax,
-                                 out_dev, s);
+                                 static_cast<const int32_t *>(h->dw_rows_par.p), (int)(int8_t)d.in_zp, h->st.zo, h->st.amin,
+                                 h->st.amax, out_dev, s);
     RequantParams rq = h->st.params();
     rq.fast = h->dw_fast ? 1 : 0;
     return launch_conv_dw(in_dev, g, static_cast<const int16_t *>(h->w16.p), static_cast<const int32_t *>(h->dw_bias.p),

@@ -187,7 +187,7 @@ int launch_conv_dw(const int8_t *in, const ConvGeom &g, const int16_t *w16, cons
 // (RequantParams::fast2) with the bias of bias_folded.
 bool conv_dw_rows_supported(const ConvGeom &g);
 std::vector<int32_t> conv_dw_rows_weights(const int8_t *w, int ch, int ks);
-int launch_conv_dw_rows(const int8_t *in, const ConvGeom &g, const int32_t *w, const int32_t *par, int zx8, int amin, int amax,
+int launch_conv_dw_rows(const int8_t *in, const ConvGeom &g, const int32_t *w, const int32_t *par, int zx8, int zo, int amin, int amax,
                         int8_t *out, hipStream_t stream);
 
 // Host tensors of one call, in and out of device memory on the null stream (host_copy.hip).  `dev` holds a multiple of 16 bytes.

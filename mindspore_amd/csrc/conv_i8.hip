@@ -566,8 +566,9 @@ int launch_conv_rows(const int8_t *in, const ConvGeom &g, int fill, const int8_t
 // belongs to.  Accumulators start from kAccBias and are requantised with one 64-bit multiply-add (RequantParams::fast2).
 // Bound by the vector ALU at large sizes (3x3: about 10 instructions per output, half of them the requantisation; one
 // multiply per product and an unpacking instruction for each operand took about 30), by latency at one image.  us per launch,
-// before (conv_dw16_kernel below) -> now: 3x3, 16 x 112 x 112 x 192 70.1 -> 22.1 (3.5 TB/s), one such image 8.6 -> 4.8; 5x5,
-// 4 x 80 x 80 x 72 16.4 -> 6.0, 1 x 64 x 64 x 64 7.1 -> 4.1.
+// conv_dw16_kernel below -> one form of requantisation and store -> now: 3x3, 16 x 112 x 112 x 192 70.1 -> 23.4 -> 21.9 (3.5 TB/s), on 128
+// channels - -> 16.2 -> 14.1, 8 x 115 x 115 x 240 - -> 16.1 -> 14.6, 32 x 56 x 56 x 144 - -> 11.5 -> 10.3, one image of 112 x 112 x 192
+// 8.6 -> 4.3 -> 4.2; 5x5, 4 x 80 x 80 x 72 16.4 -> 6.0, 1 x 64 x 64 x 64 7.1 -> 4.1.
 struct ConvDwRows {
   const int8_t *in;
   const int32_t *w;    // [KS * (KS == 3 ? 1 : 3)][C]: bytes w0..w2 0 of a window row; 5x5: w0..w3, w4 0 0 0, w3 w4 0 0
@@ -579,7 +580,14 @@ struct ConvDwRows {
   int zsplat, amin, amax;
 };
 
-template <int KS, int OT>
+// From this many channels the stores are non-temporal (STREAMED), written out while the launch runs and not at its end: a pixel's
+// channels are then at least a line.  us, temporal -> streamed: 16 x 112 x 112 on 128 channels 15.9 -> 14.3, 32 x 56 x 56 on 144
+// 11.4 -> 11.1, 8 x 115 x 115 on 240 15.9 -> 15.5; 8 x 80 x 80 on 72, 5x5 6.9 -> 7.4.
+constexpr int kDwStreamedLeast = 128;
+
+// RELU: no output is below the zero point.  The rounding's sign term is then a constant (as in kReluForm of conv_store.h).  us:
+// 16 x 112 x 112 on 128 channels 15.9 -> 15.1, 32 x 56 x 56 on 144 11.4 -> 10.5, 8 x 80 x 80 on 72, 5x5 6.95 -> 6.75.
+template <int KS, int OT, bool RELU, bool STREAMED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void conv_dw_rows_kernel(ConvDwRows g) {
   constexpr int PX = KS + 3;       // input pixels per row of four outputs
   constexpr int WR = KS == 3 ? 1 : 3;  // weight dwords per channel and window row
@@ -639,6 +647,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
   v4i par[5];
 #pragma unroll
   for (int a = 0; a < 5; ++a) par[a] = *reinterpret_cast<const v4i *>(g.par + (int64_t)a * g.ch + c0);
+  if (RELU) par[2] = par[2] + par[3] + 1;  // see kReluForm
 
 #pragma unroll
   for (int i = 0; i < OT + KS - 1; ++i) {
@@ -690,18 +699,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
       int y[4];
-      uint64_t p2[4], carry[4], unused;
       int32_t t[4];
+      if (RELU) {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const uint64_t c2 = (uint64_t)(uint32_t)par[2][c] << 32 | (uint32_t)par[1][c];
-        asm("v_mad_u64_u32 %0, %1, %2, %3, %4" : "=&v"(p2[c]), "=s"(carry[c]) : "v"(acc[o][x][c]), "v"(par[0][c]), "v"(c2));
+        for (int c = 0; c < 4; ++c) {
+          const uint64_t c2 = (uint64_t)(uint32_t)par[2][c] << 32 | (uint32_t)par[1][c];
+          t[c] = (int32_t)(((uint64_t)(uint32_t)acc[o][x][c] * (uint32_t)par[0][c] + c2) >> 32);
+        }
+      } else {
+        uint64_t p2[4], carry[4], unused;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const uint64_t c2 = (uint64_t)(uint32_t)par[2][c] << 32 | (uint32_t)par[1][c];
+          asm("v_mad_u64_u32 %0, %1, %2, %3, %4" : "=&v"(p2[c]), "=s"(carry[c]) : "v"(acc[o][x][c]), "v"(par[0][c]), "v"(c2));
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          asm("v_addc_co_u32_e64 %0, %1, %2, %3, %4"
+              : "=v"(t[c]), "=s"(unused)
+              : "v"((int32_t)(p2[c] >> 32)), "v"(par[3][c]), "s"(carry[c]));
       }
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-        asm("v_addc_co_u32_e64 %0, %1, %2, %3, %4"
-            : "=v"(t[c]), "=s"(unused)
-            : "v"((int32_t)(p2[c] >> 32)), "v"(par[3][c]), "s"(carry[c]));
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         t[c] >>= par[4][c];
@@ -709,8 +726,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
       }
       const uint32_t p01 = __builtin_amdgcn_perm((uint32_t)y[1], (uint32_t)y[0], 0x0c0c0400u);
       const uint32_t p23 = __builtin_amdgcn_perm((uint32_t)y[3], (uint32_t)y[2], 0x0c0c0400u);
-      if (oh0 + o < g.out_h && ow0 + x < g.out_w)
-        *reinterpret_cast<uint32_t *>(dst + ((int64_t)o * g.out_w + x) * g.ch) = __builtin_amdgcn_perm(p23, p01, 0x05040100u);
+      if (oh0 + o < g.out_h && ow0 + x < g.out_w) {
+        const uint32_t four = __builtin_amdgcn_perm(p23, p01, 0x05040100u);
+        uint32_t *to = reinterpret_cast<uint32_t *>(dst + ((int64_t)o * g.out_w + x) * g.ch);
+        if (STREAMED) {
+          __builtin_nontemporal_store(four, to);
+        } else {
+          *to = four;
+        }
+      }
     }
 }
 
@@ -737,16 +761,19 @@ std::vector<int32_t> conv_dw_rows_weights(const int8_t *w, int ch, int ks) {
 }
 
 template <int KS, int OT>
-static int launch_dw_rows(ConvDwRows c, int batch, hipStream_t stream) {
+static int launch_dw_rows(ConvDwRows c, int batch, int zo, hipStream_t stream) {
   c.bands = (c.out_h + OT - 1) / OT;
   c.total = batch * c.bands * c.strips * c.groups;
-  hipLaunchKernelGGL((conv_dw_rows_kernel<KS, OT>), dim3((c.total + 255) / 256), dim3(256), 0, stream, c);
+  const bool streamed = c.ch >= kDwStreamedLeast;
+  const auto kernel = c.amin >= zo ? (streamed ? conv_dw_rows_kernel<KS, OT, true, true> : conv_dw_rows_kernel<KS, OT, true, false>)
+                                   : (streamed ? conv_dw_rows_kernel<KS, OT, false, true> : conv_dw_rows_kernel<KS, OT, false, false>);
+  hipLaunchKernelGGL(kernel, dim3((c.total + 255) / 256), dim3(256), 0, stream, c);
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }
 
-int launch_conv_dw_rows(const int8_t *in, const ConvGeom &g, const int32_t *w, const int32_t *par, int zx8, int amin, int amax,
-                        int8_t *out, hipStream_t stream) {
+int launch_conv_dw_rows(const int8_t *in, const ConvGeom &g, const int32_t *w, const int32_t *par, int zx8, int zo, int amin,
+                        int amax, int8_t *out, hipStream_t stream) {
   if (!conv_dw_rows_supported(g) || ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 3) != 0) {
     set_error("conv_dw_rows: unsupported geometry");
     return MI_PARAM_INVALID;
@@ -758,12 +785,12 @@ int launch_conv_dw_rows(const int8_t *in, const ConvGeom &g, const int32_t *w, c
   // 23.8; 5x5, 1 x 64 x 64 x 64 4.1, 4.9, 6.4; 4 x 80 x 80 x 72 6.4, 6.0, 7.6.
   const int64_t flat = (int64_t)g.batch * g.out_h * c.strips * c.groups;  // threads at one row each
   if (g.kernel_h == 3) {
-    if (flat >= 1 << 20) return launch_dw_rows<3, 4>(c, g.batch, stream);
-    if (flat >= 1 << 18) return launch_dw_rows<3, 2>(c, g.batch, stream);
-    return launch_dw_rows<3, 1>(c, g.batch, stream);
+    if (flat >= 1 << 20) return launch_dw_rows<3, 4>(c, g.batch, zo, stream);
+    if (flat >= 1 << 18) return launch_dw_rows<3, 2>(c, g.batch, zo, stream);
+    return launch_dw_rows<3, 1>(c, g.batch, zo, stream);
   }
-  if (flat >= 1 << 16) return launch_dw_rows<5, 2>(c, g.batch, stream);
-  return launch_dw_rows<5, 1>(c, g.batch, stream);
+  if (flat >= 1 << 16) return launch_dw_rows<5, 2>(c, g.batch, zo, stream);
+  return launch_dw_rows<5, 1>(c, g.batch, zo, stream);
 }
 
 __global__ __launch_bounds__(256) void conv_dw_kernel(const int8_t *__restrict__ in, ConvGeom g,

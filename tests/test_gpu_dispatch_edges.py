@@ -605,3 +605,17 @@ def test_thin_convolution_channel_blocks(orc, ic, oc, act):
     orc.set_threads(16)
     case = _conv_case(rng, 3, 113, 141, ic, oc, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, False, True, act)
     assert np.array_equal(_gpu_conv(case, (1, 1), (1, 1), (0, 0, 0, 0), 1, device_tensors=True), orc.conv_int8(**case))
+
+
+# with and without an activation, channels below and from where the stores are non-temporal, tiles of one to four rows
+@pytest.mark.parametrize("ch", [4, 124, 128, 132])
+@pytest.mark.parametrize("b,ih,iw", [(1, 9, 11), (3, 50, 63), (6, 77, 81)])
+@pytest.mark.parametrize("taps,act", [(3, 0), (3, 1), (5, 3), (5, 0)])
+def test_depthwise_stride_one_activations(orc, b, ih, iw, ch, taps, act):
+    import torch
+    from tests.test_gpu_parity import _conv_case, _gpu_conv
+    rng = np.random.default_rng(ch * taps + act)
+    orc.set_threads(16)
+    pad = (taps // 2,) * 4
+    case = _conv_case(rng, b, ih, iw, ch, ch, (taps, taps), (1, 1), (1, 1), pad, True, False, True, act, dw=True)
+    assert np.array_equal(_gpu_conv(case, (1, 1), (1, 1), pad, ch, device_tensors=True), orc.conv_dw_int8(**case))
