@@ -286,7 +286,7 @@ int launch_conv_smallk(const int8_t *in, const ConvGeom &g, int fill, int k_true
 // ones by the latency of one tile.  The order of tiles over the XCDs and the number of waves change nothing; windows of many
 // loads go through LDS (conv_window.hip).  us per launch with masks and branches in every tile and divisions by the vector
 // ALU (461 instructions) / plain tiles (230) / with the requantisation and stores of conv_store.h: 32 x 224 x 224 x 3 -> 64, 7x7,
-// stride 2 25.4 / 22.6 / 20.5; 32 x 224 x 224 x 3 -> 32, 3x3, stride 2 10.6 / - / 7.7; 16 of those 6.5 / 5.65 / 5.2;
+// stride 2 25.4 / 22.6 / 20.5; 32 x 224 x 224 x 3 -> 32, 3x3, stride 2 10.3 / - / 8.7; 16 of those 6.5 / 5.65 / 5.5;
 // 16 x 160 x 160 x 3 -> 64, 3x3 14.7 / 12.4 / 10.9; 16 x 224 x 224 x 4 -> 32, 5x5 20 / 16.4 / 14.8.
 struct ConvRows {
   const int8_t *in;
@@ -297,6 +297,7 @@ struct ConvRows {
   int row_bytes;  // kernel_w * in_c
   int fill;
   int pixels;
+  bool streams;
   const int8_t *w;  // [out_c padded to 64][32 * KS]
   uint32_t magic_hw, magic_w;  // quotients by out_hw and out_w: umulhi(2 p, magic) >> shift (see magic31)
   int shift_hw, shift_w;
@@ -408,7 +409,7 @@ struct RowsStore {
     wait_for_products(acc);
     int8_t *tile_out = out + (int64_t)tile * 32 * g.out_c;
     // (no branch between the pieces of a whole tile: one's chain of dependent instructions fills the gaps of the next)
-    requant.in_form(tile * 32 + 32 <= g.pixels, n0, g.out_c, [&](auto whole, auto streamed) {
+    requant.in_form(tile * 32 + 32 <= g.pixels, n0, g.out_c, g.streams, [&](auto whole, auto streamed) {
 #pragma unroll
       for (int q = 0; q < 4; ++q)
         // (the transposition needs every lane: those whose pixel is not there store none of their channels)
@@ -520,6 +521,7 @@ int launch_conv_rows(const int8_t *in, const ConvGeom &g, int fill, const int8_t
   }
   const int64_t wgs = (pixels + 127) / 128;
   const bool two = g.out_c > 32;
+  c.streams = conv_streams(pixels, g.out_c, two ? 2 : 1);
   const RequantForm form = requant_form(rq);
   const int gy = (g.out_c + (two ? 63 : 31)) / (two ? 64 : 32);
   // as many workgroups as the registers let the device hold, so that a wave walks several tiles on one set of weights.  us at
@@ -580,9 +582,9 @@ struct ConvDwRows {
   int zsplat, amin, amax;
 };
 
-// From this many channels the stores are non-temporal (STREAMED), written out while the launch runs and not at its end: a pixel's
-// channels are then at least a line.  us, temporal -> streamed: 16 x 112 x 112 on 128 channels 15.9 -> 14.3, 32 x 56 x 56 on 144
-// 11.4 -> 11.1, 8 x 115 x 115 on 240 15.9 -> 15.5; 8 x 80 x 80 on 72, 5x5 6.9 -> 7.4.
+// Outputs of up to kStreamedMost bytes are stored non-temporally (STREAMED) from this many channels, where a pixel's are at least a
+// line.  us, temporal -> streamed: 16 x 112 x 112 on 128 channels 15.9 -> 14.3, 32 x 56 x 56 on 144 11.4 -> 11.1, 8 x 80 x 80 on 72, 5x5
+// 6.9 -> 7.4; 32 x 112 x 112 on 192 (77 MB) 43.8 -> 45.7.
 constexpr int kDwStreamedLeast = 128;
 
 // RELU: no output is below the zero point.  The rounding's sign term is then a constant (as in kReluForm of conv_store.h).  us:
@@ -764,7 +766,7 @@ template <int KS, int OT>
 static int launch_dw_rows(ConvDwRows c, int batch, int zo, hipStream_t stream) {
   c.bands = (c.out_h + OT - 1) / OT;
   c.total = batch * c.bands * c.strips * c.groups;
-  const bool streamed = c.ch >= kDwStreamedLeast;
+  const bool streamed = c.ch >= kDwStreamedLeast && (int64_t)batch * c.out_h * c.out_w * c.ch <= kStreamedMost;
   const auto kernel = c.amin >= zo ? (streamed ? conv_dw_rows_kernel<KS, OT, true, true> : conv_dw_rows_kernel<KS, OT, true, false>)
                                    : (streamed ? conv_dw_rows_kernel<KS, OT, false, true> : conv_dw_rows_kernel<KS, OT, false, false>);
   hipLaunchKernelGGL(kernel, dim3((c.total + 255) / 256), dim3(256), 0, stream, c);

@@ -32,6 +32,18 @@ __device__ __forceinline__ uint32_t quad_transpose(uint32_t d, uint32_t sel1, ui
   return __builtin_amdgcn_perm(q, r, sel2);
 }
 
+// Stores that stream are non-temporal: written out while the launch runs and not by the write-back of the L2s at its end.  For
+// outputs that the L2s (32 MB) would still hold then: of larger ones most is out by that time, and a streamed one is not in the
+// last-level cache for the launch that reads it.  And where a workgroup has all channels of its pixels, two whole blocks of them
+// or more, so that its stores write whole lines.  us, temporal -> streamed: 32 x 224 x 224 x 3 -> 64, 7x7, stride 2 (26 MB) 17.4 -> 16.5,
+// eight of them 6.35 -> 5.8; 16 x 112 x 112, 32 -> 96 8.0 -> 6.2, -> 160 12.5 -> 10.8; but -> 192 in groups of 96 14.5 -> 24.4.  Chains of
+// stem, 1x1, depthwise and 1x1: on 112 x 112, 32 -> 128 -> 32 channels, 8 images 35.0 -> 31.5; 32 -> 192 -> 32, 32 images, all streamed
+// 83 -> 94, those on 32 channels only 83 -> 91.
+constexpr int64_t kStreamedMost = (int64_t)32 << 20;
+inline bool conv_streams(int64_t pixels, int out_c, int blocks) {
+  return blocks >= 2 && out_c == 32 * blocks && pixels * out_c <= kStreamedMost;
+}
+
 // How the convolutions requantise, see requant_form.
 enum RequantForm { kGeneralForm, kCarryForm, kReluForm };
 
@@ -166,25 +178,15 @@ struct ChannelRequant {
       }
     }
   }
-  // A store streams (non-temporal: written out while the launch runs and not at its end) if its launch's stores write whole lines
-  // together, that is if a workgroup has all channels of its pixels and, from three blocks, no piece of a lane is missing.  us,
-  // temporal -> streamed: 32 x 224 x 224 x 3 -> 64, 7x7, stride 2 17.4 -> 16.5, eight of them 6.35 -> 5.8; 32 x 224 x 224 x 3 -> 32, 3x3,
-  // stride 2 9.55 -> 8.7; 16 x 112 x 112, 32 -> 96 8.0 -> 6.2, -> 160 12.5 -> 10.8; but -> 192 in groups of 96 14.5 -> 24.4, and
-  // 32 x 56 x 56, 24 -> 144 in one of 160 14.0 -> 19.3.
   // calls store(whole, streamed) with constants; whole: all pixels and channels of the tile exist
   template <typename F>
-  static __device__ __forceinline__ void in_form(bool all_pixels, int n0, int out_c, F store) {
-    const bool whole = all_pixels && n0 + 32 * OCB <= out_c, streamed = n0 == 0 && (OCB <= 2 ? out_c <= 32 * OCB : out_c == 32 * OCB);
-    if (streamed) {
-      if (whole) {
-        store(std::true_type(), std::true_type());
-      } else {
-        store(std::false_type(), std::true_type());
-      }
-    } else if (whole) {
-      store(std::true_type(), std::false_type());
-    } else {
+  static __device__ __forceinline__ void in_form(bool all_pixels, int n0, int out_c, bool streams, F store) {
+    if (!all_pixels || n0 + 32 * OCB > out_c) {
       store(std::false_type(), std::false_type());
+    } else if (streams) {
+      store(std::true_type(), std::true_type());
+    } else {
+      store(std::true_type(), std::false_type());
     }
   }
 };

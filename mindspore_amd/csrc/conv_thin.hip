@@ -19,8 +19,8 @@ typedef v4i v4i_any __attribute__((aligned(1)));
 // The pixels are the MFMA's row operand, see conv_store.h.
 // Bound by the vector ALU (the requantisation, 4 instructions per output byte) and the stores where there are more channels than
 // bytes of K, by memory where there are fewer.  us per launch, GEMM -> with a clamp, shift and carry of its own for each output
-// and temporal stores of four bytes -> now: 16 x 112 x 112, 192 -> 32 channels 45.2 -> 10.7 -> 10.4, 32 -> 64 - -> 6.9 -> 5.2, 32 -> 128
-// - -> 11.2 -> 8.9, 32 -> 192 21.0 -> 16.2 -> 14.8; 32 x 112 x 112, 32 -> 16 - -> 7.2 -> 6.4; 8 x 115 x 115, 240 -> 40 26.5 -> 9.4 -> 9.5;
+// and temporal stores of four bytes -> now: 16 x 112 x 112, 192 -> 32 channels 45.2 -> 10.7 -> 10.4, 32 -> 64 - -> 7.0 -> 5.7, 32 -> 128
+// - -> 11.2 -> 9.2, 32 -> 192 21.0 -> 16.2 -> 14.8; 8 x 115 x 115, 240 -> 40 26.5 -> 9.4 -> 9.7;
 // 4 x 80 x 80, 72 -> 24 9.0 (in two launches) -> 3.5; one image of 112 x 112, where any launch takes most of it, 192 -> 32 3.7 -> 3.8.
 struct ConvThin {
   const int8_t *in;
@@ -28,6 +28,7 @@ struct ConvThin {
   int k;       // contraction bytes
   int chunks;  // of CH steps; weights are zero from k on
   int out_c, pixels;
+  bool streams;
   const int8_t *w;  // [32 channels][step][lane][16]
 };
 
@@ -136,7 +137,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
     wait_for_products(acc);
     const int first = tile * 32, my_n = n0 + column_channel(OCB, 0, r & ~3), my_p = first + 4 * h + (lane & 3);
     int8_t *dst = out + (int64_t)my_p * g.out_c + my_n;
-    requant.in_form(first + 32 <= g.pixels, n0, g.out_c, [&](auto whole, auto streamed) {
+    requant.in_form(first + 32 <= g.pixels, n0, g.out_c, g.streams, [&](auto whole, auto streamed) {
 #pragma unroll
       for (int q = 0; q < 4; ++q)
         requant.template store<decltype(whole)::value, decltype(streamed)::value>(rq, acc, sums, q, dst + 8 * q * g.out_c,
@@ -210,7 +211,6 @@ int launch_conv_thin(const int8_t *in, int64_t pixels, int k, int oc, const int8
     return MI_PARAM_INVALID;
   }
   const ThinCut t = thin_cut(k);
-  const ConvThin c{in, pixels * k, k, t.chunks, oc, (int)pixels, w};
   const int64_t wgs = (pixels + 127) / 128;
   const RequantForm form = requant_form(rq);
   const int blocks = (oc + 31) / 32;
@@ -218,6 +218,7 @@ int launch_conv_thin(const int8_t *in, int64_t pixels, int k, int oc, const int8
   // -> 160 15.3 -> 10.9; 16 x 56 x 56, 128 -> 128 6.0 -> 5.6.  Six (too few waves) 14.7 -> 22, channels short of five 10.4 -> 14.
   const bool rows = form != kGeneralForm && oc == 32 * blocks && blocks > 3 && blocks <= 5 && wgs * blocks > 1024 && t.steps() * blocks <= 64;
   const int ocb = rows ? blocks : thin_blocks(wgs, oc), groups = (oc + 32 * ocb - 1) / (32 * ocb);
+  const ConvThin c{in, pixels * k, k, t.chunks, oc, (int)pixels, conv_streams(pixels, oc, ocb), w};
   // four workgroups per CU, which the LDS allows up to 40 KiB of weights; more would only load the weights more often
   const int most = (1024 + groups - 1) / groups;
   const dim3 grid((unsigned)(wgs < most ? wgs : most), (unsigned)groups);

@@ -25,7 +25,7 @@ namespace mi {
 // PACKED: the first layer's three or four channels, four bytes a pixel in LDS.  A window row is one or two chunks of four pixels
 // (zero weights behind its last tap and in a fourth byte that is no channel), read at any pixel.  conv_rows_kernel takes such
 // rows straight from the image in unaligned 16-byte loads, about 95 cycles of the address unit each; here a pixel's bytes are
-// loaded once, four pixels a lane.  32 x 224 x 224 x 3 -> 64, 7x7, stride 2: 20.5 us -> 16.5, of which launch and prologue 5.9,
+// loaded once, four pixels a lane.  32 x 224 x 224 x 3 -> 64, 7x7, stride 2: 20.5 us -> 14.5 to 16.5, of which launch and prologue 5.9,
 // the pixels 2, products 3, stores about 5 (26 MB); vector instructions are 255 a wave.
 struct ConvWindow {
   const int8_t *in;
@@ -37,6 +37,7 @@ struct ConvWindow {
   int cc, pitch;                         // chunks per pixel, and from one pixel to the next in LDS
   int steps;                             // of 32 bytes of K
   int weight_bytes, patch_bytes;         // in LDS, multiples of 1 KiB
+  bool streams;
   uint32_t magic_pitch, magic_patch_w, magic_tile_w, magic_cc, magic_kernel_w, magic_quads;  // ceil(2^32 / d): exact quotients for dividends < 2^16 (d >= 2; 0: d = 1)
   uint32_t magic_tiles_x, magic_tiles_y;  // see magic31
   int shift_tiles_x, shift_tiles_y;
@@ -198,7 +199,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWa
   int ty = quotient16(first, g.magic_tile_w), tx = first - ty * g.tile_w;
   uint32_t at = (uint32_t)(ty * g.out_w + tx) * g.out_c;
   wait_for_products(acc);
-  requant.in_form(true, 0, g.out_c, [&](auto whole, auto streamed) {
+  requant.in_form(true, 0, g.out_c, g.streams, [&](auto whole, auto streamed) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const uint32_t to = (ty < have_h && tx < have_w ? at : 0u) + my_n;
@@ -308,9 +309,10 @@ int launch_conv_window(const int8_t *in, const ConvGeom &g, const int8_t *fill16
   *taken = requant_form(rq) != kGeneralForm && choose_window(g, in, &t);
   if (!*taken) return MI_OK;
   const bool packed = packed_window(g);
+  const bool streams = conv_streams((int64_t)g.batch * g.out_h * g.out_w, g.out_c, g.out_c > 32 ? 2 : 1);
   ConvWindow c{in, in + (int64_t)g.batch * g.in_h * g.in_w * g.in_c - 4, g.in_h, g.in_w, g.in_c, g.out_h, g.out_w, g.out_c, g.kernel_h, g.kernel_w, g.stride_h, g.stride_w, g.dilation_h,
                g.dilation_w, g.pad_u, g.pad_l, t.tile_h, t.tile_w, t.tiles_x, t.tiles_y, t.patch_h, t.patch_w, packed ? row_chunks(g) : g.in_c / 16, t.pitch,
-               t.steps, t.weight_bytes, t.patch_bytes, magic16(t.pitch), magic16(t.patch_w), magic16(t.tile_w), magic16(packed ? row_chunks(g) : g.in_c / 16), magic16(g.kernel_w),
+               t.steps, t.weight_bytes, t.patch_bytes, streams, magic16(t.pitch), magic16(t.patch_w), magic16(t.tile_w), magic16(packed ? row_chunks(g) : g.in_c / 16), magic16(g.kernel_w),
                magic16(t.patch_w / 4), 0, 0, 0, 0, w, fill16};
   magic31(t.tiles_x, &c.magic_tiles_x, &c.shift_tiles_x);
   magic31(t.tiles_y, &c.magic_tiles_y, &c.shift_tiles_y);
