@@ -296,10 +296,20 @@ static bool choose_window(const ConvGeom &g, const void *in, WindowCut *c) {
 }
 
 typedef void (*WindowKernel)(ConvWindow, RequantParams, int8_t *);
-int conv_window_prepare_device() {  // (more than 64 KiB of dynamic LDS)
-  for (const WindowKernel kernel : {conv_window_kernel<1, false, kCarryForm>, conv_window_kernel<2, false, kCarryForm>,
-                                    conv_window_kernel<1, false, kReluForm>, conv_window_kernel<2, false, kReluForm>})
-    MI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kWindowLds));
+// [blocks of 32 channels - 1][packed][kReluForm]
+static const WindowKernel kWindowKernels[2][2][2] = {
+    {{conv_window_kernel<1, false, kCarryForm>, conv_window_kernel<1, false, kReluForm>},
+     {conv_window_kernel<1, true, kCarryForm>, conv_window_kernel<1, true, kReluForm>}},
+    {{conv_window_kernel<2, false, kCarryForm>, conv_window_kernel<2, false, kReluForm>},
+     {conv_window_kernel<2, true, kCarryForm>, conv_window_kernel<2, true, kReluForm>}}};
+
+// Dynamic LDS beyond 64 KiB has to be announced: cut_window gives all of them up to kWindowLds (packed, 8x8 windows at stride 8
+// take 77 KiB).
+int conv_window_prepare_device() {
+  for (const auto &of_blocks : kWindowKernels)
+    for (const auto &of_packed : of_blocks)
+      for (const WindowKernel kernel : of_packed)
+        MI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kWindowLds));
   return MI_OK;
 }
 
@@ -318,15 +328,7 @@ int launch_conv_window(const int8_t *in, const ConvGeom &g, const int8_t *fill16
   magic31(t.tiles_y, &c.magic_tiles_y, &c.shift_tiles_y);
   const size_t lds = (size_t)t.weight_bytes + t.patch_bytes + 8 * (size_t)t.steps;
   const dim3 grid((unsigned)t.tiles), threads(64 * kWaves);
-  const bool relu = requant_form(rq) == kReluForm;
-  auto pick = [&](auto ocb, auto form) -> WindowKernel {
-    return packed ? conv_window_kernel<decltype(ocb)::value, true, decltype(form)::value>
-                  : conv_window_kernel<decltype(ocb)::value, false, decltype(form)::value>;
-  };
-  auto pick_form = [&](auto ocb) {
-    return relu ? pick(ocb, std::integral_constant<RequantForm, kReluForm>()) : pick(ocb, std::integral_constant<RequantForm, kCarryForm>());
-  };
-  const WindowKernel kernel = g.out_c > 32 ? pick_form(std::integral_constant<int, 2>()) : pick_form(std::integral_constant<int, 1>());
+  const WindowKernel kernel = kWindowKernels[g.out_c > 32][packed][requant_form(rq) == kReluForm];
   hipLaunchKernelGGL(kernel, grid, threads, lds, stream, c, rq, out);
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;

@@ -595,6 +595,20 @@ def test_window_convolution_rectangles(orc, ic, oc, kernel, stride, dilation, pa
     assert np.array_equal(_gpu_conv(case, stride, dilation, pad, 1, device_tensors=True, exact_3x3=True), orc.conv_int8(**case))
 
 
+# rectangles of 77, 78 and 70 KiB of LDS, on three and four channels
+@pytest.mark.parametrize("ic,kernel,stride,batch,size", [(3, (8, 8), (8, 8), 11, 512), (3, (7, 7), (8, 8), 11, 512),
+                                                         (4, (16, 8), (5, 5), 5, 512)])
+@pytest.mark.parametrize("act", [0, 1])
+def test_window_convolution_most_of_the_lds(orc, ic, kernel, stride, batch, size, act):
+    import torch
+    from tests.test_gpu_parity import _conv_case, _gpu_conv
+    rng = np.random.default_rng(ic + size)
+    orc.set_threads(16)
+    pad = (0, 0, 0, 0)
+    case = _conv_case(rng, batch, size, size, ic, 64, kernel, stride, (1, 1), pad, True, False, True, act)
+    assert np.array_equal(_gpu_conv(case, stride, (1, 1), pad, 1, device_tensors=True), orc.conv_int8(**case))
+
+
 # two to five blocks of channels in a workgroup, whole and not, one group and two, K of one step to several and no multiple of them
 @pytest.mark.parametrize("ic,oc,act", [(16, 64, 0), (40, 40, 1), (24, 96, 0), (32, 112, 1), (32, 128, 0), (33, 128, 1), (200, 128, 3),
                                        (24, 160, 1), (77, 160, 0), (16, 192, 1)])
