@@ -409,11 +409,11 @@ struct RowsStore {
     wait_for_products(acc);
     int8_t *tile_out = out + (int64_t)tile * 32 * g.out_c;
     // (no branch between the pieces of a whole tile: one's chain of dependent instructions fills the gaps of the next)
-    requant.in_form(tile * 32 + 32 <= g.pixels, n0, g.out_c, g.streams, [&](auto whole, auto streamed) {
+    requant.in_form(tile * 32 + 32 <= g.pixels, n0, my_n, g.out_c, g.streams, [&](auto kind, auto streamed) {
 #pragma unroll
       for (int q = 0; q < 4; ++q)
         // (the transposition needs every lane: those whose pixel is not there store none of their channels)
-        requant.template store<decltype(whole)::value, decltype(streamed)::value>(
+        requant.template store<decltype(kind)::value, decltype(streamed)::value>(
             rq, acc, sums, q, tile_out + 8 * q * g.out_c + out_off, tile * 32 + 8 * q + my_p < g.pixels ? g.out_c - my_n : 0);
     });
   }

@@ -137,10 +137,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
     wait_for_products(acc);
     const int first = tile * 32, my_n = n0 + column_channel(OCB, 0, r & ~3), my_p = first + 4 * h + (lane & 3);
     int8_t *dst = out + (int64_t)my_p * g.out_c + my_n;
-    requant.in_form(first + 32 <= g.pixels, n0, g.out_c, g.streams, [&](auto whole, auto streamed) {
+    requant.in_form(first + 32 <= g.pixels, n0, my_n, g.out_c, g.streams, [&](auto kind, auto streamed) {
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        requant.template store<decltype(whole)::value, decltype(streamed)::value>(rq, acc, sums, q, dst + 8 * q * g.out_c,
+        requant.template store<decltype(kind)::value, decltype(streamed)::value>(rq, acc, sums, q, dst + 8 * q * g.out_c,
                                                                                   my_p + 8 * q < g.pixels ? g.out_c - my_n : 0);
     });
   }

@@ -199,11 +199,11 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWa
   int ty = quotient16(first, g.magic_tile_w), tx = first - ty * g.tile_w;
   uint32_t at = (uint32_t)(ty * g.out_w + tx) * g.out_c;
   wait_for_products(acc);
-  requant.in_form(true, 0, g.out_c, g.streams, [&](auto whole, auto streamed) {
+  requant.in_form(true, 0, my_n, g.out_c, g.streams, [&](auto kind, auto streamed) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const uint32_t to = (ty < have_h && tx < have_w ? at : 0u) + my_n;
-      requant.template store<decltype(whole)::value, decltype(streamed)::value>(rq, acc, start, q, rectangle + to, g.out_c - my_n);
+      requant.template store<decltype(kind)::value, decltype(streamed)::value>(rq, acc, start, q, rectangle + to, g.out_c - my_n);
       tx += 8, at += 8 * g.out_c;  // (a rectangle is at least that wide)
       if (tx >= g.tile_w) tx -= g.tile_w, ++ty, at += (g.out_w - g.tile_w) * g.out_c;
     }

@@ -621,6 +621,21 @@ def test_thin_convolution_channel_blocks(orc, ic, oc, act):
     assert np.array_equal(_gpu_conv(case, (1, 1), (1, 1), (0, 0, 0, 0), 1, device_tensors=True), orc.conv_int8(**case))
 
 
+# channels of which every lane has all of its quads or none, some of them, and part of one; one group and several; whole tiles of
+# pixels and a last one; the three kernels that store them (1x1, first layer, window)
+@pytest.mark.parametrize("oc", [4, 24, 36, 40, 44, 60, 64, 72, 74, 80, 144, 176, 240])
+@pytest.mark.parametrize("ic,kernel,batch,size", [(24, (1, 1), 3, 113), (3, (3, 3), 3, 113), (16, (3, 3), 5, 97)])
+def test_convolution_stores_of_partial_blocks(orc, ic, kernel, batch, size, oc):
+    import torch
+    from tests.test_gpu_parity import _conv_case, _gpu_conv
+    rng = np.random.default_rng(ic * oc)
+    orc.set_threads(16)
+    pad = (kernel[0] // 2,) * 4
+    for act in (0, 1):
+        case = _conv_case(rng, batch, size, size + 2, ic, oc, kernel, (1, 1), (1, 1), pad, True, False, True, act)
+        assert np.array_equal(_gpu_conv(case, (1, 1), (1, 1), pad, 1, device_tensors=True, exact_3x3=True), orc.conv_int8(**case))
+
+
 # with and without an activation, channels below and from where the stores are non-temporal, tiles of one to four rows
 @pytest.mark.parametrize("ch", [4, 124, 128, 132])
 @pytest.mark.parametrize("b,ih,iw", [(1, 9, 11), (3, 50, 63), (6, 77, 81)])
