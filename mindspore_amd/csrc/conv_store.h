@@ -44,6 +44,21 @@ inline bool conv_streams(int64_t pixels, int out_c, int blocks) {
   return blocks >= 2 && out_c == 32 * blocks && pixels * out_c <= kStreamedMost;
 }
 
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+
+// One store of x at any address, non-temporal or not.  (The alignment belongs to the type that is stored through: as an argument's
+// type it would be lost.)
+template <bool STREAMED, typename T>
+__device__ __forceinline__ void store_any(int8_t *to, T x) {
+  typedef T any __attribute__((aligned(1)));
+  if (STREAMED) {
+    __builtin_nontemporal_store(x, reinterpret_cast<any *>(to));
+  } else {
+    *reinterpret_cast<any *>(to) = x;
+  }
+}
+
 // What of a lane's 4 * OCB channels exists: all of them, whole quads, anything.
 enum StoreForm { kWhole, kQuads, kBytes };
 
@@ -139,24 +154,12 @@ struct ChannelRequant {
   template <StoreForm KIND, bool STREAMED>
   __device__ __forceinline__ void store(const RequantParams &rq, const v16i (&acc)[OCB], const v16i &sums, int q, int8_t *to,
                                         int have) const {
-    typedef uint32_t u32_any __attribute__((aligned(1)));
-    typedef uint32_t v2u __attribute__((ext_vector_type(2)));
-    typedef v2u v2u_any __attribute__((aligned(1)));
-    typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-    typedef v4u v4u_any __attribute__((aligned(1)));
     uint32_t four[OCB];
 #pragma unroll
     for (int ob = 0; ob < OCB; ++ob) four[ob] = four_channels(rq, acc, sums, q, ob);
-    auto put = [&](auto *at, auto x) {
-      if (STREAMED) {
-        __builtin_nontemporal_store(x, at);
-      } else {
-        *at = x;
-      }
-    };
     auto quad = [&](int ob) {
       if (KIND == kWhole || have >= 4 * ob + 4) {
-        put(reinterpret_cast<u32_any *>(to + 4 * ob), four[ob]);
+        store_any<STREAMED>(to + 4 * ob, four[ob]);
       } else if (KIND == kBytes) {
 #pragma unroll
         for (int e = 0; e < 3; ++e)
@@ -166,11 +169,11 @@ struct ChannelRequant {
 #pragma unroll
     for (int ob = 0; ob < OCB;) {
       if (ob + 4 <= OCB && KIND == kWhole) {
-        put(reinterpret_cast<v4u_any *>(to + 4 * ob), v4u{four[ob], four[ob + 1], four[ob + 2], four[ob + 3]});
+        store_any<STREAMED>(to + 4 * ob, v4u{four[ob], four[ob + 1], four[ob + 2], four[ob + 3]});
         ob += 4;
       } else if (ob + 2 <= OCB) {
         if (KIND == kWhole || have >= 4 * ob + 8) {
-          put(reinterpret_cast<v2u_any *>(to + 4 * ob), v2u{four[ob], four[ob + 1]});
+          store_any<STREAMED>(to + 4 * ob, v2u{four[ob], four[ob + 1]});
         } else {
           quad(ob);
           quad(ob + 1);

@@ -50,7 +50,6 @@ __device__ __forceinline__ int quotient16(int p, uint32_t magic) { return magic 
 constexpr int kWaves = 8;
 typedef uint32_t u32_any __attribute__((aligned(1)));
 typedef v4i v4i_4 __attribute__((aligned(4)));
-typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 typedef v4u v4u_any __attribute__((aligned(1)));
 
 template <int OCB, bool PACKED, RequantForm FORM>
