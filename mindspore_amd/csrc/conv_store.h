@@ -73,15 +73,17 @@ inline RequantForm requant_form(const RequantParams &rq) {
   return rq.amin >= rq.zo ? kReluForm : kCarryForm;
 }
 
-// The channel of a group of 32 * OCB that column r of channel block ob computes: a lane's quads of channels (after the
-// transposition), one per block, are neighbours in memory.
-__host__ __device__ __forceinline__ int column_channel(int ocb, int ob, int r) { return 4 * ocb * (r >> 2) + 4 * ob + (r & 3); }
+// The channel of a group of 32 * OCB that column r of channel block ob computes: either a lane's quads of channels (after the
+// transposition), one per block, are neighbours in memory, or the blocks are, each with stores of its own.
+__host__ __device__ __forceinline__ int column_channel(int ocb, int ob, int r, bool neighbours = true) {
+  return neighbours ? 4 * ocb * (r >> 2) + 4 * ob + (r & 3) : 32 * ob + r;
+}
 
-// acc[ob][4 * q + e] is pixel 8 * q + 4 * h + e of 32, channel n0 + column_channel(OCB, ob, r); after the transposition a lane holds
-// the quad of channels from n0 + column_channel(OCB, ob, r & ~3) of pixel 8 * q + 4 * h + (lane & 3).
+// acc[ob][4 * q + e] is pixel 8 * q + 4 * h + e of 32, channel n0 + column_channel(OCB, ob, r, NEIGHBOURS); after the transposition a lane holds
+// the quad of channels from n0 + column_channel(OCB, ob, r & ~3, NEIGHBOURS) of pixel 8 * q + 4 * h + (lane & 3).
 // Vector instructions per quad: 23 with a shift and a clamp of its own for each output and a carry, 19 in kCarryForm and 15 in
 // kReluForm, whose clamps come before the shift that saturates and packs.
-template <int OCB, RequantForm FORM>
+template <int OCB, RequantForm FORM, bool NEIGHBOURS = true>
 struct ChannelRequant {
   int32_t mult[OCB], bias[OCB], shift[OCB], lsh[OCB], zw[OCB];  // of this lane's channel of each block
   int32_t least[OCB], most[OCB];  // the output range before the shift
@@ -91,7 +93,7 @@ struct ChannelRequant {
   __device__ __forceinline__ ChannelRequant(const RequantParams &rq, int n0, int lane) {
 #pragma unroll
     for (int ob = 0; ob < OCB; ++ob) {
-      const int n = n0 + column_channel(OCB, ob, lane & 31);  // (the arrays are padded to a multiple of 256 channels)
+      const int n = n0 + column_channel(OCB, ob, lane & 31, NEIGHBOURS);  // (the arrays are padded to a multiple of 256 channels)
       shift[ob] = rq.rshift[n];
       if (FORM == kGeneralForm) {
         mult[ob] = rq.mult[n];
@@ -157,6 +159,12 @@ struct ChannelRequant {
     uint32_t four[OCB];
 #pragma unroll
     for (int ob = 0; ob < OCB; ++ob) four[ob] = four_channels(rq, acc, sums, q, ob);
+    if constexpr (!NEIGHBOURS) {  // (whole blocks only)
+#pragma unroll
+      for (int ob = 0; ob < OCB; ++ob)
+        if (KIND == kWhole || have > 0) store_any<STREAMED>(to + 32 * ob, four[ob]);
+      return;
+    }
     auto quad = [&](int ob) {
       if (KIND == kWhole || have >= 4 * ob + 4) {
         store_any<STREAMED>(to + 4 * ob, four[ob]);

@@ -611,7 +611,7 @@ def test_window_convolution_most_of_the_lds(orc, ic, kernel, stride, batch, size
 
 # two to five blocks of channels in a workgroup, whole and not, one group and two, K of one step to several and no multiple of them
 @pytest.mark.parametrize("ic,oc,act", [(16, 64, 0), (40, 40, 1), (24, 96, 0), (32, 112, 1), (32, 128, 0), (33, 128, 1), (200, 128, 3),
-                                       (24, 160, 1), (77, 160, 0), (16, 192, 1)])
+                                       (24, 160, 1), (77, 160, 0), (16, 192, 1), (64, 256, 1), (40, 256, 0), (128, 256, 3)])
 def test_thin_convolution_channel_blocks(orc, ic, oc, act):
     import torch
     from tests.test_gpu_parity import _conv_case, _gpu_conv
