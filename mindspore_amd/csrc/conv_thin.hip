@@ -61,15 +61,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
   };
 
   {
-    // operand (block ob, step, lane) holds the weights of column ob, lane % 32, as far as there are channels
-    const v4i *src = reinterpret_cast<const v4i *>(g.w);
+    // From [32 channels][step][lane], front to back, into operand order [ob][step][lane], where the channels of a group are columns
+    // of its blocks (ChannelRequant).  Fetched in operand order instead, 3 x 206 x 206, 376 -> 152 channels took 32.0 us, this 29.9;
+    // 34 x 26 x 26, 336 -> 192 9.5 / 8.8.
+    const int left = (g.out_c - n0 + 31) / 32, have = (left < OCB ? left : OCB) * steps;
+    const v4i *src = reinterpret_cast<const v4i *>(g.w) + (int64_t)(n0 / 32) * steps * 64;
     v4i *dst = reinterpret_cast<v4i *>(lds);
-    const int blocks = (g.out_c + 31) / 32;
-#pragma unroll
-    for (int ob = 0; ob < OCB; ++ob) {
-      const int n = n0 + column_channel(OCB, ob, r, NEIGHBOURS), block = min(n >> 5, blocks - 1);
 #pragma unroll 4
-      for (int s = tid >> 6; s < steps; s += 4) dst[(ob * steps + s) * 64 + lane] = src[(block * steps + s) * 64 + (n & 31) + 32 * h];
+    for (int i = __builtin_amdgcn_readfirstlane(tid >> 6); i < have; i += 4) {
+      const int b = i / steps, s = i - b * steps, n = 32 * b + r;
+      const int ob = NEIGHBOURS ? (n >> 2) % OCB : b, column = NEIGHBOURS ? 4 * (n / (4 * OCB)) + (n & 3) : r;
+      dst[(ob * steps + s) * 64 + column + 32 * h] = src[i * 64 + lane];
     }
     __syncthreads();
   }
