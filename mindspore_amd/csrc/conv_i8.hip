@@ -583,8 +583,10 @@ struct ConvDwRows {
 };
 
 // Outputs of up to kStreamedMost bytes are stored non-temporally (STREAMED) from this many channels, where a pixel's are at least a
-// line.  us, temporal -> streamed: 16 x 112 x 112 on 128 channels 15.9 -> 14.3, 32 x 56 x 56 on 144 11.4 -> 11.1, 8 x 80 x 80 on 72, 5x5
-// 6.9 -> 7.4; 32 x 112 x 112 on 192 (77 MB) 43.8 -> 45.7.
+// line; half as many bytes where pixels begin inside a line's 32-byte sectors, which two stores then share.  us, temporal -> streamed:
+// 16 x 112 x 112 on 128 channels 15.9 -> 14.3, 32 x 56 x 56 on 144 11.4 -> 11.1, 8 x 80 x 80 on 72, 5x5 6.9 -> 7.4; 32 x 112 x 112 on 192
+// (77 MB) 43.8 -> 45.7; 12 x 112 x 112 on 128 (19 MB) 11.9 -> 10.5, on 160 13.6 -> 12.9, on 140 13.4 -> 14.1; 16 x 57 x 57 (7 MB) on 140 even,
+// on 200 8.9 -> 8.4.
 constexpr int kDwStreamedLeast = 128;
 
 // RELU: no output is below the zero point.  The rounding's sign term is then a constant (as in kReluForm of conv_store.h).  us:
@@ -766,7 +768,8 @@ template <int KS, int OT>
 static int launch_dw_rows(ConvDwRows c, int batch, int zo, hipStream_t stream) {
   c.bands = (c.out_h + OT - 1) / OT;
   c.total = batch * c.bands * c.strips * c.groups;
-  const bool streamed = c.ch >= kDwStreamedLeast && (int64_t)batch * c.out_h * c.out_w * c.ch <= kStreamedMost;
+  const bool streamed = c.ch >= kDwStreamedLeast &&
+                        (int64_t)batch * c.out_h * c.out_w * c.ch <= (c.ch % 32 == 0 ? kStreamedMost : kStreamedMost / 2);
   const auto kernel = c.amin >= zo ? (streamed ? conv_dw_rows_kernel<KS, OT, true, true> : conv_dw_rows_kernel<KS, OT, true, false>)
                                    : (streamed ? conv_dw_rows_kernel<KS, OT, false, true> : conv_dw_rows_kernel<KS, OT, false, false>);
   hipLaunchKernelGGL(kernel, dim3((c.total + 255) / 256), dim3(256), 0, stream, c);
