@@ -476,6 +476,13 @@ static int prepare_rows(const int8_t *a, int rows, int k, const Workspace &ws, h
   return MI_OK;
 }
 
+// A group whose members run one by one on rows that are no whole chunks: whether all of them run on one padded copy, or those that
+// would read the rows as they are by themselves do so here too.  us, int8 out / fp32 out, one copy -> none: pairs, 200 rows,
+// 390 x 1000 10.8 -> 9.0 / 11.2 -> 10.0, 770 x 1000 11.1 -> 11.55 / 12.0 -> 12.7, 1000 x 1000 11.5 -> 10.5 / 12.3 -> 11.3; three of
+// 390 x 768 14.1 -> 13.1 / 15.1 -> 14.7, 770 x 768 15.1 -> 17.1 / 16.2 -> 18.8, 1000 x 768 15.6 -> 15.4 / 16.7 -> 16.5; four of
+// 1000 x 500 20.1 -> 20.8 / 21.9 -> 22.3.
+static bool shares_padded_copy(int count) { return count > 2; }
+
 // (the blocked copy may be absent: two rows then take the v_dot4 kernel)
 static WeightView weight_view(const RequantState &st) {
   return WeightView{static_cast<const int8_t *>(st.w.p), st.k_pad, st.ldw, static_cast<const int8_t *>(st.w_blocked.p)};
@@ -496,11 +503,15 @@ static int run_requant_gemm(RequantState &st, const int8_t *a, int64_t lda, int 
   return launch_gemm_requant(a, lda, rows, k16, w, st.n, rq, c, st.n, stream);
 }
 
+// whether the caller's rows are to be read as they are, without a padded copy
+static bool runs_on_anyrow(const RequantState &st, const int8_t *a_dev, int rows) {
+  return !whole_chunks(a_dev, st.k) && !runs_on_gemv(st, rows, round_up(st.k, 16)) && gemm_anyrow_takes(rows, st.k, weight_view(st), st.n);
+}
+
 // The same for the caller's rows, whatever their length and address.
 static int run_requant_rows(RequantState &st, const int8_t *a_dev, int rows, const Workspace &ws, int8_t *c, hipStream_t stream) {
-  const WeightView w = weight_view(st);
-  if (!whole_chunks(a_dev, st.k) && !runs_on_gemv(st, rows, round_up(st.k, 16)) && gemm_anyrow_takes(rows, st.k, w, st.n))
-    return launch_gemm_anyrow_requant(a_dev, rows, st.k, w, st.n, st.params(), c, stream);
+  if (runs_on_anyrow(st, a_dev, rows))
+    return launch_gemm_anyrow_requant(a_dev, rows, st.k, weight_view(st), st.n, st.params(), c, stream);
   const int8_t *a = nullptr;
   int64_t lda = 0;
   int k16 = 0;
@@ -893,12 +904,14 @@ int mi_matmul_run_group(mi_matmul *const *handles, int32_t count, const int8_t *
   int rc = ensure_device();
   if (rc != MI_OK) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  const int k = handles[0]->st.k;
   const int8_t *a = nullptr;
   int64_t lda = 0;
-  int k16 = 0;
-  // the activation rows are brought into the kernels' form once, for all members
-  if ((rc = prepare_rows(a_dev, rows, handles[0]->st.k, Workspace::growable(&handles[0]->a_ws), s, &a, &lda, &k16)) != MI_OK)
-    return rc;
+  int k16 = round_up(k, 16);
+  // the activation rows are brought into the kernels' form once, for all members that need it
+  auto prepare = [&] {
+    return a != nullptr ? MI_OK : prepare_rows(a_dev, rows, k, Workspace::growable(&handles[0]->a_ws), s, &a, &lda, &k16);
+  };
   // up to four members go out as one launch if they are decode-sized, or if the GEMM expects to gain by it; anything else runs
   // member by member
   const bool few = count >= 2 && count <= 4;
@@ -913,19 +926,27 @@ int mi_matmul_run_group(mi_matmul *const *handles, int32_t count, const int8_t *
     RequantParams rq[4];
     int n[4];
     for (int i = 0; i < count; ++i) {
-      const RequantState &st = handles[i]->st;
-      wv[i] = WeightView{static_cast<const int8_t *>(st.w.p), st.k_pad, st.ldw, static_cast<const int8_t *>(st.w_blocked.p)};
-      rq[i] = st.params();
-      n[i] = st.n;
+      wv[i] = weight_view(handles[i]->st);
+      rq[i] = handles[i]->st.params();
+      n[i] = handles[i]->st.n;
     }
-    if (decode) return launch_gemv_group(a, lda, rows, k16, count, wv, n, rq, c_dev, s);
-    bool taken = false;
-    rc = launch_gemm_group_requant(a, lda, rows, k16, count, wv, n, rq, c_dev, s, &taken);
-    if (rc != MI_OK || taken) return rc;
+    const TileCost *tile = decode ? nullptr : gemm_group_tile(k16, rows, k16, count, wv, n, rq);
+    if (decode || tile != nullptr) {
+      if ((rc = prepare()) != MI_OK) return rc;
+      if (decode) return launch_gemv_group(a, lda, rows, k16, count, wv, n, rq, c_dev, s);
+      return launch_gemm_group_requant(*tile, a, lda, rows, k16, count, wv, n, rq, c_dev, s);
+    }
   }
-  for (int i = 0; i < count; ++i)
-    if ((rc = run_requant_gemm(handles[i]->st, a, lda, rows, k16, c_dev[i], s)) != MI_OK)
-      return rc;
+  const bool copy = shares_padded_copy(count);
+  for (int i = 0; i < count; ++i) {
+    RequantState &st = handles[i]->st;
+    if (!copy && runs_on_anyrow(st, a_dev, rows)) {
+      rc = launch_gemm_anyrow_requant(a_dev, rows, k, weight_view(st), st.n, st.params(), c_dev[i], s);
+    } else if ((rc = prepare()) == MI_OK) {
+      rc = run_requant_gemm(st, a, lda, rows, k16, c_dev[i], s);
+    }
+    if (rc != MI_OK) return rc;
+  }
   return MI_OK;
 }
 
@@ -1522,6 +1543,28 @@ static DequantParams dequant_params(const mi_dynmm *h, float sx, int32_t zx, con
   return dq;
 }
 
+static WeightView weight_view(const mi_dynmm *h) {
+  return WeightView{static_cast<const int8_t *>(h->w.p), h->k_pad, h->ldw, static_cast<const int8_t *>(h->w_blocked.p)};
+}
+
+// decode-sized runs: the matrix-core decode kernel streams the blocked weights once (any N, any output alignment)
+// (one row runs on the row-major weights and needs no blocked copy, as long as the row fits the kernel's LDS form)
+static bool runs_on_gemv(const mi_dynmm *h, int rows) {
+  return gemv_takes_rows(rows, h->n) && (rows > kGemvDotRows || (int64_t)rows * round_up(h->k, 16) <= 150 * 1024) &&
+         (rows == 1 || (h->w_blocked.p != nullptr && h->k_pad <= 1 << 20));
+}
+
+static bool runs_on_anyrow(const mi_dynmm *h, const int8_t *a_dev, int rows) {
+  return !runs_on_gemv(h, rows) && !whole_chunks(a_dev, h->k) && gemm_anyrow_takes(rows, h->k, weight_view(h), h->n);
+}
+
+static int run_dequant_gemm(const mi_dynmm *h, const int8_t *a, int64_t lda, int rows, int k16, const DequantParams &dq, float *c_dev,
+                            hipStream_t s) {
+  const WeightView w = weight_view(h);
+  if (runs_on_gemv(h, rows)) return launch_gemv_dequant(a, lda, rows, k16, w, h->n, dq, c_dev, h->n, s);
+  return launch_gemm_dequant(a, lda, rows, k16, w, h->n, dq, c_dev, h->n, s);
+}
+
 static int dynmm_run_impl(mi_dynmm *h, const int8_t *a_dev, int32_t rows, float sx, int32_t zx,
                           const mi_dq_params *qp_dev, float *c_dev, hipStream_t s, bool per_row = false) {
   if (h == nullptr || a_dev == nullptr || c_dev == nullptr) {
@@ -1533,20 +1576,13 @@ static int dynmm_run_impl(mi_dynmm *h, const int8_t *a_dev, int32_t rows, float 
   int rc = ensure_device();
   if (rc != MI_OK) return rc;
   const DequantParams dq = dequant_params(h, sx, zx, qp_dev, per_row);
-  const WeightView w{static_cast<const int8_t *>(h->w.p), h->k_pad, h->ldw,
-                     static_cast<const int8_t *>(h->w_blocked.p)};
-  // decode-sized runs: the matrix-core decode kernel streams the blocked weights once (any N, any output alignment)
-  // (one row runs on the row-major weights and needs no blocked copy, as long as the row fits the kernel's LDS form)
-  const bool on_gemv = gemv_takes_rows(rows, h->n) && (rows > kGemvDotRows || (int64_t)rows * round_up(h->k, 16) <= 150 * 1024) &&
-                       (rows == 1 || (w.blocked != nullptr && h->k_pad <= 1 << 20));
-  if (!on_gemv && !whole_chunks(a_dev, h->k) && gemm_anyrow_takes(rows, h->k, w, h->n))
-    return launch_gemm_anyrow_dequant(a_dev, rows, h->k, w, h->n, dq, c_dev, s);
+  if (runs_on_anyrow(h, a_dev, rows))
+    return launch_gemm_anyrow_dequant(a_dev, rows, h->k, weight_view(h), h->n, dq, c_dev, s);
   const int8_t *a = nullptr;
   int64_t lda = 0;
   int k16 = 0;
   if ((rc = prepare_rows(a_dev, rows, h->k, Workspace::growable(&h->a_ws), s, &a, &lda, &k16)) != MI_OK) return rc;
-  if (on_gemv) return launch_gemv_dequant(a, lda, rows, k16, w, h->n, dq, c_dev, h->n, s);
-  return launch_gemm_dequant(a, lda, rows, k16, w, h->n, dq, c_dev, h->n, s);
+  return run_dequant_gemm(h, a, lda, rows, k16, dq, c_dev, s);
 }
 
 int mi_dynmm_reserve(mi_dynmm *h, int32_t max_rows) {
@@ -1605,13 +1641,14 @@ int mi_dynmm_run_group(mi_dynmm *const *handles, int32_t count, const int8_t *a_
   int rc = ensure_device();
   if (rc != MI_OK) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  const int k = handles[0]->k;
   const int8_t *a = nullptr;
   int64_t lda = 0;
-  int k16 = 0;
-  // the activation rows are brought into the kernels' form once, for all members
-  if ((rc = prepare_rows(a_dev, rows, handles[0]->k, Workspace::growable(&handles[0]->a_ws), s, &a, &lda, &k16)) != MI_OK)
-    return rc;
+  int k16 = round_up(k, 16);
   // as in mi_matmul_run_group
+  auto prepare = [&] {
+    return a != nullptr ? MI_OK : prepare_rows(a_dev, rows, k, Workspace::growable(&handles[0]->a_ws), s, &a, &lda, &k16);
+  };
   const bool few = count >= 2 && count <= 4;
   bool decode = few && rows <= kGemvGroupMaxRows && (rows > kGemvDotRows || (int64_t)rows * k16 <= 150 * 1024), tiles = few;
   for (int i = 0; i < count && few; ++i) {
@@ -1623,19 +1660,27 @@ int mi_dynmm_run_group(mi_dynmm *const *handles, int32_t count, const int8_t *a_
     DequantParams dq[4];
     int n[4];
     for (int i = 0; i < count; ++i) {
-      const mi_dynmm *h = handles[i];
-      wv[i] = WeightView{static_cast<const int8_t *>(h->w.p), h->k_pad, h->ldw, static_cast<const int8_t *>(h->w_blocked.p)};
-      dq[i] = dequant_params(h, (float)in_scale, in_zp, params_dev, per_row != 0);
-      n[i] = h->n;
+      wv[i] = weight_view(handles[i]);
+      dq[i] = dequant_params(handles[i], (float)in_scale, in_zp, params_dev, per_row != 0);
+      n[i] = handles[i]->n;
     }
-    if (decode) return launch_gemv_group_dequant(a, lda, rows, k16, count, wv, n, dq, c_dev, s);
-    bool taken = false;
-    rc = launch_gemm_group_dequant(a, lda, rows, k16, count, wv, n, dq, c_dev, s, &taken);
-    if (rc != MI_OK || taken) return rc;
+    const TileCost *tile = decode ? nullptr : gemm_group_tile(k16, rows, k16, count, wv, n, dq);
+    if (decode || tile != nullptr) {
+      if ((rc = prepare()) != MI_OK) return rc;
+      if (decode) return launch_gemv_group_dequant(a, lda, rows, k16, count, wv, n, dq, c_dev, s);
+      return launch_gemm_group_dequant(*tile, a, lda, rows, k16, count, wv, n, dq, c_dev, s);
+    }
   }
+  const bool copy = shares_padded_copy(count);
   for (int i = 0; i < count; ++i) {
-    if ((rc = dynmm_run_impl(handles[i], a_dev, rows, (float)in_scale, in_zp, params_dev, c_dev[i], s, per_row != 0)) != MI_OK)
-      return rc;
+    const mi_dynmm *h = handles[i];
+    const DequantParams dq = dequant_params(h, (float)in_scale, in_zp, params_dev, per_row != 0);
+    if (!copy && runs_on_anyrow(h, a_dev, rows)) {
+      rc = launch_gemm_anyrow_dequant(a_dev, rows, k, weight_view(h), h->n, dq, c_dev[i], s);
+    } else if ((rc = prepare()) == MI_OK) {
+      rc = run_dequant_gemm(h, a, lda, rows, k16, dq, c_dev[i], s);
+    }
+    if (rc != MI_OK) return rc;
   }
   return MI_OK;
 }

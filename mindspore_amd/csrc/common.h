@@ -100,11 +100,15 @@ int launch_gemm_anyrow_dequant(const int8_t *a, int m, int k, const WeightView &
                                hipStream_t stream);
 
 // Up to four weight matrices with the same K against the same activation rows as one launch; member i writes c[i] with row
-// stride n[i].  *taken: it was launched; otherwise the members are to be run one by one.
-int launch_gemm_group_requant(const int8_t *a, int64_t lda, int m, int k, int count, const WeightView *w, const int *n,
-                              const RequantParams *rq, int8_t *const *c, hipStream_t stream, bool *taken);
-int launch_gemm_group_dequant(const int8_t *a, int64_t lda, int m, int k, int count, const WeightView *w, const int *n,
-                              const DequantParams *dq, float *const *c, hipStream_t stream, bool *taken);
+// stride n[i].  gemm_group_tile: what the launch would run on, or null where the members are to be run one by one; lda: of the
+// rows that it would be given.
+struct TileCost;
+const TileCost *gemm_group_tile(int64_t lda, int m, int k, int count, const WeightView *w, const int *n, const RequantParams *rq);
+const TileCost *gemm_group_tile(int64_t lda, int m, int k, int count, const WeightView *w, const int *n, const DequantParams *dq);
+int launch_gemm_group_requant(const TileCost &tile, const int8_t *a, int64_t lda, int m, int k, int count, const WeightView *w,
+                              const int *n, const RequantParams *rq, int8_t *const *c, hipStream_t stream);
+int launch_gemm_group_dequant(const TileCost &tile, const int8_t *a, int64_t lda, int m, int k, int count, const WeightView *w,
+                              const int *n, const DequantParams *dq, float *const *c, hipStream_t stream);
 
 // Skinny-M path (m <= kGemvMaxRows): streams the weights once with 16-byte coalesced loads.
 constexpr int kGemvMaxRows = 64;

@@ -591,64 +591,68 @@ int launch_gemm_anyrow_dequant(const int8_t *a, int m, int k, const WeightView &
   return rc != MI_OK ? rc : launch_gemm_anyrow(false, dq.zw0 != 0, false, g, RequantParams{}, dq, stream);
 }
 
-// Several matrices against the same rows as one launch, where that is expected to take less than a launch each (*taken): a
+// Several matrices against the same rows as one launch, where that is expected to take less than a launch each: a
 // round of tiles more is the price of a launch that fills its last round badly, and there are fewer of those, on larger tiles.
 // us per pair of 11008 x 4096, two launches -> one: int8 output, 128 rows 33.6 -> 26.3, 256 rows 47.6 -> 34.0, 512 rows
 // 64.6 -> 51.5; fp32 output with a scale per row, 2048 rows 194.8 -> 181.
-template <typename P>
-static int pick_group(const int8_t *a, int64_t lda, int m, int k, int count, const WeightView *w, const int *n,
-                      void *const *c, const P *p, GemmGroup<P> *grp, const TileCost **tile) {
-  *tile = nullptr;
-  if (count < 2 || count > kGemmGroupMax || k < 1024 || !kblock_takes(k, lda)) return MI_OK;
+static const TileCost *group_tile(int64_t lda, int m, int k, int count, const WeightView *w, const int *n) {
+  if (count < 2 || count > kGemmGroupMax || k < 1024 || !kblock_takes(k, lda)) return nullptr;
   float alone = 0.0f, together;
   for (int i = 0; i < count; ++i) {
-    const int rc = check_args(a, lda, m, k, w[i], n[i], c[i], n[i]);
-    if (rc != MI_OK) return rc;
-    if (w[i].blocked == nullptr || w[i].k_pad != w[0].k_pad) return MI_OK;
+    if (w[i].blocked == nullptr || w[i].k_pad != w[0].k_pad) return nullptr;
     float cost;
     cheapest_tile(m, k, 1, n + i, &cost);
     alone += cost;
+  }
+  const TileCost &t = cheapest_tile(m, k, count, n, &together);
+  return together < alone ? &t : nullptr;
+}
+
+const TileCost *gemm_group_tile(int64_t lda, int m, int k, int count, const WeightView *w, const int *n, const RequantParams *rq) {
+  for (int i = 0; i < count; ++i)
+    if (rq[i].has_zw || !rq[i].fast2) return nullptr;
+  return group_tile(lda, m, k, count, w, n);
+}
+
+const TileCost *gemm_group_tile(int64_t lda, int m, int k, int count, const WeightView *w, const int *n, const DequantParams *dq) {
+  for (int i = 0; i < count; ++i)
+    if (dq[i].zw0 != 0) return nullptr;
+  return group_tile(lda, m, k, count, w, n);
+}
+
+template <typename P>
+static int fill_group(const int8_t *a, int64_t lda, int m, int k, int count, const WeightView *w, const int *n, void *const *c,
+                      const P *p, GemmGroup<P> *grp) {
+  for (int i = 0; i < count; ++i) {
+    const int rc = check_args(a, lda, m, k, w[i], n[i], c[i], n[i]);
+    if (rc != MI_OK) return rc;
     grp->n[i] = n[i];
     grp->wb[i] = w[i].blocked;
     grp->c[i] = c[i];
     grp->p[i] = p[i];
   }
-  const TileCost &t = cheapest_tile(m, k, count, n, &together);
-  if (together >= alone) return MI_OK;
   grp->g = GemmArgs{a, lda, m, k, nullptr, 0, w[0].k_pad, nullptr, 0, 0, 0, nullptr, 0};
   grp->count = count;
-  *tile = &t;
   return MI_OK;
 }
 
-int launch_gemm_group_requant(const int8_t *a, int64_t lda, int m, int k, int count, const WeightView *w, const int *n,
-                              const RequantParams *rq, int8_t *const *c, hipStream_t stream, bool *taken) {
-  *taken = false;
-  for (int i = 0; i < count; ++i)
-    if (rq[i].has_zw || !rq[i].fast2) return MI_OK;
+int launch_gemm_group_requant(const TileCost &t, const int8_t *a, int64_t lda, int m, int k, int count, const WeightView *w,
+                              const int *n, const RequantParams *rq, int8_t *const *c, hipStream_t stream) {
   GemmGroup<RequantParams> grp{};
-  const TileCost *t = nullptr;
-  const int rc = pick_group(a, lda, m, k, count, w, n, reinterpret_cast<void *const *>(c), rq, &grp, &t);
-  if (rc != MI_OK || t == nullptr) return rc;
-  *taken = true;
-  return t->ring ? launch_gemm_ring_group(10 * t->tn + t->tm, grp, stream) : launch_gemm_kblock_group(10 * t->tn + t->tm, grp, stream);
+  const int rc = fill_group(a, lda, m, k, count, w, n, reinterpret_cast<void *const *>(c), rq, &grp);
+  if (rc != MI_OK) return rc;
+  return t.ring ? launch_gemm_ring_group(10 * t.tn + t.tm, grp, stream) : launch_gemm_kblock_group(10 * t.tn + t.tm, grp, stream);
 }
 
-int launch_gemm_group_dequant(const int8_t *a, int64_t lda, int m, int k, int count, const WeightView *w, const int *n,
-                              const DequantParams *dq, float *const *c, hipStream_t stream, bool *taken) {
-  *taken = false;
-  bool nt = true;
-  for (int i = 0; i < count; ++i) {
-    if (dq[i].zw0 != 0) return MI_OK;
-    nt = nt && stream_out_hint(m, n[i]);
-  }
+int launch_gemm_group_dequant(const TileCost &t, const int8_t *a, int64_t lda, int m, int k, int count, const WeightView *w,
+                              const int *n, const DequantParams *dq, float *const *c, hipStream_t stream) {
   GemmGroup<DequantParams> grp{};
-  const TileCost *t = nullptr;
-  const int rc = pick_group(a, lda, m, k, count, w, n, reinterpret_cast<void *const *>(c), dq, &grp, &t);
-  if (rc != MI_OK || t == nullptr) return rc;
-  *taken = true;
-  return t->ring ? launch_gemm_ring_group(10 * t->tn + t->tm, nt, grp, stream)
-                 : launch_gemm_kblock_group(10 * t->tn + t->tm, nt, grp, stream);
+  const int rc = fill_group(a, lda, m, k, count, w, n, reinterpret_cast<void *const *>(c), dq, &grp);
+  if (rc != MI_OK) return rc;
+  bool nt = true;
+  for (int i = 0; i < count; ++i) nt = nt && stream_out_hint(m, n[i]);
+  return t.ring ? launch_gemm_ring_group(10 * t.tn + t.tm, nt, grp, stream)
+                : launch_gemm_kblock_group(10 * t.tn + t.tm, nt, grp, stream);
 }
 
 }  // namespace mi

@@ -211,6 +211,40 @@ def test_matmul_group_on_tiles(orc, m, k, ns, how):
             assert np.array_equal(y.cpu().numpy(), want)
 
 
+# ragged rows: members that read them as they are, alone, in pairs and beside one that needs the copy (decode-sized; on tiles of
+# another size); a copy for three and more; one launch on a copy
+@pytest.mark.parametrize("m,k,ns,copies", [(333, 1000, (1001,), False), (333, 1000, (1001, 1000), False), (70, 500, (65, 260), False),
+                                           (40, 500, (4100, 300), True), (600, 1000, (100, 3000), True), (200, 770, (768, 768, 768), True),
+                                           (333, 1400, (1000, 1000), True), (100, 200, (30, 30, 30, 30, 30), True)])
+@pytest.mark.parametrize("how", ["static", "value", "rows"])
+def test_matmul_group_on_ragged_rows(m, k, ns, copies, how):
+    """Against a call per member, with and without the room for a padded copy of the rows."""
+    import torch
+    rng = np.random.default_rng(m + k + sum(ns))
+    a = torch.from_numpy(rng.integers(-128, 128, (m, k), dtype=np.int8)).cuda()
+    args = dict(in_quant=K.QuantParam(0.03, -5)) if how == "value" else {}
+    if how == "rows":
+        a, params = K.DynamicQuantKernel(True).run_rows(torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32)).cuda())
+        args = dict(row_params=params)
+    make = lambda: [_matmul_pair(np.random.default_rng(n), n, k, False, how != "static")[4](True) for n in ns]
+    run = lambda kernels: K.matmul_run_group(kernels, a) if how == "static" else K.dynmm_run_group(kernels, a, **args)
+    want = [kern.run(a, **args) for kern in make()]
+    for kernels in (make(), make()):
+        for _ in range(2):
+            assert all(torch.equal(x, y) for x, y in zip(run(kernels), want))
+    L, kernels = K._lib.load(), make()
+    assert L.mi_debug_fail_alloc(m * ((k + 15) // 16 * 16)) == 0
+    try:
+        if copies:
+            with pytest.raises(K._lib.MiError) as e:
+                run(kernels)
+            assert e.value.code == K._lib.MI_MEMORY_FAILED
+        else:
+            assert all(torch.equal(x, y) for x, y in zip(run(kernels), want))
+    finally:
+        L.mi_debug_fail_alloc(0)
+
+
 @pytest.mark.parametrize("taps", [3, 5])
 @pytest.mark.parametrize("b,ih,iw,ch,pad", [(1, 5, 5, 4, (0, 0, 0, 0)), (1, 5, 6, 8, (1, 1, 1, 1)), (2, 7, 9, 12, (2, 0, 0, 2)),
                                             (1, 9, 11, 20, (4, 4, 4, 4)), (3, 6, 8, 192, (1, 2, 3, 0)), (1, 33, 31, 36, (1, 1, 1, 1)),
