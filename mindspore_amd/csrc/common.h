@@ -195,7 +195,7 @@ int launch_conv_dw_rows(const int8_t *in, const ConvGeom &g, const int32_t *w, c
                         int8_t *out, hipStream_t stream);
 
 // Host tensors of one call, in and out of device memory on the null stream (host_copy.hip).  `dev` holds a multiple of 16 bytes.
-// The page-locked slots that the copies go through stay for the next call while a handle that has used some lives.
+// The page-locked slots that the copies may go through (slot_pool.h) stay while a handle that has made such a call lives.
 struct HostSlots;
 class HostCopyUser {  // a member of every handle with such calls
  public:

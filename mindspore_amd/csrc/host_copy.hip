@@ -7,21 +7,21 @@
 // word per part in the page-locked memory, written behind the part's bytes.
 // MatMuls on host tensors, rows x K x N int8, us per call, hipMemcpy -> slots: 1024 x 4096 x 4096 412 -> 262,
 // 2048 x 4096 x 4096 770 -> 555, 1000 x 256 x 4096 258 -> 150, 256 x 4096 x 1024 97 -> 70, 16 x 4096 x 4096 43 -> 25,
-// 1 x 1024 x 1024 28.5 -> 17.  What is left is the bus, in and out one after the other.
+// 1 x 1024 x 1024 28.5 -> 17.  What is left is the bus, in and out one after the other.  slot_pool.h says which calls have slots.
 #include <string.h>
 
-#include <mutex>
 #include <new>
 
 #include "common.h"
+#include "slot_pool.h"
 
 namespace mi {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 
 constexpr int kWgBytes = 16384;  // 256 threads, four times 16 bytes each
-// Page-locked memory of a call, cut into slots of a chunk each.  The pages of new memory cost 0.4 us per KiB once, so calls on
-// small tensors get little; 1 MiB instead of 2 makes 262 us 303, 4 MiB 265.
+// Page-locked memory of a call, cut into slots of a chunk each.  New pages cost 0.4 us per KiB once, so calls on small tensors get
+// little; 1 MiB instead of 2 makes 262 us 303, 4 MiB 265.
 constexpr size_t kRingBytes[2] = {256 << 10, 2 << 20};
 constexpr int kMostSlots = 8;
 constexpr int kOutWgs = 16;  // us at 4 MiB out: 16 149, 32 154, 64 159, 256 230 (1000 x 256 x 4096)
@@ -56,59 +56,31 @@ struct HostSlots {
   uint32_t ticket = 0;        // of the last launch
   uint32_t pending[kMostSlots] = {};  // of the launch that uses the slot, 0: none
   HostSlots *next = nullptr;
+
+  static HostSlots *make(int size) {
+    HostSlots *s = new (std::nothrow) HostSlots();
+    if (s == nullptr) return nullptr;
+    const size_t flag_bytes = sizeof(uint32_t) * (kRingBytes[size] / kWgBytes);
+    void *p = nullptr;
+    if (hipHostMalloc(&p, kRingBytes[size] + flag_bytes, hipHostMallocCoherent | hipHostMallocPortable) != hipSuccess) {
+      (void)hipGetLastError();
+      delete s;
+      return nullptr;
+    }
+    s->size = size;
+    s->data = static_cast<char *>(p);
+    s->flags = reinterpret_cast<uint32_t *>(s->data + kRingBytes[size]);
+    memset(s->flags, 0, flag_bytes);
+    return s;
+  }
+  static void free(HostSlots *s) {
+    (void)hipHostFree(s->data);
+    delete s;
+  }
 };
 
 namespace {
-// Idle slots wait here for the next call.  Calls that run at the same time have slots of their own; at most kMostIdle stay, and
-// the last handle that made such a call takes them with it.
-constexpr int kMostIdle = 2;
-std::mutex g_mutex;
-HostSlots *g_idle[2] = {};
-int g_idle_count[2] = {}, g_users = 0;
-
-void free_slots(HostSlots *s) {
-  (void)hipHostFree(s->data);
-  delete s;
-}
-
-HostSlots *take_slots(int size) {
-  {
-    std::lock_guard<std::mutex> lock(g_mutex);
-    if (g_idle[size] != nullptr) {
-      HostSlots *s = g_idle[size];
-      g_idle[size] = s->next;
-      --g_idle_count[size];
-      return s;
-    }
-  }
-  HostSlots *s = new (std::nothrow) HostSlots();
-  if (s == nullptr) return nullptr;
-  const size_t flag_bytes = sizeof(uint32_t) * (kRingBytes[size] / kWgBytes);
-  void *p = nullptr;
-  if (hipHostMalloc(&p, kRingBytes[size] + flag_bytes, hipHostMallocCoherent | hipHostMallocPortable) != hipSuccess) {
-    (void)hipGetLastError();
-    delete s;
-    return nullptr;
-  }
-  s->size = size;
-  s->data = static_cast<char *>(p);
-  s->flags = reinterpret_cast<uint32_t *>(s->data + kRingBytes[size]);
-  memset(s->flags, 0, flag_bytes);
-  return s;
-}
-
-void give_slots(HostSlots *s) {
-  {
-    std::lock_guard<std::mutex> lock(g_mutex);
-    if (g_idle_count[s->size] < kMostIdle && g_users > 0) {
-      s->next = g_idle[s->size];
-      g_idle[s->size] = s;
-      ++g_idle_count[s->size];
-      return;
-    }
-  }
-  free_slots(s);
-}
+SlotPool<HostSlots> g_pool;
 
 // A transfer cut into chunks, of which chunk i goes through slot i % slots.
 struct Chunks {
@@ -149,7 +121,8 @@ int launch_chunks(HostSlots *s, const Chunks &c, int64_t i, int n, char *dev, bo
   return MI_OK;
 }
 
-// Until every workgroup that copies chunk i has said that it is done.
+// Until every workgroup that copies chunk i has said that it is done.  (The host spins, as hipMemcpy does: 1024 x 4096 x 4096 264 us
+// of a core per call, with hipMemcpy 423.)
 int await_chunk(HostSlots *s, const Chunks &c, int64_t i) {
   const int slot = c.slot(i), wgs = c.wgs(c.size(i));
   if (s->pending[slot] == 0) return MI_OK;
@@ -185,20 +158,7 @@ bool is_pageable(const void *p) {
 }  // namespace
 
 HostCopyUser::~HostCopyUser() {
-  if (!used_) return;
-  HostSlots *all[2];
-  {
-    std::lock_guard<std::mutex> lock(g_mutex);
-    if (--g_users > 0) return;
-    for (int i = 0; i < 2; ++i) all[i] = g_idle[i], g_idle[i] = nullptr, g_idle_count[i] = 0;
-  }
-  for (HostSlots *s : all) {
-    while (s != nullptr) {
-      HostSlots *next = s->next;
-      free_slots(s);
-      s = next;
-    }
-  }
+  if (used_) g_pool.drop_user();
 }
 
 HostCopies::HostCopies(HostCopyUser *user, size_t most_bytes) : user_(user), size_(most_bytes > kRingBytes[0] ? 1 : 0) {}
@@ -209,19 +169,17 @@ HostCopies::~HostCopies() {
   for (int i = 0; i < kMostSlots; ++i) busy = busy || slots_->pending[i] != 0;
   if (busy) (void)hipStreamSynchronize(nullptr);
   for (int i = 0; i < kMostSlots; ++i) slots_->pending[i] = 0;
-  give_slots(slots_);
+  g_pool.give(size_, slots_);
 }
 
 bool HostCopies::through_slots(const void *host, size_t bytes) {
-  if (bytes == 0 || !is_pageable(host)) return false;
-  if (slots_ == nullptr) {
-    if (!user_->used_) {
-      std::lock_guard<std::mutex> lock(g_mutex);
-      user_->used_ = true;
-      ++g_users;
-    }
-    slots_ = take_slots(size_);
+  if (bytes == 0) return false;
+  if (slots_ != nullptr) return is_pageable(host);
+  if (!user_->used_) {
+    user_->used_ = true;
+    g_pool.add_user();
   }
+  slots_ = g_pool.take(size_, bytes, [host] { return is_pageable(host); });
   return slots_ != nullptr;
 }
 

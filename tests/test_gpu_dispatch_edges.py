@@ -532,12 +532,36 @@ def test_group_of_many_kernels(dynamic):
         assert torch.equal(y, kern.run(a, **args))
 
 
+@pytest.fixture
+def host_slots():
+    """Page-locked slots of both sizes for several callers at once: calls go without until they have lost the price of a set."""
+    import threading
+    rng = np.random.default_rng(78)
+    work = [(_matmul_pair(rng, n, k, False, False)[4](True), rng.integers(-128, 128, (rows, k), dtype=np.int8))
+            for rows, k, n in ((1000, 2000, 1500), (100, 300, 500)) * 6]
+
+    def go(kern, a):
+        for _ in range(80):
+            kern.run(a)
+
+    threads = [threading.Thread(target=go, args=w) for w in work]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    yield  # (they stay while these kernels do)
+    work.clear()
+
+
 # one chunk, a last chunk of one byte, as many chunks as slots, slots used several times, on the way in, out and both
 @pytest.mark.parametrize("rows,k,n", [(1, 1, 1), (3, 70001, 2), (65537, 1, 1), (517, 1000, 64), (2099, 1001, 5), (2100, 7, 1001),
                                       (3001, 1500, 1401)])
-def test_host_tensors_in_and_out(rows, k, n):
+@pytest.mark.parametrize("slots", [False, True])
+def test_host_tensors_in_and_out(request, rows, k, n, slots):
     """Against the same kernels on device tensors."""
     import torch
+    if slots:
+        request.getfixturevalue("host_slots")
     rng = np.random.default_rng(rows + k)
     a = rng.integers(-128, 128, (rows, k), dtype=np.int8)
     dev = torch.from_numpy(a).cuda()
@@ -556,9 +580,12 @@ def test_host_tensors_in_and_out(rows, k, n):
         assert np.array_equal(dq.run_rows(x)[0] if per_row else dq.run(x)[0], there.cpu().numpy())
 
 
-def test_host_tensors_from_several_threads():
+@pytest.mark.parametrize("slots", [False, True])
+def test_host_tensors_from_several_threads(request, slots):
     import threading
     import torch
+    if slots:
+        request.getfixturevalue("host_slots")
     rng = np.random.default_rng(77)
     work = []
     for rows, k, n in ((700, 900, 1100), (64, 64, 64), (1500, 2000, 300), (2000, 300, 2000), (1, 5, 9)):
