@@ -144,8 +144,9 @@ __device__ __forceinline__ void gemm_anyrow_body(const GemmArgs &g, const Requan
 #endif
 }
 
+// (the LDS lets one workgroup into a CU: a wave per SIMD)
 template <int EPI, bool HAS_ZW, bool FAST>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_anyrow_kernel(GemmArgs g, RequantParams rq,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_anyrow_kernel(GemmArgs g, RequantParams rq,
                                                                                                      DequantParams dq) {
   gemm_anyrow_body<EPI, HAS_ZW, FAST>(g, rq, dq);
 }
