@@ -38,7 +38,8 @@ struct ConvWindow {
   int steps;                             // of 32 bytes of K
   int weight_bytes, patch_bytes;         // in LDS, multiples of 1 KiB
   bool streams;
-  uint32_t magic_pitch, magic_patch_w, magic_tile_w, magic_cc, magic_kernel_w, magic_quads;  // ceil(2^32 / d): exact quotients for dividends < 2^16 (d >= 2; 0: d = 1)
+  // ceil(2^32 / d): exact quotients for dividends < 2^16 (d >= 2; 0: d = 1)
+  uint32_t magic_pitch, magic_patch_w, magic_tile_w, magic_cc, magic_kernel_w, magic_quads;
   uint32_t magic_tiles_x, magic_tiles_y;  // see magic31
   int shift_tiles_x, shift_tiles_y;
   const int8_t *w;       // [32 channels][step][lane][16]
@@ -53,8 +54,8 @@ typedef v4i v4i_4 __attribute__((aligned(4)));
 typedef v4u v4u_any __attribute__((aligned(1)));
 
 template <int OCB, bool PACKED, RequantForm FORM>
-__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWaves / 2))) void conv_window_kernel(ConvWindow g, RequantParams rq,
-                                                                                                int8_t *__restrict__ out) {
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWaves / 2))) void conv_window_kernel(
+    ConvWindow g, RequantParams rq, int8_t *__restrict__ out) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -219,7 +220,8 @@ static std::vector<int8_t> operand_order(const int8_t *w, int oc, int k) {
     const int n = column_channel(ocb, column / 32, column % 32);
     if (n >= oc) continue;
     for (int k0 = 0; k0 < k; k0 += 16)
-      memcpy(&out[(((size_t)(column / 32) * steps + k0 / 32) * 64 + column % 32 + 32 * (k0 / 16 % 2)) * 16], w + (size_t)n * k + k0, 16);
+      memcpy(&out[(((size_t)(column / 32) * steps + k0 / 32) * 64 + column % 32 + 32 * (k0 / 16 % 2)) * 16],
+             w + (size_t)n * k + k0, 16);
   }
   return out;
 }
@@ -235,7 +237,8 @@ std::vector<int8_t> conv_window_weights(const ConvGeom &g, const int8_t *w) {
   for (int n = 0; n < g.out_c; ++n)
     for (int kh = 0; kh < g.kernel_h; ++kh)
       for (int kw = 0; kw < g.kernel_w; ++kw)
-        memcpy(&wide[(size_t)n * k + kh * row_chunks(g) * 16 + kw * 4], w + (((size_t)n * g.kernel_h + kh) * g.kernel_w + kw) * g.in_c, g.in_c);
+        memcpy(&wide[(size_t)n * k + kh * row_chunks(g) * 16 + kw * 4],
+               w + (((size_t)n * g.kernel_h + kh) * g.kernel_w + kw) * g.in_c, g.in_c);
   return operand_order(wide.data(), g.out_c, k);
 }
 
@@ -261,16 +264,19 @@ static bool cut_window(const ConvGeom &g, WindowCut *best) {
     c.tiles_y = (g.out_h + c.tile_h - 1) / c.tile_h;
     c.tile_h = (g.out_h + c.tiles_y - 1) / c.tiles_y;
     const int64_t ph = (int64_t)(c.tile_h - 1) * g.stride_h + (int64_t)(g.kernel_h - 1) * g.dilation_h + 1;
-    int64_t pw = (int64_t)(c.tile_w - 1) * g.stride_w + (packed ? 4 * row_chunks(g) : (int64_t)(g.kernel_w - 1) * g.dilation_w + 1);
+    int64_t pw = (int64_t)(c.tile_w - 1) * g.stride_w +
+                 (packed ? 4 * row_chunks(g) : (int64_t)(g.kernel_w - 1) * g.dilation_w + 1);
     if (packed) pw = (pw + 3) & ~3;
     if (ph > 4096 || pw > 4096) continue;
     c.patch_h = (int)ph;
     c.patch_w = (int)pw;
-    const int64_t bytes = ((ph + (packed ? g.dilation_h : 0)) * pw * (packed ? 4 : c.pitch * 16) + 1023) / 1024 * 1024;  // (hence fewer than 2^16 chunks)
+    const int64_t patch = (ph + (packed ? g.dilation_h : 0)) * pw * (packed ? 4 : c.pitch * 16);
+    const int64_t bytes = (patch + 1023) / 1024 * 1024;  // (at most kWindowLds, hence fewer than 2^16 chunks)
     if (c.weight_bytes + bytes + 8 * c.steps > kWindowLds) continue;
     c.patch_bytes = (int)bytes;
     c.tiles = (int64_t)c.tiles_x * c.tiles_y * g.batch;
-    if (best->tiles == 0 || c.tiles < best->tiles || (c.tiles == best->tiles && c.patch_bytes < best->patch_bytes)) *best = c;
+    const bool fewer = c.tiles < best->tiles || (c.tiles == best->tiles && c.patch_bytes < best->patch_bytes);
+    if (best->tiles == 0 || fewer) *best = c;
   }
   return best->tiles != 0;
 }
@@ -286,12 +292,16 @@ constexpr int kWindowLeastTiles = 168;
 bool conv_window_weights_wanted(const ConvGeom &g) {
   const int taps = g.kernel_h * g.kernel_w;
   if (g.in_c == 3 || g.in_c == 4)
-    return g.out_c <= 64 && g.kernel_w <= 8 && g.kernel_h <= 16 && g.dilation_w == 1 && g.kernel_h * (g.kernel_w * g.in_c > 16 ? 2 : 1) > 8;
+    return g.out_c <= 64 && g.kernel_w <= 8 && g.kernel_h <= 16 && g.dilation_w == 1 &&
+           g.kernel_h * (g.kernel_w * g.in_c > 16 ? 2 : 1) > 8;
   return (g.in_c & 15) == 0 && g.out_c <= 64 && taps > 1 && (int64_t)taps * g.in_c <= 2048;
 }
 static bool choose_window(const ConvGeom &g, const void *in, WindowCut *c) {
-  return conv_window_weights_wanted(g) && ((reinterpret_cast<uintptr_t>(in) & 15) == 0 || packed_window(g)) && (int64_t)g.batch * g.in_h * g.in_w * g.in_c >= 16 && (int64_t)g.in_h * g.in_w * g.in_c < (int64_t)1 << 31 && cut_window(g, c) && c->tiles >= kWindowLeastTiles &&
-         c->tiles * (32 * kWaves / 2) <= (int64_t)g.batch * g.out_h * g.out_w && c->tiles < 1 << 23;  // (2^32 threads)
+  const int64_t image = (int64_t)g.in_h * g.in_w * g.in_c;
+  if (!conv_window_weights_wanted(g) || g.batch * image < 16 || image >= (int64_t)1 << 31) return false;
+  if ((reinterpret_cast<uintptr_t>(in) & 15) != 0 && !packed_window(g)) return false;
+  return cut_window(g, c) && c->tiles >= kWindowLeastTiles && c->tiles < 1 << 23 &&  // (2^32 threads)
+         c->tiles * (32 * kWaves / 2) <= (int64_t)g.batch * g.out_h * g.out_w;
 }
 
 typedef void (*WindowKernel)(ConvWindow, RequantParams, int8_t *);
@@ -308,7 +318,8 @@ int conv_window_prepare_device() {
   for (const auto &of_blocks : kWindowKernels)
     for (const auto &of_packed : of_blocks)
       for (const WindowKernel kernel : of_packed)
-        MI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kWindowLds));
+        MI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         kWindowLds));
   return MI_OK;
 }
 
@@ -318,11 +329,20 @@ int launch_conv_window(const int8_t *in, const ConvGeom &g, const int8_t *fill16
   *taken = requant_form(rq) != kGeneralForm && choose_window(g, in, &t);
   if (!*taken) return MI_OK;
   const bool packed = packed_window(g);
-  const bool streams = conv_streams((int64_t)g.batch * g.out_h * g.out_w, g.out_c, g.out_c > 32 ? 2 : 1);
-  ConvWindow c{in, in + (int64_t)g.batch * g.in_h * g.in_w * g.in_c - 4, g.in_h, g.in_w, g.in_c, g.out_h, g.out_w, g.out_c, g.kernel_h, g.kernel_w, g.stride_h, g.stride_w, g.dilation_h,
-               g.dilation_w, g.pad_u, g.pad_l, t.tile_h, t.tile_w, t.tiles_x, t.tiles_y, t.patch_h, t.patch_w, packed ? row_chunks(g) : g.in_c / 16, t.pitch,
-               t.steps, t.weight_bytes, t.patch_bytes, streams, magic16(t.pitch), magic16(t.patch_w), magic16(t.tile_w), magic16(packed ? row_chunks(g) : g.in_c / 16), magic16(g.kernel_w),
-               magic16(t.patch_w / 4), 0, 0, 0, 0, w, fill16};
+  const int cc = packed ? row_chunks(g) : g.in_c / 16;
+  ConvWindow c{};
+  c.in = in;
+  c.in_last4 = in + (int64_t)g.batch * g.in_h * g.in_w * g.in_c - 4;
+  c.in_h = g.in_h, c.in_w = g.in_w, c.in_c = g.in_c, c.out_h = g.out_h, c.out_w = g.out_w, c.out_c = g.out_c;
+  c.kernel_h = g.kernel_h, c.kernel_w = g.kernel_w, c.stride_h = g.stride_h, c.stride_w = g.stride_w;
+  c.dil_h = g.dilation_h, c.dil_w = g.dilation_w, c.pad_u = g.pad_u, c.pad_l = g.pad_l;
+  c.tile_h = t.tile_h, c.tile_w = t.tile_w, c.tiles_x = t.tiles_x, c.tiles_y = t.tiles_y;
+  c.patch_h = t.patch_h, c.patch_w = t.patch_w, c.cc = cc, c.pitch = t.pitch, c.steps = t.steps;
+  c.weight_bytes = t.weight_bytes, c.patch_bytes = t.patch_bytes;
+  c.streams = conv_streams((int64_t)g.batch * g.out_h * g.out_w, g.out_c, g.out_c > 32 ? 2 : 1);
+  c.magic_pitch = magic16(t.pitch), c.magic_patch_w = magic16(t.patch_w), c.magic_tile_w = magic16(t.tile_w);
+  c.magic_cc = magic16(cc), c.magic_kernel_w = magic16(g.kernel_w), c.magic_quads = magic16(t.patch_w / 4);
+  c.w = w, c.fill16 = fill16;
   magic31(t.tiles_x, &c.magic_tiles_x, &c.shift_tiles_x);
   magic31(t.tiles_y, &c.magic_tiles_y, &c.shift_tiles_y);
   const size_t lds = (size_t)t.weight_bytes + t.patch_bytes + 8 * (size_t)t.steps;
