@@ -10,18 +10,17 @@ namespace mi {
 // Slots is a set of slots with a member `next`, made by Slots::make(size) (null: no memory) and given back by Slots::free.  A set
 // serves one call at a time; idle ones wait for the next call while a handle that makes such calls lives (add_user / drop_user).
 //
-// A set costs page-locked memory: us to allocate, touch and free, 256 KiB 80 + 110 + 50, 2 MiB 60 + 880 + 50, and about 200 where the
-// process has had and given back the pages before.  It saves a tensor about 5 us and 15 per MiB.  So tensors go without until
-// what they would have saved comes to the price of a set: a program of a few calls, or one that makes a handle for each, pays
-// nothing, and no program more than it would have saved by then.  (The first call of a process on 64 rows of 64 took 490 us
-// where it made slots, 65 without; on 1024 x 1024 640 and 465; handles of a single call on 256 x 1024 x 1024 and their destruction
-// 270 and 102.)
+// A set costs page-locked memory, about 200 us to allocate, touch and give back (where a process has the pages for the first time
+// 256 KiB take 240, 2 MiB 1000).  It saves a tensor about 5 us and 15 per MiB.  So tensors go without until what they would have
+// saved comes to the price of a set: a program of a few small calls, or one that makes a handle for each, pays nothing.
+// us, a set in the first call -> this: first call of a process on 64 rows of 64 490 -> 65 (hipMemcpy 65); a call of a new handle and its
+// destruction on 256 x 1024 x 1024 270 -> 110 (102), on 64 x 64 x 64 220 -> 75 (75).
 // As many sets as callers have met at once, up to kMostSets; callers beyond go without.
 template <typename Slots>
 class SlotPool {
  public:
   static constexpr int kSizes = 2, kMostSets = 8;
-  static constexpr float kPrice[kSizes] = {250.0f, 1000.0f}, kPriceAgain = 200.0f;  // us
+  static constexpr float kPrice = 200.0f;  // us
 
   void add_user() {
     std::lock_guard<std::mutex> lock(mutex_);
@@ -38,8 +37,7 @@ class SlotPool {
           x->next = idle;
           idle = x;
         }
-        s.made = 0;
-        s.forgone = 0.0f;
+        s = Size{};
       }
     }
     while (idle != nullptr) {
@@ -59,7 +57,7 @@ class SlotPool {
       if (s.idle == nullptr) {
         if (s.made == kMostSets) return nullptr;
         s.forgone += 5.0f + 15.0f / (1 << 20) * (float)bytes;
-        if (s.forgone < (s.made < s.most ? kPriceAgain : kPrice[size])) return nullptr;
+        if (s.forgone < kPrice) return nullptr;
       }
     }
     const bool wanted = pageable();
@@ -72,7 +70,7 @@ class SlotPool {
       }
       s.forgone = 0.0f;
       if (!wanted || s.made == kMostSets) return nullptr;
-      if (++s.made > s.most) s.most = s.made;
+      ++s.made;
     }
     Slots *x = Slots::make(size);
     if (x == nullptr) {
@@ -90,7 +88,7 @@ class SlotPool {
  private:
   struct Size {
     Slots *idle = nullptr;
-    int made = 0, most = 0;  // now, ever
+    int made = 0;
     float forgone = 0.0f;  // us
   };
   std::mutex mutex_;

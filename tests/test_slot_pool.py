@@ -63,7 +63,7 @@ int main() {
       if (s != nullptr) p.give(size, s);
     }
     CHECK(made == 1 && live == 1);
-    CHECK(first * saved(kBytes[size]) < Pool::kPrice[size] && (first + 1) * saved(kBytes[size]) >= Pool::kPrice[size]);
+    CHECK(first * saved(kBytes[size]) < Pool::kPrice && (first + 1) * saved(kBytes[size]) >= Pool::kPrice);
     // bursts of more callers than there may be sets: they stay from burst to burst, callers beyond go without
     for (int burst = 0; burst < 2000; ++burst) {
       std::vector<Set *> held;
@@ -78,13 +78,6 @@ int main() {
     p.add_user();
     p.drop_user();
     CHECK(live == Pool::kMostSets);
-    p.drop_user();
-    CHECK(live == 0);
-    // pages that the process has had before are cheaper
-    p.add_user();
-    for (first = 0; live == 0; ++first)
-      if (Set *s = p.take(size, kBytes[size], pageable)) p.give(size, s);
-    CHECK((first - 1) * saved(kBytes[size]) < Pool::kPriceAgain && first * saved(kBytes[size]) >= Pool::kPriceAgain);
     p.drop_user();
     CHECK(live == 0);
     // no page-locked memory: without, and a set as soon as there is some and it is worth it again
