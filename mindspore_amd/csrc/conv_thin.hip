@@ -19,8 +19,8 @@ typedef v4i v4i_any __attribute__((aligned(1)));
 // The pixels are the MFMA's row operand, see conv_store.h.
 // Bound by the vector ALU (the requantisation, 4 instructions per output byte) and the stores where there are more channels than
 // bytes of K, by memory where there are fewer.  us per launch, GEMM -> with a clamp, shift and carry of its own for each output
-// and temporal stores of four bytes -> now: 16 x 112 x 112, 192 -> 32 channels 45.2 -> 10.7 -> 10.4, 32 -> 64 - -> 7.0 -> 5.7, 32 -> 128
-// - -> 11.2 -> 9.2, 32 -> 192 21.0 -> 16.2 -> 14.8; 8 x 115 x 115, 240 -> 40 26.5 -> 9.4 -> 9.7;
+// and temporal stores of four bytes -> now: 16 x 112 x 112, 192 -> 32 channels 45.2 -> 10.7 -> 10.7, 32 -> 64 - -> 7.0 -> 5.5, 32 -> 128
+// - -> 11.2 -> 8.4, 32 -> 192 21.0 -> 15.6 -> 13.5, 24 -> 72 - -> 8.9 -> 7.7; 8 x 115 x 115, 240 -> 40 26.5 -> 9.4 -> 9.2;
 // 4 x 80 x 80, 72 -> 24 9.0 (in two launches) -> 3.5; one image of 112 x 112, where any launch takes most of it, 192 -> 32 3.7 -> 3.8.
 struct ConvThin {
   const int8_t *in;
