@@ -265,8 +265,7 @@ static int upload(DevBuf *b, const std::vector<T> &v) {
 // ---- shared "requantising GEMM operand" state: packed weights + per-channel epilogue arrays ------------------------
 struct RequantState {
   int n = 0, k = 0, n_pad = 0, k_pad = 0, ldw = 0;
-  DevBuf w, mult, bias2, rshift, lshift, zw;
-  DevBuf mult2, c2lo, c2hi, pre;  // the GEMM epilogue's per-channel constants (RequantParams::fast2)
+  DevBuf w, channels;  // channels: the arrays of RequantParams
   DevBuf w_blocked;  // the same weights in 1 KiB matrix-core blocks (two activation rows and more); built in create or absent
   std::vector<int32_t> h_mult, h_ls, h_rs, h_bias2;
   int32_t amin = -128, amax = 127, zo = 0;
@@ -275,20 +274,12 @@ struct RequantState {
 
   RequantParams params() const {
     RequantParams rq{};
-    rq.mult = static_cast<const int32_t *>(mult.p);
-    rq.bias2 = static_cast<const int32_t *>(bias2.p);
-    rq.rshift = static_cast<const int32_t *>(rshift.p);
-    rq.lshift = static_cast<const int32_t *>(lshift.p);
-    rq.zw = static_cast<const int32_t *>(zw.p);
+    rq.set_channels(static_cast<const RequantChannel *>(channels.p), n_pad);
     rq.zo = zo;
     rq.amin = amin;
     rq.amax = amax;
     rq.has_zw = has_zw ? 1 : 0;
     rq.fast = fast ? 1 : 0;
-    rq.mult2 = static_cast<const uint32_t *>(mult2.p);
-    rq.c2lo = static_cast<const uint32_t *>(c2lo.p);
-    rq.c2hi = static_cast<const uint32_t *>(c2hi.p);
-    rq.pre = static_cast<const int32_t *>(pre.p);
     rq.most_shift = most_shift;
     rq.fast2 = fast2 ? 1 : 0;
     return rq;
@@ -362,16 +353,21 @@ struct RequantState {
       hi[c] = (uint32_t)(c2 >> 32);
       prev[c] = (int32_t)(((uint32_t)1 << e[c]) >> 1) + (int32_t)((uint32_t)zo << e[c]) - 1;
     }
+    std::vector<int32_t> block((size_t)RequantParams::kWordsPerChannel * n_pad);
+    RequantParams at{};
+    at.set_channels(reinterpret_cast<const RequantChannel *>(block.data()), n_pad);
+    auto put = [&](const void *where, const auto &what) { memcpy(const_cast<void *>(where), what.data(), what.size() * sizeof(what[0])); };
+    std::vector<RequantChannel> each(n_pad);
+    for (int c = 0; c < n_pad; ++c) each[c] = RequantChannel{h_mult[c], h_bias2[c], (uint32_t)e[c] | (uint32_t)h_ls[c] << 8, zwv[c]};
+    put(at.each, each);
+    put(at.mult2, m2);
+    put(at.c2lo, lo);
+    put(at.c2hi, hi);
+    put(at.pre, prev);
+    put(at.rshift, e);
+    put(at.zw, zwv);
     int rc;
-    if ((rc = upload(&mult2, m2)) != MI_OK) return rc;
-    if ((rc = upload(&c2lo, lo)) != MI_OK) return rc;
-    if ((rc = upload(&c2hi, hi)) != MI_OK) return rc;
-    if ((rc = upload(&pre, prev)) != MI_OK) return rc;
-    if ((rc = upload(&mult, h_mult)) != MI_OK) return rc;
-    if ((rc = upload(&bias2, h_bias2)) != MI_OK) return rc;
-    if ((rc = upload(&rshift, e)) != MI_OK) return rc;
-    if ((rc = upload(&lshift, h_ls)) != MI_OK) return rc;
-    if ((rc = upload(&zw, zwv)) != MI_OK) return rc;
+    if ((rc = upload(&channels, block)) != MI_OK) return rc;
     if (pack_weights) {
       std::vector<int8_t> packed((size_t)n_pad * ldw, 0);
       for (int c = 0; c < n; ++c) memcpy(packed.data() + (size_t)c * ldw, w_nk + (size_t)c * k, (size_t)k);
@@ -398,15 +394,7 @@ struct RequantState {
   void release() {
     w.release();
     w_blocked.release();
-    mult.release();
-    bias2.release();
-    rshift.release();
-    lshift.release();
-    zw.release();
-    mult2.release();
-    c2lo.release();
-    c2hi.release();
-    pre.release();
+    channels.release();
   }
 };
 
@@ -575,7 +563,7 @@ struct mi_dynmm {
   int n = 0, k = 0, n_pad = 0, k_pad = 0, ldw = 0, act = 0;
   int32_t zw0 = 0;
   bool has_bias = false;
-  DevBuf w, wscale, wsum, bias, a_ws, h_in, h_out, h_params;
+  DevBuf w, channels, a_ws, h_in, h_out, h_params;  // channels: the arrays of DequantParams
   HostCopyUser host_user;
   DevBuf w_blocked;  // the weights in 1 KiB matrix-core blocks for two activation rows and more; built in create or absent
 };
@@ -1445,6 +1433,12 @@ int mi_dynquant_run_host(mi_dynquant *h, const float *x_host, int64_t n, int8_t 
 void mi_dynquant_destroy(mi_dynquant *h) { delete h; }  // every DevBuf member frees its device memory
 
 // ---------------------------------------------------------------------------------------------------------- dynmm
+static uint32_t f32_bits(float x) {
+  uint32_t u;
+  memcpy(&u, &x, sizeof u);
+  return u;
+}
+
 static int mi_dynmm_create_impl(const mi_dynmm_desc *d, const int8_t *weight_host, const float *bias_host, mi_dynmm **out) {
   if (d == nullptr || weight_host == nullptr || out == nullptr) {
     set_error("mi_dynmm_create: null argument");
@@ -1478,24 +1472,23 @@ static int mi_dynmm_create_impl(const mi_dynmm_desc *d, const int8_t *weight_hos
   const std::vector<int8_t> w_nk = packed_sdot ? unpack_4x16(weight_host, h->n, h->k)
                                                : to_nk(weight_host, h->n, h->k, d->b_transpose);
   std::vector<int8_t> packed((size_t)h->n_pad * h->ldw, 0);
-  std::vector<float> ws(h->n_pad, 0.0f), bs(h->n_pad, 0.0f);
-  std::vector<int32_t> wsum(h->n_pad, 0);
+  std::vector<int32_t> block((size_t)DequantParams::kWordsPerChannel * h->n_pad);
+  std::vector<DequantChannel> channels(h->n_pad);
   for (int c = 0; c < h->n; ++c) {
     memcpy(packed.data() + (size_t)c * h->ldw, w_nk.data() + (size_t)c * h->k, (size_t)h->k);
     int32_t s = 0;
     for (int i = 0; i < h->k; ++i) s += w_nk[(size_t)c * h->k + i];
     // a model that carries its own weight sums is computed with those (matmul_dynamic_base_int8.cc:179-183)
-    wsum[c] = (packed_sdot && d->weight_sums != nullptr) ? d->weight_sums[c] : s;
-    ws[c] = (float)d->filter_scales[d->filter_quant_num > 1 ? c : 0];
-    if (bias_host != nullptr) bs[c] = bias_host[c];
+    channels[c].wsum = (packed_sdot && d->weight_sums != nullptr) ? d->weight_sums[c] : s;
+    channels[c].wscale = (float)d->filter_scales[d->filter_quant_num > 1 ? c : 0];
+    if (bias_host != nullptr) channels[c].bias = bias_host[c];
   }
-  rc = upload(&h->w, packed);
-  if (rc == MI_OK) rc = upload(&h->wscale, ws);
-  if (rc == MI_OK) rc = upload(&h->wsum, wsum);
-  if (rc == MI_OK && h->has_bias) rc = upload(&h->bias, bs);
-  if (rc != MI_OK) {
-    return rc;
+  memcpy(block.data(), channels.data(), sizeof(DequantChannel) * channels.size());
+  for (int c = 0; c < h->n_pad; ++c) {
+    const int32_t words[3] = {(int32_t)f32_bits(channels[c].wscale), (int32_t)f32_bits(channels[c].bias), channels[c].wsum};
+    for (int i = 0; i < 3; ++i) block[(size_t)(4 + i) * h->n_pad + c] = words[i];  // (DequantParams::set_channels)
   }
+  if ((rc = upload(&h->w, packed)) != MI_OK || (rc = upload(&h->channels, block)) != MI_OK) return rc;
   if ((d->flags & MI_DYNMM_NO_DECODE_PACK) == 0) {
     // as for mi_matmul: an optimisation for few activation rows (decode), not a requirement -- without it those row
     // counts run on the GEMM tiles, and a device without room for the copy still gets a working handle
@@ -1530,9 +1523,8 @@ int mi_dynmm_create(const mi_dynmm_desc *d, const int8_t *weight_host, const flo
 
 static DequantParams dequant_params(const mi_dynmm *h, float sx, int32_t zx, const mi_dq_params *qp_dev, bool per_row) {
   DequantParams dq;
-  dq.wscale = static_cast<const float *>(h->wscale.p);
-  dq.bias = h->has_bias ? static_cast<const float *>(h->bias.p) : nullptr;
-  dq.wsum = static_cast<const int32_t *>(h->wsum.p);
+  dq.set_channels(static_cast<const DequantChannel *>(h->channels.p), h->n_pad);
+  dq.has_bias = h->has_bias ? 1 : 0;
   dq.qp_dev = qp_dev;
   dq.sx = sx;
   dq.zx = zx;

@@ -28,18 +28,26 @@ inline int64_t round_up64(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 // the weight operand: rows to a multiple of kNPad, K to a multiple of kKPad (bytes, two 128-byte GEMM steps), zero filled.
 constexpr int kNPad = 256;
 constexpr int kKPad = 256;
+__host__ __device__ inline int padded_k(int k) { return (k + kKPad - 1) & ~(kKPad - 1); }
+__host__ __device__ inline int padded_channels(int n) { return (n + kNPad - 1) & ~(kNPad - 1); }
 
 // The value the 256 x 256 GEMM tile's accumulators start from (taken out again in the epilogue); the host's proof that
 // the cheap rounding form cannot overflow includes it.
 constexpr uint32_t kAccBias = 0x2AAAAAAAu;
 
 // ---- int8 requantising epilogue parameters (device arrays are padded to kNPad entries) ----
+// What the decode kernels, whose waves finish an output per lane, need of a channel, in one load.
+struct alignas(16) RequantChannel {
+  int32_t mult;     // 31-bit mantissa
+  int32_t bias2;    // K*zx*zw - zx*sum(w) + bias
+  uint32_t shifts;  // e = -right_shift clamped to [0, 31], and above its byte the left shift (generic path only)
+  int32_t zw;       // weight zero point
+  __device__ __forceinline__ int32_t rshift() const { return (int32_t)(shifts & 31); }
+  __device__ __forceinline__ int32_t lshift() const { return (int32_t)(shifts >> 8); }
+};
 struct RequantParams {
-  const int32_t *mult;    // 31-bit mantissa per channel
-  const int32_t *bias2;   // K*zx*zw - zx*sum(w) + bias
-  const int32_t *rshift;  // e = -right_shift clamped to [0, 31]
-  const int32_t *lshift;  // left shift (generic path only)
-  const int32_t *zw;      // weight zero point per channel (HAS_ZW only)
+  const RequantChannel *each;
+  const int32_t *rshift, *zw;
   int32_t zo, amin, amax;
   int has_zw;  // any weight zero point is non-zero -> input row sums are needed
   int fast;    // host proved: all lshift == 0, 1 <= e <= 30, no mult == INT32_MIN, amin <= amax, and none of
@@ -49,18 +57,36 @@ struct RequantParams {
   //   x = high dword of (a * mult2 + c2)      == floor(((sum + bias2) * mult + 2^30) / 2^31), the doubling high mul
   //   y = clamp((x + pre + [x >= 0]) >> e)    pre = 2^(e-1) + (zo << e) - 1; [x >= 0] is the carry of a * mult2 + c2
   // mult2 = 2 * mult, c2 = 2 * (bias2 - kAccBias) * mult + 2^31 (mod 2^64, negative as a signed number), in dwords.
-  const uint32_t *mult2;
-  const uint32_t *c2lo, *c2hi;
+  const uint32_t *mult2, *c2lo, *c2hi;
   const int32_t *pre;
   int most_shift;  // the largest e
   int fast2;   // fast, and every mult >= 0, every c2 < 0, and K * 16384 + K * 128 * |zw| <= kAccBias (a in [0, 2^31))
+
+  // The arrays stand one behind the other, of `stride` channels each.  (mult2 to zw are arrays of their own because a wave reads 32
+  // to 64 channels of them: with 16 bytes a channel the window convolutions took 5 % longer.)
+  static constexpr int kWordsPerChannel = 4 + 6;
+  __host__ __device__ __forceinline__ void set_channels(const RequantChannel *block, int stride) {
+    each = block;
+    mult2 = reinterpret_cast<const uint32_t *>(block + stride);
+    c2lo = mult2 + stride;
+    c2hi = c2lo + stride;
+    pre = reinterpret_cast<const int32_t *>(c2hi + stride);
+    rshift = pre + stride;
+    zw = rshift + stride;
+  }
 };
 
 // ---- fp32 dequantising epilogue (dynamic-quant MatMul) ----
+struct alignas(16) DequantChannel {  // as RequantChannel
+  float wscale;  // (float)filter_scale (per-tensor is broadcast at Prepare)
+  int32_t wsum;  // sum_k w[n][k]
+  float bias;    // 0 where there is none
+  int32_t unused;
+};
 struct DequantParams {
-  const float *wscale;           // (float)filter_scale per channel (padded; per-tensor is broadcast at Prepare)
-  const float *bias;             // fp32 bias or nullptr
-  const int32_t *wsum;           // sum_k w[n][k]
+  const DequantChannel *each;
+  const float *wscale, *bias;
+  const int32_t *wsum;
   const mi_dq_params *qp_dev;    // input scale / zero point on the device, or nullptr -> use sx / zx below
   float sx;
   int32_t zx;
@@ -68,6 +94,15 @@ struct DequantParams {
   int32_t deep;  // true K
   int32_t act;
   int32_t per_row;  // input scale of row r is qp_dev[r].scale_f; the zero point is qp_dev[0].zero_point
+  int32_t has_bias;  // (adding a bias of 0 would turn -0 into 0)
+
+  static constexpr int kWordsPerChannel = 4 + 3;  // the arrays stand as those of RequantParams do
+  __host__ __device__ __forceinline__ void set_channels(const DequantChannel *block, int stride) {
+    each = block;
+    wscale = reinterpret_cast<const float *>(block + stride);
+    bias = wscale + stride;
+    wsum = reinterpret_cast<const int32_t *>(bias + stride);
+  }
 };
 
 // Packed weights: n_pad rows (output channels) of k_pad contraction bytes, zero filled past K, with row stride ldw.
@@ -83,10 +118,10 @@ struct WeightView {
   // when the handle is created (launch_block_weights).
   const int8_t *blocked;
 };
-inline int weight_row_stride(int k_pad) { return (k_pad / 256) % 2 == 0 ? k_pad + 256 : k_pad; }
+__host__ __device__ inline int weight_row_stride(int k_pad) { return (k_pad / 256) % 2 == 0 ? k_pad + 256 : k_pad; }
 
 // A: int8 activations [M][lda] (lda in bytes, multiple of 16, base 16-byte aligned, K % 16 == 0);
-// W: packed weights (above); C: [M][ldc] elements, any n and ldc >= n, any address of the element type.
+// W: packed weights (above); C: [M][ldc] elements, any n, ldc == n, any address of the element type.
 int launch_gemm_requant(const int8_t *a, int64_t lda, int m, int k, const WeightView &w, int n,
                         const RequantParams &rq, int8_t *c, int64_t ldc, hipStream_t stream);
 int launch_gemm_dequant(const int8_t *a, int64_t lda, int m, int k, const WeightView &w, int n,

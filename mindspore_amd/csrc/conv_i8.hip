@@ -16,6 +16,7 @@
 #include <string.h>
 
 #include "conv_store.h"
+#include "launch_args.h"
 
 namespace mi {
 
@@ -27,9 +28,8 @@ typedef v4i v4i_any __attribute__((aligned(1)));
 // 3.4 us for 333 x 1000, now 2.4, which is what any launch takes).  The last, partial chunk of a row is the row's last 16
 // bytes shifted down, so nothing past the tensor is read, nor anything before it.
 __global__ __launch_bounds__(256) void pad_rows_kernel(const int8_t *__restrict__ src, int64_t src_ld, int64_t total,
-                                                       int k, int8_t *__restrict__ dst, int chunks_per_row) {
-  for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
-       idx += (int64_t)gridDim.x * blockDim.x) {
+                                                       int k, int8_t *__restrict__ dst, int chunks_per_row, int threads) {
+  for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < total; idx += threads) {
     const int64_t row = total < 0x7fffffff ? (int64_t)((uint32_t)idx / (uint32_t)chunks_per_row)
                                            : idx / chunks_per_row;
     const int at = (int)(idx - row * chunks_per_row) * 16, have = k - at;
@@ -51,8 +51,8 @@ __global__ __launch_bounds__(256) void pad_rows_kernel(const int8_t *__restrict_
 
 int launch_pad_rows(const int8_t *src, int64_t src_ld, int rows, int k, int8_t *dst, int k16, hipStream_t stream) {
   const int64_t total = (int64_t)rows * (k16 >> 4), want = (total + 255) / 256;
-  hipLaunchKernelGGL(pad_rows_kernel, dim3((unsigned)(want < 1048576 ? want : 1048576)), dim3(256), 0, stream, src, src_ld,
-                     total, k, dst, k16 >> 4);
+  const int wgs = (int)(want < 1048576 ? want : 1048576);
+  hipLaunchKernelGGL(pad_rows_kernel, dim3(wgs), dim3(256), 0, stream, src, src_ld, total, k, dst, k16 >> 4, 256 * wgs);
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }
@@ -142,11 +142,15 @@ __global__ __launch_bounds__(256) void conv_smallk_kernel(const int8_t *__restri
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int nb = ob * 32 + q * 8 + h * 4;
-      prm[q][0] = *reinterpret_cast<const v4i *>(rq.mult + nb);
-      prm[q][1] = *reinterpret_cast<const v4i *>(rq.bias2 + nb);
-      prm[q][2] = *reinterpret_cast<const v4i *>(rq.rshift + nb);
-      prm[q][3] = *reinterpret_cast<const v4i *>(rq.zw + nb);
-      prm[q][4] = *reinterpret_cast<const v4i *>(rq.lshift + nb);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const RequantChannel ch = rq.each[nb + e];
+        prm[q][0][e] = ch.mult;
+        prm[q][1][e] = ch.bias2;
+        prm[q][2][e] = ch.rshift();
+        prm[q][3][e] = ch.zw;
+        prm[q][4][e] = ch.lshift();
+      }
     }
   };
   fetch_params(0);
@@ -290,18 +294,27 @@ int launch_conv_smallk(const int8_t *in, const ConvGeom &g, int fill, int k_true
 // 16 x 160 x 160 x 3 -> 64, 3x3 14.7 / 12.4 / 10.9; 16 x 224 x 224 x 4 -> 32, 5x5 20 / 16.4 / 14.8.
 struct ConvRows {
   const int8_t *in;
-  int in_bytes;
-  int in_h, in_w, in_c, out_w, out_hw, out_c;
-  int kernel_h, stride_h, stride_w, dil_h, pad_u, pad_l;
-  int parts;      // 16-byte chunks per window row: 1 or 2
-  int row_bytes;  // kernel_w * in_c
-  int fill;
-  int pixels;
-  bool streams;
   const int8_t *w;  // [out_c padded to 64][32 * KS]
+  int in_bytes;
+  int in_h, in_w, out_w, out_hw, out_c;
+  int stride_h, stride_w, dil_h;
+  // (small numbers share words and are shifted out of them: a byte of its own comes by a vector load)
+  uint32_t pads, sizes, shifts;
+  int pixels;
   uint32_t magic_hw, magic_w;  // quotients by out_hw and out_w: umulhi(2 p, magic) >> shift (see magic31)
-  int shift_hw, shift_w;
+  int step;                    // tiles that all workgroups of a channel group do at once
+  __host__ __device__ __forceinline__ int pad_u() const { return (int16_t)pads; }
+  __host__ __device__ __forceinline__ int pad_l() const { return (int)pads >> 16; }
+  __host__ __device__ __forceinline__ int in_c() const { return (int)(sizes & 0xff); }
+  __host__ __device__ __forceinline__ int kernel_h() const { return (int)(sizes >> 8 & 0xff); }
+  __host__ __device__ __forceinline__ int row_bytes() const { return (int)(sizes >> 16 & 0xff); }  // kernel_w * in_c
+  __host__ __device__ __forceinline__ uint32_t fill() const { return sizes >> 24; }
+  __host__ __device__ __forceinline__ int shift_hw() const { return (int)(shifts & 0xff); }
+  __host__ __device__ __forceinline__ int shift_w() const { return (int)(shifts >> 8 & 0xff); }
+  __host__ __device__ __forceinline__ bool streams() const { return (shifts >> 16) != 0; }
+  __host__ __device__ __forceinline__ int parts() const { return row_bytes() <= 16 ? 1 : 2; }  // 16-byte chunks per window row
 };
+static_assert(sizeof(ConvRows) + sizeof(RequantCall) + sizeof(int8_t *) <= kShortArgs, "see launch_args.h");
 
 // A tile's operand straight from the image: lane r (of each half) takes pixel 32 * tile + r.
 template <int KS>
@@ -314,34 +327,34 @@ struct RowsGather {
   bool plain;
 
   __device__ __forceinline__ RowsGather(const ConvRows &g_, int lane)
-      : g(g_), r(lane & 31), h(lane >> 5), part(g_.parts == 2 ? h : 0), line(g_.in_w * g_.in_c), last16(g_.in_bytes - 16) {}
-  __device__ __forceinline__ int window_row(int s) const { return g.parts == 2 ? s : 2 * s + h; }
+      : g(g_), r(lane & 31), h(lane >> 5), part(g_.parts() == 2 ? h : 0), line(g_.in_w * g_.in_c()), last16(g_.in_bytes - 16) {}
+  __device__ __forceinline__ int window_row(int s) const { return g.parts() == 2 ? s : 2 * s + h; }
   __device__ __forceinline__ void locate(int tile) {
     const int want = tile * 32 + r, p = want < g.pixels ? want : g.pixels - 1;
-    const int b = quotient31(p, g.magic_hw, g.shift_hw), rem = p - b * g.out_hw;
-    const int oh = quotient31(rem, g.magic_w, g.shift_w), ow = rem - oh * g.out_w;
+    const int b = quotient31(p, g.magic_hw, g.shift_hw()), rem = p - b * g.out_hw;
+    const int oh = quotient31(rem, g.magic_w, g.shift_w()), ow = rem - oh * g.out_w;
     img = b * (g.in_h * line);
-    ih0 = oh * g.stride_h - g.pad_u;
-    t0 = (ow * g.stride_w - g.pad_l) * g.in_c + 16 * part;
-    const int from = t0 - 16 * part, to_last = (g.parts == 2 ? KS - 1 : 2 * KS - 1) * g.dil_h;
-    plain = __all(ih0 >= 0 && ih0 + to_last < g.in_h && from >= 0 && from + g.row_bytes <= line &&
+    ih0 = oh * g.stride_h - g.pad_u();
+    t0 = (ow * g.stride_w - g.pad_l()) * g.in_c() + 16 * part;
+    const int from = t0 - 16 * part, to_last = (g.parts() == 2 ? KS - 1 : 2 * KS - 1) * g.dil_h;
+    plain = __all(ih0 >= 0 && ih0 + to_last < g.in_h && from >= 0 && from + g.row_bytes() <= line &&
                   (uint32_t)img + (uint32_t)(ih0 + to_last) * (uint32_t)line + (uint32_t)t0 <= (uint32_t)last16);
   }
   // Every load is a whole 16 bytes inside the tensor: rows above or below the image are clamped (their bytes are
   // replaced), and an address before its first or behind its last 16 bytes is moved in.
   __device__ __forceinline__ int address(int s) const {
     int kh = window_row(s);
-    kh = kh < g.kernel_h ? kh : g.kernel_h - 1;
+    kh = kh < g.kernel_h() ? kh : g.kernel_h() - 1;
     const int ih = min(max(ih0 + kh * g.dil_h, 0), g.in_h - 1);
     return img + ih * line + t0;
   }
   __device__ __forceinline__ void fetch(v4i (&x)[KS]) const {
     if (plain) {
       const int row_step = g.dil_h * line;
-      const uint32_t lane_off = (uint32_t)(img + ih0 * line + t0 + (g.parts == 2 ? 0 : h * row_step));
+      const uint32_t lane_off = (uint32_t)(img + ih0 * line + t0 + (g.parts() == 2 ? 0 : h * row_step));
       const int8_t *row = g.in;
 #pragma unroll
-      for (int s = 0; s < KS; ++s, row += g.parts == 2 ? row_step : 2 * row_step)
+      for (int s = 0; s < KS; ++s, row += g.parts() == 2 ? row_step : 2 * row_step)
         x[s] = *reinterpret_cast<const v4i_any *>(row + lane_off);
       return;
     }
@@ -362,10 +375,10 @@ struct RowsGather {
         }
       }
     }
-    const uint32_t fill4 = (uint32_t)(g.fill & 0xff) * 0x01010101u;
+    const uint32_t fill4 = g.fill() * 0x01010101u;
     uint32_t in_row[4];
     row_mask(t0, line, in_row);
-    const bool rows_inside = ih0 >= 0 && ih0 + (g.kernel_h - 1) * g.dil_h < g.in_h;
+    const bool rows_inside = ih0 >= 0 && ih0 + (g.kernel_h() - 1) * g.dil_h < g.in_h;
     if (__all(rows_inside)) {
 #pragma unroll
       for (int s = 0; s < KS; ++s)
@@ -409,7 +422,7 @@ struct RowsStore {
     wait_for_products(acc);
     int8_t *tile_out = out + (int64_t)tile * 32 * g.out_c;
     // (no branch between the pieces of a whole tile: one's chain of dependent instructions fills the gaps of the next)
-    requant.in_form(tile * 32 + 32 <= g.pixels, n0, my_n, g.out_c, g.streams, [&](auto kind, auto streamed) {
+    requant.in_form(tile * 32 + 32 <= g.pixels, n0, my_n, g.out_c, g.streams(), [&](auto kind, auto streamed) {
 #pragma unroll
       for (int q = 0; q < 4; ++q)
         // (the transposition needs every lane: those whose pixel is not there store none of their channels)
@@ -434,10 +447,11 @@ constexpr int rows_occupancy(int ks, int ocb, RequantForm form) { return form !=
 
 template <int KS, int OCB, RequantForm FORM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(rows_occupancy(KS, OCB, FORM)))) void conv_rows_kernel(
-    ConvRows g, RequantParams rq, int8_t *__restrict__ out) {
+    ConvRows g, RequantCall call, int8_t *__restrict__ out) {
+  const RequantParams rq = call.open(g.out_c);
   const int lane = threadIdx.x & 63;
   const int n0 = blockIdx.y * (32 * OCB);
-  const int tiles = (g.pixels + 31) >> 5, step = gridDim.x * 4;
+  const int tiles = (g.pixels + 31) >> 5, step = g.step;
   int tile = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (tile >= tiles) return;
 
@@ -468,7 +482,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(rows_occupa
         v4i one;
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
-          const int b = in.window_row(s) < g.kernel_h ? min(max(g.row_bytes - 16 * in.part - 4 * d, 0), 4) : 0;
+          const int b = in.window_row(s) < g.kernel_h() ? min(max(g.row_bytes() - 16 * in.part - 4 * d, 0), 4) : 0;
           one[d] = (int)(0x01010101u & (uint32_t)(((uint64_t)1 << (8 * b)) - 1));
         }
         sums = __builtin_amdgcn_mfma_i32_32x32x32_i8(x[s], one, sums, 0, 0, 0);
@@ -486,7 +500,7 @@ bool conv_rows_supported(const ConvGeom &g) {
   const int row = g.kernel_w * g.in_c, parts = row <= 16 ? 1 : 2;
   const int64_t bytes = (int64_t)g.batch * g.in_h * g.in_w * g.in_c;
   return (g.in_c & 15) != 0 && g.dilation_w == 1 && row <= 32 && (g.kernel_h * parts + 1) / 2 <= kConvRowsSteps &&
-         bytes >= 16 && bytes < (int64_t)1 << 31;
+         bytes >= 16 && bytes < (int64_t)1 << 31 && g.pad_u == (int16_t)g.pad_u && g.pad_l == (int16_t)g.pad_l;
 }
 
 // Weights [oc][kh][kw][ic] -> [oc padded to 64][steps of 32 bytes], see ConvRows.
@@ -504,24 +518,22 @@ int launch_conv_rows(const int8_t *in, const ConvGeom &g, int fill, const int8_t
   ConvRows c{};
   c.in = in;
   c.in_bytes = g.batch * g.in_h * g.in_w * g.in_c;
-  c.in_h = g.in_h, c.in_w = g.in_w, c.in_c = g.in_c;
+  c.in_h = g.in_h, c.in_w = g.in_w;
   c.out_w = g.out_w, c.out_hw = g.out_h * g.out_w, c.out_c = g.out_c;
-  c.kernel_h = g.kernel_h, c.stride_h = g.stride_h, c.stride_w = g.stride_w, c.dil_h = g.dilation_h;
-  c.pad_u = g.pad_u, c.pad_l = g.pad_l;
-  c.row_bytes = g.kernel_w * g.in_c;
-  c.parts = c.row_bytes <= 16 ? 1 : 2;
-  c.fill = fill;
+  c.stride_h = g.stride_h, c.stride_w = g.stride_w, c.dil_h = g.dilation_h;
+  c.pads = (uint32_t)(uint16_t)g.pad_u | (uint32_t)g.pad_l << 16;
+  c.sizes = (uint32_t)g.in_c | (uint32_t)g.kernel_h << 8 | (uint32_t)(g.kernel_w * g.in_c) << 16 | (uint32_t)(uint8_t)fill << 24;
   const int64_t pixels = (int64_t)g.batch * g.out_h * g.out_w;
   c.pixels = (int)pixels;
   c.w = w;
-  const int ks = (c.kernel_h * c.parts + 1) / 2;
+  const int ks = (c.kernel_h() * c.parts() + 1) / 2;
   if (!conv_rows_supported(g) || pixels < 1 || pixels > 0x7fffffff - 4096) {
     set_error("conv_rows: unsupported geometry ic=%d kernel %dx%d", g.in_c, g.kernel_h, g.kernel_w);
     return MI_PARAM_INVALID;
   }
   const int64_t wgs = (pixels + 127) / 128;
   const bool two = g.out_c > 32;
-  c.streams = conv_streams(pixels, g.out_c, two ? 2 : 1);
+  const bool streams = conv_streams(pixels, g.out_c, two ? 2 : 1);
   const RequantForm form = requant_form(rq);
   const int gy = (g.out_c + (two ? 63 : 31)) / (two ? 64 : 32);
   // as many workgroups as the registers let the device hold, so that a wave walks several tiles on one set of weights.  us at
@@ -529,11 +541,14 @@ int launch_conv_rows(const int8_t *in, const ConvGeom &g, int fill, const int8_t
   // 512 5.95, 768 5.65
   const int most = 256 * rows_occupancy(ks, two ? 2 : 1, form);
   const dim3 grid((unsigned)(wgs < most ? wgs : most), (unsigned)gy);
-  magic31(c.out_hw, &c.magic_hw, &c.shift_hw);
-  magic31(c.out_w, &c.magic_w, &c.shift_w);
+  int shift_hw, shift_w;
+  magic31(c.out_hw, &c.magic_hw, &shift_hw);
+  magic31(c.out_w, &c.magic_w, &shift_w);
+  c.shifts = (uint32_t)shift_hw | (uint32_t)shift_w << 8 | (streams ? 1u << 16 : 0u);
+  c.step = 4 * (int)grid.x;
 #define MI_ROWS_FORM(KS, FORM)                                                                              \
-  if (two) hipLaunchKernelGGL((conv_rows_kernel<KS, 2, FORM>), grid, dim3(256), 0, stream, c, rq, out);      \
-  else hipLaunchKernelGGL((conv_rows_kernel<KS, 1, FORM>), grid, dim3(256), 0, stream, c, rq, out)
+  if (two) hipLaunchKernelGGL((conv_rows_kernel<KS, 2, FORM>), grid, dim3(256), 0, stream, c, RequantCall::of(rq), out);      \
+  else hipLaunchKernelGGL((conv_rows_kernel<KS, 1, FORM>), grid, dim3(256), 0, stream, c, RequantCall::of(rq), out)
 #define MI_ROWS(KS)                     \
   case KS:                              \
     if (form == kReluForm) {            \
@@ -581,6 +596,7 @@ struct ConvDwRows {
   int total;                  // batch * bands * strips * groups
   int zsplat, amin, amax;
 };
+static_assert(sizeof(ConvDwRows) <= kShortArgs, "see launch_args.h");
 
 // Outputs of up to kStreamedMost bytes are stored non-temporally (STREAMED) from this many channels, where a pixel's are at least a
 // line; half as many bytes where pixels begin inside a line's 32-byte sectors, which two stores then share.  us, temporal -> streamed:
@@ -597,7 +613,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
   constexpr int WR = KS == 3 ? 1 : 3;  // weight dwords per channel and window row
   // as below: workgroups that share an XCD get one contiguous band of the output
   int bid = blockIdx.x;
-  const int per = gridDim.x >> 3;
+  const int per = ((g.total + 255) >> 8) >> 3;  // an eighth of the grid
   if (bid < per * 8) bid = (bid & 7) * per + (bid >> 3);
   const int idx = bid * 256 + threadIdx.x;
   if (idx >= g.total) return;
@@ -824,7 +840,8 @@ __global__ __launch_bounds__(256) void conv_dw_kernel(const int8_t *__restrict__
         acc += (uint32_t)((int32_t)xv * (int32_t)wv);
       }
     }
-    const int32_t mult = rq.mult[c], e = rq.rshift[c], ls = rq.lshift[c];
+    const RequantChannel ch = rq.each[c];
+    const int32_t mult = ch.mult, e = ch.rshift(), ls = ch.lshift();
     int32_t y = rdiv_pot(srdhm((int32_t)(acc << ls), mult), e);
     y = (int32_t)((uint32_t)y + (uint32_t)rq.zo);
     y = y > rq.amin ? y : rq.amin;  // MSMAX first, then MSMIN (conv_depthwise_int8.c:49-50)
@@ -956,17 +973,17 @@ __global__ __launch_bounds__(256) void conv_dw16_kernel(const int8_t *__restrict
     } o;
 #pragma unroll
     for (int q = 0; q < CG / 4; ++q) {
-      const v4i m4 = *reinterpret_cast<const v4i *>(rq.mult + c0 + 4 * q);
-      const v4i rs4 = *reinterpret_cast<const v4i *>(rq.rshift + c0 + 4 * q);
-      v4i ls4 = {0, 0, 0, 0};
-      if (!FAST) ls4 = *reinterpret_cast<const v4i *>(rq.lshift + c0 + 4 * q);
+      RequantChannel of[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) of[e] = rq.each[c0 + 4 * q + e];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
+        const int32_t mult = of[e].mult, shift = of[e].rshift();
         int32_t y;
         if (FAST) {
-          y = rdiv_pot_fast(srdhm_nosat((int32_t)acc[4 * q + e], m4[e]), rs4[e], (1 << rs4[e]) >> 1);
+          y = rdiv_pot_fast(srdhm_nosat((int32_t)acc[4 * q + e], mult), shift, (1 << shift) >> 1);
         } else {
-          y = rdiv_pot(srdhm((int32_t)(acc[4 * q + e] << ls4[e]), m4[e]), rs4[e]);
+          y = rdiv_pot(srdhm((int32_t)(acc[4 * q + e] << of[e].lshift()), mult), shift);
         }
         y = (int32_t)((uint32_t)y + (uint32_t)rq.zo);
         y = y > rq.amin ? y : rq.amin;  // MSMAX first, then MSMIN (conv_depthwise_int8.c:49-50)

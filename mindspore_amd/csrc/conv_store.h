@@ -96,10 +96,11 @@ struct ChannelRequant {
       const int n = n0 + column_channel(OCB, ob, lane & 31, NEIGHBOURS);  // (the arrays are padded to a multiple of 256 channels)
       shift[ob] = rq.rshift[n];
       if (FORM == kGeneralForm) {
-        mult[ob] = rq.mult[n];
-        bias[ob] = (int32_t)((uint32_t)rq.bias2[n] - kAccBias);
-        lsh[ob] = rq.lshift[n];
-        zw[ob] = rq.zw[n];
+        const RequantChannel ch = rq.each[n];
+        mult[ob] = ch.mult;
+        bias[ob] = (int32_t)((uint32_t)ch.bias2 - kAccBias);
+        lsh[ob] = ch.lshift();
+        zw[ob] = ch.zw;
       } else {
         mult[ob] = (int32_t)rq.mult2[n];
         bias[ob] = rq.pre[n];

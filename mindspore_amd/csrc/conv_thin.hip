@@ -5,6 +5,7 @@
 #include <type_traits>
 
 #include "conv_store.h"
+#include "launch_args.h"
 
 namespace mi {
 
@@ -29,16 +30,19 @@ struct ConvThin {
   int chunks;  // of CH steps; weights are zero from k on
   int out_c, pixels;
   bool streams;
+  int step;         // tiles that all workgroups of a channel group do at once
   const int8_t *w;  // [32 channels][step][lane][16]
 };
+static_assert(sizeof(ConvThin) + sizeof(RequantCall) + sizeof(int8_t *) <= kShortArgs, "see launch_args.h");
 
 template <int CH, int OCB, RequantForm FORM, bool NEIGHBOURS = true>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void conv_thin_kernel(ConvThin g, RequantParams rq,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void conv_thin_kernel(ConvThin g, RequantCall call,
                                                                                               int8_t *__restrict__ out) {
+  const RequantParams rq = call.open(g.out_c);
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5;
   const int n0 = blockIdx.y * (32 * OCB);
-  const int tiles = (g.pixels + 31) >> 5, step = gridDim.x * 4;
+  const int tiles = (g.pixels + 31) >> 5, step = g.step;
   int tile = blockIdx.x * 4 + (tid >> 6);
   const int steps = g.chunks * CH;
 
@@ -202,20 +206,20 @@ static int launch_thin(const ConvThin &c, const RequantParams &rq, int8_t *out, 
   if constexpr (OCB == 2) {
     if (form != kGeneralForm && c.out_c == 256) {
       if (form == kReluForm) {
-        hipLaunchKernelGGL((conv_thin_kernel<CH, OCB, kReluForm, false>), grid, dim3(256), lds, stream, c, rq, out);
+        hipLaunchKernelGGL((conv_thin_kernel<CH, OCB, kReluForm, false>), grid, dim3(256), lds, stream, c, RequantCall::of(rq), out);
       } else {
-        hipLaunchKernelGGL((conv_thin_kernel<CH, OCB, kCarryForm, false>), grid, dim3(256), lds, stream, c, rq, out);
+        hipLaunchKernelGGL((conv_thin_kernel<CH, OCB, kCarryForm, false>), grid, dim3(256), lds, stream, c, RequantCall::of(rq), out);
       }
       MI_HIP_CHECK(hipGetLastError());
       return MI_OK;
     }
   }
   if (form == kReluForm) {
-    hipLaunchKernelGGL((conv_thin_kernel<CH, OCB, kReluForm>), grid, dim3(256), lds, stream, c, rq, out);
+    hipLaunchKernelGGL((conv_thin_kernel<CH, OCB, kReluForm>), grid, dim3(256), lds, stream, c, RequantCall::of(rq), out);
   } else if (form == kCarryForm) {
-    hipLaunchKernelGGL((conv_thin_kernel<CH, OCB, kCarryForm>), grid, dim3(256), lds, stream, c, rq, out);
+    hipLaunchKernelGGL((conv_thin_kernel<CH, OCB, kCarryForm>), grid, dim3(256), lds, stream, c, RequantCall::of(rq), out);
   } else if constexpr (OCB <= 3) {
-    hipLaunchKernelGGL((conv_thin_kernel<CH, OCB, kGeneralForm>), grid, dim3(256), lds, stream, c, rq, out);
+    hipLaunchKernelGGL((conv_thin_kernel<CH, OCB, kGeneralForm>), grid, dim3(256), lds, stream, c, RequantCall::of(rq), out);
   }
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
@@ -235,10 +239,10 @@ int launch_conv_thin(const int8_t *in, int64_t pixels, int k, int oc, const int8
   // -> 160 15.3 -> 10.9; 16 x 56 x 56, 128 -> 128 6.0 -> 5.6.  Six (too few waves) 14.7 -> 22, channels short of five 10.4 -> 14.
   const bool rows = form != kGeneralForm && oc == 32 * blocks && blocks > 3 && blocks <= 5 && wgs * blocks > 1024 && t.steps() * blocks <= 64;
   const int ocb = rows ? blocks : thin_blocks(wgs, oc), groups = (oc + 32 * ocb - 1) / (32 * ocb);
-  const ConvThin c{in, pixels * k, k, t.chunks, oc, (int)pixels, conv_streams(pixels, oc, ocb), w};
   // four workgroups per CU, which the LDS allows up to 40 KiB of weights; more would only load the weights more often
   const int most = (1024 + groups - 1) / groups;
   const dim3 grid((unsigned)(wgs < most ? wgs : most), (unsigned)groups);
+  const ConvThin c{in, pixels * k, k, t.chunks, oc, (int)pixels, conv_streams(pixels, oc, ocb), 4 * (int)grid.x, w};
   const size_t lds = (size_t)t.steps() * ocb * 1024;
 #define MI_THIN(CH)                                                              \
   return ocb == 1   ? launch_thin<CH, 1>(c, rq, out, grid, lds, stream)          \

@@ -226,11 +226,11 @@ static_assert(sizeof(DqSlots) == kDqSlotBytes, "what the handle allocates and fi
 
 template <int T, int G>
 __global__ __launch_bounds__(T) void dq_fused_kernel(const float *__restrict__ x, int64_t n, int symmetric,
-                                                     DqSlots *slots, uint32_t launch, uint32_t patience, DqHostNote note,
+                                                     DqSlots *slots, uint32_t launch, uint32_t patience, int wgs, DqHostNote note,
                                                      mi_dq_params *__restrict__ params, int8_t *__restrict__ q) {
   __shared__ float slo[T / 64], shi[T / 64], all[2];
   __shared__ int late_wg;
-  const int tid = threadIdx.x, w = blockIdx.x, wgs = gridDim.x;
+  const int tid = threadIdx.x, w = blockIdx.x;  // of wgs
   const int64_t n4 = n >> 2, first = (int64_t)w * (T * G) + tid;
   const v4f_any *x4 = reinterpret_cast<const v4f_any *>(x);
   const bool counted = launch == 0;  // the number of this launch stands in memory
@@ -532,9 +532,10 @@ int launch_dynquant_segments(const float *x, int64_t segments, int64_t unit, int
 template <int T, int G>
 static void launch_fused(const float *x, int64_t n, int symmetric, void *slots, uint32_t launch, const DqHostNote &note,
                          mi_dq_params *params, int8_t *q, hipStream_t stream) {
-  const int64_t wgs = ((n >> 2) + T * G - 1) / (T * G);
-  hipLaunchKernelGGL((dq_fused_kernel<T, G>), dim3(wgs < 1 ? 1 : (unsigned)wgs), dim3(T), 0, stream, x, n, symmetric,
-                     static_cast<DqSlots *>(slots), launch, kDqPatience, note, params, q);
+  const int64_t want = ((n >> 2) + T * G - 1) / (T * G);
+  const int wgs = want < 1 ? 1 : (int)want;
+  hipLaunchKernelGGL((dq_fused_kernel<T, G>), dim3(wgs), dim3(T), 0, stream, x, n, symmetric,
+                     static_cast<DqSlots *>(slots), launch, kDqPatience, wgs, note, params, q);
 }
 
 int launch_dynquant(const float *x, int64_t n, int symmetric, float2 *partials, void *slots, uint32_t launch,

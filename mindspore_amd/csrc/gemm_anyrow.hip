@@ -146,16 +146,18 @@ __device__ __forceinline__ void gemm_anyrow_body(const GemmArgs &g, const Requan
 
 // (the LDS lets one workgroup into a CU: a wave per SIMD)
 template <int EPI, bool HAS_ZW, bool FAST>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_anyrow_kernel(GemmArgs g, RequantParams rq,
-                                                                                                     DequantParams dq) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_anyrow_kernel(GemmCall<EPI> call) {
+  GemmArgs g;
+  RequantParams rq;
+  DequantParams dq;
+  call.open(&g, &rq, &dq);
   gemm_anyrow_body<EPI, HAS_ZW, FAST>(g, rq, dq);
 }
 
 template <int EPI, bool HAS_ZW, bool FAST>
-static int launch(GemmArgs g, const RequantParams &rq, const DequantParams &dq, hipStream_t stream) {
-  g.tiles_m = (g.m + 63) / 64;
-  g.tiles_n = (g.n + 63) / 64;
-  hipLaunchKernelGGL((gemm_anyrow_kernel<EPI, HAS_ZW, FAST>), dim3(g.tiles_m * g.tiles_n), dim3(256), 0, stream, g, rq, dq);
+static int launch(const GemmArgs &g, const RequantParams &rq, const DequantParams &dq, hipStream_t stream) {
+  const auto call = GemmCall<EPI>::of(g, g.wb, 64, 64, rq, dq);
+  hipLaunchKernelGGL((gemm_anyrow_kernel<EPI, HAS_ZW, FAST>), call.grid(), dim3(256), 0, stream, call);
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }

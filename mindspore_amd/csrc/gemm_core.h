@@ -2,6 +2,7 @@
 #pragma once
 
 #include "common.h"
+#include "launch_args.h"
 #include "quant_math.h"
 #include "weight_loads.h"
 
@@ -35,6 +36,30 @@ struct GemmArgs {
   int64_t ldc;
 };
 
+// The arguments of one matrix as they travel; w: the form of the weights that the kernel reads, c: rows of n values.
+template <int EPI>
+struct GemmCall {
+  typedef std::conditional_t<EPI == EPI_REQUANT, RequantCall, DequantCall> Epi;
+  const int8_t *a, *w;
+  void *c;
+  int m, n, k, lda, tiles_m, tiles_n;
+  Epi epi;
+  static GemmCall of(const GemmArgs &g, const int8_t *w, int tile_n, int tile_m, const RequantParams &rq, const DequantParams &dq) {
+    GemmCall call{g.a, w, g.c, g.m, g.n, g.k, (int)g.lda, (g.m + tile_m - 1) / tile_m, (g.n + tile_n - 1) / tile_n, {}};
+    if constexpr (EPI == EPI_REQUANT) call.epi = RequantCall::of(rq);
+    else call.epi = DequantCall::of(dq, g.k);
+    return call;
+  }
+  dim3 grid() const { return dim3(tiles_m * tiles_n); }
+  __device__ __forceinline__ void open(GemmArgs *g, RequantParams *rq, DequantParams *dq) const {
+    const int k_pad = padded_k(k);
+    *g = GemmArgs{a, lda, m, k, w, weight_row_stride(k_pad), k_pad, w, n, tiles_m, tiles_n, c, n};
+    if constexpr (EPI == EPI_REQUANT) *rq = epi.open(n);
+    else *dq = epi.open(n, k);
+  }
+};
+static_assert(sizeof(GemmCall<EPI_REQUANT>) <= kShortArgs && sizeof(GemmCall<EPI_DEQUANT>) <= kShortArgs, "see launch_args.h");
+
 // Asynchronous 16-byte-per-lane copy global -> LDS: lane L's 16 bytes land at lds_wave_base + 16 * L;
 // lds_wave_base must be wave-uniform.  Completion is tracked by vmcnt, in issue order.
 __device__ __forceinline__ void async_copy16(const void *global_src, void *lds_wave_base) {
@@ -46,7 +71,7 @@ __device__ __forceinline__ void async_copy16(const void *global_src, void *lds_w
 // XCD are mapped to a compact block of tiles, 4 tiles tall: the CUs of one XCD then share operand panels in L2.
 __device__ __forceinline__ void tile_coords(const GemmArgs &g, int *tile_m, int *tile_n) {
   int id = blockIdx.x;
-  const int nb = gridDim.x, per = nb >> 3;
+  const int nb = g.tiles_m * g.tiles_n, per = nb >> 3;  // (nb: the grid)
   if (id < per * 8) id = (id & 7) * per + (id >> 3);
   constexpr int G = 4;
   const int width = G * g.tiles_n;
@@ -162,15 +187,16 @@ struct EpiParams {
         v[4] = rq.rshift[n];
         v[5] = rq.zw[n];
       } else if (EPI == EPI_REQUANT) {
-        v[0] = rq.mult[n];
-        v[1] = rq.bias2[n];
-        v[2] = rq.rshift[n];
-        v[3] = rq.zw[n];
-        v[4] = rq.lshift[n];
+        const RequantChannel ch = rq.each[n];
+        v[0] = ch.mult;
+        v[1] = ch.bias2;
+        v[2] = ch.rshift();
+        v[3] = ch.zw;
+        v[4] = ch.lshift();
       } else {
         v[0] = __float_as_int(dq.wscale[n]);
         v[1] = dq.wsum[n];
-        v[2] = dq.bias != nullptr ? __float_as_int(dq.bias[n]) : 0;
+        v[2] = __float_as_int(dq.bias[n]);
       }
     }
   }
@@ -485,7 +511,7 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[TN][TM], int (&rowsum)
     constexpr int kRowB = kDeqStageRowBytes;
     const int lane = h * 32 + r;
     const int lr = lane >> 3, lc = lane & 7;
-    const bool has_bias = dq.bias != nullptr;
+    const bool has_bias = dq.has_bias != 0;
     // The body exists three times, chosen once per tile instead of with branches around every output: full tile
     // without activation and with one input scale (no bounds compares, no clamps, the scale product hoisted), full
     // tile in general, ragged tile in general.

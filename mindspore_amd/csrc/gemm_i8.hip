@@ -84,14 +84,23 @@ __device__ __forceinline__ void hint_interleave_reads() {
 // image, or from 16 bytes of the fill value when the tap lies outside the image (conv_int8.c:758-807,877).
 struct ConvGather {
   int in_h, in_w, in_c, out_w, out_hw;
-  int kernel_w, stride_h, stride_w, dil_h, dil_w, pad_u, pad_l;
   uint32_t magic_ic, magic_kw;  // ceil(2^32 / in_c), ceil(2^32 / kernel_w): exact quotients for dividends < 2^16
-  const int8_t *fill16;
+  int16_t stride_h, stride_w, dil_h, dil_w, pad_u, pad_l;
+  int kernel_w;
 };
+// As GemmCall, of a convolution whose output pixels are the rows.
+struct ConvCall {
+  const int8_t *in, *w, *fill16;
+  int8_t *c;
+  int m, n, k;
+  ConvGather cv;
+  RequantCall epi;
+};
+static_assert(sizeof(ConvCall) <= kShortArgs, "see launch_args.h");
 
 template <int TILE_N, int TILE_M, int EPI, bool HAS_ZW, bool FAST, int NST, bool CONV>
 __device__ __forceinline__ void gemm_direct_body(const GemmArgs &g, const RequantParams &rq, const DequantParams &dq,
-                                                 const ConvGather &cv) {
+                                                 const ConvGather &cv, const int8_t *fill16) {
   constexpr int BKD = 64, PD = NST - 1;  // PD: prefetch distance in K steps
   static_assert(NST >= 3, "the loop keeps NST - 1 >= 2 tiles in flight");
   auto wrap = [](int x) { return x >= NST ? x - NST : x; };  // stage index after an increment of at most NST
@@ -162,7 +171,7 @@ __device__ __forceinline__ void gemm_direct_body(const GemmArgs &g, const Requan
       for (int i = 0; i < APW; ++i) {
         const int ih = ih0[i] + dh, iw = iw0[i] + dw;
         const bool inside = in_k && (unsigned)ih < (unsigned)cv.in_h && (unsigned)iw < (unsigned)cv.in_w;
-        async_copy16(inside ? asrc[i] + tap_off : cv.fill16, sa + i * 1024);
+        async_copy16(inside ? asrc[i] + tap_off : fill16, sa + i * 1024);
       }
       return;
     }
@@ -293,24 +302,30 @@ __device__ __forceinline__ void gemm_direct_body(const GemmArgs &g, const Requan
 }
 
 template <int TILE_N, int TILE_M, int EPI, bool HAS_ZW, bool FAST, int NST, int OCC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void gemm_direct_kernel(GemmArgs g, RequantParams rq, DequantParams dq) {
-  gemm_direct_body<TILE_N, TILE_M, EPI, HAS_ZW, FAST, NST, false>(g, rq, dq, ConvGather{});
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void gemm_direct_kernel(GemmCall<EPI> call) {
+  GemmArgs g;
+  RequantParams rq;
+  DequantParams dq;
+  call.open(&g, &rq, &dq);
+  gemm_direct_body<TILE_N, TILE_M, EPI, HAS_ZW, FAST, NST, false>(g, rq, dq, ConvGather{}, nullptr);
 }
 
 // The same GEMM with the activation operand gathered from an NHWC image (no im2col buffer).
 template <int TILE_N, int TILE_M, bool HAS_ZW, bool FAST, int NST, int OCC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void gemm_conv_kernel(GemmArgs g, ConvGather cv, RequantParams rq) {
-  gemm_direct_body<TILE_N, TILE_M, EPI_REQUANT, HAS_ZW, FAST, NST, true>(g, rq, DequantParams{}, cv);
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void gemm_conv_kernel(ConvCall call) {
+  const int k_pad = padded_k(call.k);
+  const GemmArgs g{call.in, 0, call.m, call.k, call.w, weight_row_stride(k_pad), k_pad, nullptr, call.n,
+                   (call.m + TILE_M - 1) / TILE_M, (call.n + TILE_N - 1) / TILE_N, call.c, call.n};
+  gemm_direct_body<TILE_N, TILE_M, EPI_REQUANT, HAS_ZW, FAST, NST, true>(g, call.epi.open(call.n), DequantParams{}, call.cv,
+                                                                         call.fill16);
 }
 
 // ---- host side -----------------------------------------------------------------------------------------------
 template <int TILE_N, int TILE_M, int EPI, bool HAS_ZW, bool FAST, int NST = 4, int OCC = 1>
-static int launch_cfg(GemmArgs g, const RequantParams &rq, const DequantParams &dq, hipStream_t stream) {
-  g.tiles_m = (g.m + TILE_M - 1) / TILE_M;
-  g.tiles_n = (g.n + TILE_N - 1) / TILE_N;
-  const int blocks = g.tiles_m * g.tiles_n;
+static int launch_cfg(const GemmArgs &g, const RequantParams &rq, const DequantParams &dq, hipStream_t stream) {
+  const auto call = GemmCall<EPI>::of(g, g.w, TILE_N, TILE_M, rq, dq);
   auto kern = gemm_direct_kernel<TILE_N, TILE_M, EPI, HAS_ZW, FAST, NST, OCC>;
-  hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, stream, g, rq, dq);
+  hipLaunchKernelGGL(kern, call.grid(), dim3(256), 0, stream, call);
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }
@@ -441,8 +456,9 @@ static int check_args(const int8_t *a, int64_t lda, int m, int k, const WeightVi
     set_error("gemm: null pointer");
     return MI_NULL_PTR;
   }
-  if (m <= 0 || n <= 0 || k <= 0 || (k & 15) != 0 || (lda & 15) != 0 || lda < k || k_pad % kKPad != 0 || k_pad < k ||
-      wv.ldw < k_pad || (wv.ldw & 15) != 0 || (reinterpret_cast<uintptr_t>(a) & 15) != 0 || ldc < n) {
+  // (k_pad, ldw and ldc are not handed on: the kernels know them, see GemmCall)
+  if (m <= 0 || n <= 0 || k <= 0 || (k & 15) != 0 || (lda & 15) != 0 || lda < k || lda > 0x7fffffff || k_pad != round_up(k, kKPad) ||
+      wv.ldw != weight_row_stride(k_pad) || (reinterpret_cast<uintptr_t>(a) & 15) != 0 || ldc != n) {
     set_error("gemm: unsupported operand geometry m=%d n=%d k=%d lda=%lld k_pad=%d ldc=%lld", m, n, k, (long long)lda,
               k_pad, (long long)ldc);
     return MI_PARAM_INVALID;
@@ -465,18 +481,15 @@ int launch_gemm_requant(const int8_t *a, int64_t lda, int m, int k, const Weight
 }
 
 template <int TILE_N, int TILE_M, bool HAS_ZW, bool FAST, int NST, int OCC>
-static int launch_conv_cfg(GemmArgs g, const ConvGather &cv, const RequantParams &rq, hipStream_t stream) {
-  g.tiles_m = (g.m + TILE_M - 1) / TILE_M;
-  g.tiles_n = (g.n + TILE_N - 1) / TILE_N;
+static int launch_conv_cfg(const ConvCall &call, hipStream_t stream) {
   auto kern = gemm_conv_kernel<TILE_N, TILE_M, HAS_ZW, FAST, NST, OCC>;
-  hipLaunchKernelGGL(kern, dim3(g.tiles_m * g.tiles_n), dim3(256), 0, stream, g, cv, rq);
+  hipLaunchKernelGGL(kern, dim3((call.m + TILE_M - 1) / TILE_M * ((call.n + TILE_N - 1) / TILE_N)), dim3(256), 0, stream, call);
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }
 
 template <bool HAS_ZW, bool FAST>
-static int launch_conv_pick_tile(const GemmArgs &g, const ConvGather &cv, const RequantParams &rq,
-                                 hipStream_t stream) {
+static int launch_conv_pick_tile(const ConvCall &g, hipStream_t stream) {
   const int64_t tiles_m = (int64_t)((g.m + 127) / 128) * ((g.n + 127) / 128);
   // 64 x 64 tiles, four workgroups per CU (an allocation of 132 registers let in three, of which the second round was often
   // next to empty): a step's gathered loads take longer than its products, and what hides them is other workgroups.  us per
@@ -495,16 +508,18 @@ static int launch_conv_pick_tile(const GemmArgs &g, const ConvGather &cv, const 
   // 0.92), K = 288 0.98 0.93, stride 2 1.01 1.06, K = 576 0.89 0.88, stride 2 0.93 1.01; at 900 rows 1x1 with K = 64 1.08.
   // 128 x 128 tiles against more channels as soon as there are enough of them (32 x 28 x 28, 64 -> 128 7.2, on 64 x 64 9.1).
   const int64_t rows = (g.m + 127) / 128;
-  const bool full_last_round = (rows - 1) % 1024 >= 768 && g.k >= (g.n <= 32 ? 144 : 288 * cv.stride_w);
+  const bool full_last_round = (rows - 1) % 1024 >= 768 && g.k >= (g.n <= 32 ? 144 : 288 * g.cv.stride_w);
   const bool many_rounds = rows >= 1400 && rows * g.k >= 1300000;
-  if (g.n <= 64 && (full_last_round || many_rounds)) return launch_conv_cfg<64, 256, HAS_ZW, FAST, 4, 2>(g, cv, rq, stream);
-  if (g.n > 64 && tiles_m >= 128) return launch_conv_cfg<128, 128, HAS_ZW, FAST, 4, 2>(g, cv, rq, stream);
-  return launch_conv_cfg<64, 64, HAS_ZW, FAST, 4, 4>(g, cv, rq, stream);
+  if (g.n <= 64 && (full_last_round || many_rounds)) return launch_conv_cfg<64, 256, HAS_ZW, FAST, 4, 2>(g, stream);
+  if (g.n > 64 && tiles_m >= 128) return launch_conv_cfg<128, 128, HAS_ZW, FAST, 4, 2>(g, stream);
+  return launch_conv_cfg<64, 64, HAS_ZW, FAST, 4, 4>(g, stream);
 }
 
 bool gemm_conv_supported(const ConvGeom &cg, const void *in) {
   const int64_t k = (int64_t)cg.kernel_h * cg.kernel_w * cg.in_c;
-  return (cg.in_c & 15) == 0 && k <= 65536 - 128 && (int64_t)cg.in_h * cg.in_w * cg.in_c < ((int64_t)1 << 31) &&
+  const auto fits = [](int x) { return x == (int16_t)x; };
+  return fits(cg.stride_h) && fits(cg.stride_w) && fits(cg.dilation_h) && fits(cg.dilation_w) && fits(cg.pad_u) && fits(cg.pad_l) &&
+         (cg.in_c & 15) == 0 && k <= 65536 - 128 && (int64_t)cg.in_h * cg.in_w * cg.in_c < ((int64_t)1 << 31) &&
          (int64_t)cg.batch * cg.out_h * cg.out_w < ((int64_t)1 << 31) && (reinterpret_cast<uintptr_t>(in) & 15) == 0;
 }
 
@@ -516,23 +531,22 @@ int launch_gemm_conv_requant(const int8_t *in, const ConvGeom &cg, const int8_t 
     set_error("gemm_conv: null pointer");
     return MI_NULL_PTR;
   }
-  if (!gemm_conv_supported(cg, in) || m64 <= 0 || cg.out_c <= 0 || w.k_pad % kKPad != 0 || w.k_pad < k64 ||
-      w.ldw < w.k_pad || (w.ldw & 15) != 0) {
+  if (!gemm_conv_supported(cg, in) || m64 <= 0 || cg.out_c <= 0 || w.k_pad != round_up((int)k64, kKPad) ||
+      w.ldw != weight_row_stride(w.k_pad)) {
     set_error("gemm_conv: unsupported geometry ic=%d k=%lld pixels=%lld oc=%d", cg.in_c, (long long)k64,
               (long long)m64, cg.out_c);
     return MI_PARAM_INVALID;
   }
   const auto magic = [](int d) { return d <= 1 ? 0u : (uint32_t)((((uint64_t)1 << 32) + d - 1) / (uint64_t)d); };
-  ConvGather cv{cg.in_h,     cg.in_w,       cg.in_c,       cg.out_w,  cg.out_h * cg.out_w, cg.kernel_w, cg.stride_h,
-                cg.stride_w, cg.dilation_h, cg.dilation_w, cg.pad_u,  cg.pad_l,            magic(cg.in_c),
-                magic(cg.kernel_w), fill16};
-  GemmArgs g{in, 0, (int)m64, (int)k64, w.w, w.ldw, w.k_pad, nullptr, cg.out_c, 0, 0, out, cg.out_c};
+  const ConvCall call{in, w.w, fill16, out, (int)m64, cg.out_c, (int)k64,
+                      ConvGather{cg.in_h, cg.in_w, cg.in_c, cg.out_w, cg.out_h * cg.out_w, magic(cg.in_c), magic(cg.kernel_w),
+                                 (int16_t)cg.stride_h, (int16_t)cg.stride_w, (int16_t)cg.dilation_h, (int16_t)cg.dilation_w,
+                                 (int16_t)cg.pad_u, (int16_t)cg.pad_l, cg.kernel_w},
+                      RequantCall::of(rq)};
   if (rq.has_zw) {
-    return rq.fast2 ? launch_conv_pick_tile<true, true>(g, cv, rq, stream)
-                    : launch_conv_pick_tile<true, false>(g, cv, rq, stream);
+    return rq.fast2 ? launch_conv_pick_tile<true, true>(call, stream) : launch_conv_pick_tile<true, false>(call, stream);
   }
-  return rq.fast2 ? launch_conv_pick_tile<false, true>(g, cv, rq, stream)
-                  : launch_conv_pick_tile<false, false>(g, cv, rq, stream);
+  return rq.fast2 ? launch_conv_pick_tile<false, true>(call, stream) : launch_conv_pick_tile<false, false>(call, stream);
 }
 
 int launch_gemm_dequant(const int8_t *a, int64_t lda, int m, int k, const WeightView &w, int n,
@@ -569,7 +583,7 @@ static int anyrow_args(const int8_t *a, int m, int k, const WeightView &w, int n
     set_error("gemm: null pointer");
     return MI_NULL_PTR;
   }
-  if (m <= 0 || n <= 0 || !gemm_anyrow_takes(m, k, w, n) || w.k_pad % kKPad != 0 || w.k_pad < k) {
+  if (m <= 0 || n <= 0 || !gemm_anyrow_takes(m, k, w, n) || w.k_pad != round_up(k, kKPad)) {
     set_error("gemm: unsupported operand geometry m=%d n=%d k=%d k_pad=%d", m, n, k, w.k_pad);
     return MI_PARAM_INVALID;
   }

@@ -309,7 +309,11 @@ constexpr int kblock_occupancy() {
 template <int TN, int TM, int EPI, bool HAS_ZW, bool FAST, bool WB>
 __global__ __launch_bounds__(256)
     __attribute__((amdgpu_waves_per_eu(kblock_occupancy<TN, TM>(), kblock_occupancy<TN, TM>()))) void gemm_kblock_kernel(
-        GemmArgs g, RequantParams rq, DequantParams dq) {
+        GemmCall<EPI> call) {
+  GemmArgs g;
+  RequantParams rq;
+  DequantParams dq;
+  call.open(&g, &rq, &dq);
   int tile_m, tile_n;
   tile_coords(g, &tile_m, &tile_n);
   gemm_kblock_body<TN, TM, EPI, HAS_ZW, FAST, WB>(g, rq, dq, tile_m, tile_n);
@@ -340,14 +344,12 @@ __global__ __launch_bounds__(256)
 }
 
 template <int TN, int TM, int EPI, bool HAS_ZW, bool FAST>
-static int launch_kblock(GemmArgs g, const RequantParams &rq, const DequantParams &dq, hipStream_t stream) {
-  g.tiles_m = (g.m + 64 * TM - 1) / (64 * TM);
-  g.tiles_n = (g.n + 64 * TN - 1) / (64 * TN);
-  const dim3 grid(g.tiles_m * g.tiles_n);
+static int launch_kblock(const GemmArgs &g, const RequantParams &rq, const DequantParams &dq, hipStream_t stream) {
+  const auto call = GemmCall<EPI>::of(g, g.wb != nullptr ? g.wb : g.w, 64 * TN, 64 * TM, rq, dq);
   if (g.wb != nullptr) {
-    hipLaunchKernelGGL((gemm_kblock_kernel<TN, TM, EPI, HAS_ZW, FAST, true>), grid, dim3(256), 0, stream, g, rq, dq);
+    hipLaunchKernelGGL((gemm_kblock_kernel<TN, TM, EPI, HAS_ZW, FAST, true>), call.grid(), dim3(256), 0, stream, call);
   } else if constexpr (TN == TM) {
-    hipLaunchKernelGGL((gemm_kblock_kernel<TN, TM, EPI, HAS_ZW, FAST, false>), grid, dim3(256), 0, stream, g, rq, dq);
+    hipLaunchKernelGGL((gemm_kblock_kernel<TN, TM, EPI, HAS_ZW, FAST, false>), call.grid(), dim3(256), 0, stream, call);
   } else {  // (rectangular tiles are chosen for the blocked copy only)
     set_error("gemm: the blocked weight copy is missing");
     return MI_NULL_PTR;

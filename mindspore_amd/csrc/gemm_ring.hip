@@ -231,7 +231,11 @@ constexpr int ring_occupancy() {
 template <int TN, int TM, int S, int EPI, bool HAS_ZW, bool FAST, bool STREAM>
 __global__ __launch_bounds__(256)
     __attribute__((amdgpu_waves_per_eu(ring_occupancy<TN, TM, S>(), ring_occupancy<TN, TM, S>()))) void gemm_ring_kernel(
-        GemmArgs g, RequantParams rq, DequantParams dq) {
+        GemmCall<EPI> call) {
+  GemmArgs g;
+  RequantParams rq;
+  DequantParams dq;
+  call.open(&g, &rq, &dq);
   int tile_m, tile_n;
   tile_coords(g, &tile_m, &tile_n);
   gemm_ring_body<TN, TM, S, EPI, HAS_ZW, FAST, STREAM>(g, rq, dq, tile_m, tile_n);
@@ -269,14 +273,12 @@ __global__ __launch_bounds__(256)
 constexpr int kStreamRowTiles = 2;
 
 template <int TN, int TM, int S, int EPI, bool HAS_ZW, bool FAST>
-static int launch_ring(GemmArgs g, const RequantParams &rq, const DequantParams &dq, hipStream_t stream) {
-  g.tiles_m = (g.m + 64 * TM - 1) / (64 * TM);
-  g.tiles_n = (g.n + 64 * TN - 1) / (64 * TN);
-  const dim3 grid(g.tiles_m * g.tiles_n);
-  if (g.tiles_m <= kStreamRowTiles) {
-    hipLaunchKernelGGL((gemm_ring_kernel<TN, TM, S, EPI, HAS_ZW, FAST, true>), grid, dim3(256), 0, stream, g, rq, dq);
+static int launch_ring(const GemmArgs &g, const RequantParams &rq, const DequantParams &dq, hipStream_t stream) {
+  const auto call = GemmCall<EPI>::of(g, g.wb, 64 * TN, 64 * TM, rq, dq);
+  if (call.tiles_m <= kStreamRowTiles) {
+    hipLaunchKernelGGL((gemm_ring_kernel<TN, TM, S, EPI, HAS_ZW, FAST, true>), call.grid(), dim3(256), 0, stream, call);
   } else {
-    hipLaunchKernelGGL((gemm_ring_kernel<TN, TM, S, EPI, HAS_ZW, FAST, false>), grid, dim3(256), 0, stream, g, rq, dq);
+    hipLaunchKernelGGL((gemm_ring_kernel<TN, TM, S, EPI, HAS_ZW, FAST, false>), call.grid(), dim3(256), 0, stream, call);
   }
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;

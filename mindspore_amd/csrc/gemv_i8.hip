@@ -11,11 +11,13 @@
 //     rows go through LDS.
 // Arithmetic reference: MatmulInt8Opt, mindspore/ccsrc/plugin/device/cpu/kernel/nnacl/int8/matmul_int8.c:296-331.
 #include "common.h"
+#include "launch_args.h"
 #include "quant_math.h"
+
+#include <limits.h>
 
 #include <algorithm>
 #include <type_traits>
-
 
 namespace mi {
 
@@ -51,6 +53,30 @@ struct GemvArgs {
   int8_t *c;
   int64_t ldc;
 };
+
+// The arguments of one matrix, and of N that share their rows, as they travel (see launch_args.h).
+template <bool DEQ>
+struct GemvCall {
+  typedef std::conditional_t<DEQ, DequantCall, RequantCall> Epi;
+  const int8_t *a, *w;
+  int8_t *c;
+  int lda, ldw, kchunks, n, m;
+  Epi epi;
+  template <typename P>
+  static GemvCall of(const GemvArgs &g, int m, const P &p) {
+    GemvCall call{g.a, g.w, g.c, (int)g.lda, g.ldw, g.kchunks, g.n, m, {}};
+    if constexpr (DEQ) call.epi = DequantCall::of(p, 16 * g.kchunks);
+    else call.epi = RequantCall::of(p);
+    return call;
+  }
+  template <typename P>
+  __device__ __forceinline__ void open(GemvArgs *g, P *p) const {
+    *g = GemvArgs{a, lda, kchunks, w, ldw, padded_k(16 * kchunks), n, c, n};
+    if constexpr (DEQ) *p = epi.open(n, 16 * kchunks);
+    else *p = epi.open(n);
+  }
+};
+static_assert(sizeof(GemvCall<false>) <= kShortArgs && sizeof(GemvCall<true>) <= kShortArgs, "see launch_args.h");
 
 // One wave owns R consecutive output channels and walks its R x K weight bytes as a stream of 1 KiB chunks
 // (chunk c = K segment c / R of row c % R, so one activation fragment serves R consecutive chunks).  D chunks are
@@ -102,26 +128,27 @@ __device__ __forceinline__ void gemv_i8_body(const GemvArgs &g, const RequantPar
   int32_t p_mult = 0, p_e = 0, p_ls = 0, p_bias2 = 0, p_zw = 0, d_wsum = 0, d_zx = 0;
   float d_ws = 0.0f, d_bias = 0.0f, d_sx = 0.0f;
   if (DEQ) {
-    d_ws = dq.wscale[my_n];
-    d_wsum = dq.wsum[my_n];
+    const DequantChannel ch = dq.each[my_n];
+    d_ws = ch.wscale;
+    d_wsum = ch.wsum;
+    d_bias = ch.bias;
     // The optional operands are fetched unconditionally, from an address that is valid either way, and selected
     // afterwards: a conditional fetch is a branch, and behind those branches the compiler waited for every outstanding
     // load after each of the activation fetches below (six round trips in a row: 4096 x 11008 at one row 10.9 us
     // against 9.0 for the requantising form of the same kernel).
     const bool on_dev = dq.qp_dev != nullptr;
-    const float *bias_or_any = dq.bias != nullptr ? dq.bias : dq.wscale;
-    const mi_dq_params *qp_or_any = on_dev ? dq.qp_dev : reinterpret_cast<const mi_dq_params *>(dq.wscale);
-    d_bias = bias_or_any[my_n];
+    const mi_dq_params *qp_or_any = on_dev ? dq.qp_dev : reinterpret_cast<const mi_dq_params *>(dq.each);
     const float sx_dev = qp_or_any[on_dev && dq.per_row && lane < R * M ? my_m : 0].scale_f;
     const int32_t zx_dev = qp_or_any->zero_point;
     d_sx = on_dev ? sx_dev : dq.sx;
     d_zx = on_dev ? zx_dev : dq.zx;
   } else {
-    p_mult = rq.mult[my_n];
-    p_e = rq.rshift[my_n];
-    p_ls = rq.lshift[my_n];
-    p_bias2 = rq.bias2[my_n];
-    p_zw = rq.zw[my_n];
+    const RequantChannel ch = rq.each[my_n];
+    p_mult = ch.mult;
+    p_e = ch.rshift();
+    p_ls = ch.lshift();
+    p_bias2 = ch.bias2;
+    p_zw = ch.zw;
   }
 
   // DIRECT (the whole share of the wave is in flight, total <= D): every wave fetches its own activation fragments
@@ -242,7 +269,7 @@ __device__ __forceinline__ void gemv_i8_body(const GemvArgs &g, const RequantPar
       v += (uint32_t)dq.deep * (uint32_t)d_zx * (uint32_t)dq.zw0 - (uint32_t)d_zx * (uint32_t)d_wsum;
       if (has_zw) v -= (uint32_t)dq.zw0 * (uint32_t)my_asum;
       float d = __fmul_rn(__fmul_rn(d_sx, d_ws), (float)(int32_t)v);
-      if (dq.bias != nullptr) d = __fadd_rn(d, d_bias);
+      if (dq.has_bias != 0) d = __fadd_rn(d, d_bias);
       const bool with_act = dq.act == MI_ACT_RELU || dq.act == MI_ACT_RELU6;
       const float act_lo = with_act ? 0.0f : -__builtin_inff();
       const float act_hi = dq.act == MI_ACT_RELU6 ? 6.0f : __builtin_inff();
@@ -269,12 +296,18 @@ __device__ __forceinline__ void gemv_i8_body(const GemvArgs &g, const RequantPar
 }
 
 template <int M, int R, int D, bool DIRECT, int KS>
-__global__ __launch_bounds__(256) void gemv_i8_kernel(GemvArgs g, RequantParams rq) {
+__global__ __launch_bounds__(256) void gemv_i8_kernel(GemvCall<false> call) {
+  GemvArgs g;
+  RequantParams rq;
+  call.open(&g, &rq);
   gemv_i8_body<M, R, D, DIRECT, KS, false>(g, rq, DequantParams{}, (int)blockIdx.x);
 }
 
 template <int M, int R, int D, bool DIRECT, int KS>
-__global__ __launch_bounds__(256) void gemv_i8_deq_kernel(GemvArgs g, DequantParams dq) {
+__global__ __launch_bounds__(256) void gemv_i8_deq_kernel(GemvCall<true> call) {
+  GemvArgs g;
+  DequantParams dq;
+  call.open(&g, &dq);
   gemv_i8_body<M, R, D, DIRECT, KS, true>(g, RequantParams{}, dq, (int)blockIdx.x);
 }
 
@@ -282,52 +315,130 @@ __global__ __launch_bounds__(256) void gemv_i8_deq_kernel(GemvArgs g, DequantPar
 // gate and up projections of a decoder layer): the grid is the concatenation of the members' grids, and a workgroup
 // first finds the member it belongs to.  Every field is picked with selects over constant indices, which keeps the
 // table in scalar registers (a dynamically indexed kernel argument would be copied to scratch memory).
+// Pairs have a form of their own, whose arguments fit kShortArgs.
 constexpr int kGemvGroupMax = 4;
 template <typename P>  // P: the members' epilogue parameters (RequantParams or DequantParams)
 struct GemvGroupT {
   int count;
-  int block_end[kGemvGroupMax];  // exclusive prefix sums of the members' workgroup counts
-  GemvArgs g[kGemvGroupMax];
+  GemvArgs g[kGemvGroupMax];  // of the same rows
   P rq[kGemvGroupMax];
 };
 typedef GemvGroupT<RequantParams> GemvGroup;
 typedef GemvGroupT<DequantParams> GemvGroupDeq;
 
-template <typename P>
-__device__ __forceinline__ void pick_member(const GemvGroupT<P> &grp, int block, GemvArgs *g, P *rq,
-                                            int *local_block) {
-  int member = 0;
-#pragma unroll
-  for (int i = 1; i < kGemvGroupMax; ++i)
-    if (i < grp.count && block >= grp.block_end[i - 1]) member = i;
-  *g = grp.g[0];
-  *rq = grp.rq[0];
-  *local_block = block;
-#pragma unroll
-  for (int i = 1; i < kGemvGroupMax; ++i) {
-    if (member == i) {
-      *g = grp.g[i];
-      *rq = grp.rq[i];
-      *local_block = block - grp.block_end[i - 1];
+template <int N>
+struct GemvGroupOperands {
+  const int8_t *a, *w[N];
+  int8_t *c[N];
+  int n[N];
+  int block_end[N - 1];  // exclusive prefix sums of the members' workgroup counts; INT_MAX before members that are not there
+  int ldw, kchunks, m;
+  template <typename P>
+  void fill(const GemvGroupT<P> &grp, int m_, int rows_per_block, int *blocks) {
+    *blocks = 0;
+    for (int i = 0; i < N; ++i) {
+      const GemvArgs &g = grp.g[i < grp.count ? i : 0];
+      w[i] = g.w;
+      c[i] = g.c;
+      n[i] = g.n;
+      if (i > 0) block_end[i - 1] = i < grp.count ? *blocks : INT_MAX;
+      if (i < grp.count) *blocks += (g.n + rows_per_block - 1) / rows_per_block;
     }
+    a = grp.g[0].a;
+    ldw = grp.g[0].ldw;
+    kchunks = grp.g[0].kchunks;
+    m = m_;
   }
+  __device__ __forceinline__ int member(int block) const {
+    int i = 0;
+#pragma unroll
+    for (int j = 1; j < N; ++j) i = block >= block_end[j - 1] ? j : i;
+    return i;
+  }
+  template <typename T>
+  static __device__ __forceinline__ T at(const T (&x)[N], int i) {
+    T v = x[0];
+#pragma unroll
+    for (int j = 1; j < N; ++j) v = i == j ? x[j] : v;
+    return v;
+  }
+  __device__ __forceinline__ void open(int i, GemvArgs *g, int *block) const {
+    const int columns = at(n, i);
+    *g = GemvArgs{a, 16 * kchunks, kchunks, at(w, i), ldw, padded_k(16 * kchunks), columns, at(c, i), columns};
+#pragma unroll
+    for (int j = 1; j < N; ++j)
+      if (i == j) *block -= block_end[j - 1];
+  }
+};
+
+template <int N, typename P>
+struct GemvGroupCall;
+
+template <int N>
+struct GemvGroupCall<N, RequantParams> {
+  GemvGroupOperands<N> ops;
+  RequantCall epi[N];
+  void fill(const GemvGroupT<RequantParams> &grp) {
+    for (int i = 0; i < N; ++i) epi[i] = RequantCall::of(grp.rq[i < grp.count ? i : 0]);
+  }
+  __device__ __forceinline__ void open(int i, int n, RequantParams *rq) const {
+    RequantCall e = epi[0];
+#pragma unroll
+    for (int j = 1; j < N; ++j)
+      if (i == j) e = epi[j];
+    *rq = e.open(n);
+  }
+};
+
+template <int N>
+struct GemvGroupCall<N, DequantParams> {
+  GemvGroupOperands<N> ops;
+  const mi_dq_params *qp_dev;
+  const DequantChannel *channels[N];
+  float sx;
+  int32_t zx, zw0[N];
+  uint32_t forms[N];
+  void fill(const GemvGroupT<DequantParams> &grp) {
+    for (int i = 0; i < N; ++i) {
+      const DequantCall d = DequantCall::of(grp.rq[i < grp.count ? i : 0], 16 * grp.g[0].kchunks);
+      channels[i] = d.channels;
+      zw0[i] = d.zw0;
+      forms[i] = d.forms;
+    }
+    qp_dev = grp.rq[0].qp_dev;  // (they read the same rows)
+    sx = grp.rq[0].sx;
+    zx = grp.rq[0].zx;
+  }
+  __device__ __forceinline__ void open(int i, int n, DequantParams *dq) const {
+    *dq = DequantCall{ops.at(channels, i), qp_dev, sx, zx, ops.at(zw0, i), ops.at(forms, i)}.open(n, 16 * ops.kchunks);
+  }
+};
+static_assert(sizeof(GemvGroupCall<2, RequantParams>) <= kShortArgs && sizeof(GemvGroupCall<2, DequantParams>) <= kShortArgs,
+              "see launch_args.h");
+
+template <int N, typename P>
+__device__ __forceinline__ void pick_member(const GemvGroupCall<N, P> &call, GemvArgs *g, P *p, int *block) {
+  *block = (int)blockIdx.x;
+  const int i = call.ops.member(*block);
+  call.ops.open(i, g, block);
+  call.open(i, g->n, p);
 }
 
-template <int M, int R, int D, bool DIRECT, int KS>
-__global__ __launch_bounds__(256) void gemv_i8_group_kernel(GemvGroup grp) {
+template <int M, int R, int D, bool DIRECT, int KS, int N>
+__global__ __launch_bounds__(256) void gemv_i8_group_kernel(GemvGroupCall<N, RequantParams> call) {
   GemvArgs g;
   RequantParams rq;
   int block;
-  pick_member(grp, (int)blockIdx.x, &g, &rq, &block);
+  pick_member(call, &g, &rq, &block);
   gemv_i8_body<M, R, D, DIRECT, KS, false>(g, rq, DequantParams{}, block);
 }
 
-template <int M, int R, int D, bool DIRECT, int KS>
-__global__ __launch_bounds__(256) void gemv_i8_group_deq_kernel(GemvGroupDeq grp) {
+template <int M, int R, int D, bool DIRECT, int KS, int N>
+__global__ __launch_bounds__(256) void gemv_i8_group_deq_kernel(GemvGroupCall<N, DequantParams> call) {
   GemvArgs g;
   DequantParams dq;
   int block;
-  pick_member(grp, (int)blockIdx.x, &g, &dq, &block);
+  pick_member(call, &g, &dq, &block);
   gemv_i8_body<M, R, D, DIRECT, KS, true>(g, RequantParams{}, dq, block);
 }
 
@@ -338,7 +449,7 @@ static int launch_mrdx(const GemvArgs &g, const RequantParams &rq, hipStream_t s
   const int lds_bytes = DIRECT ? 0 : M * ((g.kchunks + 63) / 64) * 1024;
   const int rows_per_block = 4 / KS * R;
   const int blocks = (g.n + rows_per_block - 1) / rows_per_block;
-  hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), lds_bytes, stream, g, rq);
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), lds_bytes, stream, GemvCall<false>::of(g, M, rq));
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }
@@ -348,40 +459,56 @@ static int launch_mrdx_deq(const GemvArgs &g, const DequantParams &dq, hipStream
   const int lds_bytes = DIRECT ? 0 : M * ((g.kchunks + 63) / 64) * 1024;
   const int rows_per_block = 4 / KS * R;
   const int blocks = (g.n + rows_per_block - 1) / rows_per_block;
-  hipLaunchKernelGGL((gemv_i8_deq_kernel<M, R, D, DIRECT, KS>), dim3(blocks), dim3(256), lds_bytes, stream, g, dq);
+  hipLaunchKernelGGL((gemv_i8_deq_kernel<M, R, D, DIRECT, KS>), dim3(blocks), dim3(256), lds_bytes, stream,
+                     GemvCall<true>::of(g, M, dq));
+  MI_HIP_CHECK(hipGetLastError());
+  return MI_OK;
+}
+
+// f(call): the arguments of the group in the form for two members or for up to four.
+template <typename P, typename F>
+static int with_group_call(const GemvGroupT<P> &grp, int m, int rows_per_block, F &&f) {
+  int blocks;
+  if (grp.count == 2) {
+    GemvGroupCall<2, P> call;
+    call.ops.fill(grp, m, rows_per_block, &blocks);
+    call.fill(grp);
+    f(call, blocks, std::integral_constant<int, 2>());
+  } else {
+    GemvGroupCall<kGemvGroupMax, P> call;
+    call.ops.fill(grp, m, rows_per_block, &blocks);
+    call.fill(grp);
+    f(call, blocks, std::integral_constant<int, kGemvGroupMax>());
+  }
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }
 
 template <int M, int R, int D, bool DIRECT, int KS, typename P>
-static int launch_group_mrdx(GemvGroupT<P> &grp, hipStream_t stream) {
+static int launch_group_mrdx(const GemvGroupT<P> &grp, hipStream_t stream) {
   const int lds_bytes = DIRECT ? 0 : M * ((grp.g[0].kchunks + 63) / 64) * 1024;
-  int blocks = 0;
-  for (int i = 0; i < grp.count; ++i) {
-    blocks += (grp.g[i].n + 4 / KS * R - 1) / (4 / KS * R);
-    grp.block_end[i] = blocks;
-  }
-  if constexpr (std::is_same<P, DequantParams>::value) {
-    hipLaunchKernelGGL((gemv_i8_group_deq_kernel<M, R, D, DIRECT, KS>), dim3(blocks), dim3(256), lds_bytes, stream, grp);
-  } else {
-    hipLaunchKernelGGL((gemv_i8_group_kernel<M, R, D, DIRECT, KS>), dim3(blocks), dim3(256), lds_bytes, stream, grp);
-  }
-  MI_HIP_CHECK(hipGetLastError());
-  return MI_OK;
+  return with_group_call(grp, M, 4 / KS * R, [&](const auto &call, int blocks, auto members) {
+    if constexpr (std::is_same<P, DequantParams>::value) {
+      hipLaunchKernelGGL((gemv_i8_group_deq_kernel<M, R, D, DIRECT, KS, decltype(members)::value>), dim3(blocks), dim3(256), lds_bytes,
+                         stream, call);
+    } else {
+      hipLaunchKernelGGL((gemv_i8_group_kernel<M, R, D, DIRECT, KS, decltype(members)::value>), dim3(blocks), dim3(256), lds_bytes,
+                         stream, call);
+    }
+  });
 }
 
 template <int M>
 static int allow_big_lds() {
   // the looping form stages the activation rows in dynamic LDS: up to 160 KiB
-  MI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(gemv_i8_kernel<M, 1, 12, false, 1>),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-  MI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(gemv_i8_group_kernel<M, 1, 12, false, 1>),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+  auto allow = [](const void *kernel) { return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); };
+  MI_HIP_CHECK(allow(reinterpret_cast<const void *>(gemv_i8_kernel<M, 1, 12, false, 1>)));
+  MI_HIP_CHECK(allow(reinterpret_cast<const void *>(gemv_i8_group_kernel<M, 1, 12, false, 1, 2>)));
+  MI_HIP_CHECK(allow(reinterpret_cast<const void *>(gemv_i8_group_kernel<M, 1, 12, false, 1, kGemvGroupMax>)));
   if (M == 1) {
-    MI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(gemv_i8_deq_kernel<1, 1, 12, false, 1>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-    MI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(gemv_i8_group_deq_kernel<1, 1, 12, false, 1>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    MI_HIP_CHECK(allow(reinterpret_cast<const void *>(gemv_i8_deq_kernel<1, 1, 12, false, 1>)));
+    MI_HIP_CHECK(allow(reinterpret_cast<const void *>(gemv_i8_group_deq_kernel<1, 1, 12, false, 1, 2>)));
+    MI_HIP_CHECK(allow(reinterpret_cast<const void *>(gemv_i8_group_deq_kernel<1, 1, 12, false, 1, kGemvGroupMax>)));
   }
   return MI_OK;
 }
@@ -422,7 +549,7 @@ static int with_config(int nseg, F &&f) {
 }
 
 template <int M, typename P>
-static int launch_group_m(GemvGroupT<P> &grp, hipStream_t stream) {  // the choice depends on K only
+static int launch_group_m(const GemvGroupT<P> &grp, hipStream_t stream) {  // the choice depends on K only
   return with_config<M>((grp.g[0].kchunks + 63) >> 6, [&](auto r, auto d, auto direct, auto ks) {
     return launch_group_mrdx<M, decltype(r)::value, decltype(d)::value, decltype(direct)::value, decltype(ks)::value>(
         grp, stream);
@@ -561,18 +688,20 @@ __device__ __forceinline__ void gemv_mfma_lds_body(const GemvArgs &g, int m_rows
     const int q = qq % (4 * RG);  // (the channel does not depend on the activation row group)
     const int n = (q >> 2) < rg_live ? n0 + (q >> 2) * 16 + 4 * grp + (q & 3) : n0;
     if (DEQ) {
-      d_ws[t] = dq.wscale[n];
-      d_wsum[t] = dq.wsum[n];
-      d_bias[t] = dq.bias != nullptr ? dq.bias[n] : 0.0f;
+      const DequantChannel ch = dq.each[n];
+      d_ws[t] = ch.wscale;
+      d_wsum[t] = ch.wsum;
+      d_bias[t] = ch.bias;
       int row = idx + 16 * (qq / (4 * RG));
       row = row < m_rows ? row : m_rows - 1;
       d_sx[t] = dq.qp_dev != nullptr ? dq.qp_dev[dq.per_row ? row : 0].scale_f : dq.sx;
     } else {
-      p_mult[t] = rq.mult[n];
-      p_e[t] = rq.rshift[n];
-      p_ls[t] = rq.lshift[n];
-      p_bias2[t] = rq.bias2[n];
-      p_zw[t] = rq.zw[n];
+      const RequantChannel ch = rq.each[n];
+      p_mult[t] = ch.mult;
+      p_e[t] = ch.rshift();
+      p_ls[t] = ch.lshift();
+      p_bias2[t] = ch.bias2;
+      p_zw[t] = ch.zw;
     }
   }
   if (DEQ) d_zx = dq.qp_dev != nullptr ? dq.qp_dev->zero_point : dq.zx;
@@ -653,7 +782,7 @@ __device__ __forceinline__ void gemv_mfma_lds_body(const GemvArgs &g, int m_rows
         v += (uint32_t)dq.deep * (uint32_t)d_zx * (uint32_t)dq.zw0 - (uint32_t)d_zx * (uint32_t)d_wsum[t];
         if (has_zw) v -= (uint32_t)dq.zw0 * (uint32_t)src[4 * RG * 64];
         float d = __fmul_rn(__fmul_rn(d_sx[t], d_ws[t]), (float)(int32_t)v);
-        if (dq.bias != nullptr) d = __fadd_rn(d, d_bias[t]);
+        if (dq.has_bias != 0) d = __fadd_rn(d, d_bias[t]);
         // (bounds that are infinite where the reference makes no comparison: false for every d, NaN included)
         const bool with_act = dq.act == MI_ACT_RELU || dq.act == MI_ACT_RELU6;
         const float act_lo = with_act ? 0.0f : -__builtin_inff();
@@ -680,31 +809,37 @@ __device__ __forceinline__ void gemv_mfma_lds_body(const GemvArgs &g, int m_rows
 }
 
 template <int WAVES, int RG, int D, int MR>
-__global__ __launch_bounds__(WAVES * 64) void gemv_mfma_lds_kernel(GemvArgs g, int m_rows, RequantParams rq) {
-  gemv_mfma_lds_body<WAVES, RG, D, MR, false>(g, m_rows, rq, DequantParams{}, (int)blockIdx.x);
+__global__ __launch_bounds__(WAVES * 64) void gemv_mfma_lds_kernel(GemvCall<false> call) {
+  GemvArgs g;
+  RequantParams rq;
+  call.open(&g, &rq);
+  gemv_mfma_lds_body<WAVES, RG, D, MR, false>(g, call.m, rq, DequantParams{}, (int)blockIdx.x);
 }
 
 template <int WAVES, int RG, int D, int MR>
-__global__ __launch_bounds__(WAVES * 64) void gemv_mfma_lds_deq_kernel(GemvArgs g, int m_rows, DequantParams dq) {
-  gemv_mfma_lds_body<WAVES, RG, D, MR, true>(g, m_rows, RequantParams{}, dq, (int)blockIdx.x);
+__global__ __launch_bounds__(WAVES * 64) void gemv_mfma_lds_deq_kernel(GemvCall<true> call) {
+  GemvArgs g;
+  DequantParams dq;
+  call.open(&g, &dq);
+  gemv_mfma_lds_body<WAVES, RG, D, MR, true>(g, call.m, RequantParams{}, dq, (int)blockIdx.x);
 }
 
-template <int WAVES, int RG, int D, int MR>
-__global__ __launch_bounds__(WAVES * 64) void gemv_mfma_lds_group_kernel(GemvGroup grp, int m_rows) {
+template <int WAVES, int RG, int D, int MR, int N>
+__global__ __launch_bounds__(WAVES * 64) void gemv_mfma_lds_group_kernel(GemvGroupCall<N, RequantParams> call) {
   GemvArgs g;
   RequantParams rq;
   int block;
-  pick_member(grp, (int)blockIdx.x, &g, &rq, &block);
-  gemv_mfma_lds_body<WAVES, RG, D, MR, false>(g, m_rows, rq, DequantParams{}, block);
+  pick_member(call, &g, &rq, &block);
+  gemv_mfma_lds_body<WAVES, RG, D, MR, false>(g, call.ops.m, rq, DequantParams{}, block);
 }
 
-template <int WAVES, int RG, int D, int MR>
-__global__ __launch_bounds__(WAVES * 64) void gemv_mfma_lds_group_deq_kernel(GemvGroupDeq grp, int m_rows) {
+template <int WAVES, int RG, int D, int MR, int N>
+__global__ __launch_bounds__(WAVES * 64) void gemv_mfma_lds_group_deq_kernel(GemvGroupCall<N, DequantParams> call) {
   GemvArgs g;
   DequantParams dq;
   int block;
-  pick_member(grp, (int)blockIdx.x, &g, &dq, &block);
-  gemv_mfma_lds_body<WAVES, RG, D, MR, true>(g, m_rows, RequantParams{}, dq, block);
+  pick_member(call, &g, &dq, &block);
+  gemv_mfma_lds_body<WAVES, RG, D, MR, true>(g, call.ops.m, RequantParams{}, dq, block);
 }
 
 template <int WAVES, int D, typename F>
@@ -721,34 +856,30 @@ static int with_row_class(int m, F &&f) {  // rows rounded up to 2, 4, 8, 16 or 
 // fragment, two steps per pass (the staging area of 64 rows and the accumulators leave room for no more).  Measured
 // against 64 x 64 GEMM tiles in us per launch at 64 rows: 4096 x 4096 11.0 -> 8.8, 4096 x 11008 27.5 -> 18.7.
 static int launch_mfma_lds_64(const GemvArgs &g, int m, const RequantParams &rq, hipStream_t stream) {
-  hipLaunchKernelGGL((gemv_mfma_lds_kernel<8, 1, 2, 64>), dim3((g.n + 15) / 16), dim3(512), 0, stream, g, m, rq);
+  hipLaunchKernelGGL((gemv_mfma_lds_kernel<8, 1, 2, 64>), dim3((g.n + 15) / 16), dim3(512), 0, stream,
+                     GemvCall<false>::of(g, m, rq));
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }
 
 static int launch_mfma_lds_deq_64(const GemvArgs &g, int m, const DequantParams &dq, hipStream_t stream) {
-  hipLaunchKernelGGL((gemv_mfma_lds_deq_kernel<8, 1, 2, 64>), dim3((g.n + 15) / 16), dim3(512), 0, stream, g, m, dq);
+  hipLaunchKernelGGL((gemv_mfma_lds_deq_kernel<8, 1, 2, 64>), dim3((g.n + 15) / 16), dim3(512), 0, stream,
+                     GemvCall<true>::of(g, m, dq));
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }
 
 template <int WAVES, int RG, int D, typename P>
-static int launch_group_mfma_lds(GemvGroupT<P> &grp, int m, hipStream_t stream) {
-  int blocks = 0;
-  for (int i = 0; i < grp.count; ++i) {
-    blocks += (grp.g[i].n + RG * 16 - 1) / (RG * 16);
-    grp.block_end[i] = blocks;
-  }
+static int launch_group_mfma_lds(const GemvGroupT<P> &grp, int m, hipStream_t stream) {
   return with_row_class<WAVES, D>(m, [&](auto mr) {
-    if constexpr (std::is_same<P, DequantParams>::value) {
-      hipLaunchKernelGGL((gemv_mfma_lds_group_deq_kernel<WAVES, RG, D, decltype(mr)::value>), dim3(blocks),
-                         dim3(WAVES * 64), 0, stream, grp, m);
-    } else {
-      hipLaunchKernelGGL((gemv_mfma_lds_group_kernel<WAVES, RG, D, decltype(mr)::value>), dim3(blocks),
-                         dim3(WAVES * 64), 0, stream, grp, m);
-    }
-    MI_HIP_CHECK(hipGetLastError());
-    return (int)MI_OK;
+    return with_group_call(grp, m, RG * 16, [&](const auto &call, int blocks, auto members) {
+      constexpr int MR = decltype(mr)::value, N = decltype(members)::value;
+      if constexpr (std::is_same<P, DequantParams>::value) {
+        hipLaunchKernelGGL((gemv_mfma_lds_group_deq_kernel<WAVES, RG, D, MR, N>), dim3(blocks), dim3(WAVES * 64), 0, stream, call);
+      } else {
+        hipLaunchKernelGGL((gemv_mfma_lds_group_kernel<WAVES, RG, D, MR, N>), dim3(blocks), dim3(WAVES * 64), 0, stream, call);
+      }
+    });
   });
 }
 
@@ -757,7 +888,7 @@ static int launch_mfma_lds(const GemvArgs &g, int m, const RequantParams &rq, hi
   const int blocks = (g.n + RG * 16 - 1) / (RG * 16);
   return with_row_class<WAVES, D>(m, [&](auto mr) {
     hipLaunchKernelGGL((gemv_mfma_lds_kernel<WAVES, RG, D, decltype(mr)::value>), dim3(blocks), dim3(WAVES * 64), 0,
-                       stream, g, m, rq);
+                       stream, GemvCall<false>::of(g, m, rq));
     MI_HIP_CHECK(hipGetLastError());
     return (int)MI_OK;
   });
@@ -790,7 +921,7 @@ static int launch_mfma_lds_deq(const GemvArgs &g, int m, const DequantParams &dq
   const int blocks = (g.n + RG * 16 - 1) / (RG * 16);
   return with_row_class<WAVES, D>(m, [&](auto mr) {
     hipLaunchKernelGGL((gemv_mfma_lds_deq_kernel<WAVES, RG, D, decltype(mr)::value>), dim3(blocks), dim3(WAVES * 64),
-                       0, stream, g, m, dq);
+                       0, stream, GemvCall<true>::of(g, m, dq));
     MI_HIP_CHECK(hipGetLastError());
     return (int)MI_OK;
   });
@@ -802,13 +933,13 @@ static bool prefers_mfma(int m, const WeightView &wv) {
   return m > kGemvDotRows || (m == 2 && wv.blocked != nullptr);
 }
 
-static int check_gemv_operands(const int8_t *a, int64_t lda, int m, int k, const WeightView &wv, int n, const int8_t *c) {
+static int check_gemv_operands(const int8_t *a, int64_t lda, int m, int k, const WeightView &wv, int n, const int8_t *c, int64_t ldc) {
   if (a == nullptr || wv.w == nullptr || c == nullptr) {
     set_error("gemv: null pointer");
     return MI_NULL_PTR;
   }
-  if (m < 1 || !gemv_takes_rows(m, n) || n <= 0 || k <= 0 || (k & 15) != 0 || (lda & 15) != 0 || lda < k ||
-      wv.k_pad % kKPad != 0 || wv.k_pad < k || wv.ldw < wv.k_pad || (wv.ldw & 15) != 0 ||
+  if (m < 1 || ldc != n || !gemv_takes_rows(m, n) || n <= 0 || k <= 0 || (k & 15) != 0 || (lda & 15) != 0 || lda < k ||
+      wv.k_pad != round_up(k, kKPad) || wv.ldw != weight_row_stride(wv.k_pad) ||
       (reinterpret_cast<uintptr_t>(a) & 15) != 0 ||
       (int64_t)(m - 1) * lda + k >= (int64_t)1 << 30 || wv.k_pad > 1 << 20 ||  // (32-bit buffer offsets)
       (m <= kGemvDotRows && (int64_t)m * round_up(k, 1024) > 160 * 1024 - 1024)) {
@@ -824,8 +955,8 @@ static int check_gemv_operands(const int8_t *a, int64_t lda, int m, int k, const
 
 int launch_gemv_group(const int8_t *a, int64_t lda, int m, int k, int count, const WeightView *wv, const int *n,
                       const RequantParams *rq, int8_t *const *c, hipStream_t stream) {
-  if (count < 1 || count > kGemvGroupMax) {
-    set_error("gemv group: %d members (1..%d)", count, kGemvGroupMax);
+  if (count < 1 || count > kGemvGroupMax || lda != k) {
+    set_error("gemv group: %d members (1..%d), rows of %d bytes %lld apart", count, kGemvGroupMax, k, (long long)lda);
     return MI_PARAM_INVALID;
   }
   if (m > kGemvGroupMaxRows) {
@@ -837,7 +968,7 @@ int launch_gemv_group(const int8_t *a, int64_t lda, int m, int k, int count, con
   int n_max = 0, k_pad_max = 0;
   bool mfma = true;  // every member has what the matrix-core kernel needs
   for (int i = 0; i < count; ++i) {
-    const int rc = check_gemv_operands(a, lda, m, k, wv[i], n[i], c[i]);
+    const int rc = check_gemv_operands(a, lda, m, k, wv[i], n[i], c[i], n[i]);
     if (rc != MI_OK) return rc;
     mfma = mfma && prefers_mfma(m, wv[i]);
     grp.g[i] = GemvArgs{a, lda, k / 16, wv[i].w, wv[i].ldw, wv[i].k_pad, n[i], c[i], n[i]};
@@ -859,7 +990,7 @@ int launch_gemv_requant(const int8_t *a, int64_t lda, int m, int k, const Weight
                         const RequantParams &rq, int8_t *c, int64_t ldc, hipStream_t stream) {
   const int8_t *w = wv.w;
   const int k_pad = wv.k_pad;
-  const int rc = check_gemv_operands(a, lda, m, k, wv, n, c);
+  const int rc = check_gemv_operands(a, lda, m, k, wv, n, c, ldc);
   if (rc != MI_OK) return rc;
   GemvArgs g{a, lda, k / 16, w, wv.ldw, k_pad, n, c, ldc};
   if (prefers_mfma(m, wv)) {
@@ -878,7 +1009,7 @@ int launch_gemv_requant(const int8_t *a, int64_t lda, int m, int k, const Weight
 // epilogue; the same configurations as for the requantising form.
 int launch_gemv_dequant(const int8_t *a, int64_t lda, int m, int k, const WeightView &wv, int n,
                         const DequantParams &dq, float *c, int64_t ldc, hipStream_t stream) {
-  const int rc = check_gemv_operands(a, lda, m, k, wv, n, reinterpret_cast<const int8_t *>(c));
+  const int rc = check_gemv_operands(a, lda, m, k, wv, n, reinterpret_cast<const int8_t *>(c), ldc);
   if (rc != MI_OK) return rc;
   if (m == 1) {  // one row: the v_dot4 kernel on the row-major weights, as for the requantising MatMul
     const GemvArgs g1{a, lda, k / 16, wv.w, wv.ldw, wv.k_pad, n, reinterpret_cast<int8_t *>(c), ldc};
@@ -902,8 +1033,8 @@ int launch_gemv_dequant(const int8_t *a, int64_t lda, int m, int k, const Weight
 // 2..32 rows on the matrix-core kernel (every member then needs its blocked weight copy).
 int launch_gemv_group_dequant(const int8_t *a, int64_t lda, int m, int k, int count, const WeightView *wv, const int *n,
                               const DequantParams *dq, float *const *c, hipStream_t stream) {
-  if (count < 1 || count > kGemvGroupMax) {
-    set_error("gemv group: %d members (1..%d)", count, kGemvGroupMax);
+  if (count < 1 || count > kGemvGroupMax || lda != k) {
+    set_error("gemv group: %d members (1..%d), rows of %d bytes %lld apart", count, kGemvGroupMax, k, (long long)lda);
     return MI_PARAM_INVALID;
   }
   if (m > kGemvGroupMaxRows) {
@@ -914,7 +1045,7 @@ int launch_gemv_group_dequant(const int8_t *a, int64_t lda, int m, int k, int co
   grp.count = count;
   int n_max = 0, k_pad_max = 0;
   for (int i = 0; i < count; ++i) {
-    const int rc = check_gemv_operands(a, lda, m, k, wv[i], n[i], reinterpret_cast<const int8_t *>(c[i]));
+    const int rc = check_gemv_operands(a, lda, m, k, wv[i], n[i], reinterpret_cast<const int8_t *>(c[i]), n[i]);
     if (rc != MI_OK) return rc;
     if (m > 1 && wv[i].blocked == nullptr) {
       set_error("gemv group: the blocked weight copy is missing");

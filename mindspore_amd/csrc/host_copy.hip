@@ -31,10 +31,10 @@ constexpr int kOutWgs = 16;  // us at 4 MiB out: 16 149, 32 154, 64 159, 256 230
 // the host can empty the first slots while the last are being filled (with a workgroup per part all parts arrived at the end).
 // Otherwise a flag says that its part has been read.
 template <bool TO_HOST>
-__global__ __launch_bounds__(256) void host_copy_kernel(const v4i *__restrict__ from, v4i *__restrict__ to, int n16, uint32_t *flags,
+__global__ __launch_bounds__(256) void host_copy_kernel(const v4i *__restrict__ from, v4i *__restrict__ to, int n16, int wgs, uint32_t *flags,
                                                         uint32_t ticket) {
   constexpr int kPart = kWgBytes / 16;
-  for (int part = blockIdx.x; part * kPart < n16; part += gridDim.x) {
+  for (int part = blockIdx.x; part * kPart < n16; part += wgs) {
     const int first = part * kPart + threadIdx.x;
     v4i v[4];
 #pragma unroll
@@ -111,10 +111,10 @@ int launch_chunks(HostSlots *s, const Chunks &c, int64_t i, int n, char *dev, bo
   uint32_t *flags = s->flags + c.first_flag(c.slot(i));
   v4i *there = reinterpret_cast<v4i *>(dev), *here = reinterpret_cast<v4i *>(staged);
   if (in) {
-    hipLaunchKernelGGL((host_copy_kernel<false>), dim3(parts), dim3(256), 0, nullptr, here, there, n16, flags, s->ticket);
+    hipLaunchKernelGGL((host_copy_kernel<false>), dim3(parts), dim3(256), 0, nullptr, here, there, n16, parts, flags, s->ticket);
   } else {
-    hipLaunchKernelGGL((host_copy_kernel<true>), dim3(parts < kOutWgs ? parts : kOutWgs), dim3(256), 0, nullptr, there, here, n16, flags,
-                       s->ticket);
+    const int wgs = parts < kOutWgs ? parts : kOutWgs;
+    hipLaunchKernelGGL((host_copy_kernel<true>), dim3(wgs), dim3(256), 0, nullptr, there, here, n16, wgs, flags, s->ticket);
   }
   MI_HIP_CHECK(hipGetLastError());
   for (int k = 0; k < n; ++k) s->pending[c.slot(i) + k] = s->ticket;

@@ -709,3 +709,13 @@ def test_depthwise_stride_one_activations(orc, b, ih, iw, ch, taps, act):
     pad = (taps // 2,) * 4
     case = _conv_case(rng, b, ih, iw, ch, ch, (taps, taps), (1, 1), (1, 1), pad, True, False, True, act, dw=True)
     assert np.array_equal(_gpu_conv(case, (1, 1), (1, 1), pad, ch, device_tensors=True), orc.conv_dw_int8(**case))
+
+
+# strides and pads at and past the 16 bits in which the gathering kernels take them; past them the window buffer serves
+@pytest.mark.parametrize("ic,kernel", [(3, (3, 3)), (16, (1, 3))])
+@pytest.mark.parametrize("far", [32767, 32768, 40000])
+def test_convolution_wide_strides_and_pads(orc, ic, kernel, far):
+    rng = np.random.default_rng(far + ic)
+    pad, stride = (kernel[0] // 2, kernel[0] // 2, far, far), (1, far)
+    case = _conv_case(rng, 2, 60, 9, ic, 40, kernel, stride, (1, 1), pad, True, False, True, 1)
+    np.testing.assert_array_equal(_gpu_conv(case, stride, (1, 1), pad), _orc_conv(orc, case))
