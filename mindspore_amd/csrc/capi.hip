@@ -38,6 +38,43 @@ static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 constexpr int kMaxDevices = 64;
 static void *g_scratch_ptr[kMaxDevices] = {};
 
+// The null stream's split_space, static as the scratch memory is; those of the library's own streams, made when first wanted.
+static __device__ __align__(256) unsigned char split_of_null_stream[kSplitBytes];
+static void *g_split_ptr[kMaxDevices] = {};
+struct SplitSpace {
+  hipStream_t stream;
+  void *p;
+  bool tried;
+};
+static std::mutex g_split_mutex;
+static std::vector<SplitSpace> g_split_spaces;
+static thread_local bool t_allocates_nothing = false;  // in mi_matmul_run_noalloc
+
+void *split_space(hipStream_t stream) {
+  if (stream == nullptr) return g_device >= 0 && g_device < kMaxDevices ? g_split_ptr[g_device] : nullptr;
+  std::lock_guard<std::mutex> lock(g_split_mutex);
+  for (SplitSpace &s : g_split_spaces) {
+    if (s.stream != stream) continue;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone) return nullptr;
+    if (!s.tried && !t_allocates_nothing) {
+      s.tried = true;
+      hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // (another thread may be capturing)
+      (void)hipThreadExchangeStreamCaptureMode(&mode);
+      void *p = nullptr;
+      if (hipMalloc(&p, kSplitBytes) == hipSuccess && hipMemsetAsync(p, 0, kSplitCounterBytes, stream) == hipSuccess) {
+        s.p = p;
+      } else {
+        (void)hipGetLastError();
+        if (p != nullptr) (void)hipFree(p);
+      }
+      (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+    return s.p;
+  }
+  return nullptr;
+}
+
 void set_error(const char *fmt, ...) {
   va_list ap;
   va_start(ap, fmt);
@@ -608,6 +645,8 @@ int mi_init(int device) {
     void *ptr = nullptr;
     MI_HIP_CHECK(hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)));  // this device's copy of the array
     g_scratch_ptr[device] = ptr;
+    MI_HIP_CHECK(hipGetSymbolAddress(&ptr, HIP_SYMBOL(split_of_null_stream)));
+    g_split_ptr[device] = ptr;
   }
   g_device = device;
   return MI_OK;
@@ -696,6 +735,11 @@ int mi_stream_create(void **out_stream) {
   if (ensure_device() != MI_OK) return MI_ERROR;
   hipStream_t s = nullptr;
   MI_HIP_CHECK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));  // default priority; independent of the null stream
+  try {
+    std::lock_guard<std::mutex> lock(g_split_mutex);
+    g_split_spaces.push_back(SplitSpace{s, nullptr, false});
+  } catch (...) {  // (unknown to split_space: its GEMMs are not split)
+  }
   *out_stream = s;
   return MI_OK;
 }
@@ -703,6 +747,17 @@ int mi_stream_create(void **out_stream) {
 int mi_stream_destroy(void *stream) {
   if (stream == nullptr) return MI_OK;
   if (ensure_device() != MI_OK) return MI_ERROR;
+  void *p = nullptr;
+  {
+    std::lock_guard<std::mutex> lock(g_split_mutex);
+    for (size_t i = 0; i < g_split_spaces.size(); ++i) {
+      if (g_split_spaces[i].stream != static_cast<hipStream_t>(stream)) continue;
+      p = g_split_spaces[i].p;
+      g_split_spaces.erase(g_split_spaces.begin() + (ptrdiff_t)i);
+      break;
+    }
+  }
+  if (p != nullptr) (void)hipFree(p);  // (waits for the device)
   MI_HIP_CHECK(hipStreamDestroy(static_cast<hipStream_t>(stream)));
   return MI_OK;
 }
@@ -968,7 +1023,10 @@ int mi_matmul_run_noalloc(mi_matmul *h, const int8_t *a_dev, int32_t rows, int8_
               "maximum is %zu; use mi_matmul_run", rows, h->st.k, h->st.n, need, kScratchBytes);
     return MI_PARAM_INVALID;
   }
-  return run_requant_rows(h->st, a_dev, rows, Workspace::region(base, a_bytes), c_dev, static_cast<hipStream_t>(stream));
+  t_allocates_nothing = true;
+  rc = run_requant_rows(h->st, a_dev, rows, Workspace::region(base, a_bytes), c_dev, static_cast<hipStream_t>(stream));
+  t_allocates_nothing = false;
+  return rc;
 }
 
 int mi_matmul_run_host(mi_matmul *h, const int8_t *a_host, int32_t rows, int8_t *c_host) {

@@ -120,6 +120,14 @@ struct WeightView {
 };
 __host__ __device__ inline int weight_row_stride(int k_pad) { return (k_pad / 256) % 2 == 0 ? k_pad + 256 : k_pad; }
 
+// Device memory through which the workgroups of a split GEMM (gemm_split.hip) hand over their sums: counters, which are zero
+// between launches, and the sums.  Null: the GEMM is not split.  Launches on one stream follow one another and share it; so there
+// is one for the null stream, and one for each stream of mi_stream_create, whose end the library sees, but not while that is
+// captured: a replay may run beside the stream.
+constexpr size_t kSplitCounterBytes = 1024, kSplitSumBytes = 256 * 256 * (4 * 64 + 16);  // 256 parts of 128 x 128 sums and row sums
+constexpr size_t kSplitBytes = kSplitCounterBytes + kSplitSumBytes;
+void *split_space(hipStream_t stream);
+
 // A: int8 activations [M][lda] (lda in bytes, multiple of 16, base 16-byte aligned, K % 16 == 0);
 // W: packed weights (above); C: [M][ldc] elements, any n, ldc == n, any address of the element type.
 int launch_gemm_requant(const int8_t *a, int64_t lda, int m, int k, const WeightView &w, int n,

@@ -69,16 +69,20 @@ __device__ __forceinline__ void async_copy16(const void *global_src, void *lds_w
 
 // Hardware deals consecutive workgroup ids round-robin over the 8 XCDs (each with its own L2), so ids that share an
 // XCD are mapped to a compact block of tiles, 4 tiles tall: the CUs of one XCD then share operand panels in L2.
-__device__ __forceinline__ void tile_coords(const GemmArgs &g, int *tile_m, int *tile_n) {
-  int id = blockIdx.x;
-  const int nb = g.tiles_m * g.tiles_n, per = nb >> 3;  // (nb: the grid)
-  if (id < per * 8) id = (id & 7) * per + (id >> 3);
+__device__ __forceinline__ int xcd_order(int id, int grid) {
+  const int per = grid >> 3;
+  return id < per * 8 ? (id & 7) * per + (id >> 3) : id;
+}
+__device__ __forceinline__ void tile_of(const GemmArgs &g, int id, int *tile_m, int *tile_n) {
   constexpr int G = 4;
   const int width = G * g.tiles_n;
   const int group = id / width, first = group * G;
   const int gsize = min(g.tiles_m - first, G);
   *tile_m = first + (id % width) % gsize;
   *tile_n = (id % width) / gsize;
+}
+__device__ __forceinline__ void tile_coords(const GemmArgs &g, int *tile_m, int *tile_n) {
+  tile_of(g, xcd_order((int)blockIdx.x, g.tiles_m * g.tiles_n), tile_m, tile_n);
 }
 
 // Several weight matrices with the same K against the same activation rows as one launch: their column tiles stand side by
@@ -602,6 +606,10 @@ int launch_gemm_kblock(int tile, bool requant, bool has_zw, bool fast, GemmArgs 
                        const DequantParams &dq, hipStream_t stream);
 int launch_gemm_ring(int tile, bool requant, bool has_zw, bool fast, GemmArgs g, const RequantParams &rq,
                      const DequantParams &dq, hipStream_t stream);
+// The ring's loop with K split over `parts` workgroups a tile (gemm_split.hip): tiles 11, 12 and 22, int8 output only in the fast2
+// form, fp32 only without weight zero points; space: what split_space gave.
+int launch_gemm_split(int tile, int parts, bool requant, bool has_zw, bool fast, const GemmArgs &g, const RequantParams &rq,
+                      const DequantParams &dq, void *space, hipStream_t stream);
 // 64 x 64 tiles over activation rows of any length, stride and address (gemm_anyrow.hip); g.k: bytes of K.
 int launch_gemm_anyrow(bool requant, bool has_zw, bool fast, const GemmArgs &g, const RequantParams &rq, const DequantParams &dq,
                        hipStream_t stream);

@@ -26,6 +26,8 @@
 // Any K that is a multiple of 16: the weights are zero padded, so an activation chunk past K only has to be a valid
 // read (it re-reads the row's last chunk).  LDS rows are XOR-swizzled in units of 16 bytes so that the 16-byte
 // fragment reads of a wave are bank-conflict free.
+#include <algorithm>
+
 #include "gemm_core.h"
 
 namespace mi {
@@ -358,6 +360,39 @@ static const TileCost &cheapest_tile(int m, int k, int count, const int *n, floa
   }
   return *best;
 }
+// K split over the workgroups of a tile (gemm_split.hip): expected to take a + b x K blocks of a part + 1.7 us for the sums' way
+// through memory + `part` for every part after the first + `wg` for every workgroup, whose sums all go that way at once.  b_far:
+// where the weights are too large to be in the caches.  The margins are for what a and b do not know.  us per launch, unsplit /
+// split, weights from memory: 65 x 3328 x 8368 24.8 / 16.6, 128 x 4096 x 11008 26.3 / 18.3, 128 x 4096 x 4096 10.7 / 9.8,
+// 64 x 6000 x 8000 21.9 / 15.8, 100 x 1024 x 4096 9.5 / 7.8, 138 x 1408 x 5632 10.9 / 9.3, 300 x 1024 x 8192 14.4 / 10.5,
+// 1000 x 512 x 8192 14.9 / 12.2, 512 x 4096 x 11008 38.1 / 35.7; not taken: 200 x 1024 x 2048 5.8 / 7.0, 197 x 768 x 3072 7.43 / 7.46,
+// 161 x 1280 x 3120 7.86 / 7.87, 512 x 4096 x 4096 13.3 / 18.5, 256 x 4096 x 4096 10.0 / 13.2, 800 x 1280 x 5120 14.5 / 15.6.
+struct SplitCost {
+  int tn, tm, most_parts;
+  float a, b, b_far, part, wg;
+};
+constexpr SplitCost kSplitCosts[] = {{1, 1, 8, 2.8f, 0.25f, 0.285f, 0.25f, 0.008f},
+                                     {1, 2, 8, 2.9f, 0.36f, 0.41f, 0.35f, 0.016f},
+                                     {2, 2, 2, 3.0f, 0.57f, 0.57f, 0.5f, 0.022f}};
+constexpr int64_t kFarWeights = 16 << 20;
+// The tile and the number of parts, or null where the unsplit launch on `whole` is expected to be as quick.
+static const SplitCost *choose_split(int m, int k, int n, const TileCost &whole, float cost, int *parts) {
+  const SplitCost *best = nullptr;
+  const int kblocks = (k + 127) / 128;
+  const bool far = (int64_t)n * k >= kFarWeights;
+  for (const SplitCost &t : kSplitCosts)
+    if (far && whole.ring && whole.tn == t.tn && whole.tm == t.tm) cost *= (t.a + t.b_far * (float)kblocks) / (t.a + t.b * (float)kblocks);
+  float least = (far ? 0.99f : 0.9f) * cost;
+  for (const SplitCost &t : kSplitCosts) {
+    const int64_t tiles = (int64_t)((m + 64 * t.tm - 1) / (64 * t.tm)) * ((n + 64 * t.tn - 1) / (64 * t.tn));
+    const int most = (int)std::min<int64_t>(256 / tiles, std::min(kblocks, t.most_parts));
+    for (int p = 2; p <= most; ++p) {
+      const float c = t.a + (far ? t.b_far : t.b) * (float)((kblocks + p - 1) / p) + 1.7f + t.part * (float)(p - 1) + t.wg * (float)(tiles * p);
+      if (c < least) best = &t, least = c, *parts = p;
+    }
+  }
+  return best;
+}
 // (the K-block loaders address activation rows with 32-bit offsets from the tile's first row)
 static bool kblock_takes(int k, int64_t lda) { return k >= 128 && lda < (1 << 23); }
 
@@ -378,6 +413,13 @@ static int launch_pick_tile(const GemmArgs &g, const RequantParams &rq, const De
     if (EPI == EPI_DEQUANT && g.k < 1024 && tiles_m >= 128) return launch_gemm_kblock(22, false, HAS_ZW, FAST, g, rq, dq, stream);
     float cost;
     const TileCost &t = cheapest_tile(g.m, g.k, 1, &g.n, &cost);
+    if (EPI == EPI_REQUANT ? FAST : !HAS_ZW) {  // (the forms that gemm_split.hip has)
+      int parts;
+      const SplitCost *split = choose_split(g.m, g.k, g.n, t, cost, &parts);
+      void *space = split != nullptr ? split_space(stream) : nullptr;
+      if (space != nullptr)
+        return launch_gemm_split(10 * split->tn + split->tm, parts, EPI == EPI_REQUANT, HAS_ZW, FAST, g, rq, dq, space, stream);
+    }
     return t.ring ? launch_gemm_ring(10 * t.tn + t.tm, EPI == EPI_REQUANT, HAS_ZW, FAST, g, rq, dq, stream)
                   : launch_gemm_kblock(10 * t.tn + t.tm, EPI == EPI_REQUANT, HAS_ZW, FAST, g, rq, dq, stream);
   }

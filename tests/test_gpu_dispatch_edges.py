@@ -720,3 +720,72 @@ def test_convolution_wide_strides_and_pads(orc, ic, kernel, far):
     pad, stride = (kernel[0] // 2, kernel[0] // 2, far, far), (1, far)
     case = _conv_case(rng, 2, 60, 9, ic, 40, kernel, stride, (1, 1), pad, True, False, True, 1)
     assert np.array_equal(_gpu_conv(case, stride, (1, 1), pad, 1, device_tensors=True, exact_3x3=True), orc.conv_int8(**case))
+
+
+# K in several parts a tile, as choose_split deals it out: 64 x 64 tiles in 5, 8, 5, 3 and 2 parts, 64 channels x 128 rows in 4 and 2,
+# 128 x 128 in 2; parts of unequal length, a last block, last rows and channels that are partly there, rows to be padded first
+@pytest.mark.parametrize("m,n,k", [(70, 200, 5632), (100, 256, 8200), (129, 257, 4100), (200, 1000, 4700), (100, 3330, 8368),
+                                   (128, 4096, 11008), (250, 4000, 11008), (300, 4096, 8192), (512, 4000, 11008)])
+@pytest.mark.parametrize("dynamic,asymmetric", [(False, False), (False, True), (True, False)])
+def test_matmul_with_k_in_parts(orc, m, n, k, dynamic, asymmetric):
+    """On the null stream, where K is split, and on another, where it is not: the same sums.  Small ones against the oracle too."""
+    import torch
+    rng = np.random.default_rng(m + n + k)
+    w, bias, sw, zw, make = _matmul_pair(rng, n, k, asymmetric, dynamic)
+    kern = make(True)
+    a = rng.integers(-128, 128, (m, k), dtype=np.int8)
+    dev = torch.from_numpy(a).cuda()
+    args = dict(in_quant=K.QuantParam(0.03, -5)) if dynamic else {}
+    torch.cuda.synchronize()
+    other = torch.cuda.Stream()
+    with torch.cuda.stream(other):
+        want = kern.run(dev, **args)
+    other.synchronize()
+    for _ in range(4):  # (the counters are left as they were found)
+        got = [kern.run(dev, **args) for _ in range(3)]
+        torch.cuda.synchronize()
+        for y in got:
+            assert torch.equal(y.view(torch.int8), want.view(torch.int8))
+    if m * n * k < 1e9:
+        orc.set_threads(16)
+        if dynamic:
+            sure = orc.dynamic_matmul(a, w, bias, 0.03, -5, sw, zw)
+        else:
+            sure = orc.matmul_int8(a, w, bias, 0.02, 7, sw, zw, float(np.float32(0.02 * 0.0055 * k ** 0.5 * 140)), 3)
+        assert np.array_equal(want.cpu().numpy(), sure)
+
+
+def test_matmul_with_k_in_parts_on_library_streams():
+    """Two threads, each with a stream of the library and a handle of its own, beside the null stream."""
+    import ctypes as C
+    import threading
+    import torch
+    L = K._lib.load()
+    rng = np.random.default_rng(5)
+    work = []
+    for i in range(3):
+        kern = _matmul_pair(rng, 1000, 4096, False, False)[4](True)
+        dev = torch.from_numpy(rng.integers(-128, 128, (150, 4096), dtype=np.int8)).cuda()
+        work.append((kern, dev, kern.run(dev), torch.empty((150, 1000), dtype=torch.int8, device="cuda")))
+    torch.cuda.synchronize()
+    failed = []
+
+    def go(kern, dev, want, out, own):
+        stream = C.c_void_p(None)
+        if own and L.mi_stream_create(C.byref(stream)) != 0:
+            failed.append("stream")
+        for _ in range(200):
+            if L.mi_matmul_run(kern._h, C.c_void_p(dev.data_ptr()), 150, C.c_void_p(out.data_ptr()), stream) != 0:
+                failed.append("run")
+        L.mi_stream_synchronize(stream)
+        if not torch.equal(out, want):
+            failed.append("result")
+        if own and L.mi_stream_destroy(stream) != 0:
+            failed.append("destroy")
+
+    threads = [threading.Thread(target=go, args=w + (i > 0,)) for i, w in enumerate(work)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed
