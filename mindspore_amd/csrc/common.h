@@ -24,6 +24,18 @@ void set_error(const char *fmt, ...);
 inline int round_up(int x, int m) { return (x + m - 1) / m * m; }
 inline int64_t round_up64(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
+// Quotients of p < 2^31 by d >= 1 as umulhi(2 p, magic) >> shift, with 2^(shift - 1) < d <= 2^shift and
+// magic = ceil(2^(31 + shift) / d): the product is p / d + p * e / (d * 2^(31 + shift)), e = magic * d - 2^(31 + shift) < 2^shift,
+// and the second term stays below 1 / d.
+inline void magic31(int d, uint32_t *magic, int *shift) {
+  int s = 0;
+  while (((int64_t)1 << s) < d) ++s;
+  *shift = s;
+  *magic = (uint32_t)((((uint64_t)1 << (31 + s)) + (uint32_t)d - 1) / (uint32_t)d);
+}
+
+__device__ __forceinline__ int quotient31(int p, uint32_t magic, int shift) { return (int)(__umulhi(2 * (uint32_t)p, magic) >> shift); }
+
 // Weight rows (output channels) and the contraction dimension are padded so that no kernel needs bounds checks on
 // the weight operand: rows to a multiple of kNPad, K to a multiple of kKPad (bytes, two 128-byte GEMM steps), zero filled.
 constexpr int kNPad = 256;

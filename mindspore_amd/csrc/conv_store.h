@@ -13,18 +13,6 @@ namespace mi {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
-// Quotients of p < 2^31 by d >= 1 as umulhi(2 p, magic) >> shift, with 2^(shift - 1) < d <= 2^shift and
-// magic = ceil(2^(31 + shift) / d): the product is p / d + p * e / (d * 2^(31 + shift)), e = magic * d - 2^(31 + shift) < 2^shift,
-// and the second term stays below 1 / d.
-inline void magic31(int d, uint32_t *magic, int *shift) {
-  int s = 0;
-  while (((int64_t)1 << s) < d) ++s;
-  *shift = s;
-  *magic = (uint32_t)((((uint64_t)1 << (31 + s)) + (uint32_t)d - 1) / (uint32_t)d);
-}
-
-__device__ __forceinline__ int quotient31(int p, uint32_t magic, int shift) { return (int)(__umulhi(2 * (uint32_t)p, magic) >> shift); }
-
 __device__ __forceinline__ uint32_t quad_transpose(uint32_t d, uint32_t sel1, uint32_t sel2) {
   const uint32_t p = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)d, 0xB1, 0xF, 0xF, true);  // lane ^ 1
   const uint32_t r = __builtin_amdgcn_perm(p, d, sel1);

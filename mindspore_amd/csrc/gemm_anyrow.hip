@@ -37,7 +37,7 @@ __device__ __forceinline__ void gemm_anyrow_body(const GemmArgs &g, const Requan
   EpiParams<TILE, EPI, FAST> epi;
   epi.fetch(rq, dq, n0, g.n, tid);
   DeqInput<1> din;
-  if (EPI == EPI_DEQUANT) din.fetch(dq, m0 + wm * 32, r, g.m);
+  if (EPI == EPI_DEQUANT) din.fetch_rows(dq, m0 + wm * 32, r, g.m);
 
   const int k64 = g.k_pad >> 6;
   const WaveWeightGroups<1> wg(g.n, n0, wave, kNPad);
@@ -120,6 +120,7 @@ __device__ __forceinline__ void gemm_anyrow_body(const GemmArgs &g, const Requan
 
   load_w(0);
   load_a(0);
+  if (EPI == EPI_DEQUANT) din.fetch_tensor(dq);
 #pragma unroll
   for (int e = 0; e < 16; ++e) acc[0][0][e] = (int)kAccBias;
   store_a(0);

@@ -34,6 +34,8 @@ struct GemmArgs {
   int tiles_m, tiles_n;
   void *c;
   int64_t ldc;
+  uint32_t group_magic;  // quotients by 4 * tiles_n (see magic31)
+  int group_shift;
 };
 
 // The arguments of one matrix as they travel; w: the form of the weights that the kernel reads, c: rows of n values.
@@ -43,19 +45,30 @@ struct GemmCall {
   const int8_t *a, *w;
   void *c;
   int m, n, k, lda, tiles_m, tiles_n;
+  uint32_t group_magic;
+  int group_shift;
   Epi epi;
   static GemmCall of(const GemmArgs &g, const int8_t *w, int tile_n, int tile_m, const RequantParams &rq, const DequantParams &dq) {
-    GemmCall call{g.a, w, g.c, g.m, g.n, g.k, (int)g.lda, (g.m + tile_m - 1) / tile_m, (g.n + tile_n - 1) / tile_n, {}};
+    GemmCall call{g.a, w, g.c, g.m, g.n, g.k, (int)g.lda, (g.m + tile_m - 1) / tile_m, (g.n + tile_n - 1) / tile_n, 0, 0, {}};
+    magic31(4 * call.tiles_n, &call.group_magic, &call.group_shift);
     if constexpr (EPI == EPI_REQUANT) call.epi = RequantCall::of(rq);
     else call.epi = DequantCall::of(dq, g.k);
     return call;
   }
   dim3 grid() const { return dim3(tiles_m * tiles_n); }
   __device__ __forceinline__ void open(GemmArgs *g, RequantParams *rq, DequantParams *dq) const {
+    // all arguments in one go: left to itself the compiler loads some where they are used, one way to memory behind the other
+    asm volatile("" ::"s"(a), "s"(w), "s"(c), "s"(m), "s"(n), "s"(k), "s"(lda), "s"(tiles_m), "s"(tiles_n), "s"(group_magic),
+                 "s"(group_shift), "s"(epi.channels));
     const int k_pad = padded_k(k);
-    *g = GemmArgs{a, lda, m, k, w, weight_row_stride(k_pad), k_pad, w, n, tiles_m, tiles_n, c, n};
-    if constexpr (EPI == EPI_REQUANT) *rq = epi.open(n);
-    else *dq = epi.open(n, k);
+    *g = GemmArgs{a, lda, m, k, w, weight_row_stride(k_pad), k_pad, w, n, tiles_m, tiles_n, c, n, group_magic, group_shift};
+    if constexpr (EPI == EPI_REQUANT) {
+      asm volatile("" ::"s"(epi.zo), "s"(epi.amin), "s"(epi.amax), "s"(epi.forms));
+      *rq = epi.open(n);
+    } else {
+      asm volatile("" ::"s"(epi.qp_dev), "s"(epi.sx), "s"(epi.zx), "s"(epi.zw0), "s"(epi.forms));
+      *dq = epi.open(n, k);
+    }
   }
 };
 static_assert(sizeof(GemmCall<EPI_REQUANT>) <= kShortArgs && sizeof(GemmCall<EPI_DEQUANT>) <= kShortArgs, "see launch_args.h");
@@ -73,16 +86,19 @@ __device__ __forceinline__ int xcd_order(int id, int grid) {
   const int per = grid >> 3;
   return id < per * 8 ? (id & 7) * per + (id >> 3) : id;
 }
+template <bool MAGIC = true>  // false: g has no group_magic
 __device__ __forceinline__ void tile_of(const GemmArgs &g, int id, int *tile_m, int *tile_n) {
   constexpr int G = 4;
   const int width = G * g.tiles_n;
-  const int group = id / width, first = group * G;
-  const int gsize = min(g.tiles_m - first, G);
-  *tile_m = first + (id % width) % gsize;
-  *tile_n = (id % width) / gsize;
+  const int group = MAGIC ? quotient31(id, g.group_magic, g.group_shift) : id / width, first = group * G;
+  const int gsize = min(g.tiles_m - first, G), rest = id - group * width;
+  // (rest < 2^29, so that its third, by a factor just above 2^32 / 3, is exact)
+  *tile_n = gsize == 4 ? rest >> 2 : gsize == 3 ? (int)__umulhi((uint32_t)rest, 0x55555556u) : gsize == 2 ? rest >> 1 : rest;
+  *tile_m = first + rest - *tile_n * gsize;
 }
+template <bool MAGIC = true>
 __device__ __forceinline__ void tile_coords(const GemmArgs &g, int *tile_m, int *tile_n) {
-  tile_of(g, xcd_order((int)blockIdx.x, g.tiles_m * g.tiles_n), tile_m, tile_n);
+  tile_of<MAGIC>(g, xcd_order((int)blockIdx.x, g.tiles_m * g.tiles_n), tile_m, tile_n);
 }
 
 // Several weight matrices with the same K against the same activation rows as one launch: their column tiles stand side by
@@ -131,6 +147,7 @@ int group_tiles(GemmGroup<P> *grp, int tile_n, int tile_m) {
     grp->first_tile[i] = grp->g.tiles_n;
     grp->g.tiles_n += (grp->n[i] + tile_n - 1) / tile_n;
   }
+  magic31(4 * grp->g.tiles_n, &grp->g.group_magic, &grp->g.group_shift);
   return grp->g.tiles_m * grp->g.tiles_n;
 }
 
@@ -222,25 +239,35 @@ struct EpiParams {
 
 // What the fp32 epilogue needs of the input's quantisation.  With DynamicQuant upstream the values live in device
 // memory; they are fetched before the main loop, which hides a dependent load of a microsecond that would otherwise
-// sit between the last MFMA and the first store of every tile.
+// sit between the last MFMA and the first store of every tile.  The rows' scales are vector loads, which the main loops want ahead of
+// their own; the tensor's come by scalar loads, and every scalar wait is for all of them: asked for before the first operand loads,
+// they held those up by their whole way to memory.
 template <int TM>
 struct DeqInput {
   float sx;
   int32_t zx;
   float sxr[TM];  // per_row: the scale of the rows this lane holds
-  __device__ __forceinline__ void fetch(const DequantParams &dq, int m_w, int r, int m_total) {
+  __device__ __forceinline__ void fetch_rows(const DequantParams &dq, int m_w, int r, int m_total) {
+    // input_per_channel_: one input scale per row (NN/int8/dynamic_matmul_int8.c:126-128)
+    if (!dq.per_row) return;
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+      int m = m_w + j * 32 + r;
+      m = m < m_total ? m : m_total - 1;
+      sxr[j] = dq.qp_dev[m].scale_f;
+    }
+  }
+  __device__ __forceinline__ void fetch_tensor(const DequantParams &dq) {  // behind the first operand loads
+    asm volatile("" ::: "memory");
     sx = dq.sx;
     zx = dq.zx;
     if (dq.qp_dev != nullptr) {
       sx = dq.qp_dev->scale_f;
       zx = dq.qp_dev->zero_point;
     }
-    // input_per_channel_: one input scale per row (NN/int8/dynamic_matmul_int8.c:126-128)
+    if (!dq.per_row) {
 #pragma unroll
-    for (int j = 0; j < TM; ++j) {
-      int m = m_w + j * 32 + r;
-      m = m < m_total ? m : m_total - 1;
-      sxr[j] = dq.per_row ? dq.qp_dev[m].scale_f : sx;
+      for (int j = 0; j < TM; ++j) sxr[j] = sx;
     }
   }
 };

@@ -118,7 +118,7 @@ __device__ __forceinline__ void gemm_direct_body(const GemmArgs &g, const Requan
   __shared__ __attribute__((aligned(1024))) char lds[NST * STAGE];
 
   int tile_m, tile_n;
-  tile_coords(g, &tile_m, &tile_n);
+  tile_coords<!CONV>(g, &tile_m, &tile_n);
   const int m0 = tile_m * TILE_M, n0 = tile_n * TILE_N;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -129,7 +129,7 @@ __device__ __forceinline__ void gemm_direct_body(const GemmArgs &g, const Requan
   EpiParams<TILE_N, EPI, FAST> epi;
   epi.fetch(rq, dq, n0, g.n, tid);
   DeqInput<TM> din;
-  if (EPI == EPI_DEQUANT) din.fetch(dq, m0 + wm * WM, r, g.m);
+  if (EPI == EPI_DEQUANT) din.fetch_rows(dq, m0 + wm * WM, r, g.m);
 
   // loader: a 1 KiB block holds 16 rows x 64 B.  Lane L fills slot (L & 3) of row (L >> 2) of its block, i.e. it
   // fetches logical chunk (L & 3) ^ swizzle(row), swizzle(row) = (row >> 1) & 3.
@@ -253,6 +253,7 @@ __device__ __forceinline__ void gemm_direct_body(const GemmArgs &g, const Requan
   };
 #pragma unroll
   for (int t = 0; t < PD; ++t) dma_tile(t, t < ktiles ? t : ktiles - 1);
+  if (EPI == EPI_DEQUANT) din.fetch_tensor(dq);
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((PD - 1) * LPW) : "memory");
   read_frag(f0, 0, 0);
   if constexpr (NST <= 4) {
@@ -317,7 +318,7 @@ template <int TILE_N, int TILE_M, bool HAS_ZW, bool FAST, int NST, int OCC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void gemm_conv_kernel(ConvCall call) {
   const int k_pad = padded_k(call.k);
   const GemmArgs g{call.in, 0, call.m, call.k, call.w, weight_row_stride(k_pad), k_pad, nullptr, call.n,
-                   (call.m + TILE_M - 1) / TILE_M, (call.n + TILE_N - 1) / TILE_N, call.c, call.n};
+                   (call.m + TILE_M - 1) / TILE_M, (call.n + TILE_N - 1) / TILE_N, call.c, call.n, 0, 0};
   gemm_direct_body<TILE_N, TILE_M, EPI_REQUANT, HAS_ZW, FAST, NST, true>(g, call.epi.open(call.n), DequantParams{}, call.cv,
                                                                          call.fill16);
 }

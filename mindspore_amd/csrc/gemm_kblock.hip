@@ -61,7 +61,7 @@ __device__ __forceinline__ void gemm_kblock_body(const GemmArgs &g, const Requan
   EpiParams<TILE_N, EPI, FAST> epi;
   epi.fetch(rq, dq, n0, g.n, tid);
   DeqInput<TM> din;
-  if (EPI == EPI_DEQUANT) din.fetch(dq, m0 + wm * 32 * TM, r, g.m);
+  if (EPI == EPI_DEQUANT) din.fetch_rows(dq, m0 + wm * 32 * TM, r, g.m);
 
   // loader: a wave fills a quarter of each slot, 16 T rows, 8 per instruction: instruction i takes rows
   // 16 T * wave + 8 * i + (lane >> 3); lane L writes position L & 7 of its row, i.e. fetches logical chunk
@@ -212,6 +212,7 @@ __device__ __forceinline__ void gemm_kblock_body(const GemmArgs &g, const Requan
   dma_w(1, last < 1 ? last : 1, 0);
   dma_w(1, last < 1 ? last : 1, 1);
   dma_a(1, last < 1 ? last : 1, 0);
+  if (EPI == EPI_DEQUANT) din.fetch_tensor(dq);
   init_accumulators();
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * TN + TM) : "memory");  // W(0) and A(0) are in
   read_frag(f0, 0, 0, 0);

@@ -56,7 +56,7 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs &g, const RequantP
   EpiParams<TILE_N, EPI, FAST> epi;
   epi.fetch(rq, dq, n0, g.n, tid);
   DeqInput<TM> din;
-  if (EPI == EPI_DEQUANT) din.fetch(dq, m0 + wm * 32 * TM, r, g.m);
+  if (EPI == EPI_DEQUANT) din.fetch_rows(dq, m0 + wm * 32 * TM, r, g.m);
 
   // loader.  W comes from the blocked copy: a wave takes TN groups of 16 channels, and an instruction fetches one 1 KiB
   // block (16 channels x 64 bytes of K, chunk by chunk: [chunk][channel]) front to back into the same order in LDS,
@@ -172,6 +172,7 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs &g, const RequantP
     if (last == S - 1) a_offsets_for_last_block();
     dma(S - 1, S - 1, at0(), at1());
   }
+  if (EPI == EPI_DEQUANT) din.fetch_tensor(dq);
   // the accumulator registers are set while the first tiles are on their way
 #pragma unroll
   for (int i = 0; i < TN; ++i)
