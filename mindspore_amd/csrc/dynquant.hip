@@ -208,9 +208,15 @@ __device__ __forceinline__ void publish_to_host(const DqHostNote &note, float sc
 // numbers from memory: a workgroup that has given up waiting raises the number past its own tag too, and one that has not has
 // seen its tag in slot 0, whose writer raises it, so in the end it is past every tag that was left in a slot.
 //
-// us per launch, eager / replayed: 8 x 4096 4.1 / 4.1, 8 x 11008 4.4 / 4.3, 4096 x 768 8.1 / 8.2, 4096 x 3072 17.2 / 17.3 (slots
-// without tags that were emptied in turn, whose turn it was in a word per slot: 4.3 / 4.1, 4.6 / 4.4, 8.4 / 8.5, 17.5 / 17.6; two
-// 8-byte loads per slot instead of one of 16: 4.5 / 4.4, 4.6 / 4.6, 8.8 / 8.9, 17.6 / 17.6).
+// (Slots without tags that were emptied in turn, whose turn it was in a word per slot, took 0.2 us more; two 8-byte loads per slot
+// instead of one of 16 0.3 to 0.7.)
+//
+// A workgroup looks at the slots for the first time when the others' words can be there (400 to 700 ns after its own, more with more
+// values a workgroup, whose arrival spreads further).  A look that comes too early costs its whole way to memory and back, and 256
+// workgroups looking over and over get in the way of the words they look for.  us per launch from a graph, first look at once / after
+// this pause / twice it: 8 x 4096 4.15 / 3.93 / 4.4, 8 x 11008 4.7 / 4.15 / 4.5, 197 x 768 4.33 / 3.95 / 4.4, 197 x 3072 6.5 / 5.5 / 5.8,
+// 481 x 2304 6.6 / 5.7, 4096 x 768 8.0 / 6.85, 4096 x 3072 17.2 / 16.55; with pauses between looks too 1 to 3 % more, with two or three
+// looks on their way at once 0.4 to 0.7 us more than without any.
 //
 // The wait is bounded: workgroups that are not resident together (the device is shared) are not waited for for ever; a
 // workgroup that has waited `patience` ticks of the 100 MHz counter reads the whole tensor itself.
@@ -276,6 +282,7 @@ __global__ __launch_bounds__(T) void dq_fused_kernel(const float *__restrict__ x
         __hip_atomic_store(&slots->range[s][0], my_lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_store(&slots->range[s][1], my_hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
+      __builtin_amdgcn_s_sleep(T * G <= 512 ? 14 : T * G <= 2048 ? 20 : 24);  // (see above)
       const uint64_t began = __builtin_amdgcn_s_memrealtime();
       bool late = false;
       // (16 bytes a load, past the caches of this XCD: two words that need not belong together, hence a tag in each)
@@ -541,7 +548,7 @@ static void launch_fused(const float *x, int64_t n, int symmetric, void *slots, 
 int launch_dynquant(const float *x, int64_t n, int symmetric, float2 *partials, void *slots, uint32_t launch,
                     const DqHostNote &note, mi_dq_params *params, int8_t *q, hipStream_t stream) {
   // One launch as long as the tensor fits the registers of one workgroup per CU.  Up to 8192 values one workgroup is
-  // faster than any exchange (about 1.2 us); from there on as many workgroups as there are slots, with the fewest
+  // faster than any exchange (about 0.9 us); from there on as many workgroups as there are slots, with the fewest
   // values per thread that allows: what counts at these sizes is the latency of each thread's chain.  us per tensor,
   // before (up to 24576 values one workgroup, else two launches) -> now: 4096 3.9 -> 2.9, 16384 5.9 -> 3.7,
   // 32768 7.2 -> 4.2, 88064 7.4 -> 4.4, 300000 7.7 -> 5.0, 1 M 8.0 -> 5.6, 4096 x 768 11.3 -> 8.9,
