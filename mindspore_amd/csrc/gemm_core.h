@@ -626,6 +626,37 @@ struct Frag {
   v4i w[TN], a[TM];
 };
 
+// Sums of the activation rows, which weights with zero points need: one v_mfma_i32_16x16x64_i8 for 32 bytes of K of 32 rows.
+// In the fragment of a 32x32x32 product lane 32 h + r holds 16 bytes of row r; the 16x16x64 product takes lane 16 c + i as 16
+// bytes of its column i.  Rows 16 .. 31 are then chunks c = 1 and 3 of columns 0 .. 15: four rows of its other operand with
+// ones at chunks 0 and 2 add up rows 0 .. 15, four with ones at 1 and 3 the rest, and the sum of row r arrives in lane r.
+// For gemm_ring.h: v_dot4, four for as many bytes, take 15 cycles each there and keep the wave from issuing anything else,
+// while the matrix cores are idle for most of a small tile.  us with v_dot4 -> this (without zero points): 128 x 2048 x 1024
+// 7.25 -> 6.05 (5.6), 400 x 2048 x 1024 7.45 -> 6.25 (5.7), 333 x 1024 x 1024 5.25 -> 4.9 (4.35), 128 x 4096 x 4096 in parts 11.0 ->
+// 10.4 (9.4).  The loops that hide the v_dot4 behind their own products gain nothing and keep them: 128 x 128 tiles 24.0 -> 24.0,
+// gemm_anyrow.hip 5.45 -> 5.5.
+template <int TM>
+struct RowSums {
+  v4i sum[TM];
+  int ones;
+  __device__ __forceinline__ void clear(int lane) {
+    const int i = lane & 15, c = lane >> 4;
+    ones = (i >> 2) < 2 && (c & 1) == (i >> 2) ? 0x01010101 : 0;
+#pragma unroll
+    for (int j = 0; j < TM; ++j) sum[j] = v4i{0, 0, 0, 0};
+  }
+  // live: this lane's 16 bytes lie inside K
+  __device__ __forceinline__ void add(const v4i (&a)[TM], bool live) {
+    const int o = live ? ones : 0;
+#pragma unroll
+    for (int j = 0; j < TM; ++j) sum[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(v4i{o, o, o, o}, a[j], sum[j], 0, 0, 0);
+  }
+  __device__ __forceinline__ void get(int (&rowsum)[TM]) const {
+#pragma unroll
+    for (int j = 0; j < TM; ++j) rowsum[j] = sum[j][0];
+  }
+};
+
 // Launches of the K-block loops (gemm_kblock.hip, gemm_ring.hip), one per tile shape: T = 10 x TN + TM, the workgroup's
 // tile being 64 TN channels x 64 TM rows.  requant: int8 output, fast2 form or not; otherwise fp32, `fast` = non-temporal
 // stores.

@@ -106,9 +106,8 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs &g, const RequantP
   typedef std::integral_constant<int, LPB> at2;
 
   v16i acc[TN][TM];
-  int rowsum[TM];
-#pragma unroll
-  for (int j = 0; j < TM; ++j) rowsum[j] = 0;
+  RowSums<TM> sums;
+  if (HAS_ZW) sums.clear(lane);
 
   const int swz = (r >> 1) & 7;
   const int w_off = (wn * 2 * TN + (r >> 4)) * 2048 + h * 256 + (r & 15) * 16, a_off = TILE_N * KB + (wm * 32 * TM + r) * KB;
@@ -124,19 +123,8 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs &g, const RequantP
       for (int j = 0; j < TM; ++j) f[q].a[j] = *reinterpret_cast<const v4i *>(ab + j * 32 * KB);
     }
   };
-  auto mma = [&](const Frag<TN, TM> &f, int chunk) {
-    if (HAS_ZW) {
-      const int ones = chunk < kchunks ? 0x01010101 : 0;
-#pragma unroll
-      for (int j = 0; j < TM; ++j) {
-        int t = rowsum[j];
-        t = __builtin_amdgcn_sdot4(f.a[j].x, ones, t, false);
-        t = __builtin_amdgcn_sdot4(f.a[j].y, ones, t, false);
-        t = __builtin_amdgcn_sdot4(f.a[j].z, ones, t, false);
-        t = __builtin_amdgcn_sdot4(f.a[j].w, ones, t, false);
-        rowsum[j] = t;
-      }
-    }
+  auto mma = [&](const Frag<TN, TM> &f, bool live) {  // live: the lane's 16 activation bytes lie inside K
+    if (HAS_ZW) sums.add(f.a, live);
 #pragma unroll
     for (int i = 0; i < TN; ++i)
 #pragma unroll
@@ -147,7 +135,7 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs &g, const RequantP
   };
   // order of one half: the fragment reads behind the first MFMAs, the loads behind the others
   auto hints = [&](auto loads_c) {
-    constexpr int LOADS = decltype(loads_c)::value, MF = 2 * TN * TM, RD = 2 * (TN + TM);
+    constexpr int LOADS = decltype(loads_c)::value, MF = 2 * (TN + HAS_ZW) * TM, RD = 2 * (TN + TM);
     constexpr int first = (MF + 1) / 2, rest = MF - first;
 #pragma unroll
     for (int m = 0; m < first; ++m) {
@@ -196,8 +184,8 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs &g, const RequantP
   while (b + S - 1 <= last) {
     read_half(fb, st, 1);
     dma(prev, b + S - 1, at1(), at2());
-    mma(fa[0], (first_block + b) * 8 + h);
-    mma(fa[1], (first_block + b) * 8 + 2 + h);
+    mma(fa[0], true);
+    mma(fa[1], true);
     hints(std::integral_constant<int, LPB - PART>());
     // loads complete in order: blocks b + 2 .. b + S - 1 may still be on their way, block b + 1 is in
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * LPB) : "memory");
@@ -205,15 +193,15 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs &g, const RequantP
     if (b + S == last) a_offsets_for_last_block();
     read_half(fa, next, 0);
     dma(st, b + S < last ? b + S : last, at0(), at1());  // (past the end: into a stage nobody reads any more)
-    mma(fb[0], (first_block + b) * 8 + 4 + h);
-    mma(fb[1], (first_block + b) * 8 + 6 + h);
+    mma(fb[0], true);
+    mma(fb[1], true);
     hints(std::integral_constant<int, PART>());
     advance();
   }
   while (b <= last) {  // the last blocks: nothing left to request
     read_half(fb, st, 1);
-    mma(fa[0], (first_block + b) * 8 + h);
-    mma(fa[1], (first_block + b) * 8 + 2 + h);
+    mma(fa[0], (first_block + b) * 8 + h < kchunks);
+    mma(fa[1], (first_block + b) * 8 + 2 + h < kchunks);
     hints(at0());
     const int later = last - b - 1;  // blocks behind b + 1 that may still be on their way
     if (S > 3 && later >= 2) {
@@ -226,13 +214,15 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs &g, const RequantP
     asm volatile("s_barrier" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
     read_half(fa, next, 0);  // (behind the last block: bytes nobody uses)
-    mma(fb[0], (first_block + b) * 8 + 4 + h);
-    mma(fb[1], (first_block + b) * 8 + 6 + h);
+    mma(fb[0], (first_block + b) * 8 + 4 + h < kchunks);
+    mma(fb[1], (first_block + b) * 8 + 6 + h < kchunks);
     hints(at0());
     advance();
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every load has landed before the LDS is reused
   __syncthreads();
+  int rowsum[TM] = {};
+  if (HAS_ZW) sums.get(rowsum);
   if constexpr (SPLIT) {
     if (!add_parts<TN, TM, HAS_ZW>(kp, acc, rowsum, reinterpret_cast<int *>(lds), tid)) return;
   }

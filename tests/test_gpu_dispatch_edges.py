@@ -789,3 +789,23 @@ def test_matmul_with_k_in_parts_on_library_streams():
     for t in threads:
         t.join()
     assert not failed
+
+
+# row sums on the matrix cores: K that ends at every 16 bytes of a block of 128, fewer blocks than stages and more, rows and
+# channels that end inside a tile; extreme values, whose sums are the largest
+@pytest.mark.parametrize("k", [16, 48, 128, 144, 176, 400, 640, 1008, 1040, 2032, 4112])
+@pytest.mark.parametrize("m,n", [(65, 65), (131, 300), (200, 1000)])
+@pytest.mark.parametrize("dynamic", [False, True])
+def test_matmul_row_sums(orc, m, n, k, dynamic):
+    import torch
+    rng = np.random.default_rng(m + n + k)
+    w, bias, sw, zw, make = _matmul_pair(rng, n, k, True, dynamic)
+    a = rng.integers(-128, 128, (m, k), dtype=np.int8)
+    a[1], a[m // 2], a[m - 1] = -128, 127, -128
+    orc.set_threads(16)
+    if dynamic:
+        want = orc.dynamic_matmul(a, w, bias, 0.03, -5, sw, zw)
+    else:
+        want = orc.matmul_int8(a, w, bias, 0.02, 7, sw, zw, float(np.float32(0.02 * 0.0055 * k ** 0.5 * 140)), 3)
+    args = dict(in_quant=K.QuantParam(0.03, -5)) if dynamic else {}
+    assert np.array_equal(make(True).run(torch.from_numpy(a).cuda(), **args).cpu().numpy(), want)
