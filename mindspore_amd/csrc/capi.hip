@@ -537,6 +537,8 @@ static bool runs_on_anyrow(const RequantState &st, const int8_t *a_dev, int rows
 static int run_requant_rows(RequantState &st, const int8_t *a_dev, int rows, const Workspace &ws, int8_t *c, hipStream_t stream) {
   if (runs_on_anyrow(st, a_dev, rows))
     return launch_gemm_anyrow_requant(a_dev, rows, st.k, weight_view(st), st.n, st.params(), c, stream);
+  if (runs_on_gemv(st, rows, round_up(st.k, 16)) && gemv_takes_any_rows(rows, st.k, weight_view(st), st.n))
+    return launch_gemv_requant(a_dev, st.k, rows, st.k, weight_view(st), st.n, st.params(), c, st.n, stream);
   const int8_t *a = nullptr;
   int64_t lda = 0;
   int k16 = 0;
@@ -1628,6 +1630,8 @@ static int dynmm_run_impl(mi_dynmm *h, const int8_t *a_dev, int32_t rows, float 
   const DequantParams dq = dequant_params(h, sx, zx, qp_dev, per_row);
   if (runs_on_anyrow(h, a_dev, rows))
     return launch_gemm_anyrow_dequant(a_dev, rows, h->k, weight_view(h), h->n, dq, c_dev, s);
+  if (runs_on_gemv(h, rows) && gemv_takes_any_rows(rows, h->k, weight_view(h), h->n))
+    return launch_gemv_dequant(a_dev, h->k, rows, h->k, weight_view(h), h->n, dq, c_dev, h->n, s);
   const int8_t *a = nullptr;
   int64_t lda = 0;
   int k16 = 0;

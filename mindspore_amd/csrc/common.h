@@ -181,6 +181,10 @@ constexpr int kGemvDotRows = 2;  // up to here the v_dot4 kernel can run (it doe
 int launch_gemv_requant(const int8_t *a, int64_t lda, int m, int k, const WeightView &w, int n,
                         const RequantParams &rq, int8_t *c, int64_t ldc, hipStream_t stream);
 
+// Whether the two launches around here also take m rows of k bytes that are no whole 16-byte chunks, or not aligned to them,
+// as they are; they then lie end to end (lda == k).
+bool gemv_takes_any_rows(int m, int k, const WeightView &w, int n);
+
 // 1..64 rows of the dynamic-quant MatMul (fp32 out) on the blocked weight copy (w.blocked must be there).
 int launch_gemv_dequant(const int8_t *a, int64_t lda, int m, int k, const WeightView &w, int n,
                         const DequantParams &dq, float *c, int64_t ldc, hipStream_t stream);

@@ -42,10 +42,23 @@ __device__ __forceinline__ int dot16(v4i w, v4i a, int acc) {
   return acc;
 }
 
+// Activation rows of K bytes, K no whole 16-byte chunks or the first row at any address (ANY below; the rows lie end to end, so K
+// is their stride).  A chunk that would reach past its row is fetched as the row's last 16 bytes ...
+typedef v4i v4i_byte __attribute__((aligned(1)));
+__device__ __forceinline__ v4i fetch_any(const int8_t *row, int at, int k) {
+  return *reinterpret_cast<const v4i_byte *>(row + (at + 16 <= k ? at : k - 16));
+}
+// ... and moved to its place, with zeros behind the row's end.
+__device__ __forceinline__ v4i end_any(v4i v, int at, int k) {
+  const int over = at + 16 - k;
+  const unsigned __int128 x = __builtin_bit_cast(unsigned __int128, v);
+  return over > 0 ? __builtin_bit_cast(v4i, x >> (8 * (over & 15))) : v;
+}
+
 struct GemvArgs {
   const int8_t *a;
   int64_t lda;
-  int kchunks;  // K / 16
+  int kchunks;  // K / 16, rounded up
   const int8_t *w;
   int ldw;    // weight row stride in bytes
   int k_pad;  // contraction extent of a (zero padded) weight row
@@ -88,12 +101,14 @@ static_assert(sizeof(GemvCall<false>) <= kShortArgs && sizeof(GemvCall<true>) <=
 // KS = 2: two neighbouring waves share their R rows, each walks one half of K (long rows: twice the waves, each with
 // half the registers, so that more of them are resident), and the even wave adds the odd wave's sums through LDS.
 // DEQ: the fp32 epilogue of the dynamic-quant MatMul (see gemv_mfma_lds_body) instead of the requantising one.
-template <int M, int R, int D, bool DIRECT, int KS, bool DEQ = false>
+// ANY: one row of any length at any address (see fetch_any).
+template <int M, int R, int D, bool DIRECT, int KS, bool DEQ, bool ANY>
 __device__ __forceinline__ void gemv_i8_body(const GemvArgs &g, const RequantParams &rq, const DequantParams &dq,
                                              int block) {
   const bool has_zw = DEQ ? dq.zw0 != 0 : rq.has_zw != 0;
   static_assert(D % R == 0, "the slot -> row mapping must be static");
   static_assert(KS == 1 || KS == 2, "one or two waves per row group");
+  static_assert(!ANY || M == 1, "one row");
   extern __shared__ __attribute__((aligned(16))) char smem[];
   v4i *sa = reinterpret_cast<v4i *>(smem);  // [M][nseg_all * 64], zero past K
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -116,6 +131,7 @@ __device__ __forceinline__ void gemv_i8_body(const GemvArgs &g, const RequantPar
     int off = seg * 1024 + lane * 16;
     off = off < last_off ? off : last_off;
     const int8_t *p = live ? wrow + (int64_t)rr * g.ldw + off : g.a;
+    if constexpr (ANY) return __builtin_nontemporal_load(reinterpret_cast<const v4i_byte *>(p));
     return __builtin_nontemporal_load(reinterpret_cast<const v4i *>(p));
   };
   v4i buf[D];
@@ -171,7 +187,9 @@ __device__ __forceinline__ void gemv_i8_body(const GemvArgs &g, const RequantPar
       for (int m = 0; m < M; ++m) {
         const int chunk = (seg0 + sgi) * 64 + lane;
         const bool live = chunk < g.kchunks && sgi < nseg;
-        if constexpr (DEQ) {
+        if constexpr (ANY) {
+          apre[sgi][m] = fetch_any(g.a, live ? chunk * 16 : 0, (int)g.lda);
+        } else if constexpr (DEQ) {
           apre[sgi][m] = __builtin_bit_cast(
               v4i, __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, live ? m * (int)g.lda + chunk * 16 : kOutOfRange, 0, 0));
         } else {
@@ -183,13 +201,24 @@ __device__ __forceinline__ void gemv_i8_body(const GemvArgs &g, const RequantPar
           apre[sgi][m].w = live ? v.w : 0;
         }
       }
+    if constexpr (ANY) {
+#pragma unroll
+      for (int sgi = 0; sgi < D / R; ++sgi) {
+        const int chunk = (seg0 + sgi) * 64 + lane;
+        const bool live = chunk < g.kchunks && sgi < nseg;
+        v4i v = apre[sgi][0];
+        if (seg0 + sgi == nseg_all - 1) v = end_any(v, chunk * 16, (int)g.lda);  // (wave-uniform)
+        apre[sgi][0] = live ? v : v4i{0, 0, 0, 0};
+      }
+    }
   } else {
 #pragma unroll
     for (int m = 0; m < M; ++m) {
       const v4i *arow = reinterpret_cast<const v4i *>(g.a + (int64_t)m * g.lda);
       for (int ch = tid; ch < kc_pad; ch += 256) {
         v4i z = {0, 0, 0, 0};
-        sa[m * kc_pad + ch] = ch < g.kchunks ? arow[ch] : z;
+        if constexpr (ANY) sa[ch] = ch < g.kchunks ? end_any(fetch_any(g.a, ch * 16, (int)g.lda), ch * 16, (int)g.lda) : z;
+        else sa[m * kc_pad + ch] = ch < g.kchunks ? arow[ch] : z;
       }
     }
     __syncthreads();
@@ -295,20 +324,20 @@ __device__ __forceinline__ void gemv_i8_body(const GemvArgs &g, const RequantPar
   }
 }
 
-template <int M, int R, int D, bool DIRECT, int KS>
+template <int M, int R, int D, bool DIRECT, int KS, bool ANY>
 __global__ __launch_bounds__(256) void gemv_i8_kernel(GemvCall<false> call) {
   GemvArgs g;
   RequantParams rq;
   call.open(&g, &rq);
-  gemv_i8_body<M, R, D, DIRECT, KS, false>(g, rq, DequantParams{}, (int)blockIdx.x);
+  gemv_i8_body<M, R, D, DIRECT, KS, false, ANY>(g, rq, DequantParams{}, (int)blockIdx.x);
 }
 
-template <int M, int R, int D, bool DIRECT, int KS>
+template <int M, int R, int D, bool DIRECT, int KS, bool ANY>
 __global__ __launch_bounds__(256) void gemv_i8_deq_kernel(GemvCall<true> call) {
   GemvArgs g;
   DequantParams dq;
   call.open(&g, &dq);
-  gemv_i8_body<M, R, D, DIRECT, KS, true>(g, RequantParams{}, dq, (int)blockIdx.x);
+  gemv_i8_body<M, R, D, DIRECT, KS, true, ANY>(g, RequantParams{}, dq, (int)blockIdx.x);
 }
 
 // Several weight matrices against the same activation rows in one launch (MatMuls that share their input, e.g. the
@@ -430,7 +459,7 @@ __global__ __launch_bounds__(256) void gemv_i8_group_kernel(GemvGroupCall<N, Req
   RequantParams rq;
   int block;
   pick_member(call, &g, &rq, &block);
-  gemv_i8_body<M, R, D, DIRECT, KS, false>(g, rq, DequantParams{}, block);
+  gemv_i8_body<M, R, D, DIRECT, KS, false, false>(g, rq, DequantParams{}, block);
 }
 
 template <int M, int R, int D, bool DIRECT, int KS, int N>
@@ -439,12 +468,12 @@ __global__ __launch_bounds__(256) void gemv_i8_group_deq_kernel(GemvGroupCall<N,
   DequantParams dq;
   int block;
   pick_member(call, &g, &dq, &block);
-  gemv_i8_body<M, R, D, DIRECT, KS, true>(g, RequantParams{}, dq, block);
+  gemv_i8_body<M, R, D, DIRECT, KS, true, false>(g, RequantParams{}, dq, block);
 }
 
-template <int M, int R, int D, bool DIRECT, int KS>
+template <int M, int R, int D, bool DIRECT, int KS, bool ANY>
 static int launch_mrdx(const GemvArgs &g, const RequantParams &rq, hipStream_t stream) {
-  auto kern = gemv_i8_kernel<M, R, D, DIRECT, KS>;
+  auto kern = gemv_i8_kernel<M, R, D, DIRECT, KS, ANY>;
   // (more than 64 KiB of dynamic LDS needs the attribute that gemv_prepare_device set when the library was initialised)
   const int lds_bytes = DIRECT ? 0 : M * ((g.kchunks + 63) / 64) * 1024;
   const int rows_per_block = 4 / KS * R;
@@ -454,12 +483,12 @@ static int launch_mrdx(const GemvArgs &g, const RequantParams &rq, hipStream_t s
   return MI_OK;
 }
 
-template <int M, int R, int D, bool DIRECT, int KS>
+template <int M, int R, int D, bool DIRECT, int KS, bool ANY>
 static int launch_mrdx_deq(const GemvArgs &g, const DequantParams &dq, hipStream_t stream) {
   const int lds_bytes = DIRECT ? 0 : M * ((g.kchunks + 63) / 64) * 1024;
   const int rows_per_block = 4 / KS * R;
   const int blocks = (g.n + rows_per_block - 1) / rows_per_block;
-  hipLaunchKernelGGL((gemv_i8_deq_kernel<M, R, D, DIRECT, KS>), dim3(blocks), dim3(256), lds_bytes, stream,
+  hipLaunchKernelGGL((gemv_i8_deq_kernel<M, R, D, DIRECT, KS, ANY>), dim3(blocks), dim3(256), lds_bytes, stream,
                      GemvCall<true>::of(g, M, dq));
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
@@ -502,11 +531,13 @@ template <int M>
 static int allow_big_lds() {
   // the looping form stages the activation rows in dynamic LDS: up to 160 KiB
   auto allow = [](const void *kernel) { return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); };
-  MI_HIP_CHECK(allow(reinterpret_cast<const void *>(gemv_i8_kernel<M, 1, 12, false, 1>)));
+  MI_HIP_CHECK(allow(reinterpret_cast<const void *>(gemv_i8_kernel<M, 1, 12, false, 1, false>)));
   MI_HIP_CHECK(allow(reinterpret_cast<const void *>(gemv_i8_group_kernel<M, 1, 12, false, 1, 2>)));
   MI_HIP_CHECK(allow(reinterpret_cast<const void *>(gemv_i8_group_kernel<M, 1, 12, false, 1, kGemvGroupMax>)));
   if (M == 1) {
-    MI_HIP_CHECK(allow(reinterpret_cast<const void *>(gemv_i8_deq_kernel<1, 1, 12, false, 1>)));
+    MI_HIP_CHECK(allow(reinterpret_cast<const void *>(gemv_i8_kernel<1, 1, 12, false, 1, true>)));
+    MI_HIP_CHECK(allow(reinterpret_cast<const void *>(gemv_i8_deq_kernel<1, 1, 12, false, 1, true>)));
+    MI_HIP_CHECK(allow(reinterpret_cast<const void *>(gemv_i8_deq_kernel<1, 1, 12, false, 1, false>)));
     MI_HIP_CHECK(allow(reinterpret_cast<const void *>(gemv_i8_group_deq_kernel<1, 1, 12, false, 1, 2>)));
     MI_HIP_CHECK(allow(reinterpret_cast<const void *>(gemv_i8_group_deq_kernel<1, 1, 12, false, 1, kGemvGroupMax>)));
   }
@@ -556,10 +587,10 @@ static int launch_group_m(const GemvGroupT<P> &grp, hipStream_t stream) {  // th
   });
 }
 
-template <int M>
+template <int M, bool ANY>
 static int launch_m(const GemvArgs &g, const RequantParams &rq, hipStream_t stream) {
   return with_config<M>((g.kchunks + 63) >> 6, [&](auto r, auto d, auto direct, auto ks) {
-    return launch_mrdx<M, decltype(r)::value, decltype(d)::value, decltype(direct)::value, decltype(ks)::value>(
+    return launch_mrdx<M, decltype(r)::value, decltype(d)::value, decltype(direct)::value, decltype(ks)::value, ANY>(
         g, rq, stream);
   });
 }
@@ -601,7 +632,8 @@ static int launch_m(const GemvArgs &g, const RequantParams &rq, hipStream_t stre
 // mindspore/ccsrc/plugin/device/cpu/kernel/nnacl/int8/dynamic_matmul_int8.c:99-143) instead of the requantising one:
 // value = sum - zx * sum_k w - zw * sum_k a + K * zx * zw, out = (sx[row] * sw[c]) * (float)value (+ bias) (activation);
 // g.c then points at floats.
-template <int WAVES, int RG, int D, int MR, bool DEQ = false>
+// ANY: rows of any length at any address, through registers (see fetch_any) instead of the buffer descriptor.
+template <int WAVES, int RG, int D, int MR, bool DEQ, bool ANY>
 __device__ __forceinline__ void gemv_mfma_lds_body(const GemvArgs &g, int m_rows, const RequantParams &rq,
                                                    const DequantParams &dq, int block) {
   const bool has_zw = DEQ ? dq.zw0 != 0 : rq.has_zw != 0;
@@ -617,7 +649,7 @@ __device__ __forceinline__ void gemv_mfma_lds_body(const GemvArgs &g, int m_rows
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int grp = lane >> 4, idx = lane & 15;
   const int n0 = block * (RG * 16);
-  const int k_bytes = g.kchunks * 16;
+  const int k_bytes = ANY ? (int)g.lda : g.kchunks * 16;
   const int total = g.k_pad >> 6;  // 64-byte steps in a (zero padded) weight row
   const int spw = (total + WAVES - 1) / WAVES;
   const int s0 = wave * spw;
@@ -650,10 +682,19 @@ __device__ __forceinline__ void gemv_mfma_lds_body(const GemvArgs &g, int m_rows
     const int kb = (sw0 + base) * 64;
     const bool any = base < spw && sw0 + base < total && kb < k_bytes;  // (wave-uniform)
     const bool live = step < spw && sw0 + step < total && kb + a_chunk[i] * 16 < k_bytes;
+    if constexpr (ANY) {
+      const bool there = live && a_off[i] != kOutOfRange;
+      return fetch_any(g.a + (there ? a_off[i] - a_chunk[i] * 16 : 0), there ? kb + a_chunk[i] * 16 : 0, k_bytes);
+    }
     return __builtin_bit_cast(
         v4i, __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, live ? a_off[i] : kOutOfRange, any ? kb : 0, 0));
   };
   auto store_a = [&](int base, int i, v4i v) {
+    if constexpr (ANY) {  // (rows that do not exist are not read back)
+      const int step = base + (a_chunk[i] >> 2), at = (sw0 + base) * 64 + a_chunk[i] * 16;
+      if ((sw0 + base) * 64 + ROWB > k_bytes) v = end_any(v, at, k_bytes);  // (wave-uniform)
+      v = step < spw && at < k_bytes ? v : v4i{0, 0, 0, 0};
+    }
     if (a_dst[i] >= 0) *reinterpret_cast<v4i *>(area + a_dst[i]) = v;
   };
   auto load_w = [&](int j, int rg) -> v4i {
@@ -808,20 +849,20 @@ __device__ __forceinline__ void gemv_mfma_lds_body(const GemvArgs &g, int m_rows
   }
 }
 
-template <int WAVES, int RG, int D, int MR>
+template <int WAVES, int RG, int D, int MR, bool ANY>
 __global__ __launch_bounds__(WAVES * 64) void gemv_mfma_lds_kernel(GemvCall<false> call) {
   GemvArgs g;
   RequantParams rq;
   call.open(&g, &rq);
-  gemv_mfma_lds_body<WAVES, RG, D, MR, false>(g, call.m, rq, DequantParams{}, (int)blockIdx.x);
+  gemv_mfma_lds_body<WAVES, RG, D, MR, false, ANY>(g, call.m, rq, DequantParams{}, (int)blockIdx.x);
 }
 
-template <int WAVES, int RG, int D, int MR>
+template <int WAVES, int RG, int D, int MR, bool ANY>
 __global__ __launch_bounds__(WAVES * 64) void gemv_mfma_lds_deq_kernel(GemvCall<true> call) {
   GemvArgs g;
   DequantParams dq;
   call.open(&g, &dq);
-  gemv_mfma_lds_body<WAVES, RG, D, MR, true>(g, call.m, RequantParams{}, dq, (int)blockIdx.x);
+  gemv_mfma_lds_body<WAVES, RG, D, MR, true, ANY>(g, call.m, RequantParams{}, dq, (int)blockIdx.x);
 }
 
 template <int WAVES, int RG, int D, int MR, int N>
@@ -830,7 +871,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_mfma_lds_group_kernel(GemvGro
   RequantParams rq;
   int block;
   pick_member(call, &g, &rq, &block);
-  gemv_mfma_lds_body<WAVES, RG, D, MR, false>(g, call.ops.m, rq, DequantParams{}, block);
+  gemv_mfma_lds_body<WAVES, RG, D, MR, false, false>(g, call.ops.m, rq, DequantParams{}, block);
 }
 
 template <int WAVES, int RG, int D, int MR, int N>
@@ -839,7 +880,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_mfma_lds_group_deq_kernel(Gem
   DequantParams dq;
   int block;
   pick_member(call, &g, &dq, &block);
-  gemv_mfma_lds_body<WAVES, RG, D, MR, true>(g, call.ops.m, RequantParams{}, dq, block);
+  gemv_mfma_lds_body<WAVES, RG, D, MR, true, false>(g, call.ops.m, RequantParams{}, dq, block);
 }
 
 template <int WAVES, int D, typename F>
@@ -855,15 +896,17 @@ static int with_row_class(int m, F &&f) {  // rows rounded up to 2, 4, 8, 16 or 
 // 33..64 rows (against at most 4096 channels, see gemv_takes_rows): four groups of 16 activation rows against every weight
 // fragment, two steps per pass (the staging area of 64 rows and the accumulators leave room for no more).  Measured
 // against 64 x 64 GEMM tiles in us per launch at 64 rows: 4096 x 4096 11.0 -> 8.8, 4096 x 11008 27.5 -> 18.7.
+template <bool ANY>
 static int launch_mfma_lds_64(const GemvArgs &g, int m, const RequantParams &rq, hipStream_t stream) {
-  hipLaunchKernelGGL((gemv_mfma_lds_kernel<8, 1, 2, 64>), dim3((g.n + 15) / 16), dim3(512), 0, stream,
+  hipLaunchKernelGGL((gemv_mfma_lds_kernel<8, 1, 2, 64, ANY>), dim3((g.n + 15) / 16), dim3(512), 0, stream,
                      GemvCall<false>::of(g, m, rq));
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }
 
+template <bool ANY>
 static int launch_mfma_lds_deq_64(const GemvArgs &g, int m, const DequantParams &dq, hipStream_t stream) {
-  hipLaunchKernelGGL((gemv_mfma_lds_deq_kernel<8, 1, 2, 64>), dim3((g.n + 15) / 16), dim3(512), 0, stream,
+  hipLaunchKernelGGL((gemv_mfma_lds_deq_kernel<8, 1, 2, 64, ANY>), dim3((g.n + 15) / 16), dim3(512), 0, stream,
                      GemvCall<true>::of(g, m, dq));
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
@@ -883,11 +926,11 @@ static int launch_group_mfma_lds(const GemvGroupT<P> &grp, int m, hipStream_t st
   });
 }
 
-template <int WAVES, int RG, int D>
+template <int WAVES, int RG, int D, bool ANY>
 static int launch_mfma_lds(const GemvArgs &g, int m, const RequantParams &rq, hipStream_t stream) {
   const int blocks = (g.n + RG * 16 - 1) / (RG * 16);
   return with_row_class<WAVES, D>(m, [&](auto mr) {
-    hipLaunchKernelGGL((gemv_mfma_lds_kernel<WAVES, RG, D, decltype(mr)::value>), dim3(blocks), dim3(WAVES * 64), 0,
+    hipLaunchKernelGGL((gemv_mfma_lds_kernel<WAVES, RG, D, decltype(mr)::value, ANY>), dim3(blocks), dim3(WAVES * 64), 0,
                        stream, GemvCall<false>::of(g, m, rq));
     MI_HIP_CHECK(hipGetLastError());
     return (int)MI_OK;
@@ -916,11 +959,11 @@ int launch_block_weights(const int8_t *w, int n_pad, int k_pad, int ldw, int8_t 
   return MI_OK;
 }
 
-template <int WAVES, int RG, int D>
+template <int WAVES, int RG, int D, bool ANY>
 static int launch_mfma_lds_deq(const GemvArgs &g, int m, const DequantParams &dq, hipStream_t stream) {
   const int blocks = (g.n + RG * 16 - 1) / (RG * 16);
   return with_row_class<WAVES, D>(m, [&](auto mr) {
-    hipLaunchKernelGGL((gemv_mfma_lds_deq_kernel<WAVES, RG, D, decltype(mr)::value>), dim3(blocks), dim3(WAVES * 64),
+    hipLaunchKernelGGL((gemv_mfma_lds_deq_kernel<WAVES, RG, D, decltype(mr)::value, ANY>), dim3(blocks), dim3(WAVES * 64),
                        0, stream, GemvCall<true>::of(g, m, dq));
     MI_HIP_CHECK(hipGetLastError());
     return (int)MI_OK;
@@ -933,14 +976,34 @@ static bool prefers_mfma(int m, const WeightView &wv) {
   return m > kGemvDotRows || (m == 2 && wv.blocked != nullptr);
 }
 
+static bool whole_rows(const int8_t *a, int64_t lda, int k) {
+  return (k & 15) == 0 && (lda & 15) == 0 && (reinterpret_cast<uintptr_t>(a) & 15) == 0;
+}
+
+// f(ANY): the kernels for whole chunks or for rows of any length at any address.
+template <typename F>
+static int with_rows(const int8_t *a, int64_t lda, int k, F &&f) {
+  return whole_rows(a, lda, k) ? f(std::false_type()) : f(std::true_type());
+}
+
+// A copy of the rows in whole chunks is a launch of its own, 2.4 us on the host and 1.4 - 1.9 us of the kernels' 2.5 - 6.  Without
+// it every workgroup moves its rows' unaligned chunks into place, which costs more where there are more rows, where K is long,
+// and where there are more workgroups than CUs.  us, copy / none (K x channels): 1 row 1001 x 1001 6.7 / 4.0, 11009 x 10000
+// 19.9 / 18.6; 4 rows 1000 x 4096 6.4 / 3.9, 8003 x 10000 16.7 / 15.0; 16 rows 1000 x 1001 6.8 / 4.2, 8003 x 4096 10.3 / 9.7,
+// 3003 x 6001 (14 rows) 1 % less, 5003 x 6001 6 % more, 8003 x 10000 20.0 / 23.6; 32 rows 4001 x 4096 8.9 / 7.8, 6001 x 1001 4 %
+// more, 11009 x 10000 38.5 / 43.8; 64 rows 2001 x 4096 7.9 / 7.1, 4001 x 4096 12.9 / 12.2, 8003 x 1001 18.2 / 19.7.
+bool gemv_takes_any_rows(int m, int k, const WeightView &w, int n) {
+  return k >= 16 && (m == 1 || w.blocked != nullptr) && (m <= 8 || k <= 4096 || (m <= 16 && n <= kGemvNarrowChannels));
+}
+
 static int check_gemv_operands(const int8_t *a, int64_t lda, int m, int k, const WeightView &wv, int n, const int8_t *c, int64_t ldc) {
   if (a == nullptr || wv.w == nullptr || c == nullptr) {
     set_error("gemv: null pointer");
     return MI_NULL_PTR;
   }
-  if (m < 1 || ldc != n || !gemv_takes_rows(m, n) || n <= 0 || k <= 0 || (k & 15) != 0 || (lda & 15) != 0 || lda < k ||
+  if (m < 1 || ldc != n || !gemv_takes_rows(m, n) || n <= 0 || k <= 0 || lda < k ||
+      (!whole_rows(a, lda, k) && (lda != k || !gemv_takes_any_rows(m, k, wv, n))) ||
       wv.k_pad != round_up(k, kKPad) || wv.ldw != weight_row_stride(wv.k_pad) ||
-      (reinterpret_cast<uintptr_t>(a) & 15) != 0 ||
       (int64_t)(m - 1) * lda + k >= (int64_t)1 << 30 || wv.k_pad > 1 << 20 ||  // (32-bit buffer offsets)
       (m <= kGemvDotRows && (int64_t)m * round_up(k, 1024) > 160 * 1024 - 1024)) {
     set_error("gemv: unsupported operand geometry m=%d n=%d k=%d lda=%lld", m, n, k, (long long)lda);
@@ -955,7 +1018,7 @@ static int check_gemv_operands(const int8_t *a, int64_t lda, int m, int k, const
 
 int launch_gemv_group(const int8_t *a, int64_t lda, int m, int k, int count, const WeightView *wv, const int *n,
                       const RequantParams *rq, int8_t *const *c, hipStream_t stream) {
-  if (count < 1 || count > kGemvGroupMax || lda != k) {
+  if (count < 1 || count > kGemvGroupMax || lda != k || !whole_rows(a, lda, k)) {
     set_error("gemv group: %d members (1..%d), rows of %d bytes %lld apart", count, kGemvGroupMax, k, (long long)lda);
     return MI_PARAM_INVALID;
   }
@@ -992,17 +1055,19 @@ int launch_gemv_requant(const int8_t *a, int64_t lda, int m, int k, const Weight
   const int k_pad = wv.k_pad;
   const int rc = check_gemv_operands(a, lda, m, k, wv, n, c, ldc);
   if (rc != MI_OK) return rc;
-  GemvArgs g{a, lda, k / 16, w, wv.ldw, k_pad, n, c, ldc};
-  if (prefers_mfma(m, wv)) {
+  GemvArgs g{a, lda, (k + 15) / 16, w, wv.ldw, k_pad, n, c, ldc};
+  if (m == 2 && !prefers_mfma(m, wv)) return launch_m<2, false>(g, rq, stream);
+  return with_rows(a, lda, k, [&](auto any) {
+    constexpr bool ANY = decltype(any)::value;
+    if (m == 1) return launch_m<1, ANY>(g, rq, stream);
     g.w = wv.blocked;
     // three 16-channel groups per workgroup (a third of the activation traffic) once there are enough channels to
     // fill the device with 8-wave workgroups and the rows are short enough for a wave's share to be in flight at once
-    if (m > 32) return launch_mfma_lds_64(g, m, rq, stream);
-    if (m > 16 && !(n >= 8192 && k_pad <= 4096)) return launch_mfma_lds<8, 1, 4>(g, m, rq, stream);
-    if (n >= 8192 && k_pad <= 4096) return launch_mfma_lds<8, 3, 4>(g, m, rq, stream);
-    return launch_mfma_lds<8, 1, 8>(g, m, rq, stream);
-  }
-  return m == 1 ? launch_m<1>(g, rq, stream) : launch_m<2>(g, rq, stream);
+    if (m > 32) return launch_mfma_lds_64<ANY>(g, m, rq, stream);
+    if (m > 16 && !(n >= 8192 && k_pad <= 4096)) return launch_mfma_lds<8, 1, 4, ANY>(g, m, rq, stream);
+    if (n >= 8192 && k_pad <= 4096) return launch_mfma_lds<8, 3, 4, ANY>(g, m, rq, stream);
+    return launch_mfma_lds<8, 1, 8, ANY>(g, m, rq, stream);
+  });
 }
 
 // The dynamic-quant MatMul at 1..64 rows: the matrix-core decode kernel on the blocked weight copy with the fp32
@@ -1011,29 +1076,32 @@ int launch_gemv_dequant(const int8_t *a, int64_t lda, int m, int k, const Weight
                         const DequantParams &dq, float *c, int64_t ldc, hipStream_t stream) {
   const int rc = check_gemv_operands(a, lda, m, k, wv, n, reinterpret_cast<const int8_t *>(c), ldc);
   if (rc != MI_OK) return rc;
-  if (m == 1) {  // one row: the v_dot4 kernel on the row-major weights, as for the requantising MatMul
-    const GemvArgs g1{a, lda, k / 16, wv.w, wv.ldw, wv.k_pad, n, reinterpret_cast<int8_t *>(c), ldc};
-    return with_config<1>((g1.kchunks + 63) >> 6, [&](auto r, auto d, auto direct, auto ks) {
-      return launch_mrdx_deq<1, decltype(r)::value, decltype(d)::value, decltype(direct)::value, decltype(ks)::value>(
-          g1, dq, stream);
-    });
-  }
-  if (wv.blocked == nullptr) {
+  if (m > 1 && wv.blocked == nullptr) {
     set_error("gemv: the blocked weight copy is missing");
     return MI_NULL_PTR;
   }
-  GemvArgs g{a, lda, k / 16, wv.blocked, wv.ldw, wv.k_pad, n, reinterpret_cast<int8_t *>(c), ldc};
+  // (one row: the v_dot4 kernel on the row-major weights, as for the requantising MatMul)
+  const GemvArgs g{a, lda, (k + 15) / 16, m == 1 ? wv.w : wv.blocked, wv.ldw, wv.k_pad, n, reinterpret_cast<int8_t *>(c), ldc};
   const bool wide = n >= 8192 && wv.k_pad <= 4096;
-  if (m > 32) return launch_mfma_lds_deq_64(g, m, dq, stream);
-  if (wide) return launch_mfma_lds_deq<8, 3, 4>(g, m, dq, stream);
-  return m > 16 ? launch_mfma_lds_deq<8, 1, 4>(g, m, dq, stream) : launch_mfma_lds_deq<8, 1, 8>(g, m, dq, stream);
+  return with_rows(a, lda, k, [&](auto any) {
+    constexpr bool ANY = decltype(any)::value;
+    if (m == 1) {
+      return with_config<1>((g.kchunks + 63) >> 6, [&](auto r, auto d, auto direct, auto ks) {
+        return launch_mrdx_deq<1, decltype(r)::value, decltype(d)::value, decltype(direct)::value, decltype(ks)::value, ANY>(
+            g, dq, stream);
+      });
+    }
+    if (m > 32) return launch_mfma_lds_deq_64<ANY>(g, m, dq, stream);
+    if (wide) return launch_mfma_lds_deq<8, 3, 4, ANY>(g, m, dq, stream);
+    return m > 16 ? launch_mfma_lds_deq<8, 1, 4, ANY>(g, m, dq, stream) : launch_mfma_lds_deq<8, 1, 8, ANY>(g, m, dq, stream);
+  });
 }
 
 // The dynamic-quant MatMuls that share their input, as one launch (mi_dynmm_run_group): one row on the dot kernel,
 // 2..32 rows on the matrix-core kernel (every member then needs its blocked weight copy).
 int launch_gemv_group_dequant(const int8_t *a, int64_t lda, int m, int k, int count, const WeightView *wv, const int *n,
                               const DequantParams *dq, float *const *c, hipStream_t stream) {
-  if (count < 1 || count > kGemvGroupMax || lda != k) {
+  if (count < 1 || count > kGemvGroupMax || lda != k || !whole_rows(a, lda, k)) {
     set_error("gemv group: %d members (1..%d), rows of %d bytes %lld apart", count, kGemvGroupMax, k, (long long)lda);
     return MI_PARAM_INVALID;
   }

@@ -809,3 +809,28 @@ def test_matmul_row_sums(orc, m, n, k, dynamic):
         want = orc.matmul_int8(a, w, bias, 0.02, 7, sw, zw, float(np.float32(0.02 * 0.0055 * k ** 0.5 * 140)), 3)
     args = dict(in_quant=K.QuantParam(0.03, -5)) if dynamic else {}
     assert np.array_equal(make(True).run(torch.from_numpy(a).cuda(), **args).cpu().numpy(), want)
+
+
+# few rows that are no whole 16-byte chunks, or start anywhere: shorter than a chunk and just longer, ends at each part of a chunk, of a
+# 64-byte step, of a wave's slice of K and of the row lengths at which the kernels change; 8200 channels for the wide form
+@pytest.mark.parametrize("k,n", [(9, 40), (17, 40), (31, 300), (63, 40), (127, 40), (250, 1001), (1001, 96), (1023, 40), (2049, 40), (4095, 33),
+                                 (6151, 40), (7005, 40), (12281, 33), (13007, 33), (770, 8200), (64, 40), (1024, 40)])
+@pytest.mark.parametrize("dynamic,asymmetric", [(False, False), (False, True), (True, False), (True, True)])
+def test_matmul_few_rows_of_any_length(orc, k, n, dynamic, asymmetric):
+    import torch
+    rng = np.random.default_rng(n + k)
+    w, bias, sw, zw, make = _matmul_pair(rng, n, k, asymmetric, dynamic)
+    kern = make(True)
+    args = dict(in_quant=K.QuantParam(0.03, -5)) if dynamic else {}
+    orc.set_threads(16)
+    for m in (1, 2, 3, 5, 8, 13, 16, 17, 32, 33, 64):
+        a = rng.integers(-128, 128, (m, k), dtype=np.int8)
+        if dynamic:
+            want = orc.dynamic_matmul(a, w, bias, 0.03, -5, sw, zw)
+        else:
+            want = orc.matmul_int8(a, w, bias, 0.02, 7, sw, zw, float(np.float32(0.02 * 0.0055 * k ** 0.5 * 140)), 3)
+        for start in (0, 1, 6, 15):
+            held = torch.full((start + m * k,), 77, dtype=torch.int8, device="cuda")
+            held[start:] = torch.from_numpy(a).cuda().reshape(-1)
+            got = kern.run(held[start:].view(m, k), **args).cpu().numpy()
+            assert np.array_equal(got, want), (m, start)
