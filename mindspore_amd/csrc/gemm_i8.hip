@@ -612,10 +612,11 @@ int launch_gemm_dequant(const int8_t *a, int64_t lda, int m, int k, const Weight
 // are the quickest they take the rows as they are, up to the K at which their unaligned loads, once per column tile, have
 // cost as much.  us, copy and tiles / this: 333 x 1001 x 1000 7.4 / 5.6, 100 x 500 x 500 7.2 / 4.4, 128 x 768 x 770 7.5 / 5.7,
 // 1000 x 1000 x 1001 8.0 / 6.8, 200 x 1000 x 1500 7.9 / 6.7, 200 x 1000 x 1793 8.5 / 9.2, x 2040 8.4 / 7.8, x 4003 12.5 / 16.5,
-// 500 x 2000 x 3001 12.3 / 14.2.
-constexpr int kAnyrowMostK = 1536;
+// 500 x 2000 x 3001 12.3 / 14.2; less than a block of 128: 65 x 120 x 64 6.4 / 3.9, 1000 x 65 x 1001 6.6 / 4.3, 200 x 17 x 4096
+// 6.3 / 4.1, 8000 x 100 x 64 7.0 / 4.2.
+constexpr int kAnyrowLeastK = 16, kAnyrowMostK = 1536;
 bool gemm_anyrow_takes(int m, int k, const WeightView &w, int n) {
-  if (w.blocked == nullptr || k < 128 || k > kAnyrowMostK || (int64_t)m * k < 16) return false;
+  if (w.blocked == nullptr || k < kAnyrowLeastK || k > kAnyrowMostK) return false;
   float cost;
   const TileCost &t = cheapest_tile(m, k, 1, &n, &cost);
   return t.ring && t.tn == 1 && t.tm == 1;

@@ -834,3 +834,25 @@ def test_matmul_few_rows_of_any_length(orc, k, n, dynamic, asymmetric):
             held[start:] = torch.from_numpy(a).cuda().reshape(-1)
             got = kern.run(held[start:].view(m, k), **args).cpu().numpy()
             assert np.array_equal(got, want), (m, start)
+
+
+# rows of less than one block of K, at any address, where the next chunk of a row lies in the rows behind it or behind the last one
+@pytest.mark.parametrize("k", [16, 17, 33, 47, 65, 100, 127])
+@pytest.mark.parametrize("m,n", [(65, 40), (130, 65), (1000, 300)])
+@pytest.mark.parametrize("dynamic,asymmetric", [(False, False), (False, True), (True, True)])
+def test_matmul_short_rows_of_any_length(orc, m, n, k, dynamic, asymmetric):
+    import torch
+    rng = np.random.default_rng(m + n + k)
+    w, bias, sw, zw, make = _matmul_pair(rng, n, k, asymmetric, dynamic)
+    a = rng.integers(-128, 128, (m, k), dtype=np.int8)
+    orc.set_threads(16)
+    if dynamic:
+        want = orc.dynamic_matmul(a, w, bias, 0.03, -5, sw, zw)
+    else:
+        want = orc.matmul_int8(a, w, bias, 0.02, 7, sw, zw, float(np.float32(0.02 * 0.0055 * k ** 0.5 * 140)), 3)
+    kern = make(True)
+    args = dict(in_quant=K.QuantParam(0.03, -5)) if dynamic else {}
+    for start in (0, 1, 15):
+        held = torch.full((start + m * k,), 77, dtype=torch.int8, device="cuda")
+        held[start:] = torch.from_numpy(a).cuda().reshape(-1)
+        assert np.array_equal(kern.run(held[start:].view(m, k), **args).cpu().numpy(), want), start
