@@ -21,9 +21,12 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 constexpr int kDqThreads = 256;
 constexpr int kDqElemsPerThread = 16;
 
+// NaN is no minimum or maximum: made quiet, since the hardware's minimum of a signalling NaN and a number is NaN.  (v_max, and half
+// of a v_min3 and a v_max3: two instructions a value, where comparisons and selections take four and their wait states.)
 __device__ __forceinline__ void upd(float v, float &lo, float &hi) {
-  lo = v < lo ? v : lo;
-  hi = v > hi ? v : hi;
+  v = __builtin_canonicalizef(v);
+  lo = __builtin_fminf(lo, v);
+  hi = __builtin_fmaxf(hi, v);
 }
 
 // Minimum and maximum over the 64 lanes of a wave, in every lane: DPP steps inside each row of 16 lanes (quad_perm
@@ -123,28 +126,43 @@ __device__ __forceinline__ int8_t quant_one(float v, float inv, float zpf) {
   return (int8_t)q;
 }
 
-// Four values -> four bytes.  quant_one in about half the instructions where |t| < 2^20 for all four: adding the
-// largest float below one half, with t's sign, and truncating rounds half away from zero exactly (a sum that should
-// stay below the next integer stays there, t = k + 0.5 ties up to it), and the clamp is one v_med3.  Infinities, NaN
-// and values a broken scale throws out of range have |t| >= 2^20 or t != t and take quant_one.
-__device__ __forceinline__ int quant_four(v4f v, float inv, float zpf) {
-  int q[4];
-  bool rare = false;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const float t = __fadd_rn(__fmul_rn(v[e], inv), zpf);
-    rare |= !(__builtin_fabsf(t) < 1048576.0f);
-    const int r = (int)__fadd_rn(t, __builtin_copysignf(0x1.fffffep-2f, t));
-    const int lo = r > -128 ? r : -128;
-    q[e] = lo < 127 ? lo : 127;
-  }
-  if (rare) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) q[e] = quant_one(v[e], inv, zpf);
-  }
+__device__ __forceinline__ int four_bytes(const int (&q)[4]) {
   const uint32_t p01 = __builtin_amdgcn_perm((uint32_t)q[1], (uint32_t)q[0], 0x0c0c0400u);
   const uint32_t p23 = __builtin_amdgcn_perm((uint32_t)q[3], (uint32_t)q[2], 0x0c0c0400u);
   return (int)__builtin_amdgcn_perm(p23, p01, 0x05040100u);
+}
+
+// Whether |t| < 2^20 for all values, given the least and the greatest of them: t does not fall as the value rises, and NaN is neither
+// (infinities, and values that a broken scale throws out of range, are not).
+__device__ __forceinline__ bool quantises_plainly(float lo, float hi, float inv, float zpf) {
+  const float a = __fadd_rn(__fmul_rn(lo, inv), zpf), b = __fadd_rn(__fmul_rn(hi, inv), zpf);
+  return __builtin_fabsf(a) < 1048576.0f && __builtin_fabsf(b) < 1048576.0f;
+}
+
+// Four such values -> four bytes, quant_one in a third of the instructions: adding the largest float below one half, with t's
+// sign, and truncating rounds half away from zero exactly (a sum that should stay below the next integer stays there,
+// t = k + 0.5 ties up to it).  The maximum of NaN and a number is the number, -128 as quant_one has it.
+// Whether that may be is one question for the whole tensor (or run), and what it is otherwise one loop: asked for every four values,
+// with the other answer beside each, a thread's values were 175 instructions a group to jump through, cold in the instruction
+// cache at every launch, of which 42 are left.  us per launch from a graph, with that and comparisons for the minimum and maximum
+// (see upd) / without the first / without both: 4096 x 768 6.75 / 6.6 / 6.35, 4096 x 3072 16.55 / 16.05 / 15.8, 600 x 4096 6.6 / 6.4 /
+// 6.1, 2000 x 4096 11.3 / 10.85 / 10.7, 6000 x 5632 55.3 / 55.4 / 50.7; a scale per row, 2048 x 4096 8.37 / 8.28 / 8.24.
+__device__ __forceinline__ int quant_four_plain(v4f v, float inv, float zpf) {
+  int q[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float t = __fadd_rn(__fmul_rn(v[e], inv), zpf);
+    const float r = __fadd_rn(t, __builtin_copysignf(0x1.fffffep-2f, t));
+    q[e] = (int)__builtin_fminf(__builtin_fmaxf(r, -128.0f), 127.0f);
+  }
+  return four_bytes(q);
+}
+
+__device__ __forceinline__ int quant_four(v4f v, float inv, float zpf) {
+  int q[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) q[e] = quant_one(v[e], inv, zpf);
+  return four_bytes(q);
 }
 
 // scale and zero point from the tensor's min and max (CalculatePerlayerScaleZp, dynamic_quant.cc:156-186)
@@ -341,10 +359,16 @@ __global__ __launch_bounds__(T) void dq_fused_kernel(const float *__restrict__ x
   }
   const float inv = __fdiv_rn(1.0f, scale_f);
   const float zpf = (float)zp;
+  if (quantises_plainly(lo, hi, inv, zpf)) {
 #pragma unroll
-  for (int j = 0; j < G; ++j) {
-    const int64_t i = first + j * T;
-    if (i < n4) *reinterpret_cast<int_any *>(q + 4 * i) = quant_four(v[j], inv, zpf);
+    for (int j = 0; j < G; ++j) {
+      const int64_t i = first + j * T;
+      if (i < n4) *reinterpret_cast<int_any *>(q + 4 * i) = quant_four_plain(v[j], inv, zpf);
+    }
+  } else {  // (from memory again: with the registers, whose numbers are constants, there would be G copies of it)
+#pragma unroll 1
+    for (int64_t i = first; i < n4 && i < first + (int64_t)G * T; i += T)
+      *reinterpret_cast<int_any *>(q + 4 * i) = quant_four(x4[i], inv, zpf);
   }
   if (has_tail) q[ti] = quant_one(tail, inv, zpf);
 }
@@ -389,11 +413,11 @@ __global__ __launch_bounds__(kDqThreads) void dq_quantize_kernel(const float *__
   const float zpf = (float)zp;
 
   if (base >= n) return;
-  if (fast) {
+  if (fast && quantises_plainly(lo, hi, inv, zpf)) {
     typedef int v4i __attribute__((ext_vector_type(4)));
     v4i o;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) o[j] = quant_four(xv[j], inv, zpf);
+    for (int j = 0; j < 4; ++j) o[j] = quant_four_plain(xv[j], inv, zpf);
     *reinterpret_cast<v4i *>(q + base) = o;
   } else {
     const int64_t end = base + kDqElemsPerThread < n ? base + kDqElemsPerThread : n;
@@ -448,10 +472,15 @@ __global__ __launch_bounds__(T == 64 ? 256 : T) void dq_rows_kernel(const float 
   if (tid == 0) publish_params(params + seg, scale_f, zp, lo, hi);
   const float inv = __fdiv_rn(1.0f, scale_f);
   const float zpf = (float)zp;
+  if (quantises_plainly(lo, hi, inv, zpf)) {
 #pragma unroll
-  for (int j = 0; j < G; ++j) {
-    const int i = tid + j * T;
-    if (i < n4) *reinterpret_cast<int_any *>(qs + 4 * i) = quant_four(v[j], inv, zpf);
+    for (int j = 0; j < G; ++j) {
+      const int i = tid + j * T;
+      if (i < n4) *reinterpret_cast<int_any *>(qs + 4 * i) = quant_four_plain(v[j], inv, zpf);
+    }
+  } else {
+#pragma unroll 1
+    for (int i = tid; i < n4; i += T) *reinterpret_cast<int_any *>(qs + 4 * i) = quant_four(x4[i], inv, zpf);
   }
   if (ti < unit) qs[ti] = quant_one(tail, inv, zpf);
 }
@@ -485,7 +514,9 @@ __global__ __launch_bounds__(1024) void dq_long_rows_kernel(const float *__restr
   if (tid == 0) publish_params(params + blockIdx.x, scale_f, zp, lo, hi);
   const float inv = __fdiv_rn(1.0f, scale_f);
   const float zpf = (float)zp;
-  for (int64_t k = tid; k < n4; k += 1024) *reinterpret_cast<int_any *>(qs + 4 * k) = quant_four(x4[k], inv, zpf);
+  const bool plain = quantises_plainly(lo, hi, inv, zpf);
+  for (int64_t k = tid; k < n4; k += 1024)
+    *reinterpret_cast<int_any *>(qs + 4 * k) = plain ? quant_four_plain(x4[k], inv, zpf) : quant_four(x4[k], inv, zpf);
   if (ti < unit) qs[ti] = quant_one(xs[ti], inv, zpf);
 }
 
@@ -506,8 +537,8 @@ int launch_dynquant_segments(const float *x, int64_t segments, int64_t unit, int
   // A wave per run where there are enough short runs to fill the device with waves; otherwise more threads per run, for
   // few runs to shorten each thread's chain and for long ones to have 2 to 6 loads of 16 bytes per thread.  us per
   // launch, before (one wave per run, two sweeps) -> now: 8 x 4096 11.6 -> 2.9, 8 x 11008 28.0 -> 3.6,
-  // 512 x 4096 14.8 -> 4.7, 4096 x 768 6.7 -> 5.2, 2048 x 4096 21.8 -> 9.1 (4.6 TB/s), 2048 x 11008 60.4 -> 20.4
-  // (5.5 TB/s; a copy reaches 5.0).  2048 x 4096 takes 10.8 with a wave and 10.1 with 512 threads per run, 197 x 768
+  // 512 x 4096 14.8 -> 4.7, 4096 x 768 6.7 -> 5.2, 2048 x 4096 21.8 -> 8.2 (5.1 TB/s), 2048 x 11008 60.4 -> 19.9
+  // (5.7 TB/s; a copy reaches 4.9).  2048 x 4096 takes 10.8 with a wave and 10.1 with 512 threads per run, 197 x 768
   // 3.0 with a wave and 2.7 with 256 threads, 4096 x 768 6.6 with 256 threads.
   const int64_t n4 = unit >> 2;
 #define MI_DQ_ROWS(T, G) launch_rows<T, G>(x, segments, (int)unit, symmetric, params, q, stream)
@@ -552,7 +583,8 @@ int launch_dynquant(const float *x, int64_t n, int symmetric, float2 *partials, 
   // values per thread that allows: what counts at these sizes is the latency of each thread's chain.  us per tensor,
   // before (up to 24576 values one workgroup, else two launches) -> now: 4096 3.9 -> 2.9, 16384 5.9 -> 3.7,
   // 32768 7.2 -> 4.2, 88064 7.4 -> 4.4, 300000 7.7 -> 5.0, 1 M 8.0 -> 5.6, 4096 x 768 11.3 -> 8.9,
-  // 2048 x 4096 20.0 -> 13.5, 4096 x 3072 26.9 -> 17.5, 2048 x 11008 40.8 -> 26.7.
+  // 2048 x 4096 20.0 -> 13.5, 4096 x 3072 26.9 -> 17.5, 2048 x 11008 40.8 -> 26.7.  (Since then the exchange and the quantising have
+  // become quicker, see above: 32768 3.9, 88064 4.0, 4096 x 768 6.35, 4096 x 3072 15.8.)
   const int64_t n4 = n >> 2;
 #define MI_DQ_FUSED(T, G)                                                        \
   do {                                                                           \

@@ -856,3 +856,29 @@ def test_matmul_short_rows_of_any_length(orc, m, n, k, dynamic, asymmetric):
         held = torch.full((start + m * k,), 77, dtype=torch.int8, device="cuda")
         held[start:] = torch.from_numpy(a).cuda().reshape(-1)
         assert np.array_equal(kern.run(held[start:].view(m, k), **args).cpu().numpy(), want), start
+
+
+# values that leave the range the quick rounding holds for, or are no numbers (0x7fa00000: a signalling NaN), in tensors and rows of every
+# kernel form; most of a tensor stays ordinary, and the parameters are the oracle's
+@pytest.mark.parametrize("bits", [0x7fc00000, 0xffc00001, 0x7fa00000, 0xffa00000, 0x7f800000, 0xff800000, 0x7f7fffff, 0x00000001, 0x80000000])
+@pytest.mark.parametrize("symmetric", [False, True])
+def test_dynamic_quant_values_out_of_line(orc, bits, symmetric):
+    import torch
+    special = np.array([bits], np.uint32).view(np.float32)[0]
+    dq = K.DynamicQuantKernel(symmetric)
+    for n in (3, 700, 4099, 8195, 40003, 300002, 1500001, 6300003, 27000003):
+        for scale in (1.0, 1e-30):
+            x = _values(np.random.default_rng(n), n) * np.float32(scale)
+            x.view(np.uint32)[[0, n // 2, n - 1]] = bits
+            q, p = dq.run(torch.from_numpy(x).cuda())
+            want, s, zp = orc.dynamic_quant(x, symmetric)
+            assert np.array_equal(q.cpu().numpy(), want), (n, scale, special)
+            assert np.array_equal([p.scale], [s], equal_nan=True) and p.zero_point == zp
+    for rows, unit in ((3, 255), (600, 515), (513, 771), (256, 1028), (257, 3075), (5, 8196), (2, 16388), (2, 65540)):
+        x = _values(np.random.default_rng(rows * unit), rows * unit).reshape(rows, unit)
+        x.view(np.uint32)[rows // 2, [0, unit // 2, unit - 1]] = bits
+        q, params = dq.run_rows(torch.from_numpy(x).cuda())
+        want, scales, zps = orc.dynamic_quant_segments(x, symmetric)
+        got = params.cpu().numpy().view([("scale", "f8"), ("scale_f", "f4"), ("zp", "i4"), ("lo", "f4"), ("hi", "f4")])
+        assert np.array_equal(q.cpu().numpy(), want), (rows, unit, special)
+        assert np.array_equal(got["scale"].reshape(-1), scales.reshape(-1), equal_nan=True) and np.array_equal(got["zp"].reshape(-1), zps.reshape(-1))
