@@ -17,7 +17,7 @@ typedef v4i v4i_byte __attribute__((aligned(1)));
 // LDS holds two sets of four blocks of both operands: one is computed on while the other arrives.  Four blocks, 64 KiB, are about
 // what a CU can have on its way.
 // Bound by launch and latency; per 512 bytes of K about 1 us, the time of 64 KiB per CU.  333 x 1001 x 1000 with weight zero
-// points 8.3 us (copy and ring) -> 5.6; more figures and where it ends are at gemm_anyrow_takes.
+// points 8.3 us (copy and ring) -> 5.35; more figures and where it ends are at gemm_anyrow_takes.
 // =====================================================================================================================
 template <int EPI, bool HAS_ZW, bool FAST>
 __device__ __forceinline__ void gemm_anyrow_body(const GemmArgs &g, const RequantParams &rq, const DequantParams &dq) {

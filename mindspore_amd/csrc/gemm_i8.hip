@@ -9,15 +9,16 @@
 // waves (2 x 2) owns a TILE_M x TILE_N output tile; the weight tile is the MFMA "A" operand (its rows are output
 // channels) and the activation tile the "B" operand, so a lane ends up holding 4 consecutive output channels of
 // one output row: the epilogue packs them into one 32-bit store, per-channel parameters are 16-byte loads, and
-// the input-row sum a lane needs is the one it accumulated itself (v_dot4 against 0x01010101).
+// the input-row sum a lane needs is the one it accumulated itself (v_dot4 against 0x01010101, or see RowSums).
 //
-// Four main loops, most of them moving tiles global -> LDS with asynchronous 16-byte-per-lane loads and reading operand
+// Several main loops, most of them moving tiles global -> LDS with asynchronous 16-byte-per-lane loads and reading operand
 // fragments for the next K sub-step from LDS while the MFMAs of the current one run.  Handles hold their weights in
 // 1 KiB matrix-core blocks beside the row-major form, and with those nearly every shape runs on K blocks of 128 bytes, on
 // the tile that launch_pick_tile expects to be the quickest:
 //   * gemm_kblock.hip: five LDS slots, one barrier per block; 256 x 256 and 192 x 256 tiles, one workgroup per CU, for the
 //     large shapes, 128 x 128 tiles, two per CU, where fp32 stores have to overlap another tile's loop;
 //   * gemm_ring.hip: a ring of stages that hold both operands, as deep as the LDS allows: every smaller tile;
+//   * gemm_split.hip: the same with the K of a tile in parts, a workgroup each, where the tiles leave CUs idle;
 //   * gemm_anyrow.hip: 64 x 64 tiles for activation rows that are no whole 16-byte chunks, where padding them first would cost
 //     more than the product;
 //   * gemm_direct_body below, K steps of 64 bytes through NST LDS stages over row-major weights: short K, handles
