@@ -448,6 +448,10 @@ constexpr int rows_occupancy(int ks, int ocb, RequantForm form) { return form !=
 template <int KS, int OCB, RequantForm FORM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(rows_occupancy(KS, OCB, FORM)))) void conv_rows_kernel(
     ConvRows g, RequantCall call, int8_t *__restrict__ out) {
+  call.load_now();
+  asm volatile("" ::"s"(g.in), "s"(g.w), "s"(g.in_bytes), "s"(g.in_h), "s"(g.in_w), "s"(g.out_w), "s"(g.out_hw), "s"(g.out_c), "s"(g.stride_h),
+               "s"(g.stride_w), "s"(g.dil_h), "s"(g.pads), "s"(g.sizes), "s"(g.shifts), "s"(g.pixels), "s"(g.magic_hw), "s"(g.magic_w),
+               "s"(g.step), "s"(out));
   const RequantParams rq = call.open(g.out_c);
   const int lane = threadIdx.x & 63;
   const int n0 = blockIdx.y * (32 * OCB);
@@ -595,6 +599,14 @@ struct ConvDwRows {
   int groups, strips, bands;  // channels / 4, output columns / 4, output rows / OT, rounded up
   int total;                  // batch * bands * strips * groups
   int zsplat, amin, amax;
+  uint32_t magic_groups, magic_strips, magic_bands, shifts;  // quotients by those (see magic31), shifts a byte each
+  void set_quotients() {
+    int s[3];
+    magic31(groups, &magic_groups, s);
+    magic31(strips, &magic_strips, s + 1);
+    magic31(bands, &magic_bands, s + 2);
+    shifts = (uint32_t)(s[0] | s[1] << 8 | s[2] << 16);
+  }
 };
 static_assert(sizeof(ConvDwRows) <= kShortArgs, "see launch_args.h");
 
@@ -607,21 +619,24 @@ constexpr int kDwStreamedLeast = 128;
 
 // RELU: no output is below the zero point.  The rounding's sign term is then a constant (as in kReluForm of conv_store.h).  us:
 // 16 x 112 x 112 on 128 channels 15.9 -> 15.1, 32 x 56 x 56 on 144 11.4 -> 10.5, 8 x 80 x 80 on 72, 5x5 6.95 -> 6.75.
+// A launch lasts a few times its way to the first input: 165 instructions with three divisions and two scalar round trips, now 110 and one.
+// us: 1 x 112 x 112 x 192 3.92 -> 3.71, 8 x 128 x 128 x 96 9.72 -> 9.53, 16 x 112 x 112 x 192 19.75 -> 19.15, 2 x 66 x 66 x 128 3.32 -> 3.16.
 template <int KS, int OT, bool RELU, bool STREAMED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void conv_dw_rows_kernel(ConvDwRows g) {
   constexpr int PX = KS + 3;       // input pixels per row of four outputs
   constexpr int WR = KS == 3 ? 1 : 3;  // weight dwords per channel and window row
+  asm volatile("" ::"s"(g.in), "s"(g.w), "s"(g.par), "s"(g.out), "s"(g.in_h), "s"(g.in_w), "s"(g.ch), "s"(g.out_h), "s"(g.out_w), "s"(g.pad_u),
+               "s"(g.pad_l), "s"(g.groups), "s"(g.strips), "s"(g.bands), "s"(g.total), "s"(g.zsplat), "s"(g.amin), "s"(g.amax),
+               "s"(g.magic_groups), "s"(g.magic_strips), "s"(g.magic_bands), "s"(g.shifts));
   // as below: workgroups that share an XCD get one contiguous band of the output
   int bid = blockIdx.x;
   const int per = ((g.total + 255) >> 8) >> 3;  // an eighth of the grid
   if (bid < per * 8) bid = (bid & 7) * per + (bid >> 3);
   const int idx = bid * 256 + threadIdx.x;
   if (idx >= g.total) return;
-  uint32_t rest = (uint32_t)idx / (uint32_t)g.groups;
-  const int c0 = (idx - (int)rest * g.groups) * 4;
-  uint32_t up = rest / (uint32_t)g.strips;
-  const int ow0 = (int)(rest - up * g.strips) * 4;
-  const int b = (int)(up / (uint32_t)g.bands), oh0 = (int)(up - b * g.bands) * OT;
+  const int rest = quotient31(idx, g.magic_groups, g.shifts & 0xff), c0 = (idx - rest * g.groups) * 4;
+  const int up = quotient31(rest, g.magic_strips, g.shifts >> 8 & 0xff), ow0 = (rest - up * g.strips) * 4;
+  const int b = quotient31(up, g.magic_bands, g.shifts >> 16), oh0 = (up - b * g.bands) * OT;
   const int ih0 = oh0 - g.pad_u, iw0 = ow0 - g.pad_l;
   const int line = g.in_w * g.ch;
 
@@ -784,6 +799,7 @@ template <int KS, int OT>
 static int launch_dw_rows(ConvDwRows c, int batch, int zo, hipStream_t stream) {
   c.bands = (c.out_h + OT - 1) / OT;
   c.total = batch * c.bands * c.strips * c.groups;
+  c.set_quotients();
   const bool streamed = c.ch >= kDwStreamedLeast &&
                         (int64_t)batch * c.out_h * c.out_w * c.ch <= (c.ch % 32 == 0 ? kStreamedMost : kStreamedMost / 2);
   const auto kernel = c.amin >= zo ? (streamed ? conv_dw_rows_kernel<KS, OT, true, true> : conv_dw_rows_kernel<KS, OT, true, false>)

@@ -38,6 +38,8 @@ static_assert(sizeof(ConvThin) + sizeof(RequantCall) + sizeof(int8_t *) <= kShor
 template <int CH, int OCB, RequantForm FORM, bool NEIGHBOURS = true>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void conv_thin_kernel(ConvThin g, RequantCall call,
                                                                                               int8_t *__restrict__ out) {
+  call.load_now();
+  asm volatile("" ::"s"(g.in), "s"(g.in_bytes), "s"(g.k), "s"(g.chunks), "s"(g.out_c), "s"(g.pixels), "s"(g.step), "s"(g.w), "s"(out));
   const RequantParams rq = call.open(g.out_c);
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5;

@@ -317,6 +317,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 // The same GEMM with the activation operand gathered from an NHWC image (no im2col buffer).
 template <int TILE_N, int TILE_M, bool HAS_ZW, bool FAST, int NST, int OCC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void gemm_conv_kernel(ConvCall call) {
+  call.epi.load_now();
+  asm volatile("" ::"s"(call.in), "s"(call.w), "s"(call.fill16), "s"(call.c), "s"(call.m), "s"(call.n), "s"(call.k), "s"(call.cv.in_h), "s"(call.cv.in_w),
+               "s"(call.cv.in_c), "s"(call.cv.out_w), "s"(call.cv.out_hw), "s"(call.cv.magic_ic), "s"(call.cv.magic_kw), "s"(call.cv.kernel_w));
   const int k_pad = padded_k(call.k);
   const GemmArgs g{call.in, 0, call.m, call.k, call.w, weight_row_stride(k_pad), k_pad, nullptr, call.n,
                    (call.m + TILE_M - 1) / TILE_M, (call.n + TILE_N - 1) / TILE_N, call.c, call.n, 0, 0};

@@ -27,6 +27,9 @@ struct RequantCall {
   static uint32_t forms_of(const RequantParams &rq) {
     return (rq.has_zw != 0 ? kHasZw : 0u) | (rq.fast != 0 ? kFast : 0u) | (rq.fast2 != 0 ? kFast2 : 0u);
   }
+  // Kernels that are short ask for all their arguments at once, with an empty asm of which they are the inputs: left to itself the compiler
+  // loads some where they are used, one way to memory behind the other.
+  __device__ __forceinline__ void load_now() const { asm volatile("" ::"s"(channels), "s"(zo), "s"(amin), "s"(amax), "s"(forms)); }
   __device__ __forceinline__ RequantParams open(int n) const {
     RequantParams rq{};
     rq.set_channels(channels, padded_channels(n));
