@@ -52,8 +52,8 @@ int mi_init(int device);
 /* Message of the last failure on the calling thread ("" if none). */
 const char *mi_last_error(void);
 /* Test aid: while `bytes` is non-zero, every device allocation the library makes for a handle (packed weights,
- * parameters, workspaces) whose size, rounded up to 4 KiB, equals `bytes` rounded up to 4 KiB fails as if the device
- * were out of memory; 0 switches it off.  Lets a test show what a handle does when one of its allocations fails. */
+ * parameters, workspaces) or a stream whose size, rounded up to 4 KiB, equals `bytes` rounded up to 4 KiB fails as if the
+ * device were out of memory; 0 switches it off.  Lets a test show what a handle does when one of its allocations fails. */
 int mi_debug_fail_alloc(size_t bytes);
 /* Test aid: how many times the library has made the host wait for a stream so far (mi_copy_to_device, mi_copy_to_host,
  * mi_stream_synchronize, mi_dynquant_get_params; the *_run_host entry points are not counted). */
@@ -393,7 +393,10 @@ int mi_stream_synchronize(void *stream);
  * provider gives every session (every mindspore::Context it is handed) a stream of its own and passes it to all run
  * and copy calls of that session, so that sessions running on different threads do not wait for one another: the
  * part of the reference this stands for is the per-kernel thread-pool context each kernel executes under
- * (mindspore/lite/src/executor/sub_graph_kernel.cc:456-466, InnerContext::thread_pool_). */
+ * (mindspore/lite/src/executor/sub_graph_kernel.cc:456-466, InnerContext::thread_pool_).
+ * MatMuls whose K is split over workgroups hand over their sums in 18 MB of device memory that a stream has from its creation
+ * to its end: mi_init allocates it for the null stream and the first seven, mi_stream_create for each further one alive at
+ * the same time.  Where there is none to be had the stream's MatMuls are not split; their results are the same. */
 int mi_stream_create(void **out_stream);
 int mi_stream_destroy(void *stream); /* NULL is allowed */
 

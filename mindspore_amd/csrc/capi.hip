@@ -17,6 +17,7 @@
 
 #include "common.h"
 #include "quant_math.h"
+#include "split_spaces.h"
 
 namespace mi {
 
@@ -38,41 +39,26 @@ static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 constexpr int kMaxDevices = 64;
 static void *g_scratch_ptr[kMaxDevices] = {};
 
-// The null stream's split_space, static as the scratch memory is; those of the library's own streams, made when first wanted.
-static __device__ __align__(256) unsigned char split_of_null_stream[kSplitBytes];
+// The null stream's split_space and those of the first few streams of the library, which mi_init allocates.  (Static, as the scratch
+// memory is, they would be filled with zeros by the host when the library is loaded: mi_init 15 -> 62 ms.)
+constexpr int kSplitSpacesKept = 8;
+static_assert(kSplitBytes % 256 == 0, "every space is aligned");
 static void *g_split_ptr[kMaxDevices] = {};
-struct SplitSpace {
-  hipStream_t stream;
-  void *p;
-  bool tried;
+struct SplitMemory {
+  typedef hipStream_t Stream;
+  static void *make(hipStream_t stream);
+  static void free(void *p);
 };
-static std::mutex g_split_mutex;
-static std::vector<SplitSpace> g_split_spaces;
-static thread_local bool t_allocates_nothing = false;  // in mi_matmul_run_noalloc
+static SplitSpaces<SplitMemory> &split_spaces() {
+  static auto *s = new SplitSpaces<SplitMemory>;  // (not destroyed with the process: others may be, and use it, later)
+  return *s;
+}
 
 void *split_space(hipStream_t stream) {
   if (stream == nullptr) return g_device >= 0 && g_device < kMaxDevices ? g_split_ptr[g_device] : nullptr;
-  std::lock_guard<std::mutex> lock(g_split_mutex);
-  for (SplitSpace &s : g_split_spaces) {
-    if (s.stream != stream) continue;
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone) return nullptr;
-    if (!s.tried && !t_allocates_nothing) {
-      s.tried = true;
-      hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // (another thread may be capturing)
-      (void)hipThreadExchangeStreamCaptureMode(&mode);
-      void *p = nullptr;
-      if (hipMalloc(&p, kSplitBytes) == hipSuccess && hipMemsetAsync(p, 0, kSplitCounterBytes, stream) == hipSuccess) {
-        s.p = p;
-      } else {
-        (void)hipGetLastError();
-        if (p != nullptr) (void)hipFree(p);
-      }
-      (void)hipThreadExchangeStreamCaptureMode(&mode);
-    }
-    return s.p;
-  }
-  return nullptr;
+  void *p = split_spaces().of(stream);
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return p != nullptr && hipStreamIsCapturing(stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone ? p : nullptr;
 }
 
 void set_error(const char *fmt, ...) {
@@ -204,6 +190,22 @@ struct DevBuf {
     bytes = 0;
   }
 };
+
+void *SplitMemory::make(hipStream_t stream) {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // (another thread may be capturing)
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  void *p = nullptr;
+  if (device_alloc(&p, (size_t)round_up64((int64_t)kSplitBytes, 4096)) != hipSuccess ||
+      hipMemsetAsync(p, 0, kSplitCounterBytes, stream) != hipSuccess) {
+    (void)hipGetLastError();
+    if (p != nullptr) (void)hipFree(p);
+    p = nullptr;
+  }
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  return p;
+}
+
+void SplitMemory::free(void *p) { (void)hipFree(p); }  // (waits for the device)
 
 // Page-locked notes of kDqHostWords words (mi_dynquant::note).  An allocation of its own takes 30 us and 200 to give
 // back, the rest of a handle 17 and 3, so handles share pages; a page goes back with the last note in it.
@@ -647,8 +649,15 @@ int mi_init(int device) {
     void *ptr = nullptr;
     MI_HIP_CHECK(hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)));  // this device's copy of the array
     g_scratch_ptr[device] = ptr;
-    MI_HIP_CHECK(hipGetSymbolAddress(&ptr, HIP_SYMBOL(split_of_null_stream)));
-    g_split_ptr[device] = ptr;
+    ptr = nullptr;
+    if (device_alloc(&ptr, kSplitSpacesKept * kSplitBytes) != hipSuccess ||
+        hipMemset2D(ptr, kSplitBytes, 0, kSplitCounterBytes, kSplitSpacesKept) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
+      (void)hipGetLastError();  // (the null stream's GEMMs are not split then)
+      if (ptr != nullptr) (void)hipFree(ptr);
+    } else {
+      g_split_ptr[device] = ptr;
+      for (int i = 1; i < kSplitSpacesKept; ++i) split_spaces().keep(device, static_cast<char *>(ptr) + i * kSplitBytes);
+    }
   }
   g_device = device;
   return MI_OK;
@@ -737,11 +746,7 @@ int mi_stream_create(void **out_stream) {
   if (ensure_device() != MI_OK) return MI_ERROR;
   hipStream_t s = nullptr;
   MI_HIP_CHECK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));  // default priority; independent of the null stream
-  try {
-    std::lock_guard<std::mutex> lock(g_split_mutex);
-    g_split_spaces.push_back(SplitSpace{s, nullptr, false});
-  } catch (...) {  // (unknown to split_space: its GEMMs are not split)
-  }
+  split_spaces().enter(s, g_device);
   *out_stream = s;
   return MI_OK;
 }
@@ -749,18 +754,15 @@ int mi_stream_create(void **out_stream) {
 int mi_stream_destroy(void *stream) {
   if (stream == nullptr) return MI_OK;
   if (ensure_device() != MI_OK) return MI_ERROR;
-  void *p = nullptr;
-  {
-    std::lock_guard<std::mutex> lock(g_split_mutex);
-    for (size_t i = 0; i < g_split_spaces.size(); ++i) {
-      if (g_split_spaces[i].stream != static_cast<hipStream_t>(stream)) continue;
-      p = g_split_spaces[i].p;
-      g_split_spaces.erase(g_split_spaces.begin() + (ptrdiff_t)i);
-      break;
-    }
-  }
-  if (p != nullptr) (void)hipFree(p);  // (waits for the device)
-  MI_HIP_CHECK(hipStreamDestroy(static_cast<hipStream_t>(stream)));
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  void *space = split_spaces().leave(s);
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  const bool settled = space != nullptr && hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone &&
+                       hipStreamSynchronize(s) == hipSuccess;
+  if (space != nullptr && !settled) (void)hipGetLastError();
+  const hipError_t e = hipStreamDestroy(s);
+  split_spaces().left(space, e == hipSuccess, settled);
+  MI_HIP_CHECK(e);
   return MI_OK;
 }
 
@@ -1025,10 +1027,7 @@ int mi_matmul_run_noalloc(mi_matmul *h, const int8_t *a_dev, int32_t rows, int8_
               "maximum is %zu; use mi_matmul_run", rows, h->st.k, h->st.n, need, kScratchBytes);
     return MI_PARAM_INVALID;
   }
-  t_allocates_nothing = true;
-  rc = run_requant_rows(h->st, a_dev, rows, Workspace::region(base, a_bytes), c_dev, static_cast<hipStream_t>(stream));
-  t_allocates_nothing = false;
-  return rc;
+  return run_requant_rows(h->st, a_dev, rows, Workspace::region(base, a_bytes), c_dev, static_cast<hipStream_t>(stream));
 }
 
 int mi_matmul_run_host(mi_matmul *h, const int8_t *a_host, int32_t rows, int8_t *c_host) {
