@@ -396,7 +396,8 @@ int mi_stream_synchronize(void *stream);
  * (mindspore/lite/src/executor/sub_graph_kernel.cc:456-466, InnerContext::thread_pool_).
  * MatMuls whose K is split over workgroups hand over their sums in 18 MB of device memory that a stream has from its creation
  * to its end: mi_init allocates it for the null stream and the first seven, mi_stream_create for each further one alive at
- * the same time.  Where there is none to be had the stream's MatMuls are not split; their results are the same. */
+ * the same time, which is freed with the last stream.  mi_stream_destroy waits for its own stream at most, but for the last
+ * one's, which may free such memory.  Where there is none to be had the stream's MatMuls are not split; their results are the same. */
 int mi_stream_create(void **out_stream);
 int mi_stream_destroy(void *stream); /* NULL is allowed */
 

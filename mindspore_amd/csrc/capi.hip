@@ -47,7 +47,7 @@ static void *g_split_ptr[kMaxDevices] = {};
 struct SplitMemory {
   typedef hipStream_t Stream;
   static void *make(hipStream_t stream);
-  static void free(void *p);
+  static bool free(void *p);
 };
 static SplitSpaces<SplitMemory> &split_spaces() {
   static auto *s = new SplitSpaces<SplitMemory>;  // (not destroyed with the process: others may be, and use it, later)
@@ -191,21 +191,36 @@ struct DevBuf {
   }
 };
 
-void *SplitMemory::make(hipStream_t stream) {
-  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // (another thread may be capturing)
+// f() where another thread may be capturing, which forbids this one what may wait for the device.
+template <typename F>
+static auto beside_captures(F &&f) {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
   (void)hipThreadExchangeStreamCaptureMode(&mode);
-  void *p = nullptr;
-  if (device_alloc(&p, (size_t)round_up64((int64_t)kSplitBytes, 4096)) != hipSuccess ||
-      hipMemsetAsync(p, 0, kSplitCounterBytes, stream) != hipSuccess) {
-    (void)hipGetLastError();
-    if (p != nullptr) (void)hipFree(p);
-    p = nullptr;
-  }
+  const auto result = f();
   (void)hipThreadExchangeStreamCaptureMode(&mode);
-  return p;
+  return result;
 }
 
-void SplitMemory::free(void *p) { (void)hipFree(p); }  // (waits for the device)
+void *SplitMemory::make(hipStream_t stream) {
+  return beside_captures([&] {
+    void *p = nullptr;
+    if (device_alloc(&p, (size_t)round_up64((int64_t)kSplitBytes, 4096)) != hipSuccess ||
+        hipMemsetAsync(p, 0, kSplitCounterBytes, stream) != hipSuccess) {
+      (void)hipGetLastError();
+      if (p != nullptr) (void)hipFree(p);
+      p = nullptr;
+    }
+    return p;
+  });
+}
+
+bool SplitMemory::free(void *p) {
+  return beside_captures([&] {
+    const bool gone = hipFree(p) == hipSuccess;
+    if (!gone) (void)hipGetLastError();
+    return gone;
+  });
+}
 
 // Page-locked notes of kDqHostWords words (mi_dynquant::note).  An allocation of its own takes 30 us and 200 to give
 // back, the rest of a handle 17 and 3, so handles share pages; a page goes back with the last note in it.
@@ -756,10 +771,13 @@ int mi_stream_destroy(void *stream) {
   if (ensure_device() != MI_OK) return MI_ERROR;
   hipStream_t s = static_cast<hipStream_t>(stream);
   void *space = split_spaces().leave(s);
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  const bool settled = space != nullptr && hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone &&
-                       hipStreamSynchronize(s) == hipSuccess;
-  if (space != nullptr && !settled) (void)hipGetLastError();
+  // (a space goes to the next stream once this one's work is done: no other's is waited for)
+  const bool settled = space != nullptr && beside_captures([&] {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone && hipStreamSynchronize(s) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+  });
   const hipError_t e = hipStreamDestroy(s);
   split_spaces().left(space, e == hipSuccess, settled);
   MI_HIP_CHECK(e);

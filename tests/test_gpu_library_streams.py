@@ -36,6 +36,11 @@ def _create(L):
     return stream
 
 
+def _destroy(L, streams):
+    for stream in streams:
+        assert L.mi_stream_destroy(stream) == lib.MI_OK
+
+
 def _run(L, kern, a, stream, rows=ROWS, run="mi_matmul_run"):
     import torch
     out = torch.full((rows, COLS), 55, dtype=torch.int8, device="cuda")
@@ -69,5 +74,91 @@ def test_runs_on_a_library_stream_allocate_nothing(matmul, memory):
         assert torch.cuda.mem_get_info()[0] == before
     finally:
         L.mi_debug_fail_alloc(0)
+    _destroy(L, streams)
+
+
+def test_the_end_of_a_stream_does_not_wait_for_others(matmul):
+    import torch
+    L, kern, a, want = matmul
+    streams = [_create(L) for _ in range(9)]
     for stream in streams:
-        assert L.mi_stream_destroy(stream) == lib.MI_OK
+        out = _run(L, kern, a, stream)
+        assert L.mi_stream_synchronize(stream) == lib.MI_OK and torch.equal(out, want)
+    busy, others = streams[0], streams[1:]
+    rng = np.random.default_rng(1)
+    n = 8192
+    big = K.MatmulInt8Kernel(rng.integers(-128, 128, (n, n), dtype=np.int8), None, K.QuantParam(0.02, 7), [K.QuantParam(0.004, 0)],
+                             K.QuantParam(1.0, 0), True, 0)
+    x = torch.zeros((n, n), dtype=torch.int8, device="cuda")
+    y = torch.empty((n, n), dtype=torch.int8, device="cuda")
+    torch.cuda.synchronize()
+    for _ in range(1000):  # about 0.3 s
+        assert L.mi_matmul_run(big._h, x.data_ptr(), n, y.data_ptr(), busy) == lib.MI_OK
+    still = torch.cuda.ExternalStream(busy.value)
+    assert not still.query()
+    _destroy(L, others)
+    assert not still.query()
+    assert L.mi_stream_synchronize(busy) == lib.MI_OK
+    _destroy(L, [busy])
+
+
+def test_streams_end_while_another_thread_captures(matmul):
+    """The capture is not disturbed, and the streams' memory is given back with the last of them."""
+    import threading
+    import torch
+    L, kern, a, want = matmul
+
+    def session(count, ends):
+        streams = [_create(L) for _ in range(count)]
+        for stream in streams:
+            out = _run(L, kern, a, stream)
+            assert L.mi_stream_synchronize(stream) == lib.MI_OK and torch.equal(out, want)
+        ends.append(streams)
+
+    first = []
+    session(10, first)  # (what the runtime keeps for ten streams)
+    _destroy(L, first[0])
+    torch.cuda.synchronize()
+    before, _ = torch.cuda.mem_get_info()
+    ends = []
+    session(10, ends)
+    failed = []
+
+    def end():
+        failed.extend(s for s in ends[0] if L.mi_stream_destroy(s) != lib.MI_OK)
+
+    out = torch.empty((ROWS, COLS), dtype=torch.int8, device="cuda")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, capture_error_mode="global"):
+        kern.run(a, out=out)
+        thread = threading.Thread(target=end)
+        thread.start()
+        thread.join()
+        kern.run(a, out=out)
+    assert not failed
+    for _ in range(3):
+        out.fill_(55)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+    assert torch.equal(kern.run(a), want)
+    assert torch.cuda.mem_get_info()[0] >= before
+
+
+def test_a_stream_made_after_another_takes_over_its_memory(matmul):
+    """Again and again, the work of the stream before still on its way when its end is asked for: the sums start anew."""
+    import torch
+    L, kern, a, want = matmul
+    held = [_create(L) for _ in range(7)]
+    outs = []
+    for _ in range(20):
+        stream = _create(L)
+        for _ in range(5):
+            outs.append(torch.full((ROWS, COLS), 55, dtype=torch.int8, device="cuda"))
+        torch.cuda.synchronize()
+        for out in outs[-5:]:
+            assert L.mi_matmul_run(kern._h, a.data_ptr(), ROWS, out.data_ptr(), stream) == lib.MI_OK
+        _destroy(L, [stream])
+    torch.cuda.synchronize()
+    assert all(torch.equal(out, want) for out in outs)
+    _destroy(L, held)

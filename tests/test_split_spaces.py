@@ -1,6 +1,7 @@
 """Whose the memory is through which split GEMMs on the library's streams hand over their sums (mindspore_amd/csrc/split_spaces.h,
 compiled for the host with spaces that are no memory): one for each stream from its creation to its end, never two streams' at
-once, never the next stream's before the last one's work is done with it."""
+once, never the next stream's before the last one's work is done with it, none given back while there are streams, all with the
+last."""
 import os
 import subprocess
 
@@ -18,7 +19,7 @@ PROGRAM = r"""
 
 static std::mutex m;
 static std::map<void *, int> made;  // -> the stream that it was made for
-static bool no_memory = false;
+static bool no_memory = false, held_up = false;
 struct Fake {
   typedef int Stream;
   static void *make(int stream) {
@@ -28,10 +29,12 @@ struct Fake {
     made[p] = stream;
     return p;
   }
-  static void free(void *p) {
+  static bool free(void *p) {
     std::lock_guard<std::mutex> lock(m);
+    if (held_up) return false;
     if (made.erase(p) != 1) { printf("freed what was not made\n"); exit(1); }
     ::free(p);
+    return true;
   }
 };
 typedef mi::SplitSpaces<Fake> Spaces;
@@ -81,8 +84,35 @@ int main() {
   s.enter(10, 0);
   CHECK(s.of(10) == nullptr && s.leave(10) == nullptr);
   no_memory = false;
-  for (int i : {1, 3, 4, 5, 6, 7, 9}) end(s, i);
+  // a made one stays for the next stream on its device, and is not given back before the last one's end
+  void *of4 = s.of(4);
+  const int so_far = (int)made.size();
+  end(s, 4);
+  CHECK((int)made.size() == so_far);
+  s.enter(11, 1), s.enter(12, 1), s.enter(13, 1);
+  CHECK((int)made.size() == so_far + 1);
+  s.enter(14, 0);
+  CHECK(s.of(14) == of4 && (int)made.size() == so_far + 1);
+  end(s, 14, true, false);  // (nobody's, but given back with the others)
+  for (int i : {1, 3, 5, 6, 7, 9, 11, 12}) {
+    end(s, i);
+    CHECK((int)made.size() == so_far + 1);
+  }
+  // if it cannot be given back then: with the next last one
+  held_up = true;
+  end(s, 13);
+  CHECK((int)made.size() == so_far + 1);
+  held_up = false;
+  s.enter(15, 1);
+  CHECK((int)made.size() == so_far + 1);
+  end(s, 15);
   CHECK(made.empty());
+  // one session after the other costs nothing
+  for (int i = 100; i < 200; ++i) {
+    s.enter(i, 0);
+    CHECK(s.of(i) != nullptr && made.empty());
+    end(s, i);
+  }
   // many threads, each with streams of its own: a space is one stream's at a time
   Spaces t;
   fill(t);
