@@ -518,12 +518,14 @@ static int prepare_rows(const int8_t *a, int rows, int k, const Workspace &ws, h
   return MI_OK;
 }
 
-// A group whose members run one by one on rows that are no whole chunks: whether all of them run on one padded copy, or those that
-// would read the rows as they are by themselves do so here too.  us, int8 out / fp32 out, one copy -> none: pairs, 200 rows,
-// 390 x 1000 10.8 -> 9.0 / 11.2 -> 10.0, 770 x 1000 11.1 -> 11.55 / 12.0 -> 12.7, 1000 x 1000 11.5 -> 10.5 / 12.3 -> 11.3; three of
-// 390 x 768 14.1 -> 13.1 / 15.1 -> 14.7, 770 x 768 15.1 -> 17.1 / 16.2 -> 18.8, 1000 x 768 15.6 -> 15.4 / 16.7 -> 16.5; four of
-// 1000 x 500 20.1 -> 20.8 / 21.9 -> 22.3.
-static bool shares_padded_copy(int count) { return count > 2; }
+// A group whose members run one by one on rows that are no whole chunks: whether a member (decode: on the decode kernels) runs on the
+// padded copy that they share, or reads the rows as they are where it would by itself.  us, int8 out / fp32 out, one copy -> none:
+// pairs, 200 rows, 390 x 1000 10.8 -> 9.0 / 11.2 -> 10.0, 770 x 1000 11.1 -> 11.55 / 12.0 -> 12.7, 1000 x 1000 11.5 -> 10.5 /
+// 12.3 -> 11.3; three of 390 x 768 14.1 -> 13.1 / 15.1 -> 14.7, 770 x 768 15.1 -> 17.1 / 16.2 -> 18.8, 1000 x 768 15.6 -> 15.4 /
+// 16.7 -> 16.5; four of 1000 x 500 20.1 -> 20.8 / 21.9 -> 22.3.  Pairs on the decode kernels, 33 rows, 1001 x 768 9.6 -> 8.8 /
+// 9.85 -> 9.0, 2001 x 768 11.5 -> 11.8 / 11.65 -> 11.95, 4001 x 768 17.6 -> 19.2 / 17.65 -> 18.1; 64 rows, 1251 x 768 12.25 -> 12.8 /
+// 12.25 -> 12.75, 3003 x 768 15.7 -> 18.05 / 15.3 -> 18.9.
+static bool shares_padded_copy(int count, bool decode) { return count > 2 || (count == 2 && decode); }
 
 // (the blocked copy may be absent: two rows then take the v_dot4 kernel)
 static WeightView weight_view(const RequantState &st) {
@@ -537,7 +539,7 @@ static bool runs_on_gemv(const RequantState &st, int rows, int k16) {
                               : gemv_takes_rows(rows, st.n) && st.w_blocked.p != nullptr && st.k_pad <= 1 << 20;
 }
 
-static int run_requant_gemm(RequantState &st, const int8_t *a, int64_t lda, int rows, int k16, int8_t *c,
+static int run_requant_gemm(const RequantState &st, const int8_t *a, int64_t lda, int rows, int k16, int8_t *c,
                             hipStream_t stream) {
   const RequantParams rq = st.params();
   const WeightView w = weight_view(st);
@@ -545,17 +547,22 @@ static int run_requant_gemm(RequantState &st, const int8_t *a, int64_t lda, int 
   return launch_gemm_requant(a, lda, rows, k16, w, st.n, rq, c, st.n, stream);
 }
 
-// whether the caller's rows are to be read as they are, without a padded copy
-static bool runs_on_anyrow(const RequantState &st, const int8_t *a_dev, int rows) {
-  return !whole_chunks(a_dev, st.k) && !runs_on_gemv(st, rows, round_up(st.k, 16)) && gemm_anyrow_takes(rows, st.k, weight_view(st), st.n);
+// Whether the caller's rows, whatever their length and address, are read as they are, without a padded copy.
+static bool reads_any_rows(const RequantState &st, const int8_t *a_dev, int rows) {
+  const WeightView w = weight_view(st);
+  if (runs_on_gemv(st, rows, round_up(st.k, 16))) return gemv_takes_any_rows(rows, st.k, w, st.n);
+  return !whole_chunks(a_dev, st.k) && gemm_anyrow_takes(rows, st.k, w, st.n);
 }
 
-// The same for the caller's rows, whatever their length and address.
-static int run_requant_rows(RequantState &st, const int8_t *a_dev, int rows, const Workspace &ws, int8_t *c, hipStream_t stream) {
-  if (runs_on_anyrow(st, a_dev, rows))
-    return launch_gemm_anyrow_requant(a_dev, rows, st.k, weight_view(st), st.n, st.params(), c, stream);
-  if (runs_on_gemv(st, rows, round_up(st.k, 16)) && gemv_takes_any_rows(rows, st.k, weight_view(st), st.n))
-    return launch_gemv_requant(a_dev, st.k, rows, st.k, weight_view(st), st.n, st.params(), c, st.n, stream);
+static int run_requant_any_rows(const RequantState &st, const int8_t *a_dev, int rows, int8_t *c, hipStream_t stream) {
+  const RequantParams rq = st.params();
+  const WeightView w = weight_view(st);
+  if (runs_on_gemv(st, rows, round_up(st.k, 16))) return launch_gemv_requant(a_dev, st.k, rows, st.k, w, st.n, rq, c, st.n, stream);
+  return launch_gemm_anyrow_requant(a_dev, rows, st.k, w, st.n, rq, c, stream);
+}
+
+static int run_requant_rows(const RequantState &st, const int8_t *a_dev, int rows, const Workspace &ws, int8_t *c, hipStream_t stream) {
+  if (reads_any_rows(st, a_dev, rows)) return run_requant_any_rows(st, a_dev, rows, c, stream);
   const int8_t *a = nullptr;
   int64_t lda = 0;
   int k16 = 0;
@@ -1002,11 +1009,10 @@ int mi_matmul_run_group(mi_matmul *const *handles, int32_t count, const int8_t *
       return launch_gemm_group_requant(*tile, a, lda, rows, k16, count, wv, n, rq, c_dev, s);
     }
   }
-  const bool copy = shares_padded_copy(count);
   for (int i = 0; i < count; ++i) {
-    RequantState &st = handles[i]->st;
-    if (!copy && runs_on_anyrow(st, a_dev, rows)) {
-      rc = launch_gemm_anyrow_requant(a_dev, rows, k, weight_view(st), st.n, st.params(), c_dev[i], s);
+    const RequantState &st = handles[i]->st;
+    if (!shares_padded_copy(count, runs_on_gemv(st, rows, k16)) && reads_any_rows(st, a_dev, rows)) {
+      rc = run_requant_any_rows(st, a_dev, rows, c_dev[i], s);
     } else if ((rc = prepare()) == MI_OK) {
       rc = run_requant_gemm(st, a, lda, rows, k16, c_dev[i], s);
     }
@@ -1623,8 +1629,17 @@ static bool runs_on_gemv(const mi_dynmm *h, int rows) {
          (rows == 1 || (h->w_blocked.p != nullptr && h->k_pad <= 1 << 20));
 }
 
-static bool runs_on_anyrow(const mi_dynmm *h, const int8_t *a_dev, int rows) {
-  return !runs_on_gemv(h, rows) && !whole_chunks(a_dev, h->k) && gemm_anyrow_takes(rows, h->k, weight_view(h), h->n);
+// as for mi_matmul
+static bool reads_any_rows(const mi_dynmm *h, const int8_t *a_dev, int rows) {
+  const WeightView w = weight_view(h);
+  if (runs_on_gemv(h, rows)) return gemv_takes_any_rows(rows, h->k, w, h->n);
+  return !whole_chunks(a_dev, h->k) && gemm_anyrow_takes(rows, h->k, w, h->n);
+}
+
+static int run_dequant_any_rows(const mi_dynmm *h, const int8_t *a_dev, int rows, const DequantParams &dq, float *c_dev, hipStream_t s) {
+  const WeightView w = weight_view(h);
+  if (runs_on_gemv(h, rows)) return launch_gemv_dequant(a_dev, h->k, rows, h->k, w, h->n, dq, c_dev, h->n, s);
+  return launch_gemm_anyrow_dequant(a_dev, rows, h->k, w, h->n, dq, c_dev, s);
 }
 
 static int run_dequant_gemm(const mi_dynmm *h, const int8_t *a, int64_t lda, int rows, int k16, const DequantParams &dq, float *c_dev,
@@ -1645,10 +1660,7 @@ static int dynmm_run_impl(mi_dynmm *h, const int8_t *a_dev, int32_t rows, float 
   int rc = ensure_device();
   if (rc != MI_OK) return rc;
   const DequantParams dq = dequant_params(h, sx, zx, qp_dev, per_row);
-  if (runs_on_anyrow(h, a_dev, rows))
-    return launch_gemm_anyrow_dequant(a_dev, rows, h->k, weight_view(h), h->n, dq, c_dev, s);
-  if (runs_on_gemv(h, rows) && gemv_takes_any_rows(rows, h->k, weight_view(h), h->n))
-    return launch_gemv_dequant(a_dev, h->k, rows, h->k, weight_view(h), h->n, dq, c_dev, h->n, s);
+  if (reads_any_rows(h, a_dev, rows)) return run_dequant_any_rows(h, a_dev, rows, dq, c_dev, s);
   const int8_t *a = nullptr;
   int64_t lda = 0;
   int k16 = 0;
@@ -1742,12 +1754,11 @@ int mi_dynmm_run_group(mi_dynmm *const *handles, int32_t count, const int8_t *a_
       return launch_gemm_group_dequant(*tile, a, lda, rows, k16, count, wv, n, dq, c_dev, s);
     }
   }
-  const bool copy = shares_padded_copy(count);
   for (int i = 0; i < count; ++i) {
     const mi_dynmm *h = handles[i];
     const DequantParams dq = dequant_params(h, (float)in_scale, in_zp, params_dev, per_row != 0);
-    if (!copy && runs_on_anyrow(h, a_dev, rows)) {
-      rc = launch_gemm_anyrow_dequant(a_dev, rows, k, weight_view(h), h->n, dq, c_dev[i], s);
+    if (!shares_padded_copy(count, runs_on_gemv(h, rows)) && reads_any_rows(h, a_dev, rows)) {
+      rc = run_dequant_any_rows(h, a_dev, rows, dq, c_dev[i], s);
     } else if ((rc = prepare()) == MI_OK) {
       rc = run_dequant_gemm(h, a, lda, rows, k16, dq, c_dev[i], s);
     }

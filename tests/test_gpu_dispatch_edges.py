@@ -245,6 +245,35 @@ def test_matmul_group_on_ragged_rows(m, k, ns, copies, how):
         L.mi_debug_fail_alloc(0)
 
 
+# a group of one on the decode kernels: one row, few, more than go out as one launch; rows shorter than a chunk, and too many long
+# ones, are copied as they are for the member alone
+@pytest.mark.parametrize("m,k,n,copies", [(1, 1001, 300, False), (8, 11009, 40, False), (16, 1001, 300, False), (33, 250, 300, False),
+                                          (64, 1001, 768, False), (5, 9, 300, True), (64, 8003, 300, True)])
+@pytest.mark.parametrize("how", ["static", "value"])
+def test_matmul_group_of_one_on_few_ragged_rows(m, k, n, copies, how):
+    """As the member alone, with and without the room for a padded copy of the rows."""
+    import torch
+    L = K._lib.init()
+    a = torch.from_numpy(np.random.default_rng(k).integers(-128, 128, (m, k), dtype=np.int8)).cuda()
+    args = dict(in_quant=K.QuantParam(0.03, -5)) if how == "value" else {}
+    make = lambda: _matmul_pair(np.random.default_rng(n), n, k, False, how != "static")[4](True)
+    group = lambda kern: (K.matmul_run_group([kern], a) if how == "static" else K.dynmm_run_group([kern], a, **args))[0]
+    want = make().run(a, **args)
+    assert torch.equal(group(make()), want)
+    alone, member = make(), make()
+    assert L.mi_debug_fail_alloc(m * ((k + 15) // 16 * 16)) == 0
+    try:
+        for run in (lambda: alone.run(a, **args), lambda: group(member)):
+            if copies:
+                with pytest.raises(K._lib.MiError) as e:
+                    run()
+                assert e.value.code == K._lib.MI_MEMORY_FAILED
+            else:
+                assert torch.equal(run(), want)
+    finally:
+        L.mi_debug_fail_alloc(0)
+
+
 @pytest.mark.parametrize("taps", [3, 5])
 @pytest.mark.parametrize("b,ih,iw,ch,pad", [(1, 5, 5, 4, (0, 0, 0, 0)), (1, 5, 6, 8, (1, 1, 1, 1)), (2, 7, 9, 12, (2, 0, 0, 2)),
                                             (1, 9, 11, 20, (4, 4, 4, 4)), (3, 6, 8, 192, (1, 2, 3, 0)), (1, 33, 31, 36, (1, 1, 1, 1)),
