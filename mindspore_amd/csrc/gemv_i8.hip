@@ -988,12 +988,20 @@ static int with_rows(const int8_t *a, int64_t lda, int k, F &&f) {
 
 // A copy of the rows in whole chunks is a launch of its own, 2.4 us on the host and 1.4 - 1.9 us of the kernels' 2.5 - 6.  Without
 // it every workgroup moves its rows' unaligned chunks into place, which costs more where there are more rows, where K is long,
-// and where there are more workgroups than CUs.  us, copy / none (K x channels): 1 row 1001 x 1001 6.7 / 4.0, 11009 x 10000
-// 19.9 / 18.6; 4 rows 1000 x 4096 6.4 / 3.9, 8003 x 10000 16.7 / 15.0; 16 rows 1000 x 1001 6.8 / 4.2, 8003 x 4096 10.3 / 9.7,
-// 3003 x 6001 (14 rows) 1 % less, 5003 x 6001 6 % more, 8003 x 10000 20.0 / 23.6; 32 rows 4001 x 4096 8.9 / 7.8, 6001 x 1001 4 %
-// more, 11009 x 10000 38.5 / 43.8; 64 rows 2001 x 4096 7.9 / 7.1, 4001 x 4096 12.9 / 12.2, 8003 x 1001 18.2 / 19.7.
+// and where there are more workgroups than CUs: most between 4097 and 8191 channels, since the form for 9 to 16 rows there takes 145
+// registers for 127, and a CU then holds one workgroup for two.  us, copy / none (rows x K x channels): 1 x 1001 x 1001 6.7 / 4.0, 1 x 11009 x 10000 19.9 / 18.6, 8 x 8003 x 6001
+// 11.8 / 10.8, 8 x 15003 x 12288 31.2 / 30.9; 9 x 11009 x 2048 9.5 / 9.2, 9 x 15003 x 2048 11.65 / 11.55, 16 x 8003 x 2048 8.9 / 8.4,
+// 16 x 9001 x 768 9.2 / 9.4, 16 x 15003 x 768 11.3 / 12.6; 12 x 501 x 6001 6.55 / 6.9, 16 x 1001 x 6001 6.8 / 6.9, 16 x 4001 x 6001
+// 8.25 / 9.25, 16 x 4001 x 12288 10.75 / 9.15; 32 x 2501 x 8100 9.85 / 9.7, 32 x 3303 x 8100 10.8 / 11.0, 32 x 4001 x 4096 8.7 / 8.0,
+// 32 x 6001 x 1001 4 % more; 48 x 4001 x 4096 11.35 / 10.55; 56 x 2501 x 4096 9.2 / 8.5, 64 x 2501 x 1500 8.6 / 8.5, 56 x 3505 x 1500
+// 9.4 / 10.2, 64 x 3505 x 1500 9.9 / 10.7.
 bool gemv_takes_any_rows(int m, int k, const WeightView &w, int n) {
-  return k >= 16 && (m == 1 || w.blocked != nullptr) && (m <= 8 || k <= 4096 || (m <= 16 && n <= kGemvNarrowChannels));
+  if (k < 16 || (m > 1 && w.blocked == nullptr)) return false;
+  const bool narrow = n <= kGemvNarrowChannels, wide = n >= 8192;  // (wide: three channel groups a workgroup)
+  if (m <= 8) return true;
+  if (m <= 16) return narrow ? (int64_t)m * k <= 128 * 1024 : wide && k <= 4096;
+  if (m <= 48) return k <= (narrow || wide ? 4096 : 3072);
+  return k <= 2560;
 }
 
 static int check_gemv_operands(const int8_t *a, int64_t lda, int m, int k, const WeightView &wv, int n, const int8_t *c, int64_t ldc) {

@@ -245,6 +245,40 @@ def test_matmul_group_on_ragged_rows(m, k, ns, copies, how):
         L.mi_debug_fail_alloc(0)
 
 
+# both sides of each line between few ragged rows as they are and on a copy: rows x K up to 16 rows against few channels, 4097 to
+# 8191 channels, more than 16 rows, more than 48
+@pytest.mark.parametrize("m,k,n,copies", [(8, 13007, 33, False), (16, 8191, 33, False), (16, 8193, 33, True), (9, 14563, 33, False),
+                                          (9, 14565, 33, True), (8, 501, 4100, False), (9, 501, 4096, False), (9, 501, 4097, True),
+                                          (16, 4001, 8191, True), (16, 4001, 8192, False), (16, 4097, 8192, True), (17, 501, 4097, False),
+                                          (17, 3071, 4097, False), (17, 3073, 4097, True), (32, 4095, 8192, False), (32, 4097, 33, True),
+                                          (48, 4095, 33, False), (49, 2559, 33, False), (49, 2561, 33, True)])
+@pytest.mark.parametrize("dynamic", [False, True])
+def test_matmul_few_ragged_rows_copied_or_not(orc, m, k, n, copies, dynamic):
+    import torch
+    L = K._lib.init()
+    rng = np.random.default_rng(n + k)
+    w, bias, sw, zw, make = _matmul_pair(rng, n, k, True, dynamic)
+    a = rng.integers(-128, 128, (m, k), dtype=np.int8)
+    dev, args = torch.from_numpy(a).cuda(), dict(in_quant=K.QuantParam(0.03, -5)) if dynamic else {}
+    kern = make(True)
+    assert L.mi_debug_fail_alloc(m * ((k + 15) // 16 * 16)) == 0
+    try:
+        if copies:
+            with pytest.raises(K._lib.MiError) as e:
+                kern.run(dev, **args)
+            assert e.value.code == K._lib.MI_MEMORY_FAILED
+        else:
+            kern.run(dev, **args)
+    finally:
+        L.mi_debug_fail_alloc(0)
+    orc.set_threads(16)
+    if dynamic:
+        want = orc.dynamic_matmul(a, w, bias, 0.03, -5, sw, zw)
+    else:
+        want = orc.matmul_int8(a, w, bias, 0.02, 7, sw, zw, float(np.float32(0.02 * 0.0055 * k ** 0.5 * 140)), 3)
+    assert np.array_equal(kern.run(dev, **args).cpu().numpy(), want)
+
+
 # a group of one on the decode kernels: one row, few, more than go out as one launch; rows shorter than a chunk, and too many long
 # ones, are copied as they are for the member alone
 @pytest.mark.parametrize("m,k,n,copies", [(1, 1001, 300, False), (8, 11009, 40, False), (16, 1001, 300, False), (33, 250, 300, False),
