@@ -58,6 +58,9 @@ int mi_debug_fail_alloc(size_t bytes);
 /* Test aid: how many times the library has made the host wait for a stream so far (mi_copy_to_device, mi_copy_to_host,
  * mi_stream_synchronize, mi_dynquant_get_params; the *_run_host entry points are not counted). */
 int64_t mi_debug_sync_count(void);
+/* Test aid: how many MatMuls the calling thread has launched with their K split over workgroups, and, where asked for, the
+ * tile (10 x channels / 64 + rows / 64) and the number of parts of the last one. */
+int64_t mi_debug_split_launches(int32_t *tile, int32_t *parts);
 const char *mi_version(void);
 
 /* ---- quant-parameter derivation (host arithmetic, no GPU needed) -------------------------------------------- */

@@ -762,6 +762,12 @@ int mi_copy_to_host_async(void *dst_host, const void *src_dev, size_t bytes, voi
 
 int64_t mi_debug_sync_count(void) { return g_sync_count.load(std::memory_order_relaxed); }
 
+int64_t mi_debug_split_launches(int32_t *tile, int32_t *parts) {
+  if (tile != nullptr) *tile = t_split_launches.tile;
+  if (parts != nullptr) *parts = t_split_launches.parts;
+  return t_split_launches.count;
+}
+
 int mi_stream_create(void **out_stream) {
   if (out_stream == nullptr) return MI_NULL_PTR;
   *out_stream = nullptr;

@@ -139,6 +139,12 @@ __host__ __device__ inline int weight_row_stride(int k_pad) { return (k_pad / 25
 constexpr size_t kSplitCounterBytes = 1024, kSplitSumBytes = 256 * 256 * (4 * 64 + 16);  // 256 parts of 128 x 128 sums and row sums
 constexpr size_t kSplitBytes = kSplitCounterBytes + kSplitSumBytes;
 void *split_space(hipStream_t stream);
+// For tests: the launches of split GEMMs of this thread so far, and the tile (as launch_gemm_split has it) and parts of the last.
+struct SplitLaunches {
+  int64_t count;
+  int32_t tile, parts;
+};
+extern thread_local SplitLaunches t_split_launches;
 
 // A: int8 activations [M][lda] (lda in bytes, multiple of 16, base 16-byte aligned, K % 16 == 0);
 // W: packed weights (above); C: [M][ldc] elements, any n, ldc == n, any address of the element type.

@@ -133,12 +133,15 @@ static int with_form(int parts, bool requant, bool has_zw, bool fast, const Gemm
   return MI_ERROR;
 }
 
+thread_local SplitLaunches t_split_launches;
+
 int launch_gemm_split(int tile, int parts, bool requant, bool has_zw, bool fast, const GemmArgs &g, const RequantParams &rq,
                       const DequantParams &dq, void *space, hipStream_t stream) {
   if (g.wb == nullptr || space == nullptr) {
     set_error("gemm: the blocked weight copy or the space for split sums is missing");
     return MI_NULL_PTR;
   }
+  t_split_launches = SplitLaunches{t_split_launches.count + 1, tile, parts};
   switch (tile) {
     case 11: return with_form<1, 1, 5>(parts, requant, has_zw, fast, g, rq, dq, space, stream);
     case 12: return with_form<1, 2, 6>(parts, requant, has_zw, fast, g, rq, dq, space, stream);

@@ -785,13 +785,23 @@ def test_convolution_wide_strides_and_pads(orc, ic, kernel, far):
     assert np.array_equal(_gpu_conv(case, stride, (1, 1), pad, 1, device_tensors=True, exact_3x3=True), orc.conv_int8(**case))
 
 
-# K in several parts a tile, as choose_split deals it out: 64 x 64 tiles in 5, 8, 5, 3 and 2 parts, 64 channels x 128 rows in 4 and 2,
-# 128 x 128 in 2; parts of unequal length, a last block, last rows and channels that are partly there, rows to be padded first
-@pytest.mark.parametrize("m,n,k", [(70, 200, 5632), (100, 256, 8200), (129, 257, 4100), (200, 1000, 4700), (100, 3330, 8368),
-                                   (128, 4096, 11008), (250, 4000, 11008), (300, 4096, 8192), (512, 4000, 11008)])
+def _split_launches():
+    """(how many split launches so far, tile and parts of the last one)"""
+    import ctypes as C
+    tile, parts = C.c_int32(0), C.c_int32(0)
+    return K._lib.load().mi_debug_split_launches(C.byref(tile), C.byref(parts)), tile.value, parts.value
+
+
+# K in several parts a tile, as choose_split deals it out: tile (10 x channels / 64 + rows / 64) and parts, up to the most of each
+# tile; parts of unequal length, a last block, last rows and channels that are partly there, rows to be padded first
+@pytest.mark.parametrize("m,n,k,tile,parts", [(70, 200, 5632, 11, 5), (100, 256, 8200, 11, 6), (129, 257, 4100, 11, 5), (200, 1000, 4700, 11, 3),
+                                              (70, 64, 11008, 11, 8), (65, 65, 16400, 11, 8), (80, 300, 8900, 11, 7),
+                                              (100, 3330, 8368, 11, 2), (128, 4096, 11008, 12, 4), (250, 4000, 11008, 12, 2),
+                                              (300, 4096, 8192, 22, 2), (512, 4000, 11008, 22, 2)])
 @pytest.mark.parametrize("dynamic,asymmetric", [(False, False), (False, True), (True, False)])
-def test_matmul_with_k_in_parts(orc, m, n, k, dynamic, asymmetric):
-    """On the null stream, where K is split, and on another, where it is not: the same sums.  Small ones against the oracle too."""
+def test_matmul_with_k_in_parts(orc, m, n, k, tile, parts, dynamic, asymmetric):
+    """On the null stream, where K is split, and on another, where it is not: the same sums.  Against the oracle too: all rows of
+    small ones, rows at the tiles' edges of the others."""
     import torch
     rng = np.random.default_rng(m + n + k)
     w, bias, sw, zw, make = _matmul_pair(rng, n, k, asymmetric, dynamic)
@@ -801,21 +811,24 @@ def test_matmul_with_k_in_parts(orc, m, n, k, dynamic, asymmetric):
     args = dict(in_quant=K.QuantParam(0.03, -5)) if dynamic else {}
     torch.cuda.synchronize()
     other = torch.cuda.Stream()
+    so_far = _split_launches()[0]
     with torch.cuda.stream(other):
         want = kern.run(dev, **args)
     other.synchronize()
+    assert _split_launches()[0] == so_far
     for _ in range(4):  # (the counters are left as they were found)
         got = [kern.run(dev, **args) for _ in range(3)]
         torch.cuda.synchronize()
         for y in got:
             assert torch.equal(y.view(torch.int8), want.view(torch.int8))
-    if m * n * k < 1e9:
-        orc.set_threads(16)
-        if dynamic:
-            sure = orc.dynamic_matmul(a, w, bias, 0.03, -5, sw, zw)
-        else:
-            sure = orc.matmul_int8(a, w, bias, 0.02, 7, sw, zw, float(np.float32(0.02 * 0.0055 * k ** 0.5 * 140)), 3)
-        assert np.array_equal(want.cpu().numpy(), sure)
+    assert _split_launches() == (so_far + 12, tile, parts)
+    rows = np.arange(m) if m * n * k < 1e9 else np.unique(np.r_[0, 1, 31, 63:65, 127:129, m // 2, m - 2, m - 1] % m)
+    orc.set_threads(16)
+    if dynamic:
+        sure = orc.dynamic_matmul(a[rows], w, bias, 0.03, -5, sw, zw)
+    else:
+        sure = orc.matmul_int8(a[rows], w, bias, 0.02, 7, sw, zw, float(np.float32(0.02 * 0.0055 * k ** 0.5 * 140)), 3)
+    assert np.array_equal(want.cpu().numpy()[rows], sure)
 
 
 def test_matmul_with_k_in_parts_on_library_streams():
@@ -840,6 +853,8 @@ def test_matmul_with_k_in_parts_on_library_streams():
         for _ in range(200):
             if L.mi_matmul_run(kern._h, C.c_void_p(dev.data_ptr()), 150, C.c_void_p(out.data_ptr()), stream) != 0:
                 failed.append("run")
+        if _split_launches()[0] != 200:  # (of this thread)
+            failed.append("not split")
         L.mi_stream_synchronize(stream)
         if not torch.equal(out, want):
             failed.append("result")

@@ -26,8 +26,13 @@ def matmul():
     with torch.cuda.stream(torch.cuda.Stream()):
         want = kern.run(a)  # on one piece of K
     torch.cuda.synchronize()
-    assert torch.equal(kern.run(a), want)
+    before = _splits(L)
+    assert torch.equal(kern.run(a), want) and _splits(L) == before + 1
     return L, kern, a, want
+
+
+def _splits(L):
+    return L.mi_debug_split_launches(None, None)
 
 
 def _create(L):
@@ -64,6 +69,7 @@ def test_runs_on_a_library_stream_allocate_nothing(matmul, memory):
     torch.equal(out, want)  # (and torch for a comparison)
     torch.cuda.synchronize()
     before, _ = torch.cuda.mem_get_info()
+    split = _splits(L)
     try:
         for _ in range(3):
             out.fill_(55)
@@ -71,7 +77,7 @@ def test_runs_on_a_library_stream_allocate_nothing(matmul, memory):
             assert L.mi_matmul_run(kern._h, a.data_ptr(), ROWS, out.data_ptr(), streams[-1]) == lib.MI_OK
             assert L.mi_stream_synchronize(streams[-1]) == lib.MI_OK
             assert torch.equal(out, want)
-        assert torch.cuda.mem_get_info()[0] == before
+        assert torch.cuda.mem_get_info()[0] == before and _splits(L) == split + (0 if memory == "none" else 3)
     finally:
         L.mi_debug_fail_alloc(0)
     _destroy(L, streams)
@@ -156,9 +162,53 @@ def test_a_stream_made_after_another_takes_over_its_memory(matmul):
         for _ in range(5):
             outs.append(torch.full((ROWS, COLS), 55, dtype=torch.int8, device="cuda"))
         torch.cuda.synchronize()
+        split = _splits(L)
         for out in outs[-5:]:
             assert L.mi_matmul_run(kern._h, a.data_ptr(), ROWS, out.data_ptr(), stream) == lib.MI_OK
+        assert _splits(L) == split + 5
         _destroy(L, [stream])
     torch.cuda.synchronize()
     assert all(torch.equal(out, want) for out in outs)
     _destroy(L, held)
+
+
+def test_the_entry_point_that_allocates_nothing_splits_on_library_streams(matmul):
+    import torch
+    L, kern, a, want = matmul
+    stream = _create(L)
+    split = _splits(L)
+    out = _run(L, kern, a, stream, run="mi_matmul_run_noalloc")
+    assert L.mi_stream_synchronize(stream) == lib.MI_OK
+    assert torch.equal(out, want) and _splits(L) == split + 1
+    _destroy(L, [stream])
+
+
+@pytest.mark.parametrize("run", ["mi_matmul_run", "mi_matmul_run_noalloc"])
+def test_captures_of_a_library_stream_are_not_split(matmul, run):
+    """Replays on another stream, beside the captured stream's own split launches: they share no memory."""
+    import torch
+    L, kern, a, want = matmul
+    stream = _create(L)
+    own = torch.cuda.ExternalStream(stream.value)
+    outs = [torch.empty((ROWS, COLS), dtype=torch.int8, device="cuda") for _ in range(8)]
+    call = lambda out: getattr(L, run)(kern._h, a.data_ptr(), ROWS, out.data_ptr(), stream)
+    split = _splits(L)
+    torch.cuda.synchronize()
+    assert call(outs[0]) == lib.MI_OK and _splits(L) == split + 1
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=own):
+        assert call(outs[1]) == lib.MI_OK and call(outs[2]) == lib.MI_OK
+    assert _splits(L) == split + 1
+    other = torch.cuda.Stream()
+    for _ in range(20):
+        for out in outs:
+            out.fill_(55)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(other):
+            graph.replay()
+        for out in outs[3:]:
+            assert call(out) == lib.MI_OK
+        torch.cuda.synchronize()
+        assert all(torch.equal(out, want) for out in outs[1:])
+    assert _splits(L) == split + 101
+    _destroy(L, [stream])
