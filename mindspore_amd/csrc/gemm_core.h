@@ -657,6 +657,13 @@ struct RowSums {
   }
 };
 
+// The ring's loops (gemm_ring.h): up to two row tiles the weights stream past the L2s, which then keep the activations that every
+// channel tile re-reads.  With more row tiles too many workgroups rely on finding them there.  us per launch, weights from HBM,
+// plain -> streamed: one row tile, 128 x 12288 x 4096 18.4 -> 16.3, 128 x 11008 x 4096 17.6 -> 16.0; two, 256 x 12288 x 4096 26.3 -> 23.4,
+// 128 x 4096 x 4096 11.8 -> 11.0; three, 300 x 5504 x 2048 (fp32) 13.9 -> 14.8; four, 197 x 768 x 3072 (fp32) 8.2 -> 9.4;
+// thirty-two, 4096 x 768 x 3072 (fp32) 16.3 -> 22.0.
+constexpr int kStreamRowTiles = 2;
+
 // Launches of the K-block loops (gemm_kblock.hip, gemm_ring.hip), one per tile shape: T = 10 x TN + TM, the workgroup's
 // tile being 64 TN channels x 64 TM rows.  requant: int8 output, fast2 form or not; otherwise fp32, `fast` = non-temporal
 // stores.

@@ -367,18 +367,21 @@ static const TileCost &cheapest_tile(int m, int k, int count, const int *n, floa
 }
 // K split over the workgroups of a tile (gemm_split.hip): expected to take a + b x K blocks of a part + 1.7 us for the sums' way
 // through memory + `part` for every part after the first + `wg` for every workgroup, whose sums all go that way at once.  b_far:
-// where the weights are too large to be in the caches.  The margins are for what a and b do not know.  us per launch, unsplit /
-// split, weights from memory: 65 x 3328 x 8368 24.8 / 16.6, 128 x 4096 x 11008 26.3 / 18.3, 128 x 4096 x 4096 10.7 / 9.8,
-// 64 x 6000 x 8000 21.9 / 15.8, 100 x 1024 x 4096 9.5 / 7.8, 138 x 1408 x 5632 10.9 / 9.3, 300 x 1024 x 8192 14.4 / 10.5,
-// 1000 x 512 x 8192 14.9 / 12.2, 512 x 4096 x 11008 38.1 / 35.7; not taken: 200 x 1024 x 2048 5.8 / 7.0, 197 x 768 x 3072 7.43 / 7.46,
-// 161 x 1280 x 3120 7.86 / 7.87, 512 x 4096 x 4096 13.3 / 18.5, 256 x 4096 x 4096 10.0 / 13.2, 800 x 1280 x 5120 14.5 / 15.6.
+// where the weights are too large to be in the caches, which holds up unsplit launches too, but not 64 x 64 tiles of more rows than
+// the weights stream past (kStreamRowTiles); b_two, where it is not 0: with two row tiles.  The margins are for what a and b do not
+// know.  us per launch, unsplit / split, weights from memory: 65 x 3328 x 8368 24.8 / 16.6, 128 x 4096 x 11008 26.3 / 18.3,
+// 128 x 4096 x 4096 10.7 / 9.8, 64 x 6000 x 8000 21.9 / 15.8, 100 x 1024 x 4096 9.5 / 7.8, 138 x 1408 x 5632 10.9 / 9.3,
+// 300 x 1024 x 8192 14.4 / 10.5, 1000 x 512 x 8192 14.9 / 12.2, 512 x 4096 x 11008 38.1 / 35.7, 176 x 2407 x 7360 18.75 / 13.6; not
+// taken: 200 x 1024 x 2048 5.8 / 7.0, 197 x 768 x 3072 7.43 / 7.46, 161 x 1280 x 3120 7.86 / 7.87, 512 x 4096 x 4096 13.3 / 18.5,
+// 256 x 4096 x 4096 10.0 / 13.2, 800 x 1280 x 5120 14.5 / 15.6, and for b_two 144 x 3756 x 10336 20.7 / 31.2, 199 x 2252 x 7888 15.5 /
+// 19.1, 232 x 2905 x 10016 24.05 / 28.1.
 struct SplitCost {
   int tn, tm, most_parts;
-  float a, b, b_far, part, wg;
+  float a, b, b_far, b_two, part, wg;
 };
-constexpr SplitCost kSplitCosts[] = {{1, 1, 8, 2.8f, 0.25f, 0.285f, 0.25f, 0.008f},
-                                     {1, 2, 8, 2.9f, 0.36f, 0.41f, 0.35f, 0.016f},
-                                     {2, 2, 2, 3.0f, 0.57f, 0.57f, 0.5f, 0.022f}};
+constexpr SplitCost kSplitCosts[] = {{1, 1, 8, 2.8f, 0.25f, 0.285f, 0, 0.25f, 0.008f},
+                                     {1, 2, 8, 2.9f, 0.36f, 0.41f, 0.55f, 0.35f, 0.016f},
+                                     {2, 2, 2, 3.0f, 0.57f, 0.57f, 0, 0.5f, 0.022f}};
 constexpr int64_t kFarWeights = 16 << 20;
 // The tile and the number of parts, or null where the unsplit launch on `whole` is expected to be as quick.
 static const SplitCost *choose_split(int m, int k, int n, const TileCost &whole, float cost, int *parts) {
@@ -386,13 +389,15 @@ static const SplitCost *choose_split(int m, int k, int n, const TileCost &whole,
   const int kblocks = (k + 127) / 128;
   const bool far = (int64_t)n * k >= kFarWeights;
   for (const SplitCost &t : kSplitCosts)
-    if (far && whole.ring && whole.tn == t.tn && whole.tm == t.tm) cost *= (t.a + t.b_far * (float)kblocks) / (t.a + t.b * (float)kblocks);
+    if (far && whole.ring && whole.tn == t.tn && whole.tm == t.tm && (t.tm > 1 || (m + 63) / 64 <= kStreamRowTiles))
+      cost *= (t.a + t.b_far * (float)kblocks) / (t.a + t.b * (float)kblocks);
   float least = (far ? 0.99f : 0.9f) * cost;
   for (const SplitCost &t : kSplitCosts) {
-    const int64_t tiles = (int64_t)((m + 64 * t.tm - 1) / (64 * t.tm)) * ((n + 64 * t.tn - 1) / (64 * t.tn));
+    const int64_t rows = (m + 64 * t.tm - 1) / (64 * t.tm), tiles = rows * ((n + 64 * t.tn - 1) / (64 * t.tn));
     const int most = (int)std::min<int64_t>(256 / tiles, std::min(kblocks, t.most_parts));
+    const float b = rows == 2 && t.b_two > 0 ? t.b_two : far ? t.b_far : t.b;
     for (int p = 2; p <= most; ++p) {
-      const float c = t.a + (far ? t.b_far : t.b) * (float)((kblocks + p - 1) / p) + 1.7f + t.part * (float)(p - 1) + t.wg * (float)(tiles * p);
+      const float c = t.a + b * (float)((kblocks + p - 1) / p) + 1.7f + t.part * (float)(p - 1) + t.wg * (float)(tiles * p);
       if (c < least) best = &t, least = c, *parts = p;
     }
   }
