@@ -1008,7 +1008,7 @@ int mi_matmul_run_group(mi_matmul *const *handles, int32_t count, const int8_t *
       rq[i] = handles[i]->st.params();
       n[i] = handles[i]->st.n;
     }
-    const TileCost *tile = decode ? nullptr : gemm_group_tile(k16, rows, k16, count, wv, n, rq);
+    const TileCost *tile = decode ? nullptr : gemm_group_tile(k16, rows, k16, count, wv, n, rq, s);
     if (decode || tile != nullptr) {
       if ((rc = prepare()) != MI_OK) return rc;
       if (decode) return launch_gemv_group(a, lda, rows, k16, count, wv, n, rq, c_dev, s);
@@ -1753,7 +1753,7 @@ int mi_dynmm_run_group(mi_dynmm *const *handles, int32_t count, const int8_t *a_
       dq[i] = dequant_params(handles[i], (float)in_scale, in_zp, params_dev, per_row != 0);
       n[i] = handles[i]->n;
     }
-    const TileCost *tile = decode ? nullptr : gemm_group_tile(k16, rows, k16, count, wv, n, dq);
+    const TileCost *tile = decode ? nullptr : gemm_group_tile(k16, rows, k16, count, wv, n, dq, s);
     if (decode || tile != nullptr) {
       if ((rc = prepare()) != MI_OK) return rc;
       if (decode) return launch_gemv_group_dequant(a, lda, rows, k16, count, wv, n, dq, c_dev, s);

@@ -162,10 +162,12 @@ int launch_gemm_anyrow_dequant(const int8_t *a, int m, int k, const WeightView &
 
 // Up to four weight matrices with the same K against the same activation rows as one launch; member i writes c[i] with row
 // stride n[i].  gemm_group_tile: what the launch would run on, or null where the members are to be run one by one; lda: of the
-// rows that it would be given.
+// rows that it would be given; stream: theirs, since members are split on some only.
 struct TileCost;
-const TileCost *gemm_group_tile(int64_t lda, int m, int k, int count, const WeightView *w, const int *n, const RequantParams *rq);
-const TileCost *gemm_group_tile(int64_t lda, int m, int k, int count, const WeightView *w, const int *n, const DequantParams *dq);
+const TileCost *gemm_group_tile(int64_t lda, int m, int k, int count, const WeightView *w, const int *n, const RequantParams *rq,
+                                hipStream_t stream);
+const TileCost *gemm_group_tile(int64_t lda, int m, int k, int count, const WeightView *w, const int *n, const DequantParams *dq,
+                                hipStream_t stream);
 int launch_gemm_group_requant(const TileCost &tile, const int8_t *a, int64_t lda, int m, int k, int count, const WeightView *w,
                               const int *n, const RequantParams *rq, int8_t *const *c, hipStream_t stream);
 int launch_gemm_group_dequant(const TileCost &tile, const int8_t *a, int64_t lda, int m, int k, int count, const WeightView *w,

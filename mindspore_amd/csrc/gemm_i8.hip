@@ -383,8 +383,8 @@ constexpr SplitCost kSplitCosts[] = {{1, 1, 8, 2.8f, 0.25f, 0.285f, 0, 0.25f, 0.
                                      {1, 2, 8, 2.9f, 0.36f, 0.41f, 0.55f, 0.35f, 0.016f},
                                      {2, 2, 2, 3.0f, 0.57f, 0.57f, 0, 0.5f, 0.022f}};
 constexpr int64_t kFarWeights = 16 << 20;
-// The tile and the number of parts, or null where the unsplit launch on `whole` is expected to be as quick.
-static const SplitCost *choose_split(int m, int k, int n, const TileCost &whole, float cost, int *parts) {
+// The tile, the number of parts and what they are expected to take, or null where the unsplit launch on `whole` is expected to be as quick.
+static const SplitCost *choose_split(int m, int k, int n, const TileCost &whole, float cost, int *parts, float *split_cost) {
   const SplitCost *best = nullptr;
   const int kblocks = (k + 127) / 128;
   const bool far = (int64_t)n * k >= kFarWeights;
@@ -401,6 +401,7 @@ static const SplitCost *choose_split(int m, int k, int n, const TileCost &whole,
       if (c < least) best = &t, least = c, *parts = p;
     }
   }
+  if (best != nullptr) *split_cost = least;
   return best;
 }
 // (the K-block loaders address activation rows with 32-bit offsets from the tile's first row)
@@ -425,7 +426,7 @@ static int launch_pick_tile(const GemmArgs &g, const RequantParams &rq, const De
     const TileCost &t = cheapest_tile(g.m, g.k, 1, &g.n, &cost);
     if (EPI == EPI_REQUANT ? FAST : !HAS_ZW) {  // (the forms that gemm_split.hip has)
       int parts;
-      const SplitCost *split = choose_split(g.m, g.k, g.n, t, cost, &parts);
+      const SplitCost *split = choose_split(g.m, g.k, g.n, t, cost, &parts, &cost);
       void *space = split != nullptr ? split_space(stream) : nullptr;
       if (space != nullptr)
         return launch_gemm_split(10 * split->tn + split->tm, parts, EPI == EPI_REQUANT, HAS_ZW, FAST, g, rq, dq, space, stream);
@@ -662,29 +663,44 @@ int launch_gemm_anyrow_dequant(const int8_t *a, int m, int k, const WeightView &
 // round of tiles more is the price of a launch that fills its last round badly, and there are fewer of those, on larger tiles.
 // us per pair of 11008 x 4096, two launches -> one: int8 output, 128 rows 33.6 -> 26.3, 256 rows 47.6 -> 34.0, 512 rows
 // 64.6 -> 51.5; fp32 output with a scale per row, 2048 rows 194.8 -> 181.
-static const TileCost *group_tile(int64_t lda, int m, int k, int count, const WeightView *w, const int *n) {
+// The one launch is never split, so few channels of long K stay apart where each member alone is split.  kManyRows: per K block on
+// 64 x 64 tiles of more rows than the weights stream past, which find them in the L2s.  us per pair (rows x channels x K), one
+// launch / two split ones: 70 x 64 x 11008 25.7 / 16.05, 70 x 64 x 8192 18.75 / 14.8, 100 x 256 x 11008 21.95 / 17.5,
+// 100 x 1024 x 11008 22.55 / 21.2, 128 x 512 x 8192 18.95 / 17.85, 200 x 64 x 16384 25.45 / 17.75, 512 x 128 x 32768 52.0 / 27.4; stay
+// together: 128 x 512 x 7168 17.1 / 18.2, 100 x 1024 x 8192 16.95 / 18.2, 128 x 768 x 8192 19.15 / 18.65, 70 x 64 x 5120 13.45 / 14.3,
+// 200 x 512 x 11008 19.55 / 21.0, 500 x 256 x 12288 20.0 / 21.4, three of 100 x 256 x 11008 26.3 / 26.3, four of 70 x 64 x 16384
+// 35.95 / 36.3.
+static const TileCost *group_tile(int64_t lda, int m, int k, int count, const WeightView *w, const int *n, hipStream_t stream) {
   if (count < 2 || count > kGemmGroupMax || k < 1024 || !kblock_takes(k, lda)) return nullptr;
-  float alone = 0.0f, together;
+  float alone = 0.0f, alone_split = 0.0f, together;
   for (int i = 0; i < count; ++i) {
     if (w[i].blocked == nullptr || w[i].k_pad != w[0].k_pad) return nullptr;
     float cost;
-    cheapest_tile(m, k, 1, n + i, &cost);
+    int parts;
+    const TileCost &whole = cheapest_tile(m, k, 1, n + i, &cost);
     alone += cost;
+    choose_split(m, k, n[i], whole, cost, &parts, &cost);  // (the members' forms are those of gemm_split.hip)
+    alone_split += cost;
   }
   const TileCost &t = cheapest_tile(m, k, count, n, &together);
-  return together < alone ? &t : nullptr;
+  if (together >= alone) return nullptr;
+  constexpr float kManyRows = 0.18f;
+  if (t.ring && t.tn == 1 && t.tm == 1 && (m + 63) / 64 > kStreamRowTiles) together = t.a + kManyRows * (float)((k + 127) / 128);
+  return together < alone_split || split_space(stream) == nullptr ? &t : nullptr;
 }
 
-const TileCost *gemm_group_tile(int64_t lda, int m, int k, int count, const WeightView *w, const int *n, const RequantParams *rq) {
+const TileCost *gemm_group_tile(int64_t lda, int m, int k, int count, const WeightView *w, const int *n, const RequantParams *rq,
+                                hipStream_t stream) {
   for (int i = 0; i < count; ++i)
     if (rq[i].has_zw || !rq[i].fast2) return nullptr;
-  return group_tile(lda, m, k, count, w, n);
+  return group_tile(lda, m, k, count, w, n, stream);
 }
 
-const TileCost *gemm_group_tile(int64_t lda, int m, int k, int count, const WeightView *w, const int *n, const DequantParams *dq) {
+const TileCost *gemm_group_tile(int64_t lda, int m, int k, int count, const WeightView *w, const int *n, const DequantParams *dq,
+                                hipStream_t stream) {
   for (int i = 0; i < count; ++i)
     if (dq[i].zw0 != 0) return nullptr;
-  return group_tile(lda, m, k, count, w, n);
+  return group_tile(lda, m, k, count, w, n, stream);
 }
 
 template <typename P>

@@ -835,6 +835,45 @@ def test_matmul_with_k_in_parts(orc, m, n, k, tile, parts, dynamic, asymmetric):
     assert np.array_equal(want.cpu().numpy()[rows], sure)
 
 
+# both sides of the line between a group's one launch and members whose K is split: at one and two row tiles and beyond, rows to be padded
+# first, members of unequal size, more than two
+@pytest.mark.parametrize("m,ns,k,apart", [(70, (64, 64), 11008, True), (70, (64, 64), 7100, True), (70, (64, 64), 5120, False),
+                                          (128, (512, 512), 8192, True), (128, (512, 512), 7168, False), (65, (1024, 64), 11008, True),
+                                          (100, (1024, 1024), 8192, False), (100, (256, 250, 256), 14336, True),
+                                          (100, (256, 250, 256), 11008, False), (200, (64, 64), 16384, True),
+                                          (200, (512, 500), 11008, False), (70, (64, 64, 64, 64), 16384, False)])
+@pytest.mark.parametrize("how", ["static", "value"])
+def test_matmul_group_apart_where_members_are_split(orc, m, ns, k, apart, how):
+    """On the null stream; on another, where nothing is split, the one launch in any case: the same sums."""
+    import torch
+    rng = np.random.default_rng(m + k)
+    a = rng.integers(-128, 128, (m, k), dtype=np.int8)
+    dev, dynamic = torch.from_numpy(a).cuda(), how == "value"
+    args = dict(in_quant=K.QuantParam(0.03, -5)) if dynamic else {}
+    pairs = [_matmul_pair(rng, n, k, False, dynamic) for n in ns]
+    kernels = [pair[4](True) for pair in pairs]
+    group = lambda: K.dynmm_run_group(kernels, dev, **args) if dynamic else K.matmul_run_group(kernels, dev)
+    torch.cuda.synchronize()
+    so_far = _split_launches()[0]
+    other = torch.cuda.Stream()
+    with torch.cuda.stream(other):
+        want = group()
+    other.synchronize()
+    assert _split_launches()[0] == so_far
+    got = group()
+    torch.cuda.synchronize()
+    assert _split_launches()[0] == so_far + (len(ns) if apart else 0)
+    rows = np.unique(np.r_[0, 1, 31, 63:65, m // 2, m - 2, m - 1])
+    orc.set_threads(16)
+    for (w, bias, sw, zw, _), y, z in zip(pairs, got, want):
+        assert torch.equal(y.view(torch.int8), z.view(torch.int8))
+        if dynamic:
+            sure = orc.dynamic_matmul(a[rows], w, bias, 0.03, -5, sw, zw)
+        else:
+            sure = orc.matmul_int8(a[rows], w, bias, 0.02, 7, sw, zw, float(np.float32(0.02 * 0.0055 * k ** 0.5 * 140)), 3)
+        assert np.array_equal(y.cpu().numpy()[rows], sure)
+
+
 def test_matmul_with_k_in_parts_on_library_streams():
     """Two threads, each with a stream of the library and a handle of its own, beside the null stream."""
     import ctypes as C
