@@ -214,6 +214,26 @@ void *SplitMemory::make(hipStream_t stream) {
   });
 }
 
+// kSplitSpacesKept of them, their counters zero; null if there is no memory for them.  (Cleared on a stream of its own: work on the null
+// stream would end other threads' captures.)
+static void *kept_split_spaces() {
+  return beside_captures([] {
+    void *p = nullptr;
+    hipStream_t s = nullptr;
+    bool ok = hipStreamCreateWithFlags(&s, hipStreamNonBlocking) == hipSuccess &&
+              device_alloc(&p, kSplitSpacesKept * kSplitBytes) == hipSuccess &&
+              hipMemset2DAsync(p, kSplitBytes, 0, kSplitCounterBytes, kSplitSpacesKept, s) == hipSuccess &&
+              hipStreamSynchronize(s) == hipSuccess;
+    if (s != nullptr) ok = hipStreamDestroy(s) == hipSuccess && ok;
+    if (!ok) {
+      (void)hipGetLastError();
+      if (p != nullptr) (void)hipFree(p);
+      p = nullptr;
+    }
+    return p;
+  });
+}
+
 bool SplitMemory::free(void *p) {
   return beside_captures([&] {
     const bool gone = hipFree(p) == hipSuccess;
@@ -671,12 +691,8 @@ int mi_init(int device) {
     void *ptr = nullptr;
     MI_HIP_CHECK(hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)));  // this device's copy of the array
     g_scratch_ptr[device] = ptr;
-    ptr = nullptr;
-    if (device_alloc(&ptr, kSplitSpacesKept * kSplitBytes) != hipSuccess ||
-        hipMemset2D(ptr, kSplitBytes, 0, kSplitCounterBytes, kSplitSpacesKept) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
-      (void)hipGetLastError();  // (the null stream's GEMMs are not split then)
-      if (ptr != nullptr) (void)hipFree(ptr);
-    } else {
+    ptr = kept_split_spaces();
+    if (ptr != nullptr) {  // (otherwise the null stream's GEMMs are not split)
       g_split_ptr[device] = ptr;
       for (int i = 1; i < kSplitSpacesKept; ++i) split_spaces().keep(device, static_cast<char *>(ptr) + i * kSplitBytes);
     }

@@ -1,6 +1,9 @@
 """MatMuls whose K is split over workgroups on streams of mi_stream_create: the memory in which they hand over their sums comes
 and goes with the streams."""
 import ctypes as C
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -212,3 +215,45 @@ def test_captures_of_a_library_stream_are_not_split(matmul, run):
         assert all(torch.equal(out, want) for out in outs[1:])
     assert _splits(L) == split + 101
     _destroy(L, [stream])
+
+
+FIRST_USE = """
+import threading
+import torch
+from mindspore_amd import lib
+x = torch.zeros(1000, device="cuda")
+stream, graph, started = torch.cuda.Stream(), torch.cuda.CUDAGraph(), []
+torch.cuda.synchronize()
+
+def start():
+    L = lib.init()
+    started.append(L)
+    stream = lib.C.c_void_p(None)
+    assert L.mi_stream_create(lib.C.byref(stream)) == lib.MI_OK and L.mi_stream_destroy(stream) == lib.MI_OK
+
+with torch.cuda.graph(graph, stream=stream, capture_error_mode="%s"):
+    x.add_(1)
+    thread = threading.Thread(target=start)
+    thread.start()
+    thread.join()
+    x.add_(1)
+for i in range(3):
+    graph.replay()
+    torch.cuda.synchronize()
+    assert started and torch.equal(x, torch.full_like(x, 2 * i + 2))
+import numpy as np
+from mindspore_amd import kernels as K
+w = np.ones((1000, 4096), np.int8)
+kern = K.MatmulInt8Kernel(w, None, K.QuantParam(0.02, 0), [K.QuantParam(0.004, 0)], K.QuantParam(1.0, 0), True, 0)
+y = kern.run(torch.ones((150, 4096), dtype=torch.int8, device="cuda"))
+assert bool((y == 0).all()) and started[0].mi_debug_split_launches(None, None) == 1
+print("ok")
+"""
+
+
+@pytest.mark.parametrize("mode", ["global", "relaxed"])
+def test_the_first_use_of_the_library_beside_a_capture(mode):
+    """Another thread's capture survives mi_init and the life of a stream, and K is split afterwards."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    out = subprocess.run([sys.executable, "-c", FIRST_USE % mode], cwd=root, capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0 and out.stdout.endswith("ok\n"), out.stdout + out.stderr[-2000:]
