@@ -440,6 +440,9 @@ struct RequantState {
     put(at.pre, prev);
     put(at.rshift, e);
     put(at.zw, zwv);
+    put(at.mult(n_pad), h_mult);
+    put(at.bias2(n_pad), h_bias2);
+    put(at.lshift(n_pad), h_ls);
     int rc;
     if ((rc = upload(&channels, block)) != MI_OK) return rc;
     if (pack_weights) {

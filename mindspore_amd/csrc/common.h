@@ -75,8 +75,13 @@ struct RequantParams {
   int fast2;   // fast, and every mult >= 0, every c2 < 0, and K * 16384 + K * 128 * |zw| <= kAccBias (a in [0, 2^31))
 
   // The arrays stand one behind the other, of `stride` channels each.  (mult2 to zw are arrays of their own because a wave reads 32
-  // to 64 channels of them: with 16 bytes a channel the window convolutions took 5 % longer.)
-  static constexpr int kWordsPerChannel = 4 + 6;
+  // to 64 channels of them: with 16 bytes a channel the window convolutions took 5 % longer.)  Behind zw stand arrays of the records'
+  // mult, bias2 and lshift, for kernels whose threads read several neighbouring channels: 4 to 16 records a thread are as many
+  // scattered loads (conv_dw16_kernel has the figures).
+  static constexpr int kWordsPerChannel = 4 + 9;
+  __host__ __device__ __forceinline__ const int32_t *mult(int stride) const { return zw + stride; }
+  __host__ __device__ __forceinline__ const int32_t *bias2(int stride) const { return zw + 2 * (int64_t)stride; }
+  __host__ __device__ __forceinline__ const int32_t *lshift(int stride) const { return zw + 3 * (int64_t)stride; }
   __host__ __device__ __forceinline__ void set_channels(const RequantChannel *block, int stride) {
     each = block;
     mult2 = reinterpret_cast<const uint32_t *>(block + stride);

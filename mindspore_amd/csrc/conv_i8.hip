@@ -137,20 +137,17 @@ __global__ __launch_bounds__(256) void conv_smallk_kernel(const int8_t *__restri
   // block's before the gather, so that they arrive behind it.  Fetched where they are used, one group of four
   // channels after the other and behind the branches of the previous group's arithmetic, they were four round trips
   // in a row at the end of a 32-channel stem.
+  const int n_pad = padded_channels(g.out_c);
   v4i prm[4][5];
   auto fetch_params = [&](int ob) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int nb = ob * 32 + q * 8 + h * 4;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const RequantChannel ch = rq.each[nb + e];
-        prm[q][0][e] = ch.mult;
-        prm[q][1][e] = ch.bias2;
-        prm[q][2][e] = ch.rshift();
-        prm[q][3][e] = ch.zw;
-        prm[q][4][e] = ch.lshift();
-      }
+      prm[q][0] = *reinterpret_cast<const v4i *>(rq.mult(n_pad) + nb);
+      prm[q][1] = *reinterpret_cast<const v4i *>(rq.bias2(n_pad) + nb);
+      prm[q][2] = *reinterpret_cast<const v4i *>(rq.rshift + nb);
+      prm[q][3] = *reinterpret_cast<const v4i *>(rq.zw + nb);
+      prm[q][4] = *reinterpret_cast<const v4i *>(rq.lshift(n_pad) + nb);
     }
   };
   fetch_params(0);
@@ -834,7 +831,7 @@ __global__ __launch_bounds__(256) void conv_dw_kernel(const int8_t *__restrict__
                                                       const int16_t *__restrict__ w16,
                                                       const int32_t *__restrict__ bias, int zx8, RequantParams rq,
                                                       int8_t *__restrict__ out) {
-  const int ch = g.out_c;
+  const int ch = g.out_c, n_pad = padded_channels(ch);
   const int64_t total = (int64_t)g.batch * g.out_h * g.out_w * ch;
   for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
        idx += (int64_t)gridDim.x * blockDim.x) {
@@ -856,8 +853,7 @@ __global__ __launch_bounds__(256) void conv_dw_kernel(const int8_t *__restrict__
         acc += (uint32_t)((int32_t)xv * (int32_t)wv);
       }
     }
-    const RequantChannel ch = rq.each[c];
-    const int32_t mult = ch.mult, e = ch.rshift(), ls = ch.lshift();
+    const int32_t mult = rq.mult(n_pad)[c], e = rq.rshift[c], ls = rq.lshift(n_pad)[c];
     int32_t y = rdiv_pot(srdhm((int32_t)(acc << ls), mult), e);
     y = (int32_t)((uint32_t)y + (uint32_t)rq.zo);
     y = y > rq.amin ? y : rq.amin;  // MSMAX first, then MSMIN (conv_depthwise_int8.c:49-50)
@@ -873,6 +869,10 @@ __global__ __launch_bounds__(256) void conv_dw_kernel(const int8_t *__restrict__
 // inner product is sum_t x_t * w_t with no subtraction.  TAPS > 0 (kernel_h * kernel_w known at compile time): the
 // loads of all taps are issued before the first multiply.  TAPS == 0: any kernel size, five taps per batch of loads.  FAST: the host
 // proved the cheap rounding form exact for every channel (no left shifts to fetch).
+// A thread reads the parameters of its CG channels from arrays, four channels a load: with RequantChannel, a load of 16 bytes per
+// channel, every channel of a wave's lines was fetched on its own.  us, records -> arrays: 3x3 at stride 2, 4 x 151 x 151 x 96
+// 14.1 -> 8.15, 16 x 135 x 135 x 128 30.6 -> 20.7; 32 x 50 x 50 x 72 with left shifts 29.7 -> 14.2; 7x7, 16 x 39 x 39 x 960 197 -> 140,
+// 1 x 30 x 30 x 72 12.9 -> 11.4.
 template <int TAPS, int CG, bool FAST>
 __global__ __launch_bounds__(256) void conv_dw16_kernel(const int8_t *__restrict__ in, ConvGeom g,
                                                         const int16_t *__restrict__ w16,
@@ -881,7 +881,7 @@ __global__ __launch_bounds__(256) void conv_dw16_kernel(const int8_t *__restrict
   static_assert(CG == 8 || CG == 16, "channels per thread");
   constexpr int XW = CG / 4;  // dwords of activations per tap
   constexpr int WQ = CG / 8;  // 16-byte vectors of int16 weights per tap
-  const int ch = g.out_c, groups = ch / CG;
+  const int ch = g.out_c, groups = ch / CG, n_pad = padded_channels(ch);
   const int64_t total = (int64_t)g.batch * g.out_h * g.out_w * groups;
   const int zsplat = (zx8 & 0xff) * 0x01010101;
   union XV {
@@ -989,17 +989,17 @@ __global__ __launch_bounds__(256) void conv_dw16_kernel(const int8_t *__restrict
     } o;
 #pragma unroll
     for (int q = 0; q < CG / 4; ++q) {
-      RequantChannel of[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) of[e] = rq.each[c0 + 4 * q + e];
+      const v4i m4 = *reinterpret_cast<const v4i *>(rq.mult(n_pad) + c0 + 4 * q);
+      const v4i rs4 = *reinterpret_cast<const v4i *>(rq.rshift + c0 + 4 * q);
+      v4i ls4 = {0, 0, 0, 0};
+      if (!FAST) ls4 = *reinterpret_cast<const v4i *>(rq.lshift(n_pad) + c0 + 4 * q);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int32_t mult = of[e].mult, shift = of[e].rshift();
         int32_t y;
         if (FAST) {
-          y = rdiv_pot_fast(srdhm_nosat((int32_t)acc[4 * q + e], mult), shift, (1 << shift) >> 1);
+          y = rdiv_pot_fast(srdhm_nosat((int32_t)acc[4 * q + e], m4[e]), rs4[e], (1 << rs4[e]) >> 1);
         } else {
-          y = rdiv_pot(srdhm((int32_t)(acc[4 * q + e] << of[e].lshift()), mult), shift);
+          y = rdiv_pot(srdhm((int32_t)(acc[4 * q + e] << ls4[e]), m4[e]), rs4[e]);
         }
         y = (int32_t)((uint32_t)y + (uint32_t)rq.zo);
         y = y > rq.amin ? y : rq.amin;  // MSMAX first, then MSMIN (conv_depthwise_int8.c:49-50)

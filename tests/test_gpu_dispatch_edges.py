@@ -1003,3 +1003,36 @@ def test_dynamic_quant_values_out_of_line(orc, bits, symmetric):
         got = params.cpu().numpy().view([("scale", "f8"), ("scale_f", "f4"), ("zp", "i4"), ("lo", "f4"), ("hi", "f4")])
         assert np.array_equal(q.cpu().numpy(), want), (rows, unit, special)
         assert np.array_equal(got["scale"].reshape(-1), scales.reshape(-1), equal_nan=True) and np.array_equal(got["zp"].reshape(-1), zps.reshape(-1))
+
+
+# channels that end inside and just past the parameters' padding, 8 and 16 of them a thread and one; left shifts (sums of a few units) and none
+@pytest.mark.parametrize("left_shifts", [False, True])
+@pytest.mark.parametrize("ch", [5, 8, 256, 264, 1008])
+@pytest.mark.parametrize("taps,stride,dil", [(3, 2, 1), (5, 2, 1), (7, 1, 1), (3, 1, 2)])
+def test_depthwise_parameters_of_many_channels(orc, taps, stride, dil, ch, left_shifts):
+    from tests.test_gpu_parity import _conv_case, _gpu_conv
+    rng = np.random.default_rng(ch * taps + left_shifts)
+    strides, dils, pad = (stride, stride), (dil, dil), (taps // 2,) * 4
+    case = _conv_case(rng, 2, 9, 8, ch, ch, (taps, taps), strides, dils, pad, True, False, not left_shifts, 0, dw=True)
+    if left_shifts:
+        case["x"] = (case["zx"] + rng.integers(-1, 2, case["x"].shape)).astype(np.int8)
+        case["w"] = rng.integers(-3, 4, case["w"].shape, dtype=np.int8)
+        case["so"] = float(case["sx"] * case["sw"].mean() / 2)
+    got = _gpu_conv(case, strides, dils, pad, ch, device_tensors=True)
+    assert np.array_equal(got, orc.conv_dw_int8(**case))
+
+
+# as above, where a lane reads four channels at a time of all parameters
+@pytest.mark.parametrize("left_shifts", [False, True])
+@pytest.mark.parametrize("oc", [4, 28, 32, 36, 128])
+def test_short_convolution_parameters(orc, oc, left_shifts):
+    from tests.test_gpu_parity import _conv_case, _gpu_conv
+    rng = np.random.default_rng(oc + left_shifts)
+    pad, dil = (1, 1, 2, 2), (1, 2)
+    case = _conv_case(rng, 2, 12, 13, 3, oc, (3, 3), (1, 1), dil, pad, True, True, not left_shifts, 0)
+    if left_shifts:
+        case["x"] = (case["zx"] + rng.integers(-1, 2, case["x"].shape)).astype(np.int8)
+        case["w"] = rng.integers(-3, 4, case["w"].shape, dtype=np.int8)
+        case["zw"] = rng.integers(-1, 2, case["zw"].shape).astype(np.int32)
+        case["so"] = float(case["sx"] * case["sw"].mean() / 2)
+    assert np.array_equal(_gpu_conv(case, (1, 1), dil, pad, 1, device_tensors=True), orc.conv_int8(**case))
