@@ -85,18 +85,30 @@ __device__ __forceinline__ void hint_interleave_reads() {
 // CONV: the activation operand is not a matrix in memory but the im2col view of an NHWC image (in_c % 16 == 0): row m
 // is output pixel m, and the 16-byte chunk at K offset k is 16 channels of tap k / in_c, fetched straight from the
 // image, or from 16 bytes of the fill value when the tap lies outside the image (conv_int8.c:758-807,877).
-struct ConvGather {
+template <typename Small>  // of strides, dilations and pads
+struct ConvGatherOf {
   int in_h, in_w, in_c, out_w, out_hw;
   uint32_t magic_ic, magic_kw;  // ceil(2^32 / in_c), ceil(2^32 / kernel_w): exact quotients for dividends < 2^16
-  int16_t stride_h, stride_w, dil_h, dil_w, pad_u, pad_l;
+  Small stride_h, stride_w, dil_h, dil_w, pad_u, pad_l;
   int kernel_w;
 };
+typedef ConvGatherOf<int16_t> ConvGatherArgs;  // as it travels
+typedef ConvGatherOf<int> ConvGather;
+__device__ __forceinline__ ConvGather open(const ConvGatherArgs &c) {
+  ConvGather cv{c.in_h, c.in_w, c.in_c, c.out_w, c.out_hw, c.magic_ic, c.magic_kw, c.stride_h, c.stride_w, c.dil_h, c.dil_w,
+                c.pad_u, c.pad_l, c.kernel_w};
+  // (in registers for good: left to itself the compiler takes the main loop's out of their shared word in every K step.  us at long K:
+  // 1 x 27 x 27, 256 -> 256, 5x5 at stride 2 21.2 -> 20.8, with left shifts 22.2 -> 21.4; 16 x 14 x 14, 256 -> 512, 3x3 at stride 2, with
+  // left shifts 10.25 -> 10.0)
+  asm volatile("" : "+s"(cv.dil_h), "+s"(cv.dil_w));
+  return cv;
+}
 // As GemmCall, of a convolution whose output pixels are the rows.
 struct ConvCall {
   const int8_t *in, *w, *fill16;
   int8_t *c;
   int m, n, k;
-  ConvGather cv;
+  ConvGatherArgs cv;
   RequantCall epi;
 };
 static_assert(sizeof(ConvCall) <= kShortArgs, "see launch_args.h");
@@ -323,7 +335,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
   const int k_pad = padded_k(call.k);
   const GemmArgs g{call.in, 0, call.m, call.k, call.w, weight_row_stride(k_pad), k_pad, nullptr, call.n,
                    (call.m + TILE_M - 1) / TILE_M, (call.n + TILE_N - 1) / TILE_N, call.c, call.n, 0, 0};
-  gemm_direct_body<TILE_N, TILE_M, EPI_REQUANT, HAS_ZW, FAST, NST, true>(g, call.epi.open(call.n), DequantParams{}, call.cv,
+  gemm_direct_body<TILE_N, TILE_M, EPI_REQUANT, HAS_ZW, FAST, NST, true>(g, call.epi.open(call.n), DequantParams{}, open(call.cv),
                                                                          call.fill16);
 }
 
@@ -592,9 +604,9 @@ int launch_gemm_conv_requant(const int8_t *in, const ConvGeom &cg, const int8_t 
   }
   const auto magic = [](int d) { return d <= 1 ? 0u : (uint32_t)((((uint64_t)1 << 32) + d - 1) / (uint64_t)d); };
   const ConvCall call{in, w.w, fill16, out, (int)m64, cg.out_c, (int)k64,
-                      ConvGather{cg.in_h, cg.in_w, cg.in_c, cg.out_w, cg.out_h * cg.out_w, magic(cg.in_c), magic(cg.kernel_w),
-                                 (int16_t)cg.stride_h, (int16_t)cg.stride_w, (int16_t)cg.dilation_h, (int16_t)cg.dilation_w,
-                                 (int16_t)cg.pad_u, (int16_t)cg.pad_l, cg.kernel_w},
+                      ConvGatherArgs{cg.in_h, cg.in_w, cg.in_c, cg.out_w, cg.out_h * cg.out_w, magic(cg.in_c), magic(cg.kernel_w),
+                                     (int16_t)cg.stride_h, (int16_t)cg.stride_w, (int16_t)cg.dilation_h, (int16_t)cg.dilation_w,
+                                     (int16_t)cg.pad_u, (int16_t)cg.pad_l, cg.kernel_w},
                       RequantCall::of(rq)};
   if (rq.has_zw) {
     return rq.fast2 ? launch_conv_pick_tile<true, true>(call, stream) : launch_conv_pick_tile<true, false>(call, stream);
