@@ -4,7 +4,8 @@
 // costs the host 2.85 us, from 128 bytes on 3.55 (empty kernels, 16 to 768 bytes; where the bus is near 2.5 throughout).  A kernel
 // that reads gridDim takes 72 bytes of hidden arguments more: with it the step is behind 40 bytes.  Launches of a few
 // microseconds run at the host's pace, so their kernels get at most kShortArgs bytes, know their grid from their own sizes, and
-// make the wider structures that the bodies work on from what they are given, in scalar registers.
+// make the wider structures that the bodies work on from what they are given, in scalar registers.  (All but the groups of GEMMs and of
+// more than two decode MatMuls, conv_window_kernel, the depthwise kernels other than conv_dw_rows_kernel, conv_smallk_kernel and im2col.)
 // (Calls through Python, 240 to 256 bytes and hidden ones -> 64 to 112: FullConnection 128 x 768 x 768 4.55 -> 4.2 us, of which its
 // kernel takes 3.9; the four convolutions of an image block 18.5 -> 16.5, their kernels 13.6.)
 #pragma once
