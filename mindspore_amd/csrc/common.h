@@ -135,7 +135,9 @@ struct WeightView {
   // when the handle is created (launch_block_weights).
   const int8_t *blocked;
 };
-__host__ __device__ inline int weight_row_stride(int k_pad) { return (k_pad / 256) % 2 == 0 ? k_pad + 256 : k_pad; }
+// (An odd multiple of 256.  Without a selection: its result is no longer scalar to the compiler, and the K-block loop on row-major
+// weights, whose descriptor has the stride in it, then went round a loop over the lanes' descriptors for each of its loads.)
+__host__ __device__ inline int weight_row_stride(int k_pad) { return k_pad | 256; }
 
 // Device memory through which the workgroups of a split GEMM (gemm_split.hip) hand over their sums: counters, which are zero
 // between launches, and the sums.  Null: the GEMM is not split.  Launches on one stream follow one another and share it; so there
