@@ -9,7 +9,7 @@ LIB = os.path.join(HERE, "libmi355x_int8.so")
 DIAG_LIB = os.path.join(HERE, "libmi355x_diag.so")  # the benchmark's measurement aids, not part of the product
 DEVICE_CALLS = os.path.join(HERE, "_device_calls.so")  # kernels.py's calls on torch device tensors
 NATIVE_BENCH = os.path.join(HERE, "native_bench")
-SOURCES = ["capi.hip", "gemm_i8.hip", "gemm_kblock.hip", "gemm_ring.hip", "gemm_split.hip", "gemm_anyrow.hip", "gemv_i8.hip", "conv_i8.hip", "conv_thin.hip", "conv_window.hip", "dynquant.hip", "host_copy.hip", "infer_shape.hip"]
+SOURCES = ["capi.hip", "gemm_i8.hip", "gemm_kblock.hip", "gemm_ring.hip", "gemm_split.hip", "gemm_anyrow.hip", "gemm_short.hip", "gemv_i8.hip", "conv_i8.hip", "conv_thin.hip", "conv_window.hip", "dynquant.hip", "host_copy.hip", "infer_shape.hip"]
 # -ffp-contract=off: the float steps of DynamicQuant / dynamic MatMul and the host-side multiplier derivation are
 # separately rounded operations in the reference and must not be fused.
 FLAGS = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-ffp-contract=off", "-fno-fast-math",

@@ -566,7 +566,8 @@ static int run_requant_gemm(const RequantState &st, const int8_t *a, int64_t lda
                             hipStream_t stream) {
   const RequantParams rq = st.params();
   const WeightView w = weight_view(st);
-  if (runs_on_gemv(st, rows, k16)) return launch_gemv_requant(a, lda, rows, k16, w, st.n, rq, c, st.n, stream);
+  if (runs_on_gemv(st, rows, k16) && !gemm_short_takes(rows, k16, w, st.n, rq))
+    return launch_gemv_requant(a, lda, rows, k16, w, st.n, rq, c, st.n, stream);
   return launch_gemm_requant(a, lda, rows, k16, w, st.n, rq, c, st.n, stream);
 }
 
@@ -574,13 +575,14 @@ static int run_requant_gemm(const RequantState &st, const int8_t *a, int64_t lda
 static bool reads_any_rows(const RequantState &st, const int8_t *a_dev, int rows) {
   const WeightView w = weight_view(st);
   if (runs_on_gemv(st, rows, round_up(st.k, 16))) return gemv_takes_any_rows(rows, st.k, w, st.n);
-  return !whole_chunks(a_dev, st.k) && gemm_anyrow_takes(rows, st.k, w, st.n);
+  return !whole_chunks(a_dev, st.k) && gemm_anyrow_takes(rows, st.k, w, st.n, st.params());
 }
 
 static int run_requant_any_rows(const RequantState &st, const int8_t *a_dev, int rows, int8_t *c, hipStream_t stream) {
   const RequantParams rq = st.params();
   const WeightView w = weight_view(st);
-  if (runs_on_gemv(st, rows, round_up(st.k, 16))) return launch_gemv_requant(a_dev, st.k, rows, st.k, w, st.n, rq, c, st.n, stream);
+  if (runs_on_gemv(st, rows, round_up(st.k, 16)) && !gemm_short_takes(rows, st.k, w, st.n, rq))
+    return launch_gemv_requant(a_dev, st.k, rows, st.k, w, st.n, rq, c, st.n, stream);
   return launch_gemm_anyrow_requant(a_dev, rows, st.k, w, st.n, rq, c, stream);
 }
 
@@ -1655,22 +1657,24 @@ static bool runs_on_gemv(const mi_dynmm *h, int rows) {
 }
 
 // as for mi_matmul
-static bool reads_any_rows(const mi_dynmm *h, const int8_t *a_dev, int rows) {
+static bool reads_any_rows(const mi_dynmm *h, const int8_t *a_dev, int rows, const DequantParams &dq) {
   const WeightView w = weight_view(h);
   if (runs_on_gemv(h, rows)) return gemv_takes_any_rows(rows, h->k, w, h->n);
-  return !whole_chunks(a_dev, h->k) && gemm_anyrow_takes(rows, h->k, w, h->n);
+  return !whole_chunks(a_dev, h->k) && gemm_anyrow_takes(rows, h->k, w, h->n, dq);
 }
 
 static int run_dequant_any_rows(const mi_dynmm *h, const int8_t *a_dev, int rows, const DequantParams &dq, float *c_dev, hipStream_t s) {
   const WeightView w = weight_view(h);
-  if (runs_on_gemv(h, rows)) return launch_gemv_dequant(a_dev, h->k, rows, h->k, w, h->n, dq, c_dev, h->n, s);
+  if (runs_on_gemv(h, rows) && !gemm_short_takes(rows, h->k, w, h->n, dq))
+    return launch_gemv_dequant(a_dev, h->k, rows, h->k, w, h->n, dq, c_dev, h->n, s);
   return launch_gemm_anyrow_dequant(a_dev, rows, h->k, w, h->n, dq, c_dev, s);
 }
 
 static int run_dequant_gemm(const mi_dynmm *h, const int8_t *a, int64_t lda, int rows, int k16, const DequantParams &dq, float *c_dev,
                             hipStream_t s) {
   const WeightView w = weight_view(h);
-  if (runs_on_gemv(h, rows)) return launch_gemv_dequant(a, lda, rows, k16, w, h->n, dq, c_dev, h->n, s);
+  if (runs_on_gemv(h, rows) && !gemm_short_takes(rows, k16, w, h->n, dq))
+    return launch_gemv_dequant(a, lda, rows, k16, w, h->n, dq, c_dev, h->n, s);
   return launch_gemm_dequant(a, lda, rows, k16, w, h->n, dq, c_dev, h->n, s);
 }
 
@@ -1685,7 +1689,7 @@ static int dynmm_run_impl(mi_dynmm *h, const int8_t *a_dev, int32_t rows, float 
   int rc = ensure_device();
   if (rc != MI_OK) return rc;
   const DequantParams dq = dequant_params(h, sx, zx, qp_dev, per_row);
-  if (reads_any_rows(h, a_dev, rows)) return run_dequant_any_rows(h, a_dev, rows, dq, c_dev, s);
+  if (reads_any_rows(h, a_dev, rows, dq)) return run_dequant_any_rows(h, a_dev, rows, dq, c_dev, s);
   const int8_t *a = nullptr;
   int64_t lda = 0;
   int k16 = 0;
@@ -1782,7 +1786,7 @@ int mi_dynmm_run_group(mi_dynmm *const *handles, int32_t count, const int8_t *a_
   for (int i = 0; i < count; ++i) {
     const mi_dynmm *h = handles[i];
     const DequantParams dq = dequant_params(h, (float)in_scale, in_zp, params_dev, per_row != 0);
-    if (!shares_padded_copy(count, runs_on_gemv(h, rows)) && reads_any_rows(h, a_dev, rows)) {
+    if (!shares_padded_copy(count, runs_on_gemv(h, rows)) && reads_any_rows(h, a_dev, rows, dq)) {
       rc = run_dequant_any_rows(h, a_dev, rows, dq, c_dev[i], s);
     } else if ((rc = prepare()) == MI_OK) {
       rc = run_dequant_gemm(h, a, lda, rows, k16, dq, c_dev[i], s);

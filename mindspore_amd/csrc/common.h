@@ -161,11 +161,17 @@ int launch_gemm_dequant(const int8_t *a, int64_t lda, int m, int k, const Weight
                         const DequantParams &dq, float *c, int64_t ldc, hipStream_t stream);
 
 // The same for activation rows of any length at any address, [m][k] without gaps, where that is quicker than a padded copy.
-bool gemm_anyrow_takes(int m, int k, const WeightView &w, int n);
+bool gemm_anyrow_takes(int m, int k, const WeightView &w, int n, const RequantParams &rq);
+bool gemm_anyrow_takes(int m, int k, const WeightView &w, int n, const DequantParams &dq);
 int launch_gemm_anyrow_requant(const int8_t *a, int m, int k, const WeightView &w, int n, const RequantParams &rq, int8_t *c,
                                hipStream_t stream);
 int launch_gemm_anyrow_dequant(const int8_t *a, int m, int k, const WeightView &w, int n, const DequantParams &dq, float *c,
                                hipStream_t stream);
+
+// Whether the launches above take m rows on the small tiles of gemm_short.hip, also where the decode kernels could: rows of any length and
+// address by the last two, whole aligned chunks by the first two as well.
+bool gemm_short_takes(int m, int k, const WeightView &w, int n, const RequantParams &rq);
+bool gemm_short_takes(int m, int k, const WeightView &w, int n, const DequantParams &dq);
 
 // Up to four weight matrices with the same K against the same activation rows as one launch; member i writes c[i] with row
 // stride n[i].  gemm_group_tile: what the launch would run on, or null where the members are to be run one by one; lda: of the

@@ -19,8 +19,9 @@
 //     large shapes, 128 x 128 tiles, two per CU, where fp32 stores have to overlap another tile's loop;
 //   * gemm_ring.hip: a ring of stages that hold both operands, as deep as the LDS allows: every smaller tile;
 //   * gemm_split.hip: the same with the K of a tile in parts, a workgroup each, where the tiles leave CUs idle;
+//   * gemm_short.hip: 32 x 32 and 64 x 32 tiles whose K the waves share, where those fit the device about once;
 //   * gemm_anyrow.hip: 64 x 64 tiles for activation rows that are no whole 16-byte chunks, where padding them first would cost
-//     more than the product;
+//     more than the product (gemm_short.hip takes such rows too);
 //   * gemm_direct_body below, K steps of 64 bytes through NST LDS stages over row-major weights: short K, handles
 //     without the blocked copy (whose large shapes run on gemm_kblock.hip's row-major form) and the convolution whose
 //     activation operand is gathered from the image.
@@ -416,6 +417,37 @@ static const SplitCost *choose_split(int m, int k, int n, const TileCost &whole,
   if (best != nullptr) *split_cost = least;
   return best;
 }
+// The tile of gemm_short.hip that is quicker than what else there is, or 0; and what it is expected to take (us, fitted like kTileCosts).
+// One 32 x 32 tile a CU, of four waves up to 12 K blocks and of eight beyond, or, from 7 blocks on, one of 64 channels x 32 rows: the
+// second workgroup of a CU competes for the operands' way into it, about 100 GB/s.  With fewer blocks the launch is most of the time, and
+// several tiles a CU still pay, with fp32 output, whose stores they spread, more of them.  us per launch, the quickest otherwise / this:
+// 33 x 1024 x 4096 7.05 / 5.2, 65 x 3072 x 1024 (288 tiles of 32 x 32, 144 of 64 x 32) 4.65 / 4.20, 128 x 4096 x 4096 (256 of 64 x 32) 9.9 / 8.9,
+// 1000 x 500 x 256 3.69 / 3.45 (512), 700 x 1024 x 512 (fp32) 4.8 / 4.24 (704); not taken: 160 x 3072 x 768 4.20 / 4.34 (480), 333 x 1536 x 512
+// 3.97 / 4.06 (528), 512 x 768 x 128 3.17 / 3.38, 200 x 3072 x 1024 4.47 / 5.24 (336 of 64 x 32: 6.7), 200 x 4096 x 4096 10.1 / 14.6 (448 of 64 x 32),
+// 65 x 4096 x 11008 18.5 / 18.8, and up to 32 rows, which the decode kernels read long K for with 16 channels a workgroup, 8 x 768 x 3072
+// 3.62 / 4.51, 32 x 4096 x 4096 6.7 / 7.6 (16 x 768 x 768 4.02 / 3.38).
+struct ShortTile {
+  int tile;  // as launch_gemm_short has it
+  float cost;
+};
+static ShortTile short_tile(int m, int k, int n, bool requant) {
+  const int kb = (k + 127) / 128;
+  const int64_t rows = (m + 31) / 32, small = rows * ((n + 31) / 32), wide = rows * ((n + 63) / 64);
+  if (kb < 2 || m <= kGemvDotRows) return {0, 0};
+  const auto cost = [kb](int waves, int64_t tiles, float a, float pass, float block, float tile) {
+    const float a_cu = (float)tiles / 256.0f;
+    return a + pass * (float)((kb + 2 * waves - 1) / (2 * waves)) + a_cu * (block * (float)kb + tile);
+  };
+  const auto four = [&] { return ShortTile{41, cost(4, small, 2.55f, 0.54f, 0.06f, 0.22f)}; };
+  if (m <= kGemvGroupMaxRows) return kb <= 12 && small <= 128 ? four() : ShortTile{0, 0};
+  if (small <= 256) return kb <= 12 ? four() : ShortTile{81, cost(8, small, 2.3f, 0.93f, 0.053f, 0.55f)};
+  if (kb < 7) return small <= (!requant ? 768 : kb == 2 ? 256 : kb < 6 ? 512 : 448) ? four() : ShortTile{0, 0};
+  return wide <= 256 && kb <= 64 ? ShortTile{82, cost(8, wide, 1.9f, 1.65f, 0.073f, 1.03f)} : ShortTile{0, 0};
+}
+// From K = 4096 on, more rows than the decode kernels take stay with K in parts (gemm_split.hip) on the streams that have memory for
+// that: its tests hold it to them.  150 x 1000 x 4096 7.7 us in parts, 5.3 here.
+static bool short_goes_first(int m, int k) { return m <= kGemvMaxRows || k < 4096; }
+
 // (the K-block loaders address activation rows with 32-bit offsets from the tile's first row)
 static bool kblock_takes(int k, int64_t lda) { return k >= 128 && lda < (1 << 23); }
 
@@ -433,6 +465,9 @@ static int launch_pick_tile(const GemmArgs &g, const RequantParams &rq, const De
   // With fp32 output and a short K two workgroups per CU overlap one's stores with the other's loop: 4096 x 768 x 768 7.6
   // against 7.9 us.
   if (g.wb != nullptr && kblock_ok && (g.k >= 1024 || tiles_m <= 256)) {
+    const bool short_form = EPI == EPI_REQUANT ? FAST : !FAST;
+    const int in_short = short_form ? short_tile(g.m, g.k, g.n, EPI == EPI_REQUANT).tile : 0;
+    if (in_short != 0 && short_goes_first(g.m, g.k)) return launch_gemm_short(in_short, false, EPI == EPI_REQUANT, HAS_ZW, g, rq, dq, stream);
     if (EPI == EPI_DEQUANT && g.k < 1024 && tiles_m >= 128) return launch_gemm_kblock(22, false, HAS_ZW, FAST, g, rq, dq, stream);
     float cost;
     const TileCost &t = cheapest_tile(g.m, g.k, 1, &g.n, &cost);
@@ -443,6 +478,7 @@ static int launch_pick_tile(const GemmArgs &g, const RequantParams &rq, const De
       if (space != nullptr)
         return launch_gemm_split(10 * split->tn + split->tm, parts, EPI == EPI_REQUANT, HAS_ZW, FAST, g, rq, dq, space, stream);
     }
+    if (in_short != 0) return launch_gemm_short(in_short, false, EPI == EPI_REQUANT, HAS_ZW, g, rq, dq, stream);
     return t.ring ? launch_gemm_ring(10 * t.tn + t.tm, EPI == EPI_REQUANT, HAS_ZW, FAST, g, rq, dq, stream)
                   : launch_gemm_kblock(10 * t.tn + t.tm, EPI == EPI_REQUANT, HAS_ZW, FAST, g, rq, dq, stream);
   }
@@ -637,38 +673,58 @@ int launch_gemm_dequant(const int8_t *a, int64_t lda, int m, int k, const Weight
 // 500 x 2000 x 3001 12.3 / 14.2; less than a block of 128: 65 x 120 x 64 6.4 / 3.9, 1000 x 65 x 1001 6.6 / 4.3, 200 x 17 x 4096
 // 6.3 / 4.1, 8000 x 100 x 64 7.0 / 4.2.
 constexpr int kAnyrowLeastK = 16, kAnyrowMostK = 1536;
-bool gemm_anyrow_takes(int m, int k, const WeightView &w, int n) {
-  if (w.blocked == nullptr || k < kAnyrowLeastK || k > kAnyrowMostK) return false;
+static bool anyrow_tiles(int m, int k, int n) {
+  if (k < kAnyrowLeastK || k > kAnyrowMostK) return false;
   float cost;
   const TileCost &t = cheapest_tile(m, k, 1, &n, &cost);
   return t.ring && t.tn == 1 && t.tm == 1;
 }
+static int short_any(int m, int k, int n, bool requant, bool short_form) {
+  return short_form && k < (1 << 23) && short_goes_first(m, k) ? short_tile(m, k, n, requant).tile : 0;
+}
+static bool takes_any(int m, int k, const WeightView &w, int n, bool requant, bool short_form) {
+  return w.blocked != nullptr && (anyrow_tiles(m, k, n) || short_any(m, k, n, requant, short_form) != 0);
+}
+static bool short_form(const RequantParams &rq, int, int) { return rq.fast2 != 0; }
+static bool short_form(const DequantParams &, int m, int n) { return !stream_out_hint(m, n); }
 
-static int anyrow_args(const int8_t *a, int m, int k, const WeightView &w, int n, void *c, GemmArgs *g) {
+bool gemm_anyrow_takes(int m, int k, const WeightView &w, int n, const RequantParams &rq) {
+  return takes_any(m, k, w, n, true, short_form(rq, m, n));
+}
+bool gemm_anyrow_takes(int m, int k, const WeightView &w, int n, const DequantParams &dq) {
+  return takes_any(m, k, w, n, false, short_form(dq, m, n));
+}
+bool gemm_short_takes(int m, int k, const WeightView &w, int n, const RequantParams &rq) {
+  return w.blocked != nullptr && short_any(m, k, n, true, short_form(rq, m, n)) != 0;
+}
+bool gemm_short_takes(int m, int k, const WeightView &w, int n, const DequantParams &dq) {
+  return w.blocked != nullptr && short_any(m, k, n, false, short_form(dq, m, n)) != 0;
+}
+
+static int launch_any_rows(bool requant, bool short_form, const int8_t *a, int m, int k, const WeightView &w, int n, const RequantParams &rq,
+                           const DequantParams &dq, void *c, hipStream_t stream) {
   if (a == nullptr || c == nullptr) {
     set_error("gemm: null pointer");
     return MI_NULL_PTR;
   }
-  if (m <= 0 || n <= 0 || !gemm_anyrow_takes(m, k, w, n) || w.k_pad != round_up(k, kKPad)) {
+  if (m <= 0 || n <= 0 || !takes_any(m, k, w, n, requant, short_form) || w.k_pad != round_up(k, kKPad)) {
     set_error("gemm: unsupported operand geometry m=%d n=%d k=%d k_pad=%d", m, n, k, w.k_pad);
     return MI_PARAM_INVALID;
   }
-  *g = GemmArgs{a, k, m, k, nullptr, 0, w.k_pad, w.blocked, n, 0, 0, c, n};
-  return MI_OK;
+  const GemmArgs g{a, k, m, k, nullptr, 0, w.k_pad, w.blocked, n, 0, 0, c, n};
+  const bool has_zw = requant ? rq.has_zw != 0 : dq.zw0 != 0, any = (k & 15) != 0 || (reinterpret_cast<uintptr_t>(a) & 15) != 0;
+  if (const int tile = short_any(m, k, n, requant, short_form)) return launch_gemm_short(tile, any, requant, has_zw, g, rq, dq, stream);
+  return launch_gemm_anyrow(requant, has_zw, rq.fast2 != 0, g, rq, dq, stream);
 }
 
 int launch_gemm_anyrow_requant(const int8_t *a, int m, int k, const WeightView &w, int n, const RequantParams &rq, int8_t *c,
                                hipStream_t stream) {
-  GemmArgs g;
-  const int rc = anyrow_args(a, m, k, w, n, c, &g);
-  return rc != MI_OK ? rc : launch_gemm_anyrow(true, rq.has_zw != 0, rq.fast2 != 0, g, rq, DequantParams{}, stream);
+  return launch_any_rows(true, short_form(rq, m, n), a, m, k, w, n, rq, DequantParams{}, c, stream);
 }
 
 int launch_gemm_anyrow_dequant(const int8_t *a, int m, int k, const WeightView &w, int n, const DequantParams &dq, float *c,
                                hipStream_t stream) {
-  GemmArgs g;
-  const int rc = anyrow_args(a, m, k, w, n, c, &g);
-  return rc != MI_OK ? rc : launch_gemm_anyrow(false, dq.zw0 != 0, false, g, RequantParams{}, dq, stream);
+  return launch_any_rows(false, short_form(dq, m, n), a, m, k, w, n, RequantParams{}, dq, c, stream);
 }
 
 // Several matrices against the same rows as one launch, where that is expected to take less than a launch each: a
@@ -682,37 +738,43 @@ int launch_gemm_anyrow_dequant(const int8_t *a, int m, int k, const WeightView &
 // together: 128 x 512 x 7168 17.1 / 18.2, 100 x 1024 x 8192 16.95 / 18.2, 128 x 768 x 8192 19.15 / 18.65, 70 x 64 x 5120 13.45 / 14.3,
 // 200 x 512 x 11008 19.55 / 21.0, 500 x 256 x 12288 20.0 / 21.4, three of 100 x 256 x 11008 26.3 / 26.3, four of 70 x 64 x 16384
 // 35.95 / 36.3.
-static const TileCost *group_tile(int64_t lda, int m, int k, int count, const WeightView *w, const int *n, hipStream_t stream) {
+static const TileCost *group_tile(int64_t lda, int m, int k, int count, const WeightView *w, const int *n, bool requant, hipStream_t stream) {
   if (count < 2 || count > kGemmGroupMax || k < 1024 || !kblock_takes(k, lda)) return nullptr;
-  float alone = 0.0f, alone_split = 0.0f, together;
+  float alone = 0.0f, alone_split = 0.0f, alone_unsplit = 0.0f, together;
   for (int i = 0; i < count; ++i) {
     if (w[i].blocked == nullptr || w[i].k_pad != w[0].k_pad) return nullptr;
     float cost;
     int parts;
     const TileCost &whole = cheapest_tile(m, k, 1, n + i, &cost);
     alone += cost;
-    choose_split(m, k, n[i], whole, cost, &parts, &cost);  // (the members' forms are those of gemm_split.hip)
+    const ShortTile in_short = short_tile(m, k, n[i], requant);  // (the members' forms are those of gemm_short.hip and gemm_split.hip)
+    alone_unsplit += in_short.tile != 0 ? in_short.cost : cost;
+    if (in_short.tile != 0 && short_goes_first(m, k)) {
+      cost = in_short.cost;
+    } else {
+      choose_split(m, k, n[i], whole, cost, &parts, &cost);
+    }
     alone_split += cost;
   }
   const TileCost &t = cheapest_tile(m, k, count, n, &together);
   if (together >= alone) return nullptr;
   constexpr float kManyRows = 0.18f;
   if (t.ring && t.tn == 1 && t.tm == 1 && (m + 63) / 64 > kStreamRowTiles) together = t.a + kManyRows * (float)((k + 127) / 128);
-  return together < alone_split || split_space(stream) == nullptr ? &t : nullptr;
+  return together < (split_space(stream) != nullptr ? alone_split : alone_unsplit) ? &t : nullptr;
 }
 
 const TileCost *gemm_group_tile(int64_t lda, int m, int k, int count, const WeightView *w, const int *n, const RequantParams *rq,
                                 hipStream_t stream) {
   for (int i = 0; i < count; ++i)
     if (rq[i].has_zw || !rq[i].fast2) return nullptr;
-  return group_tile(lda, m, k, count, w, n, stream);
+  return group_tile(lda, m, k, count, w, n, true, stream);
 }
 
 const TileCost *gemm_group_tile(int64_t lda, int m, int k, int count, const WeightView *w, const int *n, const DequantParams *dq,
                                 hipStream_t stream) {
   for (int i = 0; i < count; ++i)
     if (dq[i].zw0 != 0) return nullptr;
-  return group_tile(lda, m, k, count, w, n, stream);
+  return group_tile(lda, m, k, count, w, n, false, stream);
 }
 
 template <typename P>

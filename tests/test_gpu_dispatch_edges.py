@@ -308,6 +308,39 @@ def test_matmul_group_of_one_on_few_ragged_rows(m, k, n, copies, how):
         L.mi_debug_fail_alloc(0)
 
 
+# small products, whose K the waves of a workgroup share: two K blocks (half the waves have none), the last with one byte, a chunk and all but
+# one; up to 12 blocks and beyond (four and eight waves), 64 channels x 32 rows, one tile past 256 of each kind; last rows and channels that
+# are partly there
+@pytest.mark.parametrize("m,n,k", [(3, 1, 129), (32, 31, 144), (33, 65, 255), (64, 4095, 256), (65, 2700, 257), (95, 96, 1535), (97, 33, 1537),
+                                   (64, 100, 1536), (40, 4096, 1552), (130, 1600, 1040), (257, 1793, 897), (256, 2048, 896), (129, 2, 4095),
+                                   (70, 300, 4080), (60, 700, 4113), (500, 520, 300), (33, 1001, 9001)])
+@pytest.mark.parametrize("dynamic,asymmetric", [(False, False), (False, True), (True, False), (True, True)])
+def test_matmul_small_products(orc, m, n, k, dynamic, asymmetric):
+    """Against the oracle, bit by bit (integer sums, then a fixed sequence of rounded steps): rows at an aligned and at an odd address,
+    in the middle of larger ones' bytes, which must not count; and with a scale per row."""
+    import torch
+    rng = np.random.default_rng(m + n + k)
+    w, bias, sw, zw, make = _matmul_pair(rng, n, k, asymmetric, dynamic)
+    kern, a = make(True), rng.integers(-128, 128, (m, k), dtype=np.int8)
+    args = dict(in_quant=K.QuantParam(0.03, -5)) if dynamic else {}
+    orc.set_threads(16)
+    if dynamic:
+        want = orc.dynamic_matmul(a, w, bias, 0.03, -5, sw, zw)
+    else:
+        want = orc.matmul_int8(a, w, bias, 0.02, 7, sw, zw, float(np.float32(0.02 * 0.0055 * k ** 0.5 * 140)), 3)
+    for before in (0, 16, 1, 11):
+        flat = torch.full((before + m * k + 64,), 99, dtype=torch.int8, device="cuda")
+        flat[before:before + m * k] = torch.from_numpy(a.reshape(-1)).cuda()
+        got = kern.run(flat[before:before + m * k].view(m, k), **args).cpu().numpy()
+        assert np.array_equal(got.view(np.int8), want.view(np.int8)), before
+    if dynamic:
+        x = rng.standard_normal((m, k)).astype(np.float32)
+        q, params = K.DynamicQuantKernel(True).run_rows(torch.from_numpy(x).cuda())
+        q_want, scale, zp = orc.dynamic_quant_segments(x, True)
+        sure = orc.dynamic_matmul_rows(q_want, w, bias, scale.astype(np.float32), int(zp[0]), sw, zw)
+        assert np.array_equal(kern.run(q, row_params=params).cpu().numpy().view(np.int8), sure.view(np.int8))
+
+
 @pytest.mark.parametrize("taps", [3, 5])
 @pytest.mark.parametrize("b,ih,iw,ch,pad", [(1, 5, 5, 4, (0, 0, 0, 0)), (1, 5, 6, 8, (1, 1, 1, 1)), (2, 7, 9, 12, (2, 0, 0, 2)),
                                             (1, 9, 11, 20, (4, 4, 4, 4)), (3, 6, 8, 192, (1, 2, 3, 0)), (1, 33, 31, 36, (1, 1, 1, 1)),
