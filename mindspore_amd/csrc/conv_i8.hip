@@ -52,7 +52,7 @@ __global__ __launch_bounds__(256) void pad_rows_kernel(const int8_t *__restrict_
 int launch_pad_rows(const int8_t *src, int64_t src_ld, int rows, int k, int8_t *dst, int k16, hipStream_t stream) {
   const int64_t total = (int64_t)rows * (k16 >> 4), want = (total + 255) / 256;
   const int wgs = (int)(want < 1048576 ? want : 1048576);
-  hipLaunchKernelGGL(pad_rows_kernel, dim3(wgs), dim3(256), 0, stream, src, src_ld, total, k, dst, k16 >> 4, 256 * wgs);
+  launch_kernel(pad_rows_kernel, dim3(wgs), dim3(256), 0, stream, src, src_ld, total, k, dst, k16 >> 4, 256 * wgs);
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }
@@ -104,7 +104,7 @@ int launch_im2col(const int8_t *in, const ConvGeom &g, int fill, int8_t *dst, in
   const int64_t total = (int64_t)g.batch * g.out_h * g.out_w * (k16 >> 4);
   const int64_t want = (total + 255) / 256;
   const int blocks = (int)(want < 1 ? 1 : (want > 1048576 ? 1048576 : want));
-  hipLaunchKernelGGL(im2col_kernel, dim3(blocks), dim3(256), 0, stream, in, g, fill, dst, k16);
+  launch_kernel(im2col_kernel, dim3(blocks), dim3(256), 0, stream, in, g, fill, dst, k16);
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }
@@ -254,8 +254,8 @@ int launch_conv_smallk(const int8_t *in, const ConvGeom &g, int fill, int k_true
   const int blocks = (int)((waves + 3) / 4);
   const int ocb = (g.out_c + 31) / 32, ksteps = (k_true + 31) / 32;
 #define MI_SMALLK(KS, OB)                                                                                       \
-  hipLaunchKernelGGL((conv_smallk_kernel<KS, OB>), dim3(blocks), dim3(256), 0, stream, in, g, fill, k_true, w, ldw, \
-                     rq, out)
+  launch_kernel((conv_smallk_kernel<KS, OB>), dim3(blocks), dim3(256), 0, stream, in, g, fill, k_true, w, ldw, \
+                rq, out)
   if (ksteps == 1) {
     if (ocb == 1) MI_SMALLK(1, 1);
     else if (ocb == 2) MI_SMALLK(1, 2);
@@ -548,8 +548,8 @@ int launch_conv_rows(const int8_t *in, const ConvGeom &g, int fill, const int8_t
   c.shifts = (uint32_t)shift_hw | (uint32_t)shift_w << 8 | (streams ? 1u << 16 : 0u);
   c.step = 4 * (int)grid.x;
 #define MI_ROWS_FORM(KS, FORM)                                                                              \
-  if (two) hipLaunchKernelGGL((conv_rows_kernel<KS, 2, FORM>), grid, dim3(256), 0, stream, c, RequantCall::of(rq), out);      \
-  else hipLaunchKernelGGL((conv_rows_kernel<KS, 1, FORM>), grid, dim3(256), 0, stream, c, RequantCall::of(rq), out)
+  if (two) launch_kernel((conv_rows_kernel<KS, 2, FORM>), grid, dim3(256), 0, stream, c, RequantCall::of(rq), out);      \
+  else launch_kernel((conv_rows_kernel<KS, 1, FORM>), grid, dim3(256), 0, stream, c, RequantCall::of(rq), out)
 #define MI_ROWS(KS)                     \
   case KS:                              \
     if (form == kReluForm) {            \
@@ -801,7 +801,7 @@ static int launch_dw_rows(ConvDwRows c, int batch, int zo, hipStream_t stream) {
                         (int64_t)batch * c.out_h * c.out_w * c.ch <= (c.ch % 32 == 0 ? kStreamedMost : kStreamedMost / 2);
   const auto kernel = c.amin >= zo ? (streamed ? conv_dw_rows_kernel<KS, OT, true, true> : conv_dw_rows_kernel<KS, OT, true, false>)
                                    : (streamed ? conv_dw_rows_kernel<KS, OT, false, true> : conv_dw_rows_kernel<KS, OT, false, false>);
-  hipLaunchKernelGGL(kernel, dim3((c.total + 255) / 256), dim3(256), 0, stream, c);
+  launch_kernel(kernel, dim3((c.total + 255) / 256), dim3(256), 0, stream, c);
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }
@@ -1022,11 +1022,11 @@ static void launch_dw_vec(const int8_t *in, const ConvGeom &g, const int16_t *w1
   const int64_t want = (total + 255) / 256;
   const int blocks = (int)(want < 1 ? 1 : (want > 1048576 ? 1048576 : want));
   if (rq.fast) {
-    hipLaunchKernelGGL((conv_dw16_kernel<TAPS, CG, true>), dim3(blocks), dim3(256), 0, stream, in, g, w16, bias_folded,
-                       zx8, rq, out);
+    launch_kernel((conv_dw16_kernel<TAPS, CG, true>), dim3(blocks), dim3(256), 0, stream, in, g, w16, bias_folded,
+                  zx8, rq, out);
   } else {
-    hipLaunchKernelGGL((conv_dw16_kernel<TAPS, CG, false>), dim3(blocks), dim3(256), 0, stream, in, g, w16, bias_folded,
-                       zx8, rq, out);
+    launch_kernel((conv_dw16_kernel<TAPS, CG, false>), dim3(blocks), dim3(256), 0, stream, in, g, w16, bias_folded,
+                  zx8, rq, out);
   }
 }
 
@@ -1050,7 +1050,7 @@ int launch_conv_dw(const int8_t *in, const ConvGeom &g, const int16_t *w16, cons
     const int64_t total = (int64_t)g.batch * g.out_h * g.out_w * g.out_c;
     const int64_t want = (total + 255) / 256;
     const int blocks = (int)(want < 1 ? 1 : (want > 1048576 ? 1048576 : want));
-    hipLaunchKernelGGL(conv_dw_kernel, dim3(blocks), dim3(256), 0, stream, in, g, w16, bias, zx8, rq, out);
+    launch_kernel(conv_dw_kernel, dim3(blocks), dim3(256), 0, stream, in, g, w16, bias, zx8, rq, out);
   }
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;

@@ -208,20 +208,20 @@ static int launch_thin(const ConvThin &c, const RequantParams &rq, int8_t *out, 
   if constexpr (OCB == 2) {
     if (form != kGeneralForm && c.out_c == 256) {
       if (form == kReluForm) {
-        hipLaunchKernelGGL((conv_thin_kernel<CH, OCB, kReluForm, false>), grid, dim3(256), lds, stream, c, RequantCall::of(rq), out);
+        launch_kernel((conv_thin_kernel<CH, OCB, kReluForm, false>), grid, dim3(256), lds, stream, c, RequantCall::of(rq), out);
       } else {
-        hipLaunchKernelGGL((conv_thin_kernel<CH, OCB, kCarryForm, false>), grid, dim3(256), lds, stream, c, RequantCall::of(rq), out);
+        launch_kernel((conv_thin_kernel<CH, OCB, kCarryForm, false>), grid, dim3(256), lds, stream, c, RequantCall::of(rq), out);
       }
       MI_HIP_CHECK(hipGetLastError());
       return MI_OK;
     }
   }
   if (form == kReluForm) {
-    hipLaunchKernelGGL((conv_thin_kernel<CH, OCB, kReluForm>), grid, dim3(256), lds, stream, c, RequantCall::of(rq), out);
+    launch_kernel((conv_thin_kernel<CH, OCB, kReluForm>), grid, dim3(256), lds, stream, c, RequantCall::of(rq), out);
   } else if (form == kCarryForm) {
-    hipLaunchKernelGGL((conv_thin_kernel<CH, OCB, kCarryForm>), grid, dim3(256), lds, stream, c, RequantCall::of(rq), out);
+    launch_kernel((conv_thin_kernel<CH, OCB, kCarryForm>), grid, dim3(256), lds, stream, c, RequantCall::of(rq), out);
   } else if constexpr (OCB <= 3) {
-    hipLaunchKernelGGL((conv_thin_kernel<CH, OCB, kGeneralForm>), grid, dim3(256), lds, stream, c, RequantCall::of(rq), out);
+    launch_kernel((conv_thin_kernel<CH, OCB, kGeneralForm>), grid, dim3(256), lds, stream, c, RequantCall::of(rq), out);
   }
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;

@@ -350,7 +350,7 @@ int launch_conv_window(const int8_t *in, const ConvGeom &g, const int8_t *fill16
   const size_t lds = (size_t)t.weight_bytes + t.patch_bytes + 8 * (size_t)t.steps;
   const dim3 grid((unsigned)t.tiles), threads(64 * kWaves);
   const WindowKernel kernel = kWindowKernels[g.out_c > 32][packed][requant_form(rq) == kReluForm];
-  hipLaunchKernelGGL(kernel, grid, threads, lds, stream, c, rq, out);
+  launch_kernel(kernel, grid, threads, lds, stream, c, rq, out);
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }

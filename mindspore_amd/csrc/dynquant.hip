@@ -524,8 +524,8 @@ template <int T, int G>
 static void launch_rows(const float *x, int64_t segments, int unit, int symmetric, mi_dq_params *params, int8_t *q,
                         hipStream_t stream) {
   const int64_t blocks = T == 64 ? (segments + 3) / 4 : segments;
-  hipLaunchKernelGGL((dq_rows_kernel<T, G>), dim3((unsigned)blocks), dim3(T == 64 ? 256 : T), 0, stream, x, segments,
-                     unit, symmetric, params, q);
+  launch_kernel((dq_rows_kernel<T, G>), dim3((unsigned)blocks), dim3(T == 64 ? 256 : T), 0, stream, x, segments,
+                unit, symmetric, params, q);
 }
 
 int launch_dynquant_segments(const float *x, int64_t segments, int64_t unit, int symmetric, mi_dq_params *params,
@@ -560,8 +560,8 @@ int launch_dynquant_segments(const float *x, int64_t segments, int64_t unit, int
   else if (n4 <= 4096) MI_DQ_ROWS(512, 8);
   else if (n4 <= 16384) MI_DQ_ROWS(1024, 16);
   else
-    hipLaunchKernelGGL(dq_long_rows_kernel, dim3((unsigned)segments), dim3(1024), 0, stream, x, segments, unit, symmetric,
-                       params, q);
+    launch_kernel(dq_long_rows_kernel, dim3((unsigned)segments), dim3(1024), 0, stream, x, segments, unit, symmetric,
+                  params, q);
 #undef MI_DQ_ROWS
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
@@ -572,8 +572,8 @@ static void launch_fused(const float *x, int64_t n, int symmetric, void *slots, 
                          mi_dq_params *params, int8_t *q, hipStream_t stream) {
   const int64_t want = ((n >> 2) + T * G - 1) / (T * G);
   const int wgs = want < 1 ? 1 : (int)want;
-  hipLaunchKernelGGL((dq_fused_kernel<T, G>), dim3(wgs), dim3(T), 0, stream, x, n, symmetric,
-                     static_cast<DqSlots *>(slots), launch, kDqPatience, wgs, note, params, q);
+  launch_kernel((dq_fused_kernel<T, G>), dim3(wgs), dim3(T), 0, stream, x, n, symmetric,
+                static_cast<DqSlots *>(slots), launch, kDqPatience, wgs, note, params, q);
 }
 
 int launch_dynquant(const float *x, int64_t n, int symmetric, float2 *partials, void *slots, uint32_t launch,
@@ -612,15 +612,15 @@ int launch_dynquant(const float *x, int64_t n, int symmetric, float2 *partials, 
   // pass 1: at most one workgroup per partial a thread of pass 2 reads in a single step
   const int64_t want1 = (want + 2) / 3;
   const int nparts = (int)(want1 < 1 ? 1 : (want1 > kDqThreads ? kDqThreads : want1));
-  hipLaunchKernelGGL(dq_minmax_kernel, dim3(nparts), dim3(kDqThreads), 0, stream, x, n, partials);
+  launch_kernel(dq_minmax_kernel, dim3(nparts), dim3(kDqThreads), 0, stream, x, n, partials);
   MI_HIP_CHECK(hipGetLastError());
   const int64_t qblocks = want < 1 ? 1 : want;
   if (qblocks > 0x7fffffff) {
     set_error("dynquant: tensor too large");
     return MI_PARAM_INVALID;
   }
-  hipLaunchKernelGGL(dq_quantize_kernel, dim3((unsigned)qblocks), dim3(kDqThreads), 0, stream, x, n, symmetric,
-                     partials, nparts, note, params, q);
+  launch_kernel(dq_quantize_kernel, dim3((unsigned)qblocks), dim3(kDqThreads), 0, stream, x, n, symmetric,
+                partials, nparts, note, params, q);
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }

@@ -158,7 +158,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 template <int EPI, bool HAS_ZW, bool FAST>
 static int launch(const GemmArgs &g, const RequantParams &rq, const DequantParams &dq, hipStream_t stream) {
   const auto call = GemmCall<EPI>::of(g, g.wb, 64, 64, rq, dq);
-  hipLaunchKernelGGL((gemm_anyrow_kernel<EPI, HAS_ZW, FAST>), call.grid(), dim3(256), 0, stream, call);
+  launch_kernel((gemm_anyrow_kernel<EPI, HAS_ZW, FAST>), call.grid(), dim3(256), 0, stream, call);
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }

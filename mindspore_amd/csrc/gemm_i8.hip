@@ -345,7 +345,7 @@ template <int TILE_N, int TILE_M, int EPI, bool HAS_ZW, bool FAST, int NST = 4, 
 static int launch_cfg(const GemmArgs &g, const RequantParams &rq, const DequantParams &dq, hipStream_t stream) {
   const auto call = GemmCall<EPI>::of(g, g.w, TILE_N, TILE_M, rq, dq);
   auto kern = gemm_direct_kernel<TILE_N, TILE_M, EPI, HAS_ZW, FAST, NST, OCC>;
-  hipLaunchKernelGGL(kern, call.grid(), dim3(256), 0, stream, call);
+  launch_kernel(kern, call.grid(), dim3(256), 0, stream, call);
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }
@@ -584,7 +584,7 @@ int launch_gemm_requant(const int8_t *a, int64_t lda, int m, int k, const Weight
 template <int TILE_N, int TILE_M, bool HAS_ZW, bool FAST, int NST, int OCC>
 static int launch_conv_cfg(const ConvCall &call, hipStream_t stream) {
   auto kern = gemm_conv_kernel<TILE_N, TILE_M, HAS_ZW, FAST, NST, OCC>;
-  hipLaunchKernelGGL(kern, dim3((call.m + TILE_M - 1) / TILE_M * ((call.n + TILE_N - 1) / TILE_N)), dim3(256), 0, stream, call);
+  launch_kernel(kern, dim3((call.m + TILE_M - 1) / TILE_M * ((call.n + TILE_N - 1) / TILE_N)), dim3(256), 0, stream, call);
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }

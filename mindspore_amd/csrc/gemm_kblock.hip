@@ -348,9 +348,9 @@ template <int TN, int TM, int EPI, bool HAS_ZW, bool FAST>
 static int launch_kblock(const GemmArgs &g, const RequantParams &rq, const DequantParams &dq, hipStream_t stream) {
   const auto call = GemmCall<EPI>::of(g, g.wb != nullptr ? g.wb : g.w, 64 * TN, 64 * TM, rq, dq);
   if (g.wb != nullptr) {
-    hipLaunchKernelGGL((gemm_kblock_kernel<TN, TM, EPI, HAS_ZW, FAST, true>), call.grid(), dim3(256), 0, stream, call);
+    launch_kernel((gemm_kblock_kernel<TN, TM, EPI, HAS_ZW, FAST, true>), call.grid(), dim3(256), 0, stream, call);
   } else if constexpr (TN == TM) {
-    hipLaunchKernelGGL((gemm_kblock_kernel<TN, TM, EPI, HAS_ZW, FAST, false>), call.grid(), dim3(256), 0, stream, call);
+    launch_kernel((gemm_kblock_kernel<TN, TM, EPI, HAS_ZW, FAST, false>), call.grid(), dim3(256), 0, stream, call);
   } else {  // (rectangular tiles are chosen for the blocked copy only)
     set_error("gemm: the blocked weight copy is missing");
     return MI_NULL_PTR;
@@ -387,7 +387,7 @@ int launch_gemm_kblock(int tile, bool requant, bool has_zw, bool fast, GemmArgs 
 template <int TN, int TM>
 static int launch_group(GemmGroup<RequantParams> grp, hipStream_t stream) {
   const dim3 grid(group_tiles(&grp, 64 * TN, 64 * TM));
-  hipLaunchKernelGGL((gemm_kblock_group_kernel<TN, TM>), grid, dim3(256), 0, stream, grp);
+  launch_kernel((gemm_kblock_group_kernel<TN, TM>), grid, dim3(256), 0, stream, grp);
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }
@@ -395,7 +395,7 @@ static int launch_group(GemmGroup<RequantParams> grp, hipStream_t stream) {
 template <int TN, int TM, bool FAST>
 static int launch_group_deq(GemmGroup<DequantParams> grp, hipStream_t stream) {
   const dim3 grid(group_tiles(&grp, 64 * TN, 64 * TM));
-  hipLaunchKernelGGL((gemm_kblock_group_deq_kernel<TN, TM, FAST>), grid, dim3(256), 0, stream, grp);
+  launch_kernel((gemm_kblock_group_deq_kernel<TN, TM, FAST>), grid, dim3(256), 0, stream, grp);
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }

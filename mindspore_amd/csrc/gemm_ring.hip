@@ -45,9 +45,9 @@ template <int TN, int TM, int S, int EPI, bool HAS_ZW, bool FAST>
 static int launch_ring(const GemmArgs &g, const RequantParams &rq, const DequantParams &dq, hipStream_t stream) {
   const auto call = GemmCall<EPI>::of(g, g.wb, 64 * TN, 64 * TM, rq, dq);
   if (call.tiles_m <= kStreamRowTiles) {
-    hipLaunchKernelGGL((gemm_ring_kernel<TN, TM, S, EPI, HAS_ZW, FAST, true>), call.grid(), dim3(256), 0, stream, call);
+    launch_kernel((gemm_ring_kernel<TN, TM, S, EPI, HAS_ZW, FAST, true>), call.grid(), dim3(256), 0, stream, call);
   } else {
-    hipLaunchKernelGGL((gemm_ring_kernel<TN, TM, S, EPI, HAS_ZW, FAST, false>), call.grid(), dim3(256), 0, stream, call);
+    launch_kernel((gemm_ring_kernel<TN, TM, S, EPI, HAS_ZW, FAST, false>), call.grid(), dim3(256), 0, stream, call);
   }
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
@@ -89,9 +89,9 @@ template <int TN, int TM, int S>
 static int launch_group(GemmGroup<RequantParams> grp, hipStream_t stream) {
   const dim3 grid(group_tiles(&grp, 64 * TN, 64 * TM));
   if (grp.g.tiles_m <= kStreamRowTiles) {
-    hipLaunchKernelGGL((gemm_ring_group_kernel<TN, TM, S, true>), grid, dim3(256), 0, stream, grp);
+    launch_kernel((gemm_ring_group_kernel<TN, TM, S, true>), grid, dim3(256), 0, stream, grp);
   } else {
-    hipLaunchKernelGGL((gemm_ring_group_kernel<TN, TM, S, false>), grid, dim3(256), 0, stream, grp);
+    launch_kernel((gemm_ring_group_kernel<TN, TM, S, false>), grid, dim3(256), 0, stream, grp);
   }
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
@@ -101,9 +101,9 @@ template <int TN, int TM, int S, bool FAST>
 static int launch_group_deq(GemmGroup<DequantParams> grp, hipStream_t stream) {
   const dim3 grid(group_tiles(&grp, 64 * TN, 64 * TM));
   if (grp.g.tiles_m <= kStreamRowTiles) {
-    hipLaunchKernelGGL((gemm_ring_group_deq_kernel<TN, TM, S, FAST, true>), grid, dim3(256), 0, stream, grp);
+    launch_kernel((gemm_ring_group_deq_kernel<TN, TM, S, FAST, true>), grid, dim3(256), 0, stream, grp);
   } else {
-    hipLaunchKernelGGL((gemm_ring_group_deq_kernel<TN, TM, S, FAST, false>), grid, dim3(256), 0, stream, grp);
+    launch_kernel((gemm_ring_group_deq_kernel<TN, TM, S, FAST, false>), grid, dim3(256), 0, stream, grp);
   }
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;

@@ -268,7 +268,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2)))
 template <int WAVES, int TN, bool ANY, int EPI, bool HAS_ZW>
 static int launch(const GemmArgs &g, const RequantParams &rq, const DequantParams &dq, hipStream_t stream) {
   const auto call = GemmCall<EPI>::of(g, g.wb, 32 * TN, 32, rq, dq);
-  hipLaunchKernelGGL((gemm_short_kernel<WAVES, TN, EPI, HAS_ZW, ANY>), call.grid(), dim3(64 * WAVES), 0, stream, call);
+  launch_kernel((gemm_short_kernel<WAVES, TN, EPI, HAS_ZW, ANY>), call.grid(), dim3(64 * WAVES), 0, stream, call);
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }

@@ -114,9 +114,9 @@ static int launch(int parts, const GemmArgs &g, const RequantParams &rq, const D
   }
   const dim3 grid((unsigned)(tiles * parts));
   if (split.call.tiles_m <= kStreamRowTiles) {
-    hipLaunchKernelGGL((gemm_split_kernel<TN, TM, S, EPI, HAS_ZW, FAST, true>), grid, dim3(256), 0, stream, split);
+    launch_kernel((gemm_split_kernel<TN, TM, S, EPI, HAS_ZW, FAST, true>), grid, dim3(256), 0, stream, split);
   } else {
-    hipLaunchKernelGGL((gemm_split_kernel<TN, TM, S, EPI, HAS_ZW, FAST, false>), grid, dim3(256), 0, stream, split);
+    launch_kernel((gemm_split_kernel<TN, TM, S, EPI, HAS_ZW, FAST, false>), grid, dim3(256), 0, stream, split);
   }
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;

@@ -478,7 +478,7 @@ static int launch_mrdx(const GemvArgs &g, const RequantParams &rq, hipStream_t s
   const int lds_bytes = DIRECT ? 0 : M * ((g.kchunks + 63) / 64) * 1024;
   const int rows_per_block = 4 / KS * R;
   const int blocks = (g.n + rows_per_block - 1) / rows_per_block;
-  hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), lds_bytes, stream, GemvCall<false>::of(g, M, rq));
+  launch_kernel(kern, dim3(blocks), dim3(256), lds_bytes, stream, GemvCall<false>::of(g, M, rq));
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }
@@ -488,8 +488,8 @@ static int launch_mrdx_deq(const GemvArgs &g, const DequantParams &dq, hipStream
   const int lds_bytes = DIRECT ? 0 : M * ((g.kchunks + 63) / 64) * 1024;
   const int rows_per_block = 4 / KS * R;
   const int blocks = (g.n + rows_per_block - 1) / rows_per_block;
-  hipLaunchKernelGGL((gemv_i8_deq_kernel<M, R, D, DIRECT, KS, ANY>), dim3(blocks), dim3(256), lds_bytes, stream,
-                     GemvCall<true>::of(g, M, dq));
+  launch_kernel((gemv_i8_deq_kernel<M, R, D, DIRECT, KS, ANY>), dim3(blocks), dim3(256), lds_bytes, stream,
+                GemvCall<true>::of(g, M, dq));
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }
@@ -518,11 +518,11 @@ static int launch_group_mrdx(const GemvGroupT<P> &grp, hipStream_t stream) {
   const int lds_bytes = DIRECT ? 0 : M * ((grp.g[0].kchunks + 63) / 64) * 1024;
   return with_group_call(grp, M, 4 / KS * R, [&](const auto &call, int blocks, auto members) {
     if constexpr (std::is_same<P, DequantParams>::value) {
-      hipLaunchKernelGGL((gemv_i8_group_deq_kernel<M, R, D, DIRECT, KS, decltype(members)::value>), dim3(blocks), dim3(256), lds_bytes,
-                         stream, call);
+      launch_kernel((gemv_i8_group_deq_kernel<M, R, D, DIRECT, KS, decltype(members)::value>), dim3(blocks), dim3(256), lds_bytes,
+                    stream, call);
     } else {
-      hipLaunchKernelGGL((gemv_i8_group_kernel<M, R, D, DIRECT, KS, decltype(members)::value>), dim3(blocks), dim3(256), lds_bytes,
-                         stream, call);
+      launch_kernel((gemv_i8_group_kernel<M, R, D, DIRECT, KS, decltype(members)::value>), dim3(blocks), dim3(256), lds_bytes,
+                    stream, call);
     }
   });
 }
@@ -898,16 +898,16 @@ static int with_row_class(int m, F &&f) {  // rows rounded up to 2, 4, 8, 16 or 
 // against 64 x 64 GEMM tiles in us per launch at 64 rows: 4096 x 4096 11.0 -> 8.8, 4096 x 11008 27.5 -> 18.7.
 template <bool ANY>
 static int launch_mfma_lds_64(const GemvArgs &g, int m, const RequantParams &rq, hipStream_t stream) {
-  hipLaunchKernelGGL((gemv_mfma_lds_kernel<8, 1, 2, 64, ANY>), dim3((g.n + 15) / 16), dim3(512), 0, stream,
-                     GemvCall<false>::of(g, m, rq));
+  launch_kernel((gemv_mfma_lds_kernel<8, 1, 2, 64, ANY>), dim3((g.n + 15) / 16), dim3(512), 0, stream,
+                GemvCall<false>::of(g, m, rq));
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }
 
 template <bool ANY>
 static int launch_mfma_lds_deq_64(const GemvArgs &g, int m, const DequantParams &dq, hipStream_t stream) {
-  hipLaunchKernelGGL((gemv_mfma_lds_deq_kernel<8, 1, 2, 64, ANY>), dim3((g.n + 15) / 16), dim3(512), 0, stream,
-                     GemvCall<true>::of(g, m, dq));
+  launch_kernel((gemv_mfma_lds_deq_kernel<8, 1, 2, 64, ANY>), dim3((g.n + 15) / 16), dim3(512), 0, stream,
+                GemvCall<true>::of(g, m, dq));
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }
@@ -918,9 +918,9 @@ static int launch_group_mfma_lds(const GemvGroupT<P> &grp, int m, hipStream_t st
     return with_group_call(grp, m, RG * 16, [&](const auto &call, int blocks, auto members) {
       constexpr int MR = decltype(mr)::value, N = decltype(members)::value;
       if constexpr (std::is_same<P, DequantParams>::value) {
-        hipLaunchKernelGGL((gemv_mfma_lds_group_deq_kernel<WAVES, RG, D, MR, N>), dim3(blocks), dim3(WAVES * 64), 0, stream, call);
+        launch_kernel((gemv_mfma_lds_group_deq_kernel<WAVES, RG, D, MR, N>), dim3(blocks), dim3(WAVES * 64), 0, stream, call);
       } else {
-        hipLaunchKernelGGL((gemv_mfma_lds_group_kernel<WAVES, RG, D, MR, N>), dim3(blocks), dim3(WAVES * 64), 0, stream, call);
+        launch_kernel((gemv_mfma_lds_group_kernel<WAVES, RG, D, MR, N>), dim3(blocks), dim3(WAVES * 64), 0, stream, call);
       }
     });
   });
@@ -930,8 +930,8 @@ template <int WAVES, int RG, int D, bool ANY>
 static int launch_mfma_lds(const GemvArgs &g, int m, const RequantParams &rq, hipStream_t stream) {
   const int blocks = (g.n + RG * 16 - 1) / (RG * 16);
   return with_row_class<WAVES, D>(m, [&](auto mr) {
-    hipLaunchKernelGGL((gemv_mfma_lds_kernel<WAVES, RG, D, decltype(mr)::value, ANY>), dim3(blocks), dim3(WAVES * 64), 0,
-                       stream, GemvCall<false>::of(g, m, rq));
+    launch_kernel((gemv_mfma_lds_kernel<WAVES, RG, D, decltype(mr)::value, ANY>), dim3(blocks), dim3(WAVES * 64), 0,
+                  stream, GemvCall<false>::of(g, m, rq));
     MI_HIP_CHECK(hipGetLastError());
     return (int)MI_OK;
   });
@@ -953,8 +953,8 @@ __global__ __launch_bounds__(256) void block_weights_kernel(const int8_t *__rest
 int launch_block_weights(const int8_t *w, int n_pad, int k_pad, int ldw, int8_t *blocked, hipStream_t stream) {
   const int64_t chunks = (int64_t)n_pad * k_pad / 16;
   const int64_t want = (chunks + 255) / 256;
-  hipLaunchKernelGGL(block_weights_kernel, dim3((unsigned)(want > 65536 ? 65536 : want)), dim3(256), 0, stream, w, ldw,
-                     k_pad / 64, chunks, blocked);
+  launch_kernel(block_weights_kernel, dim3((unsigned)(want > 65536 ? 65536 : want)), dim3(256), 0, stream, w, ldw,
+                k_pad / 64, chunks, blocked);
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;
 }
@@ -963,8 +963,8 @@ template <int WAVES, int RG, int D, bool ANY>
 static int launch_mfma_lds_deq(const GemvArgs &g, int m, const DequantParams &dq, hipStream_t stream) {
   const int blocks = (g.n + RG * 16 - 1) / (RG * 16);
   return with_row_class<WAVES, D>(m, [&](auto mr) {
-    hipLaunchKernelGGL((gemv_mfma_lds_deq_kernel<WAVES, RG, D, decltype(mr)::value, ANY>), dim3(blocks), dim3(WAVES * 64),
-                       0, stream, GemvCall<true>::of(g, m, dq));
+    launch_kernel((gemv_mfma_lds_deq_kernel<WAVES, RG, D, decltype(mr)::value, ANY>), dim3(blocks), dim3(WAVES * 64),
+                  0, stream, GemvCall<true>::of(g, m, dq));
     MI_HIP_CHECK(hipGetLastError());
     return (int)MI_OK;
   });

@@ -111,10 +111,10 @@ int launch_chunks(HostSlots *s, const Chunks &c, int64_t i, int n, char *dev, bo
   uint32_t *flags = s->flags + c.first_flag(c.slot(i));
   v4i *there = reinterpret_cast<v4i *>(dev), *here = reinterpret_cast<v4i *>(staged);
   if (in) {
-    hipLaunchKernelGGL((host_copy_kernel<false>), dim3(parts), dim3(256), 0, nullptr, here, there, n16, parts, flags, s->ticket);
+    launch_kernel((host_copy_kernel<false>), dim3(parts), dim3(256), 0, nullptr, here, there, n16, parts, flags, s->ticket);
   } else {
     const int wgs = parts < kOutWgs ? parts : kOutWgs;
-    hipLaunchKernelGGL((host_copy_kernel<true>), dim3(wgs), dim3(256), 0, nullptr, there, here, n16, wgs, flags, s->ticket);
+    launch_kernel((host_copy_kernel<true>), dim3(wgs), dim3(256), 0, nullptr, there, here, n16, wgs, flags, s->ticket);
   }
   MI_HIP_CHECK(hipGetLastError());
   for (int k = 0; k < n; ++k) s->pending[c.slot(i) + k] = s->ticket;
