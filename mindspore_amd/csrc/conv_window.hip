@@ -29,6 +29,11 @@ namespace mi {
 // loaded once, four pixels a lane.  32 x 224 x 224 x 3 -> 64, 7x7, stride 2: 20.5 us -> 14.5 to 16.5, of which launch and prologue 5.9,
 // the pixels 2, products 3, stores about 5 (26 MB); 296 vector instructions a wave keep the vector ALU busy 58 % of the time, fragment
 // reads LDS 37 %.
+//
+// More than 64 channels (three and four blocks): the weights of a 3x3 on 96 channels alone are 81 KiB, so that one workgroup of eight waves
+// has the CU.  Where the GEMM's tiles of 128 channels were a quarter empty and fetched every pixel nine times that is still far quicker:
+// 32 x 56 x 56, 96 -> 96 21.7 -> 14.3, 80 -> 80 19.6 -> 14.1, 64 -> 96 16.0 -> 9.8, 64 -> 128 16.1 -> 13.2; packed, 32 x 224 x 224 x 3 -> 96,
+// 7x7, stride 2 (conv_rows_kernel) 35.9 -> 19.6.
 struct ConvWindow {
   const int8_t *in;
   const int8_t *in_last4;  // the tensor's last four bytes
@@ -56,7 +61,7 @@ typedef v4i v4i_4 __attribute__((aligned(4)));
 typedef v4u v4u_any __attribute__((aligned(1)));
 
 template <int OCB, bool PACKED, RequantForm FORM>
-__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWaves / 2))) void conv_window_kernel(
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(OCB == 4 || (OCB == 3 && !PACKED) ? kWaves / 4 : kWaves / 2))) void conv_window_kernel(
     ConvWindow g, RequantParams rq, int8_t *__restrict__ out) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5;
@@ -73,7 +78,8 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWa
   int *table = reinterpret_cast<int *>(patch + g.patch_bytes);
   // The first weights, the pixels, the last two loads of weights of each wave: the products of the first weights begin while
   // those are on their way.
-  constexpr int kLate = 2, kLateSteps = kWaves * kLate / OCB;
+  constexpr int kLate = OCB == 3 ? 3 : 2, kLateSteps = kWaves * kLate / OCB;
+  static_assert(PACKED || kLateSteps * OCB == kWaves * kLate, "every wave has as many late loads");
   const int early = PACKED ? 0 : max(g.steps - kLateSteps, 0);  // steps whose weights come first
   auto load_weights = [&](int from, int to) {
     for (int i = from * OCB + wave; i < to * OCB; i += kWaves) {
@@ -215,9 +221,12 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWa
 // ---- host side -----------------------------------------------------------------------------------------------------
 static uint32_t magic16(int d) { return d <= 1 ? 0u : (uint32_t)((((uint64_t)1 << 32) + d - 1) / (uint64_t)d); }
 
+// Blocks of 32 channels that a workgroup computes.
+static int window_blocks(const ConvGeom &g) { return (g.out_c + 31) / 32; }
+
 static std::vector<int8_t> operand_order(const int8_t *w, int oc, int k) {
-  const int steps = (k + 31) / 32, ocb = oc > 32 ? 2 : 1;
-  std::vector<int8_t> out((size_t)((oc + 31) / 32) * steps * 1024, 0);
+  const int steps = (k + 31) / 32, ocb = (oc + 31) / 32;
+  std::vector<int8_t> out((size_t)ocb * steps * 1024, 0);
   for (int column = 0; column < 32 * ocb; ++column) {
     const int n = column_channel(ocb, column / 32, column % 32);
     if (n >= oc) continue;
@@ -245,10 +254,12 @@ std::vector<int8_t> conv_window_weights(const ConvGeom &g, const int8_t *w) {
 }
 
 constexpr int kWindowLds = 80 << 10;  // two workgroups per CU
+constexpr int kWindowLdsWide = 160 << 10;  // one, of more than 64 channels
 struct WindowCut {
   int tile_h, tile_w, tiles_x, tiles_y, patch_h, patch_w, pitch, steps, weight_bytes, patch_bytes;
   int64_t tiles;
 };
+static int window_lds(const ConvGeom &g) { return window_blocks(g) > 2 && !packed_window(g) ? kWindowLdsWide : kWindowLds; }
 // The rectangles of an image that need the fewest workgroups, and of those the fewest input pixels; false if none fits.
 static bool cut_window(const ConvGeom &g, WindowCut *best) {
   const int cc = g.in_c / 16, most = 32 * kWaves;  // (tile_w <= most)
@@ -256,7 +267,7 @@ static bool cut_window(const ConvGeom &g, WindowCut *best) {
   const bool packed = packed_window(g);
   c.pitch = cc | 1;
   c.steps = packed ? (g.kernel_h * row_chunks(g) + 1) / 2 : (g.kernel_h * g.kernel_w * cc + 1) / 2;
-  c.weight_bytes = (g.out_c > 32 ? 2 : 1) * c.steps * 1024;
+  c.weight_bytes = window_blocks(g) * c.steps * 1024;
   best->tiles = 0;
   for (int nx = (g.out_w + 63) / 64, last = std::min(64, (g.out_w + 7) / 8); nx <= last; ++nx) {  // 8 to 64 pixels wide
     c.tile_w = (g.out_w + nx - 1) / nx;
@@ -274,7 +285,7 @@ static bool cut_window(const ConvGeom &g, WindowCut *best) {
     c.patch_w = (int)pw;
     const int64_t patch = (ph + (packed ? g.dilation_h : 0)) * pw * (packed ? 4 : c.pitch * 16);
     const int64_t bytes = (patch + 1023) / 1024 * 1024;  // (at most kWindowLds, hence fewer than 2^16 chunks)
-    if (c.weight_bytes + bytes + 8 * c.steps > kWindowLds) continue;
+    if (c.weight_bytes + bytes + 8 * c.steps > window_lds(g)) continue;
     c.patch_bytes = (int)bytes;
     c.tiles = (int64_t)c.tiles_x * c.tiles_y * g.batch;
     const bool fewer = c.tiles < best->tiles || (c.tiles == best->tiles && c.patch_bytes < best->patch_bytes);
@@ -283,45 +294,68 @@ static bool cut_window(const ConvGeom &g, WindowCut *best) {
   return best->tiles != 0;
 }
 
-// Up to 64 channels, which one workgroup computes (more would fetch the pixels again), rectangles for two CUs in three, and at
+// Up to 128 channels, which one workgroup computes (more would fetch the pixels again), rectangles for two CUs in three, and at
 // least half of their pixels there.  Time of this relative to the gathering GEMM, 3x3: workgroups 112 1.01, 128 1.02, 140 1.02,
 // 160 1.02, 168 0.88 0.91, 192 0.87, 196 0.89, 224 0.87, 256 0.77, 448 0.75, 1024 0.70; stride 2 256 0.74; 5x5 128 0.84, 256 0.73.
-// Rectangles filled to 0.77 0.77, 0.56 0.87, 0.39 0.90 to 1.05, 0.25 1.43, 0.19 1.40 to 2.1.  Against 65 to 128 channels 0.99 to 1.24.
+// Rectangles filled to 0.77 0.77, 0.56 0.87, 0.39 0.90 to 1.05, 0.25 1.43, 0.19 1.40 to 2.1.
+// 65 to 96 channels, of which the GEMM's 128-channel tiles leave a quarter and more empty, already from 96 workgroups: 96 -> 96 56 1.02,
+// 98 0.84, 112 0.86, 224 0.72, 448 0.66, 64 -> 96 56 1.10, 112 0.90, 448 0.61, 32 -> 72 896 0.55; 97 to 128: 64 -> 128 112 1.03, 128 1.04,
+// 224 0.84, 448 0.82, 32 -> 128 252 0.89.
 // Three or four channels: windows for which conv_rows_kernel makes five or more loads.  Time relative to that one, us: 7x7 on 3
 // channels -> 64, 49 workgroups 4.42 / 4.42, 98 4.46 / 4.48, 196 6.2 / 4.65, 392 8.55 / 6.05, 784 12.2 / 9.55, 1568 20.5 / 16.5;
-// 5x5 on 4 (five loads) 4.85 / 4.4 and 14.8 / 14.7; 5x5 on 3 (three) 4.15 / 4.18; 3x3 on 3 (two) 5.17 / 5.55 and 7.7 / 8.8.
-constexpr int kWindowLeastTiles = 168;
+// -> 96, 49 4.82 / 4.89, 98 6.71 / 5.06, 1568 35.9 / 19.6, -> 128, 98 6.78 / 5.73, 1568 38.1 / 24.0;
+// 5x5 on 4 (five loads) 4.85 / 4.4 and 14.8 / 14.7, -> 96, 90 workgroups 5.10 / 4.55; 5x5 on 3 (three) 4.15 / 4.18; 3x3 on 3 (two)
+// 5.17 / 5.55 and 7.7 / 8.8.
+constexpr int kWindowLeastTiles = 168, kWindowLeastWideTiles = 96;
+static int least_tiles(const ConvGeom &g) {
+  return window_blocks(g) == 3 || (window_blocks(g) == 4 && packed_window(g)) ? kWindowLeastWideTiles : kWindowLeastTiles;
+}
+// More than 64 channels beside several taps of 16-channel-aligned images mostly leave room for one workgroup a CU, and what counts then is
+// how many rounds of them there are beside those of the GEMM's 128 x 128 tiles, two a CU.  A round takes 0.7 of one of those for 65 to 96
+// channels, 0.85 to 0.9 for up to 128 (full rounds: 96 -> 96 8.75 / 12.5, 64 -> 128 7.85 / 9.35); two a CU as long as one of the GEMM's
+// rounds and do twice as much.  Relative time at 252 workgroups (against one of the GEMM's rounds) 0.70, 266 1.11, 280 1.18 (not taken),
+// 336 (against two) 0.78, 512 0.69, 518 0.95 (not taken); 64 -> 128 336 0.96, 518 1.14 (not taken).
+static bool wide_rounds_pay(const ConvGeom &g, const WindowCut &c) {
+  if (window_blocks(g) < 3 || packed_window(g)) return true;
+  const bool two = window_blocks(g) == 3 && c.weight_bytes + c.patch_bytes + 8 * c.steps <= kWindowLds;
+  const int64_t gemm_tiles = ((int64_t)g.batch * g.out_h * g.out_w + 127) / 128;
+  const int64_t gemm_rounds = gemm_tiles < 128 ? 1 : (gemm_tiles + 511) / 512, slots = two ? 512 : 256, rounds = (c.tiles + slots - 1) / slots;
+  return (float)rounds * (two ? 0.98f : window_blocks(g) == 3 ? 0.75f : 0.9f) < (float)gemm_rounds;
+}
 bool conv_window_weights_wanted(const ConvGeom &g) {
   const int taps = g.kernel_h * g.kernel_w;
   if (g.in_c == 3 || g.in_c == 4)
-    return g.out_c <= 64 && g.kernel_w <= 8 && g.kernel_h <= 16 && g.dilation_w == 1 &&
+    return g.out_c <= 128 && g.kernel_w <= 8 && g.kernel_h <= 16 && g.dilation_w == 1 &&
            g.kernel_h * (g.kernel_w * g.in_c > 16 ? 2 : 1) > 8;
-  return (g.in_c & 15) == 0 && g.out_c <= 64 && taps > 1 && (int64_t)taps * g.in_c <= 2048;
+  return (g.in_c & 15) == 0 && g.out_c <= 128 && taps > 1 && (int64_t)taps * g.in_c <= 2048;
 }
 static bool choose_window(const ConvGeom &g, const void *in, WindowCut *c) {
   const int64_t image = (int64_t)g.in_h * g.in_w * g.in_c;
   if (!conv_window_weights_wanted(g) || g.batch * image < 16 || image >= (int64_t)1 << 31) return false;
   if ((reinterpret_cast<uintptr_t>(in) & 15) != 0 && !packed_window(g)) return false;
-  return cut_window(g, c) && c->tiles >= kWindowLeastTiles && c->tiles < 1 << 23 &&  // (2^32 threads)
+  return cut_window(g, c) && c->tiles >= least_tiles(g) && wide_rounds_pay(g, *c) && c->tiles < 1 << 23 &&  // (2^32 threads)
          c->tiles * (32 * kWaves / 2) <= (int64_t)g.batch * g.out_h * g.out_w;
 }
 
 typedef void (*WindowKernel)(ConvWindow, RequantParams, int8_t *);
 // [blocks of 32 channels - 1][packed][kReluForm]
-static const WindowKernel kWindowKernels[2][2][2] = {
+static const WindowKernel kWindowKernels[4][2][2] = {
     {{conv_window_kernel<1, false, kCarryForm>, conv_window_kernel<1, false, kReluForm>},
      {conv_window_kernel<1, true, kCarryForm>, conv_window_kernel<1, true, kReluForm>}},
     {{conv_window_kernel<2, false, kCarryForm>, conv_window_kernel<2, false, kReluForm>},
-     {conv_window_kernel<2, true, kCarryForm>, conv_window_kernel<2, true, kReluForm>}}};
+     {conv_window_kernel<2, true, kCarryForm>, conv_window_kernel<2, true, kReluForm>}},
+    {{conv_window_kernel<3, false, kCarryForm>, conv_window_kernel<3, false, kReluForm>}, {conv_window_kernel<3, true, kCarryForm>, conv_window_kernel<3, true, kReluForm>}},
+    {{conv_window_kernel<4, false, kCarryForm>, conv_window_kernel<4, false, kReluForm>},
+     {conv_window_kernel<4, true, kCarryForm>, conv_window_kernel<4, true, kReluForm>}}};
 
 // Dynamic LDS beyond 64 KiB has to be announced: cut_window gives all of them up to kWindowLds (packed, 8x8 windows at stride 8
-// take 77 KiB).
+// take 77 KiB) or kWindowLdsWide.
 int conv_window_prepare_device() {
   for (const auto &of_blocks : kWindowKernels)
     for (const auto &of_packed : of_blocks)
       for (const WindowKernel kernel : of_packed)
         MI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         kWindowLds));
+                                         kWindowLdsWide));
   return MI_OK;
 }
 
@@ -341,7 +375,7 @@ int launch_conv_window(const int8_t *in, const ConvGeom &g, const int8_t *fill16
   c.tile_h = t.tile_h, c.tile_w = t.tile_w, c.tiles_x = t.tiles_x, c.tiles_y = t.tiles_y;
   c.patch_h = t.patch_h, c.patch_w = t.patch_w, c.cc = cc, c.pitch = t.pitch, c.steps = t.steps;
   c.weight_bytes = t.weight_bytes, c.patch_bytes = t.patch_bytes;
-  c.streams = conv_streams((int64_t)g.batch * g.out_h * g.out_w, g.out_c, g.out_c > 32 ? 2 : 1);
+  c.streams = conv_streams((int64_t)g.batch * g.out_h * g.out_w, g.out_c, window_blocks(g));
   c.magic_pitch = magic16(t.pitch), c.magic_patch_w = magic16(t.patch_w), c.magic_tile_w = magic16(t.tile_w);
   c.magic_cc = magic16(cc), c.magic_kernel_w = magic16(g.kernel_w), c.magic_quads = magic16(t.patch_w / 4);
   c.w = w, c.fill16 = fill16;
@@ -349,7 +383,7 @@ int launch_conv_window(const int8_t *in, const ConvGeom &g, const int8_t *fill16
   magic31(t.tiles_y, &c.magic_tiles_y, &c.shift_tiles_y);
   const size_t lds = (size_t)t.weight_bytes + t.patch_bytes + 8 * (size_t)t.steps;
   const dim3 grid((unsigned)t.tiles), threads(64 * kWaves);
-  const WindowKernel kernel = kWindowKernels[g.out_c > 32][packed][requant_form(rq) == kReluForm];
+  const WindowKernel kernel = kWindowKernels[window_blocks(g) - 1][packed][requant_form(rq) == kReluForm];
   launch_kernel(kernel, grid, threads, lds, stream, c, rq, out);
   MI_HIP_CHECK(hipGetLastError());
   return MI_OK;

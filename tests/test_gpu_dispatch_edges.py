@@ -138,6 +138,35 @@ def test_first_layer_convolution_long_rows(orc, kernel, ic, oc, h, w, stride, pa
     assert np.array_equal(conv.run(torch.from_numpy(x).cuda()).cpu().numpy(), want)
 
 
+# windows in LDS against 65 to 128 channels: three blocks of 32 and four, the last of them full or not; one image's rectangles short of the
+# rule's least and past it, one round more than the GEMM's; strides, dilations and uneven pads; a rectangle that fills the LDS (64 -> 128, stride 2)
+@pytest.mark.parametrize("b,ih,iw,ic,oc,taps,stride,dil,pad", [
+    (2, 170, 166, 16, 65, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)), (8, 56, 56, 32, 96, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)),
+    (24, 56, 50, 16, 97, (3, 3), (1, 1), (1, 1), (0, 2, 1, 0)), (60, 29, 31, 32, 128, (2, 3), (1, 1), (1, 2), (1, 0, 2, 1)),
+    (50, 56, 56, 64, 128, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1)), (30, 60, 61, 48, 96, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1)),
+    (7, 56, 56, 96, 90, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)), (19, 56, 56, 16, 80, (3, 5), (1, 1), (2, 1), (2, 2, 2, 2)),
+    (2, 224, 224, 3, 96, (7, 7), (2, 2), (1, 1), (3, 3, 3, 3)), (2, 220, 227, 3, 128, (7, 7), (2, 2), (1, 1), (3, 2, 3, 2)),
+    (1, 170, 163, 4, 70, (5, 5), (1, 1), (1, 1), (2, 2, 2, 2)), (2, 113, 120, 3, 101, (9, 3), (1, 1), (2, 1), (4, 4, 1, 1))])
+@pytest.mark.parametrize("act", [K.ACT_NONE, K.ACT_RELU])
+def test_convolution_windows_of_more_channels(orc, b, ih, iw, ic, oc, taps, stride, dil, pad, act):
+    import torch
+    from oracle import pyoracle
+    rng = np.random.default_rng(oc * 100 + ic)
+    w = rng.integers(-128, 128, (oc, *taps, ic), dtype=np.int8)
+    sw = rng.uniform(0.001, 0.01, oc).astype(np.float32).astype(np.float64)
+    bias, zp = rng.integers(-2000, 2001, oc).astype(np.int32), np.zeros(oc, np.int32)
+    x = rng.integers(-128, 128, (b, ih, iw, ic), dtype=np.int8)
+    shape = pyoracle.conv_shape(b, ih, iw, ic, oc, taps, stride, dil, pad)
+    so = float(np.float32(0.02 * 0.0055 * (taps[0] * taps[1] * ic) ** 0.5 * 150))
+    conv = K.ConvolutionInt8Kernel(w, bias, K.QuantParam(0.02, 4), [K.QuantParam(float(s), 0) for s in sw], K.QuantParam(so, -6), stride, dil,
+                                   pad, 1, act, exact_3x3=True)
+    orc.set_threads(16)
+    want = orc.conv_int8(x, w, bias, shape, 0.02, 4, sw, zp, so, -6, act)
+    got = conv.run(torch.from_numpy(x).cuda())
+    assert np.array_equal(got.cpu().numpy(), want)
+    assert torch.equal(conv.run(torch.from_numpy(x).cuda()), got)
+
+
 def _matmul_pair(rng, n, k, asymmetric, dynamic, **kw):
     w = rng.integers(-128, 128, (n, k), dtype=np.int8)
     sw = rng.uniform(0.001, 0.01, n).astype(np.float32).astype(np.float64)
