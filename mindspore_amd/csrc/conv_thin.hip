@@ -23,6 +23,7 @@ typedef v4i v4i_any __attribute__((aligned(1)));
 // and temporal stores of four bytes -> now: 16 x 112 x 112, 192 -> 32 channels 45.2 -> 10.7 -> 10.7, 32 -> 64 - -> 7.0 -> 5.5, 32 -> 128
 // - -> 11.2 -> 8.4, 32 -> 192 21.0 -> 15.6 -> 13.5, 24 -> 72 - -> 8.9 -> 7.7; 8 x 115 x 115, 240 -> 40 26.5 -> 9.4 -> 9.2;
 // 4 x 80 x 80, 72 -> 24 9.0 (in two launches) -> 3.5; one image of 112 x 112, where any launch takes most of it, 192 -> 32 3.7 -> 3.8.
+// G: groups of OCB x 32 channels that a workgroup computes one after the other, see launch_conv_thin.
 struct ConvThin {
   const int8_t *in;
   int64_t in_bytes;
@@ -35,7 +36,7 @@ struct ConvThin {
 };
 static_assert(sizeof(ConvThin) + sizeof(RequantCall) + sizeof(int8_t *) <= kShortArgs, "see launch_args.h");
 
-template <int CH, int OCB, RequantForm FORM, bool NEIGHBOURS = true>
+template <int CH, int OCB, RequantForm FORM, bool NEIGHBOURS = true, int G = 1>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void conv_thin_kernel(ConvThin g, RequantCall call,
                                                                                               int8_t *__restrict__ out) {
   call.load_now();
@@ -43,12 +44,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
   const RequantParams rq = call.open(g.out_c);
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5;
-  const int n0 = blockIdx.y * (32 * OCB);
+  const int n0 = blockIdx.y * (32 * OCB * G);
   const int tiles = (g.pixels + 31) >> 5, step = g.step;
   int tile = blockIdx.x * 4 + (tid >> 6);
   const int steps = g.chunks * CH;
 
-  const ChannelRequant<OCB, FORM, NEIGHBOURS> requant(rq, n0, lane);
+  auto requant_of = [&](int grp) { return ChannelRequant<OCB, FORM, NEIGHBOURS>(rq, n0 + 32 * OCB * grp, lane); };
+  const ChannelRequant<OCB, FORM, NEIGHBOURS> requant[2] = {requant_of(0), requant_of(G - 1)};
 
   int64_t at = 0;  // this lane's first byte of a tile
   auto locate = [&](int tl) {
@@ -70,14 +72,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
     // From [32 channels][step][lane], front to back, into operand order [ob][step][lane], where the channels of a group are columns
     // of its blocks (ChannelRequant).  Fetched in operand order instead, 3 x 206 x 206, 376 -> 152 channels took 32.0 us, this 29.9;
     // 34 x 26 x 26, 336 -> 192 9.5 / 8.8.
-    const int left = (g.out_c - n0 + 31) / 32, have = (left < OCB ? left : OCB) * steps;
+    const int left = (g.out_c - n0 + 31) / 32, have = (left < OCB * G ? left : OCB * G) * steps;
     const v4i *src = reinterpret_cast<const v4i *>(g.w) + (int64_t)(n0 / 32) * steps * 64;
     v4i *dst = reinterpret_cast<v4i *>(lds);
 #pragma unroll 4
     for (int i = __builtin_amdgcn_readfirstlane(tid >> 6); i < have; i += 4) {
-      const int b = i / steps, s = i - b * steps, n = 32 * b + r;
+      const int b = i / steps, s = i - b * steps, grp = b / OCB, n = 32 * (b - grp * OCB) + r;
       const int ob = NEIGHBOURS ? (n >> 2) % OCB : b, column = NEIGHBOURS ? 4 * (n / (4 * OCB)) + (n & 3) : r;
-      dst[(ob * steps + s) * 64 + column + 32 * h] = src[i * 64 + lane];
+      dst[((grp * OCB + ob) * steps + s) * 64 + column + 32 * h] = src[i * 64 + lane];
     }
     __syncthreads();
   }
@@ -92,8 +94,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
     v16i acc[OCB], sums;
 #pragma unroll
     for (int e = 0; e < 16; ++e) sums[e] = 0;
-    auto chunk = [&](int c, auto first_c) {  // the first one starts the accumulators, from one register block for all
-      v4i y[CH];
+    v4i y[CH];
+    auto take = [&](int c) {  // chunk c into y, the one behind it on its way
 #pragma unroll
       for (int s = 0; s < CH; ++s) y[s] = x[s];
       const int64_t over = at + ((c + 1) * CH - 1) * 32 - last;
@@ -113,7 +115,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
         locate(tile + step);
         fetch(x, 0);
       }
-      const char *wl = lds + c * CH * 1024 + lane * 16;
+    };
+    auto products = [&](int c, int grp, auto first_c) {  // the first ones start the accumulators, from one register block for all
+      const char *wl = lds + (grp * OCB * steps + c * CH) * 1024 + lane * 16;
 #pragma unroll
       for (int s = 0; s < CH; ++s)
 #pragma unroll
@@ -133,24 +137,39 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
         }
       }
     };
+    auto chunk = [&](int c, auto first_c) {
+      take(c);
+      products(c, 0, first_c);
+    };
+    const int first = tile * 32, my_p = first + 4 * h + (lane & 3);
+    auto finish = [&](int grp) {
+      wait_for_products(acc);
+      const int g0 = n0 + 32 * OCB * grp, my_n = g0 + column_channel(OCB, 0, r & ~3, NEIGHBOURS);
+      int8_t *dst = out + (int64_t)my_p * g.out_c + my_n;
+      requant[grp].in_form(first + 32 <= g.pixels, g0, my_n, g.out_c, g.streams, [&](auto kind, auto streamed) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          requant[grp].template store<decltype(kind)::value, decltype(streamed)::value>(rq, acc, sums, q, dst + 8 * q * g.out_c,
+                                                                                        my_p + 8 * q < g.pixels ? g.out_c - my_n : 0);
+      });
+    };
     // (One block of channels: few instructions to save, and a launch of so few that fetching the longer code shows:
     //  4 x 80 x 80, 72 -> 24 3.3 us, with the split forms 3.6.  Three blocks: 16 x 112 x 112, 32 -> 192 16.2 us, with them 14.7.)
-    if constexpr (OCB > 1) {
+    if constexpr (G == 2) {  // (a contraction of one chunk)
+      take(0);
+      products(0, 0, std::true_type());
+      finish(0);
+      products(0, 1, std::true_type());
+      finish(1);
+    } else if constexpr (OCB > 1) {
       chunk(0, std::true_type());
       for (int c = 1; c < g.chunks; ++c) chunk(c, std::false_type());
+      finish(0);
     } else {
       acc[0] = start;
       for (int c = 0; c < g.chunks; ++c) chunk(c, std::false_type());
+      finish(0);
     }
-    wait_for_products(acc);
-    const int first = tile * 32, my_n = n0 + column_channel(OCB, 0, r & ~3, NEIGHBOURS), my_p = first + 4 * h + (lane & 3);
-    int8_t *dst = out + (int64_t)my_p * g.out_c + my_n;
-    requant.in_form(first + 32 <= g.pixels, n0, my_n, g.out_c, g.streams, [&](auto kind, auto streamed) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        requant.template store<decltype(kind)::value, decltype(streamed)::value>(rq, acc, sums, q, dst + 8 * q * g.out_c,
-                                                                                  my_p + 8 * q < g.pixels ? g.out_c - my_n : 0);
-    });
   }
 }
 
@@ -203,6 +222,17 @@ std::vector<int8_t> conv_thin_weights(const int8_t *w, int oc, int k) {
 // 12.8 / 11.4; 4 x 112 x 112 8.1 / 7.25; 32 x 28 x 28, 128 -> 256 6.45 / 6.35; but 32 x 56 x 56, 64 -> 128 7.95 / 8.05; 16 x 112 x 112,
 // 32 -> 64 5.65 / 6.5.
 template <int CH, int OCB>
+static int launch_thin_pairs(const ConvThin &c, const RequantParams &rq, int8_t *out, dim3 grid, size_t lds, hipStream_t stream) {
+  if (requant_form(rq) == kReluForm) {
+    launch_kernel((conv_thin_kernel<CH, OCB, kReluForm, true, 2>), grid, dim3(256), lds, stream, c, RequantCall::of(rq), out);
+  } else {
+    launch_kernel((conv_thin_kernel<CH, OCB, kCarryForm, true, 2>), grid, dim3(256), lds, stream, c, RequantCall::of(rq), out);
+  }
+  MI_HIP_CHECK(hipGetLastError());
+  return MI_OK;
+}
+
+template <int CH, int OCB>
 static int launch_thin(const ConvThin &c, const RequantParams &rq, int8_t *out, dim3 grid, size_t lds, hipStream_t stream) {
   const RequantForm form = requant_form(rq);
   if constexpr (OCB == 2) {
@@ -240,13 +270,24 @@ int launch_conv_thin(const int8_t *in, int64_t pixels, int k, int oc, const int8
   // Four or five whole blocks in one workgroup, whose stores then stream.  us, two groups -> this: 16 x 112 x 112, 32 -> 128 11.2 -> 8.9,
   // -> 160 15.3 -> 10.9; 16 x 56 x 56, 128 -> 128 6.0 -> 5.6.  Six (too few waves) 14.7 -> 22, channels short of five 10.4 -> 14.
   const bool rows = form != kGeneralForm && oc == 32 * blocks && blocks > 3 && blocks <= 5 && wgs * blocks > 1024 && t.steps() * blocks <= 64;
-  const int ocb = rows ? blocks : thin_blocks(wgs, oc), groups = (oc + 32 * ocb - 1) / (32 * ocb);
+  const int ocb = rows ? blocks : thin_blocks(wgs, oc);
+  // Two groups one after the other by the same wave, from the same operand registers, where the output is more than the L2s hold: a group's
+  // 64 or 96 bytes of a pixel are parts of lines, of which the other group's workgroups write the rest when the line may have left.  us per
+  // launch into changing memory, a workgroup per group / per pair: 16 x 112 x 112, 32 -> 192 20.9 / 14.1, 32 images 39.2 / 25.2, 24 -> 144
+  // 35.2 / 20.9; image blocks whose expanded image stays in the last-level cache: 32 x 125 x 125, 40 -> 120 (60 MB) 82.3 / 73.5, 24 x 112 x 112
+  // (36 MB) 55.4 / 51.4, 32 x 112 x 112, 24 -> 144 (58 MB) 72.3 / 69.2, 32 -> 192 (77 MB) 79.5 / 78.1, 16 images (38.5 MB) 47.0 / 47.2; outputs
+  // that the L2s hold, with fewer waves at once 8 x 112 x 112, 32 -> 192 9.05 / 9.9, the block 31.7 / 33.8.
+  const bool pairs = form != kGeneralForm && (ocb == 2 || ocb == 3) && (blocks + ocb - 1) / ocb == 2 && t.chunks == 1 &&
+                     pixels * oc > kStreamedMost;
+  const int in_wg = pairs ? 2 * ocb : ocb, groups = (blocks + in_wg - 1) / in_wg;
   // four workgroups per CU, which the LDS allows up to 40 KiB of weights; more would only load the weights more often
   const int most = (1024 + groups - 1) / groups;
   const dim3 grid((unsigned)(wgs < most ? wgs : most), (unsigned)groups);
   const ConvThin c{in, pixels * k, k, t.chunks, oc, (int)pixels, conv_streams(pixels, oc, ocb), 4 * (int)grid.x, w};
-  const size_t lds = (size_t)t.steps() * ocb * 1024;
+  const size_t lds = (size_t)t.steps() * in_wg * 1024;
 #define MI_THIN(CH)                                                              \
+  if (pairs && ocb == 2) return launch_thin_pairs<CH, 2>(c, rq, out, grid, lds, stream); \
+  if (pairs) return launch_thin_pairs<CH, 3>(c, rq, out, grid, lds, stream);     \
   return ocb == 1   ? launch_thin<CH, 1>(c, rq, out, grid, lds, stream)          \
          : ocb == 2 ? launch_thin<CH, 2>(c, rq, out, grid, lds, stream)          \
          : ocb == 3 ? launch_thin<CH, 3>(c, rq, out, grid, lds, stream)          \

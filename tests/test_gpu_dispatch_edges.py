@@ -138,6 +138,31 @@ def test_first_layer_convolution_long_rows(orc, kernel, ic, oc, h, w, stride, pa
     assert np.array_equal(conv.run(torch.from_numpy(x).cuda()).cpu().numpy(), want)
 
 
+# 1x1 into more than 32 MB: both groups of 64 or 96 channels by one wave; whole groups, a last quad, a last byte; one to four steps of K, odd
+# rows, a last tile of pixels that is partly there
+@pytest.mark.parametrize("pixels,k,n", [((17, 103, 115), 24, 192), ((1, 500, 560), 40, 120), ((3, 300, 331), 33, 113), ((1, 479, 501), 100, 144),
+                                        ((2, 401, 299), 128, 161)])
+@pytest.mark.parametrize("act", [K.ACT_NONE, K.ACT_RELU6])
+def test_convolution_1x1_into_large_images(orc, pixels, k, n, act):
+    import torch
+    from oracle import pyoracle
+    rng = np.random.default_rng(n)
+    w = rng.integers(-128, 128, (n, 1, 1, k), dtype=np.int8)
+    sw = rng.uniform(0.001, 0.01, n).astype(np.float32).astype(np.float64)
+    bias, zp = rng.integers(-2000, 2001, n).astype(np.int32), np.zeros(n, np.int32)
+    x = rng.integers(-128, 128, (*pixels, k), dtype=np.int8)
+    assert x.size // k * n > 32 << 20
+    so = float(np.float32(0.02 * 0.0055 * k ** 0.5 * 150))
+    conv = K.ConvolutionInt8Kernel(w, bias, K.QuantParam(0.02, 4), [K.QuantParam(float(s), 0) for s in sw], K.QuantParam(so, -6), (1, 1), (1, 1),
+                                   (0, 0, 0, 0), 1, act, exact_3x3=True)
+    got = conv.run(torch.from_numpy(x).cuda()).cpu().numpy().reshape(-1, n)
+    some = np.unique(np.r_[np.arange(64), rng.integers(0, len(got), 20000), np.arange(len(got) - 64, len(got))])
+    shape = pyoracle.conv_shape(1, 1, some.size, k, n, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0))
+    orc.set_threads(16)
+    want = orc.conv_int8(np.ascontiguousarray(x.reshape(-1, k)[some]).reshape(1, 1, some.size, k), w, bias, shape, 0.02, 4, sw, zp, so, -6, act)
+    assert np.array_equal(got[some], want.reshape(-1, n))
+
+
 # windows in LDS against 65 to 128 channels: three blocks of 32 and four, the last of them full or not; one image's rectangles short of the
 # rule's least and past it, one round more than the GEMM's; strides, dilations and uneven pads; a rectangle that fills the LDS (64 -> 128, stride 2)
 @pytest.mark.parametrize("b,ih,iw,ic,oc,taps,stride,dil,pad", [
