@@ -3,7 +3,7 @@
 
 namespace mi {
 
-typedef v4i v4i_byte __attribute__((aligned(1)));
+typedef v4i v4i_word __attribute__((aligned(4)));
 
 // =====================================================================================================================
 // Small products: many small tiles, and K shared out inside the workgroup.
@@ -14,17 +14,19 @@ typedef v4i v4i_byte __attribute__((aligned(1)));
 // sums in any order are the same sums) and to requantise four channels of a row a lane.  The weights go from the blocked copy straight into
 // operand registers, whole lines an instruction; the activations through an area of LDS that is the wave's own, since operand order from
 // memory would look up 64 lines an instruction.
-// Bound by launch and latency: 3.1 us is what a launch of one K block takes.  us per launch from a graph, ring (or K in parts) -> this:
+// Bound by launch and latency: 3.1 us is what a launch of one K block takes.  us per launch from a graph (K is not in parts there), ring -> this:
 // 128 x 768 x 768 4.10 -> 3.42, 197 x 768 x 768 (fp32) 4.59 -> 3.52, 197 x 2304 x 768 (fp32) 4.79 -> 4.11, 197 x 768 x 3072 (fp32) 7.63 ->
 // 4.78, 256 x 1024 x 1024 4.44 -> 3.73, 300 x 500 x 4096 8.74 -> 5.30; 64 rows, weights from HBM, decode kernel -> this: 4096 x 4096 8.8 ->
 // 7.5, 1024 x 4096 7.9 -> 5.3.  Two K blocks a wave are on their way at a time; three or four gain nothing (128 x 768 x 768 3.47) and
 // let fewer workgroups into a CU (197 x 3072 x 768 4.71 -> 5.86).
 //
 // ANY: rows of any length at any address.  Loads from odd addresses take the address unit about 95 cycles each, so what is fetched are the
-// aligned 16-byte chunks that a row's bytes lie in, nine for 128 bytes, and LDS is read at the odd address.  A chunk may hold up to 15 bytes
-// in front of the tensor or behind it: in memory they share its 16 bytes and so its page, in the products they meet zero weights, and the row
-// sums leave them out.  333 x 1001 x 1000 with weight zero points 5.6 (gemm_anyrow.hip) -> 4.9, 100 x 500 x 500 4.27 -> 3.49,
-// 200 x 1000 x 1500 6.30 -> 4.76, 70 x 64 x 1003 5.81 -> 4.00.
+// aligned 16-byte chunks that a row's bytes lie in, nine for 128 bytes, and the row comes into place on its way out of LDS: five dwords from
+// the word it starts in and a byte shift (fragments read at odd addresses kept LDS busy for 14 cycles each, 3000 a CU at the first of the
+// following).  A chunk may hold up to 15 bytes in front of the tensor or behind it: in memory they share its 16 bytes and so its page, in
+// the products they meet zero weights (or lie in front of the row), and the row sums leave them out.  333 x 1001 x 1000 with weight zero
+// points 5.6 (gemm_anyrow.hip) -> 4.9 (odd reads) -> 4.75, 200 x 1000 x 1501 6.3 -> 4.84 -> 4.46, 90 x 700 x 3001 - -> 5.9 -> 5.1, 70 x 64 x 1003
+// 5.81 -> 4.00 -> 3.75, 100 x 500 x 501 4.27 -> 3.50 -> 3.33.
 // =====================================================================================================================
 template <int WAVES, int TN, int EPI, bool HAS_ZW, bool ANY>
 __device__ __forceinline__ void gemm_short_body(const GemmArgs &g, const RequantParams &rq, const DequantParams &dq) {
@@ -124,7 +126,8 @@ __device__ __forceinline__ void gemm_short_body(const GemmArgs &g, const Requant
   for (int i = 0; i < TN; ++i)
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[i][e] = wave == 0 ? (int)kAccBias : 0;
-  const char *const row = mine + r * PITCH + (ANY ? (skew + min(r, rows - 1) * (int)g.lda) & 15 : 0);
+  const uint32_t odd = ANY ? (uint32_t)(skew + min(r, rows - 1) * (int)g.lda) & 15 : 0;  // where in its first chunk the lane's row starts
+  const char *const row = mine + r * PITCH + (odd & ~3u);
   for (int b = first; b == first || b < end; b += D) {
 #pragma unroll
     for (int s = 0; s < D; ++s) {
@@ -148,7 +151,11 @@ __device__ __forceinline__ void gemm_short_body(const GemmArgs &g, const Requant
 #pragma unroll
         for (int f = 0; f < 4; ++f) {
           if constexpr (ANY) {
-            a[f] = *reinterpret_cast<const v4i_byte *>(row + s * SLOT + 32 * f + 16 * h);
+            const char *at = row + s * SLOT + 32 * f + 16 * h;
+            const v4i v = *reinterpret_cast<const v4i_word *>(at);
+            const uint32_t next = *reinterpret_cast<const uint32_t *>(at + 16);
+#pragma unroll
+            for (int d = 0; d < 4; ++d) a[f][d] = (int)__builtin_amdgcn_alignbyte(d < 3 ? (uint32_t)v[(d + 1) & 3] : next, (uint32_t)v[d], odd & 3);
           } else {
             a[f] = *reinterpret_cast<const v4i *>(row + s * SLOT + (((2 * f + h) ^ ((r >> 1) & 7)) << 4));
           }
