@@ -1,5 +1,6 @@
 // int8 GEMM on the matrix cores, tiles of 32 rows whose K the waves of a workgroup share (gemm_i8.hip says which shapes come here).
 #include "gemm_core.h"
+#include "row_chunks.h"
 
 namespace mi {
 
@@ -62,27 +63,20 @@ __device__ __forceinline__ void gemm_short_body(const GemmArgs &g, const Requant
   // gemm_kblock_body.  Any rows: the nine aligned chunks that a row's 128 bytes lie in.
   const int last = blocks - 1;
   const int8_t *const a_tile = g.a + (int64_t)m0 * g.lda;
-  const int skew = ANY ? (int)(reinterpret_cast<uintptr_t>(a_tile) & 15) : 0, rows = min(g.m - m0, 32);
-  const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(a_tile) - skew, (short)0, -1, 0x00020000);
+  const int rows = min(g.m - m0, 32);
+  const RowChunks ragged(reinterpret_cast<uintptr_t>(a_tile), g.m - m0, g.k);
+  const __amdgpu_buffer_rsrc_t a_rsrc =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(a_tile) - (ANY ? ragged.skew : 0), (short)0, -1, 0x00020000);
   int a_off[LOADS];
 #pragma unroll
-  for (int i = 0; i < LOADS; ++i) {
-    if constexpr (ANY) {
-      const int id = min(i * 64 + lane, 32 * 9 - 1), row = id * 57 >> 9;  // id / 9
-      a_off[i] = ((skew + min(row, rows - 1) * (int)g.lda) & ~15) + (id - 9 * row) * 16;
-    } else {
-      a_off[i] = min(8 * i + (lane >> 3), rows - 1) * (int)g.lda + (((lane & 7) ^ (lane >> 4) ^ ((i & 1) << 2)) << 4);
-    }
-  }
-  // the last chunk with a byte of the tensor in it, where a tile reaches that far
-  const int a_end = m0 + 32 >= g.m ? (skew + (rows - 1) * (int)g.lda + g.k - 1) & ~15 : 0x7fffffff;
+  for (int i = 0; i < LOADS; ++i)
+    a_off[i] = ANY ? ragged.first(i * 64 + lane)
+                   : min(8 * i + (lane >> 3), rows - 1) * (int)g.lda + (((lane & 7) ^ (lane >> 4) ^ ((i & 1) << 2)) << 4);
   auto load_a = [&](int s, int kb) {
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
-      int off = a_off[i] + kb * KB;
-      if (ANY) {
-        off = min(off, a_end);
-      } else if (kb == last) {  // (a chunk past K: the row's last one again)
+      int off = ANY ? ragged.of_block(a_off[i], kb) : a_off[i] + kb * KB;
+      if (!ANY && kb == last) {  // (a chunk past K: the row's last one again)
         const int at = ((lane & 7) ^ (lane >> 4) ^ ((i & 1) << 2)) << 4;
         off += min(g.k - 16 - last * KB - at, 0);
       }
@@ -126,7 +120,7 @@ __device__ __forceinline__ void gemm_short_body(const GemmArgs &g, const Requant
   for (int i = 0; i < TN; ++i)
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[i][e] = wave == 0 ? (int)kAccBias : 0;
-  const uint32_t odd = ANY ? (uint32_t)(skew + min(r, rows - 1) * (int)g.lda) & 15 : 0;  // where in its first chunk the lane's row starts
+  const uint32_t odd = ANY ? ragged.odd(r) : 0;
   const char *const row = mine + r * PITCH + (odd & ~3u);
   for (int b = first; b == first || b < end; b += D) {
 #pragma unroll
