@@ -445,7 +445,7 @@ static ShortTile short_tile(int m, int k, int n, bool requant) {
   return wide <= 256 && kb <= 64 ? ShortTile{82, cost(8, wide, 1.9f, 1.65f, 0.073f, 1.03f)} : ShortTile{0, 0};
 }
 // From K = 4096 on, more rows than the decode kernels take stay with K in parts (gemm_split.hip) on the streams that have memory for
-// that: its tests hold it to them.  150 x 1000 x 4096 7.7 us in parts, 5.3 here.
+// that: its tests hold it to them.  128 x 1024 x 4096 7.7 us in parts, 5.3 here.
 static bool short_goes_first(int m, int k) { return m <= kGemvMaxRows || k < 4096; }
 
 // (the K-block loaders address activation rows with 32-bit offsets from the tile's first row)
