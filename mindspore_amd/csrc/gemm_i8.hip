@@ -424,8 +424,9 @@ static const SplitCost *choose_split(int m, int k, int n, const TileCost &whole,
 // 33 x 1024 x 4096 7.05 / 5.2, 65 x 3072 x 1024 (288 tiles of 32 x 32, 144 of 64 x 32) 4.65 / 4.20, 128 x 4096 x 4096 (256 of 64 x 32) 9.9 / 8.9,
 // 1000 x 500 x 256 3.69 / 3.45 (512), 700 x 1024 x 512 (fp32) 4.8 / 4.24 (704); not taken: 160 x 3072 x 768 4.20 / 4.34 (480), 333 x 1536 x 512
 // 3.97 / 4.06 (528), 512 x 768 x 128 3.17 / 3.38, 200 x 3072 x 1024 4.47 / 5.24 (336 of 64 x 32: 6.7), 200 x 4096 x 4096 10.1 / 14.6 (448 of 64 x 32),
-// 65 x 4096 x 11008 18.5 / 18.8, and up to 32 rows, which the decode kernels read long K for with 16 channels a workgroup, 8 x 768 x 3072
-// 3.62 / 4.51, 32 x 4096 x 4096 6.7 / 7.6 (16 x 768 x 768 4.02 / 3.38).
+// 65 x 4096 x 11008 18.5 / 18.8.  Up to 32 rows, which the decode kernels read long K for with 16 channels a workgroup: 16 x 768 x 768 4.02 /
+// 3.38, 16 x 5000 x 768 4.95 / 3.41, 32 x 8192 x 1024 5.42 / 3.73, 16 x 7000 x 1536 5.42 / 4.42, 32 x 24000 x 768 (750 tiles) 10.1 / 6.1; not
+// taken: 8 x 768 x 3072 3.62 / 4.51, 32 x 4096 x 4096 6.7 / 7.6, 16 x 8192 x 1536 (256) 4.72 / 4.92, 16 x 12288 x 1024 (384) 4.52 / 5.16.
 struct ShortTile {
   int tile;  // as launch_gemm_short has it
   float cost;
@@ -439,7 +440,7 @@ static ShortTile short_tile(int m, int k, int n, bool requant) {
     return a + pass * (float)((kb + 2 * waves - 1) / (2 * waves)) + a_cu * (block * (float)kb + tile);
   };
   const auto four = [&] { return ShortTile{41, cost(4, small, 2.55f, 0.54f, 0.06f, 0.22f)}; };
-  if (m <= kGemvGroupMaxRows) return kb <= 12 && small <= 128 ? four() : ShortTile{0, 0};
+  if (m <= kGemvGroupMaxRows) return kb <= 12 && small <= (kb <= 6 ? 768 : kb <= 8 || m > 16 ? 256 : 224) ? four() : ShortTile{0, 0};
   if (small <= 256) return kb <= 12 ? four() : ShortTile{81, cost(8, small, 2.3f, 0.93f, 0.053f, 0.55f)};
   if (kb < 7) return small <= (!requant ? 768 : kb == 2 ? 256 : kb < 6 ? 512 : 448) ? four() : ShortTile{0, 0};
   return wide <= 256 && kb <= 64 ? ShortTile{82, cost(8, wide, 1.9f, 1.65f, 0.073f, 1.03f)} : ShortTile{0, 0};

@@ -367,7 +367,8 @@ def test_matmul_group_of_one_on_few_ragged_rows(m, k, n, copies, how):
 # are partly there
 @pytest.mark.parametrize("m,n,k", [(3, 1, 129), (32, 31, 144), (33, 65, 255), (64, 4095, 256), (65, 2700, 257), (95, 96, 1535), (97, 33, 1537),
                                    (64, 100, 1536), (40, 4096, 1552), (130, 1600, 1040), (257, 1793, 897), (256, 2048, 896), (129, 2, 4095),
-                                   (70, 300, 4080), (60, 700, 4113), (500, 520, 300), (33, 1001, 9001)])
+                                   (70, 300, 4080), (60, 700, 4113), (500, 520, 300), (33, 1001, 9001),
+                                   (4, 24576, 768), (16, 8192, 1024), (17, 8193, 1024), (16, 7168, 1536), (32, 8192, 1536)])
 @pytest.mark.parametrize("dynamic,asymmetric", [(False, False), (False, True), (True, False), (True, True)])
 def test_matmul_small_products(orc, m, n, k, dynamic, asymmetric):
     """Against the oracle, bit by bit (integer sums, then a fixed sequence of rounded steps): rows at an aligned and at an odd address,
