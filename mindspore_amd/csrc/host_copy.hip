@@ -6,7 +6,7 @@
 // kernel (a copy engine costs an event and its interrupt per chunk, 20 us; a launch costs 4), and what the host waits for is a
 // word per part in the page-locked memory, written behind the part's bytes.
 // MatMuls on host tensors, rows x K x N int8, us per call, hipMemcpy -> slots: 1024 x 4096 x 4096 412 -> 262,
-// 2048 x 4096 x 4096 770 -> 555, 1000 x 256 x 4096 258 -> 150, 256 x 4096 x 1024 97 -> 70, 16 x 4096 x 4096 43 -> 25,
+// 2048 x 4096 x 4096 770 -> 511 to 555, 1000 x 256 x 4096 258 -> 150, 256 x 4096 x 1024 97 -> 70, 16 x 4096 x 4096 43 -> 25,
 // 1 x 1024 x 1024 28.5 -> 17.  What is left is the bus, in and out one after the other.  slot_pool.h says which calls have slots.
 // A copy in need not wait for the copy before it, which is of other bytes into another place, and starts while that still runs: one behind
 // the other they leave the bus idle for the way to the host and back and the end of a launch, 2.5 us a chunk.  1024 x 4096 x 4096 262 -> 249,
@@ -17,6 +17,7 @@
 #include <new>
 
 #include "common.h"
+#include "flag_wait.h"
 #include "slot_pool.h"
 
 namespace mi {
@@ -105,8 +106,12 @@ struct Chunks {
   int first_flag(int slot) const { return slot * wgs(chunk); }
 };
 
-// A copy that may start before the launches in front of it are over (where the runtime does not know of that, behind them).  Whatever
-// is launched the ordinary way behind it waits for it.
+// A copy that may start before the launches in front of it are over.  hip_ext.h says of hipExtModuleLaunchKernel that GFX9 boards do not
+// support the flag, and nothing of it for this call; here it is a hint.  With it as without, results hang on this alone: what is launched
+// the ordinary way waits for everything launched before it on its stream, so a run, and through it the copies out, come behind all copies
+// in; nobody else uses a copy's bytes at either end meanwhile (the slot is filled before the launch and again after its flags, the device's
+// buffer is read by the run behind it, and the call before ended with its own run over).  No copy waits for another, and a later one
+// may be over first: await_flags and drain() know that.
 void launch_beside(const v4i *from, v4i *to, int n16, int parts, uint32_t *flags, uint32_t ticket) {
   void *list[] = {&from, &to, &n16, &parts, &flags, &ticket};
   (void)hipExtLaunchKernel(reinterpret_cast<const void *>(&host_copy_kernel<false>), dim3(parts), dim3(256), list, 0, nullptr, nullptr,
@@ -135,29 +140,37 @@ int launch_chunks(HostSlots *s, const Chunks &c, int64_t i, int n, char *dev, bo
   return MI_OK;
 }
 
-// Until every workgroup that copies chunk i has said that it is done.  (The host spins, as hipMemcpy does: 1024 x 4096 x 4096 264 us
-// of a core per call, with hipMemcpy 423.)
-int await_chunk(HostSlots *s, const Chunks &c, int64_t i) {
-  const int slot = c.slot(i), wgs = c.wgs(c.size(i));
-  if (s->pending[slot] == 0) return MI_OK;
-  const uint32_t *flags = s->flags + c.first_flag(slot);
-  for (int w = 0, spins = 0; w < wgs;) {
-    if (__atomic_load_n(flags + w, __ATOMIC_ACQUIRE) == s->pending[slot]) {
-      ++w;
-    } else if ((++spins & 0x3fff) != 0) {
-      __builtin_ia32_pause();
-    } else {  // now and then: is the stream still at it?
-      const hipError_t e = hipStreamQuery(nullptr);
-      if (e == hipErrorNotReady) continue;
-      MI_HIP_CHECK(e);
-      if (__atomic_load_n(flags + w, __ATOMIC_ACQUIRE) != s->pending[slot]) {
-        set_error("a copy between host and device ended without its result");
-        return MI_ERROR;
-      }
-    }
+// Until nothing that the null stream was given is under way: behind a launch of nothing the ordinary way, which waits for all copies.
+hipError_t drain() {
+  launch_kernel((host_copy_kernel<false>), dim3(1), dim3(256), 0, nullptr, nullptr, nullptr, 0, 1, nullptr, 0u);
+  const hipError_t launched = hipGetLastError(), over = hipStreamSynchronize(nullptr);
+  return launched != hipSuccess ? launched : over;
+}
+
+struct NullStream {  // as await_flags takes it
+  int idle(bool *idle) {
+    const hipError_t e = hipStreamQuery(nullptr);
+    *idle = e == hipSuccess;
+    if (e != hipErrorNotReady) MI_HIP_CHECK(e);
+    return MI_OK;
   }
-  s->pending[slot] = 0;
-  return MI_OK;
+  int drain() {
+    MI_HIP_CHECK(mi::drain());
+    return MI_OK;
+  }
+};
+
+// Until every workgroup that copies chunk i has said that it is done.
+int await_chunk(HostSlots *s, const Chunks &c, int64_t i) {
+  const int slot = c.slot(i);
+  if (s->pending[slot] == 0) return MI_OK;
+  const int rc = await_flags(s->flags + c.first_flag(slot), c.wgs(c.size(i)), s->pending[slot], NullStream());
+  if (rc == kFlagMissing) {
+    set_error("a copy between host and device ended without its result");
+    return MI_ERROR;
+  }
+  if (rc == MI_OK) s->pending[slot] = 0;
+  return rc;
 }
 
 // Page-locked memory, and anything else that the runtime knows, is hipMemcpy's: it needs no slots.
@@ -181,10 +194,7 @@ HostCopies::~HostCopies() {
   if (slots_ == nullptr) return;
   bool busy = false;  // (after an error: whoever has the slots next must not meet this call's copies)
   for (int i = 0; i < kMostSlots; ++i) busy = busy || slots_->pending[i] != 0;
-  if (busy) {  // (behind a launch of nothing, which waits for all copies: the last of them need not be the last to end)
-    launch_kernel((host_copy_kernel<false>), dim3(1), dim3(256), 0, nullptr, nullptr, nullptr, 0, 1, nullptr, 0u);
-    (void)hipStreamSynchronize(nullptr);
-  }
+  if (busy) (void)drain();
   for (int i = 0; i < kMostSlots; ++i) slots_->pending[i] = 0;
   g_pool.give(size_, slots_);
 }
