@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "../../include/mi355x_int8.h"
+#include "conv_geom.h"
 
 namespace mi {
 
@@ -239,10 +240,6 @@ int launch_block_weights(const int8_t *w, int n_pad, int k_pad, int ldw, int8_t 
 // Copies [rows][k] (row stride src_ld bytes) into a zero-padded [rows][k16] buffer, k16 = round_up(k, 16).
 int launch_pad_rows(const int8_t *src, int64_t src_ld, int rows, int k, int8_t *dst, int k16, hipStream_t stream);
 
-struct ConvGeom {
-  int batch, in_h, in_w, in_c, out_h, out_w, out_c;
-  int kernel_h, kernel_w, stride_h, stride_w, dilation_h, dilation_w, pad_u, pad_l;
-};
 // im2col into [batch*out_h*out_w][k16] with K order (kh, kw, ic); out-of-image taps are `fill`, the K tail is zero.
 int launch_im2col(const int8_t *in, const ConvGeom &g, int fill, int8_t *dst, int k16, hipStream_t stream);
 // Dense convolution with kernel_h * kernel_w * in_c <= 64 and out_c <= 128, out_c % 4 == 0, straight from the image
