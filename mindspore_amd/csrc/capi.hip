@@ -1253,8 +1253,14 @@ static int mi_conv_create_impl(const mi_conv_desc *d, const int8_t *weight_host,
     } else if (rc == MI_OK && h->direct_1x1 && conv_thin_supported(kdim, oc)) {
       rc = upload(&h->w_thin, conv_thin_weights(weight_host, oc, kdim));
     }
-    if (rc == MI_OK && conv_window_weights_wanted(shape) && h->st.fast2 && !h->st.has_zw)
+    if (rc == MI_OK && conv_window_weights_wanted(shape) && h->st.fast2 && !h->st.has_zw) {
+      // (an optimisation: without it images run on the kernels that read the other forms)
       rc = upload(&h->w_window, conv_window_weights(shape, weight_host));
+      if (rc == MI_MEMORY_FAILED) {
+        set_error("");
+        rc = MI_OK;
+      }
+    }
     if (rc == MI_OK) rc = upload(&h->fill16, std::vector<int8_t>(16, (int8_t)h->fill));
   }
   if (rc != MI_OK) {

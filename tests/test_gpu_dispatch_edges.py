@@ -192,6 +192,33 @@ def test_convolution_windows_of_more_channels(orc, b, ih, iw, ic, oc, taps, stri
     assert torch.equal(conv.run(torch.from_numpy(x).cuda()), got)
 
 
+@pytest.mark.parametrize("ic,oc,stride", [(64, 64, 1), (32, 96, 1), (64, 128, 2)])
+def test_convolution_without_memory_for_its_window_weights(orc, ic, oc, stride):
+    """They are a second copy: the handle is created without, and images run on the kernels that read the others."""
+    import torch
+    from mindspore_amd import lib
+    from oracle import pyoracle
+    rng = np.random.default_rng(oc)
+    w = rng.integers(-128, 128, (oc, 3, 3, ic), dtype=np.int8)
+    sw = rng.uniform(0.001, 0.01, oc).astype(np.float32).astype(np.float64)
+    bias, zp = rng.integers(-2000, 2001, oc).astype(np.int32), np.zeros(oc, np.int32)
+    x = rng.integers(-128, 128, (48, 56, 56, ic), dtype=np.int8)
+    so = float(np.float32(0.02 * 0.0055 * (9 * ic) ** 0.5 * 150))
+    make = lambda: K.ConvolutionInt8Kernel(w, bias, K.QuantParam(0.02, 4), [K.QuantParam(float(s), 0) for s in sw], K.QuantParam(so, -6),
+                                           (stride, stride), (1, 1), (1, 1, 1, 1), 1, K.ACT_NONE, exact_3x3=True)
+    L = lib.init(0)
+    assert L.mi_debug_fail_alloc((oc + 31) // 32 * (9 * ic // 32) * 1024 + 16) == 0
+    try:
+        conv = make()
+    finally:
+        L.mi_debug_fail_alloc(0)
+    orc.set_threads(16)
+    want = orc.conv_int8(x, w, bias, pyoracle.conv_shape(48, 56, 56, ic, oc, (3, 3), (stride, stride), (1, 1), (1, 1, 1, 1)),
+                         0.02, 4, sw, zp, so, -6, K.ACT_NONE)
+    for c in (conv, make()):
+        assert np.array_equal(c.run(torch.from_numpy(x).cuda()).cpu().numpy(), want)
+
+
 def _matmul_pair(rng, n, k, asymmetric, dynamic, **kw):
     w = rng.integers(-128, 128, (n, k), dtype=np.int8)
     sw = rng.uniform(0.001, 0.01, n).astype(np.float32).astype(np.float64)
