@@ -679,8 +679,8 @@ int launch_gemm_split(int tile, int parts, bool requant, bool has_zw, bool fast,
 int launch_gemm_anyrow(bool requant, bool has_zw, bool fast, const GemmArgs &g, const RequantParams &rq, const DequantParams &dq,
                        hipStream_t stream);
 // 32 x 32 tiles, or 64 channels x 32 rows, the K blocks dealt to the waves of a workgroup (gemm_short.hip).  tile: 10 x waves + blocks of 32
-// channels, 41, 81 or 82; any: rows of any length, stride and address, g.k: bytes of K.  int8 output only in the fast2 form, fp32 never with
-// non-temporal stores.
+// channels, 41, 81 or 82; any: rows of any length at any address, end to end (lda == k), g.k: bytes of K.  int8 output only in the fast2
+// form, fp32 never with non-temporal stores.
 int launch_gemm_short(int tile, bool any, bool requant, bool has_zw, const GemmArgs &g, const RequantParams &rq, const DequantParams &dq,
                       hipStream_t stream);
 // The same for a group whose members have blocked weights without zero points (and, for int8 output, the fast2 form).

@@ -300,6 +300,10 @@ int launch_gemm_short(int tile, bool any, bool requant, bool has_zw, const GemmA
     set_error("gemm: the blocked weight copy is missing");
     return MI_NULL_PTR;
   }
+  if (any && g.lda != g.k) {  // (RowChunks)
+    set_error("gemm: rows of %d bytes %lld apart", g.k, (long long)g.lda);
+    return MI_PARAM_INVALID;
+  }
   return any ? with_tile<true>(tile, requant, has_zw, g, rq, dq, stream) : with_tile<false>(tile, requant, has_zw, g, rq, dq, stream);
 }
 

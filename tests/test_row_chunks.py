@@ -1,7 +1,12 @@
 """The addresses at which gemm_short.hip reads activation rows of any length (mindspore_amd/csrc/row_chunks.h, compiled for the host): every
 chunk it fetches has a byte of the tensor in it, and every byte inside K that a lane takes out of LDS is its row's."""
 import os
+import shutil
 import subprocess
+
+import pytest
+
+from mindspore_amd import build
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -51,5 +56,35 @@ def test_row_chunks_have_bytes_of_the_tensor(tmp_path):
     src, exe = tmp_path / "chunks.cc", tmp_path / "chunks"
     src.write_text(PROGRAM)
     subprocess.check_call(["g++", "-std=c++17", "-O2", "-Wall", "-I" + ROOT, str(src), "-o", str(exe)])
+    p = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert p.returncode == 0, p.stdout
+
+
+STRIDED = r"""
+#include <stdio.h>
+#include "gemm_core.h"
+
+int main() {
+  int8_t byte = 0;
+  mi::GemmArgs g{};
+  g.a = g.wb = &byte, g.c = &byte;
+  g.m = 40, g.n = 64, g.k = 257, g.k_pad = 512, g.lda = 272, g.ldc = 64;
+  for (int tile : {41, 81, 82})
+    for (int requant = 0; requant < 2; ++requant) {
+      const int rc = mi::launch_gemm_short(tile, true, requant != 0, false, g, mi::RequantParams{}, mi::DequantParams{}, nullptr);
+      if (rc != MI_PARAM_INVALID) return printf("tile %d: status %d\n", tile, rc), 1;
+    }
+  return 0;
+}
+"""
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="no compiler for the device's headers")
+def test_rows_with_gaps_between_them_are_refused(tmp_path):
+    """The chunks are those of rows end to end: others are refused before anything is launched."""
+    src, exe = tmp_path / "strided.hip", tmp_path / "strided"
+    src.write_text(STRIDED)
+    subprocess.check_call(["hipcc", "--offload-host-only", "-std=c++17", "-I" + build.CSRC, str(src), "-o", str(exe), "-L" + build.HERE, "-lmi355x_int8",
+                           "-Wl,-rpath," + build.HERE], stderr=subprocess.DEVNULL)
     p = subprocess.run([str(exe)], capture_output=True, text=True)
     assert p.returncode == 0, p.stdout
