@@ -61,6 +61,8 @@ int64_t mi_debug_sync_count(void);
 /* Test aid: how many MatMuls the calling thread has launched with their K split over workgroups, and, where asked for, the
  * tile (10 x channels / 64 + rows / 64) and the number of parts of the last one. */
 int64_t mi_debug_split_launches(int32_t *tile, int32_t *parts);
+/* Test aid: the symbol of the kernel that the calling thread launched last, "" before the first. */
+const char *mi_debug_last_kernel(void);
 const char *mi_version(void);
 
 /* ---- quant-parameter derivation (host arithmetic, no GPU needed) -------------------------------------------- */

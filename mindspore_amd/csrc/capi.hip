@@ -789,6 +789,11 @@ int64_t mi_debug_split_launches(int32_t *tile, int32_t *parts) {
   return t_split_launches.count;
 }
 
+const char *mi_debug_last_kernel(void) {
+  const char *name = t_last_kernel != nullptr ? hipKernelNameRefByPtr(t_last_kernel, nullptr) : nullptr;
+  return name != nullptr ? name : "";
+}
+
 int mi_stream_create(void **out_stream) {
   if (out_stream == nullptr) return MI_NULL_PTR;
   *out_stream = nullptr;

@@ -12,7 +12,7 @@ MI_OK, MI_ERROR, MI_NULL_PTR, MI_PARAM_INVALID, MI_MEMORY_FAILED, MI_NOT_SUPPORT
 ACT_NONE, ACT_RELU, ACT_RELU6 = 0, 1, 3
 
 EXPORTS = [
-    "mi_init", "mi_last_error", "mi_debug_fail_alloc", "mi_debug_sync_count", "mi_debug_split_launches", "mi_version", "mi_quantize_multiplier", "mi_quantize_multiplier_single", "mi_activation_range", "mi_requant_params",
+    "mi_init", "mi_last_error", "mi_debug_fail_alloc", "mi_debug_sync_count", "mi_debug_split_launches", "mi_debug_last_kernel", "mi_version", "mi_quantize_multiplier", "mi_quantize_multiplier_single", "mi_activation_range", "mi_requant_params",
     "mi_multiply_by_quantized_multiplier",
     "mi_matmul_create", "mi_matmul_reserve", "mi_matmul_run", "mi_matmul_run_noalloc", "mi_matmul_run_host", "mi_matmul_run_group", "mi_matmul_run_batched", "mi_matmul_broadcast_offsets", "mi_matmul_get_params", "mi_matmul_destroy",
     "mi_conv_create", "mi_conv_out_shape", "mi_conv_same_pad", "mi_conv_run", "mi_conv_run_host", "mi_conv_reserve", "mi_conv_destroy",
@@ -168,6 +168,7 @@ def load():
     L.mi_debug_sync_count.restype = C.c_int64
     L.mi_debug_split_launches.argtypes = [pi32, pi32]
     L.mi_debug_split_launches.restype = C.c_int64
+    L.mi_debug_last_kernel.restype = C.c_char_p
     L.mi_stream_synchronize.argtypes = [vp]
     L.mi_stream_create.argtypes = [C.POINTER(vp)]
     L.mi_stream_destroy.argtypes = [vp]

@@ -1,11 +1,20 @@
 """Sizes at the edges of the rules by which the library picks a kernel: the last size of one variant and the first of
 the next, remainders, misaligned operands.  Full-tensor, bit-exact comparisons with the oracle."""
+import re
+
 import numpy as np
 import pytest
 
 from mindspore_amd import kernels as K
 
 pytestmark = pytest.mark.gpu
+
+
+def _last_kernel():
+    """What this thread launched last: the kernel's name and its template's arguments."""
+    symbol = K._lib.load().mi_debug_last_kernel().decode()
+    length, rest = re.match(r"_ZN2mi(\d+)(.*)", symbol).groups()
+    return rest[:int(length)], [int(v) for v in re.findall(r"L(?:[a-z]|NS_\d+[A-Za-z]+E)(\d+)E", rest[int(length):])]
 
 
 def _values(rng, n):
@@ -138,10 +147,11 @@ def test_first_layer_convolution_long_rows(orc, kernel, ic, oc, h, w, stride, pa
     assert np.array_equal(conv.run(torch.from_numpy(x).cuda()).cpu().numpy(), want)
 
 
-# 1x1 into more than 32 MB: both groups of 64 or 96 channels by one wave; whole groups, a last quad, a last byte; one to four steps of K, odd
-# rows, a last tile of pixels that is partly there
+# 1x1 into more than 32 MB: both groups of 64 or 96 channels by one wave; whole groups, a last quad, a last byte; one to four steps of K, each
+# with both kinds of group, odd rows, a last tile of pixels that is partly there
 @pytest.mark.parametrize("pixels,k,n", [((17, 103, 115), 24, 192), ((1, 500, 560), 40, 120), ((3, 300, 331), 33, 113), ((1, 479, 501), 100, 144),
-                                        ((2, 401, 299), 128, 161)])
+                                        ((2, 401, 299), 128, 161), ((1, 539, 541), 20, 116), ((2, 311, 301), 48, 180), ((1, 571, 569), 72, 104),
+                                        ((3, 257, 233), 96, 192), ((1, 523, 523), 120, 125)])
 @pytest.mark.parametrize("act", [K.ACT_NONE, K.ACT_RELU6])
 def test_convolution_1x1_into_large_images(orc, pixels, k, n, act):
     import torch
@@ -156,6 +166,8 @@ def test_convolution_1x1_into_large_images(orc, pixels, k, n, act):
     conv = K.ConvolutionInt8Kernel(w, bias, K.QuantParam(0.02, 4), [K.QuantParam(float(s), 0) for s in sw], K.QuantParam(so, -6), (1, 1), (1, 1),
                                    (0, 0, 0, 0), 1, act, exact_3x3=True)
     got = conv.run(torch.from_numpy(x).cuda()).cpu().numpy().reshape(-1, n)
+    kernel, form = _last_kernel()
+    assert kernel == "conv_thin_kernel" and form[:2] + form[3:] == [(k + 31) // 32, 3 if n > 128 else 2, 1, 2]
     some = np.unique(np.r_[np.arange(64), rng.integers(0, len(got), 20000), np.arange(len(got) - 64, len(got))])
     shape = pyoracle.conv_shape(1, 1, some.size, k, n, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0))
     orc.set_threads(16)
@@ -163,17 +175,21 @@ def test_convolution_1x1_into_large_images(orc, pixels, k, n, act):
     assert np.array_equal(got[some], want.reshape(-1, n))
 
 
-# windows in LDS against 65 to 128 channels: three blocks of 32 and four, the last of them full or not; one image's rectangles short of the
-# rule's least and past it, one round more than the GEMM's; strides, dilations and uneven pads; a rectangle that fills the LDS (64 -> 128, stride 2)
-@pytest.mark.parametrize("b,ih,iw,ic,oc,taps,stride,dil,pad", [
-    (2, 170, 166, 16, 65, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)), (8, 56, 56, 32, 96, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)),
-    (24, 56, 50, 16, 97, (3, 3), (1, 1), (1, 1), (0, 2, 1, 0)), (60, 29, 31, 32, 128, (2, 3), (1, 1), (1, 2), (1, 0, 2, 1)),
-    (50, 56, 56, 64, 128, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1)), (30, 60, 61, 48, 96, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1)),
-    (7, 56, 56, 96, 90, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)), (19, 56, 56, 16, 80, (3, 5), (1, 1), (2, 1), (2, 2, 2, 2)),
-    (2, 224, 224, 3, 96, (7, 7), (2, 2), (1, 1), (3, 3, 3, 3)), (2, 220, 227, 3, 128, (7, 7), (2, 2), (1, 1), (3, 2, 3, 2)),
-    (1, 170, 163, 4, 70, (5, 5), (1, 1), (1, 1), (2, 2, 2, 2)), (2, 113, 120, 3, 101, (9, 3), (1, 1), (2, 1), (4, 4, 1, 1))])
+# windows in LDS against 65 to 128 channels: three blocks of 32 and four, the last of them full or not; strides, dilations and uneven pads; a
+# rectangle that fills the LDS (64 -> 128, stride 2).  Not on windows: fewer rectangles than the rule's least, and one round more than the GEMM's,
+# of three blocks and of four; few rectangles of a first layer
+@pytest.mark.parametrize("b,ih,iw,ic,oc,taps,stride,dil,pad,windows", [
+    (2, 170, 166, 16, 65, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True), (8, 56, 56, 32, 96, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True),
+    (24, 56, 50, 16, 97, (3, 3), (1, 1), (1, 1), (0, 2, 1, 0), True), (60, 29, 31, 32, 128, (2, 3), (1, 1), (1, 2), (1, 0, 2, 1), True),
+    (50, 56, 56, 64, 128, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1), True), (30, 60, 61, 48, 96, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1), True),
+    (7, 56, 56, 96, 90, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True), (19, 56, 56, 16, 80, (3, 5), (1, 1), (2, 1), (2, 2, 2, 2), True),
+    (2, 224, 224, 3, 96, (7, 7), (2, 2), (1, 1), (3, 3, 3, 3), True), (2, 220, 227, 3, 128, (7, 7), (2, 2), (1, 1), (3, 2, 3, 2), True),
+    (1, 170, 163, 4, 70, (5, 5), (1, 1), (1, 1), (2, 2, 2, 2), True), (2, 113, 120, 3, 101, (9, 3), (1, 1), (2, 1), (4, 4, 1, 1), True),
+    (6, 56, 56, 32, 96, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), False), (11, 56, 56, 64, 128, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), False),
+    (19, 56, 56, 96, 96, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), False), (19, 56, 56, 64, 128, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), False),
+    (1, 224, 224, 3, 96, (7, 7), (2, 2), (1, 1), (3, 3, 3, 3), False)])
 @pytest.mark.parametrize("act", [K.ACT_NONE, K.ACT_RELU])
-def test_convolution_windows_of_more_channels(orc, b, ih, iw, ic, oc, taps, stride, dil, pad, act):
+def test_convolution_windows_of_more_channels(orc, b, ih, iw, ic, oc, taps, stride, dil, pad, windows, act):
     import torch
     from oracle import pyoracle
     rng = np.random.default_rng(oc * 100 + ic)
@@ -188,6 +204,8 @@ def test_convolution_windows_of_more_channels(orc, b, ih, iw, ic, oc, taps, stri
     orc.set_threads(16)
     want = orc.conv_int8(x, w, bias, shape, 0.02, 4, sw, zp, so, -6, act)
     got = conv.run(torch.from_numpy(x).cuda())
+    kernel, form = _last_kernel()
+    assert (kernel == "conv_window_kernel") == windows and (not windows or form[:2] == [(oc + 31) // 32, ic <= 4])
     assert np.array_equal(got.cpu().numpy(), want)
     assert torch.equal(conv.run(torch.from_numpy(x).cuda()), got)
 
@@ -236,13 +254,15 @@ def _matmul_pair(rng, n, k, asymmetric, dynamic, **kw):
     return w, bias, sw, zw.astype(np.int32), make
 
 
-# the rule picks, in this order: 64 x 64 (one K block, two, more than the ring is deep), 64 x 128, 128 x 128, 192 x 128 (the
-# last tile reaches past the packed weights), 128 x 256, 256 x 128, 192 x 256, 256 x 256 tiles
-@pytest.mark.parametrize("m,n,k", [(65, 250, 128), (65, 250, 144), (130, 200, 1040), (129, 257, 1000), (700, 2100, 160),
-                                   (700, 2101, 1025), (1000, 2500, 176), (1000, 2503, 1040), (513, 9003, 1040),
-                                   (1100, 6001, 1040), (300, 21000, 1040), (1201, 8302, 1100), (1500, 9000, 1030)])
+# the rule picks, in this order: 64 x 64 (one K block), 32 x 32 (0: gemm_short.hip; two K blocks and more), 64 x 128, 128 x 128, 192 x 128 (the
+# last tile reaches past the packed weights), 128 x 256, 256 x 128, 192 x 256, 256 x 256 tiles, and again 64 x 64 (two K blocks, more than the
+# ring is deep).  tile: 10 x channels / 64 + rows / 64
+@pytest.mark.parametrize("m,n,k,tile", [(65, 250, 128, 11), (65, 250, 144, 0), (130, 200, 1040, 0), (129, 257, 1000, 0), (700, 2100, 160, 12),
+                                        (700, 2101, 1025, 12), (1000, 2500, 176, 22), (1000, 2503, 1040, 22), (513, 9003, 1040, 32),
+                                        (1100, 6001, 1040, 24), (300, 21000, 1040, 42), (1201, 8302, 1100, 34), (1500, 9000, 1030, 44),
+                                        (700, 1100, 144, 11), (300, 1700, 1040, 11), (200, 3000, 1552, 11)])
 @pytest.mark.parametrize("dynamic,asymmetric", [(False, False), (False, True), (True, False), (True, True)])
-def test_matmul_tile_shapes(orc, m, n, k, dynamic, asymmetric):
+def test_matmul_tile_shapes(orc, m, n, k, tile, dynamic, asymmetric):
     """Against the oracle where that takes seconds at most, against the row-major kernels (which have tests of their own)
     everywhere."""
     import torch
@@ -252,6 +272,11 @@ def test_matmul_tile_shapes(orc, m, n, k, dynamic, asymmetric):
     dev = torch.from_numpy(a).cuda()
     args = dict(in_quant=K.QuantParam(0.03, -5)) if dynamic else {}
     got = make(True).run(dev, **args).cpu().numpy()
+    kernel, form = _last_kernel()
+    if tile == 0:
+        assert kernel == "gemm_short_kernel"
+    else:
+        assert kernel in ("gemm_ring_kernel", "gemm_kblock_kernel") and form[:2] == [tile // 10, tile % 10]
     assert np.array_equal(got, make(False).run(dev, **args).cpu().numpy())
     if m * n * k < 2e9:
         orc.set_threads(16)
@@ -390,14 +415,16 @@ def test_matmul_group_of_one_on_few_ragged_rows(m, k, n, copies, how):
 
 
 # small products, whose K the waves of a workgroup share: two K blocks (half the waves have none), the last with one byte, a chunk and all but
-# one; up to 12 blocks and beyond (four and eight waves), 64 channels x 32 rows, one tile past 256 of each kind; last rows and channels that
-# are partly there
-@pytest.mark.parametrize("m,n,k", [(3, 1, 129), (32, 31, 144), (33, 65, 255), (64, 4095, 256), (65, 2700, 257), (95, 96, 1535), (97, 33, 1537),
-                                   (64, 100, 1536), (40, 4096, 1552), (130, 1600, 1040), (257, 1793, 897), (256, 2048, 896), (129, 2, 4095),
-                                   (70, 300, 4080), (60, 700, 4113), (500, 520, 300), (33, 1001, 9001),
-                                   (4, 24576, 768), (16, 8192, 1024), (17, 8193, 1024), (16, 7168, 1536), (32, 8192, 1536)])
+# one; up to 12 blocks and beyond (four and eight waves), 64 channels x 32 rows, one tile past 256 of each kind (tile 0: another kernel); last
+# rows and channels that are partly there.  tile: 10 x waves + blocks of 32 channels; copied: odd rows come as whole chunks of a padded copy
+@pytest.mark.parametrize("m,n,k,tile,copied", [
+    (3, 1, 129, 41, False), (32, 31, 144, 41, False), (33, 65, 255, 41, False), (64, 4095, 256, 41, False), (65, 2700, 257, 41, False),
+    (95, 96, 1535, 41, False), (97, 33, 1537, 81, False), (64, 100, 1536, 41, False), (40, 4096, 1552, 81, False), (130, 1600, 1040, 41, False),
+    (257, 1793, 897, 0, False), (256, 2048, 896, 82, False), (129, 2, 4095, 81, False), (70, 300, 4080, 81, False), (60, 700, 4113, 81, True),
+    (500, 520, 300, 41, False), (33, 1001, 9001, 81, True), (4, 24576, 768, 41, False), (16, 8192, 1024, 41, False), (17, 8193, 1024, 0, False),
+    (16, 7168, 1536, 41, True), (32, 8192, 1536, 41, False)])
 @pytest.mark.parametrize("dynamic,asymmetric", [(False, False), (False, True), (True, False), (True, True)])
-def test_matmul_small_products(orc, m, n, k, dynamic, asymmetric):
+def test_matmul_small_products(orc, m, n, k, tile, copied, dynamic, asymmetric):
     """Against the oracle, bit by bit (integer sums, then a fixed sequence of rounded steps): rows at an aligned and at an odd address,
     in the middle of larger ones' bytes, which must not count; and with a scale per row."""
     import torch
@@ -413,7 +440,13 @@ def test_matmul_small_products(orc, m, n, k, dynamic, asymmetric):
     for before in (0, 16, 1, 11):
         flat = torch.full((before + m * k + 64,), 99, dtype=torch.int8, device="cuda")
         flat[before:before + m * k] = torch.from_numpy(a.reshape(-1)).cuda()
-        got = kern.run(flat[before:before + m * k].view(m, k), **args).cpu().numpy()
+        rows = flat[before:before + m * k].view(m, k)
+        got = kern.run(rows, **args).cpu().numpy()
+        kernel, form = _last_kernel()
+        assert (kernel == "gemm_short_kernel") == (tile != 0)
+        if tile != 0:
+            odd = (rows.data_ptr() | k) % 16 != 0
+            assert form[:2] + form[-1:] == [tile // 10, tile % 10, odd and not copied], before
         assert np.array_equal(got.view(np.int8), want.view(np.int8)), before
     if dynamic:
         x = rng.standard_normal((m, k)).astype(np.float32)

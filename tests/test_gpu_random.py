@@ -71,8 +71,8 @@ def test_random_few_tiles_long_k(orc, seed):
 @pytest.mark.parametrize("seed", [11])
 def test_random_decode_rows_against_wide_matrices(orc, seed):
     """2..32 activation rows against 8192 channels and more with K up to 4096: the matrix-core decode kernel with three
-    channel groups per workgroup (ragged last workgroups, ragged K, zero points, every activation), singly and as a
-    group launch of two members."""
+    channel groups per workgroup (ragged last workgroups, ragged K, zero points, every activation), singly (short K
+    from three rows on: 32 x 32 tiles) and as a group launch of two members."""
     import torch
     rng = np.random.default_rng(seed)
     orc.set_threads(16)
