@@ -424,13 +424,27 @@ static const SplitCost *choose_split(int m, int k, int n, const TileCost &whole,
 // 33 x 1024 x 4096 7.05 / 5.2, 65 x 3072 x 1024 (288 tiles of 32 x 32, 144 of 64 x 32) 4.65 / 4.20, 128 x 4096 x 4096 (256 of 64 x 32) 9.9 / 8.9,
 // 1000 x 500 x 256 3.69 / 3.45 (512), 700 x 1024 x 512 (fp32) 4.8 / 4.24 (704); not taken: 160 x 3072 x 768 4.20 / 4.34 (480), 333 x 1536 x 512
 // 3.97 / 4.06 (528), 512 x 768 x 128 3.17 / 3.38, 200 x 3072 x 1024 4.47 / 5.24 (336 of 64 x 32: 6.7), 200 x 4096 x 4096 10.1 / 14.6 (448 of 64 x 32),
-// 65 x 4096 x 11008 18.5 / 18.8.  Up to 32 rows, which the decode kernels read long K for with 16 channels a workgroup: 16 x 768 x 768 4.02 /
-// 3.38, 16 x 5000 x 768 4.95 / 3.41, 32 x 8192 x 1024 5.42 / 3.73, 16 x 7000 x 1536 5.42 / 4.42, 32 x 24000 x 768 (750 tiles) 10.1 / 6.1; not
-// taken: 8 x 768 x 3072 3.62 / 4.51, 32 x 4096 x 4096 6.7 / 7.6, 16 x 8192 x 1536 (256) 4.72 / 4.92, 16 x 12288 x 1024 (384) 4.52 / 5.16.
+// 65 x 4096 x 11008 18.5 / 18.8.
 struct ShortTile {
   int tile;  // as launch_gemm_short has it
   float cost;
 };
+// The most K blocks of up to 32 rows, which the decode kernels read K in 16 channels a workgroup for, three times 16 from 8192 channels on:
+// quick at long K, and quicker the fewer the rows, as long as one round of their workgroups holds all channels.  Time of this relative to
+// theirs, weights from memory, over rows of any length and int8 and fp32 output:
+//   up to 4 rows   768 channels 4 blocks 0.91 - 1.01, 6 0.95 - 1.08, 10 1.23 - 1.29; 4096 3 0.91 - 1.02, 5 1.04 - 1.15, 12 1.16 - 1.39;
+//                  6144 7 0.9 - 1.0, 9 1.05 - 1.09; 12288 3 0.96 - 1.03, 5 1.05; 16384 6 0.83 - 0.85
+//   up to 8        768 6 0.92 - 0.98, 9 1.01 - 1.12; 2048 6 0.89 - 1.06, 9 1.12 - 1.27; 4096 5 0.99 - 1.04, 9 1.16 - 1.22; 6144 12 0.92 - 1.05;
+//                  8192 5 0.94 - 0.99, 8 1.02 - 1.09; 24576 6 0.9
+//   up to 32       512 12 0.82 - 0.97; 768 12 0.91 - 1.06; 2048 8 0.83 - 0.99, 10 0.96 - 1.10; 4096 8 0.86 - 0.98, 10 0.93 - 1.09; 6144 12 0.68 -
+//                  0.99; 8192 8 0.71 - 1.01; 17 rows and more 8192 12 0.86 - 0.92
+// us: 4 x 768 x 1277 3.51 / 4.41, 8 x 2048 x 1520 3.66 / 4.48, 4 x 768 x 448 3.27 / 2.98, 16 x 5000 x 768 4.95 / 3.41, 32 x 24000 x 768 10.1 / 6.1.
+static int few_rows_most_blocks(int m, int n) {
+  const bool second_round = (n > kGemvNarrowChannels && n < 8192) || n > 12288;
+  if (m <= 4) return n <= 2048 ? 4 : second_round ? 7 : 3;
+  if (m <= 8) return n <= 2048 ? 6 : second_round ? 12 : 5;
+  return n <= 768 || second_round || (m > 16 && n >= 8192) ? 12 : 8;
+}
 static ShortTile short_tile(int m, int k, int n, bool requant) {
   const int kb = (k + 127) / 128;
   const int64_t rows = (m + 31) / 32, small = rows * ((n + 31) / 32), wide = rows * ((n + 63) / 64);
@@ -440,7 +454,8 @@ static ShortTile short_tile(int m, int k, int n, bool requant) {
     return a + pass * (float)((kb + 2 * waves - 1) / (2 * waves)) + a_cu * (block * (float)kb + tile);
   };
   const auto four = [&] { return ShortTile{41, cost(4, small, 2.55f, 0.54f, 0.06f, 0.22f)}; };
-  if (m <= kGemvGroupMaxRows) return kb <= 12 && small <= (kb <= 6 ? 768 : kb <= 8 || m > 16 ? 256 : 224) ? four() : ShortTile{0, 0};
+  if (m <= kGemvGroupMaxRows)  // (tiles: 16 x 8192 x 1536, 256 of them, 4.72 / 4.92; 16 x 12288 x 1024, 384, 4.52 / 5.16)
+    return kb <= few_rows_most_blocks(m, n) && small <= (kb <= 6 ? 768 : kb <= 8 || m > 16 ? 256 : 224) ? four() : ShortTile{0, 0};
   if (small <= 256) return kb <= 12 ? four() : ShortTile{81, cost(8, small, 2.3f, 0.93f, 0.053f, 0.55f)};
   if (kb < 7) return small <= (!requant ? 768 : kb == 2 ? 256 : kb < 6 ? 512 : 448) ? four() : ShortTile{0, 0};
   return wide <= 256 && kb <= 64 ? ShortTile{82, cost(8, wide, 1.9f, 1.65f, 0.073f, 1.03f)} : ShortTile{0, 0};

@@ -422,7 +422,13 @@ def test_matmul_group_of_one_on_few_ragged_rows(m, k, n, copies, how):
     (95, 96, 1535, 41, False), (97, 33, 1537, 81, False), (64, 100, 1536, 41, False), (40, 4096, 1552, 81, False), (130, 1600, 1040, 41, False),
     (257, 1793, 897, 0, False), (256, 2048, 896, 82, False), (129, 2, 4095, 81, False), (70, 300, 4080, 81, False), (60, 700, 4113, 81, True),
     (500, 520, 300, 41, False), (33, 1001, 9001, 81, True), (4, 24576, 768, 41, False), (16, 8192, 1024, 41, False), (17, 8193, 1024, 0, False),
-    (16, 7168, 1536, 41, True), (32, 8192, 1536, 41, False)])
+    (16, 7168, 1536, 41, True), (32, 8192, 1536, 41, False),
+    # up to 32 rows, both sides of the lines at 4, 8 and 16 rows and at 768, 2048, 4096, 8192 and 12288 channels
+    (4, 2048, 512, 41, False), (4, 2048, 513, 0, False), (4, 2049, 384, 41, False), (4, 2049, 385, 0, False), (4, 4097, 896, 41, False),
+    (4, 4097, 897, 0, False), (3, 8192, 384, 41, False), (3, 12288, 400, 0, False), (3, 12289, 400, 41, False), (5, 2048, 768, 41, False),
+    (8, 2048, 769, 0, False), (8, 2049, 640, 41, False), (8, 4096, 641, 0, False), (8, 4097, 1536, 41, False), (8, 8192, 656, 0, False),
+    (9, 768, 1536, 41, False), (16, 769, 1024, 41, False), (9, 769, 1025, 0, False), (32, 4096, 1040, 0, False), (32, 4097, 1536, 41, False),
+    (17, 8191, 1041, 41, False)])
 @pytest.mark.parametrize("dynamic,asymmetric", [(False, False), (False, True), (True, False), (True, True)])
 def test_matmul_small_products(orc, m, n, k, tile, copied, dynamic, asymmetric):
     """Against the oracle, bit by bit (integer sums, then a fixed sequence of rounded steps): rows at an aligned and at an odd address,
