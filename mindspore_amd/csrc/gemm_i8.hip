@@ -460,6 +460,15 @@ static ShortTile short_tile(int m, int k, int n, bool requant) {
   if (kb < 7) return small <= (!requant ? 768 : kb == 2 ? 256 : kb < 6 ? 512 : 448) ? four() : ShortTile{0, 0};
   return wide <= 256 && kb <= 64 ? ShortTile{82, cost(8, wide, 1.9f, 1.65f, 0.073f, 1.03f)} : ShortTile{0, 0};
 }
+// The same for rows in whole chunks, where nothing is copied for the other tiles: five row tiles of int8 that nearly fill the device read the
+// weights five times to three, up to 20 K blocks.  Time of this relative to theirs: 160 x 3072 x 1280 1.10 (5.71 / 5.15 us), 160 x 3200 x 2560
+// 1.09, 160 x 2880 x 2560 1.07, 129 x 3200 x 2560 1.06; not so 160 x 2500 x 2048 0.98, 160 x 2881 x 3072 0.94, 160 x 3200 x 3072 1.04, with fp32
+// output 160 x 3072 x 1280 1.01, 192 x 2560 1.0, 128 x 4096 0.9; rows that would have to be copied 0.76 - 0.9.
+static ShortTile short_tile_of_chunks(int m, int k, int n, bool requant) {
+  const bool full = requant && (m + 31) / 32 == 5 && (n + 63) / 64 * 5 > 224 && k <= 20 * 128;
+  const ShortTile t = short_tile(m, k, n, requant);
+  return full && t.tile == 82 ? ShortTile{0, 0} : t;
+}
 // From K = 4096 on, more rows than the decode kernels take stay with K in parts (gemm_split.hip) on the streams that have memory for
 // that: its tests hold it to them.  128 x 1024 x 4096 7.7 us in parts, 5.3 here.
 static bool short_goes_first(int m, int k) { return m <= kGemvMaxRows || k < 4096; }
@@ -482,7 +491,7 @@ static int launch_pick_tile(const GemmArgs &g, const RequantParams &rq, const De
   // against 7.9 us.
   if (g.wb != nullptr && kblock_ok && (g.k >= 1024 || tiles_m <= 256)) {
     const bool short_form = EPI == EPI_REQUANT ? FAST : !FAST;
-    const int in_short = short_form ? short_tile(g.m, g.k, g.n, EPI == EPI_REQUANT).tile : 0;
+    const int in_short = short_form ? short_tile_of_chunks(g.m, g.k, g.n, EPI == EPI_REQUANT).tile : 0;
     if (in_short != 0 && short_goes_first(g.m, g.k)) return launch_gemm_short(in_short, false, EPI == EPI_REQUANT, HAS_ZW, g, rq, dq, stream);
     if (EPI == EPI_DEQUANT && g.k < 1024 && tiles_m >= 128) return launch_gemm_kblock(22, false, HAS_ZW, FAST, g, rq, dq, stream);
     float cost;
@@ -763,7 +772,7 @@ static const TileCost *group_tile(int64_t lda, int m, int k, int count, const We
     int parts;
     const TileCost &whole = cheapest_tile(m, k, 1, n + i, &cost);
     alone += cost;
-    const ShortTile in_short = short_tile(m, k, n[i], requant);  // (the members' forms are those of gemm_short.hip and gemm_split.hip)
+    const ShortTile in_short = short_tile_of_chunks(m, k, n[i], requant);  // (the members' forms are those of gemm_short.hip and gemm_split.hip)
     alone_unsplit += in_short.tile != 0 ? in_short.cost : cost;
     if (in_short.tile != 0 && short_goes_first(m, k)) {
       cost = in_short.cost;

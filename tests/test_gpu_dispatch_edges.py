@@ -416,7 +416,8 @@ def test_matmul_group_of_one_on_few_ragged_rows(m, k, n, copies, how):
 
 # small products, whose K the waves of a workgroup share: two K blocks (half the waves have none), the last with one byte, a chunk and all but
 # one; up to 12 blocks and beyond (four and eight waves), 64 channels x 32 rows, one tile past 256 of each kind (tile 0: another kernel); last
-# rows and channels that are partly there.  tile: 10 x waves + blocks of 32 channels; copied: odd rows come as whole chunks of a padded copy
+# rows and channels that are partly there.  tile: 10 x waves + blocks of 32 channels; copied: odd rows come as whole chunks of a padded copy; None:
+# only odd rows run here, and whole chunks of int8 on another kernel
 @pytest.mark.parametrize("m,n,k,tile,copied", [
     (3, 1, 129, 41, False), (32, 31, 144, 41, False), (33, 65, 255, 41, False), (64, 4095, 256, 41, False), (65, 2700, 257, 41, False),
     (95, 96, 1535, 41, False), (97, 33, 1537, 81, False), (64, 100, 1536, 41, False), (40, 4096, 1552, 81, False), (130, 1600, 1040, 41, False),
@@ -428,7 +429,9 @@ def test_matmul_group_of_one_on_few_ragged_rows(m, k, n, copies, how):
     (4, 4097, 897, 0, False), (3, 8192, 384, 41, False), (3, 12288, 400, 0, False), (3, 12289, 400, 41, False), (5, 2048, 768, 41, False),
     (8, 2048, 769, 0, False), (8, 2049, 640, 41, False), (8, 4096, 641, 0, False), (8, 4097, 1536, 41, False), (8, 8192, 656, 0, False),
     (9, 768, 1536, 41, False), (16, 769, 1024, 41, False), (9, 769, 1025, 0, False), (32, 4096, 1040, 0, False), (32, 4097, 1536, 41, False),
-    (17, 8191, 1041, 41, False)])
+    (17, 8191, 1041, 41, False),
+    # five row tiles that nearly fill the device, and on the other side of that line
+    (160, 2817, 1280, 82, None), (129, 3200, 2560, 82, None), (160, 2816, 1280, 82, False), (129, 3200, 2576, 82, False)])
 @pytest.mark.parametrize("dynamic,asymmetric", [(False, False), (False, True), (True, False), (True, True)])
 def test_matmul_small_products(orc, m, n, k, tile, copied, dynamic, asymmetric):
     """Against the oracle, bit by bit (integer sums, then a fixed sequence of rounded steps): rows at an aligned and at an odd address,
@@ -449,9 +452,10 @@ def test_matmul_small_products(orc, m, n, k, tile, copied, dynamic, asymmetric):
         rows = flat[before:before + m * k].view(m, k)
         got = kern.run(rows, **args).cpu().numpy()
         kernel, form = _last_kernel()
-        assert (kernel == "gemm_short_kernel") == (tile != 0)
-        if tile != 0:
-            odd = (rows.data_ptr() | k) % 16 != 0
+        odd = (rows.data_ptr() | k) % 16 != 0
+        here = tile != 0 and (copied is not None or odd or dynamic)
+        assert (kernel == "gemm_short_kernel") == here
+        if here:
             assert form[:2] + form[-1:] == [tile // 10, tile % 10, odd and not copied], before
         assert np.array_equal(got.view(np.int8), want.view(np.int8)), before
     if dynamic:
