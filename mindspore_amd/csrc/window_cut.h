@@ -70,22 +70,44 @@ static inline bool cut_window(const ConvGeom &g, WindowCut *best) {
 // channels -> 64, 49 workgroups 4.42 / 4.42, 98 4.46 / 4.48, 196 6.2 / 4.65, 392 8.55 / 6.05, 784 12.2 / 9.55, 1568 20.5 / 16.5;
 // -> 96, 49 4.82 / 4.89, 98 6.71 / 5.06, 1568 35.9 / 19.6, -> 128, 98 6.78 / 5.73, 1568 38.1 / 24.0;
 // 5x5 on 4 (five loads) 4.85 / 4.4 and 14.8 / 14.7, -> 96, 90 workgroups 5.10 / 4.55; 5x5 on 3 (three) 4.15 / 4.18; 3x3 on 3 (two)
-// 5.17 / 5.55 and 7.7 / 8.8.
+// 5.17 / 5.55 and 7.7 / 8.8.  97 to 127 channels, whose stores have ragged ends in every fourth block: 96 to 167 workgroups 0.61 to 1.23 of the
+// time, on average 1.03, from 168 on 0.49 to 1.1 and 0.85; 112 and 128 channels 0.83 and 0.68.
 constexpr int kWindowLeastTiles = 168, kWindowLeastWideTiles = 96;
 static inline int least_tiles(const ConvGeom &g) {
-  return window_blocks(g) == 3 || (window_blocks(g) == 4 && packed_window(g)) ? kWindowLeastWideTiles : kWindowLeastTiles;
+  return window_blocks(g) == 3 || (window_blocks(g) == 4 && packed_window(g) && g.out_c % 16 == 0) ? kWindowLeastWideTiles : kWindowLeastTiles;
 }
-// More than 64 channels beside several taps of 16-channel-aligned images mostly leave room for one workgroup a CU, and what counts then is
-// how many rounds of them there are beside those of the GEMM's 128 x 128 tiles, two a CU.  A round takes 0.7 of one of those for 65 to 96
-// channels, 0.85 to 0.9 for up to 128 (full rounds: 96 -> 96 8.75 / 12.5, 64 -> 128 7.85 / 9.35); two a CU as long as one of the GEMM's
-// rounds and do twice as much.  Relative time at 252 workgroups (against one of the GEMM's rounds) 0.70, 266 1.11, 280 1.18 (not taken),
-// 336 (against two) 0.78, 512 0.69, 518 0.95 (not taken); 64 -> 128 336 0.96, 518 1.14 (not taken).
-static inline bool wide_rounds_pay(const ConvGeom &g, const WindowCut &c) {
+// More than 64 channels against windows of 16-channel-aligned images: what both take, in us, least squares over 1599 shapes (windows of 2 to 25
+// taps, strides 1 to 3, 14 x 14 to 112 x 112 images, 32 to 1300 rectangles; median error 3 to 5 %).  Mostly one workgroup has a CU, and what counts
+// is how many rounds of them there are beside those of the GEMM's 128 x 128 tiles, two a CU.  A rectangle holds every pixel under it, also those
+// that strides leave out, which beside few taps is more than the GEMM fetches; and channels that are no multiple of 16 have ragged stores.
+// Of the 1599, by rounds alone 994 ran here, at 0.85 of the GEMM's time on average and 117 of them at 1.03 to 1.53; by this 829, at 0.81, twelve at
+// 1.04 to 1.14; 17 that took 0.86 to 0.95 are given up.  us, GEMM / this: 32 x 56 x 56, 96 -> 96 21.7 / 14.3; not taken: 1x2, stride 2,
+// 67 x 40 x 40, 128 -> 96 5.96 / 7.73; 1x3, stride 2, 23 x 112 x 112, 64 -> 80 9.77 / 12.28; 3x3 12 x 80 x 80, 32 -> 97 14.4 / 16.1.
+static inline bool window_is_quicker(const ConvGeom &g, const WindowCut &c) {
+  struct Cost {
+    float launch, whole, part, patch, k, ragged, bytes;
+  };
+  constexpr Cost kTwo{2.5f, 1.06f, 2.8f, 0.033f, 0.66f, 0.69f, 1.38f}, kThree{1.9f, 2.55f, 0.1f, 0.026f, 0.51f, 0.25f, 0.92f},
+      kFour{2.2f, 2.7f, -0.3f, 0.027f, 0.68f, 1.88f, 1.79f};
   if (window_blocks(g) < 3 || packed_window(g)) return true;
+  // (four blocks take the registers of one workgroup)
   const bool two = window_blocks(g) == 3 && c.weight_bytes + c.patch_bytes + 8 * c.steps <= kWindowLds;
+  const Cost &cost = two ? kTwo : window_blocks(g) == 3 ? kThree : kFour;
+  const auto whole = [](int64_t tiles, int slots) { return (float)((tiles + slots - 1) / slots); };
+  const int slots = two ? 512 : 256;
   const int64_t gemm_tiles = ((int64_t)g.batch * g.out_h * g.out_w + 127) / 128;
-  const int64_t gemm_rounds = gemm_tiles < 128 ? 1 : (gemm_tiles + 511) / 512, slots = two ? 512 : 256, rounds = (c.tiles + slots - 1) / slots;
-  return (float)rounds * (two ? 0.98f : window_blocks(g) == 3 ? 0.75f : 0.9f) < (float)gemm_rounds;
+  const float k = (float)(g.kernel_h * g.kernel_w * g.in_c) / 100.0f, ragged = g.out_c % 16 != 0, bytes = g.out_c % 4 != 0;
+  const float rounds = (float)c.tiles / (float)slots, mixed = 0.6f * whole(c.tiles, slots) + 0.4f * rounds;
+  const float here = cost.launch + cost.whole * whole(c.tiles, slots) + rounds * (cost.part + cost.ragged * ragged + cost.bytes * bytes) +
+                     mixed * (cost.patch * (float)(c.patch_bytes / 1024) + cost.k * k);
+  if (gemm_tiles < 128) {  // (64 x 64 there)
+    const float part = (float)gemm_tiles / 128.0f;
+    return here < 3.88f + 0.18f * part + k * (0.35f + 0.105f * part);
+  }
+  const float gemm_rounds = (float)gemm_tiles / 512.0f, gemm_whole = whole(gemm_tiles, 512);
+  const float passed_over = (float)(g.stride_h * g.stride_w * g.in_c) / 100.0f;  // (lines of the image of which the taps read a part)
+  return here < 2.61f + 1.41f * gemm_whole + gemm_rounds * (2.11f + 1.35f * ragged + 0.48f * bytes + 0.24f * passed_over) +
+                    k * (0.274f * gemm_whole + 0.546f * gemm_rounds + 0.186f * std::min(2.0f * gemm_rounds, 1.0f));
 }
 // Geometries that the kernel has a form for, images aside.
 static inline bool window_form(const ConvGeom &g) {
@@ -95,25 +117,32 @@ static inline bool window_form(const ConvGeom &g) {
            g.kernel_h * (g.kernel_w * g.in_c > 16 ? 2 : 1) > 8;
   return (g.in_c & 15) == 0 && g.out_c <= 128 && taps > 1 && (int64_t)taps * g.in_c <= 2048;
 }
-// Whether images exist that choose_window has rectangles for: with half of a workgroup's pixels (choose_window), at least 8 wide
-// (cut_window).  No rectangle of a 3x3 on 128 channels against 97 to 128, for one, fits beside the 144 KiB of its weights.
+// Images in rectangles that are quicker than what else there is.
+static inline bool rectangles_pay(const ConvGeom &g, WindowCut *c) {
+  return cut_window(g, c) && c->tiles >= least_tiles(g) && window_is_quicker(g, *c) && c->tiles < 1 << 23 &&  // (2^32 threads)
+         c->tiles * (32 * kWaves / 2) <= (int64_t)g.batch * g.out_h * g.out_w;
+}
+// Whether there are such images, asked of as many as make one round of rectangles to eight, each a rectangle of at least half of a workgroup's
+// pixels.  No rectangle of a 3x3 on 128 channels against 97 to 128, for one, fits beside the 144 KiB of its weights.
 static inline bool window_fits(const ConvGeom &g) {
   if (!window_form(g)) return false;
-  ConvGeom least = g;
-  least.batch = 1;
-  for (least.out_w = 8; least.out_w <= 64; ++least.out_w) {
-    least.out_h = (32 * kWaves / 2 + least.out_w - 1) / least.out_w;
-    WindowCut c;
-    if (cut_window(least, &c) && c.tiles == 1) return true;
-  }
+  ConvGeom one = g;
+  for (one.out_w = 8; one.out_w <= 64; ++one.out_w)
+    for (one.out_h = 32 * kWaves / one.out_w; 2 * one.out_h * one.out_w >= 32 * kWaves; --one.out_h) {
+      WindowCut c;
+      one.batch = 1;
+      if (!cut_window(one, &c) || c.tiles != 1) continue;
+      for (const int tiles : {kWindowLeastTiles, 256, 512, 768, 2048}) {
+        c.tiles = one.batch = tiles;
+        if (window_is_quicker(one, c)) return true;
+      }
+    }
   return false;
 }
 static inline bool choose_window(const ConvGeom &g, bool aligned, WindowCut *c) {
   const int64_t image = (int64_t)g.in_h * g.in_w * g.in_c;
   if (!window_form(g) || g.batch * image < 16 || image >= (int64_t)1 << 31) return false;
-  if (!aligned && !packed_window(g)) return false;
-  return cut_window(g, c) && c->tiles >= least_tiles(g) && wide_rounds_pay(g, *c) && c->tiles < 1 << 23 &&  // (2^32 threads)
-         c->tiles * (32 * kWaves / 2) <= (int64_t)g.batch * g.out_h * g.out_w;
+  return (aligned || packed_window(g)) && rectangles_pay(g, c);
 }
 
 }  // namespace mi

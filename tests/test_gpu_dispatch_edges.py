@@ -177,17 +177,21 @@ def test_convolution_1x1_into_large_images(orc, pixels, k, n, act):
 
 # windows in LDS against 65 to 128 channels: three blocks of 32 and four, the last of them full or not; strides, dilations and uneven pads; a
 # rectangle that fills the LDS (64 -> 128, stride 2).  Not on windows: fewer rectangles than the rule's least, and one round more than the GEMM's,
-# of three blocks and of four; few rectangles of a first layer
+# of three blocks and of four; few rectangles of a first layer; four blocks with ragged stores; more pixels than the taps read
 @pytest.mark.parametrize("b,ih,iw,ic,oc,taps,stride,dil,pad,windows", [
     (2, 170, 166, 16, 65, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True), (8, 56, 56, 32, 96, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True),
-    (24, 56, 50, 16, 97, (3, 3), (1, 1), (1, 1), (0, 2, 1, 0), True), (60, 29, 31, 32, 128, (2, 3), (1, 1), (1, 2), (1, 0, 2, 1), True),
+    (24, 56, 50, 16, 97, (3, 3), (1, 1), (1, 1), (0, 2, 1, 0), False), (20, 56, 50, 64, 97, (3, 3), (1, 1), (1, 1), (0, 2, 1, 0), True), (60, 29, 31, 32, 128, (2, 3), (1, 1), (1, 2), (1, 0, 2, 1), True),
     (50, 56, 56, 64, 128, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1), True), (30, 60, 61, 48, 96, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1), True),
     (7, 56, 56, 96, 90, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True), (19, 56, 56, 16, 80, (3, 5), (1, 1), (2, 1), (2, 2, 2, 2), True),
     (2, 224, 224, 3, 96, (7, 7), (2, 2), (1, 1), (3, 3, 3, 3), True), (2, 220, 227, 3, 128, (7, 7), (2, 2), (1, 1), (3, 2, 3, 2), True),
-    (1, 170, 163, 4, 70, (5, 5), (1, 1), (1, 1), (2, 2, 2, 2), True), (2, 113, 120, 3, 101, (9, 3), (1, 1), (2, 1), (4, 4, 1, 1), True),
+    (1, 170, 163, 4, 70, (5, 5), (1, 1), (1, 1), (2, 2, 2, 2), True), (2, 113, 120, 3, 101, (9, 3), (1, 1), (2, 1), (4, 4, 1, 1), False), (4, 113, 120, 3, 101, (9, 3), (1, 1), (2, 1), (4, 4, 1, 1), True),
     (6, 56, 56, 32, 96, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), False), (11, 56, 56, 64, 128, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), False),
     (19, 56, 56, 96, 96, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), False), (19, 56, 56, 64, 128, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), False),
-    (1, 224, 224, 3, 96, (7, 7), (2, 2), (1, 1), (3, 3, 3, 3), False)])
+    (1, 224, 224, 3, 96, (7, 7), (2, 2), (1, 1), (3, 3, 3, 3), False),
+    # rectangles of more pixels than the taps read: too few, in two rounds, far more; and in one round, and where two have a CU
+    (67, 40, 40, 128, 96, (1, 2), (2, 2), (1, 1), (0, 0, 1, 1), False), (23, 112, 112, 64, 80, (1, 3), (2, 2), (1, 1), (0, 0, 1, 1), False),
+    (96, 28, 28, 64, 96, (5, 1), (2, 2), (1, 1), (2, 2, 0, 0), False), (96, 56, 56, 64, 96, (3, 1), (3, 3), (1, 1), (1, 1, 0, 0), False),
+    (57, 56, 56, 80, 96, (3, 1), (2, 2), (1, 1), (1, 1, 0, 0), True), (96, 56, 56, 16, 96, (1, 2), (2, 2), (1, 1), (0, 0, 1, 1), True)])
 @pytest.mark.parametrize("act", [K.ACT_NONE, K.ACT_RELU])
 def test_convolution_windows_of_more_channels(orc, b, ih, iw, ic, oc, taps, stride, dil, pad, windows, act):
     import torch
