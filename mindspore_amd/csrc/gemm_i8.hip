@@ -417,7 +417,8 @@ static const SplitCost *choose_split(int m, int k, int n, const TileCost &whole,
   if (best != nullptr) *split_cost = least;
   return best;
 }
-// The tile of gemm_short.hip that is quicker than what else there is, or 0; and what it is expected to take (us, fitted like kTileCosts).
+// The tile of gemm_short.hip that is quicker than what else there is, or 0; and what it is expected to take (us, fitted like kTileCosts to 756 shapes
+// with weights from memory, median error 3 to 5 %).
 // One 32 x 32 tile a CU, of four waves up to 12 K blocks and of eight beyond, or, from 7 blocks on, one of 64 channels x 32 rows: the
 // second workgroup of a CU competes for the operands' way into it, about 100 GB/s.  With fewer blocks the launch is most of the time, and
 // several tiles a CU still pay, with fp32 output, whose stores they spread, more of them.  us per launch, the quickest otherwise / this:
@@ -449,16 +450,15 @@ static ShortTile short_tile(int m, int k, int n, bool requant) {
   const int kb = (k + 127) / 128;
   const int64_t rows = (m + 31) / 32, small = rows * ((n + 31) / 32), wide = rows * ((n + 63) / 64);
   if (kb < 2 || m <= kGemvDotRows) return {0, 0};
-  const auto cost = [kb](int waves, int64_t tiles, float a, float pass, float block, float tile) {
-    const float a_cu = (float)tiles / 256.0f;
-    return a + pass * (float)((kb + 2 * waves - 1) / (2 * waves)) + a_cu * (block * (float)kb + tile);
+  const auto cost = [kb](int64_t tiles, float a, float k, float block, float tile) {
+    return a + k * (float)kb + (float)tiles / 256.0f * (block * (float)kb + tile);
   };
-  const auto four = [&] { return ShortTile{41, cost(4, small, 2.55f, 0.54f, 0.06f, 0.22f)}; };
+  const auto four = [&] { return ShortTile{41, cost(small, 2.68f, 0.083f, 0.094f, 0.22f)}; };
   if (m <= kGemvGroupMaxRows)  // (tiles: 16 x 8192 x 1536, 256 of them, 4.72 / 4.92; 16 x 12288 x 1024, 384, 4.52 / 5.16)
     return kb <= few_rows_most_blocks(m, n) && small <= (kb <= 6 ? 768 : kb <= 8 || m > 16 ? 256 : 224) ? four() : ShortTile{0, 0};
-  if (small <= 256) return kb <= 12 ? four() : ShortTile{81, cost(8, small, 2.3f, 0.93f, 0.053f, 0.55f)};
+  if (small <= 256) return kb <= 12 ? four() : ShortTile{81, cost(small, 2.53f, 0.08f, 0.04f, 0.47f)};
   if (kb < 7) return small <= (!requant ? 768 : kb == 2 ? 256 : kb < 6 ? 512 : 448) ? four() : ShortTile{0, 0};
-  return wide <= 256 && kb <= 64 ? ShortTile{82, cost(8, wide, 1.9f, 1.65f, 0.073f, 1.03f)} : ShortTile{0, 0};
+  return wide <= 256 && kb <= 64 ? ShortTile{82, cost(wide, 3.6f, 0.089f, 0.1f, -0.28f)} : ShortTile{0, 0};
 }
 // The same for rows in whole chunks, where nothing is copied for the other tiles: five row tiles of int8 that nearly fill the device read the
 // weights five times to three, up to 20 K blocks.  Time of this relative to theirs: 160 x 3072 x 1280 1.10 (5.71 / 5.15 us), 160 x 3200 x 2560

@@ -321,6 +321,23 @@ def test_matmul_group_on_tiles(orc, m, k, ns, how):
             assert np.array_equal(y.cpu().numpy(), want)
 
 
+# members that are small products alone: one launch of 64 x 64 tiles as long as that is quicker than a launch each
+@pytest.mark.parametrize("m,k,ns,together", [(65, 2048, (256, 256), True), (100, 2048, (64, 64), True), (128, 1024, (64, 64), True),
+                                             (100, 4080, (64, 64), False), (64, 3072, (512, 512), False)])
+@pytest.mark.parametrize("how", ["static", "value"])
+def test_matmul_group_of_small_products(m, k, ns, together, how):
+    import torch
+    rng = np.random.default_rng(m + k + sum(ns))
+    kernels = [_matmul_pair(rng, n, k, False, how != "static")[4](True) for n in ns]
+    a = torch.from_numpy(rng.integers(-128, 128, (m, k), dtype=np.int8)).cuda()
+    args = dict(in_quant=K.QuantParam(0.03, -5)) if how == "value" else {}
+    want = [kern.run(a, **args) for kern in kernels]
+    assert _last_kernel()[0] == "gemm_short_kernel"
+    got = K.matmul_run_group(kernels, a) if how == "static" else K.dynmm_run_group(kernels, a, **args)
+    assert ("_group_" in _last_kernel()[0]) == together
+    assert all(torch.equal(x, y) for x, y in zip(got, want))
+
+
 # ragged rows: members that read them as they are, alone, in pairs and beside one that needs the copy (decode-sized; on tiles of
 # another size); a copy for three and more; one launch on a copy
 @pytest.mark.parametrize("m,k,ns,copies", [(333, 1000, (1001,), False), (333, 1000, (1001, 1000), False), (70, 500, (65, 260), False),
