@@ -204,9 +204,9 @@ int launch_gemm_group_dequant(const TileCost &tile, const int8_t *a, int64_t lda
 // Skinny-M path (m <= kGemvMaxRows): streams the weights once with 16-byte coalesced loads.
 constexpr int kGemvMaxRows = 64;
 constexpr int kGemvGroupMaxRows = 32;  // the group launches (several matrices, one launch) stop here
-// Where gemm_short.hip does not take them (gemm_short_takes), 33..64 rows come here against at most 4096 channels, of which the kernel's workgroups hold 16 each and the GEMM's smallest
-// tile 64; against more channels the GEMM tiles have CUs enough and re-read the activations less.  us per launch at 64
-// rows, this path / the tiles: 4096 x 4096 8.8 / 11.0, 4096 x 11008 18.7 / 27.5, 768 x 3072 6.8 / 7.5, 6144 x 2048
+// 33..64 rows against at most 4096 channels come here where gemm_short.hip has no form for them (gemm_short_takes: up to 128 bytes of K, and the
+// general rounding).  Of the others, this kernel's workgroups hold 16 channels each and the GEMM's smallest tile 64; against more
+// channels the GEMM tiles have CUs enough and re-read the activations less.  us per launch at 64 rows, this path / 64 x 64 tiles and more: 4096 x 4096 8.8 / 11.0, 4096 x 11008 18.7 / 27.5, 768 x 3072 6.8 / 7.5, 6144 x 2048
 // 9.2 / 7.6, 12288 x 4096 14.5 / 13.8; at 80 rows, where a form of the kernel with eight row groups existed: 4096 x 4096
 // 11.9 / 9.8, 4096 x 11008 25.6 / 21.0, 768 x 3072 9.6 / 7.5.
 constexpr int kGemvNarrowChannels = 4096;

@@ -75,8 +75,8 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(OCB
   };
   char *patch = lds + g.weight_bytes;
   int *table = reinterpret_cast<int *>(patch + g.patch_bytes);
-  // The first weights, the pixels, the last two loads of weights of each wave: the products of the first weights begin while
-  // those are on their way.
+  // The first weights, the pixels, the last two loads of weights of each wave (three blocks: three): the products of the first weights
+  // begin while those are on their way.
   constexpr int kLate = OCB == 3 ? 3 : 2, kLateSteps = kWaves * kLate / OCB;
   static_assert(PACKED || kLateSteps * OCB == kWaves * kLate, "every wave has as many late loads");
   const int early = PACKED ? 0 : max(g.steps - kLateSteps, 0);  // steps whose weights come first
@@ -143,7 +143,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(OCB
   v16i start;
 #pragma unroll
   for (int e = 0; e < 16; ++e) start[e] = (int)kAccBias;
-  // (in order: all but a wave's last two loads are in; with fewer steps than those load, all of them are waited for)
+  // (in order: all but a wave's last kLate loads are in; with fewer steps than those load, all of them are waited for)
   if (early > 0) {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kLate) : "memory");
   } else {
@@ -254,7 +254,8 @@ static const WindowKernel kWindowKernels[4][2][2] = {
      {conv_window_kernel<1, true, kCarryForm>, conv_window_kernel<1, true, kReluForm>}},
     {{conv_window_kernel<2, false, kCarryForm>, conv_window_kernel<2, false, kReluForm>},
      {conv_window_kernel<2, true, kCarryForm>, conv_window_kernel<2, true, kReluForm>}},
-    {{conv_window_kernel<3, false, kCarryForm>, conv_window_kernel<3, false, kReluForm>}, {conv_window_kernel<3, true, kCarryForm>, conv_window_kernel<3, true, kReluForm>}},
+    {{conv_window_kernel<3, false, kCarryForm>, conv_window_kernel<3, false, kReluForm>},
+     {conv_window_kernel<3, true, kCarryForm>, conv_window_kernel<3, true, kReluForm>}},
     {{conv_window_kernel<4, false, kCarryForm>, conv_window_kernel<4, false, kReluForm>},
      {conv_window_kernel<4, true, kCarryForm>, conv_window_kernel<4, true, kReluForm>}}};
 

@@ -893,7 +893,7 @@ static int with_row_class(int m, F &&f) {  // rows rounded up to 2, 4, 8, 16 or 
   return f(integral_constant<int, 32>());
 }
 
-// 33..64 rows (against at most 4096 channels, see gemv_takes_rows): four groups of 16 activation rows against every weight
+// 33..64 rows (against at most 4096 channels, see gemv_takes_rows, of what gemm_short.hip does not take): four groups of 16 activation rows against every weight
 // fragment, two steps per pass (the staging area of 64 rows and the accumulators leave room for no more).  Measured
 // against 64 x 64 GEMM tiles in us per launch at 64 rows: 4096 x 4096 11.0 -> 8.8, 4096 x 11008 27.5 -> 18.7.
 template <bool ANY>

@@ -59,8 +59,8 @@ static inline bool cut_window(const ConvGeom &g, WindowCut *best) {
   return best->tiles != 0;
 }
 
-// Up to 128 channels, which one workgroup computes (more would fetch the pixels again), rectangles for two CUs in three, and at
-// least half of their pixels there.  Time of this relative to the gathering GEMM, 3x3: workgroups 112 1.01, 128 1.02, 140 1.02,
+// Up to 128 channels, which one workgroup computes (more would fetch the pixels again), rectangles for two CUs in three (65 to 96 channels, and
+// some first layers: three in eight), and at least half of their pixels there.  Time of this relative to the gathering GEMM, 3x3: workgroups 112 1.01, 128 1.02, 140 1.02,
 // 160 1.02, 168 0.88 0.91, 192 0.87, 196 0.89, 224 0.87, 256 0.77, 448 0.75, 1024 0.70; stride 2 256 0.74; 5x5 128 0.84, 256 0.73.
 // Rectangles filled to 0.77 0.77, 0.56 0.87, 0.39 0.90 to 1.05, 0.25 1.43, 0.19 1.40 to 2.1.
 // 65 to 96 channels, of which the GEMM's 128-channel tiles leave a quarter and more empty, already from 96 workgroups: 96 -> 96 56 1.02,
